@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define ZEN_ABI_VERSION 3 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table */
+#define ZEN_ABI_VERSION 4 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table; 4: zen_read_back, zen_count */
 
 #define ZEN_F32 0
 #define ZEN_BF16 1
@@ -471,6 +471,28 @@ int zen_bucket_sort_fits(int64_t max_count, uint32_t sentinel);
 int zen_bucket_sort_pairs(uint32_t *keys, uint32_t *vals, int64_t max_count,
                           const uint32_t *count_dev, uint32_t sentinel,
                           void *workspace, size_t workspace_bytes, int32_t *status, void *stream);
+
+/*
+ * The words a caller must know on the host before it goes on (split sizes, counts, status words): up to three
+ * segments of n words each (int64 if wide, else int32; NULL / 0: none) are widened to 64 bits and stored one
+ * after the other in host[1..] by a kernel on `stream`, and the call returns when they are there, i.e. when
+ * everything in front of it on the stream has finished.  `host` comes from zen_host_words_alloc(words): pinned,
+ * coherent host memory, which serves one call at a time (a buffer per host thread); zen_host_words_free gives
+ * it back.  These three are the only calls that allocate or that wait for the device.  No counterpart in the
+ * reference (its .tolist() and .item() calls do it, comm.py:119, tensor_load_balance.py:46-50).
+ */
+#define ZEN_READ_BACK_SEGMENTS 3
+int zen_host_words_alloc(int64_t words, int64_t **host);
+int zen_host_words_free(int64_t *host);
+int zen_read_back(const void *p0, int n0, int wide0, const void *p1, int n1, int wide1, const void *p2, int n2,
+                  int wide2, int64_t *host, int64_t words, void *stream);
+
+/*
+ * *count (int64, zeroed by the caller) += elements with key >= max(thr[0], 1); thr == NULL: the nonzero ones.
+ * Sizes the buffers of a selection that nothing is known about (tensor_load_balance.py:24-40 finds out by
+ * making the lists).
+ */
+int zen_count(const void *input, int dtype, int64_t n, const uint32_t *thr, int64_t *count, void *stream);
 
 /*
  * Reads `bytes` bytes (16-byte aligned) with coalesced non-temporal 16-byte

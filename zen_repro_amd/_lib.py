@@ -3,8 +3,9 @@ amount of torch plumbing every wrapper shares: dtype codes, stream handles,
 cached workspaces and status words.  There is no fallback: if the library is
 missing or a call fails, an exception is raised."""
 import ctypes
-import threading
 import os
+import sys
+import threading
 
 import torch  # first: makes the process use torch's HIP runtime for libzen_hip too
 
@@ -22,7 +23,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("ZEN_HIP_LIB") or os.path.join(_HERE, "csrc", "libzen_hip.so")
 
 # ZEN_ABI_VERSION of include/zen_hip.h this loader's signatures and structs are written for
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 _lib = None
 
@@ -110,6 +111,10 @@ def lib():
         "zen_sort_pairs": (i32, [vp, vp, i64, vp, i32, vp, sz, vp, vp]),
         "zen_bucket_sort_fits": (i32, [i64, ctypes.c_uint32]),
         "zen_bucket_sort_pairs": (i32, [vp, vp, i64, vp, ctypes.c_uint32, vp, sz, vp, vp]),
+        "zen_host_words_alloc": (i32, [i64, ctypes.POINTER(vp)]),
+        "zen_host_words_free": (i32, [vp]),
+        "zen_read_back": (i32, [vp, i32, i32, vp, i32, i32, vp, i32, i32, vp, i64, vp]),
+        "zen_count": (i32, [vp, i32, i64, vp, vp, vp]),
         "zen_stream_read": (i32, [vp, sz, vp, vp]),
         "zen_profile_enable": (i32, [i32]),
         "zen_profile_only": (i32, [i32]),
@@ -264,6 +269,40 @@ zeros = ZeroPool()
 
 def status_word(device):
     return zeros.take(device, 1, torch.int32)
+
+
+class _HostWords:
+    """Pinned host words of one host thread (zen_read_back stores into them); they go when the thread does."""
+
+    def __init__(self, words):
+        self.words = words
+        pinned = ctypes.c_void_p()
+        check(lib().zen_host_words_alloc(words, ctypes.byref(pinned)), "host_words")
+        self.ptr = pinned.value
+        self.view = (ctypes.c_int64 * words).from_address(self.ptr)
+
+    def __del__(self):
+        if not sys.is_finalizing() and getattr(self, "ptr", None):
+            _lib.zen_host_words_free(self.ptr)
+
+
+_host = threading.local()
+
+
+def read_back(*tensors):
+    """The values of up to three small contiguous int32 / int64 device tensors (split sizes, counts, status
+    words), one list after the other, once the current stream has got there.  The way a call on this path
+    waits for the device: one kernel instead of a conversion, a concatenation and a copy."""
+    n = sum(t.numel() for t in tensors)
+    words = getattr(_host, "words", None)
+    if words is None or words.words <= n:
+        words = _host.words = _HostWords(max(1024, 2 * n))
+    args = []
+    for t in tensors:
+        args += (t.data_ptr(), t.numel(), 1 if t.dtype == torch.int64 else 0)
+    args += (None, 0, 0) * (3 - len(tensors))
+    check(lib().zen_read_back(*args, words.ptr, words.words, stream_handle(tensors[0].device)), "read_back")
+    return words.view[1:n + 1]
 
 
 def describe_status(bits):

@@ -39,14 +39,14 @@ def _select_raw(tensor, thr, idx64, capacity=None):
     code = _lib.dtype_code(flat)
     out_idx = torch.empty(capacity, dtype=torch.int64 if idx64 else torch.int32, device=dev)
     out_val = torch.empty(capacity, dtype=flat.dtype, device=dev)
-    count = torch.zeros(1, dtype=torch.int64, device=dev)
+    count = _lib.zeros.take(dev, 1, torch.int64)
     status = _lib.status_word(dev)
     ws = _lib.scratch.get(dev, "select", L.zen_select_workspace(n, code))
     rc = L.zen_select(_lib.ptr(flat), code, n, _lib.ptr(thr), _lib.ptr(out_idx), 1 if idx64 else 0,
                       _lib.ptr(out_val), capacity, _lib.ptr(count), _lib.ptr(ws), ws.numel(),
                       _lib.ptr(status), _lib.stream_of(dev))
     _lib.check(rc, "select")
-    host = torch.cat([count, status.to(torch.int64)]).tolist()
+    host = _lib.read_back(count, status)
     kept = min(host[0], capacity)
     return out_idx[:kept], out_val[:kept], host[0], host[1]
 
@@ -121,7 +121,7 @@ class LoadBalanceAllreduce:
                                            alltoall_dense_size, _lib.ptr(ws), ws.numel(), _lib.ptr(status),
                                            _lib.stream_of(dev))
             _lib.check(rc, "decode_sparse_tensors")
-            if not int(status.item()):  # the reference's scatter_add_ raises on a bad index, also a sync
+            if not _lib.read_back(status)[0]:  # the reference's scatter_add_ raises on a bad index, also a sync
                 return dense
         ws = _lib.scratch.get(dev, "decode", L.zen_decode_dense_workspace(r, alltoall_dense_size))
         for mode in self._fast_then_general():
@@ -130,7 +130,7 @@ class LoadBalanceAllreduce:
                                     _lib.dtype_code(values), r, _lib.ptr(dense), alltoall_dense_size, mode,
                                     _lib.ptr(ws), ws.numel(), _lib.ptr(status), _lib.stream_of(dev))
             _lib.check(rc, "decode_sparse_tensors")
-            bits = int(status.item())  # the reference's scatter_add_ raises on a bad index, also a sync
+            bits = _lib.read_back(status)[0]  # the reference's scatter_add_ raises on a bad index, also a sync
             if not bits & _lib.STAT_RETRY:
                 break
         if bits:
@@ -303,7 +303,7 @@ class LoadBalanceAllreduce:
             idx, val, count, status = self.merge_sparse_flat(indices_tensors, values_tensors, dense_size,
                                                              idx64=True, mode=mode)
             r_idx, r_val, kept, r_status = self.round_merged_flat(idx, val, count, dtype)
-            host = torch.cat([kept, status.to(torch.int64), r_status.to(torch.int64)]).tolist()
+            host = _lib.read_back(kept, status, r_status)
             if host[1] & (_lib.STAT_RETRY | _lib.STAT_INTERNAL):
                 self.reset_merge_workspace(idx.device)
             if not host[1] & _lib.STAT_RETRY:
@@ -324,7 +324,7 @@ class LoadBalanceAllreduce:
         for mode in self._fast_then_general():
             idx, val, count, status = self.merge_sparse_flat(indices_tensors, values_tensors, dense_size,
                                                              idx64=True, mode=mode)
-            host = torch.cat([count, status.to(torch.int64)]).tolist()
+            host = _lib.read_back(count, status)
             if host[1] & (_lib.STAT_RETRY | _lib.STAT_INTERNAL):
                 self.reset_merge_workspace(idx.device)
             if not host[1] & _lib.STAT_RETRY:
@@ -340,15 +340,16 @@ class LoadBalanceAllreduce:
         L = _lib.lib()
         dev = torch.device("cuda", self.device)
         out = torch.empty(numel, dtype=torch.int64, device=dev)
-        counts = torch.zeros(self.partitions, dtype=torch.int64, device=dev)
+        counts = _lib.zeros.take(dev, self.partitions, torch.int64)
         ws = _lib.scratch.get(dev, "mapping", L.zen_mapping_workspace(numel, self.partitions))
         status = _lib.status_word(dev)
         rc = L.zen_mapping(numel, self.partitions, _lib.ptr(out), _lib.ptr(counts), _lib.ptr(ws), ws.numel(),
                            _lib.ptr(status), _lib.stream_of(dev))
         _lib.check(rc, "calculate_mapping")
-        sizes = torch.cat([counts, status.to(torch.int64)]).tolist()
-        if sizes.pop():
-            raise RuntimeError("calculate_mapping: " + _lib.describe_status(int(status.item())))
+        sizes = _lib.read_back(counts, status)
+        bits = sizes.pop()
+        if bits:
+            raise RuntimeError("calculate_mapping: " + _lib.describe_status(bits))
         mapping, at = [], 0
         for c in sizes:
             mapping.append(out[at:at + c])
@@ -389,7 +390,7 @@ class LoadBalanceAllreduce:
         is among sparse_indices; least significant bit first, padded to a whole
         byte (comm.py:59-85).  self.mapping[numel] must exist (comm.py:135)."""
         bitmap, status = self.encode_bitmap_flat(sparse_indices, numel)
-        bits = int(status.item())
+        bits = _lib.read_back(status)[0]
         if bits & _lib.STAT_BAD_INDEX:  # result[indices] = 1 with an index == len(result), comm.py:63
             raise IndexError("encode_bitmap: an index lies beyond the last member of the mapping")
         if bits:
@@ -401,7 +402,7 @@ class LoadBalanceAllreduce:
         bitmap_indices[i], ascending int64 (comm.py:87-99)."""
         mapping_tensor = self.mapping[numel]
         L = _lib.lib()
-        outs, counts = [], []
+        outs = []
         status = None
         for i, bitmap_tensor in enumerate(bitmap_indices):
             mapping = mapping_tensor[i]
@@ -414,20 +415,20 @@ class LoadBalanceAllreduce:
                 raise IndexError("decode_bitmap: bitmap shorter than the mapping")
             if status is None:
                 status = _lib.status_word(dev)
+                counts = _lib.zeros.take(dev, len(bitmap_indices), torch.int64)
             # a set bit costs eight bytes of output: room for every bit that can be set
             capacity = min(members, bitmap_tensor.numel() * 8)
             out = torch.empty(capacity, dtype=torch.int64, device=dev)
-            count = torch.zeros(1, dtype=torch.int64, device=dev)
+            count = counts[i:i + 1]
             ws = _lib.scratch.get(dev, "bitmap", L.zen_bitmap_decode_workspace(members))
             rc = L.zen_bitmap_decode(_lib.ptr(mapping), members, _lib.ptr(bitmap_tensor), bitmap_tensor.numel(),
                                      _lib.ptr(out), capacity, _lib.ptr(count), _lib.ptr(ws), ws.numel(),
                                      _lib.ptr(status), _lib.stream_of(dev))
             _lib.check(rc, "decode_bitmap")
             outs.append(out)
-            counts.append(count)
         if not outs:
             return []
-        host = torch.cat(counts + [status.to(torch.int64)]).tolist()
+        host = _lib.read_back(counts, status)
         if host[-1]:
             raise RuntimeError("decode_bitmap: " + _lib.describe_status(host[-1]))
         return [out[:c] for out, c in zip(outs, host)]
@@ -472,7 +473,7 @@ class LoadBalanceAllreduce:
                                 _lib.dtype_code(values), v_start, _lib.ptr(dense), _lib.ptr(ws), ws.numel(),
                                 _lib.ptr(status), _lib.stream_of(dev))
         _lib.check(rc, "decode_bitmaps_dense")
-        bits = int(status.item())  # the reference's masking and scatter_add_ raise on a mismatch, also a sync
+        bits = _lib.read_back(status)[0]  # the reference's masking and scatter_add_ raise on a mismatch, also a sync
         if bits & _lib.STAT_BAD_INDEX:
             raise IndexError("decode_bitmaps_dense: a bitmap is shorter than its partition's index list, or has "
                              "more set bits than values came with it")

@@ -58,7 +58,7 @@ class _PendingStatus:
         self.offsets = offsets
 
     def check(self):
-        bits = int(self.status.item())
+        bits = _lib.read_back(self.status)[0]
         if bits:
             raise RuntimeError("sparse_balance: " + _lib.describe_status(bits))
 

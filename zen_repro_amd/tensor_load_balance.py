@@ -119,10 +119,16 @@ class TensorPartition:
         if thr is not None:
             # thr[1] counts the multiset the threshold was computed on, which may be a sample of the tensor
             # (compress): count what passes it in the tensor itself
-            from .comm import _select_raw
+            return self._count(flat, thr) + 1024
+        return self._count(flat, None) + 1024
 
-            return _select_raw(flat, thr, False, 0)[2] + 1024
-        return int(torch.count_nonzero(flat)) + 1024
+    @staticmethod
+    def _count(flat, thr):
+        _lib.require_gpu(flat, "input")
+        count = _lib.zeros.take(flat.device, 1, torch.int64)
+        _lib.check(_lib.lib().zen_count(_lib.ptr(flat), _lib.dtype_code(flat), flat.numel(), _lib.ptr(thr),
+                                        _lib.ptr(count), _lib.stream_of(flat.device)), "count")
+        return _lib.read_back(count)[0]
 
     def _ahead_state(self, device, slot, create=False):
         # "free": per set of sampling memory, the mark behind the last call that used it; "pending": samples
@@ -341,7 +347,7 @@ class TensorPartition:
         modes = list(every)
         while modes:
             out_idx, out_val, splits, status = self.load_balance_flat(tensor, thr, capacity, k, modes[0])
-            host = torch.cat([splits, status.to(torch.int64)]).tolist()
+            host = _lib.read_back(splits, status)
             bits = host[-1]
             if bits & (_lib.STAT_RETRY | _lib.STAT_INTERNAL):
                 # a declined or aborted call may leave entries and counters behind in the table
@@ -358,9 +364,6 @@ class TensorPartition:
                 break
         if bits:
             raise RuntimeError("load_balance: " + _lib.describe_status(bits))
-        indices, values, at = [], [], 0
-        for p in range(self.partitions):
-            indices.append(out_idx[at:at + host[p]])
-            values.append(out_val[at:at + host[p]])
-            at += host[p]
-        return indices, values, splits
+        sizes = host[:-1]
+        total = sum(sizes)
+        return list(torch.split(out_idx[:total], sizes)), list(torch.split(out_val[:total], sizes)), splits
