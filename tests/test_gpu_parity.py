@@ -812,3 +812,25 @@ def test_round_merged_sums(zen, oracle, dtype, idx64, count):
     nan = torch.isnan(want)
     assert torch.equal(torch.isnan(got), nan)  # a NaN stays a NaN (which of the NaN patterns is the converter's business)
     assert torch.equal(got[~nan].view(bits), want[~nan].view(bits))
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("s", [1, 1023, 8192, 8193, 16384, 16385, 4096 * 15 + 1, 4096 * 256 + 77])
+@pytest.mark.parametrize("kind", ["normal", "sparse", "constant"])
+def test_sample_threshold_at_the_edges_of_its_kernels(zen, oracle, s, dtype, kind):
+    """One workgroup (up to 8192 positions of bf16, 16384 of fp32), a few, all of them; a sample nearly all of which is zero and one whose
+    elements are all equal, so that one histogram bin takes everything.  Keys and counts are whole numbers: exact."""
+    import importlib
+
+    C = importlib.import_module("zen_repro_amd.compress")
+    n = 70001
+    g = make_grad(oracle, n, 0.02 if kind == "sparse" else 1.0, dtype, seed=s)
+    if kind == "constant":
+        g[:] = g[5]
+    at = np.random.default_rng(s).integers(0, n, s)
+    keys = ((g & 0x7FFF) if dtype == "bf16" else (g.view(np.uint32) & 0x7FFFFFFF))[at]
+    order = np.sort(keys)[::-1]
+    for k in sorted({1, max(1, s // 100), max(1, s // 2), s}):
+        thr, status = C.sample_threshold(to_dev(g), torch.from_numpy(at).cuda(), k)
+        key, count = (int(x) & 0xFFFFFFFF for x in to_np(thr))
+        assert int(status) == 0 and key == int(order[k - 1]) and count == int((keys >= key).sum()), (k, kind)

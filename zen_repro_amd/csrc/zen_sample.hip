@@ -1,0 +1,448 @@
+// The threshold compress() applies (train.py:75-84): the k-th largest magnitude of a gathered sample.
+//
+// The sample is 1 % of a gradient bucket, at random places: what the call cannot do without is one memory line
+// per sample element.  A radix select behind a gather took 6 to 8 dependent launches, each a few microseconds of
+// work; here the histogram is taken while the elements arrive, at 15 bits of the magnitude (for bf16 the whole
+// key), so that one more workgroup finds the k-th:
+//   up to one_max() elements  one workgroup does everything in one launch, 16 elements per thread in registers;
+//   more, bf16                k_sample_count (every workgroup keeps 32768 16-bit counters in LDS and writes them
+//                             out, with sums of 64 neighbours each: nothing has to be zero beforehand and no
+//                             atomic leaves the compute unit), k_sample_pick (one workgroup);
+//   more, fp32                the elements are kept too; a third kernel lists the low halves of those in the
+//                             k-th's bin and its last workgroup picks among them.
+#include "zen_select.h"
+
+namespace zen {
+namespace {
+
+constexpr int kBins = 32768;       // 15 bits of the magnitude key
+constexpr int kBlock = 1024;
+// One workgroup as long as it takes no longer than the two (bf16) or three (fp32) launches for larger samples:
+// its counting loop costs 1.3 us per 1024 elements (10 486 fp32: 16 us, 30 000 bf16: 41 us).
+constexpr int kOneItems = 16;
+template <typename S>
+constexpr int64_t one_max() { return (sizeof(S) == 2 ? kOneItems / 2 : kOneItems) * kBlock; }
+constexpr int kGroup = 64;         // bins per sum
+constexpr int kGroups = kBins / kGroup;
+constexpr int kRound = 4;          // elements per thread in flight in the counting kernel
+constexpr int64_t kShare = 65535;  // elements a workgroup counts at most (16-bit counters)
+// the bins' 16-bit counters, two to a word, one word of padding per 32 (a thread reads 16 neighbouring words)
+constexpr int kHistWords = kBins / 2 + kBins / 64;
+__device__ inline int hist_word(int w) { return w + (w >> 5); }
+
+// Adds one to the counter of every lane's bin (lanes without `live` add nothing).  The lanes that share the
+// first live lane's bin add together: in a mostly zero gradient nearly every element meets in one bin, and a
+// wave's adds to one address are carried out one after the other.
+__device__ inline void count_bin(uint32_t *hist, uint32_t bin, bool live) {
+  const uint64_t all = __ballot(live);
+  if (!all) return;
+  const int lead = __ffsll((unsigned long long)all) - 1;
+  const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)bin, lead);
+  const uint64_t same = __ballot(live && bin == first);
+  const bool with_first = live && bin == first;
+  const uint32_t n = with_first ? (uint32_t)__popcll(same) : 1u;
+  if (live && (!with_first || lane_id() == lead)) atomicAdd(&hist[hist_word((int)(bin >> 1))], n << (16 * (bin & 1u)));
+}
+
+struct Pick {
+  uint32_t bin, above, count;  // the bin that holds the rank-th largest, elements in the bins above it and in it
+};
+
+// The bin of the histogram in LDS that holds the rank-th largest (1 <= rank <= elements counted).  By the whole
+// workgroup; smem: kBlock / 64 + 1 words; *out is valid behind the barrier at the end.
+__device__ inline void pick_bin(const uint32_t *hist, uint32_t rank, uint32_t *smem, Pick *out) {
+  constexpr int kWords = kBins / 2 / kBlock;
+  uint32_t c[kWords];
+  uint32_t mine = 0;
+#pragma unroll
+  for (int j = 0; j < kWords; ++j) {  // from the top down
+    c[j] = hist[hist_word(kBins / 2 - 1 - (int)(threadIdx.x * kWords + j))];
+    mine += (c[j] & 0xffffu) + (c[j] >> 16);
+  }
+  uint32_t total;
+  uint32_t above = block_exclusive_scan<uint32_t, kBlock>(mine, smem, &total);
+  if (above < rank && rank <= above + mine) {
+#pragma unroll
+    for (int j = 0; j < kWords; ++j) {
+#pragma unroll
+      for (int h = 1; h >= 0; --h) {
+        const uint32_t n = h ? c[j] >> 16 : c[j] & 0xffffu;
+        if (above < rank && rank <= above + n) {
+          out->bin = 2u * (uint32_t)(kBins / 2 - 1 - (int)(threadIdx.x * kWords + j)) + (uint32_t)h;
+          out->above = above;
+          out->count = n;
+        }
+        above += n;
+      }
+    }
+  }
+  __syncthreads();
+}
+
+__device__ inline void clear_hist(uint32_t *hist) {
+  for (int i = threadIdx.x; i < kHistWords; i += kBlock) hist[i] = 0;
+}
+
+// Positions at[first + i * kBlock], i < ITEMS, of the sample (those at or past `end` and those outside the tensor
+// read element 0 as zero; the latter are flagged): all loads of a round in flight together.
+template <typename S, int ITEMS>
+__device__ inline void gather(const S *__restrict__ in, int64_t n, const int64_t *__restrict__ at, int64_t first,
+                              int64_t end, S (&v)[ITEMS], int32_t *status) {
+  int64_t pos[ITEMS];
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const int64_t j = first + (int64_t)i * kBlock;
+    pos[i] = __builtin_nontemporal_load(at + (j < end ? j : end - 1));
+    if (pos[i] < 0 || pos[i] >= n) {
+      bad = true;
+      pos[i] = -1;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) v[i] = in[pos[i] >= 0 ? pos[i] : 0];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i)
+    if (pos[i] < 0) v[i] = 0;
+  if (bad) atomicOr(status, ZEN_STAT_BAD_INDEX);
+}
+
+// Everything in one workgroup.  Bound by the chain gather - histogram - search: 5 us for 93 bf16 elements (six
+// launches before: 26 us a call, now 12).
+template <typename S>
+__global__ __launch_bounds__(kBlock) void k_sample_one(const S *__restrict__ in, int64_t n,
+                                                       const int64_t *__restrict__ at, uint32_t s, uint32_t k,
+                                                       uint32_t *__restrict__ thr, int32_t *status) {
+  __shared__ uint32_t hist[kHistWords];
+  __shared__ uint32_t smem[kBlock / 64 + 1];
+  __shared__ Pick pick;
+  __shared__ uint32_t low[2];
+  clear_hist(hist);
+  if (threadIdx.x < 2) low[threadIdx.x] = 0;
+  S v[kOneItems];
+#pragma unroll
+  for (int r = 0; r < kOneItems; r += 8) {  // (a gather of eight at a time)
+    S part[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) part[i] = 0;
+    if ((uint32_t)r * kBlock < s) gather<S, 8>(in, n, at, (int64_t)threadIdx.x + (int64_t)r * kBlock, s, part, status);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[r + i] = part[i] & (S)KeyOf<S>::kMask;
+  }
+  __syncthreads();
+  constexpr int kShift = KeyOf<S>::kBits - 15;
+#pragma unroll
+  for (int i = 0; i < kOneItems; ++i) {
+    if ((uint32_t)i * kBlock >= s) break;
+    count_bin(hist, (uint32_t)v[i] >> kShift, threadIdx.x + (uint32_t)i * kBlock < s);
+  }
+  __syncthreads();
+  pick_bin(hist, k, smem, &pick);
+  const uint32_t top = pick.bin;
+  if (sizeof(S) == 2) {
+    if (threadIdx.x == 0) {
+      thr[0] = top;
+      thr[1] = pick.above + pick.count;
+    }
+    return;
+  }
+  // fp32: 15 of the 16 bits that are left, then the last
+  const uint32_t above = pick.above;
+  __syncthreads();
+  clear_hist(hist);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kOneItems; ++i) {
+    if ((uint32_t)i * kBlock >= s) break;
+    const uint32_t key = (uint32_t)v[i];
+    count_bin(hist, (key & 0xffffu) >> 1, threadIdx.x + (uint32_t)i * kBlock < s && (key >> 16) == top);
+  }
+  __syncthreads();
+  pick_bin(hist, k - above, smem, &pick);
+  const uint32_t high = (top << 15) | pick.bin;
+#pragma unroll
+  for (int i = 0; i < kOneItems; ++i) {
+    if ((uint32_t)i * kBlock >= s) break;
+    const uint32_t key = (uint32_t)v[i];
+    const bool live = threadIdx.x + (uint32_t)i * kBlock < s && (key >> 1) == high;
+    const uint64_t odd = __ballot(live && (key & 1u)), all = __ballot(live);
+    if (all && lane_id() == 0) {
+      atomicAdd(&low[1], (uint32_t)__popcll(odd));
+      atomicAdd(&low[0], (uint32_t)__popcll(all & ~odd));
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t over = above + pick.above, odd = low[1];
+    const uint32_t bit = over + odd >= k ? 1u : 0u;
+    thr[0] = (high << 1) | bit;
+    thr[1] = over + odd + (bit ? 0u : low[0]);
+  }
+}
+
+struct SampleTables {
+  uint16_t *sums;    // [workgroups][kGroups] per workgroup: elements in 64 neighbouring bins
+  uint16_t *bins;    // [workgroups][kBins]
+  uint32_t *sample;  // fp32: the magnitude keys
+  uint16_t *members; // fp32: low halves of the keys in the k-th's bin
+  uint32_t *state;   // fp32: [0] bin, [1] rank inside it, [2] elements above it, [3] members listed, [4] workgroups done
+};
+
+// Bound by the sample's lines: 2.7 M elements of a 537 MB tensor at random places are 344 MB of them, 62 us.  A
+// call took 108 us with the gather kernel and four passes behind it, now 73.
+template <typename S>
+__global__ __launch_bounds__(kBlock) void k_sample_count(const S *__restrict__ in, int64_t n,
+                                                         const int64_t *__restrict__ at, int64_t s, int64_t share,
+                                                         SampleTables tb, int32_t *status) {
+  __shared__ uint32_t hist[kHistWords];
+  constexpr int kShift = KeyOf<S>::kBits - 15;
+  clear_hist(hist);
+  __syncthreads();
+  const int64_t begin = (int64_t)blockIdx.x * share;
+  const int64_t end = begin + share < s ? begin + share : s;
+  for (int64_t j0 = begin; j0 < end; j0 += (int64_t)kRound * kBlock) {
+    S v[kRound];
+    gather<S, kRound>(in, n, at, j0 + threadIdx.x, end, v, status);
+#pragma unroll
+    for (int i = 0; i < kRound; ++i) {
+      const int64_t j = j0 + threadIdx.x + (int64_t)i * kBlock;
+      const uint32_t key = v[i] & KeyOf<S>::kMask;
+      count_bin(hist, key >> kShift, j < end);
+      if (sizeof(S) == 4 && j < end) tb.sample[j] = key;
+    }
+  }
+  __syncthreads();
+  // thread t: 16 words = 32 bins, half a group
+  uint32_t w[16];
+  uint32_t sum = 0;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    w[j] = hist[hist_word((int)threadIdx.x * 16 + j)];
+    sum += (w[j] & 0xffffu) + (w[j] >> 16);
+  }
+  uint4 *bins = reinterpret_cast<uint4 *>(tb.bins + (size_t)blockIdx.x * kBins);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) bins[threadIdx.x * 4 + j] = make_uint4(w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]);
+  sum += __shfl_xor(sum, 1, 64);
+  if ((threadIdx.x & 1u) == 0) tb.sums[(size_t)blockIdx.x * kGroups + threadIdx.x / 2] = (uint16_t)sum;
+}
+
+// Sums of 16-bit counters over the workgroups of the counting kernel: `words` columns of four counters, read by
+// kBlock / COLUMNS rows of threads side by side.  acc: [4 * COLUMNS] words of LDS, zeroed here.
+template <int COLUMNS>
+__device__ inline void sum_columns(const uint16_t *from, size_t stride, uint32_t rows, uint32_t *acc) {
+  if (threadIdx.x < 4 * COLUMNS) acc[threadIdx.x] = 0;
+  __syncthreads();
+  const uint32_t col = threadIdx.x % COLUMNS, row = threadIdx.x / COLUMNS;
+  constexpr uint32_t kRows = kBlock / COLUMNS;
+  uint32_t c[4] = {0, 0, 0, 0};
+#pragma unroll 8
+  for (uint32_t r = row; r < rows; r += kRows) {
+    const uint2 q = *reinterpret_cast<const uint2 *>(from + (size_t)r * stride + col * 4);
+    c[0] += q.x & 0xffffu;
+    c[1] += q.x >> 16;
+    c[2] += q.y & 0xffffu;
+    c[3] += q.y >> 16;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) atomicAdd(&acc[col * 4 + e], c[e]);
+  __syncthreads();
+}
+
+template <typename S>
+__global__ __launch_bounds__(kBlock) void k_sample_pick(SampleTables tb, uint32_t rows, uint32_t k,
+                                                        uint32_t *__restrict__ thr) {
+  __shared__ uint32_t acc[kGroups];
+  __shared__ uint32_t smem[kBlock / 64 + 1];
+  __shared__ uint32_t found[3];
+  sum_columns<kGroups / 4>(tb.sums, kGroups, rows, acc);
+  {
+    const uint32_t c = threadIdx.x < kGroups ? acc[kGroups - 1 - threadIdx.x] : 0u;
+    uint32_t total;
+    const uint32_t above = block_exclusive_scan<uint32_t, kBlock>(c, smem, &total);
+    if (above < k && k <= above + c) {
+      found[0] = (uint32_t)(kGroups - 1) - threadIdx.x;
+      found[1] = above;
+    }
+  }
+  __syncthreads();
+  const uint32_t group = found[0], over = found[1];
+  sum_columns<kGroup / 4>(tb.bins + (size_t)group * kGroup, kBins, rows, acc);
+  {
+    const uint32_t c = threadIdx.x < kGroup ? acc[kGroup - 1 - threadIdx.x] : 0u;
+    uint32_t total;
+    const uint32_t above = over + block_exclusive_scan<uint32_t, kBlock>(c, smem, &total);
+    if (above < k && k <= above + c) {
+      const uint32_t bin = group * kGroup + (kGroup - 1u - threadIdx.x);
+      if (sizeof(S) == 2) {
+        thr[0] = bin;
+        thr[1] = above + c;
+      } else {
+        tb.state[0] = bin;
+        tb.state[1] = k - above;
+        tb.state[2] = above;
+      }
+    }
+  }
+  if (sizeof(S) == 4 && threadIdx.x < 2) tb.state[3 + threadIdx.x] = 0;
+}
+
+// fp32: the low halves of the keys in the k-th's bin (a few thousand of millions) are listed by all workgroups;
+// the last one finds the k-th among them, eight bits at a time.
+constexpr int kMemberItems = 8;
+__global__ __launch_bounds__(kBlock) void k_sample_members(SampleTables tb, int64_t s, uint32_t *__restrict__ thr) {
+  __shared__ uint16_t mine[kBlock * kMemberItems];
+  __shared__ uint32_t n_mine, base;
+  __shared__ bool last;
+  const uint32_t top = tb.state[0];
+  for (int64_t j0 = (int64_t)blockIdx.x * kBlock * kMemberItems; j0 < s; j0 += (int64_t)gridDim.x * kBlock * kMemberItems) {
+    if (threadIdx.x == 0) n_mine = 0;
+    __syncthreads();
+    uint32_t key[kMemberItems];
+#pragma unroll
+    for (int i = 0; i < kMemberItems; ++i) {
+      const int64_t j = j0 + threadIdx.x + (int64_t)i * kBlock;
+      key[i] = j < s ? tb.sample[j] : 0xffffffffu;
+    }
+#pragma unroll
+    for (int i = 0; i < kMemberItems; ++i)
+      if ((key[i] >> 16) == top) mine[atomicAdd(&n_mine, 1u)] = (uint16_t)key[i];
+    __syncthreads();
+    if (threadIdx.x == 0 && n_mine) base = atomicAdd(&tb.state[3], n_mine);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n_mine; i += kBlock)
+      __hip_atomic_store(&tb.members[base + i], mine[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+  }
+  wait_global_acks();
+  __syncthreads();
+  if (threadIdx.x == 0) last = atomicAdd(&tb.state[4], 1u) == gridDim.x - 1u;
+  __syncthreads();
+  if (!last) return;
+  __shared__ uint32_t hist[256];
+  __shared__ uint32_t smem[kBlock / 64 + 1];
+  __shared__ uint32_t found[3];
+  const uint32_t m = load_fresh(&tb.state[3]);
+  uint32_t rank = tb.state[1], above = tb.state[2], prefix = 0;
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+    if (threadIdx.x < 256) hist[threadIdx.x] = 0;
+    __syncthreads();
+    const uint32_t rounds = (m + kBlock - 1) / kBlock;
+    for (uint32_t r = 0; r < rounds; ++r) {
+      const uint32_t j = r * kBlock + threadIdx.x;
+      const uint32_t x = j < m ? __hip_atomic_load(&tb.members[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+      const bool live = j < m && (pass == 0 || (x >> 8) == prefix);
+      const uint32_t digit = pass == 0 ? x >> 8 : x & 0xffu;
+      const uint64_t all = __ballot(live);  // equal digits add together where they are all equal (see count_bin)
+      if (all) {
+        const int lead = __ffsll((unsigned long long)all) - 1;
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)digit, lead);
+        if (__ballot(live && digit == first) == all) {
+          if (lane_id() == lead) atomicAdd(&hist[first], (uint32_t)__popcll(all));
+        } else if (live) {
+          atomicAdd(&hist[digit], 1u);
+        }
+      }
+    }
+    __syncthreads();
+    const uint32_t c = threadIdx.x < 256 ? hist[255 - threadIdx.x] : 0u;
+    uint32_t total;
+    const uint32_t before = block_exclusive_scan<uint32_t, kBlock>(c, smem, &total);
+    if (before < rank && rank <= before + c) {
+      found[0] = 255u - threadIdx.x;
+      found[1] = before;
+      found[2] = c;
+    }
+    __syncthreads();
+    prefix = (prefix << 8) | found[0];
+    rank -= found[1];
+    above += found[1];
+  }
+  if (threadIdx.x == 0) {
+    thr[0] = (top << 16) | prefix;
+    thr[1] = above + found[2];
+  }
+}
+
+// Workgroups of the counting kernel for a sample of s elements: a round each at least, one per compute unit at
+// most (the picking kernel reads a row per workgroup), unless a share outgrew the counters.
+inline int64_t sample_groups(int64_t s) {
+  int64_t g = ceil_div(s, (int64_t)kRound * kBlock);
+  if (g > 256) g = 256;
+  const int64_t least = ceil_div(s, kShare);
+  return g < least ? least : g;
+}
+
+SampleTables plan_sample(void *workspace, int64_t s, int dtype, size_t *bytes) {
+  Carver cv(workspace);
+  SampleTables tb{};
+  if (s > (dtype == ZEN_BF16 ? one_max<uint16_t>() : one_max<uint32_t>())) {
+    const size_t g = (size_t)sample_groups(s);
+    tb.state = cv.take<uint32_t>(8);
+    tb.sums = cv.take<uint16_t>(g * kGroups);
+    tb.bins = cv.take<uint16_t>(g * kBins);
+    if (dtype == ZEN_F32) {
+      tb.sample = cv.take<uint32_t>((size_t)s);
+      tb.members = cv.take<uint16_t>((size_t)s);
+    }
+  }
+  *bytes = cv.used;
+  return tb;
+}
+
+template <typename S>
+int sample_threshold_launch(const S *in, int64_t n, const int64_t *at, int64_t s, int64_t k, uint32_t *thr,
+                            void *workspace, int32_t *status, hipStream_t stream) {
+  if (s <= one_max<S>()) {
+    k_sample_one<S><<<dim3(1), dim3(kBlock), 0, stream>>>(in, n, at, (uint32_t)s, (uint32_t)k, thr, status);
+    ZEN_LAUNCH_CHECK("k_sample_one");
+    return ZEN_OK;
+  }
+  size_t bytes;
+  const SampleTables tb = plan_sample(workspace, s, sizeof(S) == 2 ? ZEN_BF16 : ZEN_F32, &bytes);
+  const int64_t groups = sample_groups(s);
+  const int64_t share = ceil_div(s, groups);
+  const int64_t rows = ceil_div(s, share);
+  k_sample_count<S><<<dim3((unsigned)rows), dim3(kBlock), 0, stream>>>(in, n, at, s, share, tb, status);
+  ZEN_LAUNCH_CHECK("k_sample_count");
+  k_sample_pick<S><<<dim3(1), dim3(kBlock), 0, stream>>>(tb, (uint32_t)rows, (uint32_t)k, thr);
+  ZEN_LAUNCH_CHECK("k_sample_pick");
+  if (sizeof(S) == 4) {
+    int64_t blocks = ceil_div(s, (int64_t)kBlock * kMemberItems);
+    if (blocks > 256) blocks = 256;
+    k_sample_members<<<dim3((unsigned)blocks), dim3(kBlock), 0, stream>>>(tb, s, thr);
+    ZEN_LAUNCH_CHECK("k_sample_members");
+  }
+  return ZEN_OK;
+}
+
+}  // namespace
+}  // namespace zen
+
+extern "C" {
+
+size_t zen_sample_threshold_workspace(int64_t s, int dtype) {
+  if (s < 0) return 0;
+  size_t bytes;
+  (void)zen::plan_sample(nullptr, s, dtype, &bytes);
+  return bytes > 256 ? bytes : 256;
+}
+
+int zen_sample_threshold(const void *input, int dtype, int64_t n, const int64_t *sample_index, int64_t s, int64_t k,
+                         uint32_t *thr, void *workspace, size_t workspace_bytes, int32_t *status, void *stream) {
+  using namespace zen;
+  if (!input || !sample_index || !thr || !workspace || !status) return fail(ZEN_EINVAL, "zen_sample_threshold: null pointer");
+  if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_sample_threshold: bad dtype");
+  if (n <= 0 || s <= 0 || s > 0x7fffffffll || k < 1 || k > s)
+    return fail(ZEN_EINVAL, "zen_sample_threshold: need n > 0 and 1 <= k <= s < 2^31");
+  if (workspace_bytes < zen_sample_threshold_workspace(s, dtype))
+    return fail(ZEN_EWORKSPACE, "zen_sample_threshold: workspace too small");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t *at = sample_index;
+  if (dtype == ZEN_BF16)
+    return sample_threshold_launch(static_cast<const uint16_t *>(input), n, at, s, k, thr, workspace, status, st);
+  return sample_threshold_launch(static_cast<const uint32_t *>(input), n, at, s, k, thr, workspace, status, st);
+}
+
+}  // extern "C"
