@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define ZEN_ABI_VERSION 4 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table; 4: zen_read_back, zen_count */
+#define ZEN_ABI_VERSION 4 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table; 4: zen_read_back, zen_count, zen_merge_rounded, zen_decode_dense_lists, zen_bitmap_dense_lists */
 
 #define ZEN_F32 0
 #define ZEN_BF16 1
@@ -314,6 +314,17 @@ int zen_merge(const void *idx, int idx64_in, const void *val, int dtype,
               int32_t *status, void *stream);
 
 /*
+ * zen_merge with every sum rounded once to the values' type `dtype` and the entries whose sum rounds to zero
+ * dropped: what comm.py:125-127 hands to the second exchange, in one call (zen_merge followed by
+ * zen_round_compact gives the same).  out_val: `dtype`.
+ */
+int zen_merge_rounded(const void *idx, int idx64_in, const void *val, int dtype,
+                      int64_t r, int64_t dense_n,
+                      void *out_idx, int idx64_out, void *out_val, int64_t capacity,
+                      int64_t *out_count, int mode, void *workspace, size_t workspace_bytes,
+                      int32_t *status, void *stream);
+
+/*
  * The merged entries on their way to the second exchange: comm.py:125-127
  * scatters the sums into a dense tensor of the gradient's type and takes its
  * nonzeros again; here every fp32 sum of zen_merge's output is rounded once to
@@ -397,6 +408,8 @@ int zen_encode_merge(const zen_encode_merge_args *args);
  * dense[0..dense_n) = 0, then dense[idx[j]] += val[j] with fp32 accumulation
  * in entry order, rounded once to `dtype`.  Replaces decode_sparse_tensors
  * (comm.py:32-44), whose result is a dense tensor in the value dtype.
+ * `mode` as for zen_merge; with ZEN_MODE_ZEROED the head of this call's
+ * workspace (zen_merge_zero_bytes()) is zero and stays so.
  */
 size_t zen_decode_dense_workspace(int64_t r, int64_t dense_n);
 int zen_decode_dense(const void *idx, int idx64_in, const void *val, int dtype,
@@ -415,6 +428,11 @@ int zen_decode_dense(const void *idx, int idx64_in, const void *val, int dtype,
  * is then unspecified and the caller repeats with zen_decode_dense.
  */
 size_t zen_decode_dense_sorted_workspace(int64_t dense_n, int nlists);
+/* The same for lists that sit anywhere (an all-gather ends in one buffer per rank): idx[l], val[l] and len[l] in
+   HOST arrays of nlists entries. */
+int zen_decode_dense_lists(const void *const *idx, int idx64_in, const void *const *val, int dtype,
+                           const int64_t *len, int nlists, void *dense, int64_t dense_n,
+                           void *workspace, size_t workspace_bytes, int32_t *status, void *stream);
 int zen_decode_dense_sorted(const void *idx, int idx64_in, const void *val, int dtype,
                             const int64_t *list_start, int nlists, void *dense, int64_t dense_n,
                             void *workspace, size_t workspace_bytes, int32_t *status, void *stream);
@@ -443,6 +461,12 @@ size_t zen_bitmap_dense_workspace(int64_t numel, int partitions);
 int zen_bitmap_dense(const void *dict, int64_t numel, int partitions, const uint8_t *bitmaps,
                      const int64_t *bitmap_start, const void *values, int dtype, const int64_t *value_start,
                      void *dense, void *workspace, size_t workspace_bytes, int32_t *status, void *stream);
+/* The same for bitmaps and value lists that sit anywhere (an all-gather ends in one buffer per rank): pointers and
+   lengths (bytes, values) in HOST arrays of `partitions` entries. */
+int zen_bitmap_dense_lists(const void *dict, int64_t numel, int partitions, const uint8_t *const *bitmaps,
+                           const int64_t *bitmap_bytes, const void *const *values, int dtype,
+                           const int64_t *value_count, void *dense, void *workspace, size_t workspace_bytes,
+                           int32_t *status, void *stream);
 
 /* --------------------------------------------------------------- utility */
 

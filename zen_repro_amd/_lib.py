@@ -98,6 +98,9 @@ def lib():
         "zen_merge_zero_bytes": (sz, []),
         "zen_merge": (i32, [vp, i32, vp, i32, i64, i64, vp, i32, vp, i64, vp, i32, vp, sz, vp, vp]),
         "zen_encode_merge": (i32, [ctypes.POINTER(EncodeMergeArgs)]),
+        "zen_merge_rounded": (i32, [vp, i32, vp, i32, i64, i64, vp, i32, vp, i64, vp, i32, vp, sz, vp, vp]),
+        "zen_decode_dense_lists": (i32, [ctypes.POINTER(vp), i32, ctypes.POINTER(vp), i32, ctypes.POINTER(i64), i32, vp, i64, vp,
+                                         sz, vp, vp]),
         "zen_decode_dense_workspace": (sz, [i64, i64]),
         "zen_decode_dense": (i32, [vp, i32, vp, i32, i64, vp, i64, i32, vp, sz, vp, vp]),
         "zen_decode_dense_sorted_workspace": (sz, [i64, i32]),
@@ -107,6 +110,8 @@ def lib():
         "zen_bitmap_dense_workspace": (sz, [i64, i32]),
         "zen_bitmap_dense": (i32, [vp, i64, i32, vp, ctypes.POINTER(ctypes.c_int64), vp, i32,
                                    ctypes.POINTER(ctypes.c_int64), vp, vp, sz, vp, vp]),
+        "zen_bitmap_dense_lists": (i32, [vp, i64, i32, ctypes.POINTER(vp), ctypes.POINTER(i64), ctypes.POINTER(vp), i32,
+                                         ctypes.POINTER(i64), vp, vp, sz, vp, vp]),
         "zen_sort_pairs_workspace": (sz, [i64]),
         "zen_sort_pairs": (i32, [vp, vp, i64, vp, i32, vp, sz, vp, vp]),
         "zen_bucket_sort_fits": (i32, [i64, ctypes.c_uint32]),

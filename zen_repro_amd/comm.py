@@ -3,7 +3,6 @@
 package: one GPU computes its own share, the full P-way partition of its
 gradient and the merge of P incoming payloads."""
 import ctypes
-import itertools
 
 import torch
 
@@ -100,42 +99,67 @@ class LoadBalanceAllreduce:
         exchange and method 1 deliver, comm.py:113-117, 142-145): the dense
         tensor is then built tile by tile without a sort; a list that is not
         ascending after all only costs the time of the attempt."""
-        lists = indices_tensors if isinstance(indices_tensors, (list, tuple)) else [indices_tensors]
-        sizes = [int(t.numel()) for t in lists]
+        L = _lib.lib()
+        if ascending:
+            dense = self._decode_ascending(indices_tensors, values_tensors, alltoall_dense_size)
+            if dense is not None:
+                return dense
         indices = self.stack_tensors(indices_tensors)
         values = self.stack_tensors(values_tensors)
         assert indices.dtype in (torch.int32, torch.int64)
         _lib.require_gpu(indices, "indices")
         _lib.require_gpu(values, "values")
         dev = values.device
-        L = _lib.lib()
         r = indices.numel()
         dense = torch.empty(alltoall_dense_size, dtype=values.dtype, device=dev)
-        if ascending and 1 <= len(sizes) <= 64 and sum(sizes) == r == values.numel():
-            starts = (ctypes.c_int64 * (len(sizes) + 1))(0, *itertools.accumulate(sizes))
-            ws = _lib.scratch.get(dev, "decode_sorted",
-                                  L.zen_decode_dense_sorted_workspace(alltoall_dense_size, len(sizes)))
-            status = _lib.status_word(dev)
-            rc = L.zen_decode_dense_sorted(_lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(values),
-                                           _lib.dtype_code(values), starts, len(sizes), _lib.ptr(dense),
-                                           alltoall_dense_size, _lib.ptr(ws), ws.numel(), _lib.ptr(status),
-                                           _lib.stream_of(dev))
-            _lib.check(rc, "decode_sparse_tensors")
-            if not _lib.read_back(status)[0]:  # the reference's scatter_add_ raises on a bad index, also a sync
-                return dense
-        ws = _lib.scratch.get(dev, "decode", L.zen_decode_dense_workspace(r, alltoall_dense_size))
+        # zeroed at first and left so by the calls, like merge_sparse_flat's
+        ws = _lib.scratch.get(dev, "decode", L.zen_decode_dense_workspace(r, alltoall_dense_size), zero=True)
         for mode in self._fast_then_general():
             status = _lib.status_word(dev)
             rc = L.zen_decode_dense(_lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(values),
-                                    _lib.dtype_code(values), r, _lib.ptr(dense), alltoall_dense_size, mode,
-                                    _lib.ptr(ws), ws.numel(), _lib.ptr(status), _lib.stream_of(dev))
+                                    _lib.dtype_code(values), r, _lib.ptr(dense), alltoall_dense_size,
+                                    mode | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status),
+                                    _lib.stream_of(dev))
+            if rc != _lib.OK:
+                ws[:L.zen_merge_zero_bytes()].zero_()
             _lib.check(rc, "decode_sparse_tensors")
             bits = _lib.read_back(status)[0]  # the reference's scatter_add_ raises on a bad index, also a sync
+            if bits & (_lib.STAT_RETRY | _lib.STAT_INTERNAL):
+                ws[:L.zen_merge_zero_bytes()].zero_()
             if not bits & _lib.STAT_RETRY:
                 break
         if bits:
             raise RuntimeError("decode_sparse_tensors: " + _lib.describe_status(bits))
         return dense
+
+    def _decode_ascending(self, indices_tensors, values_tensors, dense_size):
+        """decode_sparse_tensors of ascending lists where they are, without putting them into one buffer first;
+        None if that path does not take them (more than 64 lists, or one that is not ascending after all)."""
+        lists = indices_tensors if isinstance(indices_tensors, (list, tuple)) else [indices_tensors]
+        values = values_tensors if isinstance(values_tensors, (list, tuple)) else [values_tensors]
+        count = len(lists)
+        if not 1 <= count <= 64 or len(values) != count:
+            return None
+        for i, v in zip(lists, values):
+            if i.dtype != lists[0].dtype or v.dtype != values[0].dtype or i.numel() != v.numel():
+                return None
+            _lib.require_gpu(i, "indices")
+            _lib.require_gpu(v, "values")
+        assert lists[0].dtype in (torch.int32, torch.int64)
+        dev = values[0].device
+        L = _lib.lib()
+        dense = torch.empty(dense_size, dtype=values[0].dtype, device=dev)
+        idx_at = (ctypes.c_void_p * count)(*[t.data_ptr() for t in lists])
+        val_at = (ctypes.c_void_p * count)(*[t.data_ptr() for t in values])
+        sizes = (ctypes.c_int64 * count)(*[t.numel() for t in lists])
+        ws = _lib.scratch.get(dev, "decode_sorted", L.zen_decode_dense_sorted_workspace(dense_size, count))
+        status = _lib.status_word(dev)
+        rc = L.zen_decode_dense_lists(idx_at, int(lists[0].dtype == torch.int64), val_at, _lib.dtype_code(values[0]),
+                                      sizes, count, _lib.ptr(dense), dense_size, _lib.ptr(ws), ws.numel(),
+                                      _lib.ptr(status), _lib.stream_of(dev))
+        _lib.check(rc, "decode_sparse_tensors")
+        # the reference's scatter_add_ raises on a bad index, also a sync
+        return None if _lib.read_back(status)[0] else dense
 
     # OR-ed into the mode of every fast-mode call (_lib.MODE_SLABS keeps the calls off the wide buckets)
     fast_flags = 0
@@ -162,6 +186,10 @@ class LoadBalanceAllreduce:
         with mode=MODE_GENERAL (merge_sparse does that by itself).  Calls that
         may be in flight at the same time must use different `slot` numbers
         (a slot owns its workspace)."""
+        return self._merge(indices_tensors, values_tensors, dense_size, capacity, idx64, mode, slot, False)
+
+    def _merge(self, indices_tensors, values_tensors, dense_size, capacity, idx64, mode, slot, rounded):
+        """merge_sparse_flat; `rounded`: the sums leave in the values' type (zen_merge_rounded)."""
         indices = self.stack_tensors(indices_tensors)
         values = self.stack_tensors(values_tensors)
         _lib.require_gpu(indices, "indices")
@@ -174,16 +202,16 @@ class LoadBalanceAllreduce:
         if (mode & 0xff) == _lib.MODE_FAST:
             mode |= self.fast_flags
         out_idx = torch.empty(capacity, dtype=torch.int64 if idx64 else torch.int32, device=dev)
-        out_val = torch.empty(capacity, dtype=torch.float32, device=dev)
+        out_val = torch.empty(capacity, dtype=values.dtype if rounded else torch.float32, device=dev)
         count = _lib.zeros.take(dev, 1, torch.int64)
         status = _lib.status_word(dev)
         # The workspace is allocated zeroed and serves zen_merge only, which leaves its head (the counters
         # that must start at zero) zero again: no call spends a kernel on clearing it.
         ws = _lib.scratch.get(dev, f"merge/{slot}", L.zen_merge_workspace(r, dense_size), zero=True)
-        rc = L.zen_merge(_lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(values),
-                         _lib.dtype_code(values), r, dense_size, _lib.ptr(out_idx), 1 if idx64 else 0,
-                         _lib.ptr(out_val), capacity, _lib.ptr(count), mode | _lib.MODE_ZEROED, _lib.ptr(ws),
-                         ws.numel(), _lib.ptr(status), _lib.stream_of(dev))
+        rc = (L.zen_merge_rounded if rounded else L.zen_merge)(
+            _lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(values), _lib.dtype_code(values), r,
+            dense_size, _lib.ptr(out_idx), 1 if idx64 else 0, _lib.ptr(out_val), capacity, _lib.ptr(count),
+            mode | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status), _lib.stream_of(dev))
         if rc != _lib.OK:
             ws[:L.zen_merge_zero_bytes()].zero_()
         _lib.check(rc, "merge_sparse")
@@ -298,19 +326,25 @@ class LoadBalanceAllreduce:
 
     def merge_rounded(self, indices_tensors, values_tensors, dense_size, dtype):
         """merge_sparse followed by the rounding of round_merged_flat: (int64 indices, values of `dtype`), with
-        one host synchronisation (the result's size) instead of three."""
+        one host synchronisation (the result's size) instead of three, and in one pass where the received values
+        have that type."""
+        values_tensors = self.stack_tensors(values_tensors)
+        rounded = values_tensors.dtype == dtype
         for mode in self._fast_then_general():
-            idx, val, count, status = self.merge_sparse_flat(indices_tensors, values_tensors, dense_size,
-                                                             idx64=True, mode=mode)
-            r_idx, r_val, kept, r_status = self.round_merged_flat(idx, val, count, dtype)
-            host = _lib.read_back(kept, status, r_status)
+            idx, val, count, status = self._merge(indices_tensors, values_tensors, dense_size, None, True, mode, 0,
+                                                  rounded)
+            if rounded:
+                r_status = status
+            else:
+                idx, val, count, r_status = self.round_merged_flat(idx, val, count, dtype)
+            host = _lib.read_back(count, status, r_status)
             if host[1] & (_lib.STAT_RETRY | _lib.STAT_INTERNAL):
                 self.reset_merge_workspace(idx.device)
             if not host[1] & _lib.STAT_RETRY:
                 break
         if host[1] | host[2]:
             raise RuntimeError("merge_rounded: " + _lib.describe_status(host[1] | host[2]))
-        return r_idx[:host[0]], r_val[:host[0]]
+        return idx[:host[0]], val[:host[0]]
 
     def reset_merge_workspace(self, device, slot=0):
         """After a merge_sparse_flat whose status carried STAT_RETRY or
@@ -460,18 +494,22 @@ class LoadBalanceAllreduce:
             _lib.check(L.zen_bitmap_dense_dict(numel, self.partitions, _lib.ptr(cached), None, _lib.stream_of(dev)),
                        "decode_bitmaps_dense")
             self._dense_dicts[numel] = cached
-        bitmaps = self.stack_tensors(list(bitmap_indices))
-        values = self.stack_tensors(list(values_tensors))
-        _lib.require_gpu(values, "values")
+        values = list(values_tensors)
+        for t in values:
+            _lib.require_gpu(t, "values")
+            if t.dtype != values[0].dtype:
+                raise RuntimeError("values must have one type")
         P = self.partitions
-        bm_start = (ctypes.c_int64 * (P + 1))(0, *itertools.accumulate(int(t.numel()) for t in bitmap_indices))
-        v_start = (ctypes.c_int64 * (P + 1))(0, *itertools.accumulate(int(t.numel()) for t in values_tensors))
-        dense = torch.empty(numel, dtype=values.dtype, device=dev)
+        bm_at = (ctypes.c_void_p * P)(*[t.data_ptr() for t in bitmap_indices])
+        bm_bytes = (ctypes.c_int64 * P)(*[t.numel() for t in bitmap_indices])
+        v_at = (ctypes.c_void_p * P)(*[t.data_ptr() for t in values])
+        v_count = (ctypes.c_int64 * P)(*[t.numel() for t in values])
+        dense = torch.empty(numel, dtype=values[0].dtype, device=dev)
         ws = _lib.scratch.get(dev, "bitmap_dense", L.zen_bitmap_dense_workspace(numel, P))
         status = _lib.status_word(dev)
-        rc = L.zen_bitmap_dense(_lib.ptr(cached), numel, P, _lib.ptr(bitmaps), bm_start, _lib.ptr(values),
-                                _lib.dtype_code(values), v_start, _lib.ptr(dense), _lib.ptr(ws), ws.numel(),
-                                _lib.ptr(status), _lib.stream_of(dev))
+        rc = L.zen_bitmap_dense_lists(_lib.ptr(cached), numel, P, bm_at, bm_bytes, v_at, _lib.dtype_code(values[0]),
+                                      v_count, _lib.ptr(dense), _lib.ptr(ws), ws.numel(), _lib.ptr(status),
+                                      _lib.stream_of(dev))
         _lib.check(rc, "decode_bitmaps_dense")
         bits = _lib.read_back(status)[0]  # the reference's masking and scatter_add_ raise on a mismatch, also a sync
         if bits & _lib.STAT_BAD_INDEX:

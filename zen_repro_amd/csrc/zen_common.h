@@ -131,6 +131,8 @@ __device__ inline uint32_t probe_slot(const Probe &g, uint32_t t, int level, uin
   return part * g.npp + (h + seed) % g.npp;
 }
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
 // Element storage and magnitude keys (bit pattern with the sign cleared).
 template <typename S>
 struct KeyOf;
@@ -153,6 +155,21 @@ __device__ inline uint16_t f32_to_bf16_rne(float f) {
   u += 0x7fffu + ((u >> 16) & 1u);
   return uint16_t(u >> 16);
 }
+
+// What a merge writes for a sum: the fp32 sum itself, or the sum rounded once to bf16 (a sum that rounds to zero is
+// dropped with those that are zero; torch.nonzero keeps NaN and drops +-0).
+template <typename O>
+struct SumAs;
+template <>
+struct SumAs<float> {
+  static __device__ inline float of(float v) { return v; }
+  static __device__ inline bool kept(float v) { return v != 0.0f; }
+};
+template <>
+struct SumAs<uint16_t> {
+  static __device__ inline uint16_t of(float v) { return f32_to_bf16_rne(v); }
+  static __device__ inline bool kept(float v) { return (f32_to_bf16_rne(v) & 0x7fffu) != 0; }
+};
 
 // Waits until the global memory operations this wave has issued, stores and atomics without a return value
 // included, have been acknowledged by the place that carries them out.

@@ -11,28 +11,24 @@
 // list); then a workgroup per tile brings the tile's bit ranges and values into LDS, looks up the place of
 // every SET bit's member in the dictionary, and writes the tile once, zeros included: the dense tensor is
 // never cleared, nothing is scattered in memory, and of the dictionary only the set bits' entries are read.
-#include <mutex>
-
 #include "zen_common.h"
 
 namespace zen {
 namespace {
 
-#ifndef ZEN_FD_TILE
-#define ZEN_FD_TILE 8192
-#endif
-constexpr int kFdTile = ZEN_FD_TILE;
+constexpr int kFdTile = 8192;
 constexpr int kFdBlock = 512;
 constexpr int kFdPer = kFdTile / kFdBlock;   // consecutive indices per thread (16)
 constexpr int kFdMaxLists = 64;
 constexpr int kFdChunk = 16;                  // thread columns whose counts one thread adds up
 constexpr int kFdChunks = kFdBlock / kFdChunk;
 constexpr int kFdChunkRow = kFdChunks + 8;   // 16-bit words per list in the chunk table (rows stay 16-byte aligned)
-constexpr int kFdMaxBytes = kFdTile / 8 + 2 * kFdMaxLists;  // bitmap bytes a tile's bit ranges can span
 static_assert(kFdChunks == 32, "a wave's lower half scans the chunk sums");
 
-struct ListStarts {
-  int64_t at[kFdMaxLists + 1];
+struct FdLists {
+  const uint8_t *bitmap[kFdMaxLists];
+  const void *val[kFdMaxLists];
+  uint32_t bytes[kFdMaxLists], vals[kFdMaxLists];  // of the bitmap; values
 };
 
 __device__ inline uint32_t part_of(uint32_t t, uint32_t n, uint32_t npp) {
@@ -85,7 +81,7 @@ __global__ __launch_bounds__(kFdBlock) void k_fd_order(uint32_t n, uint32_t npp,
     const uint32_t incl = wave_inclusive_scan(total);
     if (threadIdx.x < (uint32_t)P) {
       s_base[threadIdx.x] = incl - total;
-      below[(size_t)threadIdx.x * (gridDim.x + 1) + blockIdx.x] = total;
+      below[(size_t)blockIdx.x * P + threadIdx.x] = total;
     }
   }
   __syncthreads();
@@ -100,33 +96,32 @@ __global__ __launch_bounds__(kFdBlock) void k_fd_order(uint32_t n, uint32_t npp,
   }
 }
 
-// Per list (blockIdx.x): exclusive prefix over the tiles of a [P][tiles + 1] table of counts, in place; the last
-// entry of a row receives the total.  A thread takes eight consecutive entries per round (two 16-byte loads),
-// a round covers 8192 of them.
+// Per list (blockIdx.x): exclusive prefix over the tiles of a [tiles + 1][P] table of counts, in place; the last
+// row receives the totals.  A thread takes eight consecutive tiles per round.  Run once per dictionary.
 constexpr int kFdScanBlock = 1024;
 constexpr int kFdScanPer = 8;
-__global__ __launch_bounds__(kFdScanBlock) void k_fd_scan(uint32_t *__restrict__ table, uint32_t tiles) {
+__global__ __launch_bounds__(kFdScanBlock) void k_fd_scan(uint32_t *__restrict__ table, uint32_t tiles, int P) {
   __shared__ uint32_t s_scan[kFdScanBlock / 64 + 1];
-  uint32_t *row = table + (size_t)blockIdx.x * (tiles + 1);
+  uint32_t *column = table + blockIdx.x;
   uint32_t carry = 0;
   for (uint32_t base = 0; base < tiles; base += kFdScanBlock * kFdScanPer) {
     const uint32_t first = base + threadIdx.x * kFdScanPer;
     uint32_t c[kFdScanPer], sum = 0;
 #pragma unroll
     for (int j = 0; j < kFdScanPer; ++j) {
-      c[j] = first + j < tiles ? row[first + j] : 0u;
+      c[j] = first + j < tiles ? column[(size_t)(first + j) * P] : 0u;
       sum += c[j];
     }
     uint32_t total;
     uint32_t running = carry + block_exclusive_scan<uint32_t, kFdScanBlock>(sum, s_scan, &total);
 #pragma unroll
     for (int j = 0; j < kFdScanPer; ++j) {
-      if (first + j < tiles) row[first + j] = running;
+      if (first + j < tiles) column[(size_t)(first + j) * P] = running;
       running += c[j];
     }
     carry += total;
   }
-  if (threadIdx.x == 0) row[tiles] = carry;
+  if (threadIdx.x == 0) column[(size_t)tiles * P] = carry;
 }
 
 // Set bits of bitmap `bm` in the bit range [b0, b1); bytes at or beyond `bytes` count as zero.  Read as
@@ -150,338 +145,198 @@ __device__ inline uint32_t popcount_range(const uint8_t *__restrict__ bm, int64_
   return c;
 }
 
-// Where the values of a tile start in every list, in two levels: the tiles are taken in groups of 256; a row of
-// 257 words per (list, group) holds the set bits of the group's tiles in front of each tile (entry 256: of the
-// whole group), a second table the set bits in front of each group.
+// Where the values of a tile start in every list, in two levels: the tiles are taken in groups of 256; a row of P
+// words per tile holds the set bits of the group's tiles in front of it, a row per group the set bits in front of
+// the group.
 constexpr int kFdGroup = 256;
-constexpr int kFdGroupRow = kFdGroup + 1;
 inline uint32_t fd_groups(uint32_t tiles) { return (tiles + kFdGroup - 1) / kFdGroup; }
 
 // Per (group of tiles, list): set bits in each tile's bit range of the list's bitmap, summed up inside the
 // group.  A bitmap shorter than its list (the reference's mask would not fit the member list, comm.py:97-98)
 // raises ZEN_STAT_BAD_INDEX.
 __global__ __launch_bounds__(kFdGroup) void k_fd_count(const uint32_t *__restrict__ below, uint32_t tiles, int P,
-                                                       const uint8_t *__restrict__ bitmaps, ListStarts bm,
-                                                       uint32_t *__restrict__ vstart, uint32_t *__restrict__ gsum,
-                                                       int32_t *status) {
+                                                       FdLists lists, uint32_t *__restrict__ vstart,
+                                                       uint32_t *__restrict__ gsum, int32_t *status) {
   __shared__ uint32_t s_scan[kFdGroup / 64 + 1];
   const uint32_t tile = blockIdx.x * (uint32_t)kFdGroup + threadIdx.x;
   const int p = blockIdx.y;
   uint32_t cnt = 0;
   if (tile < tiles) {
-    const size_t i = (size_t)p * (tiles + 1) + tile;
-    const uint32_t b0 = below[i], b1 = below[i + 1];
-    const int64_t bytes = bm.at[p + 1] - bm.at[p];
+    const size_t i = (size_t)tile * P + p;
+    const uint32_t b0 = below[i], b1 = below[i + P];
+    const int64_t bytes = lists.bytes[p];
     if (tile == tiles - 1 && ((int64_t)b1 + 7) / 8 > bytes) atomicOr(status, ZEN_STAT_BAD_INDEX);
-    cnt = popcount_range(bitmaps + bm.at[p], bytes, b0, b1);
+    cnt = popcount_range(lists.bitmap[p], bytes, b0, b1);
   }
   uint32_t total;
   const uint32_t before = block_exclusive_scan<uint32_t, kFdGroup>(cnt, s_scan, &total);
-  const size_t g = (size_t)p * gridDim.x + blockIdx.x;
-  vstart[g * kFdGroupRow + threadIdx.x] = before;
-  if (threadIdx.x == 0) {
-    vstart[g * kFdGroupRow + kFdGroup] = total;
-    gsum[g] = total;
-  }
+  if (tile < tiles) vstart[(size_t)tile * P + p] = before;
+  if (threadIdx.x == 0) gsum[(size_t)blockIdx.x * P + p] = total;
 }
 
 // Per list (blockIdx.x): exclusive prefix over the groups' sums, in place (a tensor of 2^31 elements has 1024 groups).
 constexpr int kFdGroupsMax = 1024;
-__global__ __launch_bounds__(kFdGroupsMax) void k_fd_groups(uint32_t *__restrict__ gsum, uint32_t groups) {
+__global__ __launch_bounds__(kFdGroupsMax) void k_fd_groups(uint32_t *__restrict__ gsum, uint32_t groups, int P) {
   __shared__ uint32_t s_scan[kFdGroupsMax / 64 + 1];
-  uint32_t *row = gsum + (size_t)blockIdx.x * groups;
-  const uint32_t v = threadIdx.x < groups ? row[threadIdx.x] : 0u;
+  uint32_t *at = gsum + (size_t)threadIdx.x * P + blockIdx.x;
+  const uint32_t v = threadIdx.x < groups ? *at : 0u;
   uint32_t total;
   const uint32_t before = block_exclusive_scan<uint32_t, kFdGroupsMax>(v, s_scan, &total);
-  if (threadIdx.x < groups) row[threadIdx.x] = before;
+  if (threadIdx.x < groups) *at = before;
 }
 
 template <typename S>
 __device__ inline S fd_value(S v);  // what a zeroed element holds after one scatter_add_ of v (comm.py:35-39)
 template <>
-__device__ inline uint16_t fd_value<uint16_t>(uint16_t v) {
-  return f32_to_bf16_rne(0.0f + KeyOf<uint16_t>::to_f32(v));
+__device__ inline uint16_t fd_value<uint16_t>(uint16_t v) {  // 0.0f + v is v, but for -0 and signalling NaNs
+  if (v == 0x8000u) v = 0;
+  return (v & 0x7fffu) > 0x7f80u ? (uint16_t)(v | 0x40u) : v;
 }
 template <>
 __device__ inline uint32_t fd_value<uint32_t>(uint32_t v) {
   return __float_as_uint(0.0f + __uint_as_float(v));
 }
 
-// A workgroup takes one tile after the other (tile = blockIdx.x, + gridDim.x, ...): the tile's bit ranges and
-// its values (contiguous stretches of the lists) come into LDS, the set bits are written out as a list, and the
-// threads take one SET bit each: its member's place in the tile is one entry of the dictionary, the value goes
-// there, into a copy of the tile in LDS that is written out once.  The next tile's table entries are asked for
-// while this tile is worked on.
-constexpr int kFdValStage = kFdTile / 8;  // values of a tile kept in LDS (tiles with more set bits fetch the rest one by one)
-constexpr int kFdHitStage = kFdTile / 8;  // set bits of a tile listed at a time
-constexpr int kFdBytesPer = (kFdMaxBytes + kFdBlock - 1) / kFdBlock;  // 3
-constexpr int kFdValsPer = kFdValStage / kFdBlock;                    // 2
-#ifndef ZEN_FD_MIN_WAVES
-#define ZEN_FD_MIN_WAVES 6  // waves per SIMD the tile kernel is compiled for: three workgroups to a compute unit
-#endif
-
-// Thread p < P: list p's members below the tile and below the next, the set bits below the tile's group, below
-// the tile inside the group, below the next tile inside the group.
-__device__ __forceinline__ void fd_fetch_dict(const uint32_t *__restrict__ below, const uint32_t *__restrict__ vstart,
-                                              const uint32_t *__restrict__ gpre, uint32_t tiles, uint32_t groups, int P,
-                                              uint32_t tile, uint32_t (&d)[5]) {
-  d[0] = d[1] = d[2] = d[3] = d[4] = 0;
-  if (threadIdx.x < (uint32_t)P) {
-    const size_t at = (size_t)threadIdx.x * (tiles + 1) + tile;
-    const size_t g = (size_t)threadIdx.x * groups + tile / kFdGroup;
-    const size_t va = g * kFdGroupRow + tile % kFdGroup;
-    d[0] = below[at];
-    d[1] = below[at + 1];
-    d[2] = gpre[g];
-    d[3] = vstart[va];
-    d[4] = vstart[va + 1];
-  }
-}
-
-constexpr int kFdByteBlocks = (kFdMaxBytes + 15) / 16;
-constexpr int kFdValBlocks = kFdValStage / 16;
-
-// Wave 0: the table of a tile's lists from the entries fetched for it.
-__device__ __forceinline__ void fd_list_table(const uint32_t (&d)[5], int P, uint4 *meta, uint4 *len, uint8_t *byte_lut,
-                                              uint8_t *val_lut) {
-  const int p = threadIdx.x;
-  uint32_t b0 = 0, cnt = 0, nb = 0, v0 = 0, nv = 0;
-  if (p < P) {
-    b0 = d[0];
-    cnt = d[1] - d[0];
-    if (cnt > (uint32_t)kFdTile) cnt = kFdTile;  // cannot be with a table this library built
-    nb = cnt ? ((b0 + cnt - 1u) >> 3) - (b0 >> 3) + 1u : 0u;
-    v0 = d[2] + d[3];
-    nv = d[4] - d[3];
-    if (nv > cnt) nv = cnt;  // cannot be (the count kernel counted the same bits)
-  }
-  const uint32_t bincl = wave_inclusive_scan(nb), vincl = wave_inclusive_scan(nv), cincl = wave_inclusive_scan(cnt);
-  if (p < P) {
-    meta[p] = make_uint4(b0, bincl - nb, v0, vincl - nv);
-    len[p] = make_uint4(cnt, nv, cincl - cnt, 0);
-  }
-  if (p == 63) meta[P] = make_uint4(0, bincl, cincl, vincl);
-  // the list that holds the first entry of every block of 16 entries of the side-by-side arrays
-  for (uint32_t blk = (bincl - nb + 15u) >> 4; (blk << 4) < bincl && blk < (uint32_t)kFdByteBlocks; ++blk) byte_lut[blk] = (uint8_t)p;
-  for (uint32_t blk = (vincl - nv + 15u) >> 4; (blk << 4) < vincl && blk < (uint32_t)kFdValBlocks; ++blk) val_lut[blk] = (uint8_t)p;
-}
-
-// A tile's bitmap bytes and values as they will lie side by side in LDS, asked for one tile ahead and kept in
-// registers meanwhile.  Entry i of such an array belongs to the last list whose stretch starts at or before i
-// (the stretches' starts ascend): the list of the block's first entry is looked up, the few lists that may start
-// inside the block are stepped over, so that every thread fetches its entries in one go instead of list after list.
-template <typename S>
-__device__ __forceinline__ void fd_fetch_lists(const uint4 *meta, int P, const uint8_t *byte_lut, const uint8_t *val_lut,
-                                               const int64_t *s_bm, const int64_t *s_vs,
-                                               const uint8_t *__restrict__ bitmaps, const S *__restrict__ values,
-                                               uint32_t (&byte_in)[kFdBytesPer], uint32_t (&byte_list)[kFdBytesPer],
-                                               S (&val_in)[kFdValsPer]) {
-  uint32_t total_bytes = meta[P].y;
-  if (total_bytes > (uint32_t)kFdMaxBytes || meta[P].z > (uint32_t)kFdTile) total_bytes = 0;
-  const uint32_t total_vals = min(meta[P].w, (uint32_t)kFdValStage);
-#pragma unroll
-  for (int k = 0; k < kFdBytesPer; ++k) {
-    const uint32_t i = threadIdx.x + (uint32_t)k * kFdBlock;
-    byte_in[k] = 0;
-    byte_list[k] = 0;
-    if (i < total_bytes) {
-      int lo = byte_lut[i >> 4];
-      while (lo + 1 < P && meta[lo + 1].y <= i) ++lo;
-      const int64_t g = (int64_t)(meta[lo].x >> 3) + (i - meta[lo].y);
-      byte_list[k] = (uint32_t)lo;
-      if (g < s_bm[lo + 1] - s_bm[lo]) byte_in[k] = bitmaps[s_bm[lo] + g];  // a short bitmap was flagged by the count kernel
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < kFdValsPer; ++k) {
-    const uint32_t i = threadIdx.x + (uint32_t)k * kFdBlock;
-    val_in[k] = 0;
-    if (i < total_vals) {
-      int lo = val_lut[i >> 4];
-      while (lo + 1 < P && meta[lo + 1].w <= i) ++lo;
-      const int64_t g = (int64_t)meta[lo].z + (i - meta[lo].w);
-      if (g < s_vs[lo + 1] - s_vs[lo]) val_in[k] = values[s_vs[lo] + g];
-    }
-  }
-}
+// One workgroup per tile.  Lane p of every wave knows list p's members in the tile, the first bit of their range
+// and where its values start; the lists' members are cut into chunks of 640, dealt to the eight waves in turn.  A
+// wave gets the chunk's bits as ten 64-bit words in scalar registers: the word is the mask of the lanes whose
+// member has a value, a lane's value is the one numbered by the set bits below it, and its place in the tile is
+// the chunk's next entry of the dictionary, so that all loads are consecutive, ten of each kind in flight.  The
+// places written are put together in LDS and leave with full-width stores.
+// Bound by memory: two bytes of dictionary and one element of output per index, and the values.  62 M bf16 elements
+// on sixteen ranks, 71 % of them set, 0.34 GB: 79 us; 268 M elements, 11 % set, 1.13 GB: 300 us.  One SET bit per
+// thread and turn, looked up in staged copies of the tile's bytes and values, took 307 and 411 us; with each value's
+// load in a branch of its own, which makes the compiler wait for it there, this kernel took 129 and 428.
+constexpr int kFdWords = 10;                 // words of a chunk: sixteen lists have 512 +- 70 members in a tile
+constexpr int kFdMembers = 64 * kFdWords;    // members of a chunk
 
 template <typename S>
-__global__ __launch_bounds__(kFdBlock, ZEN_FD_MIN_WAVES) void k_fd_tiles(const uint16_t *__restrict__ order,
-                                                                        const uint32_t *__restrict__ below,
-                                                                        const uint32_t *__restrict__ vstart,
-                                                                        const uint32_t *__restrict__ gpre, uint32_t tiles,
-                                                                        int P, uint32_t n,
-                                                                        const uint8_t *__restrict__ bitmaps, ListStarts bm,
-                                                                        const S *__restrict__ values, ListStarts vs,
-                                                                        S *__restrict__ dense, int32_t *status) {
-  // per list: first bit of the tile's range; where its bytes start in s_bl; number of the tile's first value in
-  // the list; where its values start in s_val (entry P: the totals)
-  __shared__ uint4 s_meta[2][kFdMaxLists + 1];        // two sets: this tile's and the next one's
-  __shared__ uint4 s_len[2][kFdMaxLists];             // per list: members in the tile; set bits among them; members of lower lists in the tile
-  __shared__ uint8_t s_blut[2][kFdByteBlocks + 3], s_vlut[2][kFdValBlocks];  // list of every 16th byte and value
-  __shared__ uint32_t s_front[kFdMaxLists];           // per list: set bits of the tile in the lists before it
-  __shared__ uint16_t s_bl[kFdMaxBytes + 8];          // the bitmap bytes of the tile's ranges (low half) and their list (high half)
-  __shared__ S s_val[kFdValStage];
-  __shared__ __attribute__((aligned(16))) S s_tile[kFdTile];  // the tile of the dense tensor
-  __shared__ uint32_t s_hit[kFdHitStage];             // set bits: list << 16 | place in s_bl << 3 | bit
-  __shared__ uint32_t s_scan[kFdBlock / 64 + 1];
-  // the lists' offsets, looked up by list number further down: in LDS, because a kernel argument indexed with a
-  // number that differs from lane to lane is fetched from memory, one round trip per look
-  __shared__ int64_t s_bm[kFdMaxLists + 1], s_vs[kFdMaxLists + 1];
-  if (threadIdx.x <= (uint32_t)P) {
-    s_bm[threadIdx.x] = bm.at[threadIdx.x];
-    s_vs[threadIdx.x] = vs.at[threadIdx.x];
+__global__ __launch_bounds__(kFdBlock, 8) void k_fd_tiles(const uint16_t *__restrict__ order,
+                                                       const uint32_t *__restrict__ below,
+                                                       const uint32_t *__restrict__ vstart,
+                                                       const uint32_t *__restrict__ gpre, int P, uint32_t n,
+                                                       FdLists lists, S *__restrict__ dense, int32_t *status) {
+  __shared__ __attribute__((aligned(16))) S s_tile[kFdTile];
+  const uint32_t tile = blockIdx.x;
+  const uint32_t tile_base = tile * (uint32_t)kFdTile;
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  uint32_t b0 = 0, b1 = 0, v0 = 0;
+  if (lane < P) {
+    const size_t at = (size_t)tile * P + lane;
+    b0 = below[at];
+    b1 = below[at + P];
+    v0 = vstart[at] + gpre[(size_t)(tile / kFdGroup) * P + lane];
   }
-  const uint32_t groups = (tiles + kFdGroup - 1) / kFdGroup;
-  const bool aligned = (reinterpret_cast<uintptr_t>(dense) & 15u) == 0;
-  uint32_t byte_in[kFdBytesPer], byte_list[kFdBytesPer];
-  S val_in[kFdValsPer];
-  uint32_t dn[5];
-  if (blockIdx.x >= tiles) return;
-  if (threadIdx.x < 64) {
-    fd_fetch_dict(below, vstart, gpre, tiles, groups, P, blockIdx.x, dn);
-    fd_list_table(dn, P, s_meta[0], s_len[0], s_blut[0], s_vlut[0]);
-    if (blockIdx.x + gridDim.x < tiles) fd_fetch_dict(below, vstart, gpre, tiles, groups, P, blockIdx.x + gridDim.x, dn);
+  {
+    uint4 *z = reinterpret_cast<uint4 *>(s_tile);
+#pragma unroll
+    for (int i = 0; i < (int)(kFdTile * sizeof(S) / 16) / kFdBlock; ++i) z[i * kFdBlock + threadIdx.x] = make_uint4(0, 0, 0, 0);
+  }
+  uint32_t cnt = b1 - b0;
+  if (cnt > (uint32_t)kFdTile) cnt = 0;  // cannot be with a table this library built
+  const uint32_t chunks = (cnt + kFdMembers - 1) / kFdMembers;
+  const uint32_t incl = wave_inclusive_scan(cnt), cincl = wave_inclusive_scan(chunks);
+  const uint32_t nchunks = (uint32_t)__builtin_amdgcn_readlane((int)cincl, 63);
+  const bool odd = __builtin_amdgcn_readlane((int)incl, 63) > kFdTile;  // cannot be either
+  bool bad = false;
+  __syncthreads();
+#pragma unroll 1
+  for (uint32_t c = (uint32_t)wave; c < nchunks && !odd; c += kFdBlock / 64) {
+    const int p = (int)__popcll(__ballot(cincl <= c));  // the chunk's list
+    const uint32_t j0 = (c - (uint32_t)__builtin_amdgcn_readlane((int)(cincl - chunks), p)) * kFdMembers;
+    const uint32_t members = (uint32_t)__builtin_amdgcn_readlane((int)cnt, p) - j0;  // from here on, > 0
+    const uint32_t bit0 = (uint32_t)__builtin_amdgcn_readlane((int)b0, p) + j0;
+    const uint16_t *place_at = order + tile_base + (uint32_t)__builtin_amdgcn_readlane((int)(incl - cnt), p) + j0;
+    uint32_t place[kFdWords];
+#pragma unroll
+    for (int i = 0; i < kFdWords; ++i) {
+      const uint32_t j = (uint32_t)(i * 64 + lane);
+      place[i] = __builtin_nontemporal_load(place_at + (j < members ? j : 0u));
+    }
+    // Lane i: bits [bit0 + 64 i, bit0 + 64 i + 64) of the bitmap, from the two aligned words that hold them (a
+    // word with one byte of the bitmap lies in that byte's page); bits of other tiles and past the bitmap's
+    // end count as zero.
+    const uintptr_t addr = reinterpret_cast<uintptr_t>(lists.bitmap[p]);
+    const uint64_t limit = (uint64_t)lists.bytes[p] * 8u;
+    const uint64_t *words = reinterpret_cast<const uint64_t *>(addr & ~(uintptr_t)7);
+    const uint64_t first = (uint64_t)bit0 + (addr & 7u) * 8u, over = limit + (addr & 7u) * 8u;
+    const uint64_t at = (first >> 6) + (uint64_t)lane;
+    unsigned long long w = 0;
+    if (lane <= kFdWords && at * 64u < over) w = words[at];
+    const unsigned sh = (unsigned)(first & 63u);
+    const unsigned long long up = __shfl_down(w, 1, 64);
+    unsigned long long bits = (w >> sh) | (sh ? up << (64u - sh) : 0ull);
+    {
+      uint64_t left = (uint64_t)bit0 < limit ? limit - bit0 : 0u;  // bits the bitmap has from the chunk's first on
+      if (left > members) left = members;
+      const uint64_t mine = (uint64_t)lane * 64u;
+      if (lane >= kFdWords || left <= mine) bits = 0;
+      else if (left - mine < 64u) bits &= (1ull << (left - mine)) - 1ull;
+    }
+    // set bits of the tile's range in front of the chunk: the list's earlier chunks in this tile
+    uint32_t nth = (uint32_t)__builtin_amdgcn_readlane((int)v0, p);
+    if (j0) {  // 128 bits per lane
+      const uint32_t from = bit0 - j0 + (uint32_t)lane * (kFdTile / 64);
+      const uint32_t to = from + kFdTile / 64;
+      nth += wave_sum(from < bit0 ? popcount_range(lists.bitmap[p], lists.bytes[p], from, to < bit0 ? to : bit0) : 0u);
+    }
+    nth = (uint32_t)__builtin_amdgcn_readfirstlane((int)nth);
+    const uint32_t have = lists.vals[p];
+    if (have == 0) {
+      bad = bad || __ballot(bits != 0);
+      continue;
+    }
+    const S *val = static_cast<const S *>(lists.val[p]) + nth;
+    const uint32_t last = have > nth ? have - nth - 1u : 0u;  // the loads sit in no branch: lanes without a value read a neighbour's
+    if (have <= nth) val -= nth;
+    S v[kFdWords];
+    unsigned long long word[kFdWords];
+    uint32_t front = 0;
+#pragma unroll
+    for (int i = 0; i < kFdWords; ++i) {
+      const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)bits, i);
+      const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32), i);
+      word[i] = ((unsigned long long)hi << 32) | lo;
+      const uint32_t k = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, front));
+      // (a 32-bit byte offset: k is below 640 where it matters)
+      v[i] = *reinterpret_cast<const S *>(reinterpret_cast<const char *>(val) + (uint32_t)((k < last ? k : last) * sizeof(S)));
+      front += (uint32_t)__popcll(word[i]);
+    }
+    if (nth + front > have) {  // more set bits than values: the missing ones count as unset
+      bad = true;
+      front = 0;
+#pragma unroll
+      for (int i = 0; i < kFdWords; ++i) {
+        const uint32_t k = __builtin_amdgcn_mbcnt_hi((uint32_t)(word[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)word[i], front));
+        front += (uint32_t)__popcll(word[i]);
+        word[i] &= __ballot(nth + k < have);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kFdWords; ++i)
+      if (__builtin_amdgcn_inverse_ballot_w64(word[i])) s_tile[place[i] & (uint32_t)(kFdTile - 1)] = fd_value<S>(v[i]);
   }
   __syncthreads();
-  fd_fetch_lists<S>(s_meta[0], P, s_blut[0], s_vlut[0], s_bm, s_vs, bitmaps, values, byte_in, byte_list, val_in);
-  bool bad = false;
-  int set = 0;
-  for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x, set ^= 1) {
-    const uint32_t tile_base = tile * (uint32_t)kFdTile;
-    const uint32_t next = tile + gridDim.x;
-    if (threadIdx.x < 64 && next < tiles) {
-      fd_list_table(dn, P, s_meta[set ^ 1], s_len[set ^ 1], s_blut[set ^ 1], s_vlut[set ^ 1]);
-      if (next + gridDim.x < tiles) fd_fetch_dict(below, vstart, gpre, tiles, groups, P, next + gridDim.x, dn);
-    }
-    {
-      // the tile is put together in LDS and written once at the end, with full-width stores: scattered two-byte
-      // stores to memory cost one request each
-      uint4 *z = reinterpret_cast<uint4 *>(s_tile);
+  // written out in 16-byte pieces, consecutive threads consecutive pieces: every store instruction fills whole lines
+  if ((reinterpret_cast<uintptr_t>(dense) & 15u) == 0 && tile_base + (uint32_t)kFdTile <= n) {
+    constexpr int kPieces = (int)(kFdTile * sizeof(S) / 16);
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(s_tile);
+    u32x4 *dst = reinterpret_cast<u32x4 *>(dense + tile_base);
 #pragma unroll
-      for (int i = 0; i < (int)(kFdTile * sizeof(S) / 16) / kFdBlock; ++i) z[i * kFdBlock + threadIdx.x] = make_uint4(0, 0, 0, 0);
-    }
-    uint32_t total_bytes = s_meta[set][P].y;
-    // cannot be: the lists' members in a tile add up to its size at most
-    if (total_bytes > (uint32_t)kFdMaxBytes || s_meta[set][P].z > (uint32_t)kFdTile) {
-      total_bytes = 0;
-      bad = true;
-    }
-    const uint32_t total_vals = min(s_meta[set][P].w, (uint32_t)kFdValStage);
-#pragma unroll
-    for (int k = 0; k < kFdBytesPer; ++k) {
-      const uint32_t i = threadIdx.x + (uint32_t)k * kFdBlock;
-      if (i < total_bytes) {
-        // bits outside the list's range of this tile belong to other tiles (or to nobody)
-        const uint32_t lo = byte_list[k];
-        const uint4 m = s_meta[set][lo];
-        const uint32_t cnt = s_len[set][lo].x;
-        const uint32_t first_bit = ((m.x >> 3) + (i - m.y)) << 3;
-        uint32_t byte = byte_in[k];
-        if (first_bit < m.x) byte &= 0xffu << (m.x - first_bit);
-        if (first_bit + 8u > m.x + cnt) byte &= 0xffu >> (first_bit + 8u - (m.x + cnt));
-        s_bl[i] = (uint16_t)(byte | (lo << 8));
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kFdValsPer; ++k) {
-      const uint32_t i = threadIdx.x + (uint32_t)k * kFdBlock;
-      if (i < total_vals) s_val[i] = val_in[k];
-    }
-    __syncthreads();
-    if (next < tiles) fd_fetch_lists<S>(s_meta[set ^ 1], P, s_blut[set ^ 1], s_vlut[set ^ 1], s_bm, s_vs, bitmaps, values, byte_in, byte_list, val_in);
-    // every thread takes three consecutive bytes; the set bits in front of them by a prefix sum over the threads
-    uint32_t mine[kFdBytesPer], sum = 0;
-#pragma unroll
-    for (int k = 0; k < kFdBytesPer; ++k) {
-      const uint32_t i = threadIdx.x * kFdBytesPer + k;
-      mine[k] = i < total_bytes ? (uint32_t)s_bl[i] : 0u;
-      sum += (uint32_t)__popc(mine[k] & 0xffu);
-    }
-    uint32_t before_list = 0xffffu;  // the list of the byte in front of the thread's first
-    if (threadIdx.x > 0 && threadIdx.x * kFdBytesPer <= total_bytes) before_list = s_bl[threadIdx.x * kFdBytesPer - 1] >> 8;
-    uint32_t total_hits;
-    const uint32_t first_hit = block_exclusive_scan<uint32_t, kFdBlock>(sum, s_scan, &total_hits);
-    // The set bits, listed (kFdHitStage at a time) and then taken one per thread and turn: a thread that went
-    // through the bits of its own bytes to the end would keep a whole wave busy for as long as its fullest
-    // byte takes.
-    for (uint32_t hbase = 0; hbase < total_hits; hbase += kFdHitStage) {
-      {
-        uint32_t h = first_hit, prev = before_list;
-#pragma unroll
-        for (int k = 0; k < kFdBytesPer; ++k) {
-          const uint32_t i = threadIdx.x * kFdBytesPer + k;
-          if (i < total_bytes) {
-            const uint32_t p = mine[k] >> 8;
-            if (hbase == 0 && p != prev) s_front[p] = h;  // the bytes are masked: nothing set in front of the range inside its first byte
-            prev = p;
-            for (uint32_t bits = mine[k] & 0xffu; bits; bits &= bits - 1u, ++h)
-              if (h - hbase < (uint32_t)kFdHitStage) s_hit[h - hbase] = (p << 16) | (i << 3) | ((uint32_t)__ffs((int)bits) - 1u);
-          }
-        }
-      }
-      __syncthreads();
-      const uint32_t hend = min(total_hits, hbase + (uint32_t)kFdHitStage);
-      for (uint32_t h = hbase + threadIdx.x; h < hend; h += kFdBlock) {
-        const uint32_t ent = s_hit[h - hbase];
-        const uint32_t p = ent >> 16, i = (ent >> 3) & 0x1fffu, bit = ent & 7u;
-        const uint4 m = s_meta[set][p];
-        const uint4 ln = s_len[set][p];
-        const int64_t list_vals = s_vs[p + 1] - s_vs[p];
-        const uint32_t j = (((m.x >> 3) + (i - m.y)) << 3) + bit - m.x;  // member number inside the tile (below ln.x: the bytes are masked)
-        const uint32_t nth = h - s_front[p];                            // value number inside the tile's stretch
-        const uint32_t at = order[(size_t)tile_base + ln.z + j] & (uint32_t)(kFdTile - 1);
-        const uint32_t vl = m.w + nth;
-        if (nth < ln.y && (int64_t)m.z + nth < list_vals) {
-          const S v = vl < (uint32_t)kFdValStage ? s_val[vl] : values[s_vs[p] + m.z + nth];
-          s_tile[at] = fd_value<S>(v);
-        } else {
-          bad = true;  // more set bits than values
-        }
-      }
-      __syncthreads();
-    }
-    // written out in 16-byte pieces, consecutive threads consecutive pieces: every store instruction fills whole lines
-    if (aligned && tile_base + (uint32_t)kFdTile <= n) {
-      constexpr int kPieces = (int)(kFdTile * sizeof(S) / 16);
-      const uint4 *src = reinterpret_cast<const uint4 *>(s_tile);
-      uint4 *dst = reinterpret_cast<uint4 *>(dense + tile_base);
-#pragma unroll
-      for (int i = 0; i < kPieces / kFdBlock; ++i) dst[i * kFdBlock + threadIdx.x] = src[i * kFdBlock + threadIdx.x];
-    } else {
-      for (uint32_t e = threadIdx.x; e < (uint32_t)kFdTile && tile_base + e < n; e += kFdBlock) dense[tile_base + e] = s_tile[e];
-      __syncthreads();  // here the tile is cleared again by other threads than those that have just read it
-    }
+    for (int i = 0; i < kPieces / kFdBlock; ++i)
+      __builtin_nontemporal_store(src[i * kFdBlock + threadIdx.x], dst + i * kFdBlock + threadIdx.x);
+  } else {
+    for (uint32_t e = threadIdx.x; e < (uint32_t)kFdTile && tile_base + e < n; e += kFdBlock) dense[tile_base + e] = s_tile[e];
   }
-  if (bad) atomicOr(status, ZEN_STAT_BAD_INDEX);
+  if ((bad || odd) && lane == 0) atomicOr(status, ZEN_STAT_BAD_INDEX);
 }
 
 inline uint32_t fd_tiles(int64_t numel) { return (uint32_t)ceil_div(numel, kFdTile); }
 inline size_t fd_order_bytes(int64_t numel) { return (size_t)fd_tiles(numel) * kFdTile * sizeof(uint16_t); }
 inline size_t fd_table_bytes(int64_t numel, int P) { return align_up(((size_t)fd_tiles(numel) + 1) * P * sizeof(uint32_t), 256); }
-inline size_t fd_vstart_bytes(int64_t numel, int P) {
-  return align_up((size_t)fd_groups(fd_tiles(numel)) * kFdGroupRow * P * sizeof(uint32_t), 256);
-}
+inline size_t fd_vstart_bytes(int64_t numel, int P) { return align_up((size_t)fd_tiles(numel) * P * sizeof(uint32_t), 256); }
 inline size_t fd_gsum_bytes(int64_t numel, int P) { return align_up((size_t)fd_groups(fd_tiles(numel)) * P * sizeof(uint32_t), 256); }
-
-// Workgroups of the tile kernel that fit the device at once (it walks over the tiles with that many).
-int fd_resident_blocks(const void *fn, size_t lds) {
-  struct Known { const void *fn; size_t lds; int dev; int blocks; };
-  static std::mutex mu;
-  static Known known[8];
-  static int n_known = 0;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  std::lock_guard<std::mutex> lock(mu);
-  for (int i = 0; i < n_known; ++i)
-    if (known[i].fn == fn && known[i].lds == lds && known[i].dev == dev) return known[i].blocks;
-  int per_cu = 0, cus = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kFdBlock, lds) != hipSuccess || per_cu < 1) return 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) return 0;
-  const int blocks = per_cu * cus;
-  known[n_known < 8 ? n_known++ : 7] = Known{fn, lds, dev, blocks};
-  return blocks;
-}
 
 int fd_check(int64_t numel, int partitions) {
   if (numel <= 0 || numel > 0x7fffffffll || partitions < 1 || partitions > kFdMaxLists || numel / partitions == 0)
@@ -513,14 +368,14 @@ int zen_bitmap_dense_dict(int64_t numel, int partitions, void *dict, int64_t *me
     ZEN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fd_order), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   k_fd_order<<<dim3(tiles), dim3(kFdBlock), lds, s>>>((uint32_t)numel, (uint32_t)(numel / partitions), partitions, order, below);
   ZEN_LAUNCH_CHECK("k_fd_order");
-  k_fd_scan<<<dim3((unsigned)partitions), dim3(kFdScanBlock), 0, s>>>(below, tiles);
+  k_fd_scan<<<dim3((unsigned)partitions), dim3(kFdScanBlock), 0, s>>>(below, tiles, partitions);
   ZEN_LAUNCH_CHECK("k_fd_scan");
   if (members) {  // the list lengths, for a caller that sizes bitmaps without a mapping
     for (int p = 0; p < partitions; ++p) members[p] = 0;
     ZEN_HIP_CHECK(hipStreamSynchronize(s));
     uint32_t host[kFdMaxLists];
     for (int p = 0; p < partitions; ++p) {
-      ZEN_HIP_CHECK(hipMemcpy(&host[p], below + (size_t)p * (tiles + 1) + tiles, sizeof(uint32_t), hipMemcpyDeviceToHost));
+      ZEN_HIP_CHECK(hipMemcpy(&host[p], below + (size_t)tiles * partitions + p, sizeof(uint32_t), hipMemcpyDeviceToHost));
       members[p] = host[p];
     }
   }
@@ -532,26 +387,29 @@ size_t zen_bitmap_dense_workspace(int64_t numel, int partitions) {
   return zen::fd_vstart_bytes(numel, partitions) + zen::fd_gsum_bytes(numel, partitions);
 }
 
-int zen_bitmap_dense(const void *dict, int64_t numel, int partitions, const uint8_t *bitmaps,
-                     const int64_t *bitmap_start, const void *values, int dtype, const int64_t *value_start,
-                     void *dense, void *workspace, size_t workspace_bytes, int32_t *status, void *stream) {
+int zen_bitmap_dense_lists(const void *dict, int64_t numel, int partitions, const uint8_t *const *bitmaps,
+                           const int64_t *bitmap_bytes, const void *const *values, int dtype,
+                           const int64_t *value_count, void *dense, void *workspace, size_t workspace_bytes,
+                           int32_t *status, void *stream) {
   using namespace zen;
   const int rc = fd_check(numel, partitions);
   if (rc != ZEN_OK) return rc;
   if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_bitmap_dense: bad dtype");
-  if (!dict || !bitmap_start || !value_start || !dense || !workspace || !status)
+  if (!dict || !bitmaps || !bitmap_bytes || !values || !value_count || !dense || !workspace || !status)
     return fail(ZEN_EINVAL, "zen_bitmap_dense: null pointer");
   if (workspace_bytes < zen_bitmap_dense_workspace(numel, partitions))
     return fail(ZEN_EWORKSPACE, "zen_bitmap_dense: workspace too small");
-  ListStarts bm, vs;
-  for (int p = 0; p <= partitions; ++p) {
-    bm.at[p] = bitmap_start[p];
-    vs.at[p] = value_start[p];
-    if (p && (bm.at[p] < bm.at[p - 1] || vs.at[p] < vs.at[p - 1]))
-      return fail(ZEN_EINVAL, "zen_bitmap_dense: list offsets must not decrease");
+  FdLists lists{};
+  for (int p = 0; p < partitions; ++p) {
+    if (bitmap_bytes[p] < 0 || value_count[p] < 0) return fail(ZEN_EINVAL, "zen_bitmap_dense: negative length");
+    if ((bitmap_bytes[p] > 0 && !bitmaps[p]) || (value_count[p] > 0 && !values[p]))
+      return fail(ZEN_EINVAL, "zen_bitmap_dense: null pointer");
+    // what lies beyond the members a list can have is never looked at
+    lists.bitmap[p] = bitmaps[p];
+    lists.bytes[p] = (uint32_t)(bitmap_bytes[p] < (1ll << 28) ? bitmap_bytes[p] : 1ll << 28);
+    lists.val[p] = values[p];
+    lists.vals[p] = (uint32_t)(value_count[p] < (1ll << 31) ? value_count[p] : 1ll << 31);
   }
-  if ((bm.at[partitions] > bm.at[0] && !bitmaps) || (vs.at[partitions] > vs.at[0] && !values))
-    return fail(ZEN_EINVAL, "zen_bitmap_dense: null pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const uint16_t *order = static_cast<const uint16_t *>(dict);
   const uint32_t *below = reinterpret_cast<const uint32_t *>(static_cast<const uint8_t *>(dict) + fd_order_bytes(numel));
@@ -559,28 +417,43 @@ int zen_bitmap_dense(const void *dict, int64_t numel, int partitions, const uint
   uint32_t *gsum = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(workspace) + fd_vstart_bytes(numel, partitions));
   const uint32_t tiles = fd_tiles(numel);
   const uint32_t groups = fd_groups(tiles);
-  const size_t lds = 0;
-  const void *fn = dtype == ZEN_BF16 ? reinterpret_cast<const void *>(&k_fd_tiles<uint16_t>)
-                                     : reinterpret_cast<const void *>(&k_fd_tiles<uint32_t>);
-  const int resident = fd_resident_blocks(fn, lds);
-  if (resident < 1) return fail(ZEN_EHIP, "zen_bitmap_dense: the tile kernel does not fit the device");
-  const uint32_t grid = tiles < (uint32_t)resident ? tiles : (uint32_t)resident;
   ProfScope prof(kProfDecodeFused, s);
-  k_fd_count<<<dim3(groups, (unsigned)partitions), dim3(kFdGroup), 0, s>>>(below, tiles, partitions, bitmaps, bm, vstart, gsum,
+  k_fd_count<<<dim3(groups, (unsigned)partitions), dim3(kFdGroup), 0, s>>>(below, tiles, partitions, lists, vstart, gsum,
                                                                        status);
   ZEN_LAUNCH_CHECK("k_fd_count");
-  k_fd_groups<<<dim3((unsigned)partitions), dim3(kFdGroupsMax), 0, s>>>(gsum, groups);
+  k_fd_groups<<<dim3((unsigned)partitions), dim3(kFdGroupsMax), 0, s>>>(gsum, groups, partitions);
   ZEN_LAUNCH_CHECK("k_fd_groups");
   if (dtype == ZEN_BF16)
-    k_fd_tiles<uint16_t><<<dim3(grid), dim3(kFdBlock), 0, s>>>(order, below, vstart, gsum, tiles, partitions, (uint32_t)numel,
-                                                                bitmaps, bm, static_cast<const uint16_t *>(values), vs,
-                                                                static_cast<uint16_t *>(dense), status);
+    k_fd_tiles<uint16_t><<<dim3(tiles), dim3(kFdBlock), 0, s>>>(order, below, vstart, gsum, partitions, (uint32_t)numel,
+                                                                lists, static_cast<uint16_t *>(dense), status);
   else
-    k_fd_tiles<uint32_t><<<dim3(grid), dim3(kFdBlock), 0, s>>>(order, below, vstart, gsum, tiles, partitions, (uint32_t)numel,
-                                                                bitmaps, bm, static_cast<const uint32_t *>(values), vs,
-                                                                static_cast<uint32_t *>(dense), status);
+    k_fd_tiles<uint32_t><<<dim3(tiles), dim3(kFdBlock), 0, s>>>(order, below, vstart, gsum, partitions, (uint32_t)numel,
+                                                                lists, static_cast<uint32_t *>(dense), status);
   ZEN_LAUNCH_CHECK("k_fd_tiles");
   return ZEN_OK;
+}
+
+int zen_bitmap_dense(const void *dict, int64_t numel, int partitions, const uint8_t *bitmaps,
+                     const int64_t *bitmap_start, const void *values, int dtype, const int64_t *value_start,
+                     void *dense, void *workspace, size_t workspace_bytes, int32_t *status, void *stream) {
+  using namespace zen;
+  const int rc = fd_check(numel, partitions);
+  if (rc != ZEN_OK) return rc;
+  if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_bitmap_dense: bad dtype");
+  if (!bitmap_start || !value_start) return fail(ZEN_EINVAL, "zen_bitmap_dense: null pointer");
+  const uint8_t *bitmap_at[kFdMaxLists];
+  const void *value_at[kFdMaxLists];
+  int64_t bytes[kFdMaxLists], vals[kFdMaxLists];
+  for (int p = 0; p < partitions; ++p) {
+    bytes[p] = bitmap_start[p + 1] - bitmap_start[p];
+    vals[p] = value_start[p + 1] - value_start[p];
+    if (bytes[p] < 0 || vals[p] < 0) return fail(ZEN_EINVAL, "zen_bitmap_dense: list offsets must not decrease");
+    if ((bytes[p] > 0 && !bitmaps) || (vals[p] > 0 && !values)) return fail(ZEN_EINVAL, "zen_bitmap_dense: null pointer");
+    bitmap_at[p] = bitmaps + bitmap_start[p];
+    value_at[p] = static_cast<const char *>(values) + value_start[p] * (dtype == ZEN_BF16 ? 2 : 4);
+  }
+  return zen_bitmap_dense_lists(dict, numel, partitions, bitmap_at, bytes, value_at, dtype, vals, dense, workspace,
+                                workspace_bytes, status, stream);
 }
 
 }  // extern "C"

@@ -40,10 +40,10 @@ __global__ __launch_bounds__(256) void k_merge_prep(const I *__restrict__ idx, c
 // memory by the thread that owns its head.
 __device__ inline int mrg_slot(int i) { return i + (i >> 4); }  // one pad word per 16: conflict-free strides
 
-template <typename I>
+template <typename I, typename O>
 __global__ __launch_bounds__(kMrgBlock) void k_merge_reduce(
     const uint32_t *__restrict__ keys, const uint32_t *__restrict__ perm, uint32_t r,
-    uint32_t dense_n, I *__restrict__ out_idx, float *__restrict__ out_val, int64_t capacity,
+    uint32_t dense_n, I *__restrict__ out_idx, O *__restrict__ out_val, int64_t capacity,
     ScanState st, int ntiles, int64_t *out_count, int32_t *status) {
   __shared__ uint32_t s_scan[kMrgBlock / 64 + 1];
   __shared__ uint64_t s_bcast;
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kMrgBlock) void k_merge_reduce(
         for (uint32_t g = tile_base + kMrgTile; g < r && keys[g] == k[q]; ++g)
           acc += __uint_as_float(perm[g]);
       sum[q] = acc;
-      if (acc != 0.0f) keep |= 1u << q;  // torch.nonzero keeps NaN, drops +-0
+      if (SumAs<O>::kept(acc)) keep |= 1u << q;
     }
   }
   uint32_t total;
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kMrgBlock) void k_merge_reduce(
     const uint64_t pos = tile_start + i;
     if (pos < (uint64_t)capacity) {
       out_idx[pos] = (I)s_key[i];
-      out_val[pos] = s_val[i];
+      out_val[pos] = SumAs<O>::of(s_val[i]);
     }
   }
 }
@@ -201,14 +201,14 @@ struct MergeSink {
   }
 };
 
-template <typename I, typename S>
+template <typename I, typename S, typename O>
 __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, uint32_t *__restrict__ cursor,
                                                              uint32_t *__restrict__ coarse_cursor,
                                                              const uint32_t *__restrict__ bucket_lo,
                                                              const uint32_t *__restrict__ slab_idx,
                                                              const uint32_t *__restrict__ slab_arr,
                                                              const S *__restrict__ slab_val,
-                                                             I *__restrict__ out_idx, float *__restrict__ out_val,
+                                                             I *__restrict__ out_idx, O *__restrict__ out_val,
                                                              int64_t capacity, ScanState st, int tie_bits,
                                                              int64_t *out_count, int32_t *status) {
   __shared__ SlabSortSharedT<true> sh;  // the values take the counters' place once the ranks are known
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
         acc += v[q];
         prev = k[q];
         sum[q] = acc;
-        if (k[q] != next && acc != 0.0f) keep |= 1u << q;  // torch.nonzero keeps NaN, drops +-0
+        if (k[q] != next && SumAs<O>::kept(acc)) keep |= 1u << q;
       } else {
         sum[q] = 0.0f;
       }
@@ -374,7 +374,7 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
     const uint64_t pos = tile_start + i;
     if (pos < (uint64_t)capacity) {
       out_idx[pos] = (I)sh.key[i];
-      out_val[pos] = __uint_as_float(sh.tie[i]);
+      out_val[pos] = SumAs<O>::of(__uint_as_float(sh.tie[i]));
     }
   }
   // every workgroup has read the descriptors it needs before it gets here
@@ -436,9 +436,9 @@ bool slab_merge_fits(int64_t r, int64_t dense_n, SlabGeom *geo) {
   return true;
 }
 
-template <typename I, typename S>
+template <typename I, typename S, typename O>
 int slab_merge_launch(const SlabGeom &geo, const I *idx, const S *val, int64_t r, int64_t dense_n, void *out_idx,
-                      int idx64_out, float *out_val, int64_t capacity, int64_t *out_count, void *workspace,
+                      int idx64_out, O *out_val, int64_t capacity, int64_t *out_count, void *workspace,
                       bool zeroed, int32_t *status, hipStream_t s) {
   const SlabMergePlan p = plan_slab_merge(workspace, geo, r);
   if (!zeroed) {
@@ -456,12 +456,12 @@ int slab_merge_launch(const SlabGeom &geo, const I *idx, const S *val, int64_t r
   const int tie_bits = ceil_log2_u64((uint64_t)r);  // arrival numbers are < r
   ProfScope prof(kProfMergeBucket, s);
   if (idx64_out)
-    k_merge_bucket<int64_t, S><<<dim3(geo.nbuckets), dim3(kMergeBlock), 0, s>>>(
+    k_merge_bucket<int64_t, S, O><<<dim3(geo.nbuckets), dim3(kMergeBlock), 0, s>>>(
         geo, p.feed.cursor, p.feed.coarse_cursor, p.feed.bucket_lo, p.slab_idx, p.slab_arr,
         static_cast<const S *>(p.slab_val), static_cast<int64_t *>(out_idx), out_val, capacity, st, tie_bits, out_count,
         status);
   else
-    k_merge_bucket<int32_t, S><<<dim3(geo.nbuckets), dim3(kMergeBlock), 0, s>>>(
+    k_merge_bucket<int32_t, S, O><<<dim3(geo.nbuckets), dim3(kMergeBlock), 0, s>>>(
         geo, p.feed.cursor, p.feed.coarse_cursor, p.feed.bucket_lo, p.slab_idx, p.slab_arr,
         static_cast<const S *>(p.slab_val), static_cast<int32_t *>(out_idx), out_val, capacity, st, tie_bits, out_count,
         status);
@@ -500,15 +500,22 @@ MergePlan plan_merge(void *workspace, int64_t r, int64_t dense_n) {
   return p;
 }
 
-template <typename S>
+// Whether a call with these sizes goes to the wide buckets.
+bool takes_wide(int64_t r, int64_t dense_n, int mode) {
+  return (mode & ~ZEN_MODE_ZEROED) == ZEN_MODE_FAST && wide_merge_fits(r, dense_n, wide_device_cus(), nullptr);
+}
+
+// O: float (the fp32 sums) or uint16_t (rounded once to bf16).  out_idx == nullptr: out_val is the dense tensor,
+// written whole (on the wide buckets only: takes_wide).
+template <typename S, typename O>
 int merge_launch(const void *idx, int idx64_in, const S *val, int64_t r, int64_t dense_n, void *out_idx,
-                 int idx64_out, float *out_val, int64_t capacity, int64_t *out_count, int mode, void *workspace,
+                 int idx64_out, O *out_val, int64_t capacity, int64_t *out_count, int mode, void *workspace,
                  int32_t *status, hipStream_t s) {
   const bool zeroed = (mode & ZEN_MODE_ZEROED) != 0;
-  const bool slabs_only = (mode & ZEN_MODE_SLABS) != 0;
+  const bool wide = takes_wide(r, dense_n, mode);
   mode &= ~(ZEN_MODE_ZEROED | ZEN_MODE_SLABS);
   SlabGeom geo;
-  if (mode == ZEN_MODE_FAST && !slabs_only && wide_merge_fits(r, dense_n, wide_device_cus(), nullptr)) {
+  if (wide) {
     // the zero region at the head of the workspace: the prefix state first, the cursors behind it
     Carver cv(workspace);
     unsigned long long *scan = cv.take<unsigned long long>(scan_words((int64_t)kSlabMaxBuckets));
@@ -521,8 +528,8 @@ int merge_launch(const void *idx, int idx64_in, const S *val, int64_t r, int64_t
     if (!wide_merge_list(idx, idx64_in, val, r, dense_n, cursor, static_cast<char *>(workspace) + kMergeZeroBytes,
                          wide_device_cus(), status, &list))
       return fail(ZEN_EINVAL, "zen_merge: sizes do not suit the wide buckets");
-    return wide_merge(list, sizeof(S) == 2 ? ZEN_BF16 : ZEN_F32, false, out_idx, idx64_out, out_val, capacity, out_count,
-                      scan, s);
+    return wide_merge(list, sizeof(S) == 2 ? ZEN_BF16 : ZEN_F32, out_idx, idx64_out, out_val,
+                      sizeof(O) == 2 ? ZEN_BF16 : ZEN_F32, capacity, out_count, scan, s);
   }
   if (mode == ZEN_MODE_FAST && slab_merge_fits(r, dense_n, &geo)) {
     if (idx64_in)
@@ -563,11 +570,11 @@ int merge_launch(const void *idx, int idx64_in, const S *val, int64_t r, int64_t
   const ScanState st = scan_state(p.scan, p.ntiles);
   ProfScope prof(kProfMergeReduce, s);
   if (idx64_out)
-    k_merge_reduce<int64_t><<<dim3((unsigned)p.ntiles), dim3(kMrgBlock), 0, s>>>(
+    k_merge_reduce<int64_t, O><<<dim3((unsigned)p.ntiles), dim3(kMrgBlock), 0, s>>>(
         sk, sp, (uint32_t)r, (uint32_t)dense_n, static_cast<int64_t *>(out_idx), out_val, capacity, st, p.ntiles,
         out_count, status);
   else
-    k_merge_reduce<int32_t><<<dim3((unsigned)p.ntiles), dim3(kMrgBlock), 0, s>>>(
+    k_merge_reduce<int32_t, O><<<dim3((unsigned)p.ntiles), dim3(kMrgBlock), 0, s>>>(
         sk, sp, (uint32_t)r, (uint32_t)dense_n, static_cast<int32_t *>(out_idx), out_val, capacity, st, p.ntiles,
         out_count, status);
   ZEN_LAUNCH_CHECK("k_merge_reduce");
@@ -610,9 +617,13 @@ int zen_merge_path(int64_t r, int64_t dense_n, int mode) {
   return zen::bucket_sort_fits(r, (uint32_t)dense_n) ? 1 : 0;
 }
 
-int zen_merge(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n, void *out_idx,
-              int idx64_out, float *out_val, int64_t capacity, int64_t *out_count, int mode, void *workspace,
-              size_t workspace_bytes, int32_t *status, void *stream) {
+}  // extern "C"
+
+namespace {
+
+int merge_call(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n, void *out_idx,
+               int idx64_out, void *out_val, bool round, int64_t capacity, int64_t *out_count, int mode,
+               void *workspace, size_t workspace_bytes, int32_t *status, void *stream) {
   using namespace zen;
   const char *why = "";
   if (merge_check(idx, val, dtype, r, dense_n, mode, &why) != ZEN_OK) return fail(ZEN_EINVAL, why);
@@ -625,18 +636,39 @@ int zen_merge(const void *idx, int idx64_in, const void *val, int dtype, int64_t
   }
   if (!workspace || (capacity > 0 && (!out_idx || !out_val))) return fail(ZEN_EINVAL, "zen_merge: null pointer");
   if (workspace_bytes < zen_merge_workspace(r, dense_n)) return fail(ZEN_EWORKSPACE, "zen_merge: workspace too small");
+  if (dtype == ZEN_BF16 && round)
+    return merge_launch(idx, idx64_in, static_cast<const uint16_t *>(val), r, dense_n, out_idx, idx64_out,
+                        static_cast<uint16_t *>(out_val), capacity, out_count, mode, workspace, status, s);
   if (dtype == ZEN_BF16)
-    return merge_launch(idx, idx64_in, static_cast<const uint16_t *>(val), r, dense_n, out_idx, idx64_out, out_val,
-                        capacity, out_count, mode, workspace, status, s);
-  return merge_launch(idx, idx64_in, static_cast<const uint32_t *>(val), r, dense_n, out_idx, idx64_out, out_val,
-                      capacity, out_count, mode, workspace, status, s);
+    return merge_launch(idx, idx64_in, static_cast<const uint16_t *>(val), r, dense_n, out_idx, idx64_out,
+                        static_cast<float *>(out_val), capacity, out_count, mode, workspace, status, s);
+  return merge_launch(idx, idx64_in, static_cast<const uint32_t *>(val), r, dense_n, out_idx, idx64_out,
+                      static_cast<float *>(out_val), capacity, out_count, mode, workspace, status, s);
+}
+
+}  // namespace
+
+extern "C" {
+
+int zen_merge(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n, void *out_idx,
+              int idx64_out, float *out_val, int64_t capacity, int64_t *out_count, int mode, void *workspace,
+              size_t workspace_bytes, int32_t *status, void *stream) {
+  return merge_call(idx, idx64_in, val, dtype, r, dense_n, out_idx, idx64_out, out_val, false, capacity, out_count,
+                    mode, workspace, workspace_bytes, status, stream);
+}
+
+int zen_merge_rounded(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n,
+                      void *out_idx, int idx64_out, void *out_val, int64_t capacity, int64_t *out_count, int mode,
+                      void *workspace, size_t workspace_bytes, int32_t *status, void *stream) {
+  return merge_call(idx, idx64_in, val, dtype, r, dense_n, out_idx, idx64_out, out_val, true, capacity, out_count,
+                    mode, workspace, workspace_bytes, status, stream);
 }
 
 size_t zen_decode_dense_workspace(int64_t r, int64_t dense_n) {
   if (r < 0 || dense_n <= 0) return 0;
   const size_t cap = (size_t)(r > 0 ? r : 1);
   return zen::align_up(cap * sizeof(int32_t), 256) + zen::align_up(cap * sizeof(float), 256) + 256 +
-         zen_merge_workspace(r, dense_n);
+         zen::align_up(zen_merge_workspace(r, dense_n), 256);
 }
 
 int zen_decode_dense(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, void *dense,
@@ -647,27 +679,36 @@ int zen_decode_dense(const void *idx, int idx64_in, const void *val, int dtype, 
   if (merge_check(idx, val, dtype, r, dense_n, mode, &why) != ZEN_OK) return fail(ZEN_EINVAL, why);
   if (!dense || !status) return fail(ZEN_EINVAL, "zen_decode_dense: null pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // the zero region zen_merge wants is at the head of this call's workspace too
+  Carver cv(workspace);
+  void *inner = cv.take<char>(zen_merge_workspace(r, dense_n));
+  const bool whole = r > 0 && takes_wide(r, dense_n, mode);  // the merge writes the dense tensor, zeros included
+  if (r > 0 && !workspace) return fail(ZEN_EINVAL, "zen_decode_dense: null pointer");
+  if (r > 0 && workspace_bytes < zen_decode_dense_workspace(r, dense_n))
+    return fail(ZEN_EWORKSPACE, "zen_decode_dense: workspace too small");
+  if (whole) {
+    if (dtype == ZEN_BF16)
+      return merge_launch(idx, idx64_in, static_cast<const uint16_t *>(val), r, dense_n, nullptr, 0,
+                          static_cast<uint16_t *>(dense), r, nullptr, mode, inner, status, s);
+    return merge_launch(idx, idx64_in, static_cast<const uint32_t *>(val), r, dense_n, nullptr, 0,
+                        static_cast<float *>(dense), r, nullptr, mode, inner, status, s);
+  }
   if (dtype == ZEN_BF16)
     launch_fill<uint16_t>(static_cast<uint16_t *>(dense), (uint16_t)0, (size_t)dense_n, s);
   else
     launch_fill<uint32_t>(static_cast<uint32_t *>(dense), 0u, (size_t)dense_n, s);
   ZEN_LAUNCH_CHECK("zen_decode_dense: clear");
   if (r == 0) return ZEN_OK;
-  if (!workspace) return fail(ZEN_EINVAL, "zen_decode_dense: null pointer");
-  if (workspace_bytes < zen_decode_dense_workspace(r, dense_n))
-    return fail(ZEN_EWORKSPACE, "zen_decode_dense: workspace too small");
-  Carver cv(workspace);
   int32_t *m_idx = cv.take<int32_t>((size_t)r);
   float *m_val = cv.take<float>((size_t)r);
   int64_t *m_count = cv.take<int64_t>(1);
-  void *inner = cv.take<char>(zen_merge_workspace(r, dense_n));
   int rc;
   if (dtype == ZEN_BF16)
-    rc = merge_launch(idx, idx64_in, static_cast<const uint16_t *>(val), r, dense_n, m_idx, 0, m_val, r, m_count,
-                      mode & ~ZEN_MODE_ZEROED, inner, status, s);
+    rc = merge_launch(idx, idx64_in, static_cast<const uint16_t *>(val), r, dense_n, m_idx, 0, m_val, r, m_count, mode,
+                      inner, status, s);
   else
-    rc = merge_launch(idx, idx64_in, static_cast<const uint32_t *>(val), r, dense_n, m_idx, 0, m_val, r, m_count,
-                      mode & ~ZEN_MODE_ZEROED, inner, status, s);
+    rc = merge_launch(idx, idx64_in, static_cast<const uint32_t *>(val), r, dense_n, m_idx, 0, m_val, r, m_count, mode,
+                      inner, status, s);
   if (rc != ZEN_OK) return rc;
   const unsigned blocks = (unsigned)ceil_div(r, 256);
   if (dtype == ZEN_BF16)

@@ -694,7 +694,6 @@ int select_compact(const SelectArgs &a, hipStream_t stream) {
 
 constexpr int kScatStage = 2048;
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <typename S, bool ALIGNED>
 __device__ inline void stage_load(const S *__restrict__ in, int64_t n, int64_t sub_base, uint4 (&q)[kSelVecs]) {

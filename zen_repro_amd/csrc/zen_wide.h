@@ -288,7 +288,7 @@ bool wide_merge_fits(int64_t r, int64_t dense_n, int cus, SlabGeom *geo);
 size_t wide_merge_bytes(int64_t r, int64_t dense_n, int cus);
 bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, int64_t dense_n, uint32_t *cursor,
                      void *rest, int cus, int32_t *status, WideList *list);
-int wide_merge(const WideList &list, int dtype, bool scattered, void *out_idx, int idx64_out, float *out_val,
+int wide_merge(const WideList &list, int dtype, void *out_idx, int idx64_out, void *out_val, int out_dtype,
                int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s);
 
 }  // namespace zen

@@ -61,11 +61,14 @@ struct WideMergeShared {
   int tile;
 };
 
-template <typename I, typename S>
+// O: what is written for a sum (zen_common.h).  DENSE: out_val is the dense tensor [0, dense_n); the workgroup
+// writes its bucket's range of it whole: zeros while its records are on their way (62 M bf16 elements: the fill
+// and scatter kernels in front of and behind a sparse merge took 18 + 21 us), the sums behind them at the end.
+template <typename I, typename S, typename O, bool DENSE>
 __global__ __launch_bounds__(kWideBlock) void k_wide_merge(SlabGeom geo, WideSlabs in, I *__restrict__ out_idx,
-                                                           float *__restrict__ out_val, int64_t capacity,
+                                                           O *__restrict__ out_val, int64_t capacity,
                                                            ScanState st, int tie_bits, int64_t *out_count,
-                                                           int32_t *status) {
+                                                           uint32_t dense_n, int32_t *status) {
   __shared__ WideMergeShared sh;
   const uint32_t tid = threadIdx.x;
   if (tid == 0) {
@@ -78,6 +81,20 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(SlabGeom geo, WideSla
   const uint32_t nb = geo.nbuckets;
   if (b >= nb) return;
   const uint32_t lo = geo.first_key(b);
+  if (DENSE) {
+    constexpr uint32_t V = 16 / sizeof(O);
+    const uint32_t end = b + 1 < nb ? geo.first_key(b + 1) : dense_n;
+    // the first multiple of 16 bytes in the range, as an element number of the range
+    const uint32_t skew = (uint32_t)((reinterpret_cast<uintptr_t>(out_val + lo) & 15u) / sizeof(O));
+    uint32_t head = (V - skew) % V;
+    if (head > end - lo) head = end - lo;
+    const uint32_t vecs = (end - lo - head) / V;
+    u32x4 *wide = reinterpret_cast<u32x4 *>(out_val + lo + head);
+    const u32x4 zero = {0, 0, 0, 0};
+    for (uint32_t i = tid; i < vecs; i += kWideBlock) wide[i] = zero;
+    for (uint32_t i = tid; i < head; i += kWideBlock) out_val[lo + i] = O(0);
+    for (uint32_t i = lo + head + vecs * V + tid; i < end; i += kWideBlock) out_val[i] = O(0);
+  }
   uint32_t pcount[kWideSplit];
   uint32_t longest = 0;
 #pragma unroll
@@ -308,19 +325,20 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(SlabGeom geo, WideSla
         acc += v[q];
         prev = k[q];
         sum[q] = acc;
-        if (k[q] != next && acc != 0.0f) keep |= 1u << q;  // torch.nonzero keeps NaN, drops +-0
+        if (k[q] != next && (DENSE ? acc != 0.0f : SumAs<O>::kept(acc))) keep |= 1u << q;
       } else {
         sum[q] = 0.0f;
       }
     }
   }
+  if (DENSE) wait_global_acks();  // this wave's zeros are written (the scan's barrier: everybody's)
   uint32_t total;
   const uint32_t before = block_exclusive_scan<uint32_t, kWideBlock>((uint32_t)__popc(keep), sh.scan, &total);
   // where this bucket's output starts: the sum of what all earlier buckets keep.  Every thread asks for one of
   // them (bounded wait), nobody waits for a chain of prefixes; while the answers are on their way the kept
   // entries are gathered in LDS (everybody is past reading the sorted bucket: the scan synchronised).
-  if (tid == 0) desc_store(&st.desc[b], kDescAggregate | total);
-  uint64_t d = tid < b ? desc_load(&st.desc[tid]) : kDescAggregate;
+  if (!DENSE && tid == 0) desc_store(&st.desc[b], kDescAggregate | total);
+  uint64_t d = !DENSE && tid < b ? desc_load(&st.desc[tid]) : kDescAggregate;
   uint32_t li = before;
 #pragma unroll
   for (int q = 0; q < kWmSumItems; ++q) {
@@ -341,18 +359,23 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(SlabGeom geo, WideSla
       d = desc_load(&st.desc[tid]);
     }
   }
-  uint64_t all_before;
-  block_exclusive_scan<uint64_t, kWideBlock>(d & kDescValue, sh.scan64, &all_before);  // its barriers also publish the gathered entries
-  if (b == nb - 1 && tid == 0) {
-    const uint64_t all = all_before + total;
-    *out_count = (int64_t)all;
-    if (all > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
-  }
-  for (uint32_t i = tid; i < total; i += kWideBlock) {
-    const uint64_t pos = all_before + i;
-    if (pos < (uint64_t)capacity) {
-      out_idx[pos] = (I)sh.key[i];
-      out_val[pos] = sh.val[i];
+  if (DENSE) {
+    __syncthreads();  // the gathered entries are there
+    for (uint32_t i = tid; i < total; i += kWideBlock) out_val[sh.key[i]] = SumAs<O>::of(sh.val[i]);
+  } else {
+    uint64_t all_before;
+    block_exclusive_scan<uint64_t, kWideBlock>(d & kDescValue, sh.scan64, &all_before);  // its barriers also publish the gathered entries
+    if (b == nb - 1 && tid == 0) {
+      const uint64_t all = all_before + total;
+      *out_count = (int64_t)all;
+      if (all > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
+    }
+    for (uint32_t i = tid; i < total; i += kWideBlock) {
+      const uint64_t pos = all_before + i;
+      if (pos < (uint64_t)capacity) {
+        out_idx[pos] = (I)sh.key[i];
+        out_val[pos] = SumAs<O>::of(sh.val[i]);
+      }
     }
   }
   // every workgroup has read the descriptors it needs before it gets here: the last one to finish clears the
@@ -418,11 +441,31 @@ bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, 
 
 uint32_t wide_scatter_batches(const WideList &list, int batch) { return (uint32_t)ceil_div((int64_t)list.r, batch); }
 
-// The two launches (one if the entries are in the buckets' slabs already: `scattered`).  scan: zeroed prefix
-// state for 256 buckets (descriptors, ticket, finished count), zero again when the launch ends.
-int wide_merge(const WideList &list, int dtype, bool scattered, void *out_idx, int idx64_out, float *out_val,
+template <typename S, typename O>
+static void wide_merge_launch(const WideList &list, void *out_idx, int idx64_out, O *out_val, int64_t capacity,
+                              int64_t *out_count, unsigned long long *scan, hipStream_t s) {
+  const ScanState st = scan_state(scan, (int64_t)list.geo.nbuckets);
+  const int tie_bits = ceil_log2_u64((uint64_t)list.r);  // arrival numbers are < r
+  const dim3 grid(list.geo.nbuckets), block(kWideBlock);
+  if (!out_idx)
+    k_wide_merge<int32_t, S, O, true><<<grid, block, 0, s>>>(list.geo, list.out, nullptr, out_val, capacity, st, tie_bits,
+                                                             out_count, list.dense_n, list.status);
+  else if (idx64_out)
+    k_wide_merge<int64_t, S, O, false><<<grid, block, 0, s>>>(list.geo, list.out, static_cast<int64_t *>(out_idx),
+                                                              out_val, capacity, st, tie_bits, out_count, list.dense_n,
+                                                              list.status);
+  else
+    k_wide_merge<int32_t, S, O, false><<<grid, block, 0, s>>>(list.geo, list.out, static_cast<int32_t *>(out_idx),
+                                                              out_val, capacity, st, tie_bits, out_count, list.dense_n,
+                                                              list.status);
+}
+
+// The two launches.  scan: zeroed prefix state for 256 buckets (descriptors, ticket, finished count), zero again
+// when the second ends.  out_dtype: ZEN_F32 (the sums; the only choice for fp32 values) or ZEN_BF16 (rounded).
+// out_idx == nullptr: out_val is the dense tensor.
+int wide_merge(const WideList &list, int dtype, void *out_idx, int idx64_out, void *out_val, int out_dtype,
                int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s) {
-  if (!scattered) {
+  {
     ProfScope prof(kProfWideScatter, s);
     if (dtype == ZEN_BF16)
       k_wide_scatter<uint16_t><<<dim3(wide_scatter_batches(list, kWsBatch)), dim3(kWsBlock), 0, s>>>(list);
@@ -430,25 +473,13 @@ int wide_merge(const WideList &list, int dtype, bool scattered, void *out_idx, i
       k_wide_scatter<uint32_t><<<dim3(wide_scatter_batches(list, kWsBatch)), dim3(kWsBlock), 0, s>>>(list);
     ZEN_LAUNCH_CHECK("k_wide_scatter");
   }
-  const ScanState st = scan_state(scan, (int64_t)list.geo.nbuckets);
-  const int tie_bits = ceil_log2_u64((uint64_t)list.r);  // arrival numbers are < r
   ProfScope prof(kProfWideMerge, s);
-  const dim3 grid(list.geo.nbuckets), block(kWideBlock);
-  if (dtype == ZEN_BF16) {
-    if (idx64_out)
-      k_wide_merge<int64_t, uint16_t><<<grid, block, 0, s>>>(list.geo, list.out, static_cast<int64_t *>(out_idx), out_val,
-                                                             capacity, st, tie_bits, out_count, list.status);
-    else
-      k_wide_merge<int32_t, uint16_t><<<grid, block, 0, s>>>(list.geo, list.out, static_cast<int32_t *>(out_idx), out_val,
-                                                             capacity, st, tie_bits, out_count, list.status);
-  } else {
-    if (idx64_out)
-      k_wide_merge<int64_t, uint32_t><<<grid, block, 0, s>>>(list.geo, list.out, static_cast<int64_t *>(out_idx), out_val,
-                                                             capacity, st, tie_bits, out_count, list.status);
-    else
-      k_wide_merge<int32_t, uint32_t><<<grid, block, 0, s>>>(list.geo, list.out, static_cast<int32_t *>(out_idx), out_val,
-                                                             capacity, st, tie_bits, out_count, list.status);
-  }
+  if (dtype == ZEN_F32)
+    wide_merge_launch<uint32_t>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s);
+  else if (out_dtype == ZEN_BF16)
+    wide_merge_launch<uint16_t>(list, out_idx, idx64_out, static_cast<uint16_t *>(out_val), capacity, out_count, scan, s);
+  else
+    wide_merge_launch<uint16_t>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s);
   ZEN_LAUNCH_CHECK("k_wide_merge");
   return ZEN_OK;
 }
