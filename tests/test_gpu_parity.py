@@ -834,3 +834,26 @@ def test_sample_threshold_at_the_edges_of_its_kernels(zen, oracle, s, dtype, kin
         thr, status = C.sample_threshold(to_dev(g), torch.from_numpy(at).cuda(), k)
         key, count = (int(x) & 0xFFFFFFFF for x in to_np(thr))
         assert int(status) == 0 and key == int(order[k - 1]) and count == int((keys >= key).sum()), (k, kind)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("n", [1, 511, 65536, 65537, 300001, 8192 * 2048 + 5])
+@pytest.mark.parametrize("density", [0.01, 0.125, 0.6])
+def test_ordered_compaction_at_the_edges_of_its_kernels(zen, oracle, n, dtype, density):
+    """One workgroup (up to 65536 elements) and a stretch per wave; fewer entries than an eighth of a stretch, about
+    that many (stretches on either side of it) and more; an aligned and an unaligned tensor; too little room."""
+    from zen_repro_amd.comm import _select_raw
+    from zen_repro_amd import _lib
+
+    g = make_grad(oracle, n + 1, density, dtype, seed=n)
+    keys = (g & 0x7FFF) if dtype == "bf16" else (g.view(np.uint32) & 0x7FFFFFFF)
+    d = to_dev(g)
+    for shift in (0, 1):
+        want = np.flatnonzero(keys[shift:])
+        idx, val, count, bits = _select_raw(d[shift:], None, True)
+        assert bits == 0 and count == want.size
+        assert np.array_equal(to_np(idx), want) and np.array_equal(to_np(val), to_np(to_dev(g[shift:][want])))
+        room = want.size // 2
+        idx, val, count, bits = _select_raw(d[shift:], None, False, capacity=room)
+        assert count == want.size and bits == (_lib.STAT_CAPACITY if want.size > room else 0)
+        assert np.array_equal(to_np(idx), want[:room])

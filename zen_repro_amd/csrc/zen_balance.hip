@@ -265,7 +265,7 @@ BalancePlan plan_balance(void *workspace, int64_t n, int64_t m, int dtype, int64
   p.thr = cv.take<uint32_t>(4);
   p.cand_hist = cv.take<uint32_t>((size_t)kCandHistWords);
   p.topk_scratch = cv.take<char>(topk_scratch_bytes());
-  p.select_scratch = cv.take<char>(select_scratch_bytes(n, dtype));
+  p.select_scratch = cv.take<char>(select_scratch_bytes());
   p.sort_scratch = cv.take<char>(sort_scratch_bytes((int64_t)cap));
   // m + P + 1 <= 2 m + 1 bounds the final-position keys whatever the partition count
   p.resolve_scratch = cv.take<char>(resolve_scratch_bytes((int64_t)cap, 2ull * (uint64_t)m + 1));
@@ -288,7 +288,6 @@ int select_stage(const BalancePlan &p, const void *input, int dtype, int64_t n, 
   sel.out_val = p.sel_val;
   sel.capacity = list_capacity(capacity);
   sel.out_count32 = &p.count[0];
-  sel.ordered = false;  // the sort below fixes the order
   sel.scratch = p.select_scratch;
   sel.status = status;
   *filter = nullptr;

@@ -1,0 +1,337 @@
+// Ordered compaction of a dense tensor: ascending indices and values of the selected elements (zen_select;
+// encode_sparse_tensor, comm.py:47-50).
+//
+// The tensor is cut into one stretch per wave.  A wave walks its stretch on its own, with no barrier and nobody to
+// wait for, and leaves what it selects side by side in a part of the workspace that is its own (k_compact_walk);
+// a second kernel sums up the counts in front of every stretch and moves the entries to their places
+// (k_compact_move).  A stretch with more than an eighth of its elements selected does not fit its part: the second
+// kernel walks it again and writes it straight to its place.  Up to kOneMax elements one workgroup does both steps
+// in one launch.
+// Bound by the read of the tensor and the extraction of what is selected (62 M bf16 elements, 4.4 % selected: 35 + 12
+// us, of which the read alone would take 18).  A single pass with tiles chained by
+// look-back took 88 us there: thousands of tiles draw their numbers from one counter, 11 ns each, and wait for
+// each other's prefixes.
+#include "zen_select.h"
+
+namespace zen {
+namespace {
+
+constexpr int kBlock = 256;                 // of the walking kernel
+constexpr int kMoveBlock = 1024;            // of the moving kernel: a stretch per wave
+constexpr int kMoveWaves = kMoveBlock / 64;
+constexpr int kRows = 4;                    // rows of one 16-byte vector per lane in flight
+constexpr int64_t kMaxStretches = 8192;     // 32 waves per compute unit
+constexpr int64_t kOneMax = 65536;
+template <typename S>
+constexpr int row() { return 64 * VecOf<S>::kN; }  // elements of a row
+template <typename S>
+constexpr int64_t least_stretch() { return (int64_t)row<S>() * kRows; }
+
+// Flags of the elements of one vector, element e at bit e.
+__device__ inline uint32_t vec_flags(const uint4 &q, uint32_t least, uint16_t) {
+  const uint32_t c = (0x8000u - least) * 0x00010001u;  // per 16-bit half: key + c carries into bit 15 iff key >= least
+  const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+  uint32_t x = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t m = ((w[j] & 0x7fff7fffu) + c) & 0x80008000u;
+    x |= (((m >> 15) | (m >> 30)) & 3u) << (2 * j);
+  }
+  return x;
+}
+__device__ inline uint32_t vec_flags(const uint4 &q, uint32_t least, uint32_t) {
+  return ((q.x & 0x7fffffffu) >= least ? 1u : 0u) | ((q.y & 0x7fffffffu) >= least ? 2u : 0u) |
+         ((q.z & 0x7fffffffu) >= least ? 4u : 0u) | ((q.w & 0x7fffffffu) >= least ? 8u : 0u);
+}
+__device__ inline uint16_t vec_pick(const uint4 &q, uint32_t e, uint16_t) {
+  const uint32_t a = e & 2u ? q.y : q.x, b = e & 2u ? q.w : q.z;
+  const uint32_t w = e & 4u ? b : a;
+  return (uint16_t)(e & 1u ? w >> 16 : w);
+}
+__device__ inline uint32_t vec_pick(const uint4 &q, uint32_t e, uint32_t) {
+  const uint32_t a = e & 1u ? q.y : q.x, b = e & 1u ? q.w : q.z;
+  return e & 2u ? b : a;
+}
+
+__device__ inline uint32_t scan_dpp(uint32_t x) {  // inclusive prefix sum across the 64 lanes
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);
+  return x;
+}
+
+// A wave's walk over elements [begin, end) (begin a multiple of the vector length): selected element number i goes
+// to idx[i], val[i] if i < room.  Returns how many there are.  WRITE == false: only counts.  A stretch holds fewer
+// than 2^18 elements, so that byte offsets from the (uniform) pointers fit 32 bits.
+template <typename S, bool ALIGNED, bool WRITE, typename I>
+__device__ __forceinline__ uint32_t walk(const S *__restrict__ in, int64_t begin, int64_t end, uint32_t least,
+                                I *__restrict__ idx, S *__restrict__ val, uint32_t room) {
+  constexpr int V = VecOf<S>::kN;
+  const int lane = lane_id();
+  uint32_t found = 0;
+  constexpr int64_t kStep = (int64_t)row<S>() * kRows;
+  auto load = [&](int64_t base, uint4 (&q)[kRows]) {
+    if (ALIGNED && base + kStep <= end) {
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) q[r] = *reinterpret_cast<const uint4 *>(in + base + r * row<S>() + lane * V);
+    } else {
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) {
+        S e[V];
+        load_vec<S, ALIGNED>(in, base + r * row<S>() + lane * V, end, e);  // past the end: zeros, never selected
+        __builtin_memcpy(&q[r], e, 16);
+      }
+    }
+  };
+  uint4 q[kRows], next[kRows];
+  if (begin < end) load(begin, next);
+#pragma unroll 1
+  for (int64_t base = begin; base < end; base += kStep) {
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) q[r] = next[r];
+    if (base + kStep < end) load(base + kStep, next);  // on its way while these rows are looked at
+    uint32_t x[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) x[r] = vec_flags(q[r], least, S(0));
+#pragma unroll
+    for (int r = 0; r < kRows; r += 2) {  // two rows' counts in the halves of a word (a row has 512 elements at most)
+      const uint32_t c = (uint32_t)__popc(x[r]) | ((uint32_t)__popc(x[r + 1]) << 16);
+      const uint32_t incl = scan_dpp(c);
+      const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+      if (WRITE) {
+        const uint32_t before = incl - c;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          uint32_t pos = found + (h ? (total & 0xffffu) + (before >> 16) : before & 0xffffu);
+          uint32_t bits = x[r + h];
+          const uint32_t first = (uint32_t)base + (uint32_t)((r + h) * row<S>() + lane * V);
+          while (bits) {
+            const uint32_t e = (uint32_t)__ffs((int)bits) - 1u;
+            bits &= bits - 1u;
+            if (pos < room) {
+              *reinterpret_cast<I *>(reinterpret_cast<char *>(idx) + (uint32_t)(pos * sizeof(I))) = (I)(first + e);
+              *reinterpret_cast<S *>(reinterpret_cast<char *>(val) + (uint32_t)(pos * sizeof(S))) = vec_pick(q[r + h], e, S(0));
+            }
+            ++pos;
+          }
+        }
+      }
+      found += (total & 0xffffu) + (total >> 16);
+    }
+  }
+  return found;
+}
+
+__device__ inline uint32_t least_key(const uint32_t *thr, uint32_t mask) {
+  uint32_t t = thr ? thr[0] : 1u;
+  if (t == 0) t = 1;                 // zeros are never selected
+  return t > mask ? mask + 1u : t;   // nothing qualifies
+}
+
+// Entries that still fit an output of `capacity` from place `at` on.
+__device__ inline uint32_t room_from(int64_t capacity, uint64_t at) {
+  const uint64_t left = at < (uint64_t)capacity ? (uint64_t)capacity - at : 0u;
+  return left < 0xffffffffu ? (uint32_t)left : 0xffffffffu;
+}
+
+struct Stretches {
+  int64_t len;      // elements of a stretch
+  uint32_t count;   // stretches
+  uint32_t quota;   // entries a stretch's part holds
+  uint32_t *found;  // [count]
+  int32_t *idx;     // [count * quota]
+  void *val;
+};
+
+template <typename S>
+Stretches plan_stretches(void *workspace, int64_t n, size_t *bytes) {
+  Stretches st{};
+  st.len = ceil_div(ceil_div(n > 0 ? n : 1, kMaxStretches), least_stretch<S>()) * least_stretch<S>();
+  st.count = (uint32_t)ceil_div(n > 0 ? n : 1, st.len);
+  st.quota = (uint32_t)(st.len / 8);
+  Carver cv(workspace);
+  if (n > kOneMax) {
+    st.found = cv.take<uint32_t>(st.count);
+    st.idx = cv.take<int32_t>((size_t)st.count * st.quota);
+    st.val = cv.take<S>((size_t)st.count * st.quota);
+  }
+  *bytes = cv.used;
+  return st;
+}
+
+template <typename S, bool ALIGNED>
+__global__ __launch_bounds__(kBlock, 8) void k_compact_walk(const S *__restrict__ in, int64_t n,
+                                                            const uint32_t *__restrict__ thr, Stretches st) {
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)));
+  if (w >= st.count) return;
+  const int64_t begin = (int64_t)w * st.len;
+  const int64_t end = begin + st.len < n ? begin + st.len : n;
+  const uint32_t found =
+      walk<S, ALIGNED, true>(in, begin, end, least_key(thr, KeyOf<S>::kMask), st.idx + (size_t)w * st.quota,
+                             static_cast<S *>(st.val) + (size_t)w * st.quota, st.quota);
+  if (lane_id() == 0) st.found[w] = found;
+}
+
+template <typename S, typename I, bool ALIGNED>
+__global__ __launch_bounds__(kMoveBlock) void k_compact_move(const S *__restrict__ in, int64_t n,
+                                                             const uint32_t *__restrict__ thr, Stretches st,
+                                                             I *__restrict__ out_idx, S *__restrict__ out_val,
+                                                             int64_t capacity, int64_t *out_count, int32_t *status) {
+  __shared__ uint32_t part[kMoveWaves];
+  __shared__ uint32_t own[kMoveWaves];
+  const uint32_t first = blockIdx.x * (uint32_t)kMoveWaves;
+  const uint32_t wave = threadIdx.x >> 6;
+  uint32_t sum = 0;  // a tensor has fewer than 2^31 elements
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < first; i += kMoveBlock) sum += st.found[i];
+  sum = wave_sum(sum);
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(first + wave));
+  const uint32_t mine = w < st.count ? st.found[w] : 0u;
+  if (lane_id() == 0) {
+    part[wave] = sum;
+    own[wave] = mine;
+  }
+  __syncthreads();
+  uint64_t at = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < (uint32_t)kMoveWaves; ++i) at += part[i] + (i < wave ? own[i] : 0u);
+  if (w + 1 == st.count && lane_id() == 0) {
+    *out_count = (int64_t)(at + mine);
+    if (at + mine > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
+  }
+  if (w >= st.count) return;
+  at = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) |
+       (uint32_t)__builtin_amdgcn_readfirstlane((int)at);  // the same in every lane
+  if (mine > st.quota) {
+    const int64_t begin = (int64_t)w * st.len;
+    const int64_t end = begin + st.len < n ? begin + st.len : n;
+    walk<S, ALIGNED, true>(in, begin, end, least_key(thr, KeyOf<S>::kMask), out_idx + at, out_val + at,
+                           room_from(capacity, at));
+    return;
+  }
+  const int32_t *idx = st.idx + (size_t)w * st.quota;
+  const S *val = static_cast<const S *>(st.val) + (size_t)w * st.quota;
+  constexpr int kAhead = 4;
+  for (uint32_t i0 = 0; i0 < mine; i0 += 64 * kAhead) {
+    int32_t k[kAhead];
+    S v[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const uint32_t i = i0 + (uint32_t)(j * 64 + lane_id());
+      k[j] = idx[i < mine ? i : 0u];
+      v[j] = val[i < mine ? i : 0u];
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const uint32_t i = i0 + (uint32_t)(j * 64 + lane_id());
+      if (i < mine && at + i < (uint64_t)capacity) {
+        out_idx[at + i] = (I)k[j];
+        out_val[at + i] = v[j];
+      }
+    }
+  }
+}
+
+template <typename S, typename I, bool ALIGNED>
+__global__ __launch_bounds__(kMoveBlock) void k_compact_one(const S *__restrict__ in, int64_t n,
+                                                            const uint32_t *__restrict__ thr, I *__restrict__ out_idx,
+                                                            S *__restrict__ out_val, int64_t capacity,
+                                                            int64_t *out_count, int32_t *status) {
+  __shared__ uint32_t own[kMoveWaves];
+  const uint32_t wave = threadIdx.x >> 6;
+  const uint32_t least = least_key(thr, KeyOf<S>::kMask);
+  const int64_t len = (n + kMoveWaves * row<S>() - 1) / (kMoveWaves * row<S>()) * row<S>();
+  const int64_t begin = (int64_t)wave * len < n ? (int64_t)wave * len : n;
+  const int64_t end = begin + len < n ? begin + len : n;
+  const uint32_t mine = walk<S, ALIGNED, false, I>(in, begin, end, least, nullptr, nullptr, 0);
+  if (lane_id() == 0) own[wave] = mine;
+  __syncthreads();
+  uint64_t at = 0, all = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < (uint32_t)kMoveWaves; ++i) {
+    at += i < wave ? own[i] : 0u;
+    all += own[i];
+  }
+  if (threadIdx.x == 0) {
+    *out_count = (int64_t)all;
+    if (all > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
+  }
+  at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);  // the same in every lane
+  walk<S, ALIGNED, true>(in, begin, end, least, out_idx + at, out_val + at, room_from(capacity, at));
+}
+
+template <typename S, typename I, bool ALIGNED>
+int compact_launch(const S *in, int64_t n, const uint32_t *thr, I *out_idx, S *out_val, int64_t capacity,
+                   int64_t *out_count, void *workspace, int32_t *status, hipStream_t s) {
+  ProfScope prof(kProfSelectCompact, s);
+  if (n <= kOneMax) {
+    k_compact_one<S, I, ALIGNED><<<dim3(1), dim3(kMoveBlock), 0, s>>>(in, n, thr, out_idx, out_val, capacity, out_count,
+                                                                     status);
+    ZEN_LAUNCH_CHECK("k_compact_one");
+    return ZEN_OK;
+  }
+  size_t bytes;
+  const Stretches st = plan_stretches<S>(workspace, n, &bytes);
+  k_compact_walk<S, ALIGNED><<<dim3((unsigned)ceil_div(st.count, kBlock / 64)), dim3(kBlock), 0, s>>>(in, n, thr, st);
+  ZEN_LAUNCH_CHECK("k_compact_walk");
+  k_compact_move<S, I, ALIGNED><<<dim3((unsigned)ceil_div(st.count, kMoveWaves)), dim3(kMoveBlock), 0, s>>>(
+      in, n, thr, st, out_idx, out_val, capacity, out_count, status);
+  ZEN_LAUNCH_CHECK("k_compact_move");
+  return ZEN_OK;
+}
+
+template <typename S>
+int compact_call(const void *input, int64_t n, const uint32_t *thr, void *out_idx, int idx64, void *out_val,
+                 int64_t capacity, int64_t *out_count, void *workspace, int32_t *status, hipStream_t s) {
+  const S *in = static_cast<const S *>(input);
+  S *val = static_cast<S *>(out_val);
+  const bool aligned = (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
+  if (idx64) {
+    int64_t *idx = static_cast<int64_t *>(out_idx);
+    return aligned ? compact_launch<S, int64_t, true>(in, n, thr, idx, val, capacity, out_count, workspace, status, s)
+                   : compact_launch<S, int64_t, false>(in, n, thr, idx, val, capacity, out_count, workspace, status, s);
+  }
+  int32_t *idx = static_cast<int32_t *>(out_idx);
+  return aligned ? compact_launch<S, int32_t, true>(in, n, thr, idx, val, capacity, out_count, workspace, status, s)
+                 : compact_launch<S, int32_t, false>(in, n, thr, idx, val, capacity, out_count, workspace, status, s);
+}
+
+}  // namespace
+}  // namespace zen
+
+extern "C" {
+
+size_t zen_select_workspace(int64_t n, int dtype) {
+  size_t bytes;
+  if (dtype == ZEN_BF16)
+    (void)zen::plan_stretches<uint16_t>(nullptr, n, &bytes);
+  else
+    (void)zen::plan_stretches<uint32_t>(nullptr, n, &bytes);
+  return bytes > 256 ? bytes : 256;
+}
+
+int zen_select(const void *input, int dtype, int64_t n, const uint32_t *thr, void *out_idx, int idx64,
+               void *out_val, int64_t capacity, int64_t *out_count, void *workspace, size_t workspace_bytes,
+               int32_t *status, void *stream) {
+  using namespace zen;
+  if (!out_count || !status) return fail(ZEN_EINVAL, "zen_select: null pointer");
+  if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_select: bad dtype");
+  if (n < 0 || n > 0x7fffffffll || capacity < 0) return fail(ZEN_EINVAL, "zen_select: need 0 <= n < 2^31");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (n == 0) {
+    launch_fill<int64_t>(out_count, 0, 1, s);
+    ZEN_LAUNCH_CHECK("zen_select: zero count");
+    return ZEN_OK;
+  }
+  if (!input || !workspace || (capacity > 0 && (!out_idx || !out_val)))
+    return fail(ZEN_EINVAL, "zen_select: null pointer");
+  if (workspace_bytes < zen_select_workspace(n, dtype)) return fail(ZEN_EWORKSPACE, "zen_select: workspace too small");
+  if (dtype == ZEN_BF16)
+    return compact_call<uint16_t>(input, n, thr, out_idx, idx64, out_val, capacity, out_count, workspace, status, s);
+  return compact_call<uint32_t>(input, n, thr, out_idx, idx64, out_val, capacity, out_count, workspace, status, s);
+}
+
+}  // extern "C"

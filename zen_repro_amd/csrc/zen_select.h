@@ -37,33 +37,29 @@ constexpr int kSelBlock = 256;
 constexpr int kSelVecs = 4;  // 16-byte vectors per thread and tile
 
 // Compaction of the elements with key >= max(thr[0], 1) (thr == nullptr: the
-// nonzero ones) into (index, value) lists.
+// nonzero ones) of a dense tensor into (index, value) lists, in no particular
+// order (zen_compact.hip has the ascending one).
 struct SelectArgs {
-  const void *in = nullptr;           // dense tensor, or the values of a list
+  const void *in = nullptr;
   int dtype = ZEN_F32;
-  int64_t n = 0;                      // elements (capacity of the list when n_dev is set)
-  const uint32_t *n_dev = nullptr;    // optional device-side element count (<= n)
+  int64_t n = 0;
   const uint32_t *thr = nullptr;      // optional device threshold key
-  const int32_t *src_idx = nullptr;   // list input: the index each element carries
-  void *out_idx = nullptr;
-  int idx64 = 0;                      // out_idx is int64 instead of int32
+  int32_t *out_idx = nullptr;
   void *out_val = nullptr;
   int64_t capacity = 0;
-  int64_t *out_count = nullptr;       // optional: number found (may exceed capacity)
-  uint32_t *out_count32 = nullptr;    // optional: the same clamped to capacity
-  bool ordered = true;                // ascending output (false: tiles in arrival order)
-  uint32_t *cand_hist = nullptr;      // optional (unordered mode): kCandHistWords counters, zero on entry: kCandRows
+  uint32_t *out_count32 = nullptr;    // number found, clamped to capacity
+  uint32_t *cand_hist = nullptr;      // optional: kCandHistWords counters, zero on entry: kCandRows
                                       // partial histograms of min((key - floor) >> (bf16: 0, fp32: 16), kCandBins-1)
                                       // over the selected, then a count of finished blocks
   int64_t pick_k = 0;                 // with cand_hist and pick_thr: the block that finishes last writes
   uint32_t *pick_thr = nullptr;       // pick_thr[0] = k-th largest key as far as the histogram resolves it (bf16:
                                       // exactly; fp32: its top 15 bits), pick_thr[1] = candidates at or above it;
                                       // ZEN_STAT_RETRY if the candidates are fewer than k
-  void *scratch = nullptr;            // select_scratch_bytes(n, dtype)
+  void *scratch = nullptr;            // select_scratch_bytes()
   int32_t *status = nullptr;
 };
 
-size_t select_scratch_bytes(int64_t n, int dtype);
+size_t select_scratch_bytes();
 int select_compact(const SelectArgs &args, hipStream_t stream);
 
 // Exact k-th largest magnitude key by radix select: thr[0] = key, thr[1] = number

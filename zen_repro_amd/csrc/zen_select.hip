@@ -362,11 +362,9 @@ __global__ __launch_bounds__(256) void k_compress(const S *__restrict__ in, int6
 // is thread order and one block scan of per-thread counts places everything.
 // A block walks its tile once, staging the selected (index, value) pairs in
 // LDS in ascending order; only then does it need its place in the output.
-// Ordered mode gets it from the tile-prefix protocol (the output is ascending
-// in the index); unordered mode reserves a range with one atomic add (tiles
-// land in arrival order, each tile's entries stay ascending), which callers
-// that sort afterwards prefer because no tile ever waits.  The LDS stage makes
-// the write-out coalesced.  A tile with more selected elements than the stage
+// It reserves a range with one atomic add (tiles land in arrival order, each
+// tile's entries stay ascending; the callers sort afterwards), so no tile ever
+// waits.  The LDS stage makes the write-out coalesced.  A tile with more selected elements than the stage
 // holds is walked a second time and written directly.
 //
 // A CDNA compute unit retires 64 lane-operations per clock while HBM delivers
@@ -375,11 +373,9 @@ __global__ __launch_bounds__(256) void k_compress(const S *__restrict__ in, int6
 // therefore evaluated two bf16 at a time on packed words (3 operations per
 // pair), the flags of a thread's 32 elements end in one register, and only the
 // few selected elements take the longer extraction path.
-// The input is a dense tensor (an element's index is its position) or a list
-// (src_idx gives the index carried by each element).
 
 constexpr int kSelStage = 3072;    // staged pairs per tile
-constexpr int kReserveShift = 40;  // unordered mode: tiles done above, entries reserved below
+constexpr int kReserveShift = 40;  // tiles done above, entries reserved below
 
 // Inclusive prefix sum across the 64 lanes with DPP row shifts and broadcasts.
 __device__ inline uint32_t wave_inclusive_scan_dpp(uint32_t x) {
@@ -460,11 +456,11 @@ struct Flags<uint32_t> {
   static __device__ inline uint32_t pick(const uint4 (&q)[kSelVecs], uint32_t bit);
 };
 
-template <typename S, typename I, bool ALIGNED, bool STAGED>
+template <typename S, bool ALIGNED, bool STAGED>
 __device__ inline uint32_t select_walk_tile(const S *__restrict__ in, int64_t n, uint32_t floor_key,
-                                            int64_t tile_base, int subs, const int32_t *__restrict__ src_idx,
+                                            int64_t tile_base, int subs,
                                             uint32_t *s_wave, int32_t *st_idx, S *st_val, uint32_t *s_hist,
-                                            I *__restrict__ out_idx, S *__restrict__ out_val, uint64_t out_base,
+                                            int32_t *__restrict__ out_idx, S *__restrict__ out_val, uint64_t out_base,
                                             int64_t capacity) {
   constexpr int V = VecOf<S>::kN;
   constexpr int kChunk = Flags<S>::kElems;  // elements per thread and sub-tile
@@ -520,7 +516,7 @@ __device__ inline uint32_t select_walk_tile(const S *__restrict__ in, int64_t n,
           st_val[pos] = v;
         }
       } else if (out_base + pos < (uint64_t)capacity) {
-        out_idx[out_base + pos] = (I)(src_idx ? src_idx[first + off] : first + off);
+        out_idx[out_base + pos] = (int32_t)(first + off);
         out_val[out_base + pos] = v;
       }
     }
@@ -529,75 +525,50 @@ __device__ inline uint32_t select_walk_tile(const S *__restrict__ in, int64_t n,
   return running;
 }
 
-template <typename S, typename I, bool ALIGNED, bool ORDERED>
+template <typename S, bool ALIGNED>
 __global__ __launch_bounds__(kSelBlock) void k_select_compact(
-    const S *__restrict__ in, int64_t n_max, const uint32_t *__restrict__ n_dev, const uint32_t *__restrict__ thr,
-    const int32_t *__restrict__ src_idx, I *__restrict__ out_idx, S *__restrict__ out_val, int64_t capacity,
-    ScanState st, int ntiles, int subs, uint32_t *cand_hist, uint32_t pick_k, uint32_t *pick_thr,
-    int64_t *out_count, uint32_t *out_count32, int32_t *status) {
+    const S *__restrict__ in, int64_t n, const uint32_t *__restrict__ thr, int32_t *__restrict__ out_idx,
+    S *__restrict__ out_val, int64_t capacity, unsigned long long *reserved, int ntiles, int subs, uint32_t *cand_hist,
+    uint32_t pick_k, uint32_t *pick_thr, uint32_t *out_count32, int32_t *status) {
   constexpr int kSub = kSelBlock * Flags<S>::kElems;
   __shared__ uint32_t s_wave[kSelBlock / 64];
   __shared__ uint64_t s_bcast;
-  __shared__ int s_tile;
   __shared__ int32_t st_idx[kSelStage];
   __shared__ S st_val[kSelStage];
-  __shared__ uint32_t s_hist[ORDERED ? 1 : kCandBins];
-  uint32_t *hist = (!ORDERED && cand_hist) ? s_hist : nullptr;
+  __shared__ uint32_t s_hist[kCandBins];
+  uint32_t *hist = cand_hist ? s_hist : nullptr;
   if (hist) {
     for (int i = threadIdx.x; i < kCandBins; i += kSelBlock) s_hist[i] = 0;
     __syncthreads();
   }
-  int64_t n = n_max;
-  if (n_dev && (int64_t)*n_dev < n) n = (int64_t)*n_dev;
   uint32_t floor_key = thr ? thr[0] : 1u;
   if (floor_key == 0) floor_key = 1u;  // zeros are never selected
   if (floor_key > KeyOf<S>::kMask) floor_key = KeyOf<S>::kMask + 1u;  // nothing qualifies
-
-  // ordered: tiles are taken by ticket, so that every earlier tile already runs
   {
-    int tile = (int)blockIdx.x;
-    if (ORDERED) {
-      if (threadIdx.x == 0) s_tile = (int)atomicAdd(st.ticket, 1u);
-      __syncthreads();
-      tile = s_tile;
-    }
-    if (tile >= ntiles) return;
-    const int64_t tile_base = (int64_t)tile * subs * kSub;
-    const uint32_t found = select_walk_tile<S, I, ALIGNED, true>(in, n, floor_key, tile_base, subs, src_idx, s_wave,
-                                                                 st_idx, st_val, hist, out_idx, out_val, 0, capacity);
-    uint64_t tile_start, all = 0;
-    bool last;
-    if (ORDERED) {
-      tile_start = lookback_exclusive(st, tile, found, status, &s_bcast);
-      last = tile == ntiles - 1;
-      all = tile_start + found;
-    } else {
-      if (threadIdx.x == 0)
-        s_bcast = __hip_atomic_fetch_add(st.desc, (1ull << kReserveShift) | found, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-      __syncthreads();
-      const uint64_t old = s_bcast;
-      tile_start = old & ((1ull << kReserveShift) - 1);
-      last = (int)(old >> kReserveShift) == ntiles - 1;  // every other tile has reserved already
-      all = tile_start + found;
-    }
-    if (last && threadIdx.x == 0) {
-      if (out_count) *out_count = (int64_t)all;
-      if (out_count32) *out_count32 = (uint32_t)(all < (uint64_t)capacity ? all : (uint64_t)capacity);
+    const int64_t tile_base = (int64_t)blockIdx.x * subs * kSub;
+    const uint32_t found = select_walk_tile<S, ALIGNED, true>(in, n, floor_key, tile_base, subs, s_wave, st_idx, st_val,
+                                                              hist, out_idx, out_val, 0, capacity);
+    if (threadIdx.x == 0)
+      s_bcast = __hip_atomic_fetch_add(reserved, (1ull << kReserveShift) | found, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const uint64_t old = s_bcast;
+    const uint64_t tile_start = old & ((1ull << kReserveShift) - 1), all = tile_start + found;
+    if ((int)(old >> kReserveShift) == ntiles - 1 && threadIdx.x == 0) {  // every other tile has reserved already
+      *out_count32 = (uint32_t)(all < (uint64_t)capacity ? all : (uint64_t)capacity);
       if (all > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
     }
     if (found <= (uint32_t)kSelStage) {
       for (uint32_t i = threadIdx.x; i < found; i += kSelBlock) {
         const uint64_t pos = tile_start + i;
         if (pos < (uint64_t)capacity) {
-          const int32_t at = st_idx[i];
-          out_idx[pos] = (I)(src_idx ? src_idx[at] : at);
+          out_idx[pos] = st_idx[i];
           out_val[pos] = st_val[i];
         }
       }
     } else {
-      select_walk_tile<S, I, ALIGNED, false>(in, n, floor_key, tile_base, subs, src_idx, s_wave, st_idx, st_val,
-                                             nullptr, out_idx, out_val, tile_start, capacity);
+      select_walk_tile<S, ALIGNED, false>(in, n, floor_key, tile_base, subs, s_wave, st_idx, st_val, nullptr, out_idx,
+                                          out_val, tile_start, capacity);
     }
   }
   if (hist) {
@@ -637,47 +608,36 @@ static int select_subs(int64_t n, int dtype) {
   return subs;
 }
 
-size_t select_scratch_bytes(int64_t n, int dtype) {
-  const int v = dtype == ZEN_BF16 ? 8 : 4;
-  const int64_t tile = (int64_t)kSelBlock * kSelVecs * v * select_subs(n > 0 ? n : 1, dtype);
-  const int64_t ntiles = ceil_div(n > 0 ? n : 1, tile);
-  return align_up(scan_words(ntiles) * sizeof(unsigned long long), 256);
-}
+size_t select_scratch_bytes() { return 256; }
 
-template <typename S, typename I>
+template <typename S>
 static int select_launch(const SelectArgs &a, hipStream_t stream) {
   constexpr int V = VecOf<S>::kN;
   const int subs = select_subs(a.n, a.dtype);
   const int64_t tile = (int64_t)kSelBlock * kSelVecs * V * subs;
   const int64_t ntiles = ceil_div(a.n, tile);
   if (ntiles > 0xffffff) return fail(ZEN_EINVAL, "select: too many tiles");
-  const ScanState st = scan_state(a.scratch, ntiles);
-  launch_fill<unsigned long long>(st.desc, 0ull, a.ordered ? scan_words(ntiles) : 1, stream);
-  ZEN_LAUNCH_CHECK("select: clear scan state");
+  unsigned long long *reserved = static_cast<unsigned long long *>(a.scratch);
+  launch_fill<unsigned long long>(reserved, 0ull, 1, stream);
+  ZEN_LAUNCH_CHECK("select: clear the reservations");
   const S *in = static_cast<const S *>(a.in);
-  I *out_idx = static_cast<I *>(a.out_idx);
   S *out_val = static_cast<S *>(a.out_val);
   const bool aligned = (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
   const dim3 grid((unsigned)ntiles), block(kSelBlock);
   ProfScope prof(kProfSelectCompact, stream);
-#define ZEN_SELECT_GO(AL, ORD)                                                                                 \
-  k_select_compact<S, I, AL, ORD><<<grid, block, 0, stream>>>(in, a.n, a.n_dev, a.thr, a.src_idx, out_idx,   \
-                                                              out_val, a.capacity, st, (int)ntiles, subs,    \
-                                                              a.cand_hist, (uint32_t)a.pick_k, a.pick_thr,   \
-                                                              a.out_count, a.out_count32, a.status)
-  if (aligned && a.ordered) ZEN_SELECT_GO(true, true);
-  else if (aligned) ZEN_SELECT_GO(true, false);
-  else if (a.ordered) ZEN_SELECT_GO(false, true);
-  else ZEN_SELECT_GO(false, false);
+#define ZEN_SELECT_GO(AL)                                                                                          \
+  k_select_compact<S, AL><<<grid, block, 0, stream>>>(in, a.n, a.thr, a.out_idx, out_val, a.capacity, reserved,  \
+                                                      (int)ntiles, subs, a.cand_hist, (uint32_t)a.pick_k,        \
+                                                      a.pick_thr, a.out_count32, a.status)
+  if (aligned) ZEN_SELECT_GO(true);
+  else ZEN_SELECT_GO(false);
 #undef ZEN_SELECT_GO
   ZEN_LAUNCH_CHECK("k_select_compact");
   return ZEN_OK;
 }
 
 int select_compact(const SelectArgs &a, hipStream_t stream) {
-  if (a.dtype == ZEN_BF16)
-    return a.idx64 ? select_launch<uint16_t, int64_t>(a, stream) : select_launch<uint16_t, int32_t>(a, stream);
-  return a.idx64 ? select_launch<uint32_t, int64_t>(a, stream) : select_launch<uint32_t, int32_t>(a, stream);
+  return a.dtype == ZEN_BF16 ? select_launch<uint16_t>(a, stream) : select_launch<uint32_t>(a, stream);
 }
 
 // ------------------------------------------- compaction in no particular order
@@ -1538,40 +1498,6 @@ int zen_compress(const void *input, int dtype, int64_t n, const uint32_t *thr, v
   if (dtype == ZEN_BF16)
     return compress_launch(static_cast<const uint16_t *>(input), n, thr, static_cast<uint16_t *>(out), s);
   return compress_launch(static_cast<const uint32_t *>(input), n, thr, static_cast<uint32_t *>(out), s);
-}
-
-size_t zen_select_workspace(int64_t n, int dtype) { return zen::select_scratch_bytes(n, dtype); }
-
-int zen_select(const void *input, int dtype, int64_t n, const uint32_t *thr, void *out_idx, int idx64,
-               void *out_val, int64_t capacity, int64_t *out_count, void *workspace, size_t workspace_bytes,
-               int32_t *status, void *stream) {
-  using namespace zen;
-  if (!out_count || !status) return fail(ZEN_EINVAL, "zen_select: null pointer");
-  if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_select: bad dtype");
-  if (n < 0 || n > 0x7fffffffll || capacity < 0) return fail(ZEN_EINVAL, "zen_select: need 0 <= n < 2^31");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (n == 0) {
-    launch_fill<int64_t>(out_count, 0, 1, s);
-    ZEN_LAUNCH_CHECK("zen_select: zero count");
-    return ZEN_OK;
-  }
-  if (!input || !workspace || (capacity > 0 && (!out_idx || !out_val)))
-    return fail(ZEN_EINVAL, "zen_select: null pointer");
-  if (workspace_bytes < zen_select_workspace(n, dtype)) return fail(ZEN_EWORKSPACE, "zen_select: workspace too small");
-  SelectArgs a;
-  a.in = input;
-  a.dtype = dtype;
-  a.n = n;
-  a.thr = thr;
-  a.out_idx = out_idx;
-  a.idx64 = idx64;
-  a.out_val = out_val;
-  a.capacity = capacity;
-  a.out_count = out_count;
-  a.ordered = true;
-  a.scratch = workspace;
-  a.status = status;
-  return select_compact(a, s);
 }
 
 }  // extern "C"
