@@ -53,7 +53,8 @@ extern "C" {
 /* OR-ed into the `mode` of zen_merge: the caller vouches that the first zen_merge_zero_bytes() bytes of the
    workspace are zero.  The call then skips the kernel that clears them, and leaves them zero again when it
    returns ZEN_OK and raises neither ZEN_STAT_RETRY nor ZEN_STAT_INTERNAL (after those the caller clears
-   them).  A workspace allocated zeroed and used for zen_merge only therefore needs no clearing at all. */
+   them).  A workspace allocated zeroed and used for zen_merge only therefore needs no clearing at all.
+   OR-ed into the `mode` of zen_load_balance: the caller vouches that splits[0..partitions) is zero. */
 #define ZEN_MODE_ZEROED 0x100
 /* OR-ed into the `mode` of zen_load_balance: zen_load_balance_prepare has run for this call (see there);
    ZEN_MODE_SECOND names the second of the two sets of sampling memory (without ZEN_MODE_PREPARED: the call takes
@@ -283,7 +284,7 @@ int zen_load_balance_prepare(const void *input, int dtype, int64_t n, int64_t m,
 
 /*
  * Which implementation a zen_load_balance call with these sizes takes: 0 = owner table (the general
- * mode), 1 = sort-based owner resolution, 2 = bucket slabs (large inputs whose expected output is a small
+ * mode), 1 = the same in three launches or one (tables of up to 4 Mi slots), or sort-based owner resolution, 2 = bucket slabs (large inputs whose expected output is a small
  * fraction of the table: one streaming pass, then per-bucket sorts inside LDS), 3 = wide buckets (the same
  * for an expected output of up to a few million entries: at most 256 buckets, one resident workgroup each,
  * two launches).  No counterpart in the reference; tests and benchmarks use it to know what they measured.
@@ -304,7 +305,7 @@ int zen_load_balance_path(int64_t n, int64_t m, int dtype, int64_t capacity, int
  */
 size_t zen_merge_workspace(int64_t r, int64_t dense_n);
 size_t zen_merge_zero_bytes(void); /* see ZEN_MODE_ZEROED; the same for every r and dense_n */
-/* 0 = radix sort (general mode), 1 = one bucket pass + per-range sorts, 2 = bucket slabs, 3 = wide buckets; see
+/* 0 = radix sort (general mode) or, in the fast mode, one workgroup for lists of up to 4096 entries, 1 = one bucket pass + per-range sorts, 2 = bucket slabs, 3 = wide buckets; see
    zen_load_balance_path */
 int zen_merge_path(int64_t r, int64_t dense_n, int mode);
 int zen_merge(const void *idx, int idx64_in, const void *val, int dtype,

@@ -857,3 +857,60 @@ def test_ordered_compaction_at_the_edges_of_its_kernels(zen, oracle, n, dtype, d
         idx, val, count, bits = _select_raw(d[shift:], None, False, capacity=room)
         assert count == want.size and bits == (_lib.STAT_CAPACITY if want.size > room else 0)
         assert np.array_equal(to_np(idx), want[:room])
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("n,P,density,scale,rehash", [
+    (4097, 4, 0.1, 1, 3), (32768, 256, 0.05, 1, 3), (32771, 4, 0.3, 1, 3), (32768, 2, 0.15, 1, 1),  # one workgroup, and just beyond
+    (32768, 257, 0.02, 1, 3), (20000, 8, 0.2, 2, 3),                      # more partitions, more slots than it takes
+    (262143, 16, 0.1, 1, 3), (1 << 18, 1000, 0.02, 1, 3),                 # ragged stretches, many partitions in one
+    (1048575, 2, 0.15, 1, 2), (3000001, 16, 0.1, 1, 3), (1 << 22, 64, 0.01, 1, 3),  # long serial tails; the largest
+])
+def test_load_balance_through_the_owner_table(zen, oracle, n, P, density, scale, rehash, dtype):
+    """Nonzeros, a threshold and a top-k selection, twice on the same table; whole numbers and copies: exact."""
+    g = make_grad(oracle, n, density, dtype, seed=n ^ P)
+    g[0] = 0x3F80 if dtype == "bf16" else 1.0
+    tp = zen.TensorPartition(P, scale, rehash)
+    d = to_dev(g)
+    k = max(1, int(n * density) // 2)  # fewer than there are nonzeros: the wide buckets (top-k from 2^20 slots on) decline others
+    key = oracle.kth_key(g, k)
+    masked, _ = oracle.mask_dense(g, key)
+    whole = oracle.load_balance(g, P, scale, rehash)
+    part = oracle.load_balance(masked, P, scale, rehash)
+    thr = zen.topk_threshold(d, k)
+    for (idx_o, val_o, splits_o, st_o), kw in ((whole, {}), (part, {"thr": thr}), (part, {"k": k})):
+        if st_o:
+            continue  # a serial region overflowed
+        for capacity in (len(idx_o), len(idx_o) + 77):
+            oi, ov, splits, status = tp.load_balance_flat(d, capacity=max(1, capacity), **kw)
+            assert status.item() == 0
+            assert np.array_equal(to_np(splits), splits_o)
+            assert np.array_equal(to_np(oi)[:len(idx_o)], idx_o) and np.array_equal(to_np(ov)[:len(idx_o)], val_o)
+    m, _ = oracle.table_sizes(n, P, scale)
+    assert not tp._table(d.device, m).any()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("r,n", [(1, 5000), (1023, 5000), (4096, 5000), (4096, 1 << 30), (4097, 20000), (30000, 40000), (9000, 16385)])
+@pytest.mark.parametrize("copies", [1, 16, 0])
+def test_merge_of_short_lists(zen, oracle, r, n, copies, dtype):
+    """One workgroup (up to 4096 entries) and narrow wide buckets; indices that differ, that come about sixteen times
+    and (0) that are all the same.  Sums in order of arrival: bit for bit, in fp32 and rounded once."""
+    rng = np.random.default_rng(r + n + copies)
+    distinct = 1 if copies == 0 else max(1, min(n - 1, r // copies))
+    pool = rng.choice(n - 1, distinct, replace=False) + 1 if n < 1 << 20 else rng.integers(1, n, distinct)
+    idx = rng.permutation(np.resize(pool, r)).astype(np.int32)
+    val = make_grad(oracle, r, 1.0, dtype, seed=r)
+    mi, mv = oracle.merge_sparse(idx, val, n)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    di, dv = torch.from_numpy(idx).cuda(), to_dev(val)
+    gi, gv = lba.merge_sparse(di, dv, n)
+    assert np.array_equal(to_np(gi), mi) and np.array_equal(to_np(gv).view(np.uint32), mv.view(np.uint32))
+    ri, rv = lba.merge_rounded(di, dv, n, dv.dtype)
+    want = torch.from_numpy(mv).to(dv.dtype)
+    keep = want != 0
+    assert torch.equal(ri.cpu(), torch.from_numpy(mi)[keep]) and torch.equal(rv.cpu(), want[keep])
+    if n <= 1 << 20:
+        dense = torch.zeros(n, dtype=dv.dtype)
+        dense[torch.from_numpy(mi).long()] = want
+        assert torch.equal(lba.decode_sparse_tensors(di, dv, n).cpu(), dense)

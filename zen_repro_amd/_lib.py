@@ -13,7 +13,7 @@ F32, BF16 = 0, 1
 OK, EINVAL, EHIP, EWORKSPACE = 0, -1, -2, -3
 STAT_SERIAL_OVERFLOW, STAT_CAPACITY, STAT_INTERNAL, STAT_BAD_INDEX, STAT_RETRY = 1, 2, 4, 8, 16
 MODE_FAST, MODE_GENERAL = 0, 1
-MODE_ZEROED = 0x100  # zen_merge: the head of the workspace is zero (and stays so)
+MODE_ZEROED = 0x100  # zen_merge: the head of the workspace is zero (and stays so); zen_load_balance: splits is zero
 MODE_PREPARED, MODE_SECOND, MODE_DISCARD = 0x200, 0x400, 0x800  # zen_load_balance: the sample was taken ahead (zen_load_balance_prepare)
 MODE_FLOOR = 0x1000  # zen_load_balance with k > 0: thr holds a key close to the threshold, no sample is taken
 MODE_SLABS = 0x2000  # fast mode without the wide-bucket path (bucket slabs where they fit)

@@ -287,7 +287,7 @@ class LoadBalanceAllreduce:
         a = _lib.EncodeMergeArgs(
             flat.data_ptr(), code, n, m, P, partition.rehash, thr.data_ptr() if thr is not None else None, int(k),
             thr_out.data_ptr() if thr_out is not None else None, out_idx.data_ptr(), out_val.data_ptr(), capacity,
-            splits.data_ptr(), table.data_ptr(), mode | flags, ws.data_ptr(), ws.numel(), status.data_ptr(),
+            splits.data_ptr(), table.data_ptr(), mode | flags | _lib.MODE_ZEROED, ws.data_ptr(), ws.numel(), status.data_ptr(),
             indices.data_ptr(), int(indices.dtype == torch.int64), values.data_ptr(), r, dense_size,
             m_idx.data_ptr(), 0, m_val.data_ptr(), r, count.data_ptr(),
             _lib.MODE_FAST | self.fast_flags | _lib.MODE_ZEROED, mws.data_ptr(), mws.numel(), m_status.data_ptr(),

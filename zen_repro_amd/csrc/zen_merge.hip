@@ -500,18 +500,26 @@ MergePlan plan_merge(void *workspace, int64_t r, int64_t dense_n) {
   return p;
 }
 
-// Whether a call with these sizes goes to the wide buckets.
+// Whether a call with these sizes goes to one workgroup, to the wide buckets.
+bool takes_one(int64_t r, int mode) { return (mode & 0xff) == ZEN_MODE_FAST && r <= wide_merge_one_max(); }
 bool takes_wide(int64_t r, int64_t dense_n, int mode) {
   return (mode & ~ZEN_MODE_ZEROED) == ZEN_MODE_FAST && wide_merge_fits(r, dense_n, wide_device_cus(), nullptr);
 }
+// Whether the merge writes a dense tensor whole (one workgroup writes zeros at some 100 GB/s: up to 1 MB).
+bool writes_dense(int64_t r, int64_t dense_n, int dtype, int mode) {
+  return takes_one(r, mode) ? dense_n * (dtype == ZEN_BF16 ? 2 : 4) <= (1ll << 20) : takes_wide(r, dense_n, mode);
+}
 
 // O: float (the fp32 sums) or uint16_t (rounded once to bf16).  out_idx == nullptr: out_val is the dense tensor,
-// written whole (on the wide buckets only: takes_wide).
+// written whole (where writes_dense says so).
 template <typename S, typename O>
 int merge_launch(const void *idx, int idx64_in, const S *val, int64_t r, int64_t dense_n, void *out_idx,
                  int idx64_out, O *out_val, int64_t capacity, int64_t *out_count, int mode, void *workspace,
                  int32_t *status, hipStream_t s) {
   const bool zeroed = (mode & ZEN_MODE_ZEROED) != 0;
+  if (takes_one(r, mode))
+    return wide_merge_one(idx, idx64_in, val, sizeof(S) == 2 ? ZEN_BF16 : ZEN_F32, r, dense_n, out_idx, idx64_out, out_val,
+                          sizeof(O) == 2 ? ZEN_BF16 : ZEN_F32, capacity, out_count, status, s);
   const bool wide = takes_wide(r, dense_n, mode);
   mode &= ~(ZEN_MODE_ZEROED | ZEN_MODE_SLABS);
   SlabGeom geo;
@@ -682,7 +690,7 @@ int zen_decode_dense(const void *idx, int idx64_in, const void *val, int dtype, 
   // the zero region zen_merge wants is at the head of this call's workspace too
   Carver cv(workspace);
   void *inner = cv.take<char>(zen_merge_workspace(r, dense_n));
-  const bool whole = r > 0 && takes_wide(r, dense_n, mode);  // the merge writes the dense tensor, zeros included
+  const bool whole = r > 0 && writes_dense(r, dense_n, dtype, mode);  // the merge writes the dense tensor, zeros included
   if (r > 0 && !workspace) return fail(ZEN_EINVAL, "zen_decode_dense: null pointer");
   if (r > 0 && workspace_bytes < zen_decode_dense_workspace(r, dense_n))
     return fail(ZEN_EWORKSPACE, "zen_decode_dense: workspace too small");

@@ -93,7 +93,7 @@ __device__ inline void gather(const S *__restrict__ in, int64_t n, const int64_t
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     const int64_t j = first + (int64_t)i * kBlock;
-    pos[i] = __builtin_nontemporal_load(at + (j < end ? j : end - 1));
+    pos[i] = at ? __builtin_nontemporal_load(at + (j < end ? j : end - 1)) : (j < end ? j : end - 1);
     if (pos[i] < 0 || pos[i] >= n) {
       bad = true;
       pos[i] = -1;
@@ -418,6 +418,20 @@ int sample_threshold_launch(const S *in, int64_t n, const int64_t *at, int64_t s
 }
 
 }  // namespace
+
+// The whole tensor is a sample whose positions are its own (no position array: at == nullptr).
+size_t topk_whole_bytes(int64_t n, int dtype) {
+  size_t bytes;
+  (void)plan_sample(nullptr, n, dtype, &bytes);
+  return bytes;
+}
+
+int topk_whole(const void *in, int dtype, int64_t n, int64_t k, uint32_t *thr, void *scratch, hipStream_t stream) {
+  if (dtype == ZEN_BF16)
+    return sample_threshold_launch(static_cast<const uint16_t *>(in), n, nullptr, n, k, thr, scratch, nullptr, stream);
+  return sample_threshold_launch(static_cast<const uint32_t *>(in), n, nullptr, n, k, thr, scratch, nullptr, stream);
+}
+
 }  // namespace zen
 
 extern "C" {

@@ -70,6 +70,10 @@ size_t topk_scratch_bytes();
 int topk_exact(const void *in, int dtype, int64_t n, const uint32_t *n_dev, int64_t k, uint32_t *thr,
                void *scratch, int32_t *status, int short_bit, hipStream_t stream);
 
+// The same key for a whole tensor of a few million elements in one to three launches (zen_sample.hip).
+size_t topk_whole_bytes(int64_t n, int dtype);
+int topk_whole(const void *in, int dtype, int64_t n, int64_t k, uint32_t *thr, void *scratch, hipStream_t stream);
+
 // Lower bound for that key from a 1/256 sample: thr_lo[0] is the lowest key of
 // the 15-bit magnitude bin (for bf16: the key itself) in which the sample
 // reaches the expected rank plus a safety margin.  Almost surely at least k

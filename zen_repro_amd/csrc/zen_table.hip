@@ -1,0 +1,438 @@
+// Fused load balance through the owner table, for small inputs.
+//
+// What the reference does (functions_cuda_kernel.cu:97-167, tensor_load_balance.py:13-51): every selected index goes
+// into a hash table as large as the gradient, and the table, read in slot order, is the output.  For a few million
+// slots at most that is also the quickest way: the table fits the caches, nothing has to be sorted, and the steps
+// are few (the sort-based resolution took 23 launches, most of them waiting for the one before):
+//   k_table_insert  selects while it reads the tensor and inserts with atomicMax on 0 - index (a slot belongs to the
+//                   smallest index that ever probes it; who takes a slot from a larger index continues that index's
+//                   probes, as in zen_balance.hip); an index that is out of levels takes a ticket of its partition's
+//                   serial region;
+//   k_table_count   occupied slots per stretch of the table;
+//   k_table_out     entries in slot order to their places, serial tails, split sizes; empties the table again.
+// Up to kOneSlots slots the table is kept in LDS and one workgroup does all of it (k_table_one).
+// Bound by latency: 1 Mi slots, 1 % selected: 5 + 3 + 5 us.
+#include "zen_balance.h"
+
+namespace zen {
+namespace {
+
+constexpr int kInsBlock = 512;
+constexpr int kOutBlock = 256;
+constexpr int kOutRows = 4;                                 // rows of 256 slots per wave
+constexpr uint32_t kStretch = kOutBlock / 64 * kOutRows * 256;  // slots per workgroup (4096)
+constexpr int kMaxParts = 1024;
+constexpr int kOneBlock = 1024;
+constexpr uint32_t kOneSlots = 32768;                       // 128 KB of LDS
+constexpr int kOneParts = 256;
+constexpr uint32_t kOneSerial = 3456;                       // more than a tenth of kOneSlots: more would be an overflow
+
+__device__ inline uint32_t scan64(uint32_t x) {  // inclusive prefix sum across the 64 lanes
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);
+  return x;
+}
+
+// Inserts index t.  Returns the index that ends up without a slot (0: none) and its partition.
+__device__ inline uint32_t insert(uint32_t *table, const Probe &g, uint32_t t, uint32_t *part) {
+  uint32_t cur = t;
+  int lv = 0;
+  for (;;) {
+    const uint32_t slot = probe_slot(g, cur, lv, part);
+    const uint32_t mine = 0u - cur;
+    const uint32_t old = atomicMax(&table[slot], mine);
+    if (old > mine) {  // a smaller index owns the slot: cur moves on
+      if (++lv >= g.levels) return cur;
+      continue;
+    }
+    if (old == 0u || old == mine) return 0;
+    // took the slot from a larger index, which goes on behind its first level that maps here
+    cur = 0u - old;
+    lv = 0;
+    while (lv < g.levels && probe_slot(g, cur, lv, part) != slot) ++lv;
+    if (++lv >= g.levels) return cur;
+  }
+}
+
+__device__ inline uint32_t least_key(const uint32_t *thr, uint32_t mask) {
+  uint32_t t = thr ? thr[0] : 1u;
+  if (t == 0) t = 1;
+  return t > mask ? mask + 1u : t;
+}
+
+struct Tables {
+  uint32_t *slots;       // [m] the caller's table, zero between calls
+  unsigned long long *splits;  // [P], zero: serial tickets in the upper halves while the indices are inserted
+  uint32_t *serial;      // [P * ser_cap] indices without a slot
+  uint32_t *serial_n;    // [P]
+  uint32_t *found;       // [stretches]
+  uint32_t ser_cap;
+  int parts;
+  int64_t spp;           // serial slots of the reference's table, per partition
+};
+
+template <typename S, bool ALIGNED>
+__global__ __launch_bounds__(kInsBlock) void k_table_insert(const S *__restrict__ in, int64_t n,
+                                                            const uint32_t *__restrict__ thr, Probe g, Tables tb,
+                                                            int32_t *status) {
+  // the selected indices of the workgroup's stretch side by side, so that every thread has one to insert
+  constexpr int V = VecOf<S>::kN;
+  __shared__ uint32_t list[kInsBlock * V];
+  __shared__ uint32_t count;
+  if (threadIdx.x == 0) count = 0;
+  const uint32_t least = least_key(thr, KeyOf<S>::kMask);
+  const int64_t first = ((int64_t)blockIdx.x * kInsBlock + threadIdx.x) * V;
+  S e[V];
+  load_vec<S, ALIGNED>(in, first, n, e);
+  uint32_t flags = 0;
+#pragma unroll
+  for (int i = 0; i < V; ++i) flags |= (uint32_t)((uint32_t)(e[i] & KeyOf<S>::kMask) >= least) << i;
+  if (first == 0) flags &= ~1u;  // index 0 is never transmitted
+  const uint32_t c = (uint32_t)__popc(flags);
+  const uint32_t incl = scan64(c);
+  __syncthreads();
+  uint32_t at = 0;
+  if (lane_id() == 63 && incl) at = atomicAdd(&count, incl);
+  at = (uint32_t)__builtin_amdgcn_readlane((int)at, 63) + incl - c;
+  while (flags) {
+    list[at++] = (uint32_t)first + (uint32_t)__ffs((int)flags) - 1u;
+    flags &= flags - 1u;
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < count; i += kInsBlock) {
+    uint32_t part;
+    const uint32_t left = insert(tb.slots, g, list[i], &part);
+    if (left) {
+      const uint32_t ticket = (uint32_t)(atomicAdd(&tb.splits[part], 1ull << 32) >> 32);
+      if ((int64_t)ticket >= tb.spp) atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
+      if (ticket < tb.ser_cap) tb.serial[(size_t)part * tb.ser_cap + ticket] = left;
+    }
+  }
+}
+
+// The slots [base, base + 4) of lane `lane` in row r of the wave, those past the table as empty.
+__device__ inline uint4 load_slots(const uint32_t *slots, uint32_t at, uint32_t m) {
+  if (at + 4 <= m) return *reinterpret_cast<const uint4 *>(slots + at);
+  uint4 q = make_uint4(0, 0, 0, 0);
+  if (at < m) q.x = slots[at];
+  if (at + 1 < m) q.y = slots[at + 1];
+  if (at + 2 < m) q.z = slots[at + 2];
+  return q;
+}
+__device__ inline uint32_t occupied(const uint4 &q) {
+  return (q.x ? 1u : 0u) | (q.y ? 2u : 0u) | (q.z ? 4u : 0u) | (q.w ? 8u : 0u);
+}
+__device__ inline uint32_t word_of(const uint4 &q, uint32_t e) {
+  const uint32_t a = e & 1u ? q.y : q.x, b = e & 1u ? q.w : q.z;
+  return e & 2u ? b : a;
+}
+
+__global__ __launch_bounds__(kOutBlock) void k_table_count(Tables tb, uint32_t m) {
+  __shared__ uint32_t part[kOutBlock / 64];
+  const uint32_t base = blockIdx.x * kStretch + (threadIdx.x >> 6) * (kOutRows * 256) + (uint32_t)lane_id() * 4;
+  uint32_t c = 0;
+#pragma unroll
+  for (int r = 0; r < kOutRows; ++r) c += (uint32_t)__popc(occupied(load_slots(tb.slots, base + r * 256, m)));
+  c = wave_sum(c);
+  if (lane_id() == 0) part[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t sum = 0;
+#pragma unroll
+    for (int w = 0; w < kOutBlock / 64; ++w) sum += part[w];
+    tb.found[blockIdx.x] = sum;
+  }
+  if (blockIdx.x == 0)  // the serial tickets leave the split sizes, which count the entries from here on
+    for (int p = threadIdx.x; p < tb.parts; p += kOutBlock) {
+      uint32_t s = (uint32_t)(tb.splits[p] >> 32);
+      if (s > tb.ser_cap) s = tb.ser_cap;
+      tb.serial_n[p] = s;
+      tb.splits[p] = s;
+    }
+}
+
+template <typename S>
+__global__ __launch_bounds__(kOutBlock) void k_table_out(const S *__restrict__ dense, Tables tb, uint32_t m, uint32_t npp,
+                                                         uint32_t stretches, int32_t *__restrict__ out_idx,
+                                                         S *__restrict__ out_val, uint32_t capacity, int32_t *status) {
+  __shared__ uint32_t smem[kOutBlock / 64 + 1];
+  __shared__ uint32_t before_part[kMaxParts + 1];  // serial entries of the partitions before
+  __shared__ uint32_t buf[kSerialLds];
+  __shared__ uint32_t ends_at[kOutBlock];
+  const uint32_t c = blockIdx.x, wave = threadIdx.x >> 6, lane = (uint32_t)lane_id();
+  const uint32_t base = c * kStretch + wave * (kOutRows * 256) + lane * 4;
+  uint4 q[kOutRows];
+#pragma unroll
+  for (int r = 0; r < kOutRows; ++r) q[r] = load_slots(tb.slots, base + r * 256, m);
+  // entries in front of the stretch, and serial entries in front of every partition
+  uint32_t sum = 0, front;
+  for (uint32_t i = threadIdx.x; i < c; i += kOutBlock) sum += tb.found[i];
+  block_exclusive_scan<uint32_t, kOutBlock>(sum, smem, &front);
+  uint32_t carry = 0;
+  for (int p0 = 0; p0 < tb.parts; p0 += kOutBlock) {
+    const int p = p0 + (int)threadIdx.x;
+    const uint32_t s = p < tb.parts ? tb.serial_n[p] : 0u;
+    uint32_t total;
+    const uint32_t ex = block_exclusive_scan<uint32_t, kOutBlock>(s, smem, &total);
+    if (p < tb.parts) before_part[p] = carry + ex;
+    carry += total;
+  }
+  if (threadIdx.x == 0) before_part[tb.parts] = carry;
+  uint32_t mine = 0;
+#pragma unroll
+  for (int r = 0; r < kOutRows; ++r) mine += (uint32_t)__popc(occupied(q[r]));
+  const uint32_t in_wave = wave_sum(mine);
+  if (lane == 0) smem[wave] = in_wave;
+  __syncthreads();
+  uint32_t at = front, all = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < kOutBlock / 64; ++w) {
+    at += w < wave ? smem[w] : 0u;
+    all += smem[w];
+  }
+  // The partitions of the stretch: p_first's entries from its beginning on, ...
+  const uint32_t lo = c * kStretch, hi = lo + kStretch < m ? lo + kStretch : m;  // lo < m
+  const uint32_t p_first = lo / npp, p_last = (hi - 1u) / npp;
+#pragma unroll
+  for (int r = 0; r < kOutRows; ++r) {
+    const uint32_t x = occupied(q[r]);
+    const uint32_t n = (uint32_t)__popc(x), incl = scan64(n);
+    uint32_t pos = at + incl - n;
+    for (uint32_t bits = x; bits; bits &= bits - 1u, ++pos) {
+      const uint32_t e = (uint32_t)__ffs((int)bits) - 1u;
+      const uint32_t t = 0u - word_of(q[r], e);
+      const uint32_t p = p_first == p_last ? p_first : (base + r * 256 + e) / npp;
+      const uint32_t to = pos + before_part[p];
+      if (to < capacity) {
+        out_idx[to] = (int32_t)t;
+        out_val[to] = dense[t];
+      }
+      if (p_first != p_last) atomicAdd(&tb.splits[p], 1ull);
+    }
+    at += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    if (x) {  // leave the table empty again
+      const uint32_t s0 = base + r * 256;
+      if (s0 + 4 <= m) {
+        *reinterpret_cast<uint4 *>(tb.slots + s0) = make_uint4(0, 0, 0, 0);
+      } else {
+        for (uint32_t i = 0; s0 + i < m; ++i) tb.slots[s0 + i] = 0;
+      }
+    }
+  }
+  if (p_first == p_last && threadIdx.x == 0 && all) atomicAdd(&tb.splits[p_first], (unsigned long long)all);
+  if (c == stretches - 1 && threadIdx.x == 0 && front + all + carry > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
+  // the serial tails of the partitions that end in this stretch, in ascending index order
+  for (uint32_t p = p_first; p <= p_last; ++p) {
+    const uint32_t end = (p + 1u) * npp;  // <= m
+    const uint32_t n = before_part[p + 1] - before_part[p];
+    if (end > hi || n == 0) continue;  // (uniform)
+    // entries of the stretch in front of the partition's end
+    uint32_t in_front = 0;
+#pragma unroll
+    for (int r = 0; r < kOutRows; ++r) {
+      const uint32_t s0 = base + r * 256;
+      const uint32_t keep = s0 >= end ? 0u : end - s0 >= 4u ? 15u : (1u << (end - s0)) - 1u;
+      in_front += (uint32_t)__popc(occupied(q[r]) & keep);
+    }
+    uint32_t total;
+    __syncthreads();
+    block_exclusive_scan<uint32_t, kOutBlock>(in_front, ends_at, &total);
+    const uint32_t to = front + total + before_part[p];
+    if (to + n <= capacity) {
+      for (uint32_t i = threadIdx.x; i < n; i += kOutBlock) {
+        out_idx[to + i] = (int32_t)tb.serial[(size_t)p * tb.ser_cap + i];
+        out_val[to + i] = dense[tb.serial[(size_t)p * tb.ser_cap + i]];
+      }
+      __syncthreads();
+      fix_serial_tail<S>(out_idx, out_val, dense, to, n, buf);
+      __syncthreads();
+    }
+  }
+}
+
+template <typename S, bool ALIGNED>
+__global__ __launch_bounds__(kOneBlock) void k_table_one(const S *__restrict__ in, uint32_t n,
+                                                         const uint32_t *__restrict__ thr, Probe g, int parts, int64_t spp,
+                                                         int32_t *__restrict__ out_idx, S *__restrict__ out_val,
+                                                         uint32_t capacity, int64_t *__restrict__ splits,
+                                                         int32_t *status) {
+  constexpr int V = VecOf<S>::kN;
+  __shared__ __attribute__((aligned(16))) uint32_t slots[kOneSlots];
+  __shared__ uint32_t serial[kOneSerial];       // partition << 15 | index
+  __shared__ uint32_t held[kOneParts], left[kOneParts], before_left[kOneParts];
+  __shared__ uint32_t smem[kOneBlock / 64 + 1];
+  __shared__ uint32_t serial_n;
+  const uint32_t m = g.m;
+  const uint32_t words = (m + 3u) / 4u * 4u;
+  for (uint32_t i = threadIdx.x * 4; i < words; i += kOneBlock * 4) *reinterpret_cast<uint4 *>(slots + i) = make_uint4(0, 0, 0, 0);
+  if (threadIdx.x < kOneParts) held[threadIdx.x] = left[threadIdx.x] = 0;
+  if (threadIdx.x == 0) serial_n = 0;
+  const uint32_t least = least_key(thr, KeyOf<S>::kMask);
+  __syncthreads();
+  for (uint32_t first = threadIdx.x * V; first < n; first += kOneBlock * V) {
+    S e[V];
+    load_vec<S, ALIGNED>(in, first, n, e);
+#pragma unroll 1
+    for (int i = 0; i < V; ++i) {
+      const uint32_t t = first + (uint32_t)i;
+      if ((uint32_t)(e[0] & KeyOf<S>::kMask) >= least && t != 0) {
+        uint32_t part;
+        const uint32_t out = insert(slots, g, t, &part);
+        if (out) {
+          const uint32_t at = atomicAdd(&serial_n, 1u);
+          if (at < kOneSerial) {
+            serial[at] = (part << 15) | out;
+            atomicAdd(&left[part], 1u);
+          } else {
+            atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);  // some partition has more than its tenth
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j + 1 < V; ++j) e[j] = e[j + 1];  // (the loop's body once, not once per element)
+    }
+  }
+  __syncthreads();
+  const uint32_t total_left = serial_n < kOneSerial ? serial_n : kOneSerial;
+  if (total_left > 1) sort_network(serial, total_left);
+  {
+    const uint32_t s = threadIdx.x < kOneParts ? left[threadIdx.x] : 0u;
+    uint32_t total;
+    const uint32_t ex = block_exclusive_scan<uint32_t, kOneBlock>(s, smem, &total);
+    if (threadIdx.x < kOneParts) before_left[threadIdx.x] = ex;
+    if ((int64_t)s > spp) atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
+  }
+  // a wave's slots: a sixteenth of the table, in rows of 256
+  const uint32_t wave = threadIdx.x >> 6, lane = (uint32_t)lane_id();
+  const uint32_t rows = (m + 16 * 256 - 1) / (16 * 256);
+  const uint32_t base = wave * rows * 256 + lane * 4;
+  uint32_t mine = 0;
+  for (uint32_t r = 0; r < rows; ++r) mine += (uint32_t)__popc(base + r * 256 < words ? occupied(*reinterpret_cast<const uint4 *>(slots + base + r * 256)) : 0u);
+  const uint32_t in_wave = wave_sum(mine);
+  __syncthreads();
+  if (lane == 0) smem[wave] = in_wave;
+  __syncthreads();
+  uint32_t at = 0, all = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < kOneBlock / 64; ++w) {
+    at += w < wave ? smem[w] : 0u;
+    all += smem[w];
+  }
+  for (uint32_t r = 0; r < rows; ++r) {
+    const uint32_t s0 = base + r * 256;
+    const uint4 q = s0 < words ? *reinterpret_cast<const uint4 *>(slots + s0) : make_uint4(0, 0, 0, 0);
+    const uint32_t x = occupied(q), c = (uint32_t)__popc(x), incl = scan64(c);
+    uint32_t pos = at + incl - c;
+    for (uint32_t bits = x; bits; bits &= bits - 1u, ++pos) {
+      const uint32_t e = (uint32_t)__ffs((int)bits) - 1u;
+      const uint32_t t = 0u - word_of(q, e), p = (s0 + e) / g.npp;
+      atomicAdd(&held[p], 1u);
+      const uint32_t to = pos + before_left[p];
+      if (to < capacity) {
+        out_idx[to] = (int32_t)t;
+        out_val[to] = in[t];
+      }
+    }
+    at += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+  }
+  __syncthreads();
+  {
+    const uint32_t h = threadIdx.x < kOneParts ? held[threadIdx.x] : 0u;
+    uint32_t total;
+    const uint32_t ex = block_exclusive_scan<uint32_t, kOneBlock>(h, smem, &total);
+    if ((int)threadIdx.x < parts) splits[threadIdx.x] = (int64_t)(h + left[threadIdx.x]);
+    if (threadIdx.x < kOneParts) held[threadIdx.x] = ex + h;  // entries with a slot through the partition
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < total_left; i += kOneBlock) {
+    const uint32_t t = serial[i] & 0x7fffu, to = held[serial[i] >> 15] + i;
+    if (to < capacity) {
+      out_idx[to] = (int32_t)t;
+      out_val[to] = in[t];
+    }
+  }
+  if (threadIdx.x == 0 && all + total_left > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
+}
+
+struct TablePlan {
+  uint32_t *thr;
+  Tables tb;
+  void *topk;
+  uint32_t stretches;
+  size_t bytes;
+};
+
+TablePlan plan_table(void *workspace, int64_t n, int64_t m, int dtype, int partitions) {
+  Carver cv(workspace);
+  TablePlan p{};
+  p.thr = cv.take<uint32_t>(2);
+  p.stretches = (uint32_t)ceil_div(m, (int64_t)kStretch);
+  const int64_t spp = n / partitions / 10;
+  p.tb.ser_cap = (uint32_t)(spp > 64 ? spp : 64);
+  p.tb.serial = cv.take<uint32_t>((size_t)p.tb.ser_cap * partitions);
+  p.tb.serial_n = cv.take<uint32_t>((size_t)partitions);
+  p.tb.found = cv.take<uint32_t>(p.stretches);
+  p.topk = cv.take<char>(topk_whole_bytes(n, dtype));
+  p.tb.parts = partitions;
+  p.tb.spp = spp;
+  p.bytes = cv.used;
+  return p;
+}
+
+template <typename S, bool ALIGNED>
+int table_launch(const SlabBalanceArgs &a, const TablePlan &p, const uint32_t *thr, bool zeroed, hipStream_t s) {
+  const S *in = static_cast<const S *>(a.input);
+  S *out_val = static_cast<S *>(a.out_val);
+  if (a.g.m <= kOneSlots && a.n <= (int64_t)kOneSlots && a.partitions <= kOneParts) {
+    k_table_one<S, ALIGNED><<<dim3(1), dim3(kOneBlock), 0, s>>>(in, (uint32_t)a.n, thr, a.g, a.partitions, a.spp, a.out_idx,
+                                                               out_val, (uint32_t)a.capacity, a.splits, a.status);
+    ZEN_LAUNCH_CHECK("k_table_one");
+    return ZEN_OK;
+  }
+  if (!zeroed) launch_fill<int64_t>(a.splits, 0, (size_t)a.partitions, s);
+  const int64_t blocks = ceil_div(a.n, (int64_t)kInsBlock * VecOf<S>::kN);
+  k_table_insert<S, ALIGNED><<<dim3((unsigned)blocks), dim3(kInsBlock), 0, s>>>(in, a.n, thr, a.g, p.tb, a.status);
+  ZEN_LAUNCH_CHECK("k_table_insert");
+  k_table_count<<<dim3(p.stretches), dim3(kOutBlock), 0, s>>>(p.tb, a.g.m);
+  ZEN_LAUNCH_CHECK("k_table_count");
+  k_table_out<S><<<dim3(p.stretches), dim3(kOutBlock), 0, s>>>(in, p.tb, a.g.m, a.g.npp, p.stretches, a.out_idx, out_val,
+                                                              (uint32_t)a.capacity, a.status);
+  ZEN_LAUNCH_CHECK("k_table_out");
+  return ZEN_OK;
+}
+
+}  // namespace
+
+// Tables of up to 4 Mi slots (16 MB: two readings of it cost less than the wide buckets' resident kernel, 30 us);
+// a top-k selection, whose threshold takes launches of its own here, only where the wide buckets do not apply.
+bool table_balance_fits(int64_t n, int64_t m, int partitions, int64_t k) {
+  const int64_t most = k > 0 ? (1ll << 20) - 1 : 1ll << 22;
+  return n <= (1ll << 22) && m <= most && partitions <= kMaxParts;
+}
+
+size_t table_balance_bytes(int64_t n, int64_t m, int dtype, int partitions) {
+  return table_balance_fits(n, m, partitions, 0) ? plan_table(nullptr, n, m, dtype, partitions).bytes : 0;
+}
+
+int table_load_balance(const SlabBalanceArgs &a, bool splits_zero, hipStream_t s) {
+  TablePlan p = plan_table(a.workspace, a.n, a.g.m, a.dtype, a.partitions);
+  p.tb.slots = reinterpret_cast<uint32_t *>(a.hash);
+  p.tb.splits = reinterpret_cast<unsigned long long *>(a.splits);
+  const uint32_t *thr = a.thr;
+  if (a.k > 0) {
+    uint32_t *to = a.thr_out ? a.thr_out : p.thr;
+    const int rc = topk_whole(a.input, a.dtype, a.n, a.k, to, p.topk, s);
+    if (rc != ZEN_OK) return rc;
+    thr = to;
+  }
+  const bool aligned = (reinterpret_cast<uintptr_t>(a.input) & 15u) == 0;
+  if (a.dtype == ZEN_BF16)
+    return aligned ? table_launch<uint16_t, true>(a, p, thr, splits_zero, s) : table_launch<uint16_t, false>(a, p, thr, splits_zero, s);
+  return aligned ? table_launch<uint32_t, true>(a, p, thr, splits_zero, s) : table_launch<uint32_t, false>(a, p, thr, splits_zero, s);
+}
+
+}  // namespace zen

@@ -29,10 +29,12 @@ constexpr uint32_t kWideCursorWords = kWideMaxBuckets * kWideSplit * kWidePad;
 
 // Buckets for `partitions` partitions of a key space of m keys expected to hold about `expected` records, on
 // a chip of `cus` compute units; false if the layout does not suit these sizes.  The result is a SlabGeom
-// whose sub_shift refers to kWideSubs narrow ranges.
-inline bool wide_geometry(int64_t m, int partitions, int64_t expected, int cus, SlabGeom *out) {
-  // a table of 4 MB or more: the map at its head takes at most half, the counters behind it less than 1 MB
-  if (m < (1ll << 20) || m > 0x7fffffffll || partitions < 1 || partitions > kWideMaxBuckets || m % partitions != 0 ||
+// whose sub_shift refers to kWideSubs narrow ranges.  least_m: the encode keeps its counters in the caller's table
+// (4 MB or more: the map at its head takes at most half, the counters behind it less than 1 MB); least_width: keys of
+// a bucket, at least.
+inline bool wide_geometry(int64_t m, int partitions, int64_t expected, int cus, SlabGeom *out,
+                          int64_t least_m = 1ll << 20, int64_t least_width = 4ll * kWideSubs) {
+  if (m < least_m || m > 0x7fffffffll || partitions < 1 || partitions > kWideMaxBuckets || m % partitions != 0 ||
       expected < 1)
     return false;
   int64_t most = cus < kWideMaxBuckets ? cus : kWideMaxBuckets;
@@ -41,7 +43,7 @@ inline bool wide_geometry(int64_t m, int partitions, int64_t expected, int cus, 
   if (most >= 2 * partitions && expected <= most / 2 * (int64_t)kWideTarget) most /= 2;
   int64_t bpp = most / partitions;
   const int64_t npp = m / partitions;
-  if (bpp > npp / (4 * (int64_t)kWideSubs)) bpp = npp / (4 * (int64_t)kWideSubs);  // buckets wider than their sub-ranges
+  if (bpp > npp / least_width) bpp = npp / least_width;
   if (bpp < 1) return false;
   const int64_t nb = bpp * partitions;
   if (expected / nb > (int64_t)kWideTarget) return false;
@@ -288,6 +290,12 @@ bool wide_merge_fits(int64_t r, int64_t dense_n, int cus, SlabGeom *geo);
 size_t wide_merge_bytes(int64_t r, int64_t dense_n, int cus);
 bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, int64_t dense_n, uint32_t *cursor,
                      void *rest, int cus, int32_t *status, WideList *list);
+// One workgroup straight from the list, for up to wide_merge_one_max() entries (kWideCap would fit; from about here
+// on the scatter's launch costs less than the longer chains of one workgroup): no slabs, no zeroed memory.
+constexpr int64_t wide_merge_one_max() { return 4096; }
+int wide_merge_one(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n, void *out_idx,
+                   int idx64_out, void *out_val, int out_dtype, int64_t capacity, int64_t *out_count, int32_t *status,
+                   hipStream_t s);
 int wide_merge(const WideList &list, int dtype, void *out_idx, int idx64_out, void *out_val, int out_dtype,
                int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s);
 

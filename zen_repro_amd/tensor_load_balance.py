@@ -319,8 +319,8 @@ class TensorPartition:
             thr, flags = near, flags | _lib.MODE_FLOOR
         rc = L.zen_load_balance(
             _lib.ptr(flat), code, n, m, self.partitions, self.rehash, _lib.ptr(thr), int(k), _lib.ptr(thr_out),
-            _lib.ptr(out_idx), _lib.ptr(out_val), capacity, _lib.ptr(splits), _lib.ptr(table), mode | flags,
-            _lib.ptr(ws), ws.numel(), _lib.ptr(status), _lib.stream_of(dev))
+            _lib.ptr(out_idx), _lib.ptr(out_val), capacity, _lib.ptr(splits), _lib.ptr(table),
+            mode | flags | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status), _lib.stream_of(dev))
         if rc != _lib.OK:
             table.zero_()  # a call that failed half way may have left entries behind
         _lib.check(rc, "load_balance")
