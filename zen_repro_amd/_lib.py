@@ -155,12 +155,19 @@ def dtype_code(t):
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    """What a void * argument takes: the address, or None."""
+    return t.data_ptr() if t is not None else None
 
 
 def device_index(device):
     """Index of a torch device (or of the current one if it names none)."""
-    index = device.index if isinstance(device, torch.device) else torch.device(device).index
+    try:
+        index = device.index
+        if index.__class__ is int:
+            return index
+    except AttributeError:
+        pass
+    index = torch.device(device).index
     return index if index is not None else torch.cuda.current_device()
 
 
@@ -176,14 +183,15 @@ def stream_handle(device):
 
 
 def stream_of(device):
-    return ctypes.c_void_p(stream_handle(device))
+    return stream_handle(device)
 
 
 def require_gpu(t, name):
     # extensions/cuda/functions.py:5-7 asserts; functions_cuda.cpp:11-13 raises RuntimeError
+    if t.is_cuda and t.is_contiguous():
+        return
     assert t.is_cuda, f"{name} must be a GPU tensor"
-    if not t.is_contiguous():
-        raise RuntimeError(f"{name} must be contiguous")
+    raise RuntimeError(f"{name} must be contiguous")
 
 
 class Scratch:
@@ -204,7 +212,10 @@ class Scratch:
 
     def get(self, device, name, nbytes, zero=False):
         key = (device_index(device), name)
-        bufs = self._bufs()
+        try:
+            bufs = self._local.bufs
+        except AttributeError:
+            bufs = self._bufs()
         buf = bufs.get(key)
         if buf is None or buf.numel() < nbytes:
             alloc = torch.zeros if zero else torch.empty
@@ -231,11 +242,29 @@ class ZeroPool:
 
     BLOCK = 1 << 16
     ALIGN = 16
+    WORDS = 4096  # of one type to a block of single words
 
     def __init__(self):
         self._local = threading.local()
 
     _SIZES = {torch.int32: 4, torch.int64: 8, torch.uint8: 1, torch.float32: 4}
+
+    def _blocks(self):
+        blocks = getattr(self._local, "blocks", None)
+        if blocks is None:
+            blocks = self._local.blocks = {}
+        return blocks
+
+    def word(self, device, dtype):
+        """take(device, 1, dtype) for int32 and int64, which calls need most."""
+        blocks = self._blocks()
+        key = (device_index(device), stream_handle(device), dtype)
+        entry = blocks.get(key)
+        if entry is None or entry[1] == self.WORDS:
+            entry = blocks[key] = [torch.zeros(self.WORDS, dtype=dtype, device=device), 0]
+        at = entry[1]
+        entry[1] = at + 1
+        return entry[0][at:at + 1]
 
     def take(self, device, count, dtype):
         size = self._SIZES.get(dtype)
@@ -244,9 +273,7 @@ class ZeroPool:
         nbytes = count * size
         if nbytes > self.BLOCK // 4:
             return torch.zeros(count, dtype=dtype, device=device)
-        blocks = getattr(self._local, "blocks", None)
-        if blocks is None:
-            blocks = self._local.blocks = {}
+        blocks = self._blocks()
         key = (device_index(device), stream_handle(device))
         entry = blocks.get(key)
         if entry is None or entry[1] + nbytes > self.BLOCK:
@@ -264,16 +291,17 @@ class ZeroPool:
         """Forget the current stream's block: the next piece comes from a new one.  Call this at the start of
         every HIP graph capture: the block made inside the capture, fill included, then belongs to that graph
         alone (its replays put its own status words and counts back to zero and nobody else's)."""
-        blocks = getattr(self._local, "blocks", None)
-        if blocks is not None:
-            blocks.pop((device_index(device), stream_handle(device)), None)
+        blocks = self._blocks()
+        key = (device_index(device), stream_handle(device))
+        for k in [k for k in blocks if k[:2] == key]:
+            del blocks[k]
 
 
 zeros = ZeroPool()
 
 
 def status_word(device):
-    return zeros.take(device, 1, torch.int32)
+    return zeros.word(device, torch.int32)
 
 
 class _HostWords:
@@ -292,21 +320,29 @@ class _HostWords:
 
 
 _host = threading.local()
+_NO_SEGMENT = [(None, 0, 0) * (3 - n) for n in range(4)]
 
 
 def read_back(*tensors):
     """The values of up to three small contiguous int32 / int64 device tensors (split sizes, counts, status
     words), one list after the other, once the current stream has got there.  The way a call on this path
     waits for the device: one kernel instead of a conversion, a concatenation and a copy."""
-    n = sum(t.numel() for t in tensors)
-    words = getattr(_host, "words", None)
+    args = []
+    n = 0
+    for t in tensors:
+        count = t.numel()
+        n += count
+        args += (t.data_ptr(), count, 1 if t.dtype is torch.int64 else 0)
+    args += _NO_SEGMENT[len(tensors)]
+    try:
+        words = _host.words
+    except AttributeError:
+        words = None
     if words is None or words.words <= n:
         words = _host.words = _HostWords(max(1024, 2 * n))
-    args = []
-    for t in tensors:
-        args += (t.data_ptr(), t.numel(), 1 if t.dtype == torch.int64 else 0)
-    args += (None, 0, 0) * (3 - len(tensors))
-    check(lib().zen_read_back(*args, words.ptr, words.words, stream_handle(tensors[0].device)), "read_back")
+    rc = _lib.zen_read_back(*args, words.ptr, words.words, stream_handle(tensors[0].device))
+    if rc:
+        check(rc, "read_back")
     return words.view[1:n + 1]
 
 

@@ -38,7 +38,7 @@ def _select_raw(tensor, thr, idx64, capacity=None):
     code = _lib.dtype_code(flat)
     out_idx = torch.empty(capacity, dtype=torch.int64 if idx64 else torch.int32, device=dev)
     out_val = torch.empty(capacity, dtype=flat.dtype, device=dev)
-    count = _lib.zeros.take(dev, 1, torch.int64)
+    count = _lib.zeros.word(dev, torch.int64)
     status = _lib.status_word(dev)
     ws = _lib.scratch.get(dev, "select", L.zen_select_workspace(n, code))
     rc = L.zen_select(_lib.ptr(flat), code, n, _lib.ptr(thr), _lib.ptr(out_idx), 1 if idx64 else 0,
@@ -75,7 +75,7 @@ class LoadBalanceAllreduce:
         self.tensor_partition = self.get_tensor_partition_obj(memory_scale, rehash)
         self.logger = logger
         self.mapping = {}
-        self._step_sizes = {}    # shape of an encode_merge_flat call -> (table size, workspace bytes, merge workspace bytes)
+        self._step_sizes = {}    # shape of an encode_merge_flat call -> (table size, workspace bytes, merge workspace bytes, its arguments)
         self._bitmap_ranks = {}  # numel -> (mapping list of this rank, its rank table)
         self._dense_dicts = {}   # numel -> dictionary of decode_bitmaps_dense
 
@@ -203,7 +203,7 @@ class LoadBalanceAllreduce:
             mode |= self.fast_flags
         out_idx = torch.empty(capacity, dtype=torch.int64 if idx64 else torch.int32, device=dev)
         out_val = torch.empty(capacity, dtype=values.dtype if rounded else torch.float32, device=dev)
-        count = _lib.zeros.take(dev, 1, torch.int64)
+        count = _lib.zeros.word(dev, torch.int64)
         status = _lib.status_word(dev)
         # The workspace is allocated zeroed and serves zen_merge only, which leaves its head (the counters
         # that must start at zero) zero again: no call spends a kernel on clearing it.
@@ -230,8 +230,6 @@ class LoadBalanceAllreduce:
         it has this tensor's type, the pass over this tensor takes the sample of that call along (no kernel of
         its own), as if partition.prepare(next_tensor, next_k, next_capacity, slot) had been called
         (`next_capacity`: that call's capacity, default this call's; gradient buckets differ in size)."""
-        from .tensor_load_balance import TensorPartition  # noqa: F401 (the type of `partition`)
-
         _lib.require_gpu(tensor, "input")
         flat = tensor.reshape(-1)
         indices = self.stack_tensors(recv_indices)
@@ -250,17 +248,16 @@ class LoadBalanceAllreduce:
         if sizes is None:
             m = partition.table_sizes(n)[0]
             sizes = self._step_sizes[shape] = (m, L.zen_load_balance_workspace(n, m, code, capacity, P),
-                                               L.zen_merge_workspace(r, dense_size))
-        m, ws_bytes, mws_bytes = sizes
+                                               L.zen_merge_workspace(r, dense_size), None)
+        m, ws_bytes, mws_bytes = sizes[:3]
         mode = _lib.MODE_FAST | partition.fast_flags
         out_idx = torch.empty(capacity, dtype=torch.int32, device=dev)
         out_val = torch.empty(capacity, dtype=flat.dtype, device=dev)
         m_idx = torch.empty(r, dtype=torch.int32, device=dev)
         m_val = torch.empty(r, dtype=torch.float32, device=dev)
         small = _lib.zeros.take(dev, P + 2, torch.int64)  # split sizes, merged count, the two status words
-        splits, count = small[:P], small[P:P + 1]
-        status2 = small[P + 1:P + 2].view(torch.int32)
-        status, m_status = status2[0:1], status2[1:2]
+        splits, count, status2 = small.split((P, 1, 1))
+        status, m_status = status2.view(torch.int32).split(1)
         if next_k is None:
             next_k = k
         if next_capacity is None:
@@ -284,17 +281,50 @@ class LoadBalanceAllreduce:
         nxt, nxt_table = partition._next_sample(flat, next_tensor, int(next_k), capacity, next_capacity, slot,
                                                 mode | flags, used)
         other = nxt is not None and nxt_table is not None
-        a = _lib.EncodeMergeArgs(
-            flat.data_ptr(), code, n, m, P, partition.rehash, thr.data_ptr() if thr is not None else None, int(k),
-            thr_out.data_ptr() if thr_out is not None else None, out_idx.data_ptr(), out_val.data_ptr(), capacity,
-            splits.data_ptr(), table.data_ptr(), mode | flags | _lib.MODE_ZEROED, ws.data_ptr(), ws.numel(), status.data_ptr(),
-            indices.data_ptr(), int(indices.dtype == torch.int64), values.data_ptr(), r, dense_size,
-            m_idx.data_ptr(), 0, m_val.data_ptr(), r, count.data_ptr(),
-            _lib.MODE_FAST | self.fast_flags | _lib.MODE_ZEROED, mws.data_ptr(), mws.numel(), m_status.data_ptr(),
-            _lib.stream_handle(dev), merge_stream.cuda_stream if merge_stream is not None else None,
-            nxt.data_ptr() if nxt is not None else None, int(next_k) if nxt is not None else 0,
-            nxt.numel() if other else 0, nxt_table.numel() if other else 0, next_capacity if other else 0,
-            nxt_table.data_ptr() if other else None)
+        # what only depends on the call's shape is filled in once; a copy of it takes the rest
+        base = sizes[3]
+        if base is None:
+            base = _lib.EncodeMergeArgs(dtype=code, n=n, m=m, partitions=P, rehash=partition.rehash, capacity=capacity,
+                                        r=r, dense_n=dense_size, merged_capacity=r)
+            sizes = self._step_sizes[shape] = sizes[:3] + (base,)
+        a = _lib.EncodeMergeArgs.from_buffer_copy(base)
+        a.input = flat.data_ptr()
+        a.rehash = partition.rehash
+        if thr is not None:
+            a.thr = thr.data_ptr()
+        a.k = int(k)
+        if thr_out is not None:
+            a.thr_out = thr_out.data_ptr()
+        a.out_idx = out_idx.data_ptr()
+        a.out_val = out_val.data_ptr()
+        at = small.data_ptr()
+        a.splits = at
+        a.table = table.data_ptr()
+        a.mode = mode | flags | _lib.MODE_ZEROED
+        a.workspace = ws.data_ptr()
+        a.workspace_bytes = ws.numel()
+        a.status = at + 8 * (P + 1)
+        a.recv_idx = indices.data_ptr()
+        a.recv_idx64 = indices.dtype is torch.int64
+        a.recv_val = values.data_ptr()
+        a.merged_idx = m_idx.data_ptr()
+        a.merged_val = m_val.data_ptr()
+        a.merged_count = at + 8 * P
+        a.merge_mode = _lib.MODE_FAST | self.fast_flags | _lib.MODE_ZEROED
+        a.merge_workspace = mws.data_ptr()
+        a.merge_workspace_bytes = mws.numel()
+        a.merge_status = at + 8 * (P + 1) + 4
+        a.stream = _lib.stream_handle(dev)
+        if merge_stream is not None:
+            a.merge_stream = merge_stream.cuda_stream
+        if nxt is not None:
+            a.next_input = nxt.data_ptr()
+            a.next_k = int(next_k)
+            if other:
+                a.next_n = nxt.numel()
+                a.next_m = nxt_table.numel()
+                a.next_capacity = next_capacity
+                a.next_table = nxt_table.data_ptr()
         self.last_encode_merge_args = a  # what the library was called with (its buffers live as long as the results)
         rc = L.zen_encode_merge(ctypes.byref(a))
         if rc != _lib.OK:
@@ -315,7 +345,7 @@ class LoadBalanceAllreduce:
         cap = indices.numel()
         out_idx = torch.empty_like(indices)
         out_val = torch.empty(cap, dtype=dtype, device=dev)
-        kept = _lib.zeros.take(dev, 1, torch.int64)
+        kept = _lib.zeros.word(dev, torch.int64)
         status = _lib.status_word(dev)
         ws = _lib.scratch.get(dev, "round_compact", L.zen_round_compact_workspace(cap))
         rc = L.zen_round_compact(_lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(sums), _lib.ptr(count),
@@ -602,12 +632,19 @@ def _as_one_buffer(tensors):
     first = tensors[0]
     if first.dim() != 1 or not first.is_contiguous():
         return None
+    dtype, base, size = first.dtype, first._base, first.element_size()
+    storage = None
+    at = first.data_ptr()
     total = 0
-    base = first.data_ptr()
     for t in tensors:
-        if (t.dim() != 1 or t.dtype != first.dtype or not t.is_contiguous()
-                or t.untyped_storage().data_ptr() != first.untyped_storage().data_ptr()
-                or t.data_ptr() != base + total * first.element_size()):
+        if t.dtype != dtype or t.data_ptr() != at or t.dim() != 1 or not t.is_contiguous():
             return None
-        total += t.numel()
+        if base is None or t._base is not base:  # not views of one tensor: of one storage all the same?
+            if storage is None:
+                storage = first.untyped_storage().data_ptr()
+            if t.untyped_storage().data_ptr() != storage:
+                return None
+        count = t.numel()
+        total += count
+        at += count * size
     return torch.as_strided(first, (total,), (1,))

@@ -9,11 +9,14 @@ compressed bucket, as the reference does when dp_group.size() == 1
 Stream order: the reference switches to its side stream and completes the
 future at once (train.py:165-181), leaving it to host time that the gradients
 are written before the hook reads them and that the result is complete before
-it is used.  Here the side stream first waits for the caller's current stream
-(whatever produced the bucket there has finished before the path reads it), and
-the caller's current stream waits for the side stream before the hook returns
-(whatever consumes the future's tensor in that stream's order finds it
-complete).  Neither wait blocks the host."""
+it is used.  Here a side stream that the caller names first waits for the caller's
+current stream (whatever produced the bucket there has finished before the path
+reads it), and the caller's current stream waits for the side stream before the
+hook returns (whatever consumes the future's tensor in that stream's order
+finds it complete).  Neither wait blocks the host.  Between those two waits
+nothing of the caller's can run beside the path anyway, and each costs the host
+some 14 us: without a named stream the path runs on the caller's current stream
+and there is nothing to wait for."""
 import torch
 
 from ._lib import annotate
@@ -32,7 +35,8 @@ class SparseCommHook:
                             train.py:63-64); needed only when tp_group has more
                             than one rank
     stream                  the side stream the path runs on (train.py:165);
-                            default priority
+                            default priority.  None: the caller's current one
+                            (the attribute then names the last call's)
     fused                   False: the reference's steps one by one (the bucket
                             is thresholded into a dense copy, the all-reduce
                             reads that copy); True (default): the threshold is
@@ -53,7 +57,8 @@ class SparseCommHook:
         self.method = method
         self.tp_group = tp_group
         self.all_gather = all_gather
-        self.stream = stream if stream is not None else torch.cuda.Stream()
+        self.own_stream = stream is not None
+        self.stream = stream if stream is not None else torch.cuda.current_stream()
         self.sample_index = sample_index  # callable(numel) -> int64 sample positions; None: drawn like the reference
         self.fused = fused
         self.headroom = headroom
@@ -71,25 +76,30 @@ class SparseCommHook:
             raise RuntimeError("SparseCommHook: a group of more than one rank needs a communication backend in "
                                "load_balance_allreduce.ddp")
         caller = torch.cuda.current_stream(tensors.device)
+        if not self.own_stream:
+            self.stream = caller
+            future.set_result(self._reduce(tensors, exchange))
+            return future
         self.stream.wait_stream(caller)
         with torch.cuda.stream(self.stream):
-            index = self.sample_index(tensors.numel()) if self.sample_index is not None else None
-            with annotate("compress"):  # train.py:176 (the masked copy, if one is made, comes below)
-                thr = threshold_with_allgather(self.top_k, tensors, self.tp_group, sample_index=index,
-                                               all_gather=self.all_gather)
-            if thr is None:  # a small bucket: not compressed (train.py:58-59)
-                if exchange:
-                    tensors = self.lba.zen_sparse_comm(tensors, self.method)
-            elif exchange and self.fused:
-                # about top_k per cent of the bucket pass the sampled threshold; the call grows its buffers if more do
-                room = int(tensors.numel() * self.top_k / 100 * self.headroom) + 4096
-                tensors = self.lba.zen_sparse_comm(tensors, self.method, thr=thr, capacity=min(room, tensors.numel()))
-            else:
-                tensors = mask_below(tensors.reshape(-1), thr).view_as(tensors)
-                if exchange:
-                    tensors = self.lba.zen_sparse_comm(tensors, self.method)
+            tensors = self._reduce(tensors, exchange)
         caller.wait_stream(self.stream)
         # like the reference, the future is completed at once (train.py:181): its tensor is complete in the
         # order of the caller's stream and of `self.stream`
         future.set_result(tensors)
         return future
+
+    def _reduce(self, tensors, exchange):
+        """The bucket after compression and, with more than one rank, the exchange, on the current stream."""
+        index = self.sample_index(tensors.numel()) if self.sample_index is not None else None
+        with annotate("compress"):  # train.py:176 (the masked copy, if one is made, comes below)
+            thr = threshold_with_allgather(self.top_k, tensors, self.tp_group, sample_index=index,
+                                           all_gather=self.all_gather)
+        if thr is None:  # a small bucket: not compressed (train.py:58-59)
+            return self.lba.zen_sparse_comm(tensors, self.method) if exchange else tensors
+        if exchange and self.fused:
+            # about top_k per cent of the bucket pass the sampled threshold; the call grows its buffers if more do
+            room = int(tensors.numel() * self.top_k / 100 * self.headroom) + 4096
+            return self.lba.zen_sparse_comm(tensors, self.method, thr=thr, capacity=min(room, tensors.numel()))
+        tensors = mask_below(tensors.reshape(-1), thr).view_as(tensors)
+        return self.lba.zen_sparse_comm(tensors, self.method) if exchange else tensors

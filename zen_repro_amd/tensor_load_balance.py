@@ -125,7 +125,7 @@ class TensorPartition:
     @staticmethod
     def _count(flat, thr):
         _lib.require_gpu(flat, "input")
-        count = _lib.zeros.take(flat.device, 1, torch.int64)
+        count = _lib.zeros.word(flat.device, torch.int64)
         _lib.check(_lib.lib().zen_count(_lib.ptr(flat), _lib.dtype_code(flat), flat.numel(), _lib.ptr(thr),
                                         _lib.ptr(count), _lib.stream_of(flat.device)), "count")
         return _lib.read_back(count)[0]
