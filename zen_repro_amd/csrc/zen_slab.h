@@ -30,7 +30,7 @@ constexpr int kSlabGroupLimit = 1024;                 // bounds the rank loop on
 constexpr int kSlabMaxBuckets = 4096;
 constexpr int kSlabTarget = 3584;                     // records a bucket is sized for (leaves 40 % to spare)
 constexpr int kSlabResident = 512;                    // per-bucket workgroups the chip holds at a time (256 CUs x 2)
-constexpr int kSlabMoveCap = 1024;                    // entries that may move into one bucket from elsewhere
+constexpr int kSlabPartLog2 = 10;                     // entries that may move into one bucket from elsewhere, log2
 constexpr int kSlabSerialCap = 4096;                  // overflow entries per partition the fast path carries
 
 struct SlabGeom {
@@ -42,6 +42,7 @@ struct SlabGeom {
   int sub_shift;      // key offset inside a bucket >> sub_shift = narrow range (fewer than kSlabSubs of them)
   float inv_m;        // (1 / m)(1 - 2^-20), rounded down
   float inv_npp;      // the same for npp
+  double width;       // 2^32 / bpp_mult: keys per bucket, to 53 bits
 
   // x / d for x < 2^32 and quotients below 2^11, without the long integer division sequence.  `inv` is
   // (1 / d)(1 - 2^-20): the two roundings of the float estimate (each at most 2^-24, relative) cannot lift it
@@ -66,11 +67,26 @@ struct SlabGeom {
     const uint32_t part = div_small(key, npp, inv_npp, &local);
     return part * bpp + __umulhi(local, bpp_mult);
   }
+  // ceil(sb * 2^32 / bpp_mult), the first local key of a partition's bucket sb.  The product is within 2^-20 of the
+  // true quotient, so rounding it down gives the ceiling or one less.
+  __device__ inline uint32_t first_local(uint32_t sb) const {
+    const uint32_t lo = (uint32_t)((double)sb * width);
+    return lo + (__umulhi(lo, bpp_mult) < sb ? 1u : 0u);
+  }
   __device__ inline uint32_t first_key(uint32_t b) const {  // smallest key of bucket b
     const uint32_t part = b / bpp, sb = b - part * bpp;
-    return part * npp + (uint32_t)((((uint64_t)sb << 32) + bpp_mult - 1) / bpp_mult);
+    return part * npp + first_local(sb);
+  }
+  __device__ inline uint32_t bucket_and_offset(uint32_t key, uint32_t *offset) const {  // key - first_key(bucket)
+    uint32_t local;
+    const uint32_t part = div_small(key, npp, inv_npp, &local);
+    const uint32_t sb = __umulhi(local, bpp_mult);
+    *offset = local - first_local(sb);
+    return part * bpp + sb;
   }
 };
+
+inline double slab_bucket_width(uint32_t bpp_mult) { return 4294967296.0 / (double)bpp_mult; }
 
 // Host side: geometry for `partitions` partitions of a key space of m keys (m a
 // multiple of partitions) expected to hold about `expected` records.  Returns
@@ -110,6 +126,7 @@ inline bool slab_geometry(int64_t m, int partitions, int64_t expected, int targe
   const uint64_t width = ((1ull << 32) + g.bpp_mult - 1) / g.bpp_mult + 1;  // keys per bucket, at most
   g.sub_shift = 0;
   while ((width >> g.sub_shift) >= (uint64_t)kSlabSubs) ++g.sub_shift;
+  g.width = slab_bucket_width(g.bpp_mult);
   g.inv_m = slab_inverse_below(g.m);
   g.inv_npp = slab_inverse_below(g.npp);
   *out = g;

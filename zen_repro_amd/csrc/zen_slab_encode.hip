@@ -5,7 +5,7 @@
 // (functions_cuda_kernel.cu:97-167, tensor_load_balance.py:13-51).  Here the
 // select kernel leaves its candidates in 64 coarse slabs (a coarse slab = the
 // level-1 hash slots of a group of buckets; a bucket is a range of level-1
-// slots, zen_slab.h), and five short kernels finish the job:
+// slots, zen_slab.h), and four short kernels finish the job:
 //   k_fine_scatter  the coarse slabs, filtered by the exact threshold, go to the
 //                   bucket slabs, so that every store belongs to a long run;
 //   k_slab_sort     one workgroup per bucket: sorts
@@ -16,9 +16,10 @@
 //                   with the reference's rule executed in ascending index order
 //                   (a slot belongs to the smallest index that ever probes it;
 //                   whoever takes a slot from a larger index continues that
-//                   index's probe sequence);
-//   k_slab_classify final slot of every logged entry, handed to the bucket that
-//                   slot lies in (or to the partition's serial list);
+//                   index's probe sequence).  Every bucket has a part of the map
+//                   of its own, so what finally moved into a bucket is what its
+//                   part holds; an index that ran out of levels goes to its
+//                   partition's serial list;
 //   k_slab_place    one workgroup per bucket: survivors and moved-in entries
 //                   merged by rank, written to the bucket's place in the
 //                   partition-major output; split sizes.
@@ -36,8 +37,8 @@ struct SlabTables {
   uint32_t *bucket_lo;  // [B] smallest level-1 slot of the bucket
   uint32_t *bucket_n;   // [B] selected records, sorted, in the slab
   uint32_t *removed_n;  // [B] of which lost their level-1 slot
-  uint32_t *movein_n;   // [B] entries whose final slot lies in the bucket but whose level-1 slot does not own it
-  uint32_t *serial_n;   // [P] entries that found no slot
+  uint32_t *movein_n;   // [B * kMoveinPad] occupied cells of the bucket's part of the map
+  uint32_t *serial_n;   // [P * kMoveinPad] entries that found no slot
   uint32_t *raw_idx;    // [B * kSlabCap] entries as they arrive: index ...
   void *raw_val;        // ... and value
   int32_t *slab_idx;    // [B * kSlabCap] after the sort: index | kRemovedBit, by ascending level-1 slot (the slot
@@ -45,20 +46,22 @@ struct SlabTables {
   void *slab_val;       // [B * kSlabCap] after the sort: value
   uint16_t *sub_index;  // [B * kSlabIndexLen] sorted place of the first record of every kSlabIndexStep-th narrow
                         // key range of the bucket (the last entry: the number of records)
-  uint32_t *mv_key, *mv_idx, *mv_val;  // [B * kSlabMoveCap]
   uint32_t *ser_idx;    // [P * kSlabSerialCap]
-  uint32_t *log_t, *log_v, *log_cell;  // [log_cap]
+  uint32_t *log_t;      // [log_cap] indices that lost level 1
   uint32_t *out_start;  // [B + 1] where every bucket starts in the output
-  uint32_t *done;       // [1] workgroups of k_slab_classify that have finished
-  uint32_t *final_n;    // [B + P + 2] what k_slab_place needs of the counters above, copied by the last workgroup of
-                        // k_slab_classify before it puts them back to zero: moved-in entries per bucket, serial
-                        // entries per partition, logged losers, displaced owners
-  Counters *ctr;
+  uint32_t *done;       // [1] workgroups of k_slab_chains that have finished
+  uint32_t *final_n;    // [B + P] what k_slab_place needs of the counters above, copied by the last workgroup of
+                        // k_slab_chains before it puts them back to zero: moved-in entries per bucket, serial
+                        // entries per partition
+  uint32_t *losers;     // [1] entries of log_t
   uint32_t *coarse_cursor;  // the feed's coarse cursors and, for an fp32 top-k, the refinement histogram (else
   uint32_t *refine_hist;    // null): k_slab_sort puts them back to zero
   int partitions;
   uint32_t log_cap;
 };
+
+// Device-wide atomics on one 128-byte line are carried out one after the other: four counters to a line.
+constexpr uint32_t kMoveinPad = 8;
 
 // The counters and histograms that must be zero when a call starts live in memory that is zero between calls
 // (the part of the caller's table the hash map does not use), and every one of them is put back to zero by the
@@ -155,6 +158,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabT
       tb.bucket_n[b] = 0;
       tb.removed_n[b] = 0;
     }
+    for (int j = threadIdx.x; j < kSlabIndexLen; j += kSortBlock) tb.sub_index[(size_t)b * kSlabIndexLen + j] = 0;
     return;
   }
   // every thread has read the slab's fill count (slab_rank synchronised); this workgroup was its only reader
@@ -223,36 +227,35 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabT
   if (threadIdx.x == 0) {
     tb.bucket_n[b] = n;
     tb.removed_n[b] = lost_n;
-    s_base = lost_n ? atomicAdd(&tb.ctr->losers, lost_n) : 0u;
+    s_base = lost_n ? atomicAdd(tb.losers, lost_n) : 0u;
   }
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < lost_n; i += kSortBlock) {
     const uint32_t at = s_base + i;
     const uint32_t p = sh.key[i];
-    if (at < tb.log_cap) {
+    if (at < tb.log_cap)
       tb.log_t[at] = sh.tie[p];
-      tb.log_v[at] = (uint32_t)s_val[p];
-    } else {
+    else
       atomicOr(status, ZEN_STAT_RETRY);
-    }
   }
 }
 
 // ------------------------------------------------------ levels 2 and 3
 
-// Smallest index whose level-1 slot is `slot` (kNone if nobody's), and where it sits.  The bucket's index
+// Smallest index whose level-1 slot is `slot` (kNone if nobody's), where it sits, and the slot's bucket.  The bucket's index
 // narrows the search to the records of kSlabIndexStep narrow ranges (three or four); they are fetched four at
 // a time and looked at in sorted order: by ascending slot, and in a run of equal slots the smallest index
 // comes first.
 __device__ inline uint32_t slab_head(const SlabGeom &geo, const SlabTables &tb, uint32_t slot, size_t *pos_out,
                                      uint32_t *bucket_out) {
-  const uint32_t b = geo.bucket_of(slot);
+  uint32_t off;
+  const uint32_t b = geo.bucket_and_offset(slot, &off);  // computed, not fetched: one trip less in the chain
+  *bucket_out = b;
   const int32_t *idx = tb.slab_idx + (size_t)b * kSlabCap;
-  const uint32_t n = tb.bucket_n[b];
-  const uint32_t j = ((slot - tb.bucket_lo[b]) >> geo.sub_shift) / (uint32_t)kSlabIndexStep;
+  const uint32_t j = (off >> geo.sub_shift) / (uint32_t)kSlabIndexStep;
   const uint16_t *index = tb.sub_index + (size_t)b * kSlabIndexLen;
-  uint32_t p = index[j], end = index[j + 1];
-  if (end > n) end = n;  // a bucket the sort declined has no index (and no records)
+  uint32_t p = index[j];
+  const uint32_t end = index[j + 1];
   for (; p < end; p += 4) {
     uint32_t t[4];
 #pragma unroll
@@ -264,7 +267,6 @@ __device__ inline uint32_t slab_head(const SlabGeom &geo, const SlabTables &tb, 
       if (s1 > slot) return kNone;
       if (s1 == slot) {
         *pos_out = (size_t)b * kSlabCap + p + q;
-        *bucket_out = b;
         return t[q];
       }
     }
@@ -272,89 +274,51 @@ __device__ inline uint32_t slab_head(const SlabGeom &geo, const SlabTables &tb, 
   return kNone;
 }
 
-template <typename S>
-__global__ __launch_bounds__(256) void k_slab_chains(SlabGeom geo, Probe g, SlabTables tb, unsigned long long *cells,
-                                                     uint32_t log2, int32_t *status) {
-  Counters *ctr = tb.ctr;
-  uint32_t losers = ctr->losers;
-  if (losers > tb.log_cap) losers = tb.log_cap;
-  const S *slab_val = static_cast<const S *>(tb.slab_val);
-  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < losers; i += gridDim.x * 256u) {
-    uint32_t cur = tb.log_t[i];
-    int lv = 1;
-    bool full = false;
-    for (uint32_t steps = 0; lv < g.levels; ++steps) {
-      if (steps > kChainLimit) {
-        atomicOr(status, ZEN_STAT_INTERNAL);
-        break;
-      }
-      uint32_t part;
-      const uint32_t slot = probe_slot(g, cur, lv, &part);
-      size_t head_pos = 0;
-      uint32_t head_bucket = 0;
-      const uint32_t head = slab_head(geo, tb, slot, &head_pos, &head_bucket);
-      if (head < cur) {  // a smaller index probes this slot at level 1: cur moves on
-        ++lv;
-        continue;
-      }
-      const uint32_t old = map_min(cells, log2, slot, cur, ctr, &full);
-      if (full) {
-        atomicOr(status, ZEN_STAT_RETRY);
-        break;
-      }
-      if (old < cur) {  // a smaller index got here at level 2 or 3
-        ++lv;
-        continue;
-      }
-      if (old == kNone) {
-        // first level-2/3 prober of this slot: its level-1 owner (a larger index, if any) is pushed out
-        if (head == kNone) break;
-        atomicOr(reinterpret_cast<uint32_t *>(&tb.slab_idx[head_pos]), kRemovedBit);
-        atomicAdd(&tb.removed_n[head_bucket], 1u);
-        const uint32_t at = losers + atomicAdd(&ctr->displaced, 1u);
-        if (at < tb.log_cap) {
-          tb.log_t[at] = head;
-          tb.log_v[at] = (uint32_t)slab_val[head_pos];
-        } else {
-          atomicOr(status, ZEN_STAT_RETRY);
-        }
-        cur = head;
-        lv = 1;
-        continue;
-      }
-      if (old == cur) break;
-      // took the slot from a larger index that held it at its first level mapping here
-      int lw = 1;
-      while (lw < g.levels && probe_slot(g, old, lw, &part) != slot) ++lw;
-      cur = old;
-      lv = lw + 1;
+// Enters t as a prober of `slot` in bucket b's part of the map; returns the smallest earlier prober (kNone: there was
+// none).  *full is set if the part has no room.
+__device__ inline uint32_t part_min(unsigned long long *cells, const SlabTables &tb, uint32_t b, uint32_t slot, uint32_t t,
+                                    bool *full) {
+  unsigned long long *part = cells + ((size_t)b << kSlabPartLog2);
+  constexpr uint32_t mask = (1u << kSlabPartLog2) - 1u;
+  const unsigned long long mine = ((unsigned long long)(slot + 1u) << 32) | t;
+  uint32_t h = cell_home(slot, kSlabPartLog2);
+  for (uint32_t probes = 0; probes <= mask; ++probes, h = (h + 1u) & mask) {
+    const unsigned long long cur = atomicCAS(&part[h], 0ull, mine);
+    if (cur == 0ull) {
+      atomicAdd(&tb.movein_n[b * kMoveinPad], 1u);
+      return kNone;
     }
+    if ((uint32_t)(cur >> 32) == slot + 1u) return (uint32_t)atomicMin(&part[h], mine);
   }
+  *full = true;
+  return 0u;  // pretend a smaller index owns it: the chain moves on and the call is retried anyway
 }
 
 // Where every bucket starts in the output: survivors + moved-in entries, the partition's serial entries
 // behind its last bucket.  Run by one workgroup of kSlabBlock threads once all counts are final: it is the last
-// to need the counters the chains and the classification raised with atomics, hands what k_slab_place still
-// wants of them on in final_n and puts them back to zero.
+// to need the counters the chains raised with atomics, hands what k_slab_place still wants of them on in final_n
+// and puts them back to zero.
 __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables &tb, uint32_t *s_scan) {
   constexpr int kPer = kSlabMaxBuckets / kSlabBlock;
   const uint32_t B = geo.nbuckets;
-  uint32_t c[kPer];
+  uint32_t c[kPer], mv[kPer], rm[kPer];
   uint32_t sum = 0;
+#pragma unroll
+  for (int e = 0; e < kPer; ++e) {  // no branch around the loads: all in flight together
+    const uint32_t x = threadIdx.x * kPer + e, at = x < B ? x : 0u;
+    mv[e] = load_fresh(&tb.movein_n[at * kMoveinPad]);
+    rm[e] = load_fresh(&tb.removed_n[at]);
+    c[e] = tb.bucket_n[at];
+  }
 #pragma unroll
   for (int e = 0; e < kPer; ++e) {
     const uint32_t x = threadIdx.x * kPer + e;
-    c[e] = 0;
+    c[e] = x < B ? c[e] - rm[e] + mv[e] : 0u;
     if (x < B) {
-      const uint32_t mv_raw = load_fresh(&tb.movein_n[x]);
-      const uint32_t mv = mv_raw > (uint32_t)kSlabMoveCap ? (uint32_t)kSlabMoveCap : mv_raw;
-      tb.final_n[x] = mv_raw;
-      tb.movein_n[x] = 0;
-      c[e] = tb.bucket_n[x] - load_fresh(&tb.removed_n[x]) + mv;
+      tb.final_n[x] = mv[e];
       if (x % geo.bpp == geo.bpp - 1) {
-        const uint32_t sn_raw = load_fresh(&tb.serial_n[x / geo.bpp]);
+        const uint32_t sn_raw = load_fresh(&tb.serial_n[x / geo.bpp * kMoveinPad]);
         tb.final_n[B + x / geo.bpp] = sn_raw;
-        tb.serial_n[x / geo.bpp] = 0;
         c[e] += sn_raw > (uint32_t)kSlabSerialCap ? (uint32_t)kSlabSerialCap : sn_raw;
       }
     }
@@ -369,226 +333,239 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
     running += c[e];
   }
   if (B == (uint32_t)kSlabMaxBuckets && threadIdx.x == kSlabBlock - 1) tb.out_start[B] = running;
+  for (uint32_t x = threadIdx.x; x < B; x += kSlabBlock) tb.movein_n[x * kMoveinPad] = 0;
+  for (uint32_t x = threadIdx.x; x < (uint32_t)tb.partitions; x += kSlabBlock) tb.serial_n[x * kMoveinPad] = 0;
   if (threadIdx.x == 0) {
-    const uint32_t P = (uint32_t)tb.partitions;
-    tb.final_n[B + P] = load_fresh(&tb.ctr->losers);
-    tb.final_n[B + P + 1] = load_fresh(&tb.ctr->displaced);
-    tb.ctr->logged = tb.ctr->losers = tb.ctr->claims = tb.ctr->displaced = 0;
+    *tb.losers = 0;
     *tb.done = 0;
   }
 }
 
-// Final place of every logged entry: the level-2/3 slot it holds in the map, or its partition's serial list.
-// The workgroup that finishes last then knows every count and lays out the output.
-__global__ __launch_bounds__(kSlabBlock) void k_slab_classify(SlabGeom geo, Probe g, SlabTables tb,
-                                                              const unsigned long long *__restrict__ cells,
-                                                              uint32_t log2, int64_t spp, int32_t *status) {
+// Levels 2 and 3 for the indices that lost level 1, one per thread.  Bound by latency: a probe is four or five
+// dependent trips to memory (the bucket's index, its records, the map), so that every loser has a thread of its own
+// on a full chip; nothing is counted in one place (62 M slots, 10 % taken, 300 000 losers: with one counter of the
+// map's claims and one log of the owners pushed out, whose entries another kernel classified afterwards, 338 + 220 us).
+__global__ __launch_bounds__(kSlabBlock) void k_slab_chains(SlabGeom geo, Probe g, SlabTables tb, unsigned long long *cells,
+                                                            int64_t spp, int32_t *status) {
   __shared__ uint32_t s_scan[kSlabBlock / 64 + 1];
   __shared__ bool s_last;
-  const Counters *ctr = tb.ctr;
-  uint32_t losers = ctr->losers;
+  uint32_t losers = load_fresh(tb.losers);
   if (losers > tb.log_cap) losers = tb.log_cap;
-  uint32_t total = losers + ctr->displaced;
-  if (total > tb.log_cap) total = tb.log_cap;
-  for (uint32_t i = blockIdx.x * kSlabBlock + threadIdx.x; i < total; i += gridDim.x * kSlabBlock) {
-    const uint32_t t = tb.log_t[i];
-    uint32_t part = 0, cell = kNone, slot = kNone;
-    for (int lv = 1; lv < g.levels && slot == kNone; ++lv) {
-      const uint32_t s = probe_slot(g, t, lv, &part);
-      uint32_t at = 0;
-      if (map_find(cells, log2, s, &at) == t) {
-        slot = s;
-        cell = at;
+  // workgroups without a loser are not waited for (one that starts after the last of the others has put the count
+  // back to zero sees none either)
+  uint32_t working = (losers + kSlabBlock - 1u) / kSlabBlock;
+  working = working < 1u ? 1u : working > gridDim.x ? gridDim.x : working;
+  if (blockIdx.x >= working) return;
+  for (uint32_t i = blockIdx.x * (uint32_t)kSlabBlock + threadIdx.x; i < losers; i += gridDim.x * (uint32_t)kSlabBlock) {
+    uint32_t cur = tb.log_t[i];
+    int lv = 1;
+    bool full = false;
+    for (uint32_t steps = 0;; ++steps) {
+      if (lv >= g.levels) {  // out of levels: cur has no slot
+        const uint32_t part = level1_slot(g, cur) / g.npp;
+        const uint32_t at = atomicAdd(&tb.serial_n[part * kMoveinPad], 1u);
+        if (at < (uint32_t)kSlabSerialCap)
+          tb.ser_idx[(size_t)part * kSlabSerialCap + at] = cur;
+        else  // more than the partition's serial region holds is an overflow; more than this path carries, a retry
+          atomicOr(status, (int64_t)at >= spp ? ZEN_STAT_SERIAL_OVERFLOW : ZEN_STAT_RETRY);
+        break;
       }
-    }
-    tb.log_cell[i] = cell;
-    if (slot != kNone) {
-      const uint32_t b = geo.bucket_of(slot);
-      const uint32_t at = atomicAdd(&tb.movein_n[b], 1u);
-      if (at < (uint32_t)kSlabMoveCap) {
-        const size_t dst = (size_t)b * kSlabMoveCap + at;
-        tb.mv_key[dst] = slot;
-        tb.mv_idx[dst] = t;
-        tb.mv_val[dst] = tb.log_v[i];
-      } else {
+      if (steps > kChainLimit) {
+        atomicOr(status, ZEN_STAT_INTERNAL);
+        break;
+      }
+      uint32_t part;
+      const uint32_t slot = probe_slot(g, cur, lv, &part);
+      size_t head_pos = 0;
+      uint32_t bucket = 0;
+      const uint32_t head = slab_head(geo, tb, slot, &head_pos, &bucket);
+      if (head < cur) {  // a smaller index probes this slot at level 1: cur moves on
+        ++lv;
+        continue;
+      }
+      const uint32_t old = part_min(cells, tb, bucket, slot, cur, &full);
+      if (full) {
         atomicOr(status, ZEN_STAT_RETRY);
+        break;
       }
-    } else {
-      part = level1_slot(g, t) / g.npp;
-      const uint32_t at = atomicAdd(&tb.serial_n[part], 1u);
-      if (at < (uint32_t)kSlabSerialCap)
-        tb.ser_idx[(size_t)part * kSlabSerialCap + at] = t;
-      else  // more than the partition's serial region holds is an overflow; more than this path carries, a retry
-        atomicOr(status, (int64_t)at >= spp ? ZEN_STAT_SERIAL_OVERFLOW : ZEN_STAT_RETRY);
+      if (old < cur) {  // a smaller index got here at level 2 or 3
+        ++lv;
+        continue;
+      }
+      if (old == kNone) {
+        // first level-2/3 prober of this slot: its level-1 owner (a larger index, if any) is pushed out
+        if (head == kNone) break;
+        atomicOr(reinterpret_cast<uint32_t *>(&tb.slab_idx[head_pos]), kRemovedBit);
+        atomicAdd(&tb.removed_n[bucket], 1u);
+        cur = head;
+        lv = 1;
+        continue;
+      }
+      if (old == cur) break;
+      // took the slot from a larger index that held it at its first level mapping here
+      int lw = 1;
+      while (lw < g.levels && probe_slot(g, old, lw, &part) != slot) ++lw;
+      cur = old;
+      lv = lw + 1;
     }
   }
-  // the counters above were raised with atomics that returned (movein_n, serial_n): they have been carried out
+  // the workgroup that finishes last knows every count and lays out the output
+  wait_global_acks();
   __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(tb.done, 1u) == gridDim.x - 1u;
+  if (threadIdx.x == 0) s_last = atomicAdd(tb.done, 1u) == working - 1u;
   __syncthreads();
   if (s_last) slab_output_starts(geo, tb, s_scan);
 }
 
 // ------------------------------------------------------------------ place
 
-constexpr int kPlaceRemoved = 1024;  // removed entries per bucket the place kernel keeps track of
-
-// Ranks the n (distinct) words of `a` in LDS: on return a is ascending.  Called by the whole workgroup; n is
-// small in practice (a handful), at most kSlabMoveCap.
-__device__ inline void sort_small(uint32_t *a, uint32_t n) {
-  constexpr int kPer = kSlabMoveCap / kSlabBlock;
-  uint32_t x[kPer], r[kPer];
-#pragma unroll
-  for (int e = 0; e < kPer; ++e) {
-    const uint32_t j = threadIdx.x + e * kSlabBlock;
-    x[e] = j < n ? a[j] : 0u;
-    r[e] = 0;
-    if (j < n)
-      for (uint32_t u = 0; u < n; ++u) r[e] += a[u] < x[e];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int e = 0; e < kPer; ++e)
-    if (threadIdx.x + e * kSlabBlock < n) a[r[e]] = x[e];
-  __syncthreads();
-}
-
 // The sorted slab of a bucket is almost its part of the output already: the entries that lost their slot
-// (a handful) drop out and the entries that moved in from elsewhere (another handful) slip in between.  So
-// an entry at sorted place p goes to
-//     bucket start + p - (removed entries before p) + (moved-in entries whose slot is smaller),
-// both counts being searches in two short sorted lists; consecutive lanes read consecutive entries and write
-// (almost) consecutive places, and nothing but the bucket's slots passes through LDS.
+// drop out and the entries that moved in from elsewhere slip in between.  So an entry at sorted place p goes to
+//     bucket start + p - (removed entries before p) + (moved-in entries in front of it).
+// A wave's 64 consecutive places are one stretch: how many of its entries in front of a lane's are removed is a
+// ballot, how many moved-in ones slip in there a prefix sum across the lanes, and the stretches' sums are chained
+// once per bucket.  Consecutive lanes read consecutive entries and write (almost) consecutive places.  (Both counts
+// as bisections of sorted lists: 100 us for 6.2 M entries of which 5 % had moved.)
 template <typename S>
 __global__ __launch_bounds__(kSlabBlock) void k_slab_place(SlabGeom geo, SlabTables tb, unsigned long long *cells,
-                                                           int partitions, int64_t spp,
-                                                           const S *__restrict__ dense, int32_t *__restrict__ out_idx,
-                                                           S *__restrict__ out_val, uint32_t capacity,
-                                                           int64_t *__restrict__ splits, int32_t *status) {
+                                                           int64_t spp, const S *__restrict__ dense,
+                                                           int32_t *__restrict__ out_idx, S *__restrict__ out_val,
+                                                           uint32_t capacity, int64_t *__restrict__ splits,
+                                                           int32_t *status) {
+  constexpr int kStretches = kSlabCap / 64;
+  constexpr int kCells = (1 << kSlabPartLog2) / kSlabBlock;
+  static_assert(kStretches <= 128, "two stretches per lane of a wave");
   __shared__ uint32_t s_key[kSlabCap];                 // sorted slots of the bucket
-  __shared__ uint32_t s_mk[kSlabMoveCap];              // slots of the moved-in entries, ascending
-  __shared__ uint32_t s_mp[kSlabMoveCap];              // sorted place in front of which each of them slips in
-  __shared__ uint32_t s_rm[kPlaceRemoved];             // sorted places of the removed entries, ascending
-  __shared__ int32_t s_delta[kSlabCap / 64];           // per 64 sorted places: how far their entries move
+  __shared__ uint32_t s_cnt[kSlabCap / 2 + 1];         // per sorted place, 16 bits each: the moved-in entries right in
+  uint16_t *s_front = reinterpret_cast<uint16_t *>(s_cnt);  // front of it, then those before it in its stretch
+  __shared__ uint32_t s_mk[1 << kSlabPartLog2];        // the moved-in entries' slots, by the place they slip in at
+  __shared__ uint64_t s_mask[kStretches];              // per stretch: its removed entries
+  __shared__ uint32_t s_mv[kStretches], s_rm[kStretches];  // moved-in and removed entries of the stretches before
   __shared__ uint32_t s_nrm;
-  constexpr int32_t kNoDelta = INT32_MIN;              // the stretch has no common amount
   const uint32_t b = blockIdx.x;
   const uint32_t B = geo.nbuckets;
   const size_t base = (size_t)b * kSlabCap;
   const S *slab_val = static_cast<const S *>(tb.slab_val);
-  if (threadIdx.x == 0) s_nrm = 0;
-
-  // every occupied map cell ends with the index that finally holds its slot, and that index recorded the
-  // cell: clearing by cell number leaves the borrowed memory zero again
   const uint32_t *serial_n = tb.final_n + B;
-  {
-    uint32_t losers = tb.final_n[B + tb.partitions];
-    if (losers > tb.log_cap) losers = tb.log_cap;
-    uint32_t total = losers + tb.final_n[B + tb.partitions + 1];
-    if (total > tb.log_cap) total = tb.log_cap;
-    for (uint32_t i = b * kSlabBlock + threadIdx.x; i < total; i += B * kSlabBlock) {
-      const uint32_t cell = tb.log_cell[i];
-      if (cell != kNone) cells[cell] = 0ull;
-    }
-  }
-
   const uint32_t n = tb.bucket_n[b];
-  uint32_t mv_n = tb.final_n[b];
-  if (mv_n > (uint32_t)kSlabMoveCap) mv_n = kSlabMoveCap;
+  // what the bucket's part of the map holds has moved in, and keeps to the thread that finds it; the part goes
+  // back empty
+  const uint32_t mv_n = tb.final_n[b];
+  unsigned long long *cell = cells + ((size_t)b << kSlabPartLog2) + threadIdx.x;
+  unsigned long long moved[kCells];
+#pragma unroll
+  for (int e = 0; e < kCells; ++e) moved[e] = mv_n ? cell[e * kSlabBlock] : 0ull;
   // the thread's entries (sorted places threadIdx.x + i * kSlabBlock) stay in registers; the slots go to LDS
-  // for the searches, the places of removed entries are collected
+  // for the searches
   uint32_t idx[kSlabItems];
   S val[kSlabItems];
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
     const uint32_t p = threadIdx.x + i * kSlabBlock;
-    idx[i] = kRemovedBit;
-    val[i] = 0;
-    if (p < n) {
-      idx[i] = (uint32_t)tb.slab_idx[base + p];
-      s_key[p] = geo.mod_m(poly(idx[i] & kIndexMask) + kSeed1);
-      val[i] = slab_val[base + p];
-    }
+    idx[i] = (uint32_t)tb.slab_idx[base + (p < n ? p : 0u)];
+    val[i] = slab_val[base + (p < n ? p : 0u)];
   }
-  for (uint32_t j = threadIdx.x; j < mv_n; j += kSlabBlock) s_mk[j] = tb.mv_key[(size_t)b * kSlabMoveCap + j];
-  __syncthreads();  // s_nrm is zero, s_key and s_mk are there
+  S mval[kCells];  // an entry is a copy of the element it stands for
+#pragma unroll
+  for (int e = 0; e < kCells; ++e) mval[e] = mv_n ? dense[(uint32_t)moved[e]] : S(0);
+  if (threadIdx.x == 0) s_nrm = 0;
+  for (int i = threadIdx.x; i < kSlabCap / 2 + 1; i += kSlabBlock) s_cnt[i] = 0;
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
     const uint32_t p = threadIdx.x + i * kSlabBlock;
-    if (p < n && (idx[i] & kRemovedBit)) {
-      const uint32_t at = atomicAdd(&s_nrm, 1u);
-      if (at < (uint32_t)kPlaceRemoved) s_rm[at] = p;
+    if (p < n) s_key[p] = geo.mod_m(poly(idx[i] & kIndexMask) + kSeed1);
+  }
+  __syncthreads();
+  // a moved-in entry's place: the sorted place in front of which it slips in, and its turn among those that slip
+  // in there too
+  uint32_t mplace[kCells], mturn[kCells];
+#pragma unroll
+  for (int e = 0; e < kCells; ++e) {
+    mplace[e] = mturn[e] = 0;
+    if (moved[e]) {
+      cell[e * kSlabBlock] = 0ull;
+      mplace[e] = lower_bound_u32(s_key, n, (uint32_t)(moved[e] >> 32) - 1u);
+      const uint32_t shift = 16u * (mplace[e] & 1u);
+      mturn[e] = (atomicAdd(&s_cnt[mplace[e] >> 1], 1u << shift) >> shift) & 0xffffu;
     }
   }
   __syncthreads();
-  uint32_t rm_n = s_nrm;
-  if (rm_n > (uint32_t)kPlaceRemoved) {  // more collisions than this path carries
-    if (threadIdx.x == 0) atomicOr(status, ZEN_STAT_RETRY);
-    return;
-  }
-  if (rm_n > 1) sort_small(s_rm, rm_n);
-  // moved-in entry j: its slot's rank among the moved-in slots (they are distinct: a slot has one owner), and
-  // the sorted place in front of which it slips in
-  uint32_t mj[kSlabMoveCap / kSlabBlock], mplace[kSlabMoveCap / kSlabBlock];
+  uint32_t in_front[kSlabItems];  // moved-in entries of the stretch that slip in at or before the entry's place
+  uint32_t removed = 0;           // bit i: entry i has lost its slot
 #pragma unroll
-  for (int e = 0; e < kSlabMoveCap / kSlabBlock; ++e) {
-    const uint32_t j = threadIdx.x + e * kSlabBlock;
-    mj[e] = mplace[e] = 0;
-    if (j < mv_n) {
-      const uint32_t k = s_mk[j];
-      uint32_t r = 0;
-      for (uint32_t u = 0; u < mv_n; ++u) r += s_mk[u] < k;
-      mj[e] = r;
-      mplace[e] = lower_bound_u32(s_key, n, k);
+  for (int i = 0; i < kSlabItems; ++i) {
+    const uint32_t p = threadIdx.x + i * kSlabBlock;
+    const bool gone = p < n && (idx[i] & kRemovedBit);
+    const uint64_t m = __ballot(gone);
+    removed |= (gone ? 1u : 0u) << i;
+    in_front[i] = 0;
+    if (mv_n) {
+      const uint32_t c = s_front[p];
+      in_front[i] = wave_inclusive_scan(c);
+      s_front[p] = (uint16_t)(in_front[i] - c);
+    }
+    if (lane_id() == 63) {
+      s_mask[p >> 6] = m;
+      s_mv[p >> 6] = in_front[i];
+      s_rm[p >> 6] = (uint32_t)__popcll(m);
     }
   }
   __syncthreads();
-#pragma unroll
-  for (int e = 0; e < kSlabMoveCap / kSlabBlock; ++e)
-    if (threadIdx.x + e * kSlabBlock < mv_n) s_mp[mj[e]] = mplace[e];
+  if (threadIdx.x < 64) {
+    const int l = threadIdx.x;
+    const uint32_t v0 = s_mv[l], v1 = l + 64 < kStretches ? s_mv[l + 64] : 0u;
+    const uint32_t r0 = s_rm[l], r1 = l + 64 < kStretches ? s_rm[l + 64] : 0u;
+    const uint32_t iv0 = wave_inclusive_scan(v0), iv1 = wave_inclusive_scan(v1);
+    const uint32_t ir0 = wave_inclusive_scan(r0), ir1 = wave_inclusive_scan(r1);
+    const uint32_t tv = __shfl(iv0, 63, 64), tr = __shfl(ir0, 63, 64);
+    s_mv[l] = iv0 - v0;
+    s_rm[l] = ir0 - r0;
+    if (l + 64 < kStretches) {
+      s_mv[l + 64] = tv + iv1 - v1;
+      s_rm[l + 64] = tr + ir1 - r1;
+    }
+    if (l == 63) s_nrm = tr + ir1;
+  }
   __syncthreads();
   const uint32_t out_base = tb.out_start[b];
   const uint32_t out_n = tb.out_start[b + 1] - out_base;
-  // Most stretches of 64 consecutive sorted places contain neither a removed entry nor the place where a
-  // moved-in entry slips in: all their entries move by the same amount, found once per stretch.
-  for (uint32_t c = threadIdx.x; c * 64u < n; c += kSlabBlock) {
-    const uint32_t p0 = c * 64u, p1 = p0 + 63u < n ? p0 + 63u : n - 1u;
-    uint32_t mv0 = 0, mv1 = 0, r0 = 0, r1 = 0;
-    if (mv_n) {
-      mv0 = upper_bound_u32(s_mp, mv_n, p0);
-      mv1 = upper_bound_u32(s_mp, mv_n, p1);
-    }
-    if (rm_n) {
-      r0 = lower_bound_u32(s_rm, rm_n, p0);
-      r1 = lower_bound_u32(s_rm, rm_n, p1);
-    }
-    s_delta[c] = (mv0 == mv1 && r0 == r1) ? (int32_t)(mv0 - r0) : kNoDelta;
-  }
-  __syncthreads();
   // survivors
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
     const uint32_t p = threadIdx.x + i * kSlabBlock;
-    if (p < n && !(idx[i] & kRemovedBit)) {
-      int32_t delta = s_delta[p >> 6];
-      if (delta == kNoDelta)
-        delta = (int32_t)((mv_n ? upper_bound_u32(s_mp, mv_n, p) : 0u) - (rm_n ? lower_bound_u32(s_rm, rm_n, p) : 0u));
-      const uint32_t pos = out_base + p + (uint32_t)delta;
+    const uint64_t m = __ballot((removed >> i) & 1u);
+    if (p < n && !((removed >> i) & 1u)) {
+      const uint32_t before = (uint32_t)__popcll(m & lanes_below());
+      const uint32_t pos = out_base + p + s_mv[p >> 6] + in_front[i] - s_rm[p >> 6] - before;
       if (pos < capacity) {
         out_idx[pos] = (int32_t)idx[i];
         out_val[pos] = val[i];
       }
     }
   }
-  // moved-in entries
+  if (mv_n) {  // the same for the whole workgroup
+    // the moved-in entries by the place they slip in at; several at one place (two at times) by ascending slot
+    const auto front = [&](uint32_t p) -> uint32_t {  // moved-in entries before those of place p
+      return p < (uint32_t)kSlabCap ? s_mv[p >> 6] + s_front[p] : p > (uint32_t)kSlabCap ? mv_n : mv_n - s_front[kSlabCap];
+    };
 #pragma unroll
-  for (int e = 0; e < kSlabMoveCap / kSlabBlock; ++e) {
-    const uint32_t j = threadIdx.x + e * kSlabBlock;
-    if (j < mv_n) {
-      const uint32_t pos = out_base + mplace[e] + mj[e] - (rm_n ? lower_bound_u32(s_rm, rm_n, mplace[e]) : 0u);
-      if (pos < capacity) {
-        out_idx[pos] = (int32_t)tb.mv_idx[(size_t)b * kSlabMoveCap + j];
-        out_val[pos] = (S)tb.mv_val[(size_t)b * kSlabMoveCap + j];
+    for (int e = 0; e < kCells; ++e)
+      if (moved[e]) s_mk[front(mplace[e]) + mturn[e]] = (uint32_t)(moved[e] >> 32) - 1u;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kCells; ++e) {
+      if (moved[e]) {
+        const uint32_t at = mplace[e], key = (uint32_t)(moved[e] >> 32) - 1u;
+        const uint32_t first = front(at), end = front(at + 1u);
+        uint32_t rank = first;
+        for (uint32_t u = first; u < end; ++u) rank += s_mk[u] < key;
+        const uint32_t gone =
+            at < n ? s_rm[at >> 6] + (uint32_t)__popcll(s_mask[at >> 6] & ((1ull << (at & 63u)) - 1ull)) : s_nrm;
+        const uint32_t pos = out_base + at + rank - gone;
+        if (pos < capacity) {
+          out_idx[pos] = (int32_t)(uint32_t)moved[e];
+          out_val[pos] = mval[e];
+        }
       }
     }
   }
@@ -621,7 +598,6 @@ __global__ __launch_bounds__(kSlabBlock) void k_slab_place(SlabGeom geo, SlabTab
     if ((int64_t)serial_n[part] > spp) atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
     if (hi > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
   }
-  (void)partitions;
 }
 
 struct SlabPlan {
@@ -651,9 +627,9 @@ SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partit
     p.ticket = cv.take<uint32_t>(select_stage_ticket_words());
     p.tb.cursor = cv.take<uint32_t>(B * kCursorPad);
     p.feed.coarse_cursor = cv.take<uint32_t>(feed_coarse_cursor_words());
-    p.tb.movein_n = cv.take<uint32_t>(B);
-    p.tb.serial_n = cv.take<uint32_t>((size_t)partitions);
-    p.tb.ctr = cv.take<Counters>(1);
+    p.tb.movein_n = cv.take<uint32_t>(B * kMoveinPad);
+    p.tb.serial_n = cv.take<uint32_t>((size_t)partitions * kMoveinPad);
+    p.tb.losers = cv.take<uint32_t>(1);
     p.tb.done = cv.take<uint32_t>(1);
     p.refine_hist = cv.take<uint32_t>(dtype == ZEN_BF16 ? 1 : (size_t)kRefineBins + 1);
     p.state_bytes = cv.used;
@@ -669,7 +645,7 @@ SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partit
   p.tb.refine_hist = nullptr;
   p.tb.partitions = partitions;
   p.tb.out_start = cv.take<uint32_t>(B + 1);
-  p.tb.final_n = cv.take<uint32_t>(B + (size_t)partitions + 2);
+  p.tb.final_n = cv.take<uint32_t>(B + (size_t)partitions);
   p.tb.bucket_n = cv.take<uint32_t>(B);
   p.tb.removed_n = cv.take<uint32_t>(B);
   p.tb.raw_idx = cv.take<uint32_t>(B * kSlabCap);
@@ -677,14 +653,9 @@ SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partit
   p.tb.slab_idx = cv.take<int32_t>(B * kSlabCap);
   p.tb.slab_val = cv.take<char>(B * kSlabCap * (dtype == ZEN_BF16 ? 2 : 4));
   p.tb.sub_index = cv.take<uint16_t>(B * kSlabIndexLen);
-  p.tb.mv_key = cv.take<uint32_t>(B * kSlabMoveCap);
-  p.tb.mv_idx = cv.take<uint32_t>(B * kSlabMoveCap);
-  p.tb.mv_val = cv.take<uint32_t>(B * kSlabMoveCap);
   p.tb.ser_idx = cv.take<uint32_t>((size_t)partitions * kSlabSerialCap);
   p.tb.log_cap = (uint32_t)(list_cap / 4 + 1024);
   p.tb.log_t = cv.take<uint32_t>(p.tb.log_cap);
-  p.tb.log_v = cv.take<uint32_t>(p.tb.log_cap);
-  p.tb.log_cell = cv.take<uint32_t>(p.tb.log_cap);
   p.bytes = cv.used;
   return p;
 }
@@ -709,14 +680,15 @@ int slab_launch(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPlan &p
   }
   {
     ProfScope prof(kProfSlabChains, s);
-    k_slab_chains<S><<<dim3(256), dim3(256), 0, s>>>(geo, a.g, p.tb, a.hash, a.hash_log2, a.status);
+    // (as many workgroups as the chip holds; fewer where there can be few losers)
+    const int64_t groups = ceil_div((int64_t)p.tb.log_cap / 4, (int64_t)kSlabBlock);
+    k_slab_chains<<<dim3((unsigned)(groups < 64 ? 64 : groups > 1024 ? 1024 : groups)), dim3(kSlabBlock), 0, s>>>(
+        geo, a.g, p.tb, a.hash, a.spp, a.status);
     ZEN_LAUNCH_CHECK("k_slab_chains");
-    k_slab_classify<<<dim3(128), dim3(kSlabBlock), 0, s>>>(geo, a.g, p.tb, a.hash, a.hash_log2, a.spp, a.status);
-    ZEN_LAUNCH_CHECK("k_slab_classify");
   }
   {
     ProfScope prof(kProfSlabPlace, s);
-    k_slab_place<S><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, a.partitions, a.spp, dense, a.out_idx,
+    k_slab_place<S><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, a.spp, dense, a.out_idx,
                                                          static_cast<S *>(a.out_val), (uint32_t)a.capacity, a.splits,
                                                          a.status);
     ZEN_LAUNCH_CHECK("k_slab_place");
@@ -733,7 +705,7 @@ size_t slab_balance_bytes(int64_t m, int partitions, int dtype, int64_t capacity
 }
 
 // The hash map takes the first 8 << hash_log2 bytes of the caller's table (at most half of it: zen_load_balance
-// sizes the map so); the counters sit behind it.
+// sizes the map so), of which every bucket has a part; the counters sit behind it.
 size_t slab_state_offset(uint32_t hash_log2) { return align_up((size_t)8 << hash_log2, 256); }
 
 bool slab_balance_fits(int64_t n, int64_t m, int partitions, int dtype, int64_t capacity, int64_t k, SlabGeom *geo) {
@@ -778,6 +750,9 @@ int slab_load_balance(const SlabBalanceArgs &a, hipStream_t s) {
   SlabPlan p = plan_slab(a.workspace, state, geo, a.partitions, a.dtype, list_capacity(a.capacity));
   if (slab_state_offset(a.hash_log2) + p.state_bytes > (size_t)a.g.m * sizeof(int32_t))
     return fail(ZEN_EINVAL, "slab_load_balance: table too small for the counters");
+  // never with the geometries slab_geometry gives: a bucket spans 16384 slots or more, and there is a cell for about
+  // eight slots up to 2^24 cells
+  if (((uint64_t)geo.nbuckets << kSlabPartLog2) > (1ull << a.hash_log2)) return fail(ZEN_EINVAL, "slab_load_balance: table too small for the map");
   const bool refine = a.k > 0 && a.dtype == ZEN_F32;
   if (refine) p.tb.refine_hist = p.refine_hist;
   StageArgs sc;

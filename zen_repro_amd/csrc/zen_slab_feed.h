@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kSlabBlock) void k_fine_scatter(SlabGeom geo, Coars
   const uint32_t first_bucket = c * cg.per;
   if (blockIdx.x == 0 && blockIdx.y % kCoarseSplit == 0 && threadIdx.x < cg.per &&
       first_bucket + threadIdx.x < geo.nbuckets)
-    bucket_lo[first_bucket + threadIdx.x] = geo.first_key(first_bucket + threadIdx.x);  // a 64-bit division: once per bucket
+    bucket_lo[first_bucket + threadIdx.x] = geo.first_key(first_bucket + threadIdx.x);
   uint32_t count = coarse_cursor[blockIdx.y * kCoarsePad];
   if (count > cg.cap) count = cg.cap;  // the first step flagged the overflow
   const uint32_t batch = blockIdx.x * (uint32_t)kFeedBatch;

@@ -56,6 +56,7 @@ inline bool wide_geometry(int64_t m, int partitions, int64_t expected, int cus, 
   const uint64_t width = ((1ull << 32) + g.bpp_mult - 1) / g.bpp_mult + 1;  // keys per bucket, at most
   g.sub_shift = 0;
   while ((width >> g.sub_shift) >= (uint64_t)kWideSubs) ++g.sub_shift;
+  g.width = slab_bucket_width(g.bpp_mult);
   g.inv_m = slab_inverse_below(g.m);
   g.inv_npp = slab_inverse_below(g.npp);
   *out = g;
