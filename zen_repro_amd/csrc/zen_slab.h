@@ -299,6 +299,7 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
   constexpr int kBatch = kItems % 3 == 0 ? 3 : kItems;
 #pragma unroll
   for (int h = 0; h < kItems; h += kBatch) {
+    if (live >> h == 0) continue;
     uint32_t a[kBatch][kRankAhead];
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {

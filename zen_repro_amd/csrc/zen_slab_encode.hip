@@ -254,12 +254,14 @@ __device__ inline uint32_t slab_head(const SlabGeom &geo, const SlabTables &tb, 
   const int32_t *idx = tb.slab_idx + (size_t)b * kSlabCap;
   const uint32_t j = (off >> geo.sub_shift) / (uint32_t)kSlabIndexStep;
   const uint16_t *index = tb.sub_index + (size_t)b * kSlabIndexLen;
-  uint32_t p = index[j];
-  const uint32_t end = index[j + 1];
-  for (; p < end; p += 4) {
-    uint32_t t[4];
+  uint16_t range[2];  // one load each time: a wave's lanes all read other lines
+  __builtin_memcpy(range, index + j, sizeof(range));
+  const uint32_t end = range[1];
+  for (uint32_t p = range[0]; p < end; p += 4) {
+    uint32_t t[4];  // (up to three words past the range are read and not looked at: the workspace goes on behind)
+    __builtin_memcpy(t, idx + p, sizeof(t));
 #pragma unroll
-    for (int q = 0; q < 4; ++q) t[q] = (uint32_t)idx[p + q < end ? p + q : p] & kIndexMask;
+    for (int q = 0; q < 4; ++q) t[q] &= kIndexMask;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       if (p + q >= end) return kNone;
@@ -427,7 +429,7 @@ __global__ __launch_bounds__(kSlabBlock) void k_slab_chains(SlabGeom geo, Probe 
 // once per bucket.  Consecutive lanes read consecutive entries and write (almost) consecutive places.  (Both counts
 // as bisections of sorted lists: 100 us for 6.2 M entries of which 5 % had moved.)
 template <typename S>
-__global__ __launch_bounds__(kSlabBlock) void k_slab_place(SlabGeom geo, SlabTables tb, unsigned long long *cells,
+__global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, SlabTables tb, unsigned long long *cells,
                                                            int64_t spp, const S *__restrict__ dense,
                                                            int32_t *__restrict__ out_idx, S *__restrict__ out_val,
                                                            uint32_t capacity, int64_t *__restrict__ splits,
@@ -451,6 +453,8 @@ __global__ __launch_bounds__(kSlabBlock) void k_slab_place(SlabGeom geo, SlabTab
   // what the bucket's part of the map holds has moved in, and keeps to the thread that finds it; the part goes
   // back empty
   const uint32_t mv_n = tb.final_n[b];
+  const uint32_t out_base = tb.out_start[b];
+  const uint32_t out_n = tb.out_start[b + 1] - out_base;
   unsigned long long *cell = cells + ((size_t)b << kSlabPartLog2) + threadIdx.x;
   unsigned long long moved[kCells];
 #pragma unroll
@@ -495,10 +499,14 @@ __global__ __launch_bounds__(kSlabBlock) void k_slab_place(SlabGeom geo, SlabTab
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
     const uint32_t p = threadIdx.x + i * kSlabBlock;
+    in_front[i] = 0;
+    if ((uint32_t)(i * kSlabBlock) > n) {  // the same for the whole workgroup: nothing beyond the entries
+      if (lane_id() == 63) s_mv[p >> 6] = s_rm[p >> 6] = 0;
+      continue;
+    }
     const bool gone = p < n && (idx[i] & kRemovedBit);
     const uint64_t m = __ballot(gone);
     removed |= (gone ? 1u : 0u) << i;
-    in_front[i] = 0;
     if (mv_n) {
       const uint32_t c = s_front[p];
       in_front[i] = wave_inclusive_scan(c);
@@ -527,12 +535,11 @@ __global__ __launch_bounds__(kSlabBlock) void k_slab_place(SlabGeom geo, SlabTab
     if (l == 63) s_nrm = tr + ir1;
   }
   __syncthreads();
-  const uint32_t out_base = tb.out_start[b];
-  const uint32_t out_n = tb.out_start[b + 1] - out_base;
   // survivors
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
     const uint32_t p = threadIdx.x + i * kSlabBlock;
+    if ((uint32_t)(i * kSlabBlock) >= n) break;
     const uint64_t m = __ballot((removed >> i) & 1u);
     if (p < n && !((removed >> i) & 1u)) {
       const uint32_t before = (uint32_t)__popcll(m & lanes_below());
