@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define ZEN_ABI_VERSION 4 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table; 4: zen_read_back, zen_count, zen_merge_rounded, zen_decode_dense_lists, zen_bitmap_dense_lists */
+#define ZEN_ABI_VERSION 5 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table; 4: zen_read_back, zen_count, zen_merge_rounded, zen_decode_dense_lists, zen_bitmap_dense_lists; 5: zen_table_find, zen_table_gather */
 
 #define ZEN_F32 0
 #define ZEN_BF16 1
@@ -518,6 +518,21 @@ int zen_read_back(const void *p0, int n0, int wide0, const void *p1, int n1, int
  * making the lists).
  */
 int zen_count(const void *input, int dtype, int64_t n, const uint32_t *thr, int64_t *count, void *stream);
+
+/*
+ * The lists of a filled table (tensor_load_balance.py:24-40) in two steps.  zen_table_find looks through the
+ * partitions * (m / partitions) leading slots of `table` and writes the number of nonzero entries of every
+ * partition to splits[partitions] (device); an entry that is no index of a tensor of n elements (negative ones
+ * count from its end) raises ZEN_STAT_BAD_INDEX.  zen_table_gather, with the same workspace and the splits' sum as
+ * `total`, writes the entries in slot order, partition-major, to out_idx[total] and the elements of `input` they
+ * point at to out_val[total].
+ */
+size_t zen_table_lists_workspace(int64_t m, int partitions);
+int zen_table_find(const int32_t *table, int64_t m, int partitions, int64_t n, int64_t *splits, void *workspace,
+                   size_t workspace_bytes, int32_t *status, void *stream);
+int zen_table_gather(const int32_t *table, int64_t m, int partitions, const void *input, int dtype, int64_t n,
+                     int32_t *out_idx, void *out_val, int64_t total, void *workspace, size_t workspace_bytes,
+                     void *stream);
 
 /*
  * Reads `bytes` bytes (16-byte aligned) with coalesced non-temporal 16-byte

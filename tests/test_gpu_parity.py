@@ -232,6 +232,50 @@ def test_reference_style_compaction_over_tables(zen, oracle):
     assert np.array_equal(to_np(s1 + s2), splits_o)
 
 
+@pytest.mark.parametrize("m, parts, shift, density", [
+    (1, 1, 0, 1.0), (7, 3, 1, 0.6), (1023, 1, 3, 0.2), (1025, 2, 2, 0.2), (4099, 4, 1, 0.0), (70001, 70000, 0, 0.5),
+    (100003, 16, 3, 1.0), (9000, 9000, 0, 0.3), ((1 << 23) + 5, 3, 1, 0.05)])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_table_lists(zen, oracle, m, parts, shift, density, dtype):
+    # partition edges off every vector boundary, stretches of one partition and many, full and empty tables, entries
+    # that count from the end, slots behind the last whole partition
+    n = 50000
+    rng = np.random.default_rng(m + parts)
+    table = rng.integers(-n, n, m, dtype=np.int32)
+    table[rng.random(m) >= density] = 0
+    g = make_grad(oracle, n, 1.0, dtype, seed=m)
+    room = torch.zeros(m + shift, dtype=torch.int32, device="cuda")
+    room[shift:] = to_dev(table)
+    d = to_dev(g)
+    tp = zen.TensorPartition(parts, 1, 3)
+    assert tp._plain_table(d, room[shift:])
+    idx, val, splits = tp.get_sub_sparse_tensors(d, room[shift:])
+    cut = table[:m // parts * parts].reshape(parts, -1)
+    sizes = (cut != 0).sum(1)
+    want = cut[cut != 0]
+    assert len(idx) == len(val) == parts and np.array_equal(to_np(splits), sizes)
+    assert [t.numel() for t in idx] == sizes.tolist() == [t.numel() for t in val]
+    assert np.array_equal(to_np(torch.cat(idx)), want) and np.array_equal(to_np(torch.cat(val)), g[want])
+
+
+def test_table_lists_what_torch_indexes(zen):
+    # an entry past the tensor is an error; autograd, other types and strided tensors are indexed by torch
+    g = torch.arange(100, dtype=torch.float32, device="cuda") + 1
+    mem = torch.tensor([0, 3, 0, -1, 99, 0], dtype=torch.int32, device="cuda")
+    tp = zen.TensorPartition(2, 1, 3)
+    with pytest.raises(IndexError):
+        tp.get_sub_sparse_tensors(g[:99], mem)
+    wide = g.repeat_interleave(2)[::2]
+    leaf = g.clone().requires_grad_()
+    for t in (wide, g.half(), leaf):
+        assert not tp._plain_table(t, mem)
+        idx, val, splits = tp.get_sub_sparse_tensors(t, mem)
+        assert torch.cat(idx).tolist() == [3, -1, 99] and torch.cat(val).tolist() == [4, 100, 100]
+        assert splits.tolist() == [1, 2]
+    torch.cat(val).sum().backward()
+    assert leaf.grad[99].item() == 2 and leaf.grad[3].item() == 1
+
+
 # ---------------------------------------------------------------- select
 
 

@@ -23,7 +23,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("ZEN_HIP_LIB") or os.path.join(_HERE, "csrc", "libzen_hip.so")
 
 # ZEN_ABI_VERSION of include/zen_hip.h this loader's signatures and structs are written for
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 _lib = None
 
@@ -120,6 +120,9 @@ def lib():
         "zen_host_words_free": (i32, [vp]),
         "zen_read_back": (i32, [vp, i32, i32, vp, i32, i32, vp, i32, i32, vp, i64, vp]),
         "zen_count": (i32, [vp, i32, i64, vp, vp, vp]),
+        "zen_table_lists_workspace": (sz, [i64, i32]),
+        "zen_table_find": (i32, [vp, i64, i32, i64, vp, vp, sz, vp, vp]),
+        "zen_table_gather": (i32, [vp, i64, i32, vp, i32, i64, vp, vp, i64, vp, sz, vp]),
         "zen_stream_read": (i32, [vp, sz, vp, vp]),
         "zen_profile_enable": (i32, [i32]),
         "zen_profile_only": (i32, [i32]),
@@ -192,6 +195,17 @@ def require_gpu(t, name):
         return
     assert t.is_cuda, f"{name} must be a GPU tensor"
     raise RuntimeError(f"{name} must be contiguous")
+
+
+def untransformed(*tensors):
+    """Whether nothing watches or rewrites torch's operations on these: no forward-mode level, vmap or other
+    transform, no torch mode, no subclass.  A kernel call in their place would go unnoticed."""
+    return (torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch._C._len_torch_function_stack() and not torch._C._len_torch_dispatch_stack()
+            and all(type(t) in _PLAIN for t in tensors))
+
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 class Scratch:

@@ -68,6 +68,8 @@ class TensorPartition:
         """Per-partition nonzero entries of a table and the values they point
         at (tensor_load_balance.py:24-40), as one compaction over the table."""
         flat = tensor.reshape(-1)
+        if self._plain_table(flat, memory):
+            return self._table_lists(flat, memory)
         found = self._nonzero_int32(memory)
         per_part = memory.numel() // self.partitions if self.partitions else 0
         if per_part == 0:
@@ -81,6 +83,37 @@ class TensorPartition:
         indices = [idx[cuts[p]:cuts[p + 1]] for p in range(self.partitions)]
         values = [flat[i.long()] for i in indices]
         return indices, values, splits
+
+    def _plain_table(self, flat, memory):
+        """Whether zen_table_find / zen_table_gather take these: gradients and tables as balance_sparse_tensor
+        has them.  What torch has to see (other types, autograd, transforms) is indexed by torch."""
+        return (flat.dtype in (torch.bfloat16, torch.float32) and memory.dtype == torch.int32
+                and flat.is_cuda and memory.device == flat.device and flat.is_contiguous() and memory.is_contiguous()
+                and 0 < self.partitions <= memory.numel() < 1 << 31 and flat.numel() < 1 << 31
+                and not (flat.requires_grad and torch.is_grad_enabled())
+                and _lib.untransformed(flat, memory))
+
+    def _table_lists(self, flat, memory):
+        L = _lib.lib()
+        dev = flat.device
+        m, n = memory.numel(), flat.numel()
+        splits = _lib.zeros.take(dev, self.partitions, torch.int64)
+        status = _lib.status_word(dev)
+        # not from the scratch cache: this thread may walk another table before these lists are used up
+        ws = torch.empty(L.zen_table_lists_workspace(m, self.partitions), dtype=torch.uint8, device=dev)
+        _lib.check(L.zen_table_find(_lib.ptr(memory), m, self.partitions, n, _lib.ptr(splits), _lib.ptr(ws),
+                                    ws.numel(), _lib.ptr(status), _lib.stream_of(dev)), "table_find")
+        host = _lib.read_back(splits, status)
+        if host[-1]:
+            raise IndexError("get_sub_sparse_tensors: " + _lib.describe_status(host[-1]))
+        sizes = host[:-1]
+        total = sum(sizes)
+        idx = torch.empty(total, dtype=torch.int32, device=dev)
+        val = torch.empty(total, dtype=flat.dtype, device=dev)
+        _lib.check(L.zen_table_gather(_lib.ptr(memory), m, self.partitions, _lib.ptr(flat), _lib.dtype_code(flat), n,
+                                      _lib.ptr(idx), _lib.ptr(val), total, _lib.ptr(ws), ws.numel(),
+                                      _lib.stream_of(dev)), "table_gather")
+        return list(torch.split(idx, sizes)), list(torch.split(val, sizes)), splits
 
     @staticmethod
     def _nonzero_int32(table):
