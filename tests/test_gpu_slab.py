@@ -735,3 +735,33 @@ def test_sample_taken_along_by_the_call_before(zen, oracle, dtype):
     small = ds[0][: 1 << 12]
     e, _ = lba.encode_merge_flat(tp, ds[0], caps[0], ks[0], di, dv, n, next_tensor=small, next_k=20, next_capacity=64)
     assert e[3].item() == 0 and not tp._ahead_state(ds[0].device, 0)["pending"]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_workgroups_that_take_the_next_sample_leave_their_first_tiles_to_the_others(zen, dtype):
+    """Sizes at which a workgroup has no tile of its own, one, two (as many as it leaves out), three and more, odd
+    lengths and unaligned tensors among them: the calls that take their successor's sample along return what calls
+    without one return."""
+    P = 16
+    per = {torch.bfloat16: 2, torch.float32: 1}[dtype]
+    tensors = []
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    for i, n in enumerate([(1 << 22) + 13, 7500003, 14500001, 14500000, 22000007, 30000011, 5000000]):
+        flat = torch.randn(n * per + i % 3, generator=gen, device="cuda").to(dtype)
+        tensors.append(flat[i % 3:])
+    idx = torch.arange(1, 5001, dtype=torch.int32, device="cuda")
+    val = torch.ones(5000, dtype=dtype, device="cuda")
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P), None, None)
+    tp, plain = zen.TensorPartition(P, 1, 3), zen.TensorPartition(P, 1, 3)
+    ks = [t.numel() // 200 for t in tensors]
+    caps = [k + k // 4 + 4096 for k in ks]
+    for i, t in enumerate(tensors):
+        more = {}
+        if i + 1 < len(tensors):
+            more = {"next_tensor": tensors[i + 1], "next_k": ks[i + 1], "next_capacity": caps[i + 1]}
+        e, _ = lba.encode_merge_flat(tp, t, caps[i], ks[i], idx, val, t.numel(), **more)
+        want = plain.load_balance_flat(t, capacity=caps[i], k=ks[i])
+        total = int(want[2].sum())
+        assert e[3].item() == 0 == want[3].item() and total >= ks[i]
+        for got, ref in ((e[0][:total], want[0][:total]), (e[1][:total], want[1][:total]), (e[2], want[2])):
+            assert torch.equal(got, ref)

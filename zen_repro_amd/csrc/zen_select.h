@@ -105,6 +105,7 @@ struct StageSample {
   uint32_t rank = 0;
   int block_log2 = 0;
   int64_t nblocks = 0;
+  uint32_t wgs = 0;  // workgroups that take it
   uint32_t *floor_out = nullptr;
 };
 
@@ -130,7 +131,7 @@ struct StageArgs {
   uint32_t *clear = nullptr;        // optional: clear_words words the kernel sets to zero (memory of an earlier
   uint32_t clear_words = 0;         // kernel that nobody needs any more)
   // The sample of the NEXT call on the same workspace (a tensor of this one's type and of next_n elements, 0:
-  // this one's length; next_k its k) is taken by this kernel's workgroups when they are through with their own
+  // this one's length; next_k its k) is taken by some of this kernel's workgroups before they start on their own
   // tensor: next_hist = that call's sampling memory (zero, left as k_sample_hist leaves it), next_floor
   // receives its floor key.
   const void *next_in = nullptr;

@@ -837,18 +837,23 @@ __device__ inline void stage_flush(uint32_t count, int32_t *st_idx, S *st_val, S
 // other.  A device-wide counter serves about 90 tickets per microsecond, and 768 workgroups asking one
 // counter every few microseconds would queue up for it: the workgroups form kStageGroups groups (by number
 // modulo kStageGroups) with a counter each, and ticket t of group g is short tile number g + t * kStageGroups.
+// The `late` first workgroups, which take the next call's sample first, go without the first `skip` of those
+// tiles: what the others read in the meantime.
 constexpr int kStageBig = 2;    // both tile lengths must be at least 2: the loads run two sub-tiles ahead
 constexpr int kStageSmall = 2;
 constexpr int kStageGroups = 8;
+constexpr uint32_t kStageLate = 2;   // some 8 us
 constexpr int kStageTicketPad = 32;  // words between two ticket counters: a 128-byte line each
 struct StageSched {
   uint32_t fixed;        // counter-free tiles per workgroup
+  uint32_t late, skip;
   uint32_t fixed_subs;   // sub-tiles they cover together
   uint32_t ticket_tiles; // tiles of kStageSmall sub-tiles after that
 };
 
-// LDS of a selecting workgroup that changes hands: the stage with what a flush needs, and after the last
-// flush the window of the next call's sample (16-bit counters, two to a word, a pad word per 32).
+// LDS of a selecting workgroup that changes hands: the stage with what a flush needs, and before the first
+// sub-tile the window of the next call's sample (16-bit counters, two to a word, a pad word per 32).
+constexpr int kSampleOwn = 6;        // vectors of the sample per thread
 constexpr int kSampleWindow = 8192;  // bins below a workgroup's largest sample element that it counts
 template <typename S>
 struct StageRun {
@@ -864,8 +869,11 @@ struct StageRun {
 static_assert(sizeof(StageRun<uint16_t>) == sizeof(int32_t) * kScatStage + 2 * kScatStage + sizeof(StageFlushShared),
               "the window fits where the stage is");
 
-// The sample of the NEXT call's tensor, taken by the workgroups of this call's selecting kernel when they are
-// through with their own tensor: no launch of its own, and nothing that waits.  Every workgroup histograms its
+// The sample of the NEXT call's tensor, taken by some of the workgroups of this call's selecting kernel before they
+// start on their own tensor: no launch of its own, and nothing that waits.  The chain of memory round trips this is
+// (8 us) is over long before the kernel ends, and these workgroups take fewer tiles; taken by all
+// workgroups once they were through it stood at the kernel's end (62 M bf16 elements, twelve tensors in a row, with the
+// tails and merges: 91 us a tensor, now 81).  Each histograms its
 // share of the sample (the vectors k_sample_hist would read) in a window of kSampleWindow exact bins below
 // its own largest element (a factor 2^64 in magnitude; what lies further down cannot matter unless the
 // workgroup's largest element towers that far above the threshold, and leaving it out only lowers the floor)
@@ -882,22 +890,38 @@ __device__ inline void stage_sample_next(const StageSample &smp, uint32_t *windo
   const S *in = static_cast<const S *>(smp.in);
   const int64_t n = smp.n;
   const int64_t nvec = (n + V - 1) / V;
-  const int64_t first = (int64_t)blockIdx.x * kSelBlock + threadIdx.x, step = (int64_t)gridDim.x * kSelBlock;
+  const int64_t first = (int64_t)blockIdx.x * kSelBlock + threadIdx.x, step = (int64_t)smp.wgs * kSelBlock;
   if (threadIdx.x == 0) s_top = 0;
   for (int i = threadIdx.x; i < kSampleWindow / 2 + kSampleWindow / 64; i += kSelBlock) window[i] = 0;
   __syncthreads();
+  // a thread's first vectors are loaded side by side and kept (seldom are there more)
+  const bool aligned = (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
+  S own[kSampleOwn][V];
+  int live[kSampleOwn];
+#pragma unroll
+  for (int j = 0; j < kSampleOwn; ++j) {
+    const int64_t b = first + j * step;
+    const int64_t v = b < smp.nblocks ? sample_vec(b, smp.block_log2) : nvec;
+    live[j] = 0;
+    if (v < nvec) live[j] = aligned ? load_vec<S, true>(in, v * V, n, own[j]) : load_vec<S, false>(in, v * V, n, own[j]);
+  }
   uint32_t top = 0;
-  for (int64_t b = first; b < smp.nblocks; b += step) {
-    const int64_t v = sample_vec(b, smp.block_log2);
-    if (v >= nvec) continue;
-    S e[V];
-    const int live = load_vec<S, false>(in, v * V, n, e);
+  auto largest = [&](const S (&e)[V], int count) {
 #pragma unroll
     for (int i = 0; i < V; ++i)
-      if (i < live) {
+      if (i < count) {
         const uint32_t bin = (e[i] & KeyOf<S>::kMask) >> kShift;
         top = bin > top ? bin : top;
       }
+  };
+#pragma unroll
+  for (int j = 0; j < kSampleOwn; ++j) largest(own[j], live[j]);
+  for (int64_t b = first + kSampleOwn * step; b < smp.nblocks; b += step) {
+    const int64_t v = sample_vec(b, smp.block_log2);
+    if (v >= nvec) continue;
+    S e[V];
+    const int count = load_vec<S, false>(in, v * V, n, e);
+    largest(e, count);
   }
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) {
@@ -908,25 +932,30 @@ __device__ inline void stage_sample_next(const StageSample &smp, uint32_t *windo
   __syncthreads();
   const uint32_t hi_bin = s_top;
   const uint32_t lo_bin = hi_bin >= (uint32_t)kSampleWindow - 1u ? hi_bin - ((uint32_t)kSampleWindow - 1u) : 0u;
-  for (int64_t b = first; b < smp.nblocks; b += step) {  // the same vectors again (they are in the caches now)
-    const int64_t v = sample_vec(b, smp.block_log2);
-    if (v >= nvec) continue;
-    S e[V];
-    const int live = load_vec<S, false>(in, v * V, n, e);
+  auto add = [&](const S (&e)[V], int count) {
 #pragma unroll
     for (int i = 0; i < V; ++i)
-      if (i < live) {
+      if (i < count) {
         const uint32_t bin = (e[i] & KeyOf<S>::kMask) >> kShift;
         if (bin >= lo_bin) {
           const uint32_t w = bin - lo_bin;
           atomicAdd(&window[(w >> 1) + (w >> 6)], 1u << (16 * (w & 1u)));
         }
       }
+  };
+#pragma unroll
+  for (int j = 0; j < kSampleOwn; ++j) add(own[j], live[j]);
+  for (int64_t b = first + kSampleOwn * step; b < smp.nblocks; b += step) {  // these vectors again (they are in the caches now)
+    const int64_t v = sample_vec(b, smp.block_log2);
+    if (v >= nvec) continue;
+    S e[V];
+    const int count = load_vec<S, false>(in, v * V, n, e);
+    add(e, count);
   }
   __syncthreads();
   {
     // from the top down, until the workgroup has added a few times its share of the rank (see k_sample_hist)
-    const uint64_t lim64 = 4ull * smp.rank / gridDim.x + 256ull;
+    const uint64_t lim64 = 4ull * smp.rank / smp.wgs + 256ull;
     const uint32_t limit = lim64 > 0xffffffffull ? 0xffffffffu : (uint32_t)lim64;
     uint32_t c[kWords];
     uint32_t mine = 0;
@@ -952,7 +981,7 @@ __device__ inline void stage_sample_next(const StageSample &smp, uint32_t *windo
   // the adds are carried out before the workgroup counts itself as finished (see k_sample_hist)
   wait_global_acks();
   __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(&smp.hist[kFineBins], 1u) == gridDim.x - 1;
+  if (threadIdx.x == 0) s_last = atomicAdd(&smp.hist[kFineBins], 1u) == smp.wgs - 1u;
   __syncthreads();
   if (s_last) sample_pick_block<kSelBlock>(smp.hist, smp.rank, kShift, smp.floor_out, smem);
 }
@@ -971,7 +1000,7 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
   for (uint32_t i = blockIdx.x * kSelBlock + threadIdx.x; i < clear_words; i += gridDim.x * kSelBlock) clear[i] = 0;
   __shared__ uint32_t s_wave[2][kWaves];
   __shared__ uint32_t s_next[2];
-  // the stage and what a flush needs; after the last flush, the window of the next call's sample
+  // the stage and what a flush needs; before that, the window of the next call's sample
   __shared__ StageRun<S> s_run;
   int32_t (&st_idx)[kScatStage] = s_run.run.idx;
   S (&st_val)[kScatStage] = s_run.run.val;
@@ -987,6 +1016,10 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
   if (floor_key == 0) floor_key = 1u;  // zeros are never selected
   if (floor_key > KeyOf<S>::kMask) floor_key = KeyOf<S>::kMask + 1u;  // nothing qualifies
   const int wave = threadIdx.x >> 6;
+  if (next.hist && blockIdx.x < next.wgs) {
+    stage_sample_next<S>(next, s_run.window, s_pick);
+    __syncthreads();  // the window's memory is the stage's from here on
+  }
 
   // A tile is (first sub-tile, number of sub-tiles); length 0 means there is none.  The current tile and the
   // one after it are always known (the loads run two sub-tiles ahead); the ticket of the tile after those is
@@ -994,8 +1027,11 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
   // has a whole tile's time to answer.  Three register sets take turns: while one sub-tile is examined the loads
   // of the next two are in flight.
   uint32_t cur_first = 0, cur_len = 0, nxt_first = 0, nxt_len = 0;
+  const bool late = blockIdx.x < sch.late;  // has taken a share of the next sample
   auto fixed_tile = [&](uint32_t i, uint32_t &first, uint32_t &len) {
-    first = (i * gridDim.x + blockIdx.x) * (uint32_t)kStageBig;
+    const uint32_t tile = i < sch.skip ? i * (gridDim.x - sch.late) + blockIdx.x - sch.late
+                                       : i * gridDim.x + blockIdx.x - sch.skip * sch.late;
+    first = tile * (uint32_t)kStageBig;
     len = (uint32_t)kStageBig;
   };
   auto ticket_tile = [&](uint32_t j, uint32_t &first, uint32_t &len) {
@@ -1018,6 +1054,7 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
   // tile number tn of this block if no ticket is needed for it: counter-free tiles first, then the block's
   // own first short tile
   auto known_tile = [&](uint32_t tn, uint32_t &first, uint32_t &len) {
+    if (late) tn += sch.skip;
     if (tn < sch.fixed) {
       fixed_tile(tn, first, len);
       return true;
@@ -1174,10 +1211,6 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
     const uint32_t c = s_tail;
     if (c) stage_flush<S>(c, st_idx, st_val, s_flush, hist, floor_key, out, status);
   }
-  if (next.hist) {
-    __syncthreads();  // the stage is no longer needed
-    stage_sample_next<S>(next, s_run.window, s_pick);
-  }
   if (hist) {
     __syncthreads();
     uint32_t *row = cand_hist + (size_t)(blockIdx.x % kCandRows) * kCandBins;
@@ -1236,8 +1269,6 @@ static int stage_launch(const StageArgs &a, hipStream_t stream) {
   // tickets 280 us, two thirds fixed 252, seven eighths 247, everything fixed 258)
   StageSched sch;
   sch.fixed = (uint32_t)(subs * 7 / 8 / ((int64_t)kStageBig * blocks));
-  sch.fixed_subs = sch.fixed * (uint32_t)kStageBig * (uint32_t)blocks;
-  sch.ticket_tiles = (uint32_t)ceil_div(subs - (int64_t)sch.fixed_subs, kStageSmall);
   const S *in = static_cast<const S *>(a.in);
   const bool aligned = (reinterpret_cast<uintptr_t>(in) & 15u) == 0 && a.n >= V;
   const StageSlabs out{a.geo, a.cg, a.coarse_cursor, a.coarse_words, a.wide ? 1u : 0u};
@@ -1252,7 +1283,15 @@ static int stage_launch(const StageArgs &a, hipStream_t stream) {
     next.block_log2 = sp.log2;
     next.nblocks = sp.nblocks;
     next.floor_out = a.next_floor;
+    // kSampleOwn vectors of the sample per thread, at least 64 workgroups
+    int64_t wgs = ceil_div(sp.nblocks, kSampleOwn * kSelBlock);
+    if (wgs < 64) wgs = 64;
+    next.wgs = (uint32_t)(wgs < blocks ? wgs : blocks);
   }
+  sch.late = next.wgs;
+  sch.skip = next.wgs > 0 && next.wgs < blocks ? (sch.fixed < kStageLate ? sch.fixed : kStageLate) : 0u;
+  sch.fixed_subs = (uint32_t)(((int64_t)sch.fixed * blocks - (int64_t)sch.skip * sch.late) * kStageBig);
+  sch.ticket_tiles = (uint32_t)ceil_div(subs - (int64_t)sch.fixed_subs, kStageSmall);
   ProfScope prof(kProfSelectStage, stream);
   if (aligned)
     k_select_stage<S, true><<<dim3((unsigned)blocks), dim3(kSelBlock), 0, stream>>>(
