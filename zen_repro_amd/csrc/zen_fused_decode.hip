@@ -198,24 +198,31 @@ __device__ inline uint32_t fd_value<uint32_t>(uint32_t v) {
 }
 
 // One workgroup per tile.  Lane p of every wave knows list p's members in the tile, the first bit of their range
-// and where its values start; the lists' members are cut into chunks of 640, dealt to the eight waves in turn.  A
+// and where its values start; the lists' members are cut into chunks of 640, dealt to the waves in turn.  A
 // wave gets the chunk's bits as ten 64-bit words in scalar registers: the word is the mask of the lanes whose
 // member has a value, a lane's value is the one numbered by the set bits below it, and its place in the tile is
 // the chunk's next entry of the dictionary, so that all loads are consecutive, ten of each kind in flight.  The
 // places written are put together in LDS and leave with full-width stores.
 // Bound by memory: two bytes of dictionary and one element of output per index, and the values.  62 M bf16 elements
-// on sixteen ranks, 71 % of them set, 0.34 GB: 79 us; 268 M elements, 11 % set, 1.13 GB: 300 us.  One SET bit per
+// on sixteen ranks, 71 % of them set, 0.34 GB: 79 us; 268 M elements, 11 % set, 1.13 GB: 265 us.  One SET bit per
 // thread and turn, looked up in staged copies of the tile's bytes and values, took 307 and 411 us; with each value's
-// load in a branch of its own, which makes the compiler wait for it there, this kernel took 129 and 428.
+// load in a branch of its own, which makes the compiler wait for it there, this kernel took 129 and 428 (79 and 300 without).
+// Waves of a workgroup meet at its two barriers, so small workgroups keep loads and stores going side by side as long
+// as their tiles' LDS lets a compute unit hold enough of them: 16 KB a tile for bf16, four waves (the all-reduce of
+// the 268 M elements 803 us; 837 with eight waves, 872 with two, 940 with sixteen), 32 KB for fp32, eight (200 M
+// elements, two ranks: 865; 960 with four).
+template <typename S>
+constexpr int fd_tile_block() { return sizeof(S) == 2 ? 256 : 512; }
 constexpr int kFdWords = 10;                 // words of a chunk: sixteen lists have 512 +- 70 members in a tile
 constexpr int kFdMembers = 64 * kFdWords;    // members of a chunk
 
 template <typename S>
-__global__ __launch_bounds__(kFdBlock, 8) void k_fd_tiles(const uint16_t *__restrict__ order,
+__global__ __launch_bounds__(fd_tile_block<S>(), sizeof(S) == 2 ? 6 : 8) void k_fd_tiles(const uint16_t *__restrict__ order,
                                                        const uint32_t *__restrict__ below,
                                                        const uint32_t *__restrict__ vstart,
                                                        const uint32_t *__restrict__ gpre, int P, uint32_t n,
                                                        FdLists lists, S *__restrict__ dense, int32_t *status) {
+  constexpr int kBlock = fd_tile_block<S>();
   __shared__ __attribute__((aligned(16))) S s_tile[kFdTile];
   const uint32_t tile = blockIdx.x;
   const uint32_t tile_base = tile * (uint32_t)kFdTile;
@@ -231,7 +238,7 @@ __global__ __launch_bounds__(kFdBlock, 8) void k_fd_tiles(const uint16_t *__rest
   {
     uint4 *z = reinterpret_cast<uint4 *>(s_tile);
 #pragma unroll
-    for (int i = 0; i < (int)(kFdTile * sizeof(S) / 16) / kFdBlock; ++i) z[i * kFdBlock + threadIdx.x] = make_uint4(0, 0, 0, 0);
+    for (int i = 0; i < (int)(kFdTile * sizeof(S) / 16) / kBlock; ++i) z[i * kBlock + threadIdx.x] = make_uint4(0, 0, 0, 0);
   }
   uint32_t cnt = b1 - b0;
   if (cnt > (uint32_t)kFdTile) cnt = 0;  // cannot be with a table this library built
@@ -242,7 +249,7 @@ __global__ __launch_bounds__(kFdBlock, 8) void k_fd_tiles(const uint16_t *__rest
   bool bad = false;
   __syncthreads();
 #pragma unroll 1
-  for (uint32_t c = (uint32_t)wave; c < nchunks && !odd; c += kFdBlock / 64) {
+  for (uint32_t c = (uint32_t)wave; c < nchunks && !odd; c += kBlock / 64) {
     const int p = (int)__popcll(__ballot(cincl <= c));  // the chunk's list
     const uint32_t j0 = (c - (uint32_t)__builtin_amdgcn_readlane((int)(cincl - chunks), p)) * kFdMembers;
     const uint32_t members = (uint32_t)__builtin_amdgcn_readlane((int)cnt, p) - j0;  // from here on, > 0
@@ -324,10 +331,10 @@ __global__ __launch_bounds__(kFdBlock, 8) void k_fd_tiles(const uint16_t *__rest
     const u32x4 *src = reinterpret_cast<const u32x4 *>(s_tile);
     u32x4 *dst = reinterpret_cast<u32x4 *>(dense + tile_base);
 #pragma unroll
-    for (int i = 0; i < kPieces / kFdBlock; ++i)
-      __builtin_nontemporal_store(src[i * kFdBlock + threadIdx.x], dst + i * kFdBlock + threadIdx.x);
+    for (int i = 0; i < kPieces / kBlock; ++i)
+      __builtin_nontemporal_store(src[i * kBlock + threadIdx.x], dst + i * kBlock + threadIdx.x);
   } else {
-    for (uint32_t e = threadIdx.x; e < (uint32_t)kFdTile && tile_base + e < n; e += kFdBlock) dense[tile_base + e] = s_tile[e];
+    for (uint32_t e = threadIdx.x; e < (uint32_t)kFdTile && tile_base + e < n; e += kBlock) dense[tile_base + e] = s_tile[e];
   }
   if ((bad || odd) && lane == 0) atomicOr(status, ZEN_STAT_BAD_INDEX);
 }
@@ -424,10 +431,10 @@ int zen_bitmap_dense_lists(const void *dict, int64_t numel, int partitions, cons
   k_fd_groups<<<dim3((unsigned)partitions), dim3(kFdGroupsMax), 0, s>>>(gsum, groups, partitions);
   ZEN_LAUNCH_CHECK("k_fd_groups");
   if (dtype == ZEN_BF16)
-    k_fd_tiles<uint16_t><<<dim3(tiles), dim3(kFdBlock), 0, s>>>(order, below, vstart, gsum, partitions, (uint32_t)numel,
+    k_fd_tiles<uint16_t><<<dim3(tiles), dim3(fd_tile_block<uint16_t>()), 0, s>>>(order, below, vstart, gsum, partitions, (uint32_t)numel,
                                                                 lists, static_cast<uint16_t *>(dense), status);
   else
-    k_fd_tiles<uint32_t><<<dim3(tiles), dim3(kFdBlock), 0, s>>>(order, below, vstart, gsum, partitions, (uint32_t)numel,
+    k_fd_tiles<uint32_t><<<dim3(tiles), dim3(fd_tile_block<uint32_t>()), 0, s>>>(order, below, vstart, gsum, partitions, (uint32_t)numel,
                                                                 lists, static_cast<uint32_t *>(dense), status);
   ZEN_LAUNCH_CHECK("k_fd_tiles");
   return ZEN_OK;
