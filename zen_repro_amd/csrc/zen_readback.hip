@@ -6,7 +6,7 @@
 // stores them, widened to 64 bits, into pinned host memory; the host watches the word that is stored last.  Each
 // of the two waits of a 1 Mi-element bucket's all-reduce got 13 us shorter by it (218 -> 191 us), and with the
 // counting kernel below in place of a library reduction the load balance of a 12.9 M-element fp32 tensor of
-// unknown density went from 242 to 178 us.
+// unknown density went from 242 to 178 us, before the counting kernel had 256 workgroups.
 #include <immintrin.h>  // host pass: _mm_pause
 
 #include "zen_select.h"
@@ -35,8 +35,10 @@ __global__ void k_read_back(ReadBack r, int64_t *host, int64_t ticket) {
 }
 
 // Elements with key >= max(thr[0], 1) (thr == nullptr: the nonzero ones).  Bound by the one read of the tensor:
-// four vectors per thread are in flight, a workgroup adds up in registers and touches the counter once.
-constexpr int kCountBlock = 512, kCountVecs = 4;
+// four vectors per thread are in flight, a workgroup adds up in registers and touches the counter once.  One address
+// takes an add every ten nanoseconds, so there are few workgroups: 12.9 M fp32 elements 10.3 us, 62 M bf16 20.8 (1024
+// workgroups of 512 threads, whose adds queue up: 19.3 and 24.5).
+constexpr int kCountBlock = 1024, kCountVecs = 4;
 
 template <typename S, bool ALIGNED>
 __global__ __launch_bounds__(kCountBlock) void k_count(const S *__restrict__ in, int64_t n,
@@ -73,7 +75,7 @@ template <typename S>
 void launch_count(const S *in, int64_t n, const uint32_t *thr, int64_t *count, hipStream_t s) {
   const int64_t per = (int64_t)kCountBlock * kCountVecs * VecOf<S>::kN;
   int64_t blocks = ceil_div(n, per);
-  if (blocks > 1024) blocks = 1024;  // four resident workgroups per compute unit
+  if (blocks > 256) blocks = 256;  // one per compute unit
   unsigned long long *c = reinterpret_cast<unsigned long long *>(count);
   if ((reinterpret_cast<uintptr_t>(in) & 15u) == 0)
     k_count<S, true><<<dim3((unsigned)blocks), dim3(kCountBlock), 0, s>>>(in, n, thr, c);
