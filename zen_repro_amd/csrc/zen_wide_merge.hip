@@ -62,8 +62,10 @@ struct WideMergeShared {
 };
 
 // O: what is written for a sum (zen_common.h).  DENSE: out_val is the dense tensor [0, dense_n); the workgroup
-// writes its bucket's range of it whole: zeros while its records are on their way (62 M bf16 elements: the fill
-// and scatter kernels in front of and behind a sparse merge took 18 + 21 us), the sums behind them at the end.
+// writes its bucket's range of it whole, zeros between the steps of the ranking loops, the sums behind them at the
+// end (62 M bf16 elements, 3.1 M entries: 60 us; 69 with the zeros in front of the records' loads, which then wait for
+// them to be written; the fill and scatter kernels in front of and behind a sparse merge took 18 + 21 us.  Workgroups
+// of k_wide_scatter that do nothing else cost that kernel the 17 us they save this one).
 // DIRECT: the launch is one workgroup and one bucket, and the records are the list's entries themselves.
 template <typename I, typename S, typename O, bool DENSE, bool DIRECT>
 __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__restrict__ out_idx,
@@ -85,20 +87,28 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
   const uint32_t nb = DIRECT ? 1u : geo.nbuckets;
   if (b >= nb) return;
   const uint32_t lo = DIRECT ? 0u : geo.first_key(b);
+  // The bucket's range of a dense tensor: elements up to the first multiple of 16 bytes, vectors, elements.  The
+  // vectors' zeros are stored a few at a time between the steps of the ranking loops, whose LDS round trips leave the
+  // memory idle.
+  constexpr uint32_t V = 16 / sizeof(O);
+  uint32_t zero_vecs = 0, zero_at = tid, zero_each = 0;
+  u32x4 *zero_to = nullptr;
   if (DENSE) {
-    constexpr uint32_t V = 16 / sizeof(O);
     const uint32_t end = b + 1 < nb ? geo.first_key(b + 1) : dense_n;
-    // the first multiple of 16 bytes in the range, as an element number of the range
     const uint32_t skew = (uint32_t)((reinterpret_cast<uintptr_t>(out_val + lo) & 15u) / sizeof(O));
     uint32_t head = (V - skew) % V;
     if (head > end - lo) head = end - lo;
-    const uint32_t vecs = (end - lo - head) / V;
-    u32x4 *wide = reinterpret_cast<u32x4 *>(out_val + lo + head);
-    const u32x4 zero = {0, 0, 0, 0};
-    for (uint32_t i = tid; i < vecs; i += kWideBlock) wide[i] = zero;
+    zero_vecs = (end - lo - head) / V;
+    zero_to = reinterpret_cast<u32x4 *>(out_val + lo + head);
+    zero_each = (zero_vecs + kWideBlock * 2 * kWmSteps - 1) / (kWideBlock * 2 * kWmSteps);
     for (uint32_t i = tid; i < head; i += kWideBlock) out_val[lo + i] = O(0);
-    for (uint32_t i = lo + head + vecs * V + tid; i < end; i += kWideBlock) out_val[i] = O(0);
+    for (uint32_t i = lo + head + zero_vecs * V + tid; i < end; i += kWideBlock) out_val[i] = O(0);
   }
+  auto zero_some = [&]() {
+    if (!DENSE) return;
+    const u32x4 zero = {0, 0, 0, 0};
+    for (uint32_t i = 0; i < zero_each && zero_at < zero_vecs; ++i, zero_at += kWideBlock) zero_to[zero_at] = zero;
+  };
   uint32_t pcount[kWideSplit];
   uint32_t longest = 0;
 #pragma unroll
@@ -204,6 +214,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
     }
     rotate(w);
     rotate(ps);
+    zero_some();
   }
   __syncthreads();
   // rank = records of the bucket with a smaller (index, arrival number): those of the narrow ranges before,
@@ -259,6 +270,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
     rotate(rk);  // the step's ranks enter at the end: after the last step rank i belongs to record i
 #pragma unroll
     for (int k = 0; k < kWmLanes; ++k) rk[kWmItems - kWmLanes + k] = out[k];
+    zero_some();
   }
   __syncthreads();
   {
