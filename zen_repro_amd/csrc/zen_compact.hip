@@ -7,7 +7,7 @@
 // (k_compact_move).  A stretch with more than an eighth of its elements selected does not fit its part: the second
 // kernel walks it again and writes it straight to its place.  Up to kOneMax elements one workgroup does both steps
 // in one launch.
-// Bound by the read of the tensor and the extraction of what is selected (62 M bf16 elements, 4.4 % selected: 35 + 12
+// Bound by the read of the tensor and the extraction of what is selected (62 M bf16 elements, 4.4 % selected: 28 + 12
 // us, of which the read alone would take 18).  A single pass with tiles chained by
 // look-back took 88 us there: thousands of tiles draw their numbers from one counter, 11 ns each, and wait for
 // each other's prefixes.
@@ -73,54 +73,62 @@ __device__ __forceinline__ uint32_t walk(const S *__restrict__ in, int64_t begin
   const int lane = lane_id();
   uint32_t found = 0;
   constexpr int64_t kStep = (int64_t)row<S>() * kRows;
-  auto load = [&](int64_t base, uint4 (&q)[kRows]) {
+  auto load = [&](int64_t base, uint4 &a, uint4 &b, uint4 &c, uint4 &d) {
     if (ALIGNED && base + kStep <= end) {
-#pragma unroll
-      for (int r = 0; r < kRows; ++r) q[r] = *reinterpret_cast<const uint4 *>(in + base + r * row<S>() + lane * V);
+      const S *at = in + base + lane * V;
+      a = *reinterpret_cast<const uint4 *>(at);
+      b = *reinterpret_cast<const uint4 *>(at + row<S>());
+      c = *reinterpret_cast<const uint4 *>(at + 2 * row<S>());
+      d = *reinterpret_cast<const uint4 *>(at + 3 * row<S>());
     } else {
-#pragma unroll
-      for (int r = 0; r < kRows; ++r) {
+      auto one = [&](int64_t first, uint4 &q) {
         S e[V];
-        load_vec<S, ALIGNED>(in, base + r * row<S>() + lane * V, end, e);  // past the end: zeros, never selected
-        __builtin_memcpy(&q[r], e, 16);
-      }
+        load_vec<S, ALIGNED>(in, first, end, e);  // past the end: zeros, never selected
+        __builtin_memcpy(&q, e, 16);
+      };
+      one(base + lane * V, a);
+      one(base + row<S>() + lane * V, b);
+      one(base + 2 * row<S>() + lane * V, c);
+      one(base + 3 * row<S>() + lane * V, d);
     }
   };
-  uint4 q[kRows], next[kRows];
-  if (begin < end) load(begin, next);
+  auto write = [&](const uint4 &q, uint32_t bits, uint32_t pos, uint32_t first) {
+    while (bits) {
+      const uint32_t e = (uint32_t)__ffs((int)bits) - 1u;
+      bits &= bits - 1u;
+      if (pos < room) {
+        *reinterpret_cast<I *>(reinterpret_cast<char *>(idx) + (uint32_t)(pos * sizeof(I))) = (I)(first + e);
+        *reinterpret_cast<S *>(reinterpret_cast<char *>(val) + (uint32_t)(pos * sizeof(S))) = vec_pick(q, e, S(0));
+      }
+      ++pos;
+    }
+  };
+  // two rows' counts in the halves of a word (a row has 512 elements at most)
+  auto two = [&](const uint4 &q0, const uint4 &q1, uint32_t first) {
+    const uint32_t x0 = vec_flags(q0, least, S(0)), x1 = vec_flags(q1, least, S(0));
+    const uint32_t c = (uint32_t)__popc(x0) | ((uint32_t)__popc(x1) << 16);
+    const uint32_t incl = scan_dpp(c);
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    if (WRITE) {
+      const uint32_t before = incl - c;
+      write(q0, x0, found + (before & 0xffffu), first);
+      write(q1, x1, found + (total & 0xffffu) + (before >> 16), first + (uint32_t)row<S>());
+    }
+    found += (total & 0xffffu) + (total >> 16);
+  };
+  static_assert(kRows == 4, "four rows by name");
+  uint4 a, b, c, d, na, nb, nc, nd;
+  if (begin < end) load(begin, na, nb, nc, nd);
 #pragma unroll 1
   for (int64_t base = begin; base < end; base += kStep) {
-#pragma unroll
-    for (int r = 0; r < kRows; ++r) q[r] = next[r];
-    if (base + kStep < end) load(base + kStep, next);  // on its way while these rows are looked at
-    uint32_t x[kRows];
-#pragma unroll
-    for (int r = 0; r < kRows; ++r) x[r] = vec_flags(q[r], least, S(0));
-#pragma unroll
-    for (int r = 0; r < kRows; r += 2) {  // two rows' counts in the halves of a word (a row has 512 elements at most)
-      const uint32_t c = (uint32_t)__popc(x[r]) | ((uint32_t)__popc(x[r + 1]) << 16);
-      const uint32_t incl = scan_dpp(c);
-      const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-      if (WRITE) {
-        const uint32_t before = incl - c;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          uint32_t pos = found + (h ? (total & 0xffffu) + (before >> 16) : before & 0xffffu);
-          uint32_t bits = x[r + h];
-          const uint32_t first = (uint32_t)base + (uint32_t)((r + h) * row<S>() + lane * V);
-          while (bits) {
-            const uint32_t e = (uint32_t)__ffs((int)bits) - 1u;
-            bits &= bits - 1u;
-            if (pos < room) {
-              *reinterpret_cast<I *>(reinterpret_cast<char *>(idx) + (uint32_t)(pos * sizeof(I))) = (I)(first + e);
-              *reinterpret_cast<S *>(reinterpret_cast<char *>(val) + (uint32_t)(pos * sizeof(S))) = vec_pick(q[r + h], e, S(0));
-            }
-            ++pos;
-          }
-        }
-      }
-      found += (total & 0xffffu) + (total >> 16);
-    }
+    a = na;
+    b = nb;
+    c = nc;
+    d = nd;
+    if (base + kStep < end) load(base + kStep, na, nb, nc, nd);  // on its way while these rows are looked at
+    const uint32_t first = (uint32_t)base + (uint32_t)(lane * V);
+    two(a, b, first);
+    two(c, d, first + 2u * (uint32_t)row<S>());
   }
   return found;
 }
