@@ -127,6 +127,8 @@ __global__ __launch_bounds__(kFdScanBlock) void k_fd_scan(uint32_t *__restrict__
 // Set bits of bitmap `bm` in the bit range [b0, b1); bytes at or beyond `bytes` count as zero.  Read as
 // aligned 64-bit words: a word that holds one byte of the bitmap lies in that byte's page, and what it holds
 // beside the bitmap is masked away.
+// AHEAD words are on their way at a time.
+template <int AHEAD>
 __device__ inline uint32_t popcount_range(const uint8_t *__restrict__ bm, int64_t bytes, uint32_t b0, uint32_t b1) {
   const uint64_t limit = (uint64_t)bytes * 8u;
   if (b1 > limit) b1 = (uint32_t)limit;
@@ -136,11 +138,17 @@ __device__ inline uint32_t popcount_range(const uint8_t *__restrict__ bm, int64_
   const uint64_t lo = (uint64_t)b0 + (addr & 7u) * 8u, hi = (uint64_t)b1 + (addr & 7u) * 8u;  // bit numbers from words[0] on
   const uint64_t first = lo >> 6, last = (hi - 1u) >> 6;
   uint32_t c = 0;
-  for (uint64_t w = first; w <= last; ++w) {
-    unsigned long long x = words[w];
-    if (w == first) x &= ~0ull << (lo & 63u);
-    if (w == last) x &= ~0ull >> (63u - ((hi - 1u) & 63u));
-    c += (uint32_t)__popcll(x);
+  for (uint64_t w0 = first; w0 <= last; w0 += AHEAD) {
+    unsigned long long x[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) x[j] = words[w0 + j <= last ? w0 + j : last];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      const uint64_t w = w0 + j;
+      if (w == first) x[j] &= ~0ull << (lo & 63u);
+      if (w == last) x[j] &= ~0ull >> (63u - ((hi - 1u) & 63u));
+      c += w <= last ? (uint32_t)__popcll(x[j]) : 0u;
+    }
   }
   return c;
 }
@@ -154,6 +162,7 @@ inline uint32_t fd_groups(uint32_t tiles) { return (tiles + kFdGroup - 1) / kFdG
 // Per (group of tiles, list): set bits in each tile's bit range of the list's bitmap, summed up inside the
 // group.  A bitmap shorter than its list (the reference's mask would not fit the member list, comm.py:97-98)
 // raises ZEN_STAT_BAD_INDEX.
+constexpr int kFdCountAhead = 5;  // a tile's range of a list spans eight or nine words at sixteen ranks (268 M elements: 22 us with one, 16 with five)
 __global__ __launch_bounds__(kFdGroup) void k_fd_count(const uint32_t *__restrict__ below, uint32_t tiles, int P,
                                                        FdLists lists, uint32_t *__restrict__ vstart,
                                                        uint32_t *__restrict__ gsum, int32_t *status) {
@@ -166,7 +175,7 @@ __global__ __launch_bounds__(kFdGroup) void k_fd_count(const uint32_t *__restric
     const uint32_t b0 = below[i], b1 = below[i + P];
     const int64_t bytes = lists.bytes[p];
     if (tile == tiles - 1 && ((int64_t)b1 + 7) / 8 > bytes) atomicOr(status, ZEN_STAT_BAD_INDEX);
-    cnt = popcount_range(lists.bitmap[p], bytes, b0, b1);
+    cnt = popcount_range<kFdCountAhead>(lists.bitmap[p], bytes, b0, b1);
   }
   uint32_t total;
   const uint32_t before = block_exclusive_scan<uint32_t, kFdGroup>(cnt, s_scan, &total);
@@ -286,7 +295,7 @@ __global__ __launch_bounds__(fd_tile_block<S>(), sizeof(S) == 2 ? 6 : 8) void k_
     if (j0) {  // 128 bits per lane
       const uint32_t from = bit0 - j0 + (uint32_t)lane * (kFdTile / 64);
       const uint32_t to = from + kFdTile / 64;
-      nth += wave_sum(from < bit0 ? popcount_range(lists.bitmap[p], lists.bytes[p], from, to < bit0 ? to : bit0) : 0u);
+      nth += wave_sum(from < bit0 ? popcount_range<1>(lists.bitmap[p], lists.bytes[p], from, to < bit0 ? to : bit0) : 0u);
     }
     nth = (uint32_t)__builtin_amdgcn_readfirstlane((int)nth);
     const uint32_t have = lists.vals[p];
