@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define ZEN_ABI_VERSION 5 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table; 4: zen_read_back, zen_count, zen_merge_rounded, zen_decode_dense_lists, zen_bitmap_dense_lists; 5: zen_table_find, zen_table_gather */
+#define ZEN_ABI_VERSION 6 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table; 4: zen_read_back, zen_count, zen_merge_rounded, zen_decode_dense_lists, zen_bitmap_dense_lists; 5: zen_table_find, zen_table_gather; 6: ZEN_MODE_NO_SAMPLES */
 
 #define ZEN_F32 0
 #define ZEN_BF16 1
@@ -72,6 +72,11 @@ extern "C" {
    entries (at most 256 wide buckets, one resident workgroup each, whose launches the library keeps from
    overlapping on a device) and take the bucket-slab path wherever that fits.  Results are the same. */
 #define ZEN_MODE_SLABS 0x2000
+/* OR-ed into the `mode` of zen_load_balance with k == 0: the caller vouches that no sample taken ahead
+   (zen_load_balance_prepare, zen_encode_merge's next_input) waits in `table`, that every word of it is zero.  Tables of
+   2^20 to 4 Mi slots then serve as owner tables, the quickest way at those sizes; without the flag such a call takes
+   a path that leaves waiting samples alone.  Smaller tables never hold a sample. */
+#define ZEN_MODE_NO_SAMPLES 0x4000
 
 int zen_abi_version(void);
 
@@ -249,14 +254,17 @@ int zen_select(const void *input, int dtype, int64_t n, const uint32_t *thr,
  * is partition p's length.  m is the table size of
  * tensor_load_balance.py:15-16; the serial capacity is n / partitions / 10
  * per partition (tensor_load_balance.py:18).
- * `table` is int32[m] scratch that must be all zero on entry and is all zero
+ * `table` is int32[m] scratch that must be all zero on entry (but for samples
+ * that wait for their calls, see zen_load_balance_prepare) and is all zero
  * again on return (so one allocation serves every call, and no call spends a
  * kernel on clearing counters: those live in the table too); after a call that
  * raised ZEN_STAT_RETRY or ZEN_STAT_INTERNAL, or returned an error code, its
  * contents are undefined and the caller clears it.  ZEN_MODE_GENERAL keeps the owner of every probed slot in
- * it, like the reference; ZEN_MODE_FAST sorts the selected entries by their
- * level-1 slot instead and only borrows a corner of the table as a hash map
- * for the few entries that collide (ZEN_STAT_RETRY if there are too many).
+ * it, like the reference, and so does ZEN_MODE_FAST where the table is small
+ * (below 2^20 slots; up to 4 Mi slots with k == 0 and ZEN_MODE_NO_SAMPLES; tables of up to 32768 slots are kept in
+ * LDS).  Otherwise ZEN_MODE_FAST sorts the selected entries by their level-1 slot and borrows at most half of the
+ * table as a hash map for the few entries that collide (ZEN_STAT_RETRY if there are too many), and the megabyte
+ * behind it for its counters and the samples.
  */
 size_t zen_load_balance_workspace(int64_t n, int64_t m, int dtype, int64_t capacity, int partitions);
 int zen_load_balance(const void *input, int dtype, int64_t n, int64_t m,
@@ -275,7 +283,9 @@ int zen_load_balance(const void *input, int dtype, int64_t n, int64_t m,
  * stream wait); `mode` is ZEN_MODE_FAST, with ZEN_MODE_SECOND for the second of two sets of sampling memory,
  * which lets a caller prepare call i + 1 while call i (prepared with the other set) is in flight; a set may be
  * prepared again once the call that used it has finished.  A sample that no call will pick up after all is
- * dropped with mode | ZEN_MODE_DISCARD (same arguments; the table is not all zero before that).  On paths with
+ * dropped with mode | ZEN_MODE_DISCARD (same arguments; the table is not all zero before that).  While a sample
+ * waits, the table and the workspace take other calls on paths 2 and 3 only (zen_load_balance_path): on the other
+ * paths they are used as a whole.  On paths with
  * nothing to take ahead the function does nothing and the flag is ignored.  No counterpart in the reference.
  */
 int zen_load_balance_prepare(const void *input, int dtype, int64_t n, int64_t m, int partitions, int64_t k,

@@ -515,6 +515,55 @@ def test_sample_taken_ahead_gives_the_same_result(zen, oracle):
     assert int(tp._table(g.device, m).count_nonzero()) == 0
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("n,P", [(1 << 20, 4), ((1 << 21) + 4096, 8), (1 << 22, 16)])
+def test_calls_that_take_no_sample_leave_a_waiting_one_alone(zen, oracle, n, P, dtype):
+    """Tables of 2^20 to 4 Mi slots hold the samples taken ahead and serve as owner tables for calls without a k: with
+    such calls (nonzeros, a threshold, the general mode) between a sample and its call, all of them give the oracle's
+    results, the sample is picked up (dropped in front of the general mode), and the table ends all zero."""
+    from zen_repro_amd import _lib
+
+    rng = np.random.default_rng(57)
+    sparse = make_grad(oracle, n, 0.01, dtype, seed=58)
+    full = make_grad(oracle, n, 1.0, dtype, seed=59)
+    k = n // 200
+    cap, room = k + k // 4 + 4096, n // 64 + 4096
+    key = oracle.kth_key(full, k)
+    top = oracle.load_balance(oracle.mask_dense(full, key)[0], P, 1, 3)
+    nonzeros = oracle.load_balance(sparse, P, 1, 3)
+    a, b = to_dev(sparse), to_dev(full)
+    thr = zen.topk_threshold(b, k)
+    side = torch.cuda.Stream()
+    tp = zen.TensorPartition(P, 1, 3)
+    torch.cuda.synchronize()
+
+    def check(out, want):
+        idx, val, splits, st = out
+        assert int(st.item()) == 0 and want[3] == 0
+        total = int(splits.sum())
+        assert np.array_equal(splits.cpu().numpy(), want[2])
+        assert np.array_equal(idx[:total].cpu().numpy(), want[0]) and np.array_equal(to_np(val[:total]), want[1])
+
+    calls = [lambda: (tp.load_balance_flat(a, None, room), nonzeros),
+             lambda: (tp.load_balance_flat(b, thr, room), top),
+             lambda: (tp.load_balance_flat(a, None, room, mode=_lib.MODE_GENERAL), nonzeros)]
+    for i in rng.permutation(np.repeat(np.arange(3), 2)):
+        with torch.cuda.stream(side):  # beside the call before, whose table it writes to
+            tp.prepare(b, k, cap)
+        state = tp._ahead_state(b.device, 0) if FLAGS == 0 else None
+        assert state is None or len(state["pending"]) == 1
+        out, want = calls[i]()
+        assert state is None or len(state["pending"]) == (i < 2)
+        top_out = tp.load_balance_flat(b, None, cap, k=k)
+        assert state is None or not state["pending"]
+        after = calls[i]()  # no sample waits now
+        check(out, want)
+        check(top_out, top)
+        check(*after)
+    torch.cuda.synchronize()
+    assert int(tp._table(b.device, tp.table_sizes(n)[0]).count_nonzero()) == 0
+
+
 def test_step_replayed_from_a_captured_graph(zen, oracle):
     """An encode (fused top-k) and a merge captured into a HIP graph, the merge forked onto a second stream:
     every replay, with eager calls on the same workspaces and a synchronisation in between, leaves the bytes

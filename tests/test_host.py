@@ -241,3 +241,29 @@ def test_ranges_are_off_by_default_and_cost_nothing():
         assert not isinstance(_lib.annotate("load_balance"), contextlib.nullcontext)
     finally:
         _lib.ranges_enable(was)
+
+
+def test_a_waiting_sample_keeps_the_owner_table_away(L):
+    """A sample taken ahead waits in its call's table (2^20 slots or more): a call that selects by threshold or takes
+    the nonzeros may use every word of such a table only where it is told that none waits there."""
+    from zen_repro_amd import _lib
+    from zen_repro_amd.tensor_load_balance import TensorPartition
+
+    n, room = 1 << 22, 1 << 14
+    assert L.zen_load_balance_path(n, n, _lib.BF16, room, 4, 0, _lib.MODE_FAST) in (2, 3)
+    assert L.zen_load_balance_path(n, n, _lib.BF16, room, 4, 0, _lib.MODE_FAST | _lib.MODE_NO_SAMPLES) == 1
+    assert L.zen_load_balance_path((1 << 20) - 4, (1 << 20) - 4, _lib.BF16, room, 4, 0, _lib.MODE_FAST) == 1  # holds none
+    assert L.zen_load_balance_path(n, n, _lib.BF16, room, 4, 4096, _lib.MODE_FAST | _lib.MODE_NO_SAMPLES) in (2, 3)
+
+    tp = TensorPartition.__new__(TensorPartition)
+    tp.partitions, tp.memory_scale, tp._on_buckets = 4, 1, {}
+    state, dropped = {"free": [None, None], "pending": []}, []
+    tp._ahead_state = lambda dev, slot: state
+    tp._discard = lambda entry, slot, dev: dropped.append(entry)
+    flat = torch.zeros(n, dtype=torch.bfloat16)
+    take = lambda mode: tp._take_ahead(flat, n, 0, room, None, 0, mode, None, None)
+    assert take(_lib.MODE_FAST) == (_lib.MODE_NO_SAMPLES, 0)
+    state["pending"].append("a sample")
+    assert take(_lib.MODE_FAST) == (0, 0) and state["pending"] and not dropped
+    # the general mode has no other way than through the whole table: what waits there is dropped first
+    assert take(_lib.MODE_GENERAL) == (_lib.MODE_NO_SAMPLES, 0) and not state["pending"] and dropped == ["a sample"]

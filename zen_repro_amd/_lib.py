@@ -17,13 +17,14 @@ MODE_ZEROED = 0x100  # zen_merge: the head of the workspace is zero (and stays s
 MODE_PREPARED, MODE_SECOND, MODE_DISCARD = 0x200, 0x400, 0x800  # zen_load_balance: the sample was taken ahead (zen_load_balance_prepare)
 MODE_FLOOR = 0x1000  # zen_load_balance with k > 0: thr holds a key close to the threshold, no sample is taken
 MODE_SLABS = 0x2000  # fast mode without the wide-bucket path (bucket slabs where they fit)
+MODE_NO_SAMPLES = 0x4000  # zen_load_balance with k == 0: no sample taken ahead waits in the table
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # ZEN_HIP_LIB names another build of the library (a debug build, a build with other compile-time settings)
 LIB_PATH = os.environ.get("ZEN_HIP_LIB") or os.path.join(_HERE, "csrc", "libzen_hip.so")
 
 # ZEN_ABI_VERSION of include/zen_hip.h this loader's signatures and structs are written for
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 _lib = None
 

@@ -330,7 +330,7 @@ class LoadBalanceAllreduce:
         if rc != _lib.OK:
             mws[:L.zen_merge_zero_bytes()].zero_()
         _lib.check(rc, "encode_merge")
-        partition._after_call(dev, slot, int(k), used)
+        partition._after_call(flat, int(k), capacity, slot, mode | flags, used)
         if nxt is not None:
             partition._sample_taken(nxt, int(next_k), next_capacity, ws, slot, 1 - used)
         return (out_idx, out_val, splits, status), (m_idx, m_val, count, m_status)

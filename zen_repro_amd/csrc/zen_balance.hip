@@ -378,10 +378,10 @@ size_t zen_load_balance_workspace(int64_t n, int64_t m, int dtype, int64_t capac
 }
 
 int zen_load_balance_path(int64_t n, int64_t m, int dtype, int64_t capacity, int partitions, int64_t k, int mode) {
-  const bool slabs_only = (mode & ZEN_MODE_SLABS) != 0;
+  const bool slabs_only = (mode & ZEN_MODE_SLABS) != 0, no_samples = (mode & ZEN_MODE_NO_SAMPLES) != 0;
   mode &= 0xff;
   if (mode != ZEN_MODE_FAST || partitions <= 0 || m <= 0 || m % partitions != 0) return 0;
-  if (!slabs_only && zen::table_balance_fits(n, m, partitions, k)) return 1;
+  if (!slabs_only && zen::table_balance_fits(n, m, partitions, k, no_samples)) return 1;
   if (!slabs_only && zen::wide_balance_fits(m, partitions, capacity, k, zen::wide_device_cus(), nullptr)) return 3;
   if (zen::slab_balance_fits(n, m, partitions, dtype, capacity, k, nullptr)) return 2;
   return m >= 4096 ? 1 : 0;
@@ -411,7 +411,7 @@ int zen_load_balance_prepare(const void *input, int dtype, int64_t n, int64_t m,
     return fail(ZEN_EWORKSPACE, "zen_load_balance_prepare: workspace too small");
   const int second = (mode & ZEN_MODE_SECOND) != 0;
   if ((mode & 0xff) != ZEN_MODE_FAST || k == 0 || (reinterpret_cast<uintptr_t>(table) & 7u) != 0 ||
-      (!(mode & ZEN_MODE_SLABS) && table_balance_fits(n, m, partitions, k)) ||
+      (!(mode & ZEN_MODE_SLABS) && table_balance_fits(n, m, partitions, k, false)) ||
       (!slab_balance_fits(n, m, partitions, dtype, capacity, k, nullptr) &&
        !wide_balance_fits(m, partitions, capacity, k, wide_device_cus(), nullptr)))
     return ZEN_OK;  // nothing to take ahead on the other paths
@@ -456,7 +456,8 @@ int load_balance_call(const void *input, int dtype, int64_t n, int64_t m, int pa
   }
   const bool slabs_only = (mode & ZEN_MODE_SLABS) != 0;
   const bool splits_zero = (mode & ZEN_MODE_ZEROED) != 0;
-  mode &= ~(ZEN_MODE_PREPARED | ZEN_MODE_SECOND | ZEN_MODE_FLOOR | ZEN_MODE_SLABS | ZEN_MODE_ZEROED);
+  const bool no_samples = (mode & ZEN_MODE_NO_SAMPLES) != 0;
+  mode &= ~(ZEN_MODE_PREPARED | ZEN_MODE_SECOND | ZEN_MODE_FLOOR | ZEN_MODE_SLABS | ZEN_MODE_ZEROED | ZEN_MODE_NO_SAMPLES);
   if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_load_balance: bad dtype");
   if (mode != ZEN_MODE_FAST && mode != ZEN_MODE_GENERAL) return fail(ZEN_EINVAL, "zen_load_balance: bad mode");
   if (n <= 0 || n > 0x7fffffffll || m <= 0 || m > 0x7fffffffll || partitions <= 0 || partitions > 65535 ||
@@ -476,7 +477,7 @@ int load_balance_call(const void *input, int dtype, int64_t n, int64_t m, int pa
   const uint32_t drop_key = (uint32_t)partitions * (g.npp + 1u);
   const int bits = ceil_log2_u64(drop_key);
   const bool small = mode == ZEN_MODE_FAST && !slabs_only && (reinterpret_cast<uintptr_t>(table) & 15u) == 0 &&
-                     table_balance_fits(n, m, partitions, k);
+                     table_balance_fits(n, m, partitions, k, no_samples);
   const bool wide = mode == ZEN_MODE_FAST && !slabs_only && (reinterpret_cast<uintptr_t>(table) & 7u) == 0 &&
                     wide_balance_fits(m, partitions, capacity, k, wide_device_cus(), nullptr);
   if (small || wide || (mode == ZEN_MODE_FAST && (reinterpret_cast<uintptr_t>(table) & 7u) == 0 &&

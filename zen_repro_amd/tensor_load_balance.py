@@ -44,6 +44,7 @@ class TensorPartition:
         self._tables = {}
         self._ahead = {}  # (device, slot) -> samples taken ahead of their calls (prepare)
         self._samples_next = {}  # shape of a call -> whether its pass over the tensor can take the next sample along
+        self._on_buckets = {}  # shape of a call -> whether it takes a path that leaves waiting samples alone
 
     # ------------------------------------------------------------ sizes
     def table_sizes(self, numel):
@@ -256,15 +257,35 @@ class TensorPartition:
         state["pending"].append((nxt.data_ptr(), nxt.numel(), next_k, capacity, ws.data_ptr(), which,
                                  _Mark(torch.cuda.current_stream(dev)), _lib.dtype_code(nxt), ws.numel()))
 
+    def _leaves_samples(self, flat, k, capacity, mode):
+        """Whether a call leaves the samples that wait on its slot alone.  The bucket paths do; the others take the
+        floors' place in the workspace, and the owner-table paths every word of the table."""
+        key = (flat.numel(), flat.dtype, k, capacity, mode & (0xff | _lib.MODE_SLABS | _lib.MODE_NO_SAMPLES))
+        able = self._on_buckets.get(key)
+        if able is None:
+            if len(self._on_buckets) >= 256:  # capacities may differ from call to call
+                self._on_buckets.clear()
+            able = self._on_buckets[key] = _lib.lib().zen_load_balance_path(
+                key[0], self.table_sizes(key[0])[0], _lib.dtype_code(flat), capacity, self.partitions, k,
+                key[4]) in (2, 3)
+        return able
+
     def _take_ahead(self, flat, n, k, capacity, ws, slot, mode, thr, near):
         """The sample taken ahead for the call that is about to be made, if there is one: (mode flags that tell
         the library, the set of sampling memory the call will use).  Samples taken for other calls stay where
-        they are; one that its bucket will never pick up (same tensor and size, other arguments) is dropped."""
+        they are, unless this call takes a path that has no place for them: then they are dropped, and their
+        calls sample for themselves.  So is one that its bucket will never pick up (same tensor and size, other
+        arguments)."""
         dev = flat.device
         state = self._ahead_state(dev, slot)  # None: no sample was ever taken ahead for this slot
-        if state is None or k <= 0:
-            return 0, 0
-        L = _lib.lib()
+        if state is None:
+            return (_lib.MODE_NO_SAMPLES if k <= 0 else 0), 0
+        if state["pending"] and not self._leaves_samples(flat, k, capacity, mode):
+            while state["pending"]:
+                self._discard(state["pending"].pop(0), slot, dev)
+        if k <= 0:
+            # a sample waits in the table of its call: that one must not become an owner table meanwhile
+            return (0 if state["pending"] else _lib.MODE_NO_SAMPLES), 0
         want = (flat.data_ptr(), n, k, capacity, ws.data_ptr())
         ahead = None
         for i, entry in enumerate(state["pending"]):
@@ -304,11 +325,17 @@ class TensorPartition:
             (_lib.MODE_SECOND if a_which else 0), ctypes.c_void_p(a_ws), a_bytes, _lib.stream_of(dev)),
             "load_balance discard")
 
-    def _after_call(self, dev, slot, k, used):
-        """The set of sampling memory a top-k call used is free again once the call has finished."""
-        state = self._ahead_state(dev, slot)
-        if k > 0 and state is not None:
-            state["free"][used] = _Mark(torch.cuda.current_stream(dev))
+    def _after_call(self, flat, k, capacity, slot, mode, used):
+        """The set of sampling memory a top-k call used is free again once the call has finished; both sets are, if
+        it took a path that uses the table and the workspace as a whole."""
+        state = self._ahead_state(flat.device, slot)
+        if state is None:
+            return
+        if not self._leaves_samples(flat, k, capacity, mode):
+            mark = _Mark(torch.cuda.current_stream(flat.device))
+            state["free"] = [mark, mark]
+        elif k > 0:
+            state["free"][used] = _Mark(torch.cuda.current_stream(flat.device))
 
     def load_balance_flat(self, tensor, thr=None, capacity=None, k=0, mode=_lib.MODE_FAST, thr_out=None, slot=0,
                           near=None):
@@ -357,7 +384,7 @@ class TensorPartition:
         if rc != _lib.OK:
             table.zero_()  # a call that failed half way may have left entries behind
         _lib.check(rc, "load_balance")
-        self._after_call(dev, slot, int(k), used)
+        self._after_call(flat, int(k), capacity, slot, mode | flags, used)
         return out_idx, out_val, splits, status
 
     def load_balance(self, tensor, thr=None, capacity=None, k=0, mode=None, grow=None):
