@@ -400,8 +400,8 @@ typedef struct zen_encode_merge_args {
      gives the next call's selection its floor (its workgroups do it when they are through with their own
      tensor: no kernel of its own, nothing that waits), in the set of sampling memory this call does not use.
      The next call says so like after zen_load_balance_prepare: ZEN_MODE_PREPARED, with ZEN_MODE_SECOND unless
-     THIS call's mode has ZEN_MODE_SECOND.  zen_encode_merge_samples_next tells whether a call with these sizes
-     does it (the other paths ignore the fields).  next_input must be readable in the order of `stream`.
+     THIS call's mode has ZEN_MODE_SECOND.  zen_encode_merge_samples_next tells whether a call with these sizes,
+     its own k and its mode does it (the other paths ignore the fields).  next_input must be readable in the order of `stream`.
        A next call of another size (gradient buckets differ in length) names its own n, m, capacity and table
      in next_n, next_m, next_capacity and next_table (0 / NULL: this call's); its sizes must take path 2 or 3
      (zen_load_balance_path), or the call is refused with ZEN_EINVAL: only those paths keep sampling memory in

@@ -786,6 +786,42 @@ def test_sample_taken_along_by_the_call_before(zen, oracle, dtype):
     assert e[3].item() == 0 and not tp._ahead_state(ds[0].device, 0)["pending"]
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("n,P", [(1 << 20, 4), (1 << 22, 16)])
+def test_calls_without_a_k_around_calls_that_sample(zen, oracle, n, P, dtype):
+    """encode_merge_flat with k == 0 and a next tensor whose call has a k, and the other way round, on tables that
+    serve as owner tables for the one and hold samples for the other: the oracle's results, every call in one go."""
+    sparse = make_grad(oracle, n, 0.01, dtype, seed=61)
+    full = make_grad(oracle, n, 1.0, dtype, seed=62)
+    k = n // 200
+    cap = n // 64 + 4096
+    top = oracle.load_balance(oracle.mask_dense(full, oracle.kth_key(full, k))[0], P, 1, 3)
+    nonzeros = oracle.load_balance(sparse, P, 1, 3)
+    rng = np.random.default_rng(63)
+    ci, cv = payloads(oracle, rng, n, P, 900, 0.25, dtype)
+    ci = ci.astype(np.int32)
+    want_m = oracle.merge_sparse(ci, cv, n)
+    a, b, di, dv = to_dev(sparse), to_dev(full), to_dev(ci), to_dev(cv)
+    tp = zen.TensorPartition(P, 1, 3)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P), None, None)
+    steps = [(a, 0), (b, k), (a, 0), (a, 0), (b, k), (b, k), (a, 0), (b, k)]
+    outs = []
+    for (t, kk), nxt in zip(steps, steps[1:] + [(None, None)]):
+        outs.append(lba.encode_merge_flat(tp, t, cap, kk, di, dv, n, next_tensor=nxt[0], next_k=nxt[1]))
+    for (t, kk), (e, mg) in zip(steps, outs):
+        idx_o, val_o, splits_o, st_o = top if kk else nonzeros
+        total = int(splits_o.sum())
+        assert st_o == 0 and e[3].item() == 0 and mg[3].item() == 0
+        assert np.array_equal(to_np(e[2]), splits_o)
+        assert np.array_equal(to_np(e[0])[:total], idx_o) and np.array_equal(to_np(e[1])[:total], val_o)
+        cnt = int(mg[2])
+        assert cnt == len(want_m[0]) and np.array_equal(to_np(mg[0])[:cnt], want_m[0].astype(np.int32))
+        assert np.array_equal(to_np(mg[1])[:cnt].view(np.uint32), want_m[1].view(np.uint32))
+    state = tp._ahead_state(a.device, 0)
+    assert state is None or not state["pending"]
+    assert not tp._table(a.device, tp.table_sizes(n)[0]).any()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_workgroups_that_take_the_next_sample_leave_their_first_tiles_to_the_others(zen, dtype):
     """Sizes at which a workgroup has no tile of its own, one, two (as many as it leaves out), three and more, odd

@@ -267,3 +267,22 @@ def test_a_waiting_sample_keeps_the_owner_table_away(L):
     assert take(_lib.MODE_FAST) == (0, 0) and state["pending"] and not dropped
     # the general mode has no other way than through the whole table: what waits there is dropped first
     assert take(_lib.MODE_GENERAL) == (_lib.MODE_NO_SAMPLES, 0) and not state["pending"] and dropped == ["a sample"]
+
+
+def test_only_a_call_that_samples_books_the_next_sample(L):
+    """Whether a call takes its successor's sample along follows from the call's own path: a call through the owner
+    table does not, whatever the successor's k is, and so there is nothing for the successor to pick up."""
+    from zen_repro_amd import _lib
+    from zen_repro_amd.tensor_load_balance import TensorPartition
+
+    n, room = 1 << 22, 1 << 14
+    tp = TensorPartition.__new__(TensorPartition)
+    tp.partitions, tp.memory_scale, tp._samples_next = 4, 1, {}
+    state = {"free": [None, None], "pending": []}
+    tp._ahead_state = lambda dev, slot, create=False: state
+    flat, nxt = torch.zeros(n, dtype=torch.bfloat16), torch.ones(n, dtype=torch.bfloat16)
+    book = lambda k, mode: tp._next_sample(flat, k, nxt, 4096, room, room, 0, mode, 0)[0]
+    for _ in range(2):  # the second time from the cache
+        assert book(0, _lib.MODE_FAST | _lib.MODE_NO_SAMPLES) is None
+        assert book(0, _lib.MODE_FAST).data_ptr() == nxt.data_ptr()
+        assert book(4096, _lib.MODE_FAST).data_ptr() == nxt.data_ptr()

@@ -278,7 +278,7 @@ class LoadBalanceAllreduce:
         thr = None
         if near is not None and k > 0:
             thr, flags = near, flags | _lib.MODE_FLOOR
-        nxt, nxt_table = partition._next_sample(flat, next_tensor, int(next_k), capacity, next_capacity, slot,
+        nxt, nxt_table = partition._next_sample(flat, int(k), next_tensor, int(next_k), capacity, next_capacity, slot,
                                                 mode | flags, used)
         other = nxt is not None and nxt_table is not None
         # what only depends on the call's shape is filled in once; a copy of it takes the rest

@@ -216,7 +216,7 @@ class TensorPartition:
         state["pending"].append((flat.data_ptr(), n, int(k), capacity, ws.data_ptr(), which, _Mark(stream), code,
                                  ws.numel()))
 
-    def _next_sample(self, flat, next_tensor, next_k, capacity, next_capacity, slot, mode, used):
+    def _next_sample(self, flat, k, next_tensor, next_k, capacity, next_capacity, slot, mode, used):
         """(flat view of `next_tensor`, its table or None if it has this call's size) if the call that is about
         to be made can take that tensor's sample along (same type, paths that sample, the other set of sampling
         memory free), else (None, None)."""
@@ -227,18 +227,21 @@ class TensorPartition:
                 or (mode & 0xff) != _lib.MODE_FAST):
             return None, None
         n, n2 = flat.numel(), nxt.numel()
-        key = (n, n2, flat.dtype, capacity, next_capacity, next_k, mode & (0xff | _lib.MODE_SLABS))
+        key = (n, n2, flat.dtype, k, capacity, next_capacity, next_k,
+               mode & (0xff | _lib.MODE_SLABS | _lib.MODE_NO_SAMPLES))
         able = self._samples_next.get(key)
         if able is None:
             L = _lib.lib()
             m, _ = self.table_sizes(n)
             m2, _ = self.table_sizes(n2)
             code = _lib.dtype_code(flat)
-            # this call must be on a path whose pass over the tensor samples, the next one on a path that picks
-            # a sample up from its table
+            # this call (its own k says which path it takes) must be on one whose pass over the tensor samples, the
+            # next one on a path that picks a sample up from its table
+            if len(self._samples_next) >= 256:  # sizes may differ from call to call
+                self._samples_next.clear()
             able = self._samples_next[key] = bool(
-                L.zen_encode_merge_samples_next(n, m, code, capacity, self.partitions, next_k, key[6])
-                and L.zen_load_balance_path(n2, m2, code, next_capacity, self.partitions, next_k, key[6]) in (2, 3))
+                L.zen_encode_merge_samples_next(n, m, code, capacity, self.partitions, k, key[7])
+                and L.zen_load_balance_path(n2, m2, code, next_capacity, self.partitions, next_k, key[7]) in (2, 3))
         if not able:
             return None, None
         state = self._ahead_state(flat.device, slot, create=True)
