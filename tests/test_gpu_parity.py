@@ -759,6 +759,32 @@ def test_decode_ascending_declines_what_is_not_ascending(zen, oracle):
                                      _lib.ptr(ws), ws.numel(), _lib.ptr(status), None) == _lib.EWORKSPACE
 
 
+@pytest.mark.parametrize("form", ["strided indices", "strided values", "two index types", "two value types", "one buffer"])
+def test_decode_ascending_lists_in_any_layout(zen, oracle, form):
+    """Ascending lists that are no plain runs of one type are put into one buffer first and decoded all the same."""
+    rng = np.random.default_rng(72)
+    n = 40000
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    idx, val = ascending_lists(oracle, rng, n, 4, 3000, 0.2, "f32", np.int64)
+    if form == "two value types":  # both types hold the values exactly
+        val = [oracle.bf16_bits_to_f32(oracle.f32_to_bf16_bits(v)) for v in val]
+    d_idx, d_val = [to_dev(i) for i in idx], [to_dev(v) for v in val]
+    want = oracle.decode(np.concatenate(idx), np.concatenate(val), n, "f32acc")
+    strided = lambda t: torch.stack([t, torch.full_like(t, 7)], dim=1)[:, 0]
+    if form == "strided indices":
+        d_idx[2] = strided(d_idx[2])
+    elif form == "strided values":
+        d_val = [strided(v) for v in d_val]
+    elif form == "two index types":
+        d_idx[1] = d_idx[1].int()
+    elif form == "two value types":
+        d_val[3] = d_val[3].bfloat16()
+    else:
+        d_val = torch.cat(d_val)
+    got = lba.decode_sparse_tensors(d_idx, d_val, n, ascending=True)
+    assert got.dtype == torch.float32 and np.array_equal(to_np(got).view(np.uint32), want.view(np.uint32))
+
+
 def test_stack_tensors_views_are_not_copied(zen):
     buf = torch.arange(100, device="cuda", dtype=torch.int32)
     parts = [buf[0:10], buf[10:45], buf[45:100]]

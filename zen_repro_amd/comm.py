@@ -133,20 +133,28 @@ class LoadBalanceAllreduce:
         return dense
 
     def _decode_ascending(self, indices_tensors, values_tensors, dense_size):
-        """decode_sparse_tensors of ascending lists where they are, without putting them into one buffer first;
-        None if that path does not take them (more than 64 lists, or one that is not ascending after all)."""
+        """decode_sparse_tensors of ascending lists where they are; put into one buffer first only if they are no
+        plain runs of one type, with a value list to each index list.  None if that path does not take them (more
+        than 64 lists, or one that is not ascending after all)."""
         lists = indices_tensors if isinstance(indices_tensors, (list, tuple)) else [indices_tensors]
         values = values_tensors if isinstance(values_tensors, (list, tuple)) else [values_tensors]
         count = len(lists)
-        if not 1 <= count <= 64 or len(values) != count:
+        if not 1 <= count <= 64 or not values:
             return None
-        for i, v in zip(lists, values):
-            if i.dtype != lists[0].dtype or v.dtype != values[0].dtype or i.numel() != v.numel():
-                return None
-            _lib.require_gpu(i, "indices")
-            _lib.require_gpu(v, "values")
-        assert lists[0].dtype in (torch.int32, torch.int64)
         dev = values[0].device
+        if len(values) != count or any(
+                i.dtype != lists[0].dtype or v.dtype != values[0].dtype or i.numel() != v.numel()
+                or i.device != dev or v.device != dev or not i.is_contiguous() or not v.is_contiguous()
+                for i, v in zip(lists, values)):
+            sizes = [t.numel() for t in lists]
+            indices = self.stack_tensors(indices_tensors)
+            values = self.stack_tensors(values_tensors)
+            _lib.require_gpu(indices, "indices")
+            if not sum(sizes) == indices.numel() == values.numel() or indices.device != values.device:
+                return None
+            lists, values = torch.split(indices, sizes), torch.split(values, sizes)
+        _lib.require_gpu(values[0], "values")
+        assert lists[0].dtype in (torch.int32, torch.int64)
         L = _lib.lib()
         dense = torch.empty(dense_size, dtype=values[0].dtype, device=dev)
         idx_at = (ctypes.c_void_p * count)(*[t.data_ptr() for t in lists])
