@@ -292,6 +292,24 @@ def test_bitmaps_to_dense_in_one_pass_matches_oracle(zen, oracle, n, P, frac, dt
     assert np.array_equal(to_np(got), _dense_truth(oracle, n, idx, val))
 
 
+@pytest.mark.parametrize("form", ["strided values", "two value types"])
+def test_bitmaps_to_dense_with_values_in_any_layout(zen, oracle, form):
+    """Value lists that are not contiguous, or of two types (the dense tensor then has the one that holds both)."""
+    n, P = 1 << 16, 4
+    mp, idx, val = _shards(oracle, n, P, 0.1, "f32", seed=8)
+    if form == "two value types":  # both types hold the values exactly
+        val = [oracle.bf16_bits_to_f32(oracle.f32_to_bf16_bits(v)) for v in val]
+    bitmaps = [to_dev(oracle.bitmap_encode(mp[p], idx[p])) for p in range(P)]
+    values = [to_dev(v) for v in val]
+    if form == "strided values":
+        values = [torch.stack([v, torch.full_like(v, 7)], dim=1)[:, 0] for v in values]
+    else:
+        values[1] = values[1].bfloat16()
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P, 0), None, None)
+    got = lba.decode_bitmaps_dense(bitmaps, values, n)
+    assert got.dtype == torch.float32 and np.array_equal(to_np(got), _dense_truth(oracle, n, idx, val))
+
+
 def test_bitmaps_to_dense_edge_cases(zen, oracle):
     n, P = 1 << 18, 8
     mp, idx, val = _shards(oracle, n, P, 0.1, "f32", seed=3)

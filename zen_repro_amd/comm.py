@@ -522,7 +522,12 @@ class LoadBalanceAllreduce:
             if t.dtype != torch.uint8:
                 raise RuntimeError("bitmap must be uint8")
         L = _lib.lib()
-        dev = values_tensors[0].device
+        values = list(values_tensors)
+        dev = values[0].device
+        if any(t.dtype != values[0].dtype or t.device != dev or not t.is_contiguous() for t in values):
+            # lists that are no plain runs of one type: in one buffer, of the type that holds them all
+            values = torch.split(self.stack_tensors(values), [t.numel() for t in values])
+        _lib.require_gpu(values[0], "values")
         cached = self._dense_dicts.get(numel)
         if cached is None:
             nbytes = L.zen_bitmap_dense_dict_bytes(numel, self.partitions)
@@ -532,11 +537,6 @@ class LoadBalanceAllreduce:
             _lib.check(L.zen_bitmap_dense_dict(numel, self.partitions, _lib.ptr(cached), None, _lib.stream_of(dev)),
                        "decode_bitmaps_dense")
             self._dense_dicts[numel] = cached
-        values = list(values_tensors)
-        for t in values:
-            _lib.require_gpu(t, "values")
-            if t.dtype != values[0].dtype:
-                raise RuntimeError("values must have one type")
         P = self.partitions
         bm_at = (ctypes.c_void_p * P)(*[t.data_ptr() for t in bitmap_indices])
         bm_bytes = (ctypes.c_int64 * P)(*[t.numel() for t in bitmap_indices])
