@@ -960,6 +960,30 @@ def test_load_balance_through_the_owner_table(zen, oracle, n, P, density, scale,
     assert not tp._table(d.device, m).any()
 
 
+@pytest.mark.parametrize("words", [1, 1023, 1024, (1 << 16) - 1, 1 << 16, (1 << 19) + 1])
+def test_read_back_of_any_length(zen, words):
+    """Both types, a word and a list of `words` of them, up to and past what goes through the pinned buffer."""
+    from zen_repro_amd import _lib
+
+    wide = torch.arange(words, dtype=torch.int64, device="cuda") * (1 << 33) - 5
+    narrow = torch.tensor([-7], dtype=torch.int32, device="cuda")
+    assert list(_lib.read_back(wide, narrow)) == wide.tolist() + [-7]
+    assert list(_lib.read_back(narrow, wide.int(), narrow)) == [-7] + wide.int().tolist() + [-7]
+
+
+def test_table_lists_of_very_many_partitions(zen, oracle):
+    """get_sub_sparse_tensors with 2^19 partitions of eight slots."""
+    P = 1 << 19
+    rng = np.random.default_rng(81)
+    g_np = rng.standard_normal(8 * P).astype(np.float32)
+    memory = np.where(rng.random(8 * P) < 0.2, rng.integers(1, 8 * P, 8 * P), 0).astype(np.int32)
+    tp = zen.TensorPartition(P, 1, 3)
+    indices, values, splits = tp.get_sub_sparse_tensors(to_dev(g_np), to_dev(memory))
+    assert np.array_equal(to_np(splits), (memory.reshape(P, 8) != 0).sum(axis=1))
+    assert len(indices) == P and np.array_equal(to_np(torch.cat(indices)), memory[memory != 0])
+    assert np.array_equal(to_np(torch.cat(values)), g_np[memory[memory != 0]])
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("r,n", [(1, 5000), (1023, 5000), (4096, 5000), (4096, 1 << 30), (4097, 20000), (30000, 40000), (9000, 16385)])
 @pytest.mark.parametrize("copies", [1, 16, 0])

@@ -286,3 +286,11 @@ def test_only_a_call_that_samples_books_the_next_sample(L):
         assert book(0, _lib.MODE_FAST | _lib.MODE_NO_SAMPLES) is None
         assert book(0, _lib.MODE_FAST).data_ptr() == nxt.data_ptr()
         assert book(4096, _lib.MODE_FAST).data_ptr() == nxt.data_ptr()
+
+
+def test_read_back_of_more_words_than_the_pinned_buffer_holds():
+    """Split sizes of hundreds of thousands of partitions come back as plain copies."""
+    from zen_repro_amd import _lib
+
+    splits, status = torch.arange(1 << 20, dtype=torch.int64), torch.full((1,), 8, dtype=torch.int32)
+    assert _lib.read_back(splits, status) == list(range(1 << 20)) + [8]

@@ -336,6 +336,9 @@ class _HostWords:
 
 _host = threading.local()
 _NO_SEGMENT = [(None, 0, 0) * (3 - n) for n in range(4)]
+# Longer lists (split sizes of very many partitions) come as plain copies: one workgroup stores the words, and a
+# thread's pinned memory stays below a megabyte.
+_READ_BACK_MOST = 1 << 16
 
 
 def read_back(*tensors):
@@ -348,13 +351,15 @@ def read_back(*tensors):
         count = t.numel()
         n += count
         args += (t.data_ptr(), count, 1 if t.dtype is torch.int64 else 0)
+    if n > _READ_BACK_MOST:
+        return [word for t in tensors for word in t.tolist()]
     args += _NO_SEGMENT[len(tensors)]
     try:
         words = _host.words
     except AttributeError:
         words = None
     if words is None or words.words <= n:
-        words = _host.words = _HostWords(max(1024, 2 * n))
+        words = _host.words = _HostWords(max(1024, min(2 * n, _READ_BACK_MOST + 1)))
     rc = _lib.zen_read_back(*args, words.ptr, words.words, stream_handle(tensors[0].device))
     if rc:
         check(rc, "read_back")
