@@ -294,3 +294,40 @@ def test_read_back_of_more_words_than_the_pinned_buffer_holds():
 
     splits, status = torch.arange(1 << 20, dtype=torch.int64), torch.full((1,), 8, dtype=torch.int32)
     assert _lib.read_back(splits, status) == list(range(1 << 20)) + [8]
+
+
+@pytest.mark.parametrize("capturing", [False, True])
+def test_a_hook_without_a_stream_keeps_its_calls_in_order(monkeypatch, capturing):
+    """The calls of one hook share workspaces: one that finds another current stream than the last waits for that
+    one's; calls that stay on a stream wait for nothing."""
+    import zen_repro_amd as zen
+    from zen_repro_amd.hook import SparseCommHook
+
+    class Stream:
+        def __init__(self):
+            self.waited = []
+
+        def wait_stream(self, other):
+            self.waited.append(other)
+
+    a, b = Stream(), Stream()
+    now = [a]
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: now[0])
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+
+    class Bucket:
+        def buffer(self):
+            return torch.zeros(8)
+
+    class Lba:
+        process_group = zen.LocalGroup(1)
+
+    ran_on = []
+    hook = SparseCommHook(Lba(), 1, 2, zen.LocalGroup(1))
+    hook._reduce = lambda tensors, exchange: ran_on.append((now[0], list(now[0].waited))) or tensors
+    hook(None, Bucket())  # passes the first bucket through
+    for stream in (a, a, b, b, a):
+        now[0] = stream
+        hook(None, Bucket())
+    waits = [[], [], [a], [a], [b]] if not capturing else [[]] * 5
+    assert ran_on == list(zip((a, a, b, b, a), waits))

@@ -16,7 +16,11 @@ hook returns (whatever consumes the future's tensor in that stream's order
 finds it complete).  Neither wait blocks the host.  Between those two waits
 nothing of the caller's can run beside the path anyway, and each costs the host
 some 14 us: without a named stream the path runs on the caller's current stream
-and there is nothing to wait for."""
+and there is nothing to wait for, unless that is another stream than the last
+call's.  The calls of a hook share their workspaces, so this one then waits for
+that one's, as it would on a stream of the hook's own (not while the stream is
+being captured into a graph, where what came before the capture has to have
+finished anyway)."""
 import torch
 
 from ._lib import annotate
@@ -77,6 +81,8 @@ class SparseCommHook:
                                "load_balance_allreduce.ddp")
         caller = torch.cuda.current_stream(tensors.device)
         if not self.own_stream:
+            if caller != self.stream and not torch.cuda.is_current_stream_capturing():
+                caller.wait_stream(self.stream)
             self.stream = caller
             future.set_result(self._reduce(tensors, exchange))
             return future
