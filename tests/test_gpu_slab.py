@@ -564,6 +564,34 @@ def test_calls_that_take_no_sample_leave_a_waiting_one_alone(zen, oracle, n, P, 
     assert int(tp._table(b.device, tp.table_sizes(n)[0]).count_nonzero()) == 0
 
 
+def test_a_table_made_on_another_stream_is_waited_for(zen, oracle):
+    """The first prepare of a size makes the table on its own stream, behind whatever that one is busy with; calls of
+    other buckets on the current stream, which have no sample to wait for, find it filled all the same."""
+    n, P = 1 << 22, 16
+    a_np = make_grad(oracle, n, 0.01, "bf16", seed=65)
+    b_np = make_grad(oracle, n, 1.0, "bf16", seed=66)
+    k = n // 200
+    cap, room = k + k // 4 + 4096, n // 64 + 4096
+    top = oracle.load_balance(oracle.mask_dense(b_np, oracle.kth_key(b_np, k))[0], P, 1, 3)
+    nonzeros = oracle.load_balance(a_np, P, 1, 3)
+    a, b, c = to_dev(a_np), to_dev(b_np), to_dev(b_np)
+    busy = torch.ones(2048, 2048, device="cuda")
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    tp = zen.TensorPartition(P, 1, 3)
+    with torch.cuda.stream(side):
+        for _ in range(20):
+            busy = busy @ busy * 1e-4
+        tp.prepare(b, k, cap)
+    outs = [(tp.load_balance_flat(a, None, room), nonzeros), (tp.load_balance_flat(c, None, cap, k=k), top),
+            (tp.load_balance_flat(b, None, cap, k=k), top)]
+    for (idx, val, splits, st), (idx_o, val_o, splits_o, st_o) in outs:
+        assert int(st.item()) == 0 and st_o == 0
+        total = int(splits.sum())
+        assert np.array_equal(splits.cpu().numpy(), splits_o)
+        assert np.array_equal(idx[:total].cpu().numpy(), idx_o) and np.array_equal(to_np(val[:total]), val_o)
+
+
 def test_step_replayed_from_a_captured_graph(zen, oracle):
     """An encode (fused top-k) and a merge captured into a HIP graph, the merge forked onto a second stream:
     every replay, with eager calls on the same workspaces and a synchronisation in between, leaves the bytes

@@ -331,3 +331,31 @@ def test_a_hook_without_a_stream_keeps_its_calls_in_order(monkeypatch, capturing
         hook(None, Bucket())
     waits = [[], [], [a], [a], [b]] if not capturing else [[]] * 5
     assert ran_on == list(zip((a, a, b, b, a), waits))
+
+
+@pytest.mark.parametrize("capturing", [False, True])
+def test_a_kept_buffer_is_waited_for_and_held_by_every_stream(monkeypatch, capturing):
+    """A stream's first use of a buffer made on another one waits for its making and is remembered by the
+    allocator; uses on the maker's stream, and second uses, do neither."""
+    from zen_repro_amd import _lib
+
+    log = []
+
+    class Stream:
+        def __init__(self, handle):
+            self.cuda_stream = handle
+
+        def wait_stream(self, other):
+            log.append(("wait", self.cuda_stream, other.cuda_stream))
+
+    class Buffer:
+        def record_stream(self, stream):
+            log.append(("hold", stream.cuda_stream))
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    streams = {h: Stream(h) for h in (1, 2, 3)}
+    buf = Buffer()
+    kept = _lib.Kept(buf, streams[1])
+    for h in (1, 2, 1, 2, 3):
+        assert kept.on(h, lambda: streams[h]) is buf
+    assert log == ([] if capturing else [("wait", 2, 1), ("hold", 2), ("wait", 3, 1), ("hold", 3)])

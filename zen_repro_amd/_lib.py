@@ -209,6 +209,29 @@ def untransformed(*tensors):
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
+class Kept:
+    """A buffer that is kept from call to call, and the streams it is used on.  A stream other than the one it
+    was made on waits for its making (its fill) at its first use there, and the memory is not handed out again
+    before the work of every such stream is done.  Neither while a stream is being captured into a graph: what
+    came before the capture has finished, and whoever replays the graph keeps the buffer."""
+
+    __slots__ = ("buf", "maker", "seen")
+
+    def __init__(self, buf, maker):
+        self.buf = buf
+        self.maker = maker
+        self.seen = {maker.cuda_stream}
+
+    def on(self, handle, stream):
+        """The buffer, for use on the stream `handle` (`stream`: a function that gives it as a torch stream)."""
+        if handle not in self.seen and not torch.cuda.is_current_stream_capturing():
+            stream = stream()
+            stream.wait_stream(self.maker)
+            self.buf.record_stream(stream)
+            self.seen.add(handle)
+        return self.buf
+
+
 class Scratch:
     """Cache of raw byte buffers per device and host thread, grown on demand
     and reused.  A buffer is tied to the stream order of its users, like any
@@ -226,17 +249,19 @@ class Scratch:
         return bufs
 
     def get(self, device, name, nbytes, zero=False):
-        key = (device_index(device), name)
+        index = device_index(device)
+        key = (index, name)
         try:
             bufs = self._local.bufs
         except AttributeError:
             bufs = self._bufs()
-        buf = bufs.get(key)
-        if buf is None or buf.numel() < nbytes:
+        kept = bufs.get(key)
+        if kept is None or kept.buf.numel() < nbytes:
             alloc = torch.zeros if zero else torch.empty
             buf = alloc(max(int(nbytes), 256), dtype=torch.uint8, device=device)
-            bufs[key] = buf
-        return buf
+            bufs[key] = Kept(buf, torch.cuda.current_stream(index))
+            return buf
+        return kept.on(stream_handle(device), lambda: torch.cuda.current_stream(index))
 
     def drop(self):
         """Forget the calling thread's buffers."""

@@ -135,13 +135,13 @@ class TensorPartition:
         bucket, train.py:167-185), so a handful of tables is kept, least
         recently used first out."""
         key = (device if isinstance(device, torch.device) else torch.device(device), m, slot)
-        t = self._tables.pop(key, None)
-        if t is None:
+        kept = self._tables.pop(key, None)
+        if kept is None:
             while len(self._tables) >= self._MAX_TABLES:
                 self._tables.pop(next(iter(self._tables)))
-            t = torch.zeros(m, dtype=torch.int32, device=device)
-        self._tables[key] = t  # most recently used last
-        return t
+            kept = _lib.Kept(torch.zeros(m, dtype=torch.int32, device=device), torch.cuda.current_stream(device))
+        self._tables[key] = kept  # most recently used last
+        return kept.on(_lib.stream_handle(device), lambda: torch.cuda.current_stream(device))
 
     def _honest_capacity(self, flat, thr, k):
         """Room for the selection without guessing `numel` (which would take a
