@@ -592,6 +592,43 @@ def test_a_table_made_on_another_stream_is_waited_for(zen, oracle):
         assert np.array_equal(idx[:total].cpu().numpy(), idx_o) and np.array_equal(to_np(val[:total]), val_o)
 
 
+def test_merge_on_a_stream_that_runs_ahead(zen, oracle):
+    """With the merge on a stream of its own and the current stream busy with something long, the merge comes before
+    everything that the current stream still has to do: its count, status and workspace have to be zero by then, on
+    the first call, whose blocks and workspaces are new, and on later ones with larger workspaces and new blocks."""
+    from zen_repro_amd import _lib
+
+    n, P = 1 << 22, 16
+    a_np = make_grad(oracle, n, 0.01, "bf16", seed=67)
+    cap = n // 64 + 4096
+    want_e = oracle.load_balance(a_np, P, 1, 3)
+    rng = np.random.default_rng(68)
+    a = to_dev(a_np)
+    busy = torch.ones(2048, 2048, device="cuda")
+    side = torch.cuda.Stream()
+    tp = zen.TensorPartition(P, 1, 3)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P), None, None)
+    for per_peer in (3000, 9000, 9000):
+        ci, cv = payloads(oracle, rng, n, P, per_peer, 0.25, "bf16")
+        ci = ci.astype(np.int32)
+        di, dv = to_dev(ci), to_dev(cv)
+        want_i, want_v = oracle.merge_sparse(ci, cv, n)
+        torch.cuda.synchronize()
+        _lib.zeros.fresh(a.device)
+        with torch.cuda.stream(side):
+            _lib.zeros.fresh(a.device)
+        for _ in range(20):
+            busy = busy @ busy * 1e-4
+        (idx, val, splits, st), (m_idx, m_val, count, m_st) = lba.encode_merge_flat(tp, a, cap, 0, di, dv, n,
+                                                                                   merge_stream=side)
+        torch.cuda.current_stream().wait_stream(side)
+        assert int(st.item()) == 0 and int(m_st.item()) == 0 and int(count) == len(want_i)
+        assert np.array_equal(to_np(m_idx)[:len(want_i)], want_i.astype(np.int32))
+        assert np.array_equal(to_np(m_val)[:len(want_i)].view(np.uint32), want_v.view(np.uint32))
+        total = int(splits.sum())
+        assert np.array_equal(to_np(splits), want_e[2]) and np.array_equal(to_np(idx)[:total], want_e[0])
+
+
 def test_step_replayed_from_a_captured_graph(zen, oracle):
     """An encode (fused top-k) and a merge captured into a HIP graph, the merge forked onto a second stream:
     every replay, with eager calls on the same workspaces and a synchronisation in between, leaves the bytes

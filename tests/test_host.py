@@ -305,6 +305,7 @@ def test_a_hook_without_a_stream_keeps_its_calls_in_order(monkeypatch, capturing
 
     class Stream:
         def __init__(self):
+            self.cuda_stream = id(self)
             self.waited = []
 
         def wait_stream(self, other):
@@ -349,13 +350,21 @@ def test_a_kept_buffer_is_waited_for_and_held_by_every_stream(monkeypatch, captu
             log.append(("wait", self.cuda_stream, other.cuda_stream))
 
     class Buffer:
+        def numel(self):
+            return 256
+
         def record_stream(self, stream):
             log.append(("hold", stream.cuda_stream))
 
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
     streams = {h: Stream(h) for h in (1, 2, 3)}
     buf = Buffer()
-    kept = _lib.Kept(buf, streams[1])
-    for h in (1, 2, 1, 2, 3):
-        assert kept.on(h, lambda: streams[h]) is buf
+    now = [1]
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: streams[now[0]])
+    monkeypatch.setattr(_lib, "current_handle", lambda index: now[0])
+    scratch = _lib.Scratch()
+    scratch._bufs()[0, "a"] = _lib.Kept(buf, streams[1])
+    for now[0] in (1, 2, 1, 2):
+        assert scratch.get(torch.device("cuda", 0), "a", 1) is buf
+    assert scratch.get(torch.device("cuda", 0), "a", 1, stream=streams[3]) is buf
     assert log == ([] if capturing else [("wait", 2, 1), ("hold", 2), ("wait", 3, 1), ("hold", 3)])

@@ -175,15 +175,14 @@ def device_index(device):
     return index if index is not None else torch.cuda.current_device()
 
 
-_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+# The current stream of the device of that index as an integer handle (hipStream_t).  Asked on every call of the hot
+# path: torch's own shortcut, where it has one, is several microseconds quicker than a Stream object.
+current_handle = getattr(torch._C, "_cuda_getCurrentRawStream",
+                         lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def stream_handle(device):
-    """The current stream of `device` as an integer handle (hipStream_t).  Asked on every call of the hot
-    path: torch's own shortcut, where it has one, is several microseconds quicker than a Stream object."""
-    if _raw_stream is not None:
-        return _raw_stream(device_index(device))
-    return torch.cuda.current_stream(device).cuda_stream
+    return current_handle(device_index(device))
 
 
 def stream_of(device):
@@ -222,14 +221,13 @@ class Kept:
         self.maker = maker
         self.seen = {maker.cuda_stream}
 
-    def on(self, handle, stream):
-        """The buffer, for use on the stream `handle` (`stream`: a function that gives it as a torch stream)."""
-        if handle not in self.seen and not torch.cuda.is_current_stream_capturing():
-            stream = stream()
+    def join(self, stream, new=False):
+        """A stream that is not in `seen` comes to use the buffer (`new`: which has just been made, in the same
+        capture if there is one)."""
+        if new or not torch.cuda.is_current_stream_capturing():
             stream.wait_stream(self.maker)
             self.buf.record_stream(stream)
-            self.seen.add(handle)
-        return self.buf
+            self.seen.add(stream.cuda_stream)
 
 
 class Scratch:
@@ -248,7 +246,9 @@ class Scratch:
             bufs = self._local.bufs = {}
         return bufs
 
-    def get(self, device, name, nbytes, zero=False):
+    def get(self, device, name, nbytes, zero=False, stream=None):
+        """The buffer `name` of at least `nbytes` bytes (zeroed when it is made if `zero`), for use on `stream`
+        (None: the current one)."""
         index = device_index(device)
         key = (index, name)
         try:
@@ -259,9 +259,12 @@ class Scratch:
         if kept is None or kept.buf.numel() < nbytes:
             alloc = torch.zeros if zero else torch.empty
             buf = alloc(max(int(nbytes), 256), dtype=torch.uint8, device=device)
-            bufs[key] = Kept(buf, torch.cuda.current_stream(index))
-            return buf
-        return kept.on(stream_handle(device), lambda: torch.cuda.current_stream(index))
+            kept = bufs[key] = Kept(buf, torch.cuda.current_stream(index))
+            if stream is not None and stream.cuda_stream not in kept.seen:
+                kept.join(stream, new=True)
+        elif (stream.cuda_stream if stream is not None else current_handle(index)) not in kept.seen:
+            kept.join(torch.cuda.current_stream(index) if stream is None else stream)
+        return kept.buf
 
     def drop(self):
         """Forget the calling thread's buffers."""
@@ -306,19 +309,28 @@ class ZeroPool:
         entry[1] = at + 1
         return entry[0][at:at + 1]
 
-    def take(self, device, count, dtype):
+    def take(self, device, count, dtype, stream=None):
+        """`count` zeros of `dtype`.  `stream`: a stream beside the current one that uses them too, and may be far
+        ahead of it: it waits for the fill of every block, once."""
         size = self._SIZES.get(dtype)
         if size is None:
             size = torch.empty((), dtype=dtype).element_size()
         nbytes = count * size
         if nbytes > self.BLOCK // 4:
-            return torch.zeros(count, dtype=dtype, device=device)
+            piece = torch.zeros(count, dtype=dtype, device=device)
+            if stream is not None:
+                stream.wait_stream(torch.cuda.current_stream(device))
+            return piece
         blocks = self._blocks()
         key = (device_index(device), stream_handle(device))
         entry = blocks.get(key)
         if entry is None or entry[1] + nbytes > self.BLOCK:
-            # the block, how much of it is handed out, and views of it by element type (made when first asked for)
-            entry = blocks[key] = [torch.zeros(self.BLOCK, dtype=torch.uint8, device=device), 0, {}]
+            # the block, how much of it is handed out, views of it by element type (made when first asked for), and
+            # the streams its fill lies before
+            entry = blocks[key] = [torch.zeros(self.BLOCK, dtype=torch.uint8, device=device), 0, {}, {key[1]}]
+        if stream is not None and stream.cuda_stream not in entry[3]:
+            stream.wait_stream(torch.cuda.current_stream(device))
+            entry[3].add(stream.cuda_stream)
         at = entry[1]
         entry[1] = (at + nbytes + self.ALIGN - 1) // self.ALIGN * self.ALIGN
         typed = entry[2].get(dtype)

@@ -142,10 +142,8 @@ class LoadBalanceAllreduce:
         if not 1 <= count <= 64 or not values:
             return None
         dev = values[0].device
-        if len(values) != count or any(
-                i.dtype != lists[0].dtype or v.dtype != values[0].dtype or i.numel() != v.numel()
-                or i.device != dev or v.device != dev or not i.is_contiguous() or not v.is_contiguous()
-                for i, v in zip(lists, values)):
+        if len(values) != count or not _plain_runs(lists) or not _plain_runs(values) or any(
+                i.numel() != v.numel() or i.get_device() != v.get_device() for i, v in zip(lists, values)):
             sizes = [t.numel() for t in lists]
             indices = self.stack_tensors(indices_tensors)
             values = self.stack_tensors(values_tensors)
@@ -232,7 +230,9 @@ class LoadBalanceAllreduce:
         k=k, slot=slot, thr_out=thr_out, near=near) of the rank's own gradient and merge_sparse_flat(recv_indices,
         recv_values, dense_size, slot=slot) of the entries it received, whose values have the gradient's type.
         Returns the two calls' tuples.  Everything is enqueued on the current stream unless `merge_stream` (a
-        torch stream in whose order the received entries are ready) takes the merge.  A sample taken ahead with
+        torch stream in whose order the received entries are ready) takes the merge; the results' memory comes from
+        the current stream's pool, so a caller that has dropped results makes `merge_stream` wait for the current
+        stream before the next call.  A sample taken ahead with
         partition.prepare() is picked up as load_balance_flat would.  `next_tensor` (ready in the current stream's
         order) is the gradient of the call that follows on this slot, `next_k` its k (default: this call's): if
         it has this tensor's type, the pass over this tensor takes the sample of that call along (no kernel of
@@ -263,7 +263,8 @@ class LoadBalanceAllreduce:
         out_val = torch.empty(capacity, dtype=flat.dtype, device=dev)
         m_idx = torch.empty(r, dtype=torch.int32, device=dev)
         m_val = torch.empty(r, dtype=torch.float32, device=dev)
-        small = _lib.zeros.take(dev, P + 2, torch.int64)  # split sizes, merged count, the two status words
+        # split sizes, merged count, the two status words
+        small = _lib.zeros.take(dev, P + 2, torch.int64, merge_stream)
         splits, count, status2 = small.split((P, 1, 1))
         status, m_status = status2.view(torch.int32).split(1)
         if next_k is None:
@@ -280,7 +281,7 @@ class LoadBalanceAllreduce:
                     n2, partition.table_sizes(n2)[0], code, next_capacity, P)
             ws_bytes = max(ws_bytes, bytes2)
         ws = _lib.scratch.get(dev, f"load_balance/{slot}", ws_bytes)
-        mws = _lib.scratch.get(dev, f"merge/{slot}", mws_bytes, zero=True)
+        mws = _lib.scratch.get(dev, f"merge/{slot}", mws_bytes, zero=True, stream=merge_stream)
         table = partition._table(dev, m, slot)
         flags, used = partition._take_ahead(flat, n, int(k), capacity, ws, slot, mode, None, near)
         thr = None
@@ -524,7 +525,7 @@ class LoadBalanceAllreduce:
         L = _lib.lib()
         values = list(values_tensors)
         dev = values[0].device
-        if any(t.dtype != values[0].dtype or t.device != dev or not t.is_contiguous() for t in values):
+        if not _plain_runs(values):
             # lists that are no plain runs of one type: in one buffer, of the type that holds them all
             values = torch.split(self.stack_tensors(values), [t.numel() for t in values])
         _lib.require_gpu(values[0], "values")
@@ -630,6 +631,15 @@ class LoadBalanceAllreduce:
             values_tensors = ddp.allgather_padding(sparse_values)
         with ann("decode_sparse_tensors"):
             return self.decode_sparse_tensors(indices_tensors, values_tensors, numel, ascending=True)
+
+
+def _plain_runs(tensors):
+    """Whether the tensors are contiguous, of one type and on one device: what a kernel takes by their addresses."""
+    dtype, at = tensors[0].dtype, tensors[0].get_device()
+    for t in tensors:
+        if t.dtype is not dtype or t.get_device() != at or not t.is_contiguous():
+            return False
+    return True
 
 
 def _as_one_buffer(tensors):

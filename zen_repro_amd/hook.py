@@ -81,7 +81,7 @@ class SparseCommHook:
                                "load_balance_allreduce.ddp")
         caller = torch.cuda.current_stream(tensors.device)
         if not self.own_stream:
-            if caller != self.stream and not torch.cuda.is_current_stream_capturing():
+            if caller.cuda_stream != self.stream.cuda_stream and not torch.cuda.is_current_stream_capturing():
                 caller.wait_stream(self.stream)
             self.stream = caller
             future.set_result(self._reduce(tensors, exchange))

@@ -141,7 +141,9 @@ class TensorPartition:
                 self._tables.pop(next(iter(self._tables)))
             kept = _lib.Kept(torch.zeros(m, dtype=torch.int32, device=device), torch.cuda.current_stream(device))
         self._tables[key] = kept  # most recently used last
-        return kept.on(_lib.stream_handle(device), lambda: torch.cuda.current_stream(device))
+        if _lib.stream_handle(device) not in kept.seen:
+            kept.join(torch.cuda.current_stream(device))
+        return kept.buf
 
     def _honest_capacity(self, flat, thr, k):
         """Room for the selection without guessing `numel` (which would take a
