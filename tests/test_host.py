@@ -368,3 +368,23 @@ def test_a_kept_buffer_is_waited_for_and_held_by_every_stream(monkeypatch, captu
         assert scratch.get(torch.device("cuda", 0), "a", 1) is buf
     assert scratch.get(torch.device("cuda", 0), "a", 1, stream=streams[3]) is buf
     assert log == ([] if capturing else [("wait", 2, 1), ("hold", 2), ("wait", 3, 1), ("hold", 3)])
+
+
+def test_compaction_kernels_keep_their_rows_in_registers(tmp_path):
+    """The rows a wave has in flight are the kernels' speed: none of their registers may end up in memory, for
+    aligned tensors and for views that begin at an odd element."""
+    import shutil
+    import subprocess
+
+    csrc = os.path.join(ROOT, "zen_repro_amd", "csrc")
+    plan = subprocess.run(["make", "-C", csrc, "-n", "-B", "--no-print-directory", "zen_compact.o"],
+                          capture_output=True, text=True, check=True).stdout
+    command = plan.strip().splitlines()[-1].split()
+    if not shutil.which(command[0]):
+        pytest.skip("no compiler")
+    out = str(tmp_path / "zen_compact.s")
+    command = command[:command.index("-c")] + ["--cuda-device-only", "-S", "zen_compact.hip", "-o", out]
+    subprocess.run(command, cwd=csrc, check=True, stderr=subprocess.DEVNULL)
+    spills = re.findall(r"\.name:\s+(\S+).*?\.vgpr_spill_count:\s+(\d+)", open(out).read(), flags=re.S)
+    walks = [int(n) for name, n in spills if "k_compact" in name]
+    assert len(walks) >= 12 and not any(walks)
