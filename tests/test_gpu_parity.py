@@ -971,6 +971,27 @@ def test_read_back_of_any_length(zen, words):
     assert list(_lib.read_back(narrow, wide.int(), narrow)) == [-7] + wide.int().tolist() + [-7]
 
 
+def test_read_back_leaves_the_core_to_others_in_a_long_wait(zen):
+    """Behind tens of milliseconds of work the waiting thread sleeps nearly all the time, and what comes back is what
+    the stream's work left."""
+    import time
+
+    from zen_repro_amd import _lib
+
+    x = torch.ones(8192, 8192, device="cuda")
+    word = torch.zeros(1, dtype=torch.int64, device="cuda")
+    _lib.read_back(word)
+    y = x @ x
+    torch.cuda.synchronize()
+    for _ in range(6):
+        y = x @ x
+    word += 5
+    wall, core = time.perf_counter(), time.thread_time()
+    assert list(_lib.read_back(word)) == [5]
+    wall, core = time.perf_counter() - wall, time.thread_time() - core
+    assert core < max(0.5 * wall, 0.004)  # a millisecond is watched through
+
+
 def test_table_lists_of_very_many_partitions(zen, oracle):
     """get_sub_sparse_tensors with 2^19 partitions of eight slots."""
     P = 1 << 19

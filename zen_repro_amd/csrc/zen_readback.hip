@@ -9,6 +9,9 @@
 // unknown density went from 242 to 178 us, before the counting kernel had 256 workgroups.
 #include <immintrin.h>  // host pass: _mm_pause
 
+#include <chrono>
+#include <thread>
+
 #include "zen_select.h"
 
 namespace zen {
@@ -19,6 +22,8 @@ struct ReadBack {
   int32_t count[ZEN_READ_BACK_SEGMENTS];
   int32_t wide[ZEN_READ_BACK_SEGMENTS];  // 64-bit words (else 32)
 };
+
+constexpr std::chrono::nanoseconds kSpin(1000000), kNap(1000000);
 
 __global__ void k_read_back(ReadBack r, int64_t *host, int64_t ticket) {
   int at = 1;
@@ -119,19 +124,27 @@ int zen_read_back(const void *p0, int n0, int wide0, const void *p1, int n1, int
   k_read_back<<<dim3(1), dim3(64), 0, s>>>(r, host, ticket);
   ZEN_LAUNCH_CHECK("k_read_back");
   const int64_t *flag = host;
-  // the stream is asked now and then: it says when something on it has failed, and its end is the end of the wait
+  // The waits of a call are short: this core watches for the answer.  A longer one is for what the stream has to wait
+  // for itself (an exchange, other ranks): then the core is left to others, for a sixteenth of the time waited so far
+  // and a millisecond at most, and the stream is asked every time, which says when something on it has failed.  (The
+  // runtime's own waits keep the core busy from beginning to end, hipEventBlockingSync or not.)
+  using clock = std::chrono::steady_clock;
+  const auto begin = clock::now();
   for (uint32_t spins = 1;; ++spins) {
     if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == ticket) return ZEN_OK;
     _mm_pause();
-    if ((spins & 0xfffffu) == 0) {
-      const hipError_t e = hipStreamQuery(s);
-      if (e == hipErrorNotReady) continue;
-      ZEN_HIP_CHECK(e);
-      ZEN_HIP_CHECK(hipStreamSynchronize(s));
-      return __atomic_load_n(flag, __ATOMIC_ACQUIRE) == ticket
-                 ? ZEN_OK
-                 : fail(ZEN_EHIP, "zen_read_back: the stream ended without an answer");
-    }
+    if ((spins & 63u) == 0 && clock::now() - begin > kSpin) break;
+  }
+  for (;;) {
+    const auto nap = (clock::now() - begin) / 16;
+    std::this_thread::sleep_for(nap < kNap ? nap : kNap);
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == ticket) return ZEN_OK;
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady) continue;
+    ZEN_HIP_CHECK(e);
+    return __atomic_load_n(flag, __ATOMIC_ACQUIRE) == ticket
+               ? ZEN_OK
+               : fail(ZEN_EHIP, "zen_read_back: the stream ended without an answer");
   }
 }
 
