@@ -629,6 +629,20 @@ def test_merge_on_a_stream_that_runs_ahead(zen, oracle):
         assert np.array_equal(to_np(splits), want_e[2]) and np.array_equal(to_np(idx)[:total], want_e[0])
 
 
+def test_sizes_kept_by_shape_are_bounded(zen, monkeypatch):
+    """Steps that receive another number of entries each time: what is kept by the shape of a step stays small."""
+    n, P = 1 << 20, 4
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P), None, None)
+    monkeypatch.setattr(lba, "_MOST_SHAPES", 8)
+    grad = torch.zeros(n, device="cuda")
+    grad[5::100] = 1.0
+    for r in range(1, 30):
+        idx = torch.arange(1, r + 1, dtype=torch.int32, device="cuda")
+        e, (_, _, count, status) = lba.encode_merge_flat(lba.tensor_partition, grad, n // 64, 0, idx, idx.float(), n)
+        assert int(count) == r and not int(status) and int(e[2].sum()) == grad[5::100].numel()
+        assert len(lba._step_sizes) <= 8
+
+
 def test_step_replayed_from_a_captured_graph(zen, oracle):
     """An encode (fused top-k) and a merge captured into a HIP graph, the merge forked onto a second stream:
     every replay, with eager calls on the same workspaces and a synchronisation in between, leaves the bytes

@@ -79,6 +79,8 @@ class LoadBalanceAllreduce:
         self._bitmap_ranks = {}  # numel -> (mapping list of this rank, its rank table)
         self._dense_dicts = {}   # numel -> dictionary of decode_bitmaps_dense
 
+    _MOST_SHAPES = 1024
+
     def get_tensor_partition_obj(self, memory_scale, rehash):
         return TensorPartition(partitions=self.partitions, memory_scale=memory_scale, rehash=rehash)
 
@@ -254,6 +256,8 @@ class LoadBalanceAllreduce:
         shape = (n, code, capacity, P, partition.memory_scale, r, dense_size)
         sizes = self._step_sizes.get(shape)
         if sizes is None:
+            if len(self._step_sizes) >= self._MOST_SHAPES:  # the number received may differ from call to call
+                self._step_sizes.clear()
             m = partition.table_sizes(n)[0]
             sizes = self._step_sizes[shape] = (m, L.zen_load_balance_workspace(n, m, code, capacity, P),
                                                L.zen_merge_workspace(r, dense_size), None)
