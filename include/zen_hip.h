@@ -2,7 +2,9 @@
  * libzen_hip: MI355X (gfx950) implementation of ZEN's sparse-gradient
  * select / hash-partition / merge path.  Plain C ABI: device pointers, sizes
  * and a HIP stream.  No torch types, no hidden allocation, no host
- * synchronisation: every call only enqueues kernels on `stream`.
+ * synchronisation: every call only enqueues kernels on `stream`, but for
+ * zen_host_words_alloc / _free and zen_read_back, which exist to wait,
+ * zen_bitmap_dense_dict with `members`, and zen_profile_read.
  *
  * Conventions
  *   - every pointer is DEVICE memory unless a comment says "host";
@@ -188,9 +190,9 @@ int zen_topk_threshold(const void *input, int dtype, int64_t n, int64_t k,
  * sample the reference draws with torch.randint and gathers with
  * tensor[sample_index] before its topk.  sample_index: int64 positions on the
  * device, each in [0, n) (one outside sets ZEN_STAT_BAD_INDEX and counts as a
- * zero); 1 <= k <= s.  One gather kernel writes the sample into the workspace,
- * the radix select of zen_topk_threshold runs on it; nothing is allocated and
- * nothing waits for the device.
+ * zero); 1 <= k <= s.  The histogram is taken while the sample arrives: one
+ * launch for small samples, two (bf16) or three (fp32) for larger ones; nothing
+ * is allocated and nothing waits for the device.
  */
 size_t zen_sample_threshold_workspace(int64_t s, int dtype);
 int zen_sample_threshold(const void *input, int dtype, int64_t n,
@@ -293,9 +295,10 @@ int zen_load_balance_prepare(const void *input, int dtype, int64_t n, int64_t m,
                              size_t workspace_bytes, void *stream);
 
 /*
- * Which implementation a zen_load_balance call with these sizes takes: 0 = owner table (the general
- * mode), 1 = the same in three launches or one (tables of up to 4 Mi slots), or sort-based owner resolution, 2 = bucket slabs (large inputs whose expected output is a small
- * fraction of the table: one streaming pass, then per-bucket sorts inside LDS), 3 = wide buckets (the same
+ * Which implementation a zen_load_balance call with these sizes and this mode takes: 0 = owner table (the
+ * general mode), 1 = the same in three launches or one (tables below 2^20 slots, up to 4 Mi slots with k == 0 and
+ * ZEN_MODE_NO_SAMPLES) or sort-based owner resolution, 2 = bucket slabs (large inputs whose expected output is a
+ * small fraction of the table: one streaming pass, then per-bucket sorts inside LDS), 3 = wide buckets (the same
  * for an expected output of up to a few million entries: at most 256 buckets, one resident workgroup each,
  * two launches).  No counterpart in the reference; tests and benchmarks use it to know what they measured.
  */
@@ -315,8 +318,8 @@ int zen_load_balance_path(int64_t n, int64_t m, int dtype, int64_t capacity, int
  */
 size_t zen_merge_workspace(int64_t r, int64_t dense_n);
 size_t zen_merge_zero_bytes(void); /* see ZEN_MODE_ZEROED; the same for every r and dense_n */
-/* 0 = radix sort (general mode) or, in the fast mode, one workgroup for lists of up to 4096 entries, 1 = one bucket pass + per-range sorts, 2 = bucket slabs, 3 = wide buckets; see
-   zen_load_balance_path */
+/* 0 = radix sort (general mode) or, in the fast mode, one workgroup for lists of up to 4096 entries, 1 = one bucket
+   pass + per-range sorts, 2 = bucket slabs, 3 = wide buckets; see zen_load_balance_path */
 int zen_merge_path(int64_t r, int64_t dense_n, int mode);
 int zen_merge(const void *idx, int idx64_in, const void *val, int dtype,
               int64_t r, int64_t dense_n,
@@ -359,7 +362,8 @@ int zen_round_compact(const void *idx, int idx64, const float *sums,
  * load_balance before it, decode_sparse_tensors + encode_sparse_tensor after it) for a caller that holds the
  * received entries of the previous bucket while it encodes the next one.  The encode is enqueued on `stream`,
  * the merge on `merge_stream` (NULL: on `stream`, behind the encode); results and status words are those of
- * the two calls.  No counterpart in the reference: it exists so that a hook crosses the language boundary once
+ * the two calls.  What the merge finds zeroed (its status, count and ZEN_MODE_ZEROED workspace) has to be so in the
+ * order of `merge_stream`.  No counterpart in the reference: it exists so that a hook crosses the language boundary once
  * per bucket.
  */
 typedef struct zen_encode_merge_args {
@@ -397,8 +401,8 @@ typedef struct zen_encode_merge_args {
   void *stream, *merge_stream;
   /* Optional (NULL / 0: none): the gradient of the NEXT call on this workspace, of this one's type and
      partitions, and that call's k.  On the fast paths the pass over `input` then also takes the sample that
-     gives the next call's selection its floor (its workgroups do it when they are through with their own
-     tensor: no kernel of its own, nothing that waits), in the set of sampling memory this call does not use.
+     gives the next call's selection its floor (some of its workgroups do it first and leave their first tiles to
+     the others: no kernel of its own, nothing that waits), in the set of sampling memory this call does not use.
      The next call says so like after zen_load_balance_prepare: ZEN_MODE_PREPARED, with ZEN_MODE_SECOND unless
      THIS call's mode has ZEN_MODE_SECOND.  zen_encode_merge_samples_next tells whether a call with these sizes,
      its own k and its mode does it (the other paths ignore the fields).  next_input must be readable in the order of `stream`.
@@ -513,7 +517,7 @@ int zen_bucket_sort_pairs(uint32_t *keys, uint32_t *vals, int64_t max_count,
  * after the other in host[1..] by a kernel on `stream`, and the call returns when they are there, i.e. when
  * everything in front of it on the stream has finished.  `host` comes from zen_host_words_alloc(words): pinned,
  * coherent host memory, which serves one call at a time (a buffer per host thread); zen_host_words_free gives
- * it back.  These three are the only calls that allocate or that wait for the device.  No counterpart in the
+ * it back.  A wait of more than a millisecond leaves the core to other threads.  No counterpart in the
  * reference (its .tolist() and .item() calls do it, comm.py:119, tensor_load_balance.py:46-50).
  */
 #define ZEN_READ_BACK_SEGMENTS 3

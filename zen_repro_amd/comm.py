@@ -237,7 +237,8 @@ class LoadBalanceAllreduce:
         stream before the next call.  A sample taken ahead with
         partition.prepare() is picked up as load_balance_flat would.  `next_tensor` (ready in the current stream's
         order) is the gradient of the call that follows on this slot, `next_k` its k (default: this call's): if
-        it has this tensor's type, the pass over this tensor takes the sample of that call along (no kernel of
+        it has this tensor's type and this call takes a path that samples (with k == 0, small tensors do not), the
+        pass over this tensor takes the sample of that call along (no kernel of
         its own), as if partition.prepare(next_tensor, next_k, next_capacity, slot) had been called
         (`next_capacity`: that call's capacity, default this call's; gradient buckets differ in size)."""
         _lib.require_gpu(tensor, "input")

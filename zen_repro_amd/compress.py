@@ -27,7 +27,7 @@ def topk_threshold(tensor, k):
 def sample_threshold(tensor, sample_index, k):
     """(thr, status): thr as topk_threshold returns it for the multiset tensor.reshape(-1)[sample_index] (the
     sample of train.py:78-80), status int32[1] on the device (STAT_BAD_INDEX: a position outside the tensor).
-    One gather kernel and the radix select, no intermediate tensor, no host sync."""
+    One to three kernels that take the histogram while the sample arrives, no intermediate tensor, no host sync."""
     _lib.require_gpu(tensor, "input")
     _lib.require_gpu(sample_index, "sample_index")
     flat = tensor.reshape(-1)
