@@ -691,17 +691,19 @@ __device__ inline void stage_load_fast(const S *__restrict__ in, uint32_t last_v
   }
 }
 
-// Word w (0..15) of the 64 bytes a thread holds, without indexing registers dynamically.
+// Word w (0..15) of the 64 bytes a thread holds, without indexing registers dynamically: four levels of selects by
+// the bits of w (a compare and a select per word cost twice the instructions).
 __device__ inline uint32_t pick_word(const uint4 (&q)[kSelVecs], int w) {
-  uint32_t r = 0;
+  static_assert(kSelVecs == 4, "four levels");
+  const bool b0 = w & 1, b1 = w & 2, b2 = w & 4, b3 = w & 8;
+  uint32_t v[kSelVecs];
 #pragma unroll
   for (int j = 0; j < kSelVecs; ++j) {
-    r = w == 4 * j ? q[j].x : r;
-    r = w == 4 * j + 1 ? q[j].y : r;
-    r = w == 4 * j + 2 ? q[j].z : r;
-    r = w == 4 * j + 3 ? q[j].w : r;
+    const uint32_t lo = b0 ? q[j].y : q[j].x, hi = b0 ? q[j].w : q[j].z;
+    v[j] = b1 ? hi : lo;
   }
-  return r;
+  const uint32_t lo = b2 ? v[1] : v[0], hi = b2 ? v[3] : v[2];
+  return b3 ? hi : lo;
 }
 // The element a flag bit stands for, straight from the flag's number (word 4j + w, half h for bf16).
 __device__ inline uint16_t Flags<uint16_t>::pick(const uint4 (&q)[kSelVecs], uint32_t bit) {
@@ -732,7 +734,6 @@ struct StageSlabs {
   CoarseGeom cg;     // wide: groups = buckets, per = 1, cap = entries per part
   uint32_t *cursor;  // part cursors
   uint32_t *words;   // word planes
-  uint32_t wide;
 };
 
 constexpr int kStageDstMax = 256;  // destinations of a flush, at most (one counter per thread)
@@ -749,7 +750,7 @@ struct StageFlushShared {
 // its index), the stage is put in destination order in place, every destination's run is reserved with one
 // atomic and consecutive lanes write consecutive places.  Element 0 is not handed on (index 0 is never
 // transmitted: 0 is the table's empty marker, tensor_load_balance.py:31), but counts in the histogram.
-template <typename S>
+template <typename S, bool WIDE>
 __device__ inline void stage_flush(uint32_t count, int32_t *st_idx, S *st_val, StageFlushShared &fl,
                                    uint32_t *s_hist, uint32_t floor_key, const StageSlabs &out, int32_t *status) {
   constexpr int kPer = kScatStage / kSelBlock;
@@ -777,7 +778,7 @@ __device__ inline void stage_flush(uint32_t count, int32_t *st_idx, S *st_val, S
       if (t[i] != 0) {
         uint32_t rem;
         const uint32_t bucket = out.geo.bucket_of(out.geo.mod_m(poly(t[i]) + kSeed1));
-        d[i] = out.wide ? bucket : SlabGeom::div_small(bucket, out.cg.per, out.cg.inv_per, &rem);
+        d[i] = WIDE ? bucket : SlabGeom::div_small(bucket, out.cg.per, out.cg.inv_per, &rem);
         r[i] = atomicAdd(&fl.cnt[d[i]], 1u);
       }
     }
@@ -814,7 +815,7 @@ __device__ inline void stage_flush(uint32_t count, int32_t *st_idx, S *st_val, S
     if (at < out.cg.cap) {
       const size_t o = (size_t)(g * kCoarseSplit + part) * out.cg.cap + at;
       const uint32_t idx = (uint32_t)st_idx[p];
-      if (out.wide) {
+      if (WIDE) {
         // one 8-byte record per candidate: a run of eight fills two 32-byte sectors (three planes of their
         // own cost three partly filled ones per run, and the scattered stores are what a flush spends its
         // time on)
@@ -986,7 +987,14 @@ __device__ inline void stage_sample_next(const StageSample &smp, uint32_t *windo
   if (s_last) sample_pick_block<kSelBlock>(smp.hist, smp.rank, kShift, smp.floor_out, smem);
 }
 
-template <typename S, bool ALIGNED>
+// WIDE: the destinations are wide buckets, else coarse slabs.  Where a thread finds a candidate's value again: on the
+// way to coarse slabs (selections of many millions) in a copy of the sub-tile in LDS, six instructions per candidate;
+// picked out of the registers that are loaded it costs 24, and the wave does so as often as its fullest lane has
+// candidates (62 M bf16, 10 % selected: 77 -> 56 us; 5 %: 52 -> 41; 268 M, 1 %: 94 -> 88).  On the way to wide buckets
+// it is picked out of the registers: one candidate in two hundred, and 48 KB less LDS per compute unit leave room for the
+// merge's kernels beside this one (743 M, 0.5 %, with a merge on another stream: 417 us a step, with the copy 496: the
+// third workgroup of many units then starts behind the merge's).
+template <typename S, bool ALIGNED, bool WIDE>
 __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
     const S *__restrict__ in, int64_t n, const uint32_t *__restrict__ thr, StageSlabs out, uint32_t *ticket,
     StageSched sch, uint32_t *cand_hist, uint32_t pick_k, uint32_t *pick_thr, uint32_t *pick_above,
@@ -995,11 +1003,13 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
   constexpr int V = VecOf<S>::kN;
   constexpr int kSub = kSelBlock * kSelVecs * V;
   constexpr int kWaves = kSelBlock / 64;
+  constexpr bool TILE = !WIDE || !ALIGNED;  // (unaligned, the loads leave no registers for the selects either)
   // what the kernel before this one needed at zero and nobody needs any more (the sample's histogram): back
   // to zero, a slice per workgroup
   for (uint32_t i = blockIdx.x * kSelBlock + threadIdx.x; i < clear_words; i += gridDim.x * kSelBlock) clear[i] = 0;
   __shared__ uint32_t s_wave[2][kWaves];
   __shared__ uint32_t s_next[2];
+  __shared__ __attribute__((aligned(16))) S s_tile[TILE ? kSub : 1];
   // the stage and what a flush needs; before that, the window of the next call's sample
   __shared__ StageRun<S> s_run;
   int32_t (&st_idx)[kScatStage] = s_run.run.idx;
@@ -1096,6 +1106,10 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
           if (vec0 + (uint32_t)j * kSelBlock + threadIdx.x >= full_vecs) x &= ~Flags<S>::vec_mask(j);
       }
     }
+    if (TILE && __any(x != 0)) {  // for this thread alone: no barrier
+#pragma unroll
+      for (int j = 0; j < kSelVecs; ++j) reinterpret_cast<uint4 *>(s_tile)[j * kSelBlock + threadIdx.x] = cur[j];
+    }
     const uint32_t cnt = (uint32_t)__popc(x);
     const uint32_t incl = wave_inclusive_scan_dpp(cnt);
     if ((threadIdx.x & 63) == 63) s_wave[par & 1][wave] = incl;
@@ -1114,32 +1128,26 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
       if (w < wave) before += t;
       total += t;
     }
-    const uint32_t all = x;
-    const uint32_t first_elem = (uint32_t)sub_base + threadIdx.x * (uint32_t)V;  // indices are below 2^31
+    const uint32_t own = threadIdx.x * (uint32_t)V;
+    uint32_t pos = before;  // a thread's candidates take their places in the order of their flag bits
     uint32_t done = 0;
     for (;;) {
       const uint32_t room = (uint32_t)kScatStage - count;
-      const uint32_t hi = done + room;
-      uint32_t y = x;
-      while (y) {
-        const uint32_t bit = (uint32_t)__ffs((int)y) - 1u;
-        y &= y - 1;
-        // the thread's candidates take their places in the order of their flag bits (the stage has no order
-        // to keep, and a place counted off the flag word costs two instructions)
-        const uint32_t pos = before + (uint32_t)__popc(all & ((1u << bit) - 1u));
-        if (pos < hi) {
-          x &= ~(1u << bit);
-          const uint32_t at = count + pos - done;
-          st_idx[at] = (int32_t)(first_elem + Flags<S>::elem_step(bit));
-          st_val[at] = Flags<S>::pick(cur, bit);
-        }
+      const uint32_t hi = done + room, shift = count - done;
+      while (x != 0 && pos < hi) {
+        const uint32_t bit = (uint32_t)__ffs((int)x) - 1u;
+        x &= x - 1;
+        const uint32_t elem = own + Flags<S>::elem_step(bit);  // inside the sub-tile
+        st_idx[pos + shift] = (int32_t)((uint32_t)sub_base + elem);  // indices are below 2^31
+        st_val[pos + shift] = TILE ? s_tile[elem] : Flags<S>::pick(cur, bit);
+        ++pos;
       }
       const uint32_t take = total - done < room ? total - done : room;
       count += take;
       done += take;
       if (count < (uint32_t)kScatStage) break;
       __syncthreads();
-      stage_flush<S>(count, st_idx, st_val, s_flush, hist, floor_key, out, status);
+      stage_flush<S, WIDE>(count, st_idx, st_val, s_flush, hist, floor_key, out, status);
       count = 0;
       if (done == total) break;
     }
@@ -1192,7 +1200,7 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
     if (!step(qc, qb)) break;
   }
   __syncthreads();
-  if (count) stage_flush<S>(count, st_idx, st_val, s_flush, hist, floor_key, out, status);
+  if (count) stage_flush<S, WIDE>(count, st_idx, st_val, s_flush, hist, floor_key, out, status);
   if (ALIGNED && blockIdx.x == 0 && (int64_t)full_vecs * V < n) {
     // the elements behind the last complete vector (fewer than V): a small stage of their own
     if (threadIdx.x == 0) {
@@ -1209,7 +1217,7 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
     }
     __syncthreads();
     const uint32_t c = s_tail;
-    if (c) stage_flush<S>(c, st_idx, st_val, s_flush, hist, floor_key, out, status);
+    if (c) stage_flush<S, WIDE>(c, st_idx, st_val, s_flush, hist, floor_key, out, status);
   }
   if (hist) {
     __syncthreads();
@@ -1257,8 +1265,7 @@ static int stage_launch(const StageArgs &a, hipStream_t stream) {
   const int64_t sub = (int64_t)kSelBlock * kSelVecs * V;
   const int64_t subs = ceil_div(a.n > 0 ? a.n : 1, sub);
   if (subs > 0x3fffffff) return fail(ZEN_EINVAL, "select_stage: tensor too large");
-  // three workgroups per compute unit (measured: two are 10 % slower, four no faster); their LDS, 60 KB per
-  // unit, leaves room for another stream's kernels next to this long one
+  // three workgroups per compute unit (measured: two are 10 % slower, four no faster)
 #ifndef ZEN_STAGE_WGS
 #define ZEN_STAGE_WGS 3
 #endif
@@ -1271,7 +1278,7 @@ static int stage_launch(const StageArgs &a, hipStream_t stream) {
   sch.fixed = (uint32_t)(subs * 7 / 8 / ((int64_t)kStageBig * blocks));
   const S *in = static_cast<const S *>(a.in);
   const bool aligned = (reinterpret_cast<uintptr_t>(in) & 15u) == 0 && a.n >= V;
-  const StageSlabs out{a.geo, a.cg, a.coarse_cursor, a.coarse_words, a.wide ? 1u : 0u};
+  const StageSlabs out{a.geo, a.cg, a.coarse_cursor, a.coarse_words};
   StageSample next;
   if (a.next_in && a.next_hist && a.next_k > 0) {
     const int64_t next_n = a.next_n > 0 ? a.next_n : a.n;  // the next tensor has this one's type
@@ -1293,14 +1300,11 @@ static int stage_launch(const StageArgs &a, hipStream_t stream) {
   sch.fixed_subs = (uint32_t)(((int64_t)sch.fixed * blocks - (int64_t)sch.skip * sch.late) * kStageBig);
   sch.ticket_tiles = (uint32_t)ceil_div(subs - (int64_t)sch.fixed_subs, kStageSmall);
   ProfScope prof(kProfSelectStage, stream);
-  if (aligned)
-    k_select_stage<S, true><<<dim3((unsigned)blocks), dim3(kSelBlock), 0, stream>>>(
-        in, a.n, a.thr, out, a.ticket, sch, a.cand_hist, (uint32_t)a.pick_k, a.pick_thr, a.pick_above, a.thr_copy,
-        a.clear, a.clear_words, a.floor_margin, next, a.status);
-  else
-    k_select_stage<S, false><<<dim3((unsigned)blocks), dim3(kSelBlock), 0, stream>>>(
-        in, a.n, a.thr, out, a.ticket, sch, a.cand_hist, (uint32_t)a.pick_k, a.pick_thr, a.pick_above, a.thr_copy,
-        a.clear, a.clear_words, a.floor_margin, next, a.status);
+  const auto kernel = aligned ? (a.wide ? k_select_stage<S, true, true> : k_select_stage<S, true, false>)
+                              : (a.wide ? k_select_stage<S, false, true> : k_select_stage<S, false, false>);
+  kernel<<<dim3((unsigned)blocks), dim3(kSelBlock), 0, stream>>>(
+      in, a.n, a.thr, out, a.ticket, sch, a.cand_hist, (uint32_t)a.pick_k, a.pick_thr, a.pick_above, a.thr_copy,
+      a.clear, a.clear_words, a.floor_margin, next, a.status);
   ZEN_LAUNCH_CHECK("k_select_stage");
   return ZEN_OK;
 }
