@@ -125,6 +125,30 @@ def test_slab_load_balance_odd_length_unaligned_and_empty(zen, oracle, dtype):
     assert status.item() == 0 and int(splits.sum()) == 0
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("P,scale,rehash", [
+    (8, 21, 3),       # buckets of 131 075 slots: just past the narrowest width the bucket kernels come in
+    (64, 100, 2),     # the second width
+    (3000, 5000, 3),  # 333 333 slots: as many buckets as there may be, and wider than two workgroups to a unit allow
+])
+def test_slab_load_balance_at_every_bucket_width(zen, oracle, P, scale, rehash, dtype):
+    from zen_repro_amd import _lib
+
+    n = 200000 // P * P
+    g = make_grad(oracle, n, 0.3, dtype, seed=P + scale)
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, scale, rehash)
+    capacity = len(idx_o) + 1024
+    if not FLAGS and lb_path(zen, n, P, dtype, capacity, scale=scale) != WIDE:
+        pytest.skip("covered by the other run")
+    assert st_o == 0 and on_fast_path(lb_path(zen, n, P, dtype, capacity, scale=scale))
+    tp = zen.TensorPartition(P, scale, rehash)
+    oi, ov, splits, status = tp.load_balance_flat(to_dev(g), capacity=capacity, mode=_lib.MODE_FAST)
+    assert status.item() == 0
+    assert np.array_equal(to_np(splits), splits_o)
+    assert np.array_equal(to_np(oi)[:len(idx_o)], idx_o)
+    assert np.array_equal(to_np(ov)[:len(idx_o)], val_o)
+
+
 def test_slab_load_balance_declines_and_general_mode_takes_over(zen, oracle):
     """One rehash level at 15 % load sends every level-1 loser to the serial
     lists: far more than the slab path carries per partition.  It must say so

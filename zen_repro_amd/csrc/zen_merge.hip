@@ -211,7 +211,7 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
                                                              I *__restrict__ out_idx, O *__restrict__ out_val,
                                                              int64_t capacity, ScanState st, int tie_bits,
                                                              int64_t *out_count, int32_t *status) {
-  __shared__ SlabSortSharedT<true> sh;  // the values take the counters' place once the ranks are known
+  __shared__ SlabSortShared sh;  // the values take the counters' place once the ranks are known
   __shared__ uint64_t s_scan64[kMergeBlock / 64 + 1];
   __shared__ int s_tile;
   if (threadIdx.x == 0) s_tile = (int)atomicAdd(st.ticket, 1u);
@@ -437,7 +437,7 @@ SlabMergePlan plan_slab_merge(void *workspace, const SlabGeom &geo, int64_t r) {
 
 bool slab_merge_fits(int64_t r, int64_t dense_n, SlabGeom *geo) {
   SlabGeom g;
-  if (r < (1 << 15) || r > 0x7ffffffell || !slab_geometry(dense_n, 1, r, kMergeTarget, &g)) return false;
+  if (r < (1 << 15) || r > 0x7ffffffell || !slab_geometry(dense_n, 1, r, kMergeTarget, 0, 0, &g)) return false;
   if (g.sub_shift + ceil_log2_u64((uint64_t)r) > 32) return false;  // (index inside a narrow range, arrival number) must fit a word
   if (geo) *geo = g;
   return true;

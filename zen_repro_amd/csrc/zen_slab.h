@@ -39,6 +39,7 @@ struct SlabGeom {
   uint32_t bpp;       // buckets per partition
   uint32_t bpp_mult;  // floor(bpp * 2^32 / npp)
   uint32_t nbuckets;  // partitions * bpp
+  uint32_t span;      // keys of one bucket, at most
   int sub_shift;      // key offset inside a bucket >> sub_shift = narrow range (fewer than kSlabSubs of them)
   float inv_m;        // (1 / m)(1 - 2^-20), rounded down
   float inv_npp;      // the same for npp
@@ -89,8 +90,10 @@ struct SlabGeom {
 inline double slab_bucket_width(uint32_t bpp_mult) { return 4294967296.0 / (double)bpp_mult; }
 
 // Host side: geometry for `partitions` partitions of a key space of m keys (m a
-// multiple of partitions) expected to hold about `expected` records.  Returns
-// false if the slab layout does not suit these sizes.
+// multiple of partitions) expected to hold about `expected` records, its buckets
+// good_span keys wide or less where the number of buckets allows that (0: any
+// width).  Returns false if the slab layout does not suit these sizes or a bucket
+// would be wider than most_span keys.
 inline float slab_inverse_below(uint32_t d) {
   const double want = (1.0 / (double)d) * (1.0 - 1.0 / 1048576.0);
   float f = (float)want;
@@ -98,7 +101,8 @@ inline float slab_inverse_below(uint32_t d) {
   return f;
 }
 
-inline bool slab_geometry(int64_t m, int partitions, int64_t expected, int target, SlabGeom *out) {
+inline bool slab_geometry(int64_t m, int partitions, int64_t expected, int target, int64_t good_span, int64_t most_span,
+                          SlabGeom *out) {
   if (m < (1ll << 22) || m > 0x7fffffffll || partitions < 1 || partitions > kSlabMaxBuckets || m % partitions != 0 ||
       expected < 1)
     return false;
@@ -113,9 +117,14 @@ inline bool slab_geometry(int64_t m, int partitions, int64_t expected, int targe
     const int64_t fewer = (rounds - 1) * kSlabResident / partitions;
     if (fewer >= 1 && expected / (fewer * partitions) <= (int64_t)kSlabCap * 3 / 4) bpp = fewer;
   }
+  const int64_t npp = m / partitions;
+  if (good_span > 0) {
+    int64_t wanted = ceil_div(npp, good_span);
+    if (wanted * partitions > kSlabMaxBuckets) wanted = kSlabMaxBuckets / partitions;
+    if (bpp < wanted) bpp = wanted;
+  }
   const int64_t nb = bpp * partitions;
   if (expected / nb > (int64_t)kSlabCap * 3 / 4) return false;  // too many records per bucket
-  const int64_t npp = m / partitions;
   if (npp / bpp < 4 * kSlabSubs) return false;                  // buckets narrower than their sub-ranges
   SlabGeom g;
   g.m = (uint32_t)m;
@@ -124,6 +133,8 @@ inline bool slab_geometry(int64_t m, int partitions, int64_t expected, int targe
   g.bpp_mult = (uint32_t)(((uint64_t)bpp << 32) / (uint64_t)npp);
   g.nbuckets = (uint32_t)nb;
   const uint64_t width = ((1ull << 32) + g.bpp_mult - 1) / g.bpp_mult + 1;  // keys per bucket, at most
+  if (most_span > 0 && width > (uint64_t)most_span) return false;
+  g.span = (uint32_t)width;
   g.sub_shift = 0;
   while ((width >> g.sub_shift) >= (uint64_t)kSlabSubs) ++g.sub_shift;
   g.width = slab_bucket_width(g.bpp_mult);
@@ -143,26 +154,13 @@ __device__ inline uint32_t sub_place(uint32_t s) {
   return s < (uint32_t)kSlabSubs ? (s % kPer) * BLOCK + s / kPer : s;
 }
 
-// Shared memory of the in-LDS sort.  slab_rank does not touch `tie`, and a caller that fills it only after
-// slab_rank has returned and has no use for `cnt` from then on lets the two share their memory (OVERLAY):
+// Shared memory of the in-LDS sort.  slab_rank does not touch `tie`: a caller fills it only after
+// slab_rank has returned and has no use for `cnt` from then on, so that the two share their memory:
 // LDS decides how many workgroups share a compute unit.
-template <bool OVERLAY>
-struct SlabSortSharedT;
 constexpr int kSlabQueueCap = kSlabCap - kSlabSubs - 1;  // large-group records a workgroup sets aside
 constexpr int kSlabInline = 4;                            // groups up to this size are ranked by their own threads
 constexpr int kSlabQueueMin = 256;                        // records in larger groups below which nothing is set aside
-template <>
-struct SlabSortSharedT<false> {
-  static constexpr bool kQueue = false;
-  uint32_t key[kSlabCap];
-  uint32_t tie[kSlabCap];
-  uint32_t cnt[kSlabSubs + 1];
-  uint32_t scan[kSlabMaxBlock / 64 + 1];
-  uint32_t bad;
-};
-template <>
-struct SlabSortSharedT<true> {
-  static constexpr bool kQueue = true;
+struct SlabSortShared {
   uint32_t key[kSlabCap];
   union {
     uint32_t tie[kSlabCap];
@@ -174,27 +172,12 @@ struct SlabSortSharedT<true> {
   uint32_t scan[kSlabMaxBlock / 64 + 1];
   uint32_t bad;
 };
-
-// The same sharing of memory without the queue (the queue's code costs slab_rank registers).
-struct SlabSortSharedNoQueue {
-  static constexpr bool kQueue = false;
-  uint32_t key[kSlabCap];
-  union {
-    uint32_t tie[kSlabCap];
-    uint32_t cnt[kSlabSubs + 1];
-  };
-  uint32_t scan[kSlabMaxBlock / 64 + 1];
-  uint32_t bad;
-};
-
 static_assert(kSlabSubs + 1 <= kSlabCap, "the counters fit under the ties");
-using SlabSortShared = SlabSortSharedT<false>;
 
 // Number of words in sh.key[b0, b1) that are smaller than w.  The words are fetched four at a time (places past
 // the end are pulled back onto the last word and not counted): a loop that fetches one word per turn waits
 // for LDS once per word, and that wait is what such a loop spends its time on.
-template <typename Shared>
-__device__ inline uint32_t slab_count_less(const Shared &sh, uint32_t b0, uint32_t b1, uint32_t w) {
+__device__ inline uint32_t slab_count_less(const SlabSortShared &sh, uint32_t b0, uint32_t b1, uint32_t w) {
   uint32_t less = 0;
   const uint32_t last = b1 - 1u;
   for (uint32_t u = b0; u < b1; u += 4) {
@@ -214,15 +197,15 @@ __device__ inline uint32_t slab_count_less(const Shared &sh, uint32_t b0, uint32
 // inside its group every record counts the words smaller than its own: the first kSlabInline words of every
 // record's group are fetched in one go (all of them in flight together), which settles groups up to that size.
 // Where many records share a key (a merge of payloads that overlap) a few lanes of every wave would then walk
-// through groups of dozens while the others wait: with a Shared that has a queue, records of groups larger
+// through groups of dozens while the others wait: records of groups larger
 // than kSlabInline are set aside instead (their places in the queue follow from the same prefix sums as the
 // groups' places: the counters carry both, 16 bits each) and handed out again afterwards, one per lane, so
 // that the lanes of a wave walk through large groups together.  Returns false (for every thread) if a
 // group is too large for that; else rank[i] for live records and *n_out = number of live records.  On return
 // sh.key / sh.tie may be overwritten at once (sh.tie is not touched at all), and the low 16 bits of
 // sh.cnt[sub_place(s)] hold the sorted place of the first record of narrow range s.
-template <int BLOCK, typename Shared>
-__device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
+template <int BLOCK>
+__device__ inline bool slab_rank(SlabSortShared &sh, const SlabGeom &geo, int tie_bits,
                                  const uint32_t (&off)[kSlabCap / BLOCK], const uint32_t (&tie)[kSlabCap / BLOCK],
                                  uint32_t live, uint32_t (&rank)[kSlabCap / BLOCK], uint32_t *n_out) {
   static_assert(BLOCK <= kSlabMaxBlock && kSlabCap % BLOCK == 0 && kSlabSubs % BLOCK == 0, "workgroup size");
@@ -266,7 +249,7 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
   if (sh.bad) return false;
   const uint32_t totals = sh.cnt[kSlabSubs];
   // a few large groups are not worth the extra barrier
-  const bool set_aside = Shared::kQueue && (totals >> 16) >= (uint32_t)kSlabQueueMin;
+  const bool set_aside = (totals >> 16) >= (uint32_t)kSlabQueueMin;
   constexpr uint32_t kSetAside = 0x80000000u;
   uint32_t g0[kItems], g1[kItems], word[kItems];
 #pragma unroll
@@ -278,14 +261,12 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
       g1[i] = sh.cnt[sub_place<BLOCK>(sub[i] + 1)] & 0xffffu;
       word[i] = ((off[i] & low_mask) << tie_bits) | tie[i];
       sh.key[g0[i] + at[i]] = word[i];
-      if constexpr (Shared::kQueue) {
-        static_assert(kSlabSubs <= (1 << 12) && kSlabGroupLimit <= (1 << 19), "a queue entry is one word");
-        const uint32_t q = (here >> 16) + at[i];
-        if (set_aside && g1[i] - g0[i] > (uint32_t)kSlabInline && q < (uint32_t)kSlabQueueCap) {
-          sh.queue[q] = sub[i] | (at[i] << 12);  // sub < 2^12, at < group size <= kSlabGroupLimit
-          rank[i] = kSetAside | q;
-          g1[i] = g0[i];  // nothing left to do for it below
-        }
+      static_assert(kSlabSubs <= (1 << 12) && kSlabGroupLimit <= (1 << 19), "a queue entry is one word");
+      const uint32_t q = (here >> 16) + at[i];
+      if (set_aside && g1[i] - g0[i] > (uint32_t)kSlabInline && q < (uint32_t)kSlabQueueCap) {
+        sh.queue[q] = sub[i] | (at[i] << 12);  // sub < 2^12, at < group size <= kSlabGroupLimit
+        rank[i] = kSetAside | q;
+        g1[i] = g0[i];  // nothing left to do for it below
       }
     }
   }
@@ -322,26 +303,62 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
       }
     }
   }
-  if constexpr (Shared::kQueue) {
-    if (set_aside) {
-      const uint32_t queued = (totals >> 16) < (uint32_t)kSlabQueueCap ? (totals >> 16) : (uint32_t)kSlabQueueCap;
-      // the thread that takes a queue entry also overwrites it with the rank
+  if (set_aside) {
+    const uint32_t queued = (totals >> 16) < (uint32_t)kSlabQueueCap ? (totals >> 16) : (uint32_t)kSlabQueueCap;
+    // the thread that takes a queue entry also overwrites it with the rank
 #pragma unroll 1
-      for (uint32_t q = threadIdx.x; q < queued; q += BLOCK) {
-        const uint32_t e = sh.queue[q];
-        const uint32_t b0 = sh.cnt[sub_place<BLOCK>(e & 4095u)] & 0xffffu;
-        const uint32_t b1 = sh.cnt[sub_place<BLOCK>((e & 4095u) + 1)] & 0xffffu;
-        sh.queue[q] = b0 + slab_count_less(sh, b0, b1, sh.key[b0 + (e >> 12)]);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < kItems; ++i)
-        if (rank[i] & kSetAside) rank[i] = sh.queue[rank[i] & ~kSetAside];
+    for (uint32_t q = threadIdx.x; q < queued; q += BLOCK) {
+      const uint32_t e = sh.queue[q];
+      const uint32_t b0 = sh.cnt[sub_place<BLOCK>(e & 4095u)] & 0xffffu;
+      const uint32_t b1 = sh.cnt[sub_place<BLOCK>((e & 4095u) + 1)] & 0xffffu;
+      sh.queue[q] = b0 + slab_count_less(sh, b0, b1, sh.key[b0 + (e >> 12)]);
     }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kItems; ++i)
+      if (rank[i] & kSetAside) rank[i] = sh.queue[rank[i] & ~kSetAside];
   }
   *n_out = totals & 0xffffu;
   __syncthreads();
   return true;
 }
+
+// Which keys of a bucket are taken, one bit each, and how many of them lie before every 64th key: a key's place among
+// those that are taken is then two look-ups and a count of bits, whatever order the records come in.  SPAN: keys of a
+// bucket, at most; `words` of the bitmap's words are in use.
+template <uint32_t SPAN>
+struct SlabTaken {
+  static constexpr uint32_t kWords = (SPAN + 63) / 64;
+  uint64_t bits[kWords];
+  uint16_t before[kWords];
+
+  template <int BLOCK>
+  __device__ inline void clear(uint32_t words) {
+    for (uint32_t i = threadIdx.x; i < words; i += BLOCK) bits[i] = 0;
+  }
+  // Marks key `off`; the bits of its half word before that (`mark` 0: nothing is marked).
+  __device__ inline uint32_t take(uint32_t off, uint32_t mark) {
+    return atomicOr(reinterpret_cast<uint32_t *>(bits) + (off >> 5), mark << (off & 31u));
+  }
+  // Fills `before`, by the whole workgroup between barriers; returns the number of keys taken.
+  template <int BLOCK>
+  __device__ inline uint32_t count(uint32_t words, uint32_t *scan) {
+    const uint32_t per = (words + BLOCK - 1) / BLOCK | 1u;  // odd: the lanes of a wave on different banks
+    const uint32_t first = threadIdx.x * per, end = first + per < words ? first + per : words;
+    uint32_t sum = 0;
+    for (uint32_t i = first; i < end; ++i) sum += (uint32_t)__popcll(bits[i]);
+    uint32_t total;
+    uint32_t run = block_exclusive_scan<uint32_t, BLOCK>(sum, scan, &total);
+    for (uint32_t i = first; i < end; ++i) {
+      before[i] = (uint16_t)run;
+      run += (uint32_t)__popcll(bits[i]);
+    }
+    return total;
+  }
+  // Keys taken below `off`.
+  __device__ inline uint32_t place(uint32_t off) const {
+    return before[off >> 6] + (uint32_t)__popcll(bits[off >> 6] & ((1ull << (off & 63u)) - 1ull));
+  }
+};
 
 }  // namespace zen

@@ -8,10 +8,10 @@
 // slots, zen_slab.h), and four short kernels finish the job:
 //   k_fine_scatter  the coarse slabs, filtered by the exact threshold, go to the
 //                   bucket slabs, so that every store belongs to a long run;
-//   k_slab_sort     one workgroup per bucket: sorts
-//                   the bucket by (level-1 slot, index) inside LDS; in a run of
-//                   equal slots the first entry (smallest index) is the slot's
-//                   level-1 owner, the others lost level 1 and are logged;
+//   k_slab_sort     one workgroup per bucket: puts the bucket in the order of its
+//                   level-1 slots by a bitmap of them in LDS; of the entries that
+//                   share a slot the one with the smallest index is its level-1
+//                   owner, the others lost level 1 and are logged;
 //   k_slab_chains   levels 2 and 3 for the losers through a small hash map,
 //                   with the reference's rule executed in ascending index order
 //                   (a slot belongs to the smallest index that ever probes it;
@@ -20,8 +20,8 @@
 //                   of its own, so what finally moved into a bucket is what its
 //                   part holds; an index that ran out of levels goes to its
 //                   partition's serial list;
-//   k_slab_place    one workgroup per bucket: survivors and moved-in entries
-//                   merged by rank, written to the bucket's place in the
+//   k_slab_place    one workgroup per bucket: survivors and moved-in entries by
+//                   the same kind of bitmap to the bucket's place in the
 //                   partition-major output; split sizes.
 #include "zen_balance.h"
 #include "zen_hashmap.h"
@@ -35,8 +35,8 @@ namespace {
 struct SlabTables {
   uint32_t *cursor;     // [B * kCursorPad] records in the bucket's slab, at [b * kCursorPad]
   uint32_t *bucket_lo;  // [B] smallest level-1 slot of the bucket
-  uint32_t *bucket_n;   // [B] selected records, sorted, in the slab
-  uint32_t *removed_n;  // [B] of which lost their level-1 slot
+  uint32_t *bucket_n;   // [B] level-1 owners, sorted, in the slab
+  uint32_t *removed_n;  // [B] of which were pushed out of their slot
   uint32_t *movein_n;   // [B * kMoveinPad] occupied cells of the bucket's part of the map
   uint32_t *serial_n;   // [P * kMoveinPad] entries that found no slot
   uint32_t *raw_idx;    // [B * kSlabCap] entries as they arrive: index ...
@@ -103,140 +103,137 @@ struct EncodeSink {
 
 // ------------------------------------------------------------ sort a bucket
 
-// Twice the threads of the other per-bucket kernels, half the records each: the phases of this kernel are
-// chains of LDS round trips, and eight waves per SIMD hide them better than four (38 -> 30 us); it needs
-// fewer than 64 registers, so two workgroups still share a compute unit.
+// Keys of a bucket: the three widths the per-bucket kernels come in.  Their bitmaps decide how much LDS a workgroup
+// takes: up to the second width two workgroups share a compute unit, and the number of buckets is raised to stay
+// within it (slab_geometry) until there are kSlabMaxBuckets of them.
+constexpr uint32_t kSlabSpan1 = 1u << 17, kSlabSpan2 = 5u << 16, kSlabSpan3 = 9u << 16;
+
 constexpr int kSortBlock = 1024;
 constexpr int kSortItems = kSlabCap / kSortBlock;
 
-template <typename S>
-__global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabTables tb, int32_t *status) {
-  // the ties take the place of the counters once the ranks are known: with 32-bit values the kernel would
-  // otherwise need 88 KB of LDS, one workgroup to a compute unit instead of two
-  __shared__ SlabSortSharedNoQueue sh;
-  __shared__ S s_val[kSlabCap];
-  __shared__ uint32_t s_lost, s_base;
+template <typename S, uint32_t SPAN>
+struct SlabSortLds {
+  uint32_t idx[kSlabCap];  // the sorted indices
+  union {
+    SlabTaken<SPAN> taken;
+    S val[kSlabCap];       // once the ranks are known: the sorted values
+  };
+  uint32_t scan[kSortBlock / 64 + 1];
+  uint32_t shared, lost, base;
+};
+
+// Sorts a bucket's records by level-1 slot; of those that share a slot the smallest index owns it, the others are
+// logged and not kept.  A bucket has a few to a few hundred slots per record, so the slots are marked in a bitmap: a
+// record's place is the number of marks below its own, and whoever finds its slot marked already is settled by the
+// smallest index afterwards.  Bound by the LDS round trips (six records a thread, two workgroups a compute unit) and by
+// the 12 to 16 bytes a record moves: 62 M slots, 6.2 M bf16 records 48 us, 3.1 M 24.  (Grouped by narrow key ranges and ranked by comparing the words of a group, with
+// the owners found by walking the sorted runs: 64 and 33.)
+template <typename S, uint32_t SPAN>
+__global__ __launch_bounds__(kSortBlock, SPAN <= kSlabSpan2 ? 8 : 4) void k_slab_sort(SlabGeom geo, SlabTables tb,
+                                                                                  int32_t *status) {
+  __shared__ SlabSortLds<S, SPAN> sh;
   const uint32_t b = blockIdx.x;
   const size_t base = (size_t)b * kSlabCap;
+  const uint32_t words = (geo.span + 63u) / 64u;
   uint32_t n_raw = tb.cursor[b * kCursorPad];
   if (n_raw > (uint32_t)kSlabCap) n_raw = kSlabCap;  // the scatter flagged the overflow
   const uint32_t lo = tb.bucket_lo[b];
   S *slab_val = static_cast<S *>(tb.slab_val);
-  if (threadIdx.x == 0) s_lost = 0;
+  if (threadIdx.x == 0) sh.shared = sh.lost = 0;
+  sh.taken.template clear<kSortBlock>(words);
   // the kernels before this one were the last to need these: back to zero, a slice per workgroup
   for (uint32_t i = b * kSortBlock + threadIdx.x; i < kCoarseCursorWords; i += gridDim.x * kSortBlock)
     tb.coarse_cursor[i] = 0;
   if (tb.refine_hist)
     for (uint32_t i = b * kSortBlock + threadIdx.x; i <= (uint32_t)kRefineBins; i += gridDim.x * kSortBlock)
       tb.refine_hist[i] = 0;
-  uint32_t off[kSortItems], idx[kSortItems], pos[kSortItems], rank[kSortItems];
+  uint32_t off[kSortItems], idx[kSortItems], rank[kSortItems];
   S val[kSortItems];
-  uint32_t live = 0;
+  uint32_t live = 0, owner = 0;
+  // rows past the records are left out (the same for the whole workgroup): a bucket is seldom more than half full, and
+  // the instructions for the other half cost 24 of 72 us
+  auto row = [&](int i) { return (uint32_t)(i * kSortBlock) < n_raw; };
 #pragma unroll
   for (int i = 0; i < kSortItems; ++i) {
     const uint32_t j = threadIdx.x + i * kSortBlock;
-    // no branch around the loads (places past the end are pulled back onto the slab's first record): they are
+    idx[i] = 0;
+    val[i] = 0;
+    if (!row(i)) continue;
+    // no branch around a wave's loads (places past the end are pulled back onto the slab's first record): they are
     // all in flight together
     const size_t from = base + (j < n_raw ? j : 0u);
     idx[i] = tb.raw_idx[from];
     val[i] = static_cast<const S *>(tb.raw_val)[from];
-    off[i] = pos[i] = 0;
-    if (j < n_raw) {
-      off[i] = geo.mod_m(poly(idx[i]) + kSeed1) - lo;  // the level-1 slot again: cheaper than carrying it along
-      pos[i] = j;
-      live |= 1u << i;
-    }
+    if (j < n_raw) live |= 1u << i;
   }
-  // ties between equal slots are broken by the record's place in the slab (13 bits, so a record is one word
-  // while it is ranked); the runs of equal slots, few and short, are put right afterwards
-  static_assert(kSlabCap <= (1 << 13), "slab places in 13 bits");
-  uint32_t n = 0;
-  if (!slab_rank<kSortBlock>(sh, geo, 13, off, pos, live, rank, &n)) {
-    if (threadIdx.x == 0) {
-      tb.cursor[b * kCursorPad] = 0;
-      atomicOr(status, ZEN_STAT_RETRY);
-      tb.bucket_n[b] = 0;
-      tb.removed_n[b] = 0;
-    }
-    for (int j = threadIdx.x; j < kSlabIndexLen; j += kSortBlock) tb.sub_index[(size_t)b * kSlabIndexLen + j] = 0;
-    return;
-  }
-  // every thread has read the slab's fill count (slab_rank synchronised); this workgroup was its only reader
+  __syncthreads();  // the bitmap is clear, and everybody has read the slab's fill count
   if (threadIdx.x == 0) tb.cursor[b * kCursorPad] = 0;
-  // the counters hold where every narrow range starts in the sorted bucket: every kSlabIndexStep-th goes to
-  // the index (before the counters' memory is used for the ties below)
-  for (int j = threadIdx.x; j < kSlabIndexLen; j += kSortBlock)
-    tb.sub_index[(size_t)b * kSlabIndexLen + j] = (uint16_t)sh.cnt[sub_place<kSortBlock>((uint32_t)j * kSlabIndexStep)];
+  // no branch around a wave's marks either: a lane without a record marks nothing
+#pragma unroll
+  for (int i = 0; i < kSortItems; ++i) {
+    off[i] = rank[i] = 0;
+    if (row(i)) {
+      off[i] = geo.mod_m(poly(idx[i]) + kSeed1) - lo;  // the level-1 slot again: cheaper than carrying it along
+      if (!(live & (1u << i))) off[i] = 0;
+      rank[i] = sh.taken.take(off[i], (live >> i) & 1u);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kSortItems; ++i)
+    if ((live & (1u << i)) && !((rank[i] >> (off[i] & 31u)) & 1u)) owner |= 1u << i;  // the first to mark its slot
+  if (owner != live) sh.shared = 1;
+  __syncthreads();
+  const uint32_t n = sh.taken.template count<kSortBlock>(words, sh.scan);
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kSortItems; ++i) {
-    if (live & (1u << i)) {
-      sh.key[rank[i]] = off[i];
-      sh.tie[rank[i]] = idx[i];
-      s_val[rank[i]] = val[i];
+    if (row(i)) {
+      rank[i] = sh.taken.place(off[i]);
+      if (owner & (1u << i)) sh.idx[rank[i]] = idx[i];
     }
   }
-  __syncthreads();
-  // a run of equal slots gets its smallest index in front (the thread at the run's first place does it)
-  for (uint32_t p = threadIdx.x; p + 1 < n; p += kSortBlock) {
-    const uint32_t k = sh.key[p];
-    if (sh.key[p + 1] == k && (p == 0 || sh.key[p - 1] != k)) {
-      uint32_t best = p;
-      for (uint32_t u = p + 1; u < n && sh.key[u] == k; ++u)
-        if (sh.tie[u] < sh.tie[best]) best = u;
-      if (best != p) {
-        const uint32_t ti = sh.tie[p];
-        const S tv = s_val[p];
-        sh.tie[p] = sh.tie[best];
-        s_val[p] = s_val[best];
-        sh.tie[best] = ti;
-        s_val[best] = tv;
-      }
-    }
+  // every kSlabIndexStep-th narrow range's first sorted place goes to the index
+  for (int j = threadIdx.x; j < kSlabIndexLen; j += kSortBlock) {
+    const uint32_t first = (uint32_t)j * kSlabIndexStep << geo.sub_shift;
+    tb.sub_index[(size_t)b * kSlabIndexLen + j] = (uint16_t)(first < geo.span ? sh.taken.place(first) : n);
   }
   __syncthreads();
-  // In a run of equal slots the first entry has the smallest index: the slot's level-1 owner.  The others
-  // lost level 1.  Their places in the sorted slab are collected where the slots were, once every thread has
-  // looked at those (a bucket has at most kSlabSubs of them, else the call is declined).
-  uint32_t lost_mask = 0;
-#pragma unroll 1
-  for (int i = 0; i < kSortItems; ++i) {
-    const uint32_t p = threadIdx.x + (uint32_t)i * kSortBlock;
-    if (p < n) {
-      const uint32_t k = sh.key[p];
-      const bool lost = p > 0 && sh.key[p - 1] == k;
-      tb.slab_idx[base + p] = (int32_t)(sh.tie[p] | (lost ? kRemovedBit : 0u));
-      slab_val[base + p] = s_val[p];  // every thread has read its records: in place is safe
-      lost_mask |= lost ? 1u << i : 0u;
-    }
+  if (sh.shared) {  // (the same for the whole workgroup)
+#pragma unroll
+    for (int i = 0; i < kSortItems; ++i)
+      if ((live & ~owner) & (1u << i)) atomicMin(&sh.idx[rank[i]], idx[i]);
+    __syncthreads();
+    owner = 0;
+#pragma unroll
+    for (int i = 0; i < kSortItems; ++i)
+      if ((live & (1u << i)) && sh.idx[rank[i]] == idx[i]) owner |= 1u << i;
   }
+  const uint32_t losers = live & ~owner;
+  uint32_t at = losers ? atomicAdd(&sh.lost, (uint32_t)__popc(losers)) : 0u;
+#pragma unroll
+  for (int i = 0; i < kSortItems; ++i)
+    if (owner & (1u << i)) sh.val[rank[i]] = val[i];  // (the bitmap has done its work)
   __syncthreads();
-#pragma unroll 1
-  for (int i = 0; i < kSortItems; ++i) {
-    if (lost_mask & (1u << i)) {
-      const uint32_t at = atomicAdd(&s_lost, 1u);
-      if (at < (uint32_t)kSlabSubs) sh.key[at] = threadIdx.x + (uint32_t)i * kSortBlock;
-    }
-  }
-  __syncthreads();
-  uint32_t lost_n = s_lost;
-  if (lost_n > (uint32_t)kSlabSubs) {
-    if (threadIdx.x == 0) atomicOr(status, ZEN_STAT_RETRY);
-    lost_n = kSlabSubs;
-  }
   if (threadIdx.x == 0) {
     tb.bucket_n[b] = n;
-    tb.removed_n[b] = lost_n;
-    s_base = lost_n ? atomicAdd(tb.losers, lost_n) : 0u;
+    tb.removed_n[b] = 0;
+    sh.base = sh.lost ? atomicAdd(tb.losers, sh.lost) : 0u;
+  }
+  for (uint32_t p = threadIdx.x; p < n; p += kSortBlock) {
+    tb.slab_idx[base + p] = (int32_t)sh.idx[p];
+    slab_val[base + p] = sh.val[p];
   }
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < lost_n; i += kSortBlock) {
-    const uint32_t at = s_base + i;
-    const uint32_t p = sh.key[i];
-    if (at < tb.log_cap)
-      tb.log_t[at] = sh.tie[p];
-    else
-      atomicOr(status, ZEN_STAT_RETRY);
+  at += sh.base;
+#pragma unroll
+  for (int i = 0; i < kSortItems; ++i) {
+    if (losers & (1u << i)) {
+      if (at < tb.log_cap)
+        tb.log_t[at] = idx[i];
+      else
+        atomicOr(status, ZEN_STAT_RETRY);
+      ++at;
+    }
   }
 }
 
@@ -421,187 +418,126 @@ __global__ __launch_bounds__(kSlabBlock) void k_slab_chains(SlabGeom geo, Probe 
 
 // ------------------------------------------------------------------ place
 
-// The sorted slab of a bucket is almost its part of the output already: the entries that lost their slot
-// drop out and the entries that moved in from elsewhere slip in between.  So an entry at sorted place p goes to
-//     bucket start + p - (removed entries before p) + (moved-in entries in front of it).
-// A wave's 64 consecutive places are one stretch: how many of its entries in front of a lane's are removed is a
-// ballot, how many moved-in ones slip in there a prefix sum across the lanes, and the stretches' sums are chained
-// once per bucket.  Consecutive lanes read consecutive entries and write (almost) consecutive places.  (Both counts
-// as bisections of sorted lists: 100 us for 6.2 M entries of which 5 % had moved.)
-template <typename S>
-__global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, SlabTables tb, unsigned long long *cells,
+// A bucket's part of the output is its taken slots in order: the owners that nobody pushed out and the entries that moved
+// in.  Both are marked in a bitmap of the slots, and an entry goes to the bucket's start plus the number of marks below
+// its own.  Consecutive lanes read consecutive entries and write (almost) consecutive places.  (Removed and moved-in
+// entries counted per stretch of 64 sorted places, with a bisection for every moved-in one: 62 M slots, 6.2 M records, 5 %
+// moved: 63 us, now 48; both counts as bisections of sorted lists: 100.)
+template <uint32_t SPAN>
+struct SlabPlaceLds {
+  union {
+    SlabTaken<SPAN> taken;
+    uint32_t serial[kSlabSerialCap];
+  };
+  uint32_t scan[kSlabBlock / 64 + 1];
+};
+
+template <typename S, uint32_t SPAN>
+__global__ __launch_bounds__(kSlabBlock, SPAN <= kSlabSpan2 ? 6 : 2) void k_slab_place(SlabGeom geo, SlabTables tb, unsigned long long *cells,
                                                            int64_t spp, const S *__restrict__ dense,
                                                            int32_t *__restrict__ out_idx, S *__restrict__ out_val,
                                                            uint32_t capacity, int64_t *__restrict__ splits,
                                                            int32_t *status) {
-  constexpr int kStretches = kSlabCap / 64;
   constexpr int kCells = (1 << kSlabPartLog2) / kSlabBlock;
-  static_assert(kStretches <= 128, "two stretches per lane of a wave");
-  __shared__ uint32_t s_key[kSlabCap];                 // sorted slots of the bucket
-  __shared__ uint32_t s_cnt[kSlabCap / 2 + 1];         // per sorted place, 16 bits each: the moved-in entries right in
-  uint16_t *s_front = reinterpret_cast<uint16_t *>(s_cnt);  // front of it, then those before it in its stretch
-  __shared__ uint32_t s_mk[1 << kSlabPartLog2];        // the moved-in entries' slots, by the place they slip in at
-  __shared__ uint64_t s_mask[kStretches];              // per stretch: its removed entries
-  __shared__ uint32_t s_mv[kStretches], s_rm[kStretches];  // moved-in and removed entries of the stretches before
-  __shared__ uint32_t s_nrm;
+  __shared__ SlabPlaceLds<SPAN> sh;
   const uint32_t b = blockIdx.x;
   const uint32_t B = geo.nbuckets;
   const size_t base = (size_t)b * kSlabCap;
+  const uint32_t words = (geo.span + 63u) / 64u;
   const S *slab_val = static_cast<const S *>(tb.slab_val);
   const uint32_t *serial_n = tb.final_n + B;
   const uint32_t n = tb.bucket_n[b];
   // what the bucket's part of the map holds has moved in, and keeps to the thread that finds it; the part goes
   // back empty
   const uint32_t mv_n = tb.final_n[b];
+  const uint32_t lo = tb.bucket_lo[b];
   const uint32_t out_base = tb.out_start[b];
-  const uint32_t out_n = tb.out_start[b + 1] - out_base;
   unsigned long long *cell = cells + ((size_t)b << kSlabPartLog2) + threadIdx.x;
   unsigned long long moved[kCells];
 #pragma unroll
   for (int e = 0; e < kCells; ++e) moved[e] = mv_n ? cell[e * kSlabBlock] : 0ull;
-  // the thread's entries (sorted places threadIdx.x + i * kSlabBlock) stay in registers; the slots go to LDS
-  // for the searches
   uint32_t idx[kSlabItems];
   S val[kSlabItems];
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
     const uint32_t p = threadIdx.x + i * kSlabBlock;
+    idx[i] = kRemovedBit;
+    val[i] = 0;
+    if ((uint32_t)(i * kSlabBlock) >= n) continue;  // the same for the whole workgroup
     idx[i] = (uint32_t)tb.slab_idx[base + (p < n ? p : 0u)];
     val[i] = slab_val[base + (p < n ? p : 0u)];
+    if (p >= n) idx[i] = kRemovedBit;
   }
+  sh.taken.template clear<kSlabBlock>(words);
   S mval[kCells];  // an entry is a copy of the element it stands for
 #pragma unroll
   for (int e = 0; e < kCells; ++e) mval[e] = mv_n ? dense[(uint32_t)moved[e]] : S(0);
-  if (threadIdx.x == 0) s_nrm = 0;
-  for (int i = threadIdx.x; i < kSlabCap / 2 + 1; i += kSlabBlock) s_cnt[i] = 0;
+  __syncthreads();
+  uint32_t off[kSlabItems], moff[kCells];
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
-    const uint32_t p = threadIdx.x + i * kSlabBlock;
-    if (p < n) s_key[p] = geo.mod_m(poly(idx[i] & kIndexMask) + kSeed1);
+    off[i] = 0;
+    if ((uint32_t)(i * kSlabBlock) < n && !(idx[i] & kRemovedBit)) {
+      off[i] = geo.mod_m(poly(idx[i]) + kSeed1) - lo;
+      sh.taken.take(off[i], 1u);
+    }
   }
-  __syncthreads();
-  // a moved-in entry's place: the sorted place in front of which it slips in, and its turn among those that slip
-  // in there too
-  uint32_t mplace[kCells], mturn[kCells];
 #pragma unroll
   for (int e = 0; e < kCells; ++e) {
-    mplace[e] = mturn[e] = 0;
+    moff[e] = 0;
     if (moved[e]) {
       cell[e * kSlabBlock] = 0ull;
-      mplace[e] = lower_bound_u32(s_key, n, (uint32_t)(moved[e] >> 32) - 1u);
-      const uint32_t shift = 16u * (mplace[e] & 1u);
-      mturn[e] = (atomicAdd(&s_cnt[mplace[e] >> 1], 1u << shift) >> shift) & 0xffffu;
+      moff[e] = (uint32_t)(moved[e] >> 32) - 1u - lo;
+      sh.taken.take(moff[e], 1u);
     }
   }
   __syncthreads();
-  uint32_t in_front[kSlabItems];  // moved-in entries of the stretch that slip in at or before the entry's place
-  uint32_t removed = 0;           // bit i: entry i has lost its slot
+  const uint32_t own_n = sh.taken.template count<kSlabBlock>(words, sh.scan);  // survivors + moved-in
+  __syncthreads();
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
-    const uint32_t p = threadIdx.x + i * kSlabBlock;
-    in_front[i] = 0;
-    if ((uint32_t)(i * kSlabBlock) > n) {  // the same for the whole workgroup: nothing beyond the entries
-      if (lane_id() == 63) s_mv[p >> 6] = s_rm[p >> 6] = 0;
-      continue;
-    }
-    const bool gone = p < n && (idx[i] & kRemovedBit);
-    const uint64_t m = __ballot(gone);
-    removed |= (gone ? 1u : 0u) << i;
-    if (mv_n) {
-      const uint32_t c = s_front[p];
-      in_front[i] = wave_inclusive_scan(c);
-      s_front[p] = (uint16_t)(in_front[i] - c);
-    }
-    if (lane_id() == 63) {
-      s_mask[p >> 6] = m;
-      s_mv[p >> 6] = in_front[i];
-      s_rm[p >> 6] = (uint32_t)__popcll(m);
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x < 64) {
-    const int l = threadIdx.x;
-    const uint32_t v0 = s_mv[l], v1 = l + 64 < kStretches ? s_mv[l + 64] : 0u;
-    const uint32_t r0 = s_rm[l], r1 = l + 64 < kStretches ? s_rm[l + 64] : 0u;
-    const uint32_t iv0 = wave_inclusive_scan(v0), iv1 = wave_inclusive_scan(v1);
-    const uint32_t ir0 = wave_inclusive_scan(r0), ir1 = wave_inclusive_scan(r1);
-    const uint32_t tv = __shfl(iv0, 63, 64), tr = __shfl(ir0, 63, 64);
-    s_mv[l] = iv0 - v0;
-    s_rm[l] = ir0 - r0;
-    if (l + 64 < kStretches) {
-      s_mv[l + 64] = tv + iv1 - v1;
-      s_rm[l + 64] = tr + ir1 - r1;
-    }
-    if (l == 63) s_nrm = tr + ir1;
-  }
-  __syncthreads();
-  // survivors
-#pragma unroll
-  for (int i = 0; i < kSlabItems; ++i) {
-    const uint32_t p = threadIdx.x + i * kSlabBlock;
-    if ((uint32_t)(i * kSlabBlock) >= n) break;
-    const uint64_t m = __ballot((removed >> i) & 1u);
-    if (p < n && !((removed >> i) & 1u)) {
-      const uint32_t before = (uint32_t)__popcll(m & lanes_below());
-      const uint32_t pos = out_base + p + s_mv[p >> 6] + in_front[i] - s_rm[p >> 6] - before;
+    if ((uint32_t)(i * kSlabBlock) < n && !(idx[i] & kRemovedBit)) {
+      const uint32_t pos = out_base + sh.taken.place(off[i]);
       if (pos < capacity) {
         out_idx[pos] = (int32_t)idx[i];
         out_val[pos] = val[i];
       }
     }
   }
-  if (mv_n) {  // the same for the whole workgroup
-    // the moved-in entries by the place they slip in at; several at one place (two at times) by ascending slot
-    const auto front = [&](uint32_t p) -> uint32_t {  // moved-in entries before those of place p
-      return p < (uint32_t)kSlabCap ? s_mv[p >> 6] + s_front[p] : p > (uint32_t)kSlabCap ? mv_n : mv_n - s_front[kSlabCap];
-    };
 #pragma unroll
-    for (int e = 0; e < kCells; ++e)
-      if (moved[e]) s_mk[front(mplace[e]) + mturn[e]] = (uint32_t)(moved[e] >> 32) - 1u;
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < kCells; ++e) {
-      if (moved[e]) {
-        const uint32_t at = mplace[e], key = (uint32_t)(moved[e] >> 32) - 1u;
-        const uint32_t first = front(at), end = front(at + 1u);
-        uint32_t rank = first;
-        for (uint32_t u = first; u < end; ++u) rank += s_mk[u] < key;
-        const uint32_t gone =
-            at < n ? s_rm[at >> 6] + (uint32_t)__popcll(s_mask[at >> 6] & ((1ull << (at & 63u)) - 1ull)) : s_nrm;
-        const uint32_t pos = out_base + at + rank - gone;
-        if (pos < capacity) {
-          out_idx[pos] = (int32_t)(uint32_t)moved[e];
-          out_val[pos] = mval[e];
-        }
+  for (int e = 0; e < kCells; ++e) {
+    if (moved[e]) {
+      const uint32_t pos = out_base + sh.taken.place(moff[e]);
+      if (pos < capacity) {
+        out_idx[pos] = (int32_t)(uint32_t)moved[e];
+        out_val[pos] = mval[e];
       }
     }
   }
   const uint32_t part = b / geo.bpp;
-  const bool last_of_part = b % geo.bpp == geo.bpp - 1;
   uint32_t serial = 0;
-  if (last_of_part) {
+  if (b % geo.bpp == geo.bpp - 1) {  // the partition's last bucket
     serial = serial_n[part];
     if (serial > (uint32_t)kSlabSerialCap) serial = kSlabSerialCap;
   }
-  const uint32_t own_n = out_n - serial;  // survivors + moved-in
   if (serial) {
     // the partition's overflow entries in ascending index order (the reference hands its tickets to
     // ascending thread ids, functions_cuda_kernel.cu:107-108), behind everything that found a slot
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < serial; i += kSlabBlock) s_key[i] = tb.ser_idx[(size_t)part * kSlabSerialCap + i];
+    for (uint32_t i = threadIdx.x; i < serial; i += kSlabBlock) sh.serial[i] = tb.ser_idx[(size_t)part * kSlabSerialCap + i];
     __syncthreads();
-    sort_network(s_key, serial);
+    sort_network(sh.serial, serial);
     for (uint32_t i = threadIdx.x; i < serial; i += kSlabBlock) {
       const uint32_t pos = out_base + own_n + i;
       if (pos < capacity) {
-        out_idx[pos] = (int32_t)s_key[i];
-        out_val[pos] = dense[s_key[i]];
+        out_idx[pos] = (int32_t)sh.serial[i];
+        out_val[pos] = dense[sh.serial[i]];
       }
     }
   }
   if (b % geo.bpp == 0 && threadIdx.x == 0) {
-    const uint32_t lo = tb.out_start[b], hi = tb.out_start[b + geo.bpp];
-    splits[part] = (int64_t)(hi - lo);
+    const uint32_t lo_at = tb.out_start[b], hi = tb.out_start[b + geo.bpp];
+    splits[part] = (int64_t)(hi - lo_at);
     if ((int64_t)serial_n[part] > spp) atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
     if (hi > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
   }
@@ -667,8 +603,8 @@ SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partit
   return p;
 }
 
-template <typename S>
-int slab_launch(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPlan &p, hipStream_t s) {
+template <typename S, uint32_t SPAN>
+int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPlan &p, hipStream_t s) {
   const uint32_t B = geo.nbuckets;
   const uint32_t *filter = a.k > 0 ? p.thr : nullptr;
   const S *dense = static_cast<const S *>(a.input);
@@ -682,7 +618,7 @@ int slab_launch(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPlan &p
   }
   {
     ProfScope prof(kProfSlabSort, s);
-    k_slab_sort<S><<<dim3(B), dim3(kSortBlock), 0, s>>>(geo, p.tb, a.status);
+    k_slab_sort<S, SPAN><<<dim3(B), dim3(kSortBlock), 0, s>>>(geo, p.tb, a.status);
     ZEN_LAUNCH_CHECK("k_slab_sort");
   }
   {
@@ -695,19 +631,31 @@ int slab_launch(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPlan &p
   }
   {
     ProfScope prof(kProfSlabPlace, s);
-    k_slab_place<S><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, a.spp, dense, a.out_idx,
-                                                         static_cast<S *>(a.out_val), (uint32_t)a.capacity, a.splits,
-                                                         a.status);
+    k_slab_place<S, SPAN><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, a.spp, dense, a.out_idx,
+                                                               static_cast<S *>(a.out_val), (uint32_t)a.capacity,
+                                                               a.splits, a.status);
     ZEN_LAUNCH_CHECK("k_slab_place");
   }
   return ZEN_OK;
+}
+
+template <typename S>
+int slab_launch(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPlan &p, hipStream_t s) {
+  if (geo.span <= kSlabSpan1) return slab_launch_span<S, kSlabSpan1>(a, geo, p, s);
+  if (geo.span <= kSlabSpan2) return slab_launch_span<S, kSlabSpan2>(a, geo, p, s);
+  return slab_launch_span<S, kSlabSpan3>(a, geo, p, s);
+}
+
+bool encode_geometry(int64_t m, int partitions, int64_t capacity, SlabGeom *geo) {
+  // (a few thousand keys below the width: the divisions round the buckets up)
+  return slab_geometry(m, partitions, capacity, kSlabTarget, (int64_t)kSlabSpan2 - 4096, kSlabSpan3, geo);
 }
 
 }  // namespace
 
 size_t slab_balance_bytes(int64_t m, int partitions, int dtype, int64_t capacity) {
   SlabGeom geo;
-  if (!slab_geometry(m, partitions, capacity, kSlabTarget, &geo)) return 0;
+  if (!encode_geometry(m, partitions, capacity, &geo)) return 0;
   return plan_slab(nullptr, nullptr, geo, partitions, dtype, list_capacity(capacity)).bytes;
 }
 
@@ -720,7 +668,7 @@ bool slab_balance_fits(int64_t n, int64_t m, int partitions, int dtype, int64_t 
   (void)k;
   if (capacity > 0x1fffffffll) return false;
   SlabGeom g;
-  if (!slab_geometry(m, partitions, capacity, kSlabTarget, &g)) return false;
+  if (!encode_geometry(m, partitions, capacity, &g)) return false;
   // slab_geometry wants m >= 2^22: a table of 16 MB or more, of which the map takes at most half and the
   // counters less than 1 MB
   if (geo) *geo = g;
