@@ -53,16 +53,6 @@ __device__ inline uint32_t vec_pick(const uint4 &q, uint32_t e, uint32_t) {
   return e & 2u ? b : a;
 }
 
-__device__ inline uint32_t scan_dpp(uint32_t x) {  // inclusive prefix sum across the 64 lanes
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);
-  return x;
-}
-
 // Sixteen bytes from an address that is a multiple of 16 or, !ALIGNED, of an element's size only (a view that begins
 // at an odd element): one load either way.
 template <typename S, bool ALIGNED>
@@ -123,7 +113,7 @@ __device__ __forceinline__ uint32_t walk(const S *__restrict__ in, int64_t begin
   auto two = [&](const uint4 &q0, const uint4 &q1, uint32_t first) {
     const uint32_t x0 = vec_flags(q0, least, S(0)), x1 = vec_flags(q1, least, S(0));
     const uint32_t c = (uint32_t)__popc(x0) | ((uint32_t)__popc(x1) << 16);
-    const uint32_t incl = scan_dpp(c);
+    const uint32_t incl = wave_inclusive_scan(c);
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
     if (WRITE) {
       const uint32_t before = incl - c;

@@ -377,17 +377,6 @@ __global__ __launch_bounds__(256) void k_compress(const S *__restrict__ in, int6
 constexpr int kSelStage = 3072;    // staged pairs per tile
 constexpr int kReserveShift = 40;  // tiles done above, entries reserved below
 
-// Inclusive prefix sum across the 64 lanes with DPP row shifts and broadcasts.
-__device__ inline uint32_t wave_inclusive_scan_dpp(uint32_t x) {
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);  // row_shr:2
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);  // row_shr:4
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);  // row_shr:8
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15 -> rows 1,3
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31 -> rows 2,3
-  return x;
-}
-
 // Flags of the elements a thread owns in one sub-tile, one bit per element,
 // plus the translation between bit positions and element offsets.
 template <typename S>
@@ -488,7 +477,7 @@ __device__ inline uint32_t select_walk_tile(const S *__restrict__ in, int64_t n,
     if (first + kChunk > n) x &= first < n ? Flags<S>::below((int)(n - first)) : 0u;
     const uint32_t cnt = (uint32_t)__popc(x);
     // block-wide exclusive prefix of cnt
-    const uint32_t incl = wave_inclusive_scan_dpp(cnt);
+    const uint32_t incl = wave_inclusive_scan(cnt);
     if ((threadIdx.x & 63) == 63) s_wave[wave] = incl;
     __syncthreads();
     uint32_t before = running + incl - cnt, total = 0;
@@ -1111,7 +1100,7 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
       for (int j = 0; j < kSelVecs; ++j) reinterpret_cast<uint4 *>(s_tile)[j * kSelBlock + threadIdx.x] = cur[j];
     }
     const uint32_t cnt = (uint32_t)__popc(x);
-    const uint32_t incl = wave_inclusive_scan_dpp(cnt);
+    const uint32_t incl = wave_inclusive_scan(cnt);
     if ((threadIdx.x & 63) == 63) s_wave[par & 1][wave] = incl;
     const bool hand_over = ticket_pending && sub + 1 == cur_len;
     if (hand_over && threadIdx.x == 0) s_next[turn & 1] = drawn;

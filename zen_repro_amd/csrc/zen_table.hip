@@ -27,16 +27,6 @@ constexpr uint32_t kOneSlots = 32768;                       // 128 KB of LDS
 constexpr int kOneParts = 256;
 constexpr uint32_t kOneSerial = 3456;                       // more than a tenth of kOneSlots: more would be an overflow
 
-__device__ inline uint32_t scan64(uint32_t x) {  // inclusive prefix sum across the 64 lanes
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);
-  return x;
-}
-
 // Inserts index t.  Returns the index that ends up without a slot (0: none) and its partition.
 __device__ inline uint32_t insert(uint32_t *table, const Probe &g, uint32_t t, uint32_t *part) {
   uint32_t cur = t;
@@ -93,7 +83,7 @@ __global__ __launch_bounds__(kInsBlock) void k_table_insert(const S *__restrict_
   for (int i = 0; i < V; ++i) flags |= (uint32_t)((uint32_t)(e[i] & KeyOf<S>::kMask) >= least) << i;
   if (first == 0) flags &= ~1u;  // index 0 is never transmitted
   const uint32_t c = (uint32_t)__popc(flags);
-  const uint32_t incl = scan64(c);
+  const uint32_t incl = wave_inclusive_scan(c);
   __syncthreads();
   uint32_t at = 0;
   if (lane_id() == 63 && incl) at = atomicAdd(&count, incl);
@@ -200,7 +190,7 @@ __global__ __launch_bounds__(kOutBlock) void k_table_out(const S *__restrict__ d
 #pragma unroll
   for (int r = 0; r < kOutRows; ++r) {
     const uint32_t x = occupied(q[r]);
-    const uint32_t n = (uint32_t)__popc(x), incl = scan64(n);
+    const uint32_t n = (uint32_t)__popc(x), incl = wave_inclusive_scan(n);
     uint32_t pos = at + incl - n;
     for (uint32_t bits = x; bits; bits &= bits - 1u, ++pos) {
       const uint32_t e = (uint32_t)__ffs((int)bits) - 1u;
@@ -325,7 +315,7 @@ __global__ __launch_bounds__(kOneBlock) void k_table_one(const S *__restrict__ i
   for (uint32_t r = 0; r < rows; ++r) {
     const uint32_t s0 = base + r * 256;
     const uint4 q = s0 < words ? *reinterpret_cast<const uint4 *>(slots + s0) : make_uint4(0, 0, 0, 0);
-    const uint32_t x = occupied(q), c = (uint32_t)__popc(x), incl = scan64(c);
+    const uint32_t x = occupied(q), c = (uint32_t)__popc(x), incl = wave_inclusive_scan(c);
     uint32_t pos = at + incl - c;
     for (uint32_t bits = x; bits; bits &= bits - 1u, ++pos) {
       const uint32_t e = (uint32_t)__ffs((int)bits) - 1u;
