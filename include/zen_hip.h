@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define ZEN_ABI_VERSION 6 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table; 4: zen_read_back, zen_count, zen_merge_rounded, zen_decode_dense_lists, zen_bitmap_dense_lists; 5: zen_table_find, zen_table_gather; 6: ZEN_MODE_NO_SAMPLES */
+#define ZEN_ABI_VERSION 7 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table; 4: zen_read_back, zen_count, zen_merge_rounded, zen_decode_dense_lists, zen_bitmap_dense_lists; 5: zen_table_find, zen_table_gather; 6: ZEN_MODE_NO_SAMPLES; 7: zen_load_balance_sizes, zen_merge_rounded_count */
 
 #define ZEN_F32 0
 #define ZEN_BF16 1
@@ -277,6 +277,21 @@ int zen_load_balance(const void *input, int dtype, int64_t n, int64_t m,
                      int32_t *status, void *stream);
 
 /*
+ * zen_load_balance for a caller that has to know the split sizes before it goes
+ * on (tensor_load_balance.py:46-50): returns when host[1 + p] = splits[p] and
+ * host[1 + partitions] = *status are there, of `words` words from
+ * zen_host_words_alloc (at least partitions + 2; one call at a time on a set of
+ * words).  The entries themselves are complete on the stream, as always, and
+ * may still be on their way to their places when the call returns.
+ */
+int zen_load_balance_sizes(const void *input, int dtype, int64_t n, int64_t m,
+                           int partitions, int rehash, const uint32_t *thr, int64_t k,
+                           uint32_t *thr_out, int32_t *out_idx, void *out_val,
+                           int64_t capacity, int64_t *splits, int32_t *table, int mode,
+                           void *workspace, size_t workspace_bytes, int32_t *status,
+                           int64_t *host, int64_t words, void *stream);
+
+/*
  * The part of a top-k zen_load_balance call (k > 0, ZEN_MODE_FAST) that only needs the tensor: the sample
  * that gives the one-pass selection its floor.  Taken ahead, on another stream, it runs beside whatever the
  * main stream is still busy with (the previous gradient bucket's sort and placement, say) instead of in front
@@ -337,6 +352,18 @@ int zen_merge_rounded(const void *idx, int idx64_in, const void *val, int dtype,
                       void *out_idx, int idx64_out, void *out_val, int64_t capacity,
                       int64_t *out_count, int mode, void *workspace, size_t workspace_bytes,
                       int32_t *status, void *stream);
+
+/*
+ * The same for a caller that has to know the entries' number before it goes on:
+ * returns when host[1] = *out_count and host[2] = *status are there, of `words`
+ * words from zen_host_words_alloc (at least 3).  The outputs are complete on
+ * the stream, as always.
+ */
+int zen_merge_rounded_count(const void *idx, int idx64_in, const void *val, int dtype,
+                            int64_t r, int64_t dense_n,
+                            void *out_idx, int idx64_out, void *out_val, int64_t capacity,
+                            int64_t *out_count, int mode, void *workspace, size_t workspace_bytes,
+                            int32_t *status, int64_t *host, int64_t words, void *stream);
 
 /*
  * The merged entries on their way to the second exchange: comm.py:125-127

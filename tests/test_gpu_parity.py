@@ -1029,3 +1029,44 @@ def test_merge_of_short_lists(zen, oracle, r, n, copies, dtype):
         dense = torch.zeros(n, dtype=dv.dtype)
         dense[torch.from_numpy(mi).long()] = want
         assert torch.equal(lba.decode_sparse_tensors(di, dv, n).cpu(), dense)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("n,P,flags", [
+    (3000, 5, 0),               # one workgroup
+    (300000, 7, 0),             # the owner table
+    (6000000, 3, 0),            # wide buckets
+    (6000000, 3, "slabs"),      # bucket slabs: the sizes come before the entries are in their places
+    (300000, 600, "general"),
+])
+def test_sizes_the_host_is_told_by_the_calls_own_kernels(zen, oracle, n, P, flags, dtype):
+    from zen_repro_amd import _lib
+
+    mode = {0: None, "slabs": _lib.MODE_FAST | _lib.MODE_SLABS, "general": _lib.MODE_GENERAL}[flags]
+    g = make_grad(oracle, n, 0.05, dtype, seed=n + P)
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, 3)
+    assert st_o == 0
+    tp = zen.TensorPartition(P, 1, 3)
+    d = to_dev(g)
+    for rep in range(3):  # the same words are asked again
+        indices, values, splits = tp.load_balance(d, mode=mode)
+        assert [t.numel() for t in indices] == [t.numel() for t in values] == splits_o.tolist()
+        assert np.array_equal(to_np(splits), splits_o)
+        assert np.array_equal(to_np(torch.cat(indices)), idx_o) and np.array_equal(to_np(torch.cat(values)), val_o)
+        zeros = tp.load_balance(torch.zeros_like(d), mode=mode)
+        assert [t.numel() for t in zeros[0]] == [0] * P and not zeros[2].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("r,n", [(0, 1000), (1, 1000), (3000, 20000), (20000, 40000), (200000, 1 << 23)])
+def test_count_the_host_is_told_by_the_merge(zen, r, n, dtype):
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    gen = torch.Generator(device="cuda").manual_seed(r + n)
+    idx = torch.randint(0, n, (r,), generator=gen, device="cuda", dtype=torch.int32)
+    val = torch.randint(1, 4, (r,), generator=gen, device="cuda").to(dtype)  # sums are exact
+    want = torch.zeros(n, device="cuda").scatter_add_(0, idx.long(), val.float())
+    at = torch.nonzero(want).view(-1)
+    for flags in (0, zen._lib.MODE_SLABS):
+        lba.fast_flags = flags
+        got_idx, got_val = lba.merge_rounded(idx, val, n, dtype)
+        assert torch.equal(got_idx, at) and torch.equal(got_val, want[at].to(dtype))

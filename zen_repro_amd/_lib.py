@@ -24,7 +24,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("ZEN_HIP_LIB") or os.path.join(_HERE, "csrc", "libzen_hip.so")
 
 # ZEN_ABI_VERSION of include/zen_hip.h this loader's signatures and structs are written for
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 _lib = None
 
@@ -92,6 +92,8 @@ def lib():
         "zen_select": (i32, [vp, i32, i64, vp, vp, i32, vp, i64, vp, vp, sz, vp, vp]),
         "zen_load_balance_workspace": (sz, [i64, i64, i32, i64, i32]),
         "zen_load_balance": (i32, [vp, i32, i64, i64, i32, i32, vp, i64, vp, vp, vp, i64, vp, vp, i32, vp, sz, vp, vp]),
+        "zen_load_balance_sizes": (i32, [vp, i32, i64, i64, i32, i32, vp, i64, vp, vp, vp, i64, vp, vp, i32, vp, sz, vp, vp, i64,
+                                         vp]),
         "zen_load_balance_prepare": (i32, [vp, i32, i64, i64, i32, i64, i64, vp, i32, vp, sz, vp]),
         "zen_load_balance_path": (i32, [i64, i64, i32, i64, i32, i64, i32]),
         "zen_merge_workspace": (sz, [i64, i64]),
@@ -100,6 +102,7 @@ def lib():
         "zen_merge": (i32, [vp, i32, vp, i32, i64, i64, vp, i32, vp, i64, vp, i32, vp, sz, vp, vp]),
         "zen_encode_merge": (i32, [ctypes.POINTER(EncodeMergeArgs)]),
         "zen_merge_rounded": (i32, [vp, i32, vp, i32, i64, i64, vp, i32, vp, i64, vp, i32, vp, sz, vp, vp]),
+        "zen_merge_rounded_count": (i32, [vp, i32, vp, i32, i64, i64, vp, i32, vp, i64, vp, i32, vp, sz, vp, vp, i64, vp]),
         "zen_decode_dense_lists": (i32, [ctypes.POINTER(vp), i32, ctypes.POINTER(vp), i32, ctypes.POINTER(i64), i32, vp, i64, vp,
                                          sz, vp, vp]),
         "zen_decode_dense_workspace": (sz, [i64, i64]),
@@ -378,6 +381,17 @@ _NO_SEGMENT = [(None, 0, 0) * (3 - n) for n in range(4)]
 _READ_BACK_MOST = 1 << 16
 
 
+def host_words(n):
+    """This host thread's pinned words, with room for `n` (at most _READ_BACK_MOST) of an answer."""
+    try:
+        words = _host.words
+    except AttributeError:
+        words = None
+    if words is None or words.words <= n:
+        words = _host.words = _HostWords(max(1024, min(2 * n, _READ_BACK_MOST + 1)))
+    return words
+
+
 def read_back(*tensors):
     """The values of up to three small contiguous int32 / int64 device tensors (split sizes, counts, status
     words), one list after the other, once the current stream has got there.  The way a call on this path
@@ -391,12 +405,7 @@ def read_back(*tensors):
     if n > _READ_BACK_MOST:
         return [word for t in tensors for word in t.tolist()]
     args += _NO_SEGMENT[len(tensors)]
-    try:
-        words = _host.words
-    except AttributeError:
-        words = None
-    if words is None or words.words <= n:
-        words = _host.words = _HostWords(max(1024, min(2 * n, _READ_BACK_MOST + 1)))
+    words = host_words(n)
     rc = _lib.zen_read_back(*args, words.ptr, words.words, stream_handle(tensors[0].device))
     if rc:
         check(rc, "read_back")

@@ -196,8 +196,9 @@ class LoadBalanceAllreduce:
         (a slot owns its workspace)."""
         return self._merge(indices_tensors, values_tensors, dense_size, capacity, idx64, mode, slot, False)
 
-    def _merge(self, indices_tensors, values_tensors, dense_size, capacity, idx64, mode, slot, rounded):
-        """merge_sparse_flat; `rounded`: the sums leave in the values' type (zen_merge_rounded)."""
+    def _merge(self, indices_tensors, values_tensors, dense_size, capacity, idx64, mode, slot, rounded, words=None):
+        """merge_sparse_flat; `rounded`: the sums leave in the values' type (zen_merge_rounded), and with `words` (of
+        _lib.host_words) the count and the status are there when this returns."""
         indices = self.stack_tensors(indices_tensors)
         values = self.stack_tensors(values_tensors)
         _lib.require_gpu(indices, "indices")
@@ -216,10 +217,13 @@ class LoadBalanceAllreduce:
         # The workspace is allocated zeroed and serves zen_merge only, which leaves its head (the counters
         # that must start at zero) zero again: no call spends a kernel on clearing it.
         ws = _lib.scratch.get(dev, f"merge/{slot}", L.zen_merge_workspace(r, dense_size), zero=True)
-        rc = (L.zen_merge_rounded if rounded else L.zen_merge)(
-            _lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(values), _lib.dtype_code(values), r,
-            dense_size, _lib.ptr(out_idx), 1 if idx64 else 0, _lib.ptr(out_val), capacity, _lib.ptr(count),
-            mode | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status), _lib.stream_of(dev))
+        args = (_lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(values), _lib.dtype_code(values), r,
+                dense_size, _lib.ptr(out_idx), 1 if idx64 else 0, _lib.ptr(out_val), capacity, _lib.ptr(count),
+                mode | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status))
+        if words is not None:
+            rc = L.zen_merge_rounded_count(*args, words.ptr, words.words, _lib.stream_of(dev))
+        else:
+            rc = (L.zen_merge_rounded if rounded else L.zen_merge)(*args, _lib.stream_of(dev))
         if rc != _lib.OK:
             ws[:L.zen_merge_zero_bytes()].zero_()
         _lib.check(rc, "merge_sparse")
@@ -375,13 +379,14 @@ class LoadBalanceAllreduce:
         values_tensors = self.stack_tensors(values_tensors)
         rounded = values_tensors.dtype == dtype
         for mode in self._fast_then_general():
+            words = _lib.host_words(2) if rounded else None
             idx, val, count, status = self._merge(indices_tensors, values_tensors, dense_size, None, True, mode, 0,
-                                                  rounded)
+                                                  rounded, words)
             if rounded:
-                r_status = status
+                host = words.view[1:3] + [0]
             else:
                 idx, val, count, r_status = self.round_merged_flat(idx, val, count, dtype)
-            host = _lib.read_back(count, status, r_status)
+                host = _lib.read_back(count, status, r_status)
             if host[1] & (_lib.STAT_RETRY | _lib.STAT_INTERNAL):
                 self.reset_merge_workspace(idx.device)
             if not host[1] & _lib.STAT_RETRY:

@@ -148,6 +148,7 @@ struct SlabBalanceArgs {
   void *next_state = nullptr;        // the zero-between-calls memory in the next call's table (null: this call's)
   bool second = false;        // the call's sample uses the second set of sampling memory (always so with prepared == 2)
   bool only_prepare = false;  // take the sample for that set and nothing else
+  HostAsk ask;                // the split sizes, then the status word, for the host
   bool discard = false;       // with only_prepare: clear the set's sampling memory instead (a sample nobody picks up)
 };
 bool slab_balance_fits(int64_t n, int64_t m, int partitions, int dtype, int64_t capacity, int64_t k, SlabGeom *geo);

@@ -444,7 +444,8 @@ int load_balance_call(const void *input, int dtype, int64_t n, int64_t m, int pa
                       const uint32_t *thr, int64_t k, uint32_t *thr_out, int32_t *out_idx, void *out_val,
                       int64_t capacity, int64_t *splits, int32_t *table, int mode, void *workspace,
                       size_t workspace_bytes, int32_t *status, void *stream, const void *next_input, int64_t next_k,
-                      int64_t next_n, int64_t next_m, int64_t next_capacity, int32_t *next_table) {
+                      int64_t next_n, int64_t next_m, int64_t next_capacity, int32_t *next_table,
+                      const zen::HostAsk &ask = {}) {
   using namespace zen;
   const int prepared = (mode & ZEN_MODE_PREPARED) ? ((mode & ZEN_MODE_SECOND) ? 2 : 1) : 0;
   const bool second_set = (mode & ZEN_MODE_SECOND) != 0;
@@ -503,6 +504,7 @@ int load_balance_call(const void *input, int dtype, int64_t n, int64_t m, int pa
     sa.prepared = near_key ? 0 : prepared;
     sa.second = second_set;
     sa.near_key = near_key;
+    sa.ask = ask;
     if (small) return table_load_balance(sa, splits_zero, s);
     if (next_input && next_k > 0) {
       sa.next_input = next_input;
@@ -626,6 +628,24 @@ int zen_load_balance(const void *input, int dtype, int64_t n, int64_t m, int par
                      size_t workspace_bytes, int32_t *status, void *stream) {
   return load_balance_call(input, dtype, n, m, partitions, rehash, thr, k, thr_out, out_idx, out_val, capacity, splits,
                            table, mode, workspace, workspace_bytes, status, stream, nullptr, 0, 0, 0, 0, nullptr);
+}
+
+int zen_load_balance_sizes(const void *input, int dtype, int64_t n, int64_t m, int partitions, int rehash,
+                           const uint32_t *thr, int64_t k, uint32_t *thr_out, int32_t *out_idx, void *out_val,
+                           int64_t capacity, int64_t *splits, int32_t *table, int mode, void *workspace,
+                           size_t workspace_bytes, int32_t *status, int64_t *host, int64_t words, void *stream) {
+  using namespace zen;
+  HostAnswer answer;
+  bool answered = false;
+  int rc = host_ask(host, words, (int64_t)partitions + 1, &answer);
+  if (rc != ZEN_OK) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  rc = load_balance_call(input, dtype, n, m, partitions, rehash, thr, k, thr_out, out_idx, out_val, capacity, splits, table,
+                         mode, workspace, workspace_bytes, status, stream, nullptr, 0, 0, 0, 0, nullptr, HostAsk{answer, &answered});
+  if (rc == ZEN_OK && !answered) rc = host_answer_launch(answer, splits, partitions, status, 1, s);
+  if (rc == ZEN_OK) return host_wait(answer, s);
+  if (answered) (void)hipStreamSynchronize(s);  // an answer may be on its way: not into a later call's words
+  return rc;
 }
 
 int zen_encode_merge_samples_next(int64_t n, int64_t m, int dtype, int64_t capacity, int partitions, int64_t k,

@@ -181,6 +181,38 @@ __device__ inline uint32_t load_fresh(const uint32_t *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Where the host waits for what a call has to know there (zen_readback.hip): pinned words, of which word 0 takes the
+// ticket once the others hold the answer.  The kernel that knows the answer stores it, where that is one of the call's
+// own: no launch for it, and what is left of the call's work runs while the host goes on.
+struct HostAnswer {
+  int64_t *host = nullptr;  // null: nobody asks
+  int64_t ticket = 0;
+};
+struct HostAsk {  // the same on its way through host code
+  HostAnswer answer;
+  bool *answered = nullptr;  // set where kernels of the call's own answer
+};
+// Past the caches, so that nothing has to be written back for the host to see it.
+__device__ inline void host_store(int64_t *p, int64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// By the whole workgroup, behind its stores of the answer's words.
+__device__ inline void host_answered(const HostAnswer &a) {
+  wait_global_acks();
+  __syncthreads();
+  if (threadIdx.x == 0) host_store(a.host, a.ticket);
+}
+// The status word (and a count in front of it, where there is one), once every workgroup that changes them has been
+// waited for.  By the whole workgroup.
+__device__ inline void host_answer_count(const HostAnswer &a, const int64_t *count, const int32_t *status) {
+  if (!a.host) return;
+  if (threadIdx.x == 0) {
+    host_store(a.host + 1, count ? __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0);
+    host_store(a.host + 2, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  }
+  host_answered(a);
+}
+
 __device__ inline int lane_id() { return int(__lane_id()); }
 
 __device__ inline uint64_t lanes_below() {  // mask of lanes with a smaller id
@@ -369,5 +401,14 @@ bool bucket_sort_fits(int64_t expected, uint32_t sentinel);
 int bucket_sort_pairs(uint32_t *keys_a, uint32_t *vals_a, uint32_t *keys_b, uint32_t *vals_b, int64_t max_count,
                       const uint32_t *count_dev, uint32_t sentinel, void *scratch, int32_t *status,
                       hipStream_t stream, uint32_t *more_a = nullptr, uint32_t *more_b = nullptr);
+
+// ------------------------------------------------- answers to the host (zen_readback.hip)
+
+// The answer a call on `host` (words of them) with `need` words besides word 0 will get; null words: an error.
+int host_ask(int64_t *host, int64_t words, int64_t need, HostAnswer *answer);
+// One kernel that answers with the words two arrays hold, for calls whose kernels do not.
+int host_answer_launch(const HostAnswer &answer, const int64_t *first, int n0, const int32_t *second, int n1, hipStream_t s);
+// Returns when the answer is there, or with the stream's error.
+int host_wait(const HostAnswer &answer, hipStream_t s);
 
 }  // namespace zen

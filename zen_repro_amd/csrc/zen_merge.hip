@@ -210,7 +210,7 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
                                                              const S *__restrict__ slab_val,
                                                              I *__restrict__ out_idx, O *__restrict__ out_val,
                                                              int64_t capacity, ScanState st, int tie_bits,
-                                                             int64_t *out_count, int32_t *status) {
+                                                             int64_t *out_count, HostAnswer answer, int32_t *status) {
   __shared__ SlabSortShared sh;  // the values take the counters' place once the ranks are known
   __shared__ uint64_t s_scan64[kMergeBlock / 64 + 1];
   __shared__ int s_tile;
@@ -374,7 +374,8 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
   const uint64_t tile_start = all_before;
   if (b == nb - 1 && threadIdx.x == 0) {
     const uint64_t all = tile_start + total;
-    *out_count = (int64_t)all;
+    // (for the launch's last workgroup to read, on another die maybe)
+    __hip_atomic_store(out_count, (int64_t)all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (all > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
   }
   for (uint32_t i = threadIdx.x; i < total; i += kMergeBlock) {
@@ -386,6 +387,7 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
   }
   // every workgroup has read the descriptors it needs before it gets here
   uint32_t *finished = reinterpret_cast<uint32_t *>(st.desc + nb + 1);
+  if (answer.host) wait_global_acks();  // its share of the status word, and the count
   __syncthreads();
   if (threadIdx.x == 0) s_tile = atomicAdd(finished, 1u) == (uint32_t)nb - 1u;
   __syncthreads();
@@ -395,6 +397,7 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
       *st.ticket = 0;
       *finished = 0;
     }
+    host_answer_count(answer, out_count, status);
   }
 }
 
@@ -446,7 +449,7 @@ bool slab_merge_fits(int64_t r, int64_t dense_n, SlabGeom *geo) {
 template <typename I, typename S, typename O>
 int slab_merge_launch(const SlabGeom &geo, const I *idx, const S *val, int64_t r, int64_t dense_n, void *out_idx,
                       int idx64_out, O *out_val, int64_t capacity, int64_t *out_count, void *workspace,
-                      bool zeroed, int32_t *status, hipStream_t s) {
+                      bool zeroed, int32_t *status, hipStream_t s, const HostAsk &ask) {
   const SlabMergePlan p = plan_slab_merge(workspace, geo, r);
   if (!zeroed) {
     launch_fill<unsigned long long>(p.scan, 0ull, p.zero_bytes / sizeof(unsigned long long), s);
@@ -466,13 +469,14 @@ int slab_merge_launch(const SlabGeom &geo, const I *idx, const S *val, int64_t r
     k_merge_bucket<int64_t, S, O><<<dim3(geo.nbuckets), dim3(kMergeBlock), 0, s>>>(
         geo, p.feed.cursor, p.feed.coarse_cursor, p.feed.bucket_lo, p.slab_idx, p.slab_arr,
         static_cast<const S *>(p.slab_val), static_cast<int64_t *>(out_idx), out_val, capacity, st, tie_bits, out_count,
-        status);
+        ask.answer, status);
   else
     k_merge_bucket<int32_t, S, O><<<dim3(geo.nbuckets), dim3(kMergeBlock), 0, s>>>(
         geo, p.feed.cursor, p.feed.coarse_cursor, p.feed.bucket_lo, p.slab_idx, p.slab_arr,
         static_cast<const S *>(p.slab_val), static_cast<int32_t *>(out_idx), out_val, capacity, st, tie_bits, out_count,
-        status);
+        ask.answer, status);
   ZEN_LAUNCH_CHECK("k_merge_bucket");
+  if (ask.answer.host) *ask.answered = true;
   return ZEN_OK;
 }
 
@@ -522,11 +526,11 @@ bool writes_dense(int64_t r, int64_t dense_n, int dtype, int mode) {
 template <typename S, typename O>
 int merge_launch(const void *idx, int idx64_in, const S *val, int64_t r, int64_t dense_n, void *out_idx,
                  int idx64_out, O *out_val, int64_t capacity, int64_t *out_count, int mode, void *workspace,
-                 int32_t *status, hipStream_t s) {
+                 int32_t *status, hipStream_t s, const HostAsk &ask = {}) {
   const bool zeroed = (mode & ZEN_MODE_ZEROED) != 0;
   if (takes_one(r, mode))
     return wide_merge_one(idx, idx64_in, val, sizeof(S) == 2 ? ZEN_BF16 : ZEN_F32, r, dense_n, out_idx, idx64_out, out_val,
-                          sizeof(O) == 2 ? ZEN_BF16 : ZEN_F32, capacity, out_count, status, s);
+                          sizeof(O) == 2 ? ZEN_BF16 : ZEN_F32, capacity, out_count, status, s, ask);
   const bool wide = takes_wide(r, dense_n, mode);
   mode &= ~(ZEN_MODE_ZEROED | ZEN_MODE_SLABS);
   SlabGeom geo;
@@ -544,14 +548,14 @@ int merge_launch(const void *idx, int idx64_in, const S *val, int64_t r, int64_t
                          wide_device_cus(), status, &list))
       return fail(ZEN_EINVAL, "zen_merge: sizes do not suit the wide buckets");
     return wide_merge(list, sizeof(S) == 2 ? ZEN_BF16 : ZEN_F32, out_idx, idx64_out, out_val,
-                      sizeof(O) == 2 ? ZEN_BF16 : ZEN_F32, capacity, out_count, scan, s);
+                      sizeof(O) == 2 ? ZEN_BF16 : ZEN_F32, capacity, out_count, scan, s, ask);
   }
   if (mode == ZEN_MODE_FAST && slab_merge_fits(r, dense_n, &geo)) {
     if (idx64_in)
       return slab_merge_launch(geo, static_cast<const int64_t *>(idx), val, r, dense_n, out_idx, idx64_out, out_val,
-                               capacity, out_count, workspace, zeroed, status, s);
+                               capacity, out_count, workspace, zeroed, status, s, ask);
     return slab_merge_launch(geo, static_cast<const int32_t *>(idx), val, r, dense_n, out_idx, idx64_out, out_val,
-                             capacity, out_count, workspace, zeroed, status, s);
+                             capacity, out_count, workspace, zeroed, status, s, ask);
   }
   MergePlan p = plan_merge(workspace, r, dense_n);
   const unsigned blocks = (unsigned)ceil_div(r, 256);
@@ -638,7 +642,7 @@ namespace {
 
 int merge_call(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n, void *out_idx,
                int idx64_out, void *out_val, bool round, int64_t capacity, int64_t *out_count, int mode,
-               void *workspace, size_t workspace_bytes, int32_t *status, void *stream) {
+               void *workspace, size_t workspace_bytes, int32_t *status, void *stream, const zen::HostAsk &ask = {}) {
   using namespace zen;
   const char *why = "";
   if (merge_check(idx, val, dtype, r, dense_n, mode, &why) != ZEN_OK) return fail(ZEN_EINVAL, why);
@@ -653,12 +657,12 @@ int merge_call(const void *idx, int idx64_in, const void *val, int dtype, int64_
   if (workspace_bytes < zen_merge_workspace(r, dense_n)) return fail(ZEN_EWORKSPACE, "zen_merge: workspace too small");
   if (dtype == ZEN_BF16 && round)
     return merge_launch(idx, idx64_in, static_cast<const uint16_t *>(val), r, dense_n, out_idx, idx64_out,
-                        static_cast<uint16_t *>(out_val), capacity, out_count, mode, workspace, status, s);
+                        static_cast<uint16_t *>(out_val), capacity, out_count, mode, workspace, status, s, ask);
   if (dtype == ZEN_BF16)
     return merge_launch(idx, idx64_in, static_cast<const uint16_t *>(val), r, dense_n, out_idx, idx64_out,
-                        static_cast<float *>(out_val), capacity, out_count, mode, workspace, status, s);
+                        static_cast<float *>(out_val), capacity, out_count, mode, workspace, status, s, ask);
   return merge_launch(idx, idx64_in, static_cast<const uint32_t *>(val), r, dense_n, out_idx, idx64_out,
-                      static_cast<float *>(out_val), capacity, out_count, mode, workspace, status, s);
+                      static_cast<float *>(out_val), capacity, out_count, mode, workspace, status, s, ask);
 }
 
 }  // namespace
@@ -677,6 +681,24 @@ int zen_merge_rounded(const void *idx, int idx64_in, const void *val, int dtype,
                       void *workspace, size_t workspace_bytes, int32_t *status, void *stream) {
   return merge_call(idx, idx64_in, val, dtype, r, dense_n, out_idx, idx64_out, out_val, true, capacity, out_count,
                     mode, workspace, workspace_bytes, status, stream);
+}
+
+int zen_merge_rounded_count(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n,
+                            void *out_idx, int idx64_out, void *out_val, int64_t capacity, int64_t *out_count, int mode,
+                            void *workspace, size_t workspace_bytes, int32_t *status, int64_t *host, int64_t words,
+                            void *stream) {
+  using namespace zen;
+  HostAnswer answer;
+  bool answered = false;
+  int rc = host_ask(host, words, 2, &answer);
+  if (rc != ZEN_OK) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  rc = merge_call(idx, idx64_in, val, dtype, r, dense_n, out_idx, idx64_out, out_val, true, capacity, out_count, mode,
+                  workspace, workspace_bytes, status, stream, HostAsk{answer, &answered});
+  if (rc == ZEN_OK && !answered) rc = host_answer_launch(answer, out_count, 1, status, 1, s);
+  if (rc == ZEN_OK) return host_wait(answer, s);
+  if (answered) (void)hipStreamSynchronize(s);  // an answer may be on its way: not into a later call's words
+  return rc;
 }
 
 size_t zen_decode_dense_workspace(int64_t r, int64_t dense_n) {

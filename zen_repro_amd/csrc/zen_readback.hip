@@ -30,13 +30,11 @@ __global__ void k_read_back(ReadBack r, int64_t *host, int64_t ticket) {
 #pragma unroll
   for (int s = 0; s < ZEN_READ_BACK_SEGMENTS; ++s) {
     for (int i = threadIdx.x; i < r.count[s]; i += blockDim.x)
-      host[at + i] = r.wide[s] ? static_cast<const int64_t *>(r.from[s])[i]
-                               : (int64_t) static_cast<const int32_t *>(r.from[s])[i];
+      host_store(host + at + i, r.wide[s] ? static_cast<const int64_t *>(r.from[s])[i]
+                                          : (int64_t) static_cast<const int32_t *>(r.from[s])[i]);
     at += r.count[s];
   }
-  __threadfence_system();
-  __syncthreads();
-  if (threadIdx.x == 0) __hip_atomic_store(host, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  host_answered(HostAnswer{host, ticket});
 }
 
 // Elements with key >= max(thr[0], 1) (thr == nullptr: the nonzero ones).  Bound by the one read of the tensor:
@@ -89,6 +87,46 @@ void launch_count(const S *in, int64_t n, const uint32_t *thr, int64_t *count, h
 }
 
 }  // namespace
+
+int host_ask(int64_t *host, int64_t words, int64_t need, HostAnswer *answer) {
+  if (!host || words < need + 1) return fail(ZEN_EINVAL, "host words missing or too few");
+  answer->host = host;
+  answer->ticket = host[0] + 1;
+  return ZEN_OK;
+}
+
+int host_answer_launch(const HostAnswer &answer, const int64_t *first, int n0, const int32_t *second, int n1, hipStream_t s) {
+  const ReadBack r{{first, second, nullptr}, {n0, n1, 0}, {1, 0, 0}};
+  k_read_back<<<dim3(1), dim3(64), 0, s>>>(r, answer.host, answer.ticket);
+  ZEN_LAUNCH_CHECK("k_read_back");
+  return ZEN_OK;
+}
+
+int host_wait(const HostAnswer &answer, hipStream_t s) {
+  // The waits of a call are short: this core watches for the answer.  A longer one is for what the stream has to wait
+  // for itself (an exchange, other ranks): then the core is left to others, for a sixteenth of the time waited so far
+  // and a millisecond at most, and the stream is asked every time, which says when something on it has failed.  (The
+  // runtime's own waits keep the core busy from beginning to end, hipEventBlockingSync or not.)
+  using clock = std::chrono::steady_clock;
+  const auto begin = clock::now();
+  for (uint32_t spins = 1;; ++spins) {
+    if (__atomic_load_n(answer.host, __ATOMIC_ACQUIRE) == answer.ticket) return ZEN_OK;
+    _mm_pause();
+    if ((spins & 63u) == 0 && clock::now() - begin > kSpin) break;
+  }
+  for (;;) {
+    const auto nap = (clock::now() - begin) / 16;
+    std::this_thread::sleep_for(nap < kNap ? nap : kNap);
+    if (__atomic_load_n(answer.host, __ATOMIC_ACQUIRE) == answer.ticket) return ZEN_OK;
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady) continue;
+    ZEN_HIP_CHECK(e);
+    return __atomic_load_n(answer.host, __ATOMIC_ACQUIRE) == answer.ticket
+               ? ZEN_OK
+               : fail(ZEN_EHIP, "zen_read_back: the stream ended without an answer");
+  }
+}
+
 }  // namespace zen
 
 extern "C" {
@@ -123,29 +161,7 @@ int zen_read_back(const void *p0, int n0, int wide0, const void *p1, int n1, int
   const int64_t ticket = host[0] + 1;
   k_read_back<<<dim3(1), dim3(64), 0, s>>>(r, host, ticket);
   ZEN_LAUNCH_CHECK("k_read_back");
-  const int64_t *flag = host;
-  // The waits of a call are short: this core watches for the answer.  A longer one is for what the stream has to wait
-  // for itself (an exchange, other ranks): then the core is left to others, for a sixteenth of the time waited so far
-  // and a millisecond at most, and the stream is asked every time, which says when something on it has failed.  (The
-  // runtime's own waits keep the core busy from beginning to end, hipEventBlockingSync or not.)
-  using clock = std::chrono::steady_clock;
-  const auto begin = clock::now();
-  for (uint32_t spins = 1;; ++spins) {
-    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == ticket) return ZEN_OK;
-    _mm_pause();
-    if ((spins & 63u) == 0 && clock::now() - begin > kSpin) break;
-  }
-  for (;;) {
-    const auto nap = (clock::now() - begin) / 16;
-    std::this_thread::sleep_for(nap < kNap ? nap : kNap);
-    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == ticket) return ZEN_OK;
-    const hipError_t e = hipStreamQuery(s);
-    if (e == hipErrorNotReady) continue;
-    ZEN_HIP_CHECK(e);
-    return __atomic_load_n(flag, __ATOMIC_ACQUIRE) == ticket
-               ? ZEN_OK
-               : fail(ZEN_EHIP, "zen_read_back: the stream ended without an answer");
-  }
+  return host_wait(HostAnswer{host, ticket}, s);
 }
 
 int zen_count(const void *input, int dtype, int64_t n, const uint32_t *thr, int64_t *count, void *stream) {

@@ -19,10 +19,10 @@
 //                   index's probe sequence).  Every bucket has a part of the map
 //                   of its own, so what finally moved into a bucket is what its
 //                   part holds; an index that ran out of levels goes to its
-//                   partition's serial list;
+//                   partition's serial list; split sizes;
 //   k_slab_place    one workgroup per bucket: survivors and moved-in entries by
 //                   the same kind of bitmap to the bucket's place in the
-//                   partition-major output; split sizes.
+//                   partition-major output.
 #include "zen_balance.h"
 #include "zen_hashmap.h"
 #include "zen_slab.h"
@@ -296,8 +296,9 @@ __device__ inline uint32_t part_min(unsigned long long *cells, const SlabTables 
 // Where every bucket starts in the output: survivors + moved-in entries, the partition's serial entries
 // behind its last bucket.  Run by one workgroup of kSlabBlock threads once all counts are final: it is the last
 // to need the counters the chains raised with atomics, hands what k_slab_place still wants of them on in final_n
-// and puts them back to zero.
-__device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables &tb, uint32_t *s_scan) {
+// and puts them back to zero.  What the status word can come to is known here too (k_slab_place adds nothing).
+__device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables &tb, uint32_t *s_scan, int64_t spp,
+                                          uint32_t capacity, int64_t *splits, const HostAnswer &answer, int32_t *status) {
   constexpr int kPer = kSlabMaxBuckets / kSlabBlock;
   const uint32_t B = geo.nbuckets;
   uint32_t c[kPer], mv[kPer], rm[kPer];
@@ -338,6 +339,21 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
     *tb.losers = 0;
     *tb.done = 0;
   }
+  // the split sizes: the host has them while the entries are still on their way to their places
+  __syncthreads();
+  for (uint32_t p = threadIdx.x; p < (uint32_t)tb.partitions; p += kSlabBlock) {
+    const int64_t size = (int64_t)(tb.out_start[(p + 1u) * geo.bpp] - tb.out_start[p * geo.bpp]);
+    splits[p] = size;
+    if (answer.host) host_store(answer.host + 1 + p, size);
+    if ((int64_t)tb.final_n[B + p] > spp) atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
+  }
+  if (threadIdx.x == 0 && tb.out_start[B] > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
+  if (answer.host) {
+    wait_global_acks();
+    __syncthreads();
+    if (threadIdx.x == 0) host_store(answer.host + 1 + tb.partitions, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    host_answered(answer);
+  }
 }
 
 // Levels 2 and 3 for the indices that lost level 1, one per thread.  Bound by latency: a probe is four or five
@@ -345,7 +361,8 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
 // on a full chip; nothing is counted in one place (62 M slots, 10 % taken, 300 000 losers: with one counter of the
 // map's claims and one log of the owners pushed out, whose entries another kernel classified afterwards, 338 + 220 us).
 __global__ __launch_bounds__(kSlabBlock) void k_slab_chains(SlabGeom geo, Probe g, SlabTables tb, unsigned long long *cells,
-                                                            int64_t spp, int32_t *status) {
+                                                            int64_t spp, uint32_t capacity, int64_t *__restrict__ splits,
+                                                            HostAnswer answer, int32_t *status) {
   __shared__ uint32_t s_scan[kSlabBlock / 64 + 1];
   __shared__ bool s_last;
   uint32_t losers = load_fresh(tb.losers);
@@ -413,7 +430,7 @@ __global__ __launch_bounds__(kSlabBlock) void k_slab_chains(SlabGeom geo, Probe 
   __syncthreads();
   if (threadIdx.x == 0) s_last = atomicAdd(tb.done, 1u) == working - 1u;
   __syncthreads();
-  if (s_last) slab_output_starts(geo, tb, s_scan);
+  if (s_last) slab_output_starts(geo, tb, s_scan, spp, capacity, splits, answer, status);
 }
 
 // ------------------------------------------------------------------ place
@@ -434,10 +451,8 @@ struct SlabPlaceLds {
 
 template <typename S, uint32_t SPAN>
 __global__ __launch_bounds__(kSlabBlock, SPAN <= kSlabSpan2 ? 6 : 2) void k_slab_place(SlabGeom geo, SlabTables tb, unsigned long long *cells,
-                                                           int64_t spp, const S *__restrict__ dense,
-                                                           int32_t *__restrict__ out_idx, S *__restrict__ out_val,
-                                                           uint32_t capacity, int64_t *__restrict__ splits,
-                                                           int32_t *status) {
+                                                           const S *__restrict__ dense, int32_t *__restrict__ out_idx,
+                                                           S *__restrict__ out_val, uint32_t capacity) {
   constexpr int kCells = (1 << kSlabPartLog2) / kSlabBlock;
   __shared__ SlabPlaceLds<SPAN> sh;
   const uint32_t b = blockIdx.x;
@@ -535,12 +550,6 @@ __global__ __launch_bounds__(kSlabBlock, SPAN <= kSlabSpan2 ? 6 : 2) void k_slab
       }
     }
   }
-  if (b % geo.bpp == 0 && threadIdx.x == 0) {
-    const uint32_t lo_at = tb.out_start[b], hi = tb.out_start[b + geo.bpp];
-    splits[part] = (int64_t)(hi - lo_at);
-    if ((int64_t)serial_n[part] > spp) atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
-    if (hi > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
-  }
 }
 
 struct SlabPlan {
@@ -626,14 +635,14 @@ int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPl
     // (as many workgroups as the chip holds; fewer where there can be few losers)
     const int64_t groups = ceil_div((int64_t)p.tb.log_cap / 4, (int64_t)kSlabBlock);
     k_slab_chains<<<dim3((unsigned)(groups < 64 ? 64 : groups > 1024 ? 1024 : groups)), dim3(kSlabBlock), 0, s>>>(
-        geo, a.g, p.tb, a.hash, a.spp, a.status);
+        geo, a.g, p.tb, a.hash, a.spp, (uint32_t)a.capacity, a.splits, a.ask.answer, a.status);
     ZEN_LAUNCH_CHECK("k_slab_chains");
+    if (a.ask.answer.host) *a.ask.answered = true;
   }
   {
     ProfScope prof(kProfSlabPlace, s);
-    k_slab_place<S, SPAN><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, a.spp, dense, a.out_idx,
-                                                               static_cast<S *>(a.out_val), (uint32_t)a.capacity,
-                                                               a.splits, a.status);
+    k_slab_place<S, SPAN><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, dense, a.out_idx,
+                                                               static_cast<S *>(a.out_val), (uint32_t)a.capacity);
     ZEN_LAUNCH_CHECK("k_slab_place");
   }
   return ZEN_OK;

@@ -249,7 +249,7 @@ __global__ __launch_bounds__(kOneBlock) void k_table_one(const S *__restrict__ i
                                                          const uint32_t *__restrict__ thr, Probe g, int parts, int64_t spp,
                                                          int32_t *__restrict__ out_idx, S *__restrict__ out_val,
                                                          uint32_t capacity, int64_t *__restrict__ splits,
-                                                         int32_t *status) {
+                                                         HostAnswer answer, int32_t *status) {
   constexpr int V = VecOf<S>::kN;
   __shared__ __attribute__((aligned(16))) uint32_t slots[kOneSlots];
   __shared__ uint32_t serial[kOneSerial];       // partition << 15 | index
@@ -334,7 +334,10 @@ __global__ __launch_bounds__(kOneBlock) void k_table_one(const S *__restrict__ i
     const uint32_t h = threadIdx.x < kOneParts ? held[threadIdx.x] : 0u;
     uint32_t total;
     const uint32_t ex = block_exclusive_scan<uint32_t, kOneBlock>(h, smem, &total);
-    if ((int)threadIdx.x < parts) splits[threadIdx.x] = (int64_t)(h + left[threadIdx.x]);
+    if ((int)threadIdx.x < parts) {
+      splits[threadIdx.x] = (int64_t)(h + left[threadIdx.x]);
+      if (answer.host) host_store(answer.host + 1 + threadIdx.x, (int64_t)(h + left[threadIdx.x]));
+    }
     if (threadIdx.x < kOneParts) held[threadIdx.x] = ex + h;  // entries with a slot through the partition
   }
   __syncthreads();
@@ -346,6 +349,12 @@ __global__ __launch_bounds__(kOneBlock) void k_table_one(const S *__restrict__ i
     }
   }
   if (threadIdx.x == 0 && all + total_left > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
+  if (answer.host) {
+    wait_global_acks();
+    __syncthreads();
+    if (threadIdx.x == 0) host_store(answer.host + 1 + parts, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    host_answered(answer);
+  }
 }
 
 struct TablePlan {
@@ -379,8 +388,10 @@ int table_launch(const SlabBalanceArgs &a, const TablePlan &p, const uint32_t *t
   S *out_val = static_cast<S *>(a.out_val);
   if (a.g.m <= kOneSlots && a.n <= (int64_t)kOneSlots && a.partitions <= kOneParts) {
     k_table_one<S, ALIGNED><<<dim3(1), dim3(kOneBlock), 0, s>>>(in, (uint32_t)a.n, thr, a.g, a.partitions, a.spp, a.out_idx,
-                                                               out_val, (uint32_t)a.capacity, a.splits, a.status);
+                                                               out_val, (uint32_t)a.capacity, a.splits, a.ask.answer,
+                                                               a.status);
     ZEN_LAUNCH_CHECK("k_table_one");
+    if (a.ask.answer.host) *a.ask.answered = true;
     return ZEN_OK;
   }
   if (!zeroed) launch_fill<int64_t>(a.splits, 0, (size_t)a.partitions, s);

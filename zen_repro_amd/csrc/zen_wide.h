@@ -296,8 +296,8 @@ bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, 
 constexpr int64_t wide_merge_one_max() { return 4096; }
 int wide_merge_one(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n, void *out_idx,
                    int idx64_out, void *out_val, int out_dtype, int64_t capacity, int64_t *out_count, int32_t *status,
-                   hipStream_t s);
+                   hipStream_t s, const HostAsk &ask = {});
 int wide_merge(const WideList &list, int dtype, void *out_idx, int idx64_out, void *out_val, int out_dtype,
-               int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s);
+               int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s, const HostAsk &ask = {});
 
 }  // namespace zen

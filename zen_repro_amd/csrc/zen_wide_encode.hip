@@ -242,7 +242,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
                                                           S *__restrict__ out_val, uint32_t capacity,
                                                           int64_t *__restrict__ splits, uint32_t *clear,
                                                           uint32_t clear_words, uint32_t *clear_too,
-                                                          uint32_t clear_too_words, int32_t *status) {
+                                                          uint32_t clear_too_words, HostAnswer answer, int32_t *status) {
   __shared__ WideShared<S> sh;
   const uint32_t b = blockIdx.x, B = geo.nbuckets, bpp = geo.bpp;
   const uint32_t part = b / bpp;
@@ -749,7 +749,8 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
       }
     }
     if (last_of_part && tid == 0) {
-      splits[part] = (int64_t)(in_part + own_n + serial);
+      // (for the launch's last workgroup to read, on another die maybe)
+      __hip_atomic_store(&splits[part], (int64_t)(in_part + own_n + serial), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if ((int64_t)serial_raw > spp) atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
       if (out_base + own_n + serial > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
     }
@@ -787,6 +788,13 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   if (sh.flag & 2u) {
     for (uint32_t i = tid; i < B; i += kWideBlock) tb.desc[i] = 0ull;
     if (tid == 0) *tb.done = 0;
+    if (answer.host) {  // every workgroup's stores and atomics were carried out before it counted itself as finished
+      for (uint32_t p = tid; p < (uint32_t)tb.partitions; p += kWideBlock)
+        host_store(answer.host + 1 + p, __hip_atomic_load(&splits[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      if (tid == 0)
+        host_store(answer.host + 1 + tb.partitions, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      host_answered(answer);
+    }
   }
   WIDE_MARK(14);
 }
@@ -950,13 +958,14 @@ int wide_load_balance(const SlabBalanceArgs &a, size_t state_offset, hipStream_t
       k_wide_tail<uint16_t><<<dim3(geo.nbuckets), dim3(kWideBlock), 0, s>>>(
           geo, a.g, p.tb, filter, a.hash, a.spp, static_cast<const uint16_t *>(a.input), a.out_idx,
           static_cast<uint16_t *>(a.out_val), (uint32_t)a.capacity, a.splits, clear, clear_words, clear_too,
-          clear_too_words, a.status);
+          clear_too_words, a.ask.answer, a.status);
     else
       k_wide_tail<uint32_t><<<dim3(geo.nbuckets), dim3(kWideBlock), 0, s>>>(
           geo, a.g, p.tb, filter, a.hash, a.spp, static_cast<const uint32_t *>(a.input), a.out_idx,
           static_cast<uint32_t *>(a.out_val), (uint32_t)a.capacity, a.splits, clear, clear_words, clear_too,
-          clear_too_words, a.status);
+          clear_too_words, a.ask.answer, a.status);
     ZEN_LAUNCH_CHECK("k_wide_tail");
+    if (a.ask.answer.host) *a.ask.answered = true;
   }
   return wide_line_leave(s);
 }

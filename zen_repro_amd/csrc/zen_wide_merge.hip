@@ -70,7 +70,8 @@ struct WideMergeShared {
 template <typename I, typename S, typename O, bool DENSE, bool DIRECT>
 __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__restrict__ out_idx,
                                                            O *__restrict__ out_val, int64_t capacity,
-                                                           ScanState st, int tie_bits, int64_t *out_count) {
+                                                           ScanState st, int tie_bits, int64_t *out_count,
+                                                           HostAnswer answer) {
   __shared__ WideMergeShared sh;
   const SlabGeom &geo = list.geo;
   const WideSlabs &in = list.out;
@@ -405,7 +406,8 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
     block_exclusive_scan<uint64_t, kWideBlock>(d & kDescValue, sh.scan64, &all_before);  // its barriers also publish the gathered entries
     if (b == nb - 1 && tid == 0) {
       const uint64_t all = all_before + total;
-      *out_count = (int64_t)all;
+      // (for the launch's last workgroup to read, on another die maybe)
+      __hip_atomic_store(out_count, (int64_t)all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (all > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
     }
     for (uint32_t i = tid; i < total; i += kWideBlock) {
@@ -416,7 +418,12 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
       }
     }
   }
-  if (DIRECT) return;
+  if (answer.host) wait_global_acks();  // its share of the status word, and the count
+  if (DIRECT) {
+    __syncthreads();
+    host_answer_count(answer, DENSE ? nullptr : out_count, status);
+    return;
+  }
   // every workgroup has read the descriptors it needs before it gets here: the last one to finish clears the
   // prefix state
   uint32_t *finished = reinterpret_cast<uint32_t *>(st.desc + nb + 1);
@@ -429,6 +436,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
       *st.ticket = 0;
       *finished = 0;
     }
+    host_answer_count(answer, DENSE ? nullptr : out_count, status);
   }
 }
 
@@ -490,35 +498,37 @@ uint32_t wide_scatter_batches(const WideList &list, int batch) { return (uint32_
 
 template <typename S, typename O, bool DIRECT>
 static void wide_merge_launch(const WideList &list, void *out_idx, int idx64_out, O *out_val, int64_t capacity,
-                              int64_t *out_count, unsigned long long *scan, hipStream_t s) {
+                              int64_t *out_count, unsigned long long *scan, hipStream_t s, const HostAsk &ask) {
   const ScanState st = scan_state(scan, (int64_t)list.geo.nbuckets);
   const int tie_bits = ceil_log2_u64((uint64_t)list.r);  // arrival numbers are < r
   const dim3 grid(DIRECT ? 1u : list.geo.nbuckets), block(kWideBlock);
   if (!out_idx)
-    k_wide_merge<int32_t, S, O, true, DIRECT><<<grid, block, 0, s>>>(list, nullptr, out_val, capacity, st, tie_bits, out_count);
+    k_wide_merge<int32_t, S, O, true, DIRECT><<<grid, block, 0, s>>>(list, nullptr, out_val, capacity, st, tie_bits, out_count,
+                                                                         ask.answer);
   else if (idx64_out)
     k_wide_merge<int64_t, S, O, false, DIRECT><<<grid, block, 0, s>>>(list, static_cast<int64_t *>(out_idx), out_val, capacity,
-                                                                     st, tie_bits, out_count);
+                                                                     st, tie_bits, out_count, ask.answer);
   else
     k_wide_merge<int32_t, S, O, false, DIRECT><<<grid, block, 0, s>>>(list, static_cast<int32_t *>(out_idx), out_val, capacity,
-                                                                     st, tie_bits, out_count);
+                                                                     st, tie_bits, out_count, ask.answer);
 }
 
 template <bool DIRECT>
 static void wide_merge_typed(const WideList &list, int dtype, void *out_idx, int idx64_out, void *out_val, int out_dtype,
-                             int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s) {
+                             int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s,
+                             const HostAsk &ask) {
   if (dtype == ZEN_F32)
-    wide_merge_launch<uint32_t, float, DIRECT>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s);
+    wide_merge_launch<uint32_t, float, DIRECT>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s, ask);
   else if (out_dtype == ZEN_BF16)
-    wide_merge_launch<uint16_t, uint16_t, DIRECT>(list, out_idx, idx64_out, static_cast<uint16_t *>(out_val), capacity, out_count, scan, s);
+    wide_merge_launch<uint16_t, uint16_t, DIRECT>(list, out_idx, idx64_out, static_cast<uint16_t *>(out_val), capacity, out_count, scan, s, ask);
   else
-    wide_merge_launch<uint16_t, float, DIRECT>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s);
+    wide_merge_launch<uint16_t, float, DIRECT>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s, ask);
 }
 
 // out_dtype and out_idx as for wide_merge below.  Any indices: a narrow range takes whatever comes.
 int wide_merge_one(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n, void *out_idx,
                    int idx64_out, void *out_val, int out_dtype, int64_t capacity, int64_t *out_count, int32_t *status,
-                   hipStream_t s) {
+                   hipStream_t s, const HostAsk &ask) {
   WideList list{};
   while ((dense_n >> list.geo.sub_shift) >= kWideSubs) ++list.geo.sub_shift;  // 17 at most: with 14 bits of arrival number a word
   list.geo.nbuckets = 1;
@@ -529,8 +539,9 @@ int wide_merge_one(const void *idx, int idx64_in, const void *val, int dtype, in
   list.idx64 = idx64_in;
   list.status = status;
   ProfScope prof(kProfWideMerge, s);
-  wide_merge_typed<true>(list, dtype, out_idx, idx64_out, out_val, out_dtype, capacity, out_count, nullptr, s);
+  wide_merge_typed<true>(list, dtype, out_idx, idx64_out, out_val, out_dtype, capacity, out_count, nullptr, s, ask);
   ZEN_LAUNCH_CHECK("k_wide_merge");
+  if (ask.answer.host) *ask.answered = true;
   return ZEN_OK;
 }
 
@@ -538,7 +549,7 @@ int wide_merge_one(const void *idx, int idx64_in, const void *val, int dtype, in
 // when the second ends.  out_dtype: ZEN_F32 (the sums; the only choice for fp32 values) or ZEN_BF16 (rounded).
 // out_idx == nullptr: out_val is the dense tensor.
 int wide_merge(const WideList &list, int dtype, void *out_idx, int idx64_out, void *out_val, int out_dtype,
-               int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s) {
+               int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s, const HostAsk &ask) {
   {
     ProfScope prof(kProfWideScatter, s);
     if (dtype == ZEN_BF16)
@@ -548,8 +559,9 @@ int wide_merge(const WideList &list, int dtype, void *out_idx, int idx64_out, vo
     ZEN_LAUNCH_CHECK("k_wide_scatter");
   }
   ProfScope prof(kProfWideMerge, s);
-  wide_merge_typed<false>(list, dtype, out_idx, idx64_out, out_val, out_dtype, capacity, out_count, scan, s);
+  wide_merge_typed<false>(list, dtype, out_idx, idx64_out, out_val, out_dtype, capacity, out_count, scan, s, ask);
   ZEN_LAUNCH_CHECK("k_wide_merge");
+  if (ask.answer.host) *ask.answered = true;
   return ZEN_OK;
 }
 

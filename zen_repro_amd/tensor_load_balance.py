@@ -359,6 +359,11 @@ class TensorPartition:
         Calls that may be in flight at the same time (different streams, e.g.
         one gradient bucket's encode next to the previous bucket's) must use
         different `slot` numbers: a slot owns its workspace and its table."""
+        return self._fused(tensor, thr, capacity, k, mode, thr_out, slot, near, None)
+
+    def _fused(self, tensor, thr, capacity, k, mode, thr_out, slot, near, words):
+        """load_balance_flat; with `words` (of _lib.host_words) the split sizes and the status are there when this
+        returns."""
         _lib.require_gpu(tensor, "input")
         flat = tensor.reshape(-1)
         n = flat.numel()
@@ -382,10 +387,13 @@ class TensorPartition:
         flags, used = self._take_ahead(flat, n, int(k), capacity, ws, slot, mode, thr, near)
         if near is not None and k > 0 and thr is None:
             thr, flags = near, flags | _lib.MODE_FLOOR
-        rc = L.zen_load_balance(
-            _lib.ptr(flat), code, n, m, self.partitions, self.rehash, _lib.ptr(thr), int(k), _lib.ptr(thr_out),
-            _lib.ptr(out_idx), _lib.ptr(out_val), capacity, _lib.ptr(splits), _lib.ptr(table),
-            mode | flags | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status), _lib.stream_of(dev))
+        args = (_lib.ptr(flat), code, n, m, self.partitions, self.rehash, _lib.ptr(thr), int(k), _lib.ptr(thr_out),
+                _lib.ptr(out_idx), _lib.ptr(out_val), capacity, _lib.ptr(splits), _lib.ptr(table),
+                mode | flags | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status))
+        if words is None:
+            rc = L.zen_load_balance(*args, _lib.stream_of(dev))
+        else:
+            rc = L.zen_load_balance_sizes(*args, words.ptr, words.words, _lib.stream_of(dev))
         if rc != _lib.OK:
             table.zero_()  # a call that failed half way may have left entries behind
         _lib.check(rc, "load_balance")
@@ -396,7 +404,9 @@ class TensorPartition:
         """Returns (indices[P], values[P], splits) like the reference
         (tensor_load_balance.py:43-51).  The per-partition tensors are views of
         two contiguous buffers; slicing them needs the split sizes on the
-        host, which is this call's only synchronisation.  Without a `capacity`
+        host, which is this call's only synchronisation: what they hold is
+        complete on the current stream, and may still be on its way when the
+        call returns.  Without a `capacity`
         one is worked out and the call is repeated with four times as much
         when the selection turns out larger; `grow=True` asks for the same
         with a capacity that is the caller's estimate."""
@@ -411,8 +421,9 @@ class TensorPartition:
                  [_lib.MODE_GENERAL]) if mode is None else [mode]
         modes = list(every)
         while modes:
-            out_idx, out_val, splits, status = self.load_balance_flat(tensor, thr, capacity, k, modes[0])
-            host = _lib.read_back(splits, status)
+            words = _lib.host_words(self.partitions + 1)
+            out_idx, out_val, splits, _ = self._fused(tensor, thr, capacity, k, modes[0], None, 0, None, words)
+            host = words.view[1:self.partitions + 2]
             bits = host[-1]
             if bits & (_lib.STAT_RETRY | _lib.STAT_INTERNAL):
                 # a declined or aborted call may leave entries and counters behind in the table
