@@ -4,7 +4,7 @@
 // per sample element.  A radix select behind a gather took 6 to 8 dependent launches, each a few microseconds of
 // work; here the histogram is taken while the elements arrive, at 15 bits of the magnitude (for bf16 the whole
 // key), so that one more workgroup finds the k-th:
-//   up to one_max() elements  one workgroup does everything in one launch, 16 elements per thread in registers;
+//   up to one_max() elements  one workgroup does everything in one launch, the elements in registers;
 //   more, bf16                k_sample_count (every workgroup keeps 32768 16-bit counters in LDS and writes them
 //                             out, with sums of 64 neighbours each: nothing has to be zero beforehand and no
 //                             atomic leaves the compute unit), k_sample_pick (one workgroup);
@@ -17,11 +17,14 @@ namespace {
 
 constexpr int kBins = 32768;       // 15 bits of the magnitude key
 constexpr int kBlock = 1024;
-// One workgroup as long as it takes no longer than the two (bf16) or three (fp32) launches for larger samples:
-// its counting loop costs 1.3 us per 1024 elements (10 486 fp32: 16 us, 30 000 bf16: 41 us).
-constexpr int kOneItems = 16;
+// One workgroup as long as it takes no longer than the two (bf16) or three (fp32) launches for larger samples: every
+// 1024 elements cost it 2.5 us, the gather of a single compute unit and its counting loop.  A call in one launch and
+// in several, us: bf16 1024 elements 9.8 and 13, 4096 17.8 and 13.6, 8192 28.8 and 14.0; fp32 1024 elements 12.9 and
+// 20, 4096 21.0 and 20.5, 10 486 39.0 and 20.6.
 template <typename S>
-constexpr int64_t one_max() { return (sizeof(S) == 2 ? kOneItems / 2 : kOneItems) * kBlock; }
+constexpr int one_items() { return sizeof(S) == 2 ? 2 : 4; }
+template <typename S>
+constexpr int64_t one_max() { return one_items<S>() * kBlock; }
 constexpr int kGroup = 64;         // bins per sum
 constexpr int kGroups = kBins / kGroup;
 constexpr int kRound = 4;          // elements per thread in flight in the counting kernel
@@ -100,7 +103,7 @@ __device__ inline void gather(const S *__restrict__ in, int64_t n, const int64_t
     }
   }
 #pragma unroll
-  for (int i = 0; i < ITEMS; ++i) v[i] = in[pos[i] >= 0 ? pos[i] : 0];
+  for (int i = 0; i < ITEMS; ++i) v[i] = __builtin_nontemporal_load(in + (pos[i] >= 0 ? pos[i] : 0));
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i)
     if (pos[i] < 0) v[i] = 0;
@@ -119,21 +122,15 @@ __global__ __launch_bounds__(kBlock) void k_sample_one(const S *__restrict__ in,
   __shared__ uint32_t low[2];
   clear_hist(hist);
   if (threadIdx.x < 2) low[threadIdx.x] = 0;
-  S v[kOneItems];
+  constexpr int kItems = one_items<S>();
+  S v[kItems];
+  gather<S, kItems>(in, n, at, threadIdx.x, s, v, status);
 #pragma unroll
-  for (int r = 0; r < kOneItems; r += 8) {  // (a gather of eight at a time)
-    S part[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) part[i] = 0;
-    if ((uint32_t)r * kBlock < s) gather<S, 8>(in, n, at, (int64_t)threadIdx.x + (int64_t)r * kBlock, s, part, status);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[r + i] = part[i] & (S)KeyOf<S>::kMask;
-  }
+  for (int i = 0; i < kItems; ++i) v[i] &= (S)KeyOf<S>::kMask;
   __syncthreads();
   constexpr int kShift = KeyOf<S>::kBits - 15;
 #pragma unroll
-  for (int i = 0; i < kOneItems; ++i) {
-    if ((uint32_t)i * kBlock >= s) break;
+  for (int i = 0; i < kItems; ++i) {
     count_bin(hist, (uint32_t)v[i] >> kShift, threadIdx.x + (uint32_t)i * kBlock < s);
   }
   __syncthreads();
@@ -152,8 +149,7 @@ __global__ __launch_bounds__(kBlock) void k_sample_one(const S *__restrict__ in,
   clear_hist(hist);
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kOneItems; ++i) {
-    if ((uint32_t)i * kBlock >= s) break;
+  for (int i = 0; i < kItems; ++i) {
     const uint32_t key = (uint32_t)v[i];
     count_bin(hist, (key & 0xffffu) >> 1, threadIdx.x + (uint32_t)i * kBlock < s && (key >> 16) == top);
   }
@@ -161,8 +157,7 @@ __global__ __launch_bounds__(kBlock) void k_sample_one(const S *__restrict__ in,
   pick_bin(hist, k - above, smem, &pick);
   const uint32_t high = (top << 15) | pick.bin;
 #pragma unroll
-  for (int i = 0; i < kOneItems; ++i) {
-    if ((uint32_t)i * kBlock >= s) break;
+  for (int i = 0; i < kItems; ++i) {
     const uint32_t key = (uint32_t)v[i];
     const bool live = threadIdx.x + (uint32_t)i * kBlock < s && (key >> 1) == high;
     const uint64_t odd = __ballot(live && (key & 1u)), all = __ballot(live);
@@ -188,8 +183,10 @@ struct SampleTables {
   uint32_t *state;   // fp32: [0] bin, [1] rank inside it, [2] elements above it, [3] members listed, [4] workgroups done
 };
 
-// Bound by the sample's lines: 2.7 M elements of a 537 MB tensor at random places are 344 MB of them, 62 us.  A
-// call took 108 us with the gather kernel and four passes behind it, now 73.
+// Bound by the sample's lines: 2.7 M elements of a 537 MB tensor at random places are 344 MB of them, 62 us at the
+// rate of a copy.  The gather's loads are streamed (nontemporal): of a line one element is wanted, and a tensor of
+// gigabytes would only push others out.  The kernel alone 70 us with plain loads, 63.5 so; with the tensor cold in
+// every cache 120 and 72 a call.
 template <typename S>
 __global__ __launch_bounds__(kBlock) void k_sample_count(const S *__restrict__ in, int64_t n,
                                                          const int64_t *__restrict__ at, int64_t s, int64_t share,
@@ -365,10 +362,16 @@ __global__ __launch_bounds__(kBlock) void k_sample_members(SampleTables tb, int6
   }
 }
 
-// Workgroups of the counting kernel for a sample of s elements: a round each at least, one per compute unit at
-// most (the picking kernel reads a row per workgroup), unless a share outgrew the counters.
+// Workgroups of the counting kernel for a sample of s elements: up to 64, an element per thread (a call for 10 486
+// bf16 elements 14.0 us, with four per thread 18.8; 128 660 on 64 workgroups 19.6, on 32 22.1); beyond that a round
+// of four each, so that the picking kernel, which reads a row per workgroup, has fewer (619 534 elements: 151 rows
+// 29.5, 256 rows 31.4); one per compute unit at most, unless a share outgrew the counters.
+constexpr int64_t kSpread = 64;
 inline int64_t sample_groups(int64_t s) {
-  int64_t g = ceil_div(s, (int64_t)kRound * kBlock);
+  int64_t g = ceil_div(s, (int64_t)kBlock);
+  if (g > kSpread) g = kSpread;
+  const int64_t full = ceil_div(s, (int64_t)kRound * kBlock);
+  if (g < full) g = full;
   if (g > 256) g = 256;
   const int64_t least = ceil_div(s, kShare);
   return g < least ? least : g;
