@@ -370,6 +370,46 @@ def test_a_kept_buffer_is_waited_for_and_held_by_every_stream(monkeypatch, captu
     assert log == ([] if capturing else [("wait", 2, 1), ("hold", 2), ("wait", 3, 1), ("hold", 3)])
 
 
+def test_streams_wait_for_a_call_that_returned_before_its_kernels_were_through(monkeypatch):
+    """Split sizes reach the host before the last kernel of a load balance is done with the workspace: the streams
+    that have used it before wait for the call's stream at their next use, the call's own does not."""
+    from zen_repro_amd import _lib
+
+    log = []
+
+    class Stream:
+        def __init__(self, handle):
+            self.cuda_stream = handle
+
+        def wait_stream(self, other):
+            log.append((self.cuda_stream, other.cuda_stream))
+
+    class Buffer:
+        def numel(self):
+            return 256
+
+        def record_stream(self, stream):
+            pass
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    streams = {h: Stream(h) for h in (1, 2, 3)}
+    now = [1]
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: streams[now[0]])
+    monkeypatch.setattr(_lib, "current_handle", lambda index: now[0])
+    device = torch.device("cuda", 0)
+    scratch = _lib.Scratch()
+    scratch._bufs()[0, "a"] = _lib.Kept(Buffer(), streams[1])
+    scratch.left_running(device, "a")  # stream 1, the only one so far
+    now[0] = 2
+    scratch.get(device, "a", 1)
+    assert log == [(2, 1)]
+    scratch.left_running(device, "a")
+    for now[0] in (2, 1, 2, 1):
+        scratch.get(device, "a", 1)
+    scratch.get(device, "a", 1, stream=streams[3])
+    assert log == [(2, 1), (1, 2), (3, 2)]
+
+
 def test_compaction_kernels_keep_their_rows_in_registers(tmp_path):
     """The rows a wave has in flight are the kernels' speed: none of their registers may end up in memory, for
     aligned tensors and for views that begin at an odd element."""

@@ -232,6 +232,13 @@ class Kept:
             self.buf.record_stream(stream)
             self.seen.add(stream.cuda_stream)
 
+    def left_running(self, device):
+        """A call that waits for its sizes has returned while its last kernels may still use the buffer on the
+        current stream: every other stream waits for that at its next use, like for the making."""
+        if len(self.seen) > 1:  # else no stream but this one has used it
+            self.maker = torch.cuda.current_stream(device)
+            self.seen = {self.maker.cuda_stream}
+
 
 class Scratch:
     """Cache of raw byte buffers per device and host thread, grown on demand
@@ -268,6 +275,10 @@ class Scratch:
         elif (stream.cuda_stream if stream is not None else current_handle(index)) not in kept.seen:
             kept.join(torch.cuda.current_stream(index) if stream is None else stream)
         return kept.buf
+
+    def left_running(self, device, name):
+        """See Kept.left_running."""
+        self._bufs()[device_index(device), name].left_running(device)
 
     def drop(self):
         """Forget the calling thread's buffers."""

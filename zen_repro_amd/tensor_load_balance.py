@@ -384,6 +384,7 @@ class TensorPartition:
         nbytes = L.zen_load_balance_workspace(n, m, code, capacity, self.partitions)
         ws = _lib.scratch.get(dev, f"load_balance/{slot}", nbytes)
         table = self._table(dev, m, slot)
+        kept = self._tables[dev, m, slot]
         flags, used = self._take_ahead(flat, n, int(k), capacity, ws, slot, mode, thr, near)
         if near is not None and k > 0 and thr is None:
             thr, flags = near, flags | _lib.MODE_FLOOR
@@ -397,6 +398,9 @@ class TensorPartition:
         if rc != _lib.OK:
             table.zero_()  # a call that failed half way may have left entries behind
         _lib.check(rc, "load_balance")
+        if words is not None:
+            _lib.scratch.left_running(dev, f"load_balance/{slot}")
+            kept.left_running(dev)
         self._after_call(flat, int(k), capacity, slot, mode | flags, used)
         return out_idx, out_val, splits, status
 
