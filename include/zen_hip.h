@@ -571,6 +571,14 @@ int zen_count(const void *input, int dtype, int64_t n, const uint32_t *thr, int6
 size_t zen_table_lists_workspace(int64_t m, int partitions);
 int zen_table_find(const int32_t *table, int64_t m, int partitions, int64_t n, int64_t *splits, void *workspace,
                    size_t workspace_bytes, int32_t *status, void *stream);
+/*
+ * zen_table_find, of at most ZEN_TABLE_SIZES_MOST partitions, that returns when the split sizes and then *status are in the host words [1, partitions + 2), `host`
+ * and `words` from zen_host_words_alloc (at least partitions + 2).  marks: 2 * partitions + 66 zeroed device words.
+ */
+#define ZEN_TABLE_SIZES_MOST 1024
+int zen_table_find_sizes(const int32_t *table, int64_t m, int partitions, int64_t n, int64_t *splits, int64_t *marks,
+                         void *workspace, size_t workspace_bytes, int32_t *status, int64_t *host, int64_t words,
+                         void *stream);
 int zen_table_gather(const int32_t *table, int64_t m, int partitions, const void *input, int dtype, int64_t n,
                      int32_t *out_idx, void *out_val, int64_t total, void *workspace, size_t workspace_bytes,
                      void *stream);

@@ -258,6 +258,37 @@ def test_table_lists(zen, oracle, m, parts, shift, density, dtype):
     assert np.array_equal(to_np(torch.cat(idx)), want) and np.array_equal(to_np(torch.cat(val)), g[want])
 
 
+@pytest.mark.parametrize("m, parts", [(1, 1), (5000, 1), (1 << 24, 1), ((1 << 23) + 4, 5), (16400, 1024), (16400, 1025)])
+def test_table_lists_by_either_entry(zen, m, parts):
+    # the walk that adds up the partitions' sizes itself (one to 64 groups of workgroups a partition, partitions of a
+    # single one) and the one with a workgroup behind it for that; the gather that follows either
+    from zen_repro_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(m + parts)
+    n = 100000
+    table = torch.randint(1, n, (m,), generator=gen, device="cuda", dtype=torch.int32)
+    table *= torch.rand(m, generator=gen, device="cuda") < 0.05
+    grad = torch.randn(n, generator=gen, device="cuda")
+    cut = table[:m // parts * parts]
+    want, sizes = cut[cut != 0], (cut.view(parts, -1) != 0).sum(1)
+    idx, val, splits = zen.TensorPartition(parts, 1, 3).get_sub_sparse_tensors(grad, table)
+    assert torch.equal(splits, sizes) and [t.numel() for t in idx] == sizes.tolist()
+    assert torch.equal(torch.cat(idx), want) and torch.equal(torch.cat(val), grad[want.long()])
+    L, dev = _lib.lib(), table.device
+    ws = torch.empty(L.zen_table_lists_workspace(m, parts), dtype=torch.uint8, device=dev)
+    splits, status = torch.full((parts,), -1, device=dev), torch.zeros(1, dtype=torch.int32, device=dev)
+    assert L.zen_table_find(_lib.ptr(table), m, parts, n, _lib.ptr(splits), _lib.ptr(ws), ws.numel(), _lib.ptr(status),
+                            _lib.stream_of(dev)) == 0
+    total = int(sizes.sum())
+    out_idx, out_val = torch.empty_like(want), torch.empty(total, device=dev)
+    assert L.zen_table_gather(_lib.ptr(table), m, parts, _lib.ptr(grad), 0, n, _lib.ptr(out_idx), _lib.ptr(out_val), total,
+                              _lib.ptr(ws), ws.numel(), _lib.stream_of(dev)) == 0
+    assert torch.equal(splits, sizes) and torch.equal(out_idx, want) and torch.equal(out_val, grad[want.long()])
+    words = _lib.host_words(parts + 1)
+    rc = L.zen_table_find_sizes(_lib.ptr(table), m, parts, n, _lib.ptr(splits), None, _lib.ptr(ws), ws.numel(),
+                                _lib.ptr(status), words.ptr, words.words, _lib.stream_of(dev))
+    assert rc == -1  # the zeroed words are missing
+
+
 def test_table_lists_what_torch_indexes(zen):
     # an entry past the tensor is an error; autograd, other types and strided tensors are indexed by torch
     g = torch.arange(100, dtype=torch.float32, device="cuda") + 1

@@ -25,6 +25,7 @@ LIB_PATH = os.environ.get("ZEN_HIP_LIB") or os.path.join(_HERE, "csrc", "libzen_
 
 # ZEN_ABI_VERSION of include/zen_hip.h this loader's signatures and structs are written for
 ABI_VERSION = 7
+TABLE_SIZES_MOST = 1024  # ZEN_TABLE_SIZES_MOST
 
 _lib = None
 
@@ -126,6 +127,7 @@ def lib():
         "zen_count": (i32, [vp, i32, i64, vp, vp, vp]),
         "zen_table_lists_workspace": (sz, [i64, i32]),
         "zen_table_find": (i32, [vp, i64, i32, i64, vp, vp, sz, vp, vp]),
+        "zen_table_find_sizes": (i32, [vp, i64, i32, i64, vp, vp, vp, sz, vp, vp, i64, vp]),
         "zen_table_gather": (i32, [vp, i64, i32, vp, i32, i64, vp, vp, i64, vp, sz, vp]),
         "zen_stream_read": (i32, [vp, sz, vp, vp]),
         "zen_profile_enable": (i32, [i32]),

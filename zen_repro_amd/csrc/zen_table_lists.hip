@@ -3,10 +3,10 @@
 //
 // Every partition is cut into stretches of equal length, one per wave, so that no stretch crosses a partition's
 // edge and the split sizes are sums of whole stretches.  k_table_walk leaves a stretch's entries side by side in the
-// workspace, k_table_offsets turns the stretches' counts into places and split sizes, and, once the host has made
-// buffers of just that size, k_table_gather moves the entries there and fetches their values.
+// workspace and its last workgroup tells the host the split sizes; once the host has made buffers of just that size,
+// k_table_gather moves the entries there and fetches their values.
 // Bound by the read of the table and by the random lines the values lie on.  16.7 M slots of 5 % filled, eight
-// partitions, bf16: 18 + 9 + 18 us, and with the wait for the sizes and the overflow region 130 us for the two calls.
+// partitions, bf16: 21 + 18 us.
 // A compaction to (position, entry) lists, a search for the partitions' edges and two library launches per
 // partition for the values took 330 us there, in 35 launches instead of 8.
 #include "zen_common.h"
@@ -21,6 +21,14 @@ constexpr int64_t kStep = kRow * kRows;
 constexpr int64_t kMaxStretches = 8192;    // 32 waves per compute unit
 constexpr int kScanBlock = 1024;
 constexpr int kMoveBlock = 256;
+
+// Up to here the walk adds up the partitions' sizes while it runs and the gather finds its places from the stretches'
+// counts; with more partitions one workgroup does both in between (16.7 M slots, eight partitions: walk 15.6, sizes
+// and places 8.5, read-back for the host 2.5 us and two gaps between launches; now 21 in one, the call's table, lists
+// and those of its overflow region together 203 -> 197 us).  The bound keeps the marks and the answer small; sums over
+// the counts, at most 8192 of them up to here, would grow with the partitions.
+constexpr int kMostMarked = ZEN_TABLE_SIZES_MOST;
+constexpr int kMarkGroup = 32;             // workgroups that count themselves as finished in one word
 
 struct TablePlan {
   int64_t per_part;  // slots of a partition
@@ -49,11 +57,20 @@ TablePlan plan_table(void *workspace, int64_t m, int partitions, size_t *bytes) 
 
 __device__ inline bool filled(int32_t e) { return (e & 0x7fffffff) != 0; }
 
-__global__ __launch_bounds__(kBlock, 8) void k_table_walk(const int32_t *__restrict__ table, int64_t n, TablePlan tp,
-                                                          int32_t *status) {
-  const int64_t w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)));
-  if (w >= tp.count) return;
-  const int64_t part = w / tp.cpp;
+// Zeroed words in which finished workgroups count themselves and their entries: per group of up to kMarkGroup
+// workgroups of a partition, then per partition, then once per partition in `done`.  (Adds to one word are carried out
+// one after the other, 11 ns each.)
+struct TableMarks {
+  unsigned long long *group;
+  unsigned long long *part;
+  uint32_t *done;
+  uint32_t parts, per_part, groups;  // partitions; workgroups and groups of one
+};
+constexpr int kMarkShift = 40;  // arrivals above, entries below
+
+// The entries of stretch w (of partition `part`) to the workspace: how many there are; `bad` if one is no index.
+__device__ inline uint32_t walk_stretch(const int32_t *__restrict__ table, int64_t n, const TablePlan &tp, int64_t part,
+                                        int64_t w, bool &bad) {
   const int64_t lo = part * tp.per_part + (w - part * tp.cpp) * tp.len;
   const int64_t last = (part + 1) * tp.per_part;
   const int64_t hi = lo + tp.len < last ? lo + tp.len : last;
@@ -78,7 +95,6 @@ __global__ __launch_bounds__(kBlock, 8) void k_table_walk(const int32_t *__restr
   };
   int32_t *out = tp.entries + lo;
   uint32_t found = 0;
-  bool bad = false;
   int4 q[kRows], next[kRows];
   load(first, next);
 #pragma unroll 1
@@ -104,11 +120,69 @@ __global__ __launch_bounds__(kBlock, 8) void k_table_walk(const int32_t *__restr
       found += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
     }
   }
-  const uint64_t any_bad = __ballot(bad);
-  if (lane == 0) {
-    tp.found[w] = found;
-    if (any_bad) atomicOr(status, ZEN_STAT_BAD_INDEX);
+  return found;
+}
+
+template <bool MARKED>
+__global__ __launch_bounds__(kBlock, 8) void k_table_walk(const int32_t *__restrict__ table, int64_t n, TablePlan tp,
+                                                          TableMarks marks, int64_t *__restrict__ splits,
+                                                          HostAnswer answer, int32_t *status) {
+  constexpr int kWaves = kBlock / 64;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  int64_t part, w;
+  if (MARKED) {  // a workgroup's stretches are of one partition
+    part = blockIdx.x / marks.per_part;
+    w = (int64_t)(blockIdx.x - (uint32_t)part * marks.per_part) * kWaves + wave;
+    w = w < tp.cpp ? part * tp.cpp + w : tp.count;
+  } else {
+    w = (int64_t)blockIdx.x * kWaves + wave;
+    part = w / tp.cpp;
   }
+  uint32_t found = 0;
+  if (w < tp.count) {
+    bool bad = false;
+    found = walk_stretch(table, n, tp, part, w, bad);
+    const uint64_t any_bad = __ballot(bad);
+    if (lane_id() == 0) {
+      tp.found[w] = found;
+      if (any_bad) atomicOr(status, ZEN_STAT_BAD_INDEX);
+    }
+  }
+  if (!MARKED) return;
+  __shared__ uint32_t held[kWaves];
+  __shared__ bool last;
+  if (lane_id() == 0) {
+    held[wave] = found;
+    wait_global_acks();  // the wave's share of the status word
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    constexpr unsigned long long kEntries = (1ull << kMarkShift) - 1ull, kArrived = 1ull << kMarkShift;
+    unsigned long long mine = 0;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) mine += held[i];
+    const uint32_t own = blockIdx.x - (uint32_t)part * marks.per_part;
+    const uint32_t group = own / kMarkGroup;
+    const uint32_t left = marks.per_part - group * kMarkGroup;
+    last = false;
+    unsigned long long old = atomicAdd(&marks.group[(uint32_t)part * marks.groups + group], kArrived | mine);
+    if ((old >> kMarkShift) + 1u == (left < (uint32_t)kMarkGroup ? left : (uint32_t)kMarkGroup)) {
+      mine += old & kEntries;
+      old = atomicAdd(&marks.part[part], kArrived | mine);
+      if ((old >> kMarkShift) + 1u == marks.groups) last = atomicAdd(marks.done, 1u) == marks.parts - 1u;
+    }
+  }
+  __syncthreads();
+  if (!last) return;
+  for (uint32_t p = threadIdx.x; p < marks.parts; p += kBlock) {
+    const int64_t size = (int64_t)(__hip_atomic_load(&marks.part[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
+                                   ((1ull << kMarkShift) - 1ull));
+    splits[p] = size;
+    host_store(answer.host + 1 + p, size);
+  }
+  if (threadIdx.x == 0)
+    host_store(answer.host + 1 + marks.parts, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  host_answered(answer);
 }
 
 // Places of the stretches and the partitions' sizes.  One workgroup, one round: there are 8192 stretches unless there
@@ -140,15 +214,37 @@ __global__ __launch_bounds__(kScanBlock) void k_table_offsets(TablePlan tp, int 
     splits[p] = (int64_t)tp.at[(p + 1) * tp.cpp] - (int64_t)tp.at[p * tp.cpp];
 }
 
-template <typename S>
+// PLACED: k_table_offsets has left the stretches' places; else they are sums of the counts in front of them.
+template <typename S, bool PLACED>
 __global__ __launch_bounds__(kMoveBlock) void k_table_gather(const S *__restrict__ in, int64_t n, TablePlan tp,
                                                              int32_t *__restrict__ out_idx, S *__restrict__ out_val,
                                                              int64_t total) {
-  const int64_t w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kMoveBlock / 64) + (threadIdx.x >> 6)));
+  constexpr int kWaves = kMoveBlock / 64;
+  static_assert(kWaves == 4, "a workgroup's counts are a vector");
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t w = (int64_t)blockIdx.x * kWaves + wave;
+  uint32_t at = 0;
+  if (!PLACED) {
+    __shared__ uint32_t sums[kWaves];
+    const uint4 *found = reinterpret_cast<const uint4 *>(tp.found);
+    uint32_t sum = 0;
+#pragma unroll 8
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kMoveBlock) {
+      const uint4 q = found[i];
+      sum += (q.x + q.y) + (q.z + q.w);
+    }
+    sum = wave_sum(sum);
+    if (lane_id() == 0) sums[wave] = sum;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) at += sums[i];
+    for (int i = 0; i < wave; ++i) at += w < tp.count ? tp.found[(int64_t)blockIdx.x * kWaves + i] : 0u;
+    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+  }
   if (w >= tp.count) return;
+  if (PLACED) at = tp.at[w];
   const int64_t part = w / tp.cpp;
   const int32_t *from = tp.entries + part * tp.per_part + (w - part * tp.cpp) * tp.len;
-  const uint32_t at = tp.at[w];
   const uint32_t mine = tp.found[w];
   constexpr uint32_t kAhead = 4;
   for (uint32_t i0 = 0; i0 < mine; i0 += 64 * kAhead) {
@@ -173,6 +269,26 @@ __global__ __launch_bounds__(kMoveBlock) void k_table_gather(const S *__restrict
       }
     }
   }
+}
+
+int table_find(const int32_t *table, int64_t n, const TablePlan &tp, int partitions, int64_t *splits, int32_t *status,
+               hipStream_t s) {
+  k_table_walk<false><<<dim3((unsigned)ceil_div(tp.count, kBlock / 64)), dim3(kBlock), 0, s>>>(
+      table, n, tp, TableMarks{}, nullptr, HostAnswer{}, status);
+  ZEN_LAUNCH_CHECK("k_table_walk");
+  k_table_offsets<<<dim3(1), dim3(kScanBlock), 0, s>>>(tp, partitions, splits);
+  ZEN_LAUNCH_CHECK("k_table_offsets");
+  return ZEN_OK;
+}
+
+template <typename S>
+int table_gather(const void *input, int64_t n, const TablePlan &tp, int partitions, int32_t *out_idx, void *out_val,
+                 int64_t total, hipStream_t s) {
+  const auto kernel = partitions > kMostMarked ? k_table_gather<S, true> : k_table_gather<S, false>;
+  kernel<<<dim3((unsigned)ceil_div(tp.count, kMoveBlock / 64)), dim3(kMoveBlock), 0, s>>>(
+      static_cast<const S *>(input), n, tp, out_idx, static_cast<S *>(out_val), total);
+  ZEN_LAUNCH_CHECK("k_table_gather");
+  return ZEN_OK;
 }
 
 int table_args(const char *what, const int32_t *table, int64_t m, int partitions, int64_t n, void *workspace,
@@ -205,11 +321,34 @@ int zen_table_find(const int32_t *table, int64_t m, int partitions, int64_t n, i
   hipStream_t s = static_cast<hipStream_t>(stream);
   size_t bytes;
   const TablePlan tp = plan_table(workspace, m, partitions, &bytes);
-  k_table_walk<<<dim3((unsigned)ceil_div(tp.count, kBlock / 64)), dim3(kBlock), 0, s>>>(table, n, tp, status);
+  return table_find(table, n, tp, partitions, splits, status, s);
+}
+
+int zen_table_find_sizes(const int32_t *table, int64_t m, int partitions, int64_t n, int64_t *splits, int64_t *marks,
+                         void *workspace, size_t workspace_bytes, int32_t *status, int64_t *host, int64_t words,
+                         void *stream) {
+  using namespace zen;
+  if (!splits || !marks || !status) return fail(ZEN_EINVAL, "zen_table_find_sizes: null pointer");
+  if (partitions > kMostMarked) return fail(ZEN_EINVAL, "zen_table_find_sizes: too many partitions");
+  int rc = table_args("zen_table_find_sizes: bad argument or workspace", table, m, partitions, n, workspace,
+                      workspace_bytes);
+  if (rc != ZEN_OK) return rc;
+  HostAnswer answer;
+  rc = host_ask(host, words, (int64_t)partitions + 1, &answer);
+  if (rc != ZEN_OK) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  size_t bytes;
+  const TablePlan tp = plan_table(workspace, m, partitions, &bytes);
+  TableMarks tm;
+  tm.parts = (uint32_t)partitions;
+  tm.per_part = (uint32_t)ceil_div(tp.cpp, (int64_t)(kBlock / 64));
+  tm.groups = (uint32_t)ceil_div((int64_t)tm.per_part, (int64_t)kMarkGroup);
+  tm.group = reinterpret_cast<unsigned long long *>(marks);
+  tm.part = tm.group + (size_t)tm.groups * tm.parts;
+  tm.done = reinterpret_cast<uint32_t *>(tm.part + tm.parts);
+  k_table_walk<true><<<dim3(tm.per_part * tm.parts), dim3(kBlock), 0, s>>>(table, n, tp, tm, splits, answer, status);
   ZEN_LAUNCH_CHECK("k_table_walk");
-  k_table_offsets<<<dim3(1), dim3(kScanBlock), 0, s>>>(tp, partitions, splits);
-  ZEN_LAUNCH_CHECK("k_table_offsets");
-  return ZEN_OK;
+  return host_wait(answer, s);
 }
 
 int zen_table_gather(const int32_t *table, int64_t m, int partitions, const void *input, int dtype, int64_t n,
@@ -225,15 +364,8 @@ int zen_table_gather(const int32_t *table, int64_t m, int partitions, const void
   hipStream_t s = static_cast<hipStream_t>(stream);
   size_t bytes;
   const TablePlan tp = plan_table(workspace, m, partitions, &bytes);
-  const dim3 grid((unsigned)ceil_div(tp.count, kMoveBlock / 64));
-  if (dtype == ZEN_BF16)
-    k_table_gather<uint16_t><<<grid, dim3(kMoveBlock), 0, s>>>(static_cast<const uint16_t *>(input), n, tp, out_idx,
-                                                              static_cast<uint16_t *>(out_val), total);
-  else
-    k_table_gather<uint32_t><<<grid, dim3(kMoveBlock), 0, s>>>(static_cast<const uint32_t *>(input), n, tp, out_idx,
-                                                              static_cast<uint32_t *>(out_val), total);
-  ZEN_LAUNCH_CHECK("k_table_gather");
-  return ZEN_OK;
+  return dtype == ZEN_BF16 ? table_gather<uint16_t>(input, n, tp, partitions, out_idx, out_val, total, s)
+                           : table_gather<uint32_t>(input, n, tp, partitions, out_idx, out_val, total, s);
 }
 
 }  // extern "C"

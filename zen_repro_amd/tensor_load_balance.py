@@ -98,13 +98,22 @@ class TensorPartition:
         L = _lib.lib()
         dev = flat.device
         m, n = memory.numel(), flat.numel()
-        splits = _lib.zeros.take(dev, self.partitions, torch.int64)
+        parts = self.partitions
+        # beside the split sizes, the words in which the walk adds them up
+        splits, marks = _lib.zeros.take(dev, 3 * parts + 66, torch.int64).split((parts, 2 * parts + 66))
         status = _lib.status_word(dev)
         # not from the scratch cache: this thread may walk another table before these lists are used up
-        ws = torch.empty(L.zen_table_lists_workspace(m, self.partitions), dtype=torch.uint8, device=dev)
-        _lib.check(L.zen_table_find(_lib.ptr(memory), m, self.partitions, n, _lib.ptr(splits), _lib.ptr(ws),
-                                    ws.numel(), _lib.ptr(status), _lib.stream_of(dev)), "table_find")
-        host = _lib.read_back(splits, status)
+        ws = torch.empty(L.zen_table_lists_workspace(m, parts), dtype=torch.uint8, device=dev)
+        if parts <= _lib.TABLE_SIZES_MOST:
+            words = _lib.host_words(parts + 1)
+            _lib.check(L.zen_table_find_sizes(_lib.ptr(memory), m, parts, n, _lib.ptr(splits), _lib.ptr(marks),
+                                              _lib.ptr(ws), ws.numel(), _lib.ptr(status), words.ptr, words.words,
+                                              _lib.stream_of(dev)), "table_find")
+            host = words.view[1:parts + 2]
+        else:
+            _lib.check(L.zen_table_find(_lib.ptr(memory), m, parts, n, _lib.ptr(splits), _lib.ptr(ws), ws.numel(),
+                                        _lib.ptr(status), _lib.stream_of(dev)), "table_find")
+            host = _lib.read_back(splits, status)
         if host[-1]:
             raise IndexError("get_sub_sparse_tensors: " + _lib.describe_status(host[-1]))
         sizes = host[:-1]
