@@ -237,6 +237,16 @@ int zen_select(const void *input, int dtype, int64_t n, const uint32_t *thr,
                void *out_idx, int idx64, void *out_val, int64_t capacity,
                int64_t *out_count, void *workspace, size_t workspace_bytes,
                int32_t *status, void *stream);
+/*
+ * zen_select that returns when the count and *status are in the host words 1
+ * and 2, `host` and `words` from zen_host_words_alloc (at least 3).  The
+ * entries are complete on the stream, as always, and so is the use of the
+ * workspace.
+ */
+int zen_select_count(const void *input, int dtype, int64_t n, const uint32_t *thr,
+                     void *out_idx, int idx64, void *out_val, int64_t capacity,
+                     int64_t *out_count, void *workspace, size_t workspace_bytes,
+                     int32_t *status, int64_t *host, int64_t words, void *stream);
 
 /* ---------------------------------------------------------- load balance */
 
@@ -458,6 +468,11 @@ int zen_decode_dense(const void *idx, int idx64_in, const void *val, int dtype,
                      int64_t r, void *dense, int64_t dense_n, int mode,
                      void *workspace, size_t workspace_bytes,
                      int32_t *status, void *stream);
+/* zen_decode_dense that returns when *status is in host word 1, `host` and `words` from zen_host_words_alloc (at
+ * least 2). */
+int zen_decode_dense_status(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, void *dense,
+                            int64_t dense_n, int mode, void *workspace, size_t workspace_bytes, int32_t *status,
+                            int64_t *host, int64_t words, void *stream);
 
 /*
  * The same for payloads that arrive as `nlists` strictly ascending index lists back to back (list l is

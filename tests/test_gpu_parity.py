@@ -1101,3 +1101,26 @@ def test_count_the_host_is_told_by_the_merge(zen, r, n, dtype):
         lba.fast_flags = flags
         got_idx, got_val = lba.merge_rounded(idx, val, n, dtype)
         assert torch.equal(got_idx, at) and torch.equal(got_val, want[at].to(dtype))
+
+
+@pytest.mark.parametrize("n", [1, 65536, 65537, 1000003])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_count_the_host_is_told_by_the_selection(zen, n, dtype):
+    """In one workgroup and in stretches, with room for all and for some; the workspace is used again at once, by the
+    same stream and by another one."""
+    from zen_repro_amd import comm
+
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    a, b = ((torch.randn(n, generator=gen, device="cuda") *
+             (torch.rand(n, generator=gen, device="cuda") < 0.3)).to(dtype) for _ in range(2))
+    want = [torch.nonzero(t).view(-1) for t in (a, b)]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    for capacity in (n, max(1, want[0].numel() // 2)):
+        out = [comm._select_raw(a, None, True, capacity), comm._select_raw(b, None, True, n)]
+        with torch.cuda.stream(side):
+            out.append(comm._select_raw(a, None, True, capacity))
+        torch.cuda.synchronize()
+        for (idx, val, count, bits), at, t, room in zip(out, (want[0], want[1], want[0]), (a, b, a), (capacity, n, capacity)):
+            assert count == at.numel() and bits == (zen._lib.STAT_CAPACITY if count > room else 0)
+            assert torch.equal(idx, at[:room]) and torch.equal(val, t[at[:room]])

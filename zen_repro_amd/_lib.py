@@ -91,6 +91,7 @@ def lib():
         "zen_compress": (i32, [vp, i32, i64, vp, vp, vp]),
         "zen_select_workspace": (sz, [i64, i32]),
         "zen_select": (i32, [vp, i32, i64, vp, vp, i32, vp, i64, vp, vp, sz, vp, vp]),
+        "zen_select_count": (i32, [vp, i32, i64, vp, vp, i32, vp, i64, vp, vp, sz, vp, vp, i64, vp]),
         "zen_load_balance_workspace": (sz, [i64, i64, i32, i64, i32]),
         "zen_load_balance": (i32, [vp, i32, i64, i64, i32, i32, vp, i64, vp, vp, vp, i64, vp, vp, i32, vp, sz, vp, vp]),
         "zen_load_balance_sizes": (i32, [vp, i32, i64, i64, i32, i32, vp, i64, vp, vp, vp, i64, vp, vp, i32, vp, sz, vp, vp, i64,
@@ -108,6 +109,7 @@ def lib():
                                          sz, vp, vp]),
         "zen_decode_dense_workspace": (sz, [i64, i64]),
         "zen_decode_dense": (i32, [vp, i32, vp, i32, i64, vp, i64, i32, vp, sz, vp, vp]),
+        "zen_decode_dense_status": (i32, [vp, i32, vp, i32, i64, vp, i64, i32, vp, sz, vp, vp, i64, vp]),
         "zen_decode_dense_sorted_workspace": (sz, [i64, i32]),
         "zen_decode_dense_sorted": (i32, [vp, i32, vp, i32, ctypes.POINTER(ctypes.c_int64), i32, vp, i64, vp, sz, vp, vp]),
         "zen_bitmap_dense_dict_bytes": (sz, [i64, i32]),

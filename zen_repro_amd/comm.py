@@ -28,7 +28,7 @@ class LocalGroup:
 def _select_raw(tensor, thr, idx64, capacity=None):
     """(indices, values, count, status bits) of the selected elements of a flat tensor, ascending; the count
     is that of all elements that pass, also beyond `capacity` (then the bits hold STAT_CAPACITY and the first
-    `capacity` entries are there).  Synchronises."""
+    `capacity` entries are there).  Waits for the count; the entries are complete on the current stream."""
     flat = tensor.reshape(-1)
     n = flat.numel()
     dev = flat.device
@@ -41,11 +41,13 @@ def _select_raw(tensor, thr, idx64, capacity=None):
     count = _lib.zeros.word(dev, torch.int64)
     status = _lib.status_word(dev)
     ws = _lib.scratch.get(dev, "select", L.zen_select_workspace(n, code))
-    rc = L.zen_select(_lib.ptr(flat), code, n, _lib.ptr(thr), _lib.ptr(out_idx), 1 if idx64 else 0,
-                      _lib.ptr(out_val), capacity, _lib.ptr(count), _lib.ptr(ws), ws.numel(),
-                      _lib.ptr(status), _lib.stream_of(dev))
+    words = _lib.host_words(2)
+    rc = L.zen_select_count(_lib.ptr(flat), code, n, _lib.ptr(thr), _lib.ptr(out_idx), 1 if idx64 else 0,
+                            _lib.ptr(out_val), capacity, _lib.ptr(count), _lib.ptr(ws), ws.numel(),
+                            _lib.ptr(status), words.ptr, words.words, _lib.stream_of(dev))
     _lib.check(rc, "select")
-    host = _lib.read_back(count, status)
+    _lib.scratch.left_running(dev, "select")
+    host = words.view[1:3]
     kept = min(host[0], capacity)
     return out_idx[:kept], out_val[:kept], host[0], host[1]
 
@@ -118,14 +120,15 @@ class LoadBalanceAllreduce:
         ws = _lib.scratch.get(dev, "decode", L.zen_decode_dense_workspace(r, alltoall_dense_size), zero=True)
         for mode in self._fast_then_general():
             status = _lib.status_word(dev)
-            rc = L.zen_decode_dense(_lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(values),
-                                    _lib.dtype_code(values), r, _lib.ptr(dense), alltoall_dense_size,
-                                    mode | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status),
-                                    _lib.stream_of(dev))
+            words = _lib.host_words(1)
+            rc = L.zen_decode_dense_status(_lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(values),
+                                           _lib.dtype_code(values), r, _lib.ptr(dense), alltoall_dense_size,
+                                           mode | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status),
+                                           words.ptr, words.words, _lib.stream_of(dev))
             if rc != _lib.OK:
                 ws[:L.zen_merge_zero_bytes()].zero_()
             _lib.check(rc, "decode_sparse_tensors")
-            bits = _lib.read_back(status)[0]  # the reference's scatter_add_ raises on a bad index, also a sync
+            bits = words.view[1]  # the reference's scatter_add_ raises on a bad index, also a sync
             if bits & (_lib.STAT_RETRY | _lib.STAT_INTERNAL):
                 ws[:L.zen_merge_zero_bytes()].zero_()
             if not bits & _lib.STAT_RETRY:

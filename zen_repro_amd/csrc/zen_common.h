@@ -202,13 +202,13 @@ __device__ inline void host_answered(const HostAnswer &a) {
   __syncthreads();
   if (threadIdx.x == 0) host_store(a.host, a.ticket);
 }
-// The status word (and a count in front of it, where there is one), once every workgroup that changes them has been
-// waited for.  By the whole workgroup.
+// A count and the status word behind it (no count: the status word alone), once every workgroup that changes them has
+// been waited for.  By the whole workgroup.
 __device__ inline void host_answer_count(const HostAnswer &a, const int64_t *count, const int32_t *status) {
   if (!a.host) return;
   if (threadIdx.x == 0) {
-    host_store(a.host + 1, count ? __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0);
-    host_store(a.host + 2, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (count) host_store(a.host + 1, __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    host_store(a.host + (count ? 2 : 1), (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   }
   host_answered(a);
 }

@@ -199,11 +199,26 @@ __global__ __launch_bounds__(kBlock, 8) void k_compact_walk(const S *__restrict_
   if (lane_id() == 0) st.found[w] = found;
 }
 
+// By the one thread that knows how many there are.  The host goes on from here, beside the move.
+__device__ inline void count_known(uint64_t all, int64_t capacity, int64_t *out_count, const HostAnswer &answer,
+                                   int32_t *status) {
+  *out_count = (int64_t)all;
+  int32_t bits = 0;
+  if (all > (uint64_t)capacity) bits = atomicOr(status, ZEN_STAT_CAPACITY) | ZEN_STAT_CAPACITY;
+  else if (answer.host) bits = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!answer.host) return;
+  host_store(answer.host + 1, (int64_t)all);
+  host_store(answer.host + 2, (int64_t)bits);
+  wait_global_acks();
+  host_store(answer.host, answer.ticket);
+}
+
 template <typename S, typename I, bool ALIGNED>
 __global__ __launch_bounds__(kMoveBlock) void k_compact_move(const S *__restrict__ in, int64_t n,
                                                              const uint32_t *__restrict__ thr, Stretches st,
                                                              I *__restrict__ out_idx, S *__restrict__ out_val,
-                                                             int64_t capacity, int64_t *out_count, int32_t *status) {
+                                                             int64_t capacity, int64_t *out_count, HostAnswer answer,
+                                                             int32_t *status) {
   __shared__ uint32_t part[kMoveWaves];
   __shared__ uint32_t own[kMoveWaves];
   const uint32_t first = blockIdx.x * (uint32_t)kMoveWaves;
@@ -222,10 +237,8 @@ __global__ __launch_bounds__(kMoveBlock) void k_compact_move(const S *__restrict
   uint64_t at = 0;
 #pragma unroll
   for (uint32_t i = 0; i < (uint32_t)kMoveWaves; ++i) at += part[i] + (i < wave ? own[i] : 0u);
-  if (w + 1 == st.count && lane_id() == 0) {
-    *out_count = (int64_t)(at + mine);
-    if (at + mine > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
-  }
+  if (w + 1 == st.count && lane_id() == 0)
+    count_known(at + mine, capacity, out_count, answer, status);
   if (w >= st.count) return;
   at = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) |
        (uint32_t)__builtin_amdgcn_readfirstlane((int)at);  // the same in every lane
@@ -263,7 +276,7 @@ template <typename S, typename I, bool ALIGNED>
 __global__ __launch_bounds__(kMoveBlock) void k_compact_one(const S *__restrict__ in, int64_t n,
                                                             const uint32_t *__restrict__ thr, I *__restrict__ out_idx,
                                                             S *__restrict__ out_val, int64_t capacity,
-                                                            int64_t *out_count, int32_t *status) {
+                                                            int64_t *out_count, HostAnswer answer, int32_t *status) {
   __shared__ uint32_t own[kMoveWaves];
   const uint32_t wave = threadIdx.x >> 6;
   const uint32_t least = least_key(thr, KeyOf<S>::kMask);
@@ -279,21 +292,18 @@ __global__ __launch_bounds__(kMoveBlock) void k_compact_one(const S *__restrict_
     at += i < wave ? own[i] : 0u;
     all += own[i];
   }
-  if (threadIdx.x == 0) {
-    *out_count = (int64_t)all;
-    if (all > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
-  }
+  if (threadIdx.x == 0) count_known(all, capacity, out_count, answer, status);
   at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);  // the same in every lane
   walk<S, ALIGNED, true>(in, begin, end, least, out_idx + at, out_val + at, room_from(capacity, at));
 }
 
 template <typename S, typename I, bool ALIGNED>
 int compact_launch(const S *in, int64_t n, const uint32_t *thr, I *out_idx, S *out_val, int64_t capacity,
-                   int64_t *out_count, void *workspace, int32_t *status, hipStream_t s) {
+                   int64_t *out_count, void *workspace, int32_t *status, const HostAnswer &answer, hipStream_t s) {
   ProfScope prof(kProfSelectCompact, s);
   if (n <= kOneMax) {
     k_compact_one<S, I, ALIGNED><<<dim3(1), dim3(kMoveBlock), 0, s>>>(in, n, thr, out_idx, out_val, capacity, out_count,
-                                                                     status);
+                                                                     answer, status);
     ZEN_LAUNCH_CHECK("k_compact_one");
     return ZEN_OK;
   }
@@ -302,25 +312,46 @@ int compact_launch(const S *in, int64_t n, const uint32_t *thr, I *out_idx, S *o
   k_compact_walk<S, ALIGNED><<<dim3((unsigned)ceil_div(st.count, kBlock / 64)), dim3(kBlock), 0, s>>>(in, n, thr, st);
   ZEN_LAUNCH_CHECK("k_compact_walk");
   k_compact_move<S, I, ALIGNED><<<dim3((unsigned)ceil_div(st.count, kMoveWaves)), dim3(kMoveBlock), 0, s>>>(
-      in, n, thr, st, out_idx, out_val, capacity, out_count, status);
+      in, n, thr, st, out_idx, out_val, capacity, out_count, answer, status);
   ZEN_LAUNCH_CHECK("k_compact_move");
   return ZEN_OK;
 }
 
 template <typename S>
 int compact_call(const void *input, int64_t n, const uint32_t *thr, void *out_idx, int idx64, void *out_val,
-                 int64_t capacity, int64_t *out_count, void *workspace, int32_t *status, hipStream_t s) {
+                 int64_t capacity, int64_t *out_count, void *workspace, int32_t *status, const HostAnswer &answer,
+                 hipStream_t s) {
   const S *in = static_cast<const S *>(input);
   S *val = static_cast<S *>(out_val);
   const bool aligned = (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
   if (idx64) {
     int64_t *idx = static_cast<int64_t *>(out_idx);
-    return aligned ? compact_launch<S, int64_t, true>(in, n, thr, idx, val, capacity, out_count, workspace, status, s)
-                   : compact_launch<S, int64_t, false>(in, n, thr, idx, val, capacity, out_count, workspace, status, s);
+    return aligned ? compact_launch<S, int64_t, true>(in, n, thr, idx, val, capacity, out_count, workspace, status, answer, s)
+                   : compact_launch<S, int64_t, false>(in, n, thr, idx, val, capacity, out_count, workspace, status, answer, s);
   }
   int32_t *idx = static_cast<int32_t *>(out_idx);
-  return aligned ? compact_launch<S, int32_t, true>(in, n, thr, idx, val, capacity, out_count, workspace, status, s)
-                 : compact_launch<S, int32_t, false>(in, n, thr, idx, val, capacity, out_count, workspace, status, s);
+  return aligned ? compact_launch<S, int32_t, true>(in, n, thr, idx, val, capacity, out_count, workspace, status, answer, s)
+                 : compact_launch<S, int32_t, false>(in, n, thr, idx, val, capacity, out_count, workspace, status, answer, s);
+}
+
+int select_call(const void *input, int dtype, int64_t n, const uint32_t *thr, void *out_idx, int idx64, void *out_val,
+                int64_t capacity, int64_t *out_count, void *workspace, size_t workspace_bytes, int32_t *status,
+                void *stream, const HostAnswer &answer = {}) {
+  if (!out_count || !status) return fail(ZEN_EINVAL, "zen_select: null pointer");
+  if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_select: bad dtype");
+  if (n < 0 || n > 0x7fffffffll || capacity < 0) return fail(ZEN_EINVAL, "zen_select: need 0 <= n < 2^31");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (n == 0) {
+    launch_fill<int64_t>(out_count, 0, 1, s);
+    ZEN_LAUNCH_CHECK("zen_select: zero count");
+    return ZEN_OK;
+  }
+  if (!input || !workspace || (capacity > 0 && (!out_idx || !out_val)))
+    return fail(ZEN_EINVAL, "zen_select: null pointer");
+  if (workspace_bytes < zen_select_workspace(n, dtype)) return fail(ZEN_EWORKSPACE, "zen_select: workspace too small");
+  if (dtype == ZEN_BF16)
+    return compact_call<uint16_t>(input, n, thr, out_idx, idx64, out_val, capacity, out_count, workspace, status, answer, s);
+  return compact_call<uint32_t>(input, n, thr, out_idx, idx64, out_val, capacity, out_count, workspace, status, answer, s);
 }
 
 }  // namespace
@@ -340,22 +371,22 @@ size_t zen_select_workspace(int64_t n, int dtype) {
 int zen_select(const void *input, int dtype, int64_t n, const uint32_t *thr, void *out_idx, int idx64,
                void *out_val, int64_t capacity, int64_t *out_count, void *workspace, size_t workspace_bytes,
                int32_t *status, void *stream) {
+  return zen::select_call(input, dtype, n, thr, out_idx, idx64, out_val, capacity, out_count, workspace, workspace_bytes,
+                          status, stream);
+}
+
+int zen_select_count(const void *input, int dtype, int64_t n, const uint32_t *thr, void *out_idx, int idx64,
+                     void *out_val, int64_t capacity, int64_t *out_count, void *workspace, size_t workspace_bytes,
+                     int32_t *status, int64_t *host, int64_t words, void *stream) {
   using namespace zen;
-  if (!out_count || !status) return fail(ZEN_EINVAL, "zen_select: null pointer");
-  if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_select: bad dtype");
-  if (n < 0 || n > 0x7fffffffll || capacity < 0) return fail(ZEN_EINVAL, "zen_select: need 0 <= n < 2^31");
+  HostAnswer answer;
+  int rc = host_ask(host, words, 2, &answer);
+  if (rc != ZEN_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (n == 0) {
-    launch_fill<int64_t>(out_count, 0, 1, s);
-    ZEN_LAUNCH_CHECK("zen_select: zero count");
-    return ZEN_OK;
-  }
-  if (!input || !workspace || (capacity > 0 && (!out_idx || !out_val)))
-    return fail(ZEN_EINVAL, "zen_select: null pointer");
-  if (workspace_bytes < zen_select_workspace(n, dtype)) return fail(ZEN_EWORKSPACE, "zen_select: workspace too small");
-  if (dtype == ZEN_BF16)
-    return compact_call<uint16_t>(input, n, thr, out_idx, idx64, out_val, capacity, out_count, workspace, status, s);
-  return compact_call<uint32_t>(input, n, thr, out_idx, idx64, out_val, capacity, out_count, workspace, status, s);
+  rc = select_call(input, dtype, n, thr, out_idx, idx64, out_val, capacity, out_count, workspace, workspace_bytes,
+                   status, stream, answer);
+  if (rc == ZEN_OK && n == 0) rc = host_answer_launch(answer, out_count, 1, status, 1, s);
+  return rc == ZEN_OK ? host_wait(answer, s) : rc;
 }
 
 }  // extern "C"

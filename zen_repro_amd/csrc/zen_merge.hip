@@ -708,10 +708,14 @@ size_t zen_decode_dense_workspace(int64_t r, int64_t dense_n) {
          zen::align_up(zen_merge_workspace(r, dense_n), 256);
 }
 
-int zen_decode_dense(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, void *dense,
-                     int64_t dense_n, int mode, void *workspace, size_t workspace_bytes, int32_t *status,
-                     void *stream) {
-  using namespace zen;
+}  // extern "C"
+
+namespace zen {
+namespace {
+
+int decode_call(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, void *dense, int64_t dense_n,
+                int mode, void *workspace, size_t workspace_bytes, int32_t *status, void *stream,
+                const HostAsk &ask = {}) {
   const char *why = "";
   if (merge_check(idx, val, dtype, r, dense_n, mode, &why) != ZEN_OK) return fail(ZEN_EINVAL, why);
   if (!dense || !status) return fail(ZEN_EINVAL, "zen_decode_dense: null pointer");
@@ -726,9 +730,9 @@ int zen_decode_dense(const void *idx, int idx64_in, const void *val, int dtype, 
   if (whole) {
     if (dtype == ZEN_BF16)
       return merge_launch(idx, idx64_in, static_cast<const uint16_t *>(val), r, dense_n, nullptr, 0,
-                          static_cast<uint16_t *>(dense), r, nullptr, mode, inner, status, s);
+                          static_cast<uint16_t *>(dense), r, nullptr, mode, inner, status, s, ask);
     return merge_launch(idx, idx64_in, static_cast<const uint32_t *>(val), r, dense_n, nullptr, 0,
-                        static_cast<float *>(dense), r, nullptr, mode, inner, status, s);
+                        static_cast<float *>(dense), r, nullptr, mode, inner, status, s, ask);
   }
   if (dtype == ZEN_BF16)
     launch_fill<uint16_t>(static_cast<uint16_t *>(dense), (uint16_t)0, (size_t)dense_n, s);
@@ -756,6 +760,34 @@ int zen_decode_dense(const void *idx, int idx64_in, const void *val, int dtype, 
                                                                  (uint32_t)dense_n);
   ZEN_LAUNCH_CHECK("k_scatter_dense");
   return ZEN_OK;
+}
+
+}  // namespace
+}  // namespace zen
+
+extern "C" {
+
+int zen_decode_dense(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, void *dense,
+                     int64_t dense_n, int mode, void *workspace, size_t workspace_bytes, int32_t *status,
+                     void *stream) {
+  return zen::decode_call(idx, idx64_in, val, dtype, r, dense, dense_n, mode, workspace, workspace_bytes, status, stream);
+}
+
+int zen_decode_dense_status(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, void *dense,
+                            int64_t dense_n, int mode, void *workspace, size_t workspace_bytes, int32_t *status,
+                            int64_t *host, int64_t words, void *stream) {
+  using namespace zen;
+  HostAnswer answer;
+  bool answered = false;
+  int rc = host_ask(host, words, 1, &answer);
+  if (rc != ZEN_OK) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  rc = decode_call(idx, idx64_in, val, dtype, r, dense, dense_n, mode, workspace, workspace_bytes, status, stream,
+                   HostAsk{answer, &answered});
+  if (rc == ZEN_OK && !answered) rc = host_answer_launch(answer, nullptr, 0, status, 1, s);
+  if (rc == ZEN_OK) return host_wait(answer, s);
+  if (answered) (void)hipStreamSynchronize(s);  // an answer may be on its way: not into a later call's words
+  return rc;
 }
 
 }  // extern "C"
