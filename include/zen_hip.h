@@ -124,9 +124,9 @@ int zen_mapping(int64_t n, int partitions, int64_t *out, int64_t *counts,
  * only the first *idx_n_dev count if that device counter is given.  rank_at is
  * optional: the rank dictionary zen_bitmap_ranks builds for this mapping and
  * `numel` (zen_bitmap_rank_words(numel) words, 16-byte aligned: members below
- * every multiple of 512 and one membership bit per index value; to be kept
+ * every multiple of 96 and one membership bit per index value; to be kept
  * with the mapping, which the reference caches too, comm.py:132-134).  With it
- * a lookup is two loads instead of a search through the list from an
+ * a lookup is one load instead of a search through the list from an
  * interpolated guess, and indices >= numel count as beyond the last member.
  * For indices in [0, numel) the result is the same with and without.  A position past the end
  * of the list (torch raises an IndexError there) sets ZEN_STAT_BAD_INDEX.

@@ -31,6 +31,27 @@ def lba_with_mapping(zen, n, P, rank):
     return lba
 
 
+@pytest.mark.parametrize("n, P", [(1, 1), (95, 1), (96, 2), (97, 1), (193, 3), (12 * 96 + 1, 4), (9000, 2)])
+def test_bitmap_rank_entries(zen, oracle, n, P):
+    """Every index of [0, n) by itself, around the edges of the rank dictionary's entries; lists that ascend, that
+    repeat an index, that descend, and of lengths around what a workgroup takes."""
+    n = n // P * P
+    rng = np.random.default_rng(n)
+    for rank in range(P):
+        lba = lba_with_mapping(zen, n, P, rank)
+        members = oracle.mapping(n, P)[rank]
+        if not len(members):
+            continue
+        fits = np.arange(members[-1] + 1)  # an index that is no member marks the next one
+        lists = [fits, fits[::-1].copy(), np.sort(np.concatenate([fits, fits]))]
+        lists += [np.sort(rng.choice(fits, size)) for size in (1, 63, 64, 65, 255, 1023, 1024, 1025)]
+        lists += [fits[i:i + 1] for i in range(max(0, len(fits) - 200), len(fits), 7)]
+        for idx in lists:
+            assert np.array_equal(to_np(lba.encode_bitmap(to_dev(idx), n)), oracle.bitmap_encode(members, idx))
+        with pytest.raises(IndexError):
+            lba.encode_bitmap(to_dev(np.array([members[-1] + 1])), n)
+
+
 @pytest.mark.parametrize("idx_dtype", [torch.int64, torch.int32])
 @pytest.mark.parametrize("n,P,rank,frac", [
     (1 << 12, 8, 3, 0.05),

@@ -3,8 +3,8 @@
 // per member, least significant bit first inside each byte.
 //
 // Encode is a lookup per index.  A rank dictionary kept next to the mapping
-// (members below every multiple of 512, plus one membership bit per index
-// value) answers it with two loads; without the dictionary the position is
+// (members below every multiple of 96, plus one membership bit per index
+// value) answers it with one load; without the dictionary the position is
 // estimated by interpolation (the members are spread evenly, that is what the
 // hash is for), bracketed by doubling steps and found by bisection.  Decode is a compaction of the set bits: count per
 // block, scan the block counts, write mapping[position] for every set bit.
@@ -51,23 +51,19 @@ __device__ inline int64_t member_lower_bound_near(const int64_t *__restrict__ ma
   return hi;
 }
 
-// Rank dictionary of one partition's member list, kept next to the list: the index range is cut into blocks
-// of 512 values; rank[b] = number of members below block b (one more entry at the end = the member count),
-// followed by 512 membership bits per block.  The position of any index is then rank[b] + the number of
-// membership bits below it in its block: two loads that neighbouring indices share, 1/8 byte per index value
-// instead of a search through eight-byte members.
-constexpr int kBmShift = 9;
-constexpr int kBmBlockWords = (1 << kBmShift) / 32;  // 16 words = one 64-byte line per block
+// Rank dictionary of one partition's member list, kept next to the list: per 96 index values, 16 bytes with the number
+// of members below them and their membership bits.  The position of any index is then that number plus the set bits
+// below its own: one load that neighbouring indices share, a sixth of a byte per index value, instead of a search
+// through eight-byte members.  (Blocks of 512 bits with their ranks in an array of their own are an eighth of a byte, but
+// sixteen words to mask and count per index: the marking kernel 21.5 us where it takes 12.)
+constexpr uint32_t kBmValues = 96;
 
+// One thread per block: a bisection for its first member, which the others follow in the list.
 __global__ __launch_bounds__(kBmBlock) void k_bitmap_ranks(const int64_t *__restrict__ map, int64_t count,
-                                                           int64_t blocks, uint32_t *__restrict__ rank_at) {
+                                                           int64_t blocks, uint4 *__restrict__ ranks) {
   const int64_t b = (int64_t)blockIdx.x * kBmBlock + threadIdx.x;
-  if (b > blocks) return;
-  if (b == blocks) {
-    rank_at[b] = (uint32_t)count;
-    return;
-  }
-  const int64_t v = b << kBmShift;
+  if (b >= blocks) return;
+  const int64_t v = b * kBmValues;
   int64_t lo = -1, hi = count;
   while (hi - lo > 1) {
     const int64_t mid = lo + ((hi - lo) >> 1);
@@ -76,38 +72,41 @@ __global__ __launch_bounds__(kBmBlock) void k_bitmap_ranks(const int64_t *__rest
     else
       hi = mid;
   }
-  rank_at[b] = (uint32_t)hi;
-}
-
-// One thread per block: the block's members (consecutive in the list) become its 512 membership bits.
-__global__ __launch_bounds__(kBmBlock) void k_bitmap_members(const int64_t *__restrict__ map, int64_t blocks,
-                                                             const uint32_t *__restrict__ rank_at,
-                                                             uint32_t *__restrict__ bits) {
-  const int64_t b = (int64_t)blockIdx.x * kBmBlock + threadIdx.x;
-  if (b >= blocks) return;
-  uint32_t w[kBmBlockWords];
+  uint32_t w[kBmValues / 32] = {};
+  for (int64_t j = hi; j < count && map[j] < v + kBmValues; ++j) {
+    const uint32_t off = (uint32_t)(map[j] - v);
 #pragma unroll
-  for (int q = 0; q < kBmBlockWords; ++q) w[q] = 0;
-  for (int64_t j = rank_at[b]; j < (int64_t)rank_at[b + 1]; ++j) {
-    const uint32_t off = (uint32_t)(map[j] & ((1 << kBmShift) - 1));
-#pragma unroll
-    for (int q = 0; q < kBmBlockWords; ++q) w[q] |= (off >> 5) == (uint32_t)q ? 1u << (off & 31) : 0u;
+    for (uint32_t q = 0; q < kBmValues / 32; ++q) w[q] |= (off >> 5) == q ? 1u << (off & 31) : 0u;
   }
-  uint4 *out = reinterpret_cast<uint4 *>(bits + b * kBmBlockWords);
-#pragma unroll
-  for (int q = 0; q < kBmBlockWords / 4; ++q) out[q] = make_uint4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
+  ranks[b] = make_uint4((uint32_t)hi, w[0], w[1], w[2]);
 }
 
-// One index per thread, neighbouring threads neighbouring indices; the indices may come in any order.
+// Index v's place among the members (`count`: behind the last).
 // Without the dictionary the position is estimated by interpolation over the whole list (the members are
 // spread evenly, that is what the hash is for; float arithmetic lands within a few thousand places) and
 // corrected by a search around the estimate.
-template <typename I>
-__global__ __launch_bounds__(kBmBlock) void k_bitmap_mark(const int64_t *__restrict__ map, int64_t count,
-                                                          const I *__restrict__ idx, int64_t idx_n,
-                                                          const int64_t *__restrict__ idx_n_dev,
-                                                          const uint32_t *__restrict__ rank_at, int64_t rank_blocks,
-                                                          uint32_t *__restrict__ words, int32_t *status) {
+__device__ inline int64_t member_place(const int64_t *__restrict__ map, int64_t count, int64_t v) {
+  const int64_t first = map[0], last = map[count - 1];
+  if (v <= first) return 0;
+  if (v > last) return count;
+  const float slope = (float)(count - 1) / (float)(last - first);
+  int64_t g = (int64_t)((float)(v - first) * slope);
+  g = g > count - 1 ? count - 1 : (g < 0 ? 0 : g);
+  return member_lower_bound_near(map, count, g, 64, v);
+}
+
+// kBmEach indices per thread, those of a wave's row neighbours; the indices may come in any order.  Bound by the trips
+// to memory (the index, the dictionary's line, the bitmap's word), of which
+// four of each kind are in flight.  2.8 M of the 3.9 M members of a sixteenth of 62 M indices 12.0 us, 2.1 M of the
+// 16.8 M of 268 M 13.9; with one index per thread, lines of 512 membership bits and the neighbours' bits gathered
+// through lane permutes 25.9 and 22.8.  (One, two, eight indices per thread: 14.0, 13.2, 14.0 and 13.7, 13.8, 15.0.)
+constexpr int kBmEach = 4;
+template <typename I, bool RANKS>
+__global__ __launch_bounds__(kBmBlock, 4) void k_bitmap_mark(const int64_t *__restrict__ map, int64_t count,
+                                                             const I *__restrict__ idx, int64_t idx_n,
+                                                             const int64_t *__restrict__ idx_n_dev,
+                                                             const uint4 *__restrict__ ranks, int64_t numel,
+                                                             uint32_t *__restrict__ words, int32_t *status) {
   int64_t n = idx_n;
   if (idx_n_dev) {
     const int64_t d = *idx_n_dev;
@@ -117,68 +116,71 @@ __global__ __launch_bounds__(kBmBlock) void k_bitmap_mark(const int64_t *__restr
     if (n > 0 && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(status, ZEN_STAT_BAD_INDEX);
     return;
   }
-  const int64_t j = (int64_t)blockIdx.x * kBmBlock + threadIdx.x;
-  const bool live = j < n;
-  const int64_t v = live ? (int64_t)idx[j] : 0;
-  int64_t pos;
-  if (!live) {
-    pos = count;
-  } else if (rank_at) {
-    if (v < 0) {
-      pos = 0;
-    } else if ((v >> kBmShift) >= rank_blocks) {
-      pos = count;  // beyond the index range: beyond every member
-    } else {
-      const int64_t b = v >> kBmShift;
-      const uint4 *line = reinterpret_cast<const uint4 *>(rank_at + (rank_blocks + 1 + 3) / 4 * 4 + b * kBmBlockWords);
-      const uint32_t off = (uint32_t)(v & ((1 << kBmShift) - 1));
-      uint32_t below = rank_at[b];
+  const int64_t j0 = (int64_t)blockIdx.x * (kBmBlock * kBmEach) + threadIdx.x;
+  if (j0 - (int64_t)threadIdx.x >= n) return;
+  int64_t v[kBmEach];
+  uint32_t pos[kBmEach];  // below 2^31
 #pragma unroll
-      for (int q = 0; q < kBmBlockWords / 4; ++q) {
-        const uint4 m = line[q];
-        const uint32_t ws[4] = {m.x, m.y, m.z, m.w};
+  for (int i = 0; i < kBmEach; ++i) {  // (a place past the end reads the last index and marks nothing)
+    const int64_t j = j0 + i * kBmBlock;
+    v[i] = (int64_t)idx[j < n ? j : n - 1];
+  }
+  if (RANKS) {
+    uint4 entry[kBmEach];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t first_bit = (uint32_t)(q * 4 + e) * 32u;
-          uint32_t x = ws[e];
-          if (off <= first_bit)
-            x = 0;
-          else if (off - first_bit < 32u)
-            x &= (1u << (off - first_bit)) - 1u;
-          below += (uint32_t)__popc(x);
-        }
-      }
-      pos = below;
+    for (int i = 0; i < kBmEach; ++i)  // in no branch, so that all are in flight together
+      entry[i] = ranks[v[i] < 0 || v[i] >= numel ? 0u : (uint32_t)v[i] / kBmValues];
+#pragma unroll
+    for (int i = 0; i < kBmEach; ++i) {
+      const uint32_t off = (uint32_t)v[i] % kBmValues;
+      const uint32_t below = (1u << (off & 31u)) - 1u;  // of the bits in the index's own word
+      const uint32_t all = entry[i].x + (uint32_t)__popc(entry[i].y & (off < 32u ? below : ~0u)) +
+                           (uint32_t)__popc(off < 32u ? 0u : entry[i].z & (off < 64u ? below : ~0u)) +
+                           (uint32_t)__popc(off < 64u ? 0u : entry[i].w & below);
+      // an index beyond the index range is beyond every member
+      pos[i] = v[i] < 0 ? 0u : v[i] >= numel ? (uint32_t)count : all;
     }
   } else {
-    const int64_t first = map[0], last = map[count - 1];
-    if (v <= first) {
-      pos = 0;
-    } else if (v > last) {
-      pos = count;
-    } else {
-      const float slope = (float)(count - 1) / (float)(last - first);
-      int64_t g = (int64_t)((float)(v - first) * slope);
-      g = g > count - 1 ? count - 1 : (g < 0 ? 0 : g);
-      pos = member_lower_bound_near(map, count, g, 64, v);
-    }
+#pragma unroll
+    for (int i = 0; i < kBmEach; ++i) pos[i] = (uint32_t)member_place(map, count, v[i]);
   }
-  // Neighbouring lanes often mark the same word (ascending indices: positions a few places apart).  Each lane
-  // gathers the bits of the lanes before it that name the same word; only the last lane of such a stretch
-  // goes to memory.  (A lane may also pick up bits of the same word from further away: harmless for an OR.)
-  const bool bad = !live || pos >= count;
-  if (live && bad) atomicOr(status, ZEN_STAT_BAD_INDEX);  // torch raises an index error here (comm.py:63)
-  const uint32_t word = bad ? 0xffffffffu : (uint32_t)(pos >> 5);
-  uint32_t bits = bad ? 0u : 1u << (pos & 31);
+  // Neighbouring lanes often mark the same word (ascending indices: positions a few places apart): of the lanes that
+  // do, the last one goes to memory.
   const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t w2 = (uint32_t)__shfl_up((int)word, off);
-    const uint32_t b2 = (uint32_t)__shfl_up((int)bits, off);
-    if (lane >= off && w2 == word) bits |= b2;
+  for (int i = 0; i < kBmEach; ++i) {
+    const bool live = j0 + i * kBmBlock < n;
+    const bool bad = !live || pos[i] >= (uint32_t)count;
+    if (live && bad) atomicOr(status, ZEN_STAT_BAD_INDEX);  // torch raises an index error here (comm.py:63)
+    const uint32_t word = bad ? 0xffffffffu : pos[i] >> 5;
+    uint32_t bits = bad ? 0u : 1u << (pos[i] & 31u);
+    const uint32_t prev = (uint32_t)__shfl_up((int)word, 1), before = (uint32_t)__shfl_up((int)pos[i], 1);
+    const uint64_t starts = __ballot(lane == 0 || word != prev);  // stretches of lanes that name one word
+    if (__ballot(lane > 0 && !bad && before >= pos[i])) {
+      // not strictly ascending: a lane gathers the bits of the lanes before it that name the same word.  (It may also
+      // pick up bits of the same word from further away: harmless for an OR.)
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t w2 = (uint32_t)__shfl_up((int)word, off);
+        const uint32_t b2 = (uint32_t)__shfl_up((int)bits, off);
+        if (lane >= off && w2 == word) bits |= b2;
+      }
+    } else {
+      // all bits of a stretch are different: their OR is their sum
+      const uint32_t upto = wave_inclusive_scan(bits);
+      const int first = 63 - __clzll((long long)(starts & (~0ull >> (63 - lane))));
+      bits = upto - (uint32_t)__shfl((int)(upto - bits), first);
+    }
+    if (!bad && (lane == 63 || ((starts >> lane) & 2ull))) atomicOr(&words[word], bits);
   }
-  const uint32_t next = (uint32_t)__shfl_down((int)word, 1);
-  if (!bad && (lane == 63 || next != word)) atomicOr(&words[word], bits);
+}
+
+template <typename I>
+void launch_mark(const int64_t *map, int64_t count, const I *idx, int64_t idx_n, const int64_t *idx_n_dev,
+                 const uint32_t *rank_at, int64_t numel, uint32_t *words, int32_t *status, hipStream_t s) {
+  const auto kernel = rank_at ? k_bitmap_mark<I, true> : k_bitmap_mark<I, false>;
+  kernel<<<dim3((unsigned)ceil_div(idx_n, (int64_t)kBmBlock * kBmEach)), dim3(kBmBlock), 0, s>>>(
+      map, count, idx, idx_n, idx_n_dev, reinterpret_cast<const uint4 *>(rank_at), numel, words, status);
 }
 
 // Bits of the 16 bitmap bytes of thread t of block b that lie below `count` positions, as four words.
@@ -289,9 +291,7 @@ size_t zen_bitmap_words(int64_t mapping_n) { return mapping_n > 0 ? (size_t)((ma
 
 size_t zen_bitmap_rank_words(int64_t numel) {
   if (numel <= 0) return 0;
-  const size_t blocks = (size_t)(((numel - 1) >> zen::kBmShift) + 1);
-  // the membership lines start on a 16-byte boundary: blocks + 1 rank words are padded to a multiple of four
-  return (blocks + 1 + 3) / 4 * 4 + blocks * zen::kBmBlockWords;
+  return (size_t)zen::ceil_div(numel, (int64_t)zen::kBmValues) * 4;
 }
 
 int zen_bitmap_ranks(const int64_t *mapping_p, int64_t mapping_n, int64_t numel, uint32_t *rank_at, void *stream) {
@@ -301,13 +301,10 @@ int zen_bitmap_ranks(const int64_t *mapping_p, int64_t mapping_n, int64_t numel,
   if (!rank_at || (mapping_n > 0 && !mapping_p)) return fail(ZEN_EINVAL, "zen_bitmap_ranks: null pointer");
   if (reinterpret_cast<uintptr_t>(rank_at) & 15u) return fail(ZEN_EINVAL, "zen_bitmap_ranks: table not 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t blocks = ((numel - 1) >> kBmShift) + 1;
-  k_bitmap_ranks<<<dim3((unsigned)ceil_div(blocks + 1, kBmBlock)), dim3(kBmBlock), 0, s>>>(mapping_p, mapping_n, blocks,
-                                                                                         rank_at);
+  const int64_t blocks = ceil_div(numel, (int64_t)kBmValues);
+  k_bitmap_ranks<<<dim3((unsigned)ceil_div(blocks, kBmBlock)), dim3(kBmBlock), 0, s>>>(mapping_p, mapping_n, blocks,
+                                                                                     reinterpret_cast<uint4 *>(rank_at));
   ZEN_LAUNCH_CHECK("k_bitmap_ranks");
-  k_bitmap_members<<<dim3((unsigned)ceil_div(blocks, kBmBlock)), dim3(kBmBlock), 0, s>>>(
-      mapping_p, blocks, rank_at, rank_at + (blocks + 1 + 3) / 4 * 4);
-  ZEN_LAUNCH_CHECK("k_bitmap_members");
   return ZEN_OK;
 }
 
@@ -325,17 +322,13 @@ int zen_bitmap_encode(const int64_t *mapping_p, int64_t mapping_n, const void *i
   launch_fill<uint32_t>(bitmap_words, 0u, zen_bitmap_words(mapping_n), s);
   ZEN_LAUNCH_CHECK("zen_bitmap_encode: clear");
   if (idx_n == 0) return ZEN_OK;
-  const int64_t blocks = ceil_div(idx_n, kBmBlock);
-  if (blocks > 0x7fffffffll) return fail(ZEN_EINVAL, "zen_bitmap_encode: too many indices");
-  const int64_t rank_blocks = rank_at ? ((numel - 1) >> kBmShift) + 1 : 0;
+  if (ceil_div(idx_n, kBmBlock) > 0x7fffffffll) return fail(ZEN_EINVAL, "zen_bitmap_encode: too many indices");
   if (idx64)
-    k_bitmap_mark<int64_t><<<dim3((unsigned)blocks), dim3(kBmBlock), 0, s>>>(
-        mapping_p, mapping_n, static_cast<const int64_t *>(idx), idx_n, idx_n_dev, rank_at, rank_blocks,
-        bitmap_words, status);
+    launch_mark(mapping_p, mapping_n, static_cast<const int64_t *>(idx), idx_n, idx_n_dev, rank_at, numel, bitmap_words,
+                status, s);
   else
-    k_bitmap_mark<int32_t><<<dim3((unsigned)blocks), dim3(kBmBlock), 0, s>>>(
-        mapping_p, mapping_n, static_cast<const int32_t *>(idx), idx_n, idx_n_dev, rank_at, rank_blocks,
-        bitmap_words, status);
+    launch_mark(mapping_p, mapping_n, static_cast<const int32_t *>(idx), idx_n, idx_n_dev, rank_at, numel, bitmap_words,
+                status, s);
   ZEN_LAUNCH_CHECK("k_bitmap_mark");
   return ZEN_OK;
 }
