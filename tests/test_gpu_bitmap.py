@@ -331,6 +331,27 @@ def test_bitmaps_to_dense_with_values_in_any_layout(zen, oracle, form):
     assert got.dtype == torch.float32 and np.array_equal(to_np(got), _dense_truth(oracle, n, idx, val))
 
 
+@pytest.mark.parametrize("special", range(12))
+@pytest.mark.parametrize("n, P", [(8192, 1), (24576 + 80, 1), (3 * 8192 + 17, 3), (1 << 17, 16)])
+def test_bitmaps_to_dense_special_values(zen, oracle, n, P, special):
+    """0.0f + v for one element that needs it (-0, NaNs of either sign, quiet or not) and for those that do not, alone
+    among ordinary ones, in whole tiles and in the last one; every member set, so that the values end with the list."""
+    n = n // P * P
+    bits = [0x8000, 0x7f81, 0x7fbf, 0x7fc0, 0x7fff, 0xff81, 0xffbf, 0xffff, 0x7f80, 0xff80, 0x0001, 0x8001][special]
+    mp = oracle.mapping(n, P)
+    values = [np.full(len(m), 0x3f80, np.uint16) for m in mp]
+    at = [len(m) * special // 12 for m in mp]
+    want = np.full(n, 0x3f80, np.uint16)
+    for p in range(P):
+        values[p][at[p]] = bits
+        quiet = bits | 0x40 if bits & 0x7fff > 0x7f80 else 0 if bits == 0x8000 else bits
+        want[mp[p][at[p]]] = quiet
+    bitmaps = [to_dev(oracle.bitmap_encode(m, m)) for m in mp]
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P, 0), None, None)
+    got = lba.decode_bitmaps_dense(bitmaps, [torch.from_numpy(v.view(np.int16)).cuda().view(torch.bfloat16) for v in values], n)
+    assert np.array_equal(got.view(torch.int16).cpu().numpy().view(np.uint16), want)
+
+
 def test_bitmaps_to_dense_edge_cases(zen, oracle):
     n, P = 1 << 18, 8
     mp, idx, val = _shards(oracle, n, P, 0.1, "f32", seed=3)

@@ -28,7 +28,7 @@ static_assert(kFdChunks == 32, "a wave's lower half scans the chunk sums");
 struct FdLists {
   const uint8_t *bitmap[kFdMaxLists];
   const void *val[kFdMaxLists];
-  uint32_t bytes[kFdMaxLists], vals[kFdMaxLists];  // of the bitmap; values
+  uint32_t bytes[kFdMaxLists], vals[kFdMaxLists];  // of the bitmap (2^28 at most: its bits fit 32 bits); values
 };
 
 __device__ inline uint32_t part_of(uint32_t t, uint32_t n, uint32_t npp) {
@@ -194,6 +194,9 @@ __global__ __launch_bounds__(kFdGroupsMax) void k_fd_groups(uint32_t *__restrict
   if (threadIdx.x < groups) *at = before;
 }
 
+constexpr int kFdWords = 9;                  // words of a chunk: sixteen lists have 512 members in a tile, few more than 576
+constexpr int kFdMembers = 64 * kFdWords;    // members of a chunk
+
 template <typename S>
 __device__ inline S fd_value(S v);  // what a zeroed element holds after one scatter_add_ of v (comm.py:35-39)
 template <>
@@ -206,14 +209,75 @@ __device__ inline uint32_t fd_value<uint32_t>(uint32_t v) {
   return __float_as_uint(0.0f + __uint_as_float(v));
 }
 
+// fd_value of all elements of some pieces of a tile.  bf16 elements that need it are rare (-0 and NaNs), and three
+// packed comparisons per pair find out that there is none.
+template <int N>
+__device__ inline void fd_values(u32x4 (&piece)[N], uint32_t) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) piece[i][e] = fd_value<uint32_t>(piece[i][e]);
+}
+template <int N>
+__device__ inline void fd_values(u32x4 (&piece)[N], uint16_t) {
+  typedef short i16x2 __attribute__((ext_vector_type(2)));
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  i16x2 most = {0, 0}, least = {0, 0};
+  u16x2 top = {0, 0};
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t x = piece[i][e];
+      most = __builtin_elementwise_max(most, __builtin_bit_cast(i16x2, x));
+      least = __builtin_elementwise_min(least, __builtin_bit_cast(i16x2, x));
+      top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, x));
+    }
+  // a NaN with a clear sign bit, -0, a NaN with the sign bit set
+  if (most.x <= 0x7f80 && most.y <= 0x7f80 && least.x != -0x8000 && least.y != -0x8000 && top.x <= 0xff80 && top.y <= 0xff80)
+    return;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      piece[i][e] = (uint32_t)fd_value<uint16_t>((uint16_t)piece[i][e]) |
+                    (uint32_t)fd_value<uint16_t>((uint16_t)(piece[i][e] >> 16)) << 16;
+}
+
+// Lane i < kFdWords: bits [bit0 + 64 i, bit0 + 64 i + 64) of a bitmap of `limit` bits, from the two aligned words that
+// hold them (a word with one byte of the bitmap lies in that byte's page); bits past `members` and past the bitmap's end
+// are zero.
+__device__ inline unsigned long long fd_chunk_bits(const uint8_t *bitmap, uint32_t limit, uint32_t bit0, uint32_t members) {
+  const uintptr_t addr = reinterpret_cast<uintptr_t>(bitmap);
+  const uint64_t *words = reinterpret_cast<const uint64_t *>(addr & ~(uintptr_t)7);
+  const uint32_t first = bit0 + (uint32_t)(addr & 7u) * 8u;
+  const uint32_t sh = first & 63u;
+  const uint32_t has = bit0 < limit ? limit - bit0 : 0u;  // bits the bitmap has from the chunk's first on
+  const uint32_t left = has < members ? has : members;
+  const uint32_t lane = (uint32_t)lane_id();
+  unsigned long long w = 0;
+  if (lane * 64u < sh + left && left && lane <= (uint32_t)kFdWords) w = words[(first >> 6) + lane];
+  const unsigned long long up = __shfl_down(w, 1, 64);
+  unsigned long long bits = (w >> sh) | ((up << 1) << (63u - sh));
+  if (lane >= (uint32_t)kFdWords || left <= lane * 64u) bits = 0;
+  else if (left - lane * 64u < 64u) bits &= (1ull << (left - lane * 64u)) - 1ull;
+  return bits;
+}
+
 // One workgroup per tile.  Lane p of every wave knows list p's members in the tile, the first bit of their range
-// and where its values start; the lists' members are cut into chunks of 640, dealt to the waves in turn.  A
-// wave gets the chunk's bits as ten 64-bit words in scalar registers: the word is the mask of the lanes whose
+// and where its values start; the lists' members are cut into chunks of 576, dealt to the waves in turn.  A
+// wave gets the chunk's bits as nine 64-bit words in scalar registers: the word is the mask of the lanes whose
 // member has a value, a lane's value is the one numbered by the set bits below it, and its place in the tile is
-// the chunk's next entry of the dictionary, so that all loads are consecutive, ten of each kind in flight.  The
+// the chunk's next entry of the dictionary, so that all loads are consecutive, nine of each kind in flight.  The
 // places written are put together in LDS and leave with full-width stores.
 // Bound by memory: two bytes of dictionary and one element of output per index, and the values.  62 M bf16 elements
-// on sixteen ranks, 71 % of them set, 0.34 GB: 79 us; 268 M elements, 11 % set, 1.13 GB: 265 us.  One SET bit per
+// on sixteen ranks, 71 % of them set, 0.34 GB: 73 us; 268 M elements, 11 % set, 1.13 GB: 241 us, 4.7 TB/s.
+// What a 64th of a chunk costs beside its loads counts too: places read without a look at the end of the list (the
+// dictionary goes on behind it), values clamped only where they end, and 0.0f + v taken for what is written out as a
+// whole instead of each value: 260 -> 249 us; chunks of nine words instead of ten, of which two were past most lists'
+// ends, 241.  Slower: the bits by scalar loads (289; nine cache lines one after the other), the low bytes of the places
+// alone with the high ones counted from where they wrap (0.86 GB, 275: seven instructions more per word).
+// One SET bit per
 // thread and turn, looked up in staged copies of the tile's bytes and values, took 307 and 411 us; with each value's
 // load in a branch of its own, which makes the compiler wait for it there, this kernel took 129 and 428 (79 and 300 without).
 // Waves of a workgroup meet at its two barriers, so small workgroups keep loads and stores going side by side as long
@@ -222,8 +286,6 @@ __device__ inline uint32_t fd_value<uint32_t>(uint32_t v) {
 // elements, two ranks: 865; 960 with four).
 template <typename S>
 constexpr int fd_tile_block() { return sizeof(S) == 2 ? 256 : 512; }
-constexpr int kFdWords = 10;                 // words of a chunk: sixteen lists have 512 +- 70 members in a tile
-constexpr int kFdMembers = 64 * kFdWords;    // members of a chunk
 
 template <typename S>
 __global__ __launch_bounds__(fd_tile_block<S>(), sizeof(S) == 2 ? 6 : 8) void k_fd_tiles(const uint16_t *__restrict__ order,
@@ -266,30 +328,9 @@ __global__ __launch_bounds__(fd_tile_block<S>(), sizeof(S) == 2 ? 6 : 8) void k_
     const uint16_t *place_at = order + tile_base + (uint32_t)__builtin_amdgcn_readlane((int)(incl - cnt), p) + j0;
     uint32_t place[kFdWords];
 #pragma unroll
-    for (int i = 0; i < kFdWords; ++i) {
-      const uint32_t j = (uint32_t)(i * 64 + lane);
-      place[i] = __builtin_nontemporal_load(place_at + (j < members ? j : 0u));
-    }
-    // Lane i: bits [bit0 + 64 i, bit0 + 64 i + 64) of the bitmap, from the two aligned words that hold them (a
-    // word with one byte of the bitmap lies in that byte's page); bits of other tiles and past the bitmap's
-    // end count as zero.
-    const uintptr_t addr = reinterpret_cast<uintptr_t>(lists.bitmap[p]);
-    const uint64_t limit = (uint64_t)lists.bytes[p] * 8u;
-    const uint64_t *words = reinterpret_cast<const uint64_t *>(addr & ~(uintptr_t)7);
-    const uint64_t first = (uint64_t)bit0 + (addr & 7u) * 8u, over = limit + (addr & 7u) * 8u;
-    const uint64_t at = (first >> 6) + (uint64_t)lane;
-    unsigned long long w = 0;
-    if (lane <= kFdWords && at * 64u < over) w = words[at];
-    const unsigned sh = (unsigned)(first & 63u);
-    const unsigned long long up = __shfl_down(w, 1, 64);
-    unsigned long long bits = (w >> sh) | (sh ? up << (64u - sh) : 0ull);
-    {
-      uint64_t left = (uint64_t)bit0 < limit ? limit - bit0 : 0u;  // bits the bitmap has from the chunk's first on
-      if (left > members) left = members;
-      const uint64_t mine = (uint64_t)lane * 64u;
-      if (lane >= kFdWords || left <= mine) bits = 0;
-      else if (left - mine < 64u) bits &= (1ull << (left - mine)) - 1ull;
-    }
+    for (int i = 0; i < kFdWords; ++i)  // (past the members: the next list's, or what follows the last)
+      place[i] = __builtin_nontemporal_load(place_at + lane + i * 64);
+    const unsigned long long bits = fd_chunk_bits(lists.bitmap[p], lists.bytes[p] * 8u, bit0, members);
     // set bits of the tile's range in front of the chunk: the list's earlier chunks in this tile
     uint32_t nth = (uint32_t)__builtin_amdgcn_readlane((int)v0, p);
     if (j0) {  // 128 bits per lane
@@ -299,57 +340,76 @@ __global__ __launch_bounds__(fd_tile_block<S>(), sizeof(S) == 2 ? 6 : 8) void k_
     }
     nth = (uint32_t)__builtin_amdgcn_readfirstlane((int)nth);
     const uint32_t have = lists.vals[p];
-    if (have == 0) {
-      bad = bad || __ballot(bits != 0);
-      continue;
-    }
-    const S *val = static_cast<const S *>(lists.val[p]) + nth;
-    const uint32_t last = have > nth ? have - nth - 1u : 0u;  // the loads sit in no branch: lanes without a value read a neighbour's
-    if (have <= nth) val -= nth;
-    S v[kFdWords];
     unsigned long long word[kFdWords];
-    uint32_t front = 0;
+    uint32_t set = 0;
 #pragma unroll
     for (int i = 0; i < kFdWords; ++i) {
       const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)bits, i);
       const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32), i);
       word[i] = ((unsigned long long)hi << 32) | lo;
-      const uint32_t k = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, front));
-      // (a 32-bit byte offset: k is below 640 where it matters)
-      v[i] = *reinterpret_cast<const S *>(reinterpret_cast<const char *>(val) + (uint32_t)((k < last ? k : last) * sizeof(S)));
-      front += (uint32_t)__popcll(word[i]);
+      set += (uint32_t)__popcll(word[i]);
     }
-    if (nth + front > have) {  // more set bits than values: the missing ones count as unset
+    if (nth + set > have) {  // more set bits than values: the missing ones count as unset
       bad = true;
-      front = 0;
+      uint32_t front = 0;
+      set = 0;
 #pragma unroll
       for (int i = 0; i < kFdWords; ++i) {
         const uint32_t k = __builtin_amdgcn_mbcnt_hi((uint32_t)(word[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)word[i], front));
         front += (uint32_t)__popcll(word[i]);
         word[i] &= __ballot(nth + k < have);
+        set += (uint32_t)__popcll(word[i]);
+      }
+    }
+    if (set == 0) continue;
+    // A member's value is the one numbered by the set bits below it.  The loads sit in no branch: lanes without a value
+    // read that of the next that has one, or, at the end of all values, the last.
+    const char *val = reinterpret_cast<const char *>(static_cast<const S *>(lists.val[p]) + nth);
+    S v[kFdWords];
+    uint32_t front = 0;
+    if (nth + set < have) {
+#pragma unroll
+      for (int i = 0; i < kFdWords; ++i) {
+        const uint32_t k = __builtin_amdgcn_mbcnt_hi((uint32_t)(word[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)word[i], front));
+        v[i] = *reinterpret_cast<const S *>(val + (uint32_t)(k * sizeof(S)));
+        front += (uint32_t)__popcll(word[i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < kFdWords; ++i) {
+        const uint32_t k = __builtin_amdgcn_mbcnt_hi((uint32_t)(word[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)word[i], front));
+        v[i] = *reinterpret_cast<const S *>(val + (uint32_t)((k < set ? k : set - 1u) * sizeof(S)));
+        front += (uint32_t)__popcll(word[i]);
       }
     }
 #pragma unroll
     for (int i = 0; i < kFdWords; ++i)
-      if (__builtin_amdgcn_inverse_ballot_w64(word[i])) s_tile[place[i] & (uint32_t)(kFdTile - 1)] = fd_value<S>(v[i]);
+      if (__builtin_amdgcn_inverse_ballot_w64(word[i])) s_tile[place[i] & (uint32_t)(kFdTile - 1)] = v[i];
   }
   __syncthreads();
   // written out in 16-byte pieces, consecutive threads consecutive pieces: every store instruction fills whole lines
   if ((reinterpret_cast<uintptr_t>(dense) & 15u) == 0 && tile_base + (uint32_t)kFdTile <= n) {
-    constexpr int kPieces = (int)(kFdTile * sizeof(S) / 16);
+    constexpr int kPieces = (int)(kFdTile * sizeof(S) / 16) / kBlock;
     const u32x4 *src = reinterpret_cast<const u32x4 *>(s_tile);
     u32x4 *dst = reinterpret_cast<u32x4 *>(dense + tile_base);
+    u32x4 piece[kPieces];
 #pragma unroll
-    for (int i = 0; i < kPieces / kBlock; ++i)
-      __builtin_nontemporal_store(src[i * kBlock + threadIdx.x], dst + i * kBlock + threadIdx.x);
+    for (int i = 0; i < kPieces; ++i) piece[i] = src[i * kBlock + threadIdx.x];
+    fd_values(piece, S(0));
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) __builtin_nontemporal_store(piece[i], dst + i * kBlock + threadIdx.x);
   } else {
-    for (uint32_t e = threadIdx.x; e < (uint32_t)kFdTile && tile_base + e < n; e += kBlock) dense[tile_base + e] = s_tile[e];
+    for (uint32_t e = threadIdx.x; e < (uint32_t)kFdTile && tile_base + e < n; e += kBlock)
+      dense[tile_base + e] = fd_value<S>(s_tile[e]);
   }
   if ((bad || odd) && lane == 0) atomicOr(status, ZEN_STAT_BAD_INDEX);
 }
 
 inline uint32_t fd_tiles(int64_t numel) { return (uint32_t)ceil_div(numel, kFdTile); }
-inline size_t fd_order_bytes(int64_t numel) { return (size_t)fd_tiles(numel) * kFdTile * sizeof(uint16_t); }
+// (a chunk's places are read as if it were full)
+inline size_t fd_order_bytes(int64_t numel) {
+  return align_up(((size_t)fd_tiles(numel) * kFdTile + kFdMembers) * sizeof(uint16_t), 256);
+}
 inline size_t fd_table_bytes(int64_t numel, int P) { return align_up(((size_t)fd_tiles(numel) + 1) * P * sizeof(uint32_t), 256); }
 inline size_t fd_vstart_bytes(int64_t numel, int P) { return align_up((size_t)fd_tiles(numel) * P * sizeof(uint32_t), 256); }
 inline size_t fd_gsum_bytes(int64_t numel, int P) { return align_up((size_t)fd_groups(fd_tiles(numel)) * P * sizeof(uint32_t), 256); }
