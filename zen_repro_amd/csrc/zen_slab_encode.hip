@@ -356,11 +356,13 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
   }
 }
 
-// Levels 2 and 3 for the indices that lost level 1, one per thread.  Bound by latency: a probe is four or five
-// dependent trips to memory (the bucket's index, its records, the map), so that every loser has a thread of its own
-// on a full chip; nothing is counted in one place (62 M slots, 10 % taken, 300 000 losers: with one counter of the
+// Levels 2 and 3 for the indices that lost level 1, one per thread.  Bound by latency while losers are few (110 000: a
+// wave 15 us; a probe is four or five dependent trips to memory, the bucket's index, its records, the map) and by the
+// device-wide atomics, two or three a loser at 21 a nanosecond, when they are many (436 000: a wave 50 us).  Every loser
+// has a thread of its own on a full chip: with the scalar registers the compiler takes by itself three workgroups fit a
+// compute unit, and the last of 851 began when the first had ended (93 us, with four 83).  Nothing is counted in one place (62 M slots, 10 % taken, 300 000 losers: with one counter of the
 // map's claims and one log of the owners pushed out, whose entries another kernel classified afterwards, 338 + 220 us).
-__global__ __launch_bounds__(kSlabBlock) void k_slab_chains(SlabGeom geo, Probe g, SlabTables tb, unsigned long long *cells,
+__global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Probe g, SlabTables tb, unsigned long long *cells,
                                                             int64_t spp, uint32_t capacity, int64_t *__restrict__ splits,
                                                             HostAnswer answer, int32_t *status) {
   __shared__ uint32_t s_scan[kSlabBlock / 64 + 1];
