@@ -1103,6 +1103,26 @@ def test_count_the_host_is_told_by_the_merge(zen, r, n, dtype):
         assert torch.equal(got_idx, at) and torch.equal(got_val, want[at].to(dtype))
 
 
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("n", [65537, 65536 + 2048, 65536 + 2049, 200001, 20000000])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_selection_of_every_density(zen, n, shift, dtype):
+    """What a wave keeps of its findings is full at 512: rows with none, with a few, with all of their elements, and
+    stretches with one kind of row behind the other; stretches cut off in a row, views from an odd element on."""
+    from zen_repro_amd import comm
+
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    room = torch.randn(n + shift, generator=gen, device="cuda").to(dtype)
+    at = torch.arange(n + shift, device="cuda")
+    lots = torch.rand(n + shift, generator=gen, device="cuda")
+    for keep in (lots < 0.0, lots < 0.002, lots < 0.1, lots < 0.124, lots < 0.5, lots < 2.0, at // 512 % 3 == 0,
+                 (at // 256 % 5 == 0) | (lots < 0.05), at >= n + shift - 1):
+        t = torch.where(keep, room, torch.zeros_like(room))[shift:]
+        want = torch.nonzero(t).view(-1)
+        idx, val, count, bits = comm._select_raw(t, None, True)
+        assert count == want.numel() and bits == 0 and torch.equal(idx, want) and torch.equal(val, t[want])
+
+
 @pytest.mark.parametrize("n", [1, 65536, 65537, 1000003])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_count_the_host_is_told_by_the_selection(zen, n, dtype):

@@ -54,38 +54,55 @@ __device__ inline uint32_t vec_pick(const uint4 &q, uint32_t e, uint32_t) {
 }
 
 // Sixteen bytes from an address that is a multiple of 16 or, !ALIGNED, of an element's size only (a view that begins
-// at an odd element): one load either way.
-template <typename S, bool ALIGNED>
+// at an odd element): one load either way.  ONCE: nobody looks at them again (a streamed load).
+template <typename S, bool ALIGNED, bool ONCE>
 __device__ inline uint4 load16(const S *at) {
   uint4 q;
-  if (ALIGNED)
+  if (ALIGNED && ONCE) {
+    const u32x4 t = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(at));
+    __builtin_memcpy(&q, &t, 16);
+  } else if (ALIGNED) {
     q = *reinterpret_cast<const uint4 *>(at);
-  else
+  } else {
     __builtin_memcpy(&q, at, 16);
+  }
   return q;
 }
 
+// What a wave has found and not yet written out.  A store on its way holds up the next rows' elements (a wave's loads
+// are waited for together with the stores behind them), so that the walk keeps its findings here and writes them out
+// together: 62 M bf16 elements, 3.4 % found, 32 us with each written at once, 27.6 so (and the move behind it 11.1 and
+// 8.8, since a streamed tensor leaves the findings in the caches); 62 M fp32 elements, 10 % found, 67 and 56.  The
+// read alone takes 21.
+constexpr uint32_t kHeld = 512;
+template <typename S>
+struct Held {
+  int32_t idx[kHeld];
+  S val[kHeld];
+};
+
 // A wave's walk over elements [begin, end) (begin a multiple of the vector length): selected element number i goes
 // to idx[i], val[i] if i < room.  Returns how many there are.  WRITE == false: only counts.  A stretch holds fewer
-// than 2^18 elements, so that byte offsets from the (uniform) pointers fit 32 bits.
-template <typename S, bool ALIGNED, bool WRITE, typename I>
+// than 2^18 elements, so that byte offsets from the (uniform) pointers fit 32 bits.  HOLD: by way of `held`.
+template <typename S, bool ALIGNED, bool WRITE, bool HOLD = false, typename I>
 __device__ __forceinline__ uint32_t walk(const S *__restrict__ in, int64_t begin, int64_t end, uint32_t least,
-                                I *__restrict__ idx, S *__restrict__ val, uint32_t room) {
+                                I *__restrict__ idx, S *__restrict__ val, uint32_t room, Held<S> *held = nullptr) {
   constexpr int V = VecOf<S>::kN;
   const int lane = lane_id();
   uint32_t found = 0;
+  uint32_t kept = 0;  // in `held`: the last ones found
   constexpr int64_t kStep = (int64_t)row<S>() * kRows;
-  // Unaligned, the steps in flight are whole ones, and the rest of the stretch follows row by row: with the rows'
+  // Unaligned or held, the steps in flight are whole ones, and the rest of the stretch follows row by row: with the rows'
   // elements loaded one by one in this loop, 47 of its registers went to memory and were read again at every step
   // (62 M bf16 elements from an odd one on: 97 us, now 38; fp32, where they fitted, 84 and 61).
-  const int64_t whole = ALIGNED ? end : begin + (end - begin) / kStep * kStep;
+  const int64_t whole = ALIGNED && !HOLD ? end : begin + (end - begin) / kStep * kStep;
   auto load = [&](int64_t base, uint4 &a, uint4 &b, uint4 &c, uint4 &d) {
-    if (!ALIGNED || base + kStep <= end) {
+    if (!ALIGNED || HOLD || base + kStep <= end) {
       const S *at = in + base + lane * V;
-      a = load16<S, ALIGNED>(at);
-      b = load16<S, ALIGNED>(at + row<S>());
-      c = load16<S, ALIGNED>(at + 2 * row<S>());
-      d = load16<S, ALIGNED>(at + 3 * row<S>());
+      a = load16<S, ALIGNED, HOLD>(at);
+      b = load16<S, ALIGNED, HOLD>(at + row<S>());
+      c = load16<S, ALIGNED, HOLD>(at + 2 * row<S>());
+      d = load16<S, ALIGNED, HOLD>(at + 3 * row<S>());
     } else {
       auto one = [&](int64_t first, uint4 &q) {
         S e[V];
@@ -109,14 +126,47 @@ __device__ __forceinline__ uint32_t walk(const S *__restrict__ in, int64_t begin
       ++pos;
     }
   };
+  auto hold = [&](const uint4 &q, uint32_t bits, uint32_t pos, uint32_t first) {
+    while (bits) {
+      const uint32_t e = (uint32_t)__ffs((int)bits) - 1u;
+      bits &= bits - 1u;
+      held->idx[pos] = (int32_t)(first + e);
+      held->val[pos] = vec_pick(q, e, S(0));
+      ++pos;
+    }
+  };
+  auto write_held = [&]() {
+    __builtin_amdgcn_wave_barrier();
+    for (uint32_t i = (uint32_t)lane; i < kept; i += 64u) {
+      const uint32_t pos = found - kept + i;
+      if (pos < room) {
+        idx[pos] = (I)held->idx[i];
+        val[pos] = held->val[i];
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    kept = 0;
+  };
   // two rows' counts in the halves of a word (a row has 512 elements at most)
   auto two = [&](const uint4 &q0, const uint4 &q1, uint32_t first) {
     const uint32_t x0 = vec_flags(q0, least, S(0)), x1 = vec_flags(q1, least, S(0));
     const uint32_t c = (uint32_t)__popc(x0) | ((uint32_t)__popc(x1) << 16);
     const uint32_t incl = wave_inclusive_scan(c);
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    const uint32_t before = incl - c;
+    if (HOLD) {
+      static_assert(row<S>() <= (int)kHeld, "a row fits");
+      if (kept + (total & 0xffffu) > kHeld) write_held();
+      hold(q0, x0, kept + (before & 0xffffu), first);
+      kept += total & 0xffffu;
+      found += total & 0xffffu;
+      if (kept + (total >> 16) > kHeld) write_held();
+      hold(q1, x1, kept + (before >> 16), first + (uint32_t)row<S>());
+      kept += total >> 16;
+      found += total >> 16;
+      return;
+    }
     if (WRITE) {
-      const uint32_t before = incl - c;
       write(q0, x0, found + (before & 0xffffu), first);
       write(q1, x1, found + (total & 0xffffu) + (before >> 16), first + (uint32_t)row<S>());
     }
@@ -136,16 +186,17 @@ __device__ __forceinline__ uint32_t walk(const S *__restrict__ in, int64_t begin
     two(a, b, first);
     two(c, d, first + 2u * (uint32_t)row<S>());
   }
-  if constexpr (!ALIGNED) {
+  if constexpr (!ALIGNED || HOLD) {
 #pragma unroll 1
     for (int64_t base = whole; base < end; base += row<S>()) {
       S e[V];
-      load_vec<S, false>(in, base + lane * V, end, e);
+      load_vec<S, ALIGNED>(in, base + lane * V, end, e);
       uint4 q;
       __builtin_memcpy(&q, e, 16);
       two(q, make_uint4(0, 0, 0, 0), (uint32_t)base + (uint32_t)(lane * V));
     }
   }
+  if (HOLD) write_held();
   return found;
 }
 
@@ -189,13 +240,15 @@ Stretches plan_stretches(void *workspace, int64_t n, size_t *bytes) {
 template <typename S, bool ALIGNED>
 __global__ __launch_bounds__(kBlock, 8) void k_compact_walk(const S *__restrict__ in, int64_t n,
                                                             const uint32_t *__restrict__ thr, Stretches st) {
-  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)));
+  __shared__ Held<S> held[kBlock / 64];  // of a wave each
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t w = blockIdx.x * (uint32_t)(kBlock / 64) + wave;
   if (w >= st.count) return;
   const int64_t begin = (int64_t)w * st.len;
   const int64_t end = begin + st.len < n ? begin + st.len : n;
   const uint32_t found =
-      walk<S, ALIGNED, true>(in, begin, end, least_key(thr, KeyOf<S>::kMask), st.idx + (size_t)w * st.quota,
-                             static_cast<S *>(st.val) + (size_t)w * st.quota, st.quota);
+      walk<S, ALIGNED, true, true>(in, begin, end, least_key(thr, KeyOf<S>::kMask), st.idx + (size_t)w * st.quota,
+                                   static_cast<S *>(st.val) + (size_t)w * st.quota, st.quota, &held[wave]);
   if (lane_id() == 0) st.found[w] = found;
 }
 
@@ -283,7 +336,7 @@ __global__ __launch_bounds__(kMoveBlock) void k_compact_one(const S *__restrict_
   const int64_t len = (n + kMoveWaves * row<S>() - 1) / (kMoveWaves * row<S>()) * row<S>();
   const int64_t begin = (int64_t)wave * len < n ? (int64_t)wave * len : n;
   const int64_t end = begin + len < n ? begin + len : n;
-  const uint32_t mine = walk<S, ALIGNED, false, I>(in, begin, end, least, nullptr, nullptr, 0);
+  const uint32_t mine = walk<S, ALIGNED, false, false, I>(in, begin, end, least, nullptr, nullptr, 0);
   if (lane_id() == 0) own[wave] = mine;
   __syncthreads();
   uint64_t at = 0, all = 0;
