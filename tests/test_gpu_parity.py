@@ -1103,6 +1103,35 @@ def test_count_the_host_is_told_by_the_merge(zen, r, n, dtype):
         assert torch.equal(got_idx, at) and torch.equal(got_val, want[at].to(dtype))
 
 
+@pytest.mark.parametrize("s", [1, 2048, 2049, 3072, 3073, 16384, 16385, 65536, 65537, 270000])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sample_threshold_of_every_size(zen, s, dtype):
+    """One workgroup, several with the search in the second launch, with a third: the k-th largest and how many reach
+    it, for distinct magnitudes, few different ones, magnitudes that share their upper half, and mostly zeros."""
+    from zen_repro_amd import _lib
+
+    L, dev = _lib.lib(), torch.device("cuda", torch.cuda.current_device())
+    gen = torch.Generator(device="cuda").manual_seed(s)
+    n = 300007
+    noise = torch.randn(n, generator=gen, device="cuda")
+    near = (torch.randint(0x3f800000, 0x3f800900, (n,), generator=gen, device="cuda", dtype=torch.int32)).view(torch.float32)
+    at = torch.randint(0, n, (s,), generator=gen, device="cuda")
+    for values in (noise, (noise * 3).round(), near, noise * (noise > 2.5)):
+        t = values.to(dtype)
+        code = _lib.dtype_code(t)
+        keys = t[at].float().abs().view(torch.int32)
+        ordered = torch.sort(keys, descending=True)[0]
+        ws = torch.empty(L.zen_sample_threshold_workspace(s, code), dtype=torch.uint8, device=dev)
+        for k in {1, s, max(1, s // 20), max(1, s // 2)}:
+            thr = torch.full((2,), -1, dtype=torch.int32, device=dev)
+            status = torch.zeros(1, dtype=torch.int32, device=dev)
+            assert L.zen_sample_threshold(_lib.ptr(t), code, n, _lib.ptr(at), s, k, _lib.ptr(thr), _lib.ptr(ws), ws.numel(),
+                                          _lib.ptr(status), _lib.stream_of(dev)) == 0
+            want = ordered[k - 1].item()
+            assert thr.tolist() == [want >> 16 if dtype == torch.bfloat16 else want, (keys >= want).sum().item()]
+            assert status.item() == 0
+
+
 @pytest.mark.parametrize("shift", [0, 1])
 @pytest.mark.parametrize("n", [65537, 65536 + 2048, 65536 + 2049, 200001, 20000000])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

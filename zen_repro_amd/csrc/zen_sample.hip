@@ -8,8 +8,9 @@
 //   more, bf16                k_sample_count (every workgroup keeps 32768 16-bit counters in LDS and writes them
 //                             out, with sums of 64 neighbours each: nothing has to be zero beforehand and no
 //                             atomic leaves the compute unit), k_sample_pick (one workgroup);
-//   more, fp32                the elements are kept too; a third kernel lists the low halves of those in the
-//                             k-th's bin and its last workgroup picks among them.
+//   more, fp32                the elements are kept too, and the low halves of those in the k-th's bin decide: in the
+//                             picking workgroup up to 16 384 elements, else a third kernel lists them and its last
+//                             workgroup picks among them.
 #include "zen_select.h"
 
 namespace zen {
@@ -17,16 +18,19 @@ namespace {
 
 constexpr int kBins = 32768;       // 15 bits of the magnitude key
 constexpr int kBlock = 1024;
-// One workgroup as long as it takes no longer than the two (bf16) or three (fp32) launches for larger samples: every
+// One workgroup as long as it takes no longer than the two launches for larger samples: every
 // 1024 elements cost it 2.5 us, the gather of a single compute unit and its counting loop.  A call in one launch and
-// in several, us: bf16 1024 elements 9.8 and 13, 4096 17.8 and 13.6, 8192 28.8 and 14.0; fp32 1024 elements 12.9 and
-// 20, 4096 21.0 and 20.5, 10 486 39.0 and 20.6.
+// in two, us: bf16 1024 elements 9.8 and 13, 4096 17.8 and 13.6, 8192 28.8 and 14.0; fp32 2048 elements 15.0 and 17,
+// 4096 19.7 and 17.2, 10 486 39.0 and 17.1.
 template <typename S>
-constexpr int one_items() { return sizeof(S) == 2 ? 2 : 4; }
+constexpr int one_items() { return sizeof(S) == 2 ? 2 : 3; }
 template <typename S>
 constexpr int64_t one_max() { return one_items<S>() * kBlock; }
 constexpr int kGroup = 64;         // bins per sum
 constexpr int kGroups = kBins / kGroup;
+// elements per thread up to which the picking workgroup looks at an fp32 sample's low halves itself (a call for 10 486
+// elements 20.4 us with the third launch, 17.1 without; 32 registers for them 18.1, and 20.0 instead of 22.0 at 32 768)
+constexpr int kFewItems = 16;
 constexpr int kRound = 4;          // elements per thread in flight in the counting kernel
 constexpr int64_t kShare = 65535;  // elements a workgroup counts at most (16-bit counters)
 // the bins' 16-bit counters, two to a word, one word of padding per 32 (a thread reads 16 neighbouring words)
@@ -246,9 +250,68 @@ __device__ inline void sum_columns(const uint16_t *from, size_t stride, uint32_t
   __syncthreads();
 }
 
-template <typename S>
-__global__ __launch_bounds__(kBlock) void k_sample_pick(SampleTables tb, uint32_t rows, uint32_t k,
+// fp32: the threshold among the m elements in the k-th's bin `top`, by their low halves at(0..m), eight bits at a time;
+// rank: the k-th's inside the bin, above: elements in the bins above it.  By the whole workgroup.
+template <typename At>
+__device__ inline void low_halves(uint32_t m, uint32_t top, uint32_t rank, uint32_t above, uint32_t *__restrict__ thr, At at) {
+  __shared__ uint32_t hist[256];
+  __shared__ uint32_t smem[kBlock / 64 + 1];
+  __shared__ uint32_t found[3];
+  uint32_t prefix = 0;
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+    if (threadIdx.x < 256) hist[threadIdx.x] = 0;
+    __syncthreads();
+    const uint32_t rounds = (m + kBlock - 1) / kBlock;
+    for (uint32_t r = 0; r < rounds; ++r) {
+      const uint32_t j = r * kBlock + threadIdx.x;
+      const uint32_t x = j < m ? at(j) : 0u;
+      const bool live = j < m && (pass == 0 || (x >> 8) == prefix);
+      const uint32_t digit = pass == 0 ? x >> 8 : x & 0xffu;
+      const uint64_t all = __ballot(live);  // equal digits add together where they are all equal (see count_bin)
+      if (all) {
+        const int lead = __ffsll((unsigned long long)all) - 1;
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)digit, lead);
+        if (__ballot(live && digit == first) == all) {
+          if (lane_id() == lead) atomicAdd(&hist[first], (uint32_t)__popcll(all));
+        } else if (live) {
+          atomicAdd(&hist[digit], 1u);
+        }
+      }
+    }
+    __syncthreads();
+    const uint32_t c = threadIdx.x < 256 ? hist[255 - threadIdx.x] : 0u;
+    uint32_t total;
+    const uint32_t before = block_exclusive_scan<uint32_t, kBlock>(c, smem, &total);
+    if (before < rank && rank <= before + c) {
+      found[0] = 255u - threadIdx.x;
+      found[1] = before;
+      found[2] = c;
+    }
+    __syncthreads();
+    prefix = (prefix << 8) | found[0];
+    rank -= found[1];
+    above += found[1];
+  }
+  if (threadIdx.x == 0) {
+    thr[0] = (top << 16) | prefix;
+    thr[1] = above + found[2];
+  }
+}
+
+// FEW (fp32): the sample's keys are few enough for this workgroup's registers, and it finishes the search itself.
+template <typename S, bool FEW>
+__global__ __launch_bounds__(kBlock) void k_sample_pick(SampleTables tb, uint32_t rows, uint32_t s, uint32_t k,
                                                         uint32_t *__restrict__ thr) {
+  constexpr int kItems = FEW ? kFewItems : 1;
+  uint32_t key[kItems];
+  if (FEW) {  // on their way while the bin is found
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      const uint32_t j = threadIdx.x + (uint32_t)i * kBlock;
+      key[i] = tb.sample[j < s ? j : 0u];
+    }
+  }
   __shared__ uint32_t acc[kGroups];
   __shared__ uint32_t smem[kBlock / 64 + 1];
   __shared__ uint32_t found[3];
@@ -275,13 +338,30 @@ __global__ __launch_bounds__(kBlock) void k_sample_pick(SampleTables tb, uint32_
         thr[0] = bin;
         thr[1] = above + c;
       } else {
-        tb.state[0] = bin;
-        tb.state[1] = k - above;
-        tb.state[2] = above;
+        if (FEW) {
+          found[0] = bin;
+          found[1] = above;
+        } else {
+          tb.state[0] = bin;
+          tb.state[1] = k - above;
+          tb.state[2] = above;
+        }
       }
     }
   }
-  if (sizeof(S) == 4 && threadIdx.x < 2) tb.state[3 + threadIdx.x] = 0;
+  if (sizeof(S) == 4 && !FEW && threadIdx.x < 2) tb.state[3 + threadIdx.x] = 0;
+  if (FEW) {
+    __shared__ uint16_t members[kFewItems * kBlock];
+    __shared__ uint32_t listed;
+    if (threadIdx.x == 0) listed = 0;
+    __syncthreads();
+    const uint32_t top = found[0], above = found[1];
+#pragma unroll
+    for (int i = 0; i < kItems; ++i)
+      if (threadIdx.x + (uint32_t)i * kBlock < s && (key[i] >> 16) == top) members[atomicAdd(&listed, 1u)] = (uint16_t)key[i];
+    __syncthreads();
+    low_halves(listed, top, k - above, above, thr, [&](uint32_t j) -> uint32_t { return members[j]; });
+  }
 }
 
 // fp32: the low halves of the keys in the k-th's bin (a few thousand of millions) are listed by all workgroups;
@@ -316,50 +396,10 @@ __global__ __launch_bounds__(kBlock) void k_sample_members(SampleTables tb, int6
   if (threadIdx.x == 0) last = atomicAdd(&tb.state[4], 1u) == gridDim.x - 1u;
   __syncthreads();
   if (!last) return;
-  __shared__ uint32_t hist[256];
-  __shared__ uint32_t smem[kBlock / 64 + 1];
-  __shared__ uint32_t found[3];
   const uint32_t m = load_fresh(&tb.state[3]);
-  uint32_t rank = tb.state[1], above = tb.state[2], prefix = 0;
-#pragma unroll
-  for (int pass = 0; pass < 2; ++pass) {
-    if (threadIdx.x < 256) hist[threadIdx.x] = 0;
-    __syncthreads();
-    const uint32_t rounds = (m + kBlock - 1) / kBlock;
-    for (uint32_t r = 0; r < rounds; ++r) {
-      const uint32_t j = r * kBlock + threadIdx.x;
-      const uint32_t x = j < m ? __hip_atomic_load(&tb.members[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-      const bool live = j < m && (pass == 0 || (x >> 8) == prefix);
-      const uint32_t digit = pass == 0 ? x >> 8 : x & 0xffu;
-      const uint64_t all = __ballot(live);  // equal digits add together where they are all equal (see count_bin)
-      if (all) {
-        const int lead = __ffsll((unsigned long long)all) - 1;
-        const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)digit, lead);
-        if (__ballot(live && digit == first) == all) {
-          if (lane_id() == lead) atomicAdd(&hist[first], (uint32_t)__popcll(all));
-        } else if (live) {
-          atomicAdd(&hist[digit], 1u);
-        }
-      }
-    }
-    __syncthreads();
-    const uint32_t c = threadIdx.x < 256 ? hist[255 - threadIdx.x] : 0u;
-    uint32_t total;
-    const uint32_t before = block_exclusive_scan<uint32_t, kBlock>(c, smem, &total);
-    if (before < rank && rank <= before + c) {
-      found[0] = 255u - threadIdx.x;
-      found[1] = before;
-      found[2] = c;
-    }
-    __syncthreads();
-    prefix = (prefix << 8) | found[0];
-    rank -= found[1];
-    above += found[1];
-  }
-  if (threadIdx.x == 0) {
-    thr[0] = (top << 16) | prefix;
-    thr[1] = above + found[2];
-  }
+  low_halves(m, top, tb.state[1], tb.state[2], thr, [&](uint32_t j) -> uint32_t {
+    return __hip_atomic_load(&tb.members[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  });
 }
 
 // Workgroups of the counting kernel for a sample of s elements: up to 64, an element per thread (a call for 10 486
@@ -409,9 +449,11 @@ int sample_threshold_launch(const S *in, int64_t n, const int64_t *at, int64_t s
   const int64_t rows = ceil_div(s, share);
   k_sample_count<S><<<dim3((unsigned)rows), dim3(kBlock), 0, stream>>>(in, n, at, s, share, tb, status);
   ZEN_LAUNCH_CHECK("k_sample_count");
-  k_sample_pick<S><<<dim3(1), dim3(kBlock), 0, stream>>>(tb, (uint32_t)rows, (uint32_t)k, thr);
+  const bool few = sizeof(S) == 4 && s <= kFewItems * kBlock;
+  const auto pick = few ? k_sample_pick<S, sizeof(S) == 4> : k_sample_pick<S, false>;
+  pick<<<dim3(1), dim3(kBlock), 0, stream>>>(tb, (uint32_t)rows, (uint32_t)s, (uint32_t)k, thr);
   ZEN_LAUNCH_CHECK("k_sample_pick");
-  if (sizeof(S) == 4) {
+  if (sizeof(S) == 4 && !few) {
     int64_t blocks = ceil_div(s, (int64_t)kBlock * kMemberItems);
     if (blocks > 256) blocks = 256;
     k_sample_members<<<dim3((unsigned)blocks), dim3(kBlock), 0, stream>>>(tb, s, thr);
