@@ -3,7 +3,8 @@
  * select / hash-partition / merge path.  Plain C ABI: device pointers, sizes
  * and a HIP stream.  No torch types, no hidden allocation, no host
  * synchronisation: every call only enqueues kernels on `stream`, but for
- * zen_host_words_alloc / _free and zen_read_back, which exist to wait,
+ * zen_host_words_alloc / _free, zen_read_back and the calls that take host
+ * words (_sizes, _count, _status), which exist to wait,
  * zen_bitmap_dense_dict with `members`, and zen_profile_read.
  *
  * Conventions
