@@ -953,3 +953,31 @@ def test_workgroups_that_take_the_next_sample_leave_their_first_tiles_to_the_oth
         assert e[3].item() == 0 == want[3].item() and total >= ks[i]
         for got, ref in ((e[0][:total], want[0][:total]), (e[1][:total], want[1][:total]), (e[2], want[2])):
             assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("dtype, sub", [(torch.bfloat16, 8192), (torch.float32, 4096)])
+@pytest.mark.parametrize("more", [-4097, -1, 0, 1, 8191])
+def test_every_element_is_looked_at_once(zen, dtype, sub, more):
+    """Around the tensor length where the select kernel hands out more of its tiles by ticket (sixteen sub-tiles for
+    each of three workgroups per compute unit), with and without the next call's sample taken along: the sent entries
+    are the tensor's, each once."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n, P = sub * 16 * 3 * cus + more, 4
+    k = n // 200
+    gen = torch.Generator(device="cuda").manual_seed(sub + more)
+    grad = torch.randn(n, generator=gen, device="cuda").to(dtype)
+    grad[-3:] = 9
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P), None, None)
+    recv = (torch.arange(1, 5000, device="cuda", dtype=torch.int32), torch.ones(4999, device="cuda", dtype=dtype))
+    for nxt in (None, grad):
+        thr = torch.zeros(2, dtype=torch.int32, device="cuda")
+        (idx, val, splits, status), _ = lba.encode_merge_flat(lba.tensor_partition, grad, k + k // 4 + 4096, k, *recv, n,
+                                                              thr_out=thr, next_tensor=nxt)
+        key, reached = thr.tolist()
+        least = torch.tensor([key << 16 if dtype == torch.bfloat16 else key], dtype=torch.int32).view(torch.float32).item()
+        passed = grad.abs() >= least
+        assert status.item() == 0 and reached >= k and reached == int(passed.sum())
+        passed[0] = False  # index 0 is never sent
+        want, total = torch.nonzero(passed).view(-1), int(splits.sum())
+        order = torch.sort(idx[:total])
+        assert torch.equal(order[0].long(), want) and torch.equal(val[:total][order[1]], grad[want])

@@ -832,6 +832,7 @@ __device__ inline void stage_flush(uint32_t count, int32_t *st_idx, S *st_val, S
 constexpr int kStageBig = 2;    // both tile lengths must be at least 2: the loads run two sub-tiles ahead
 constexpr int kStageSmall = 2;
 constexpr int kStageGroups = 8;
+constexpr int64_t kStageFew = 16;    // sub-tiles per workgroup below which more of them go out by ticket
 constexpr uint32_t kStageLate = 2;   // some 8 us
 constexpr int kStageTicketPad = 32;  // words between two ticket counters: a 128-byte line each
 struct StageSched {
@@ -1262,9 +1263,13 @@ static int stage_launch(const StageArgs &a, hipStream_t stream) {
   const int64_t least = ceil_div(subs, kStageSmall);
   if (blocks > least) blocks = least;
   // seven eighths of the tensor in counter-free tiles, the rest through tickets (measured on 1.5 GB: all
-  // tickets 280 us, two thirds fixed 252, seven eighths 247, everything fixed 258)
+  // tickets 280 us, two thirds fixed 252, seven eighths 247, everything fixed 258).  Half of it where a workgroup has few
+  // sub-tiles: one that a merge on another stream kept off its compute unit, or that took the next call's sample, is a
+  // larger part of the pass late then (twelve buckets of 62 M bf16 elements, ten sub-tiles each: 936 -> 920 us a pass,
+  // all tickets 933; 268 M, 42 each: 733 -> 738; 2^30 fp32, 341 each: 1105 -> 1155).
   StageSched sch;
-  sch.fixed = (uint32_t)(subs * 7 / 8 / ((int64_t)kStageBig * blocks));
+  const int64_t fixed_subs = subs < kStageFew * blocks ? subs / 2 : subs * 7 / 8;
+  sch.fixed = (uint32_t)(fixed_subs / ((int64_t)kStageBig * blocks));
   const S *in = static_cast<const S *>(a.in);
   const bool aligned = (reinterpret_cast<uintptr_t>(in) & 15u) == 0 && a.n >= V;
   const StageSlabs out{a.geo, a.cg, a.coarse_cursor, a.coarse_words};
