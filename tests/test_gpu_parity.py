@@ -1103,7 +1103,7 @@ def test_count_the_host_is_told_by_the_merge(zen, r, n, dtype):
         assert torch.equal(got_idx, at) and torch.equal(got_val, want[at].to(dtype))
 
 
-@pytest.mark.parametrize("s", [1, 2048, 2049, 3072, 3073, 16384, 16385, 65536, 65537, 270000])
+@pytest.mark.parametrize("s", [1, 1024, 1025, 5120, 5121, 16384, 16385, 65536, 65537, 270000])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_sample_threshold_of_every_size(zen, s, dtype):
     """One workgroup, several with the search in the second launch, with a third: the k-th largest and how many reach

@@ -4,7 +4,7 @@
 // per sample element.  A radix select behind a gather took 6 to 8 dependent launches, each a few microseconds of
 // work; here the histogram is taken while the elements arrive, at 15 bits of the magnitude (for bf16 the whole
 // key), so that one more workgroup finds the k-th:
-//   up to one_max() elements  one workgroup does everything in one launch, the elements in registers;
+//   up to kOneMax elements    one workgroup does everything in one launch, the elements in registers;
 //   more, bf16                k_sample_count (every workgroup keeps 32768 16-bit counters in LDS and writes them
 //                             out, with sums of 64 neighbours each: nothing has to be zero beforehand and no
 //                             atomic leaves the compute unit), k_sample_pick (one workgroup);
@@ -18,14 +18,14 @@ namespace {
 
 constexpr int kBins = 32768;       // 15 bits of the magnitude key
 constexpr int kBlock = 1024;
-// One workgroup as long as it takes no longer than the two launches for larger samples: every
-// 1024 elements cost it 2.5 us, the gather of a single compute unit and its counting loop.  A call in one launch and
-// in two, us: bf16 1024 elements 9.8 and 13, 4096 17.8 and 13.6, 8192 28.8 and 14.0; fp32 2048 elements 15.0 and 17,
-// 4096 19.7 and 17.2, 10 486 39.0 and 17.1.
-template <typename S>
-constexpr int one_items() { return sizeof(S) == 2 ? 2 : 3; }
-template <typename S>
-constexpr int64_t one_max() { return one_items<S>() * kBlock; }
+// One workgroup as long as that is no slower than the two launches for larger samples: every 1024 elements cost it
+// 2.5 us, the gather of a single compute unit and its counting loop, and the other way costs a launch of the host's.  A
+// call in one launch and in two, us by events: bf16 1024 elements 9.8 and 13, 4096 17.8 and 13.6, 8192 28.8 and 14.0;
+// fp32 2048 elements 15.0 and 17, 4096 19.7 and 17.2, 10 486 39.0 and 17.1.  In front of a compress and a load balance,
+// which are bound by the host, one launch stays ahead a little longer: 4565 bf16 elements 100 and 104.5 us a pass, 4000
+// fp32 102.5 and 105, but 7000 bf16 106 and 103.
+constexpr int kOneItems = 5;
+constexpr int64_t kOneMax = kOneItems * kBlock;
 constexpr int kGroup = 64;         // bins per sum
 constexpr int kGroups = kBins / kGroup;
 // elements per thread up to which the picking workgroup looks at an fp32 sample's low halves itself (a call for 10 486
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(kBlock) void k_sample_one(const S *__restrict__ in,
   __shared__ uint32_t low[2];
   clear_hist(hist);
   if (threadIdx.x < 2) low[threadIdx.x] = 0;
-  constexpr int kItems = one_items<S>();
+  constexpr int kItems = kOneItems;
   S v[kItems];
   gather<S, kItems>(in, n, at, threadIdx.x, s, v, status);
 #pragma unroll
@@ -420,7 +420,7 @@ inline int64_t sample_groups(int64_t s) {
 SampleTables plan_sample(void *workspace, int64_t s, int dtype, size_t *bytes) {
   Carver cv(workspace);
   SampleTables tb{};
-  if (s > (dtype == ZEN_BF16 ? one_max<uint16_t>() : one_max<uint32_t>())) {
+  if (s > kOneMax) {
     const size_t g = (size_t)sample_groups(s);
     tb.state = cv.take<uint32_t>(8);
     tb.sums = cv.take<uint16_t>(g * kGroups);
@@ -437,7 +437,7 @@ SampleTables plan_sample(void *workspace, int64_t s, int dtype, size_t *bytes) {
 template <typename S>
 int sample_threshold_launch(const S *in, int64_t n, const int64_t *at, int64_t s, int64_t k, uint32_t *thr,
                             void *workspace, int32_t *status, hipStream_t stream) {
-  if (s <= one_max<S>()) {
+  if (s <= kOneMax) {
     k_sample_one<S><<<dim3(1), dim3(kBlock), 0, stream>>>(in, n, at, (uint32_t)s, (uint32_t)k, thr, status);
     ZEN_LAUNCH_CHECK("k_sample_one");
     return ZEN_OK;
