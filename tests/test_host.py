@@ -410,6 +410,62 @@ def test_streams_wait_for_a_call_that_returned_before_its_kernels_were_through(m
     assert log == [(2, 1), (1, 2), (3, 2)]
 
 
+@pytest.mark.parametrize("call", ["load_balance", "encode_sparse_tensor", "decode_sparse_tensors", "merge_rounded"])
+@pytest.mark.parametrize("code", [0, -2])
+def test_calls_that_return_early_leave_their_buffers_marked(monkeypatch, call, code):
+    """The four calls whose kernels tell the host sizes or a status return while the last of them may still use the
+    call's workspace (and table).  Two streams that have both used one take turns: each waits for the other's call,
+    one that failed on the device's side among them (what clears the buffer again comes behind it)."""
+    import zen_repro_amd as zen
+    from zen_repro_amd import _lib
+
+    class Stream:
+        def __init__(self, handle):
+            self.cuda_stream = handle
+
+    class Library:  # every size 256, nothing launched
+        def __getattr__(self, name):
+            if name == "zen_last_error":
+                return lambda: b"the device"
+            told = name.endswith(("_sizes", "_count", "_status"))
+            return lambda *args: 0 if name == "zen_merge_zero_bytes" else code if told else 256
+
+    class Words:
+        ptr, words, view = 0, 64, [0] * 64
+
+    waits, now = [], [1]
+    streams = {h: Stream(h) for h in (1, 2)}
+
+    def join(kept, stream, new=False):
+        waits.append((stream.cuda_stream, kept.maker.cuda_stream))
+        kept.seen.add(stream.cuda_stream)
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: streams[now[0]])
+    monkeypatch.setattr(_lib, "lib", Library)
+    monkeypatch.setattr(_lib, "device_index", lambda device: 0)
+    monkeypatch.setattr(_lib, "current_handle", lambda index: now[0])
+    monkeypatch.setattr(_lib, "require_gpu", lambda t, name: None)
+    monkeypatch.setattr(_lib, "host_words", lambda n: Words)
+    monkeypatch.setattr(_lib, "scratch", _lib.Scratch())
+    monkeypatch.setattr(_lib, "zeros", _lib.ZeroPool())
+    monkeypatch.setattr(_lib.Kept, "join", join)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    dense, idx = torch.ones(64), torch.arange(8, dtype=torch.int32)
+    run = {"load_balance": lambda: lba.tensor_partition.load_balance(dense, capacity=64),
+           "encode_sparse_tensor": lambda: lba.encode_sparse_tensor(dense),
+           "decode_sparse_tensors": lambda: lba.decode_sparse_tensors(idx, dense[:8], 64),
+           "merge_rounded": lambda: lba.merge_rounded(idx, dense[:8], 64, torch.float32)}[call]
+    for now[0] in (1, 1, 2, 2, 1, 2):
+        if code:
+            with pytest.raises(RuntimeError, match="the device"):
+                run()
+        else:
+            run()
+    buffers = 2 if call == "load_balance" else 1
+    assert waits == [w for w in [(2, 1), (1, 2), (2, 1)] for _ in range(buffers)]
+
+
 def test_compaction_kernels_keep_their_rows_in_registers(tmp_path):
     """The rows a wave has in flight are the kernels' speed: none of their registers may end up in memory, for
     aligned tensors and for views that begin at an odd element."""

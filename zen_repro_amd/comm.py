@@ -45,8 +45,8 @@ def _select_raw(tensor, thr, idx64, capacity=None):
     rc = L.zen_select_count(_lib.ptr(flat), code, n, _lib.ptr(thr), _lib.ptr(out_idx), 1 if idx64 else 0,
                             _lib.ptr(out_val), capacity, _lib.ptr(count), _lib.ptr(ws), ws.numel(),
                             _lib.ptr(status), words.ptr, words.words, _lib.stream_of(dev))
-    _lib.check(rc, "select")
     _lib.scratch.left_running(dev, "select")
+    _lib.check(rc, "select")
     host = words.view[1:3]
     kept = min(host[0], capacity)
     return out_idx[:kept], out_val[:kept], host[0], host[1]
@@ -125,6 +125,7 @@ class LoadBalanceAllreduce:
                                            _lib.dtype_code(values), r, _lib.ptr(dense), alltoall_dense_size,
                                            mode | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status),
                                            words.ptr, words.words, _lib.stream_of(dev))
+            _lib.scratch.left_running(dev, "decode")
             if rc != _lib.OK:
                 ws[:L.zen_merge_zero_bytes()].zero_()
             _lib.check(rc, "decode_sparse_tensors")
@@ -225,6 +226,7 @@ class LoadBalanceAllreduce:
                 mode | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status))
         if words is not None:
             rc = L.zen_merge_rounded_count(*args, words.ptr, words.words, _lib.stream_of(dev))
+            _lib.scratch.left_running(dev, f"merge/{slot}")
         else:
             rc = (L.zen_merge_rounded if rounded else L.zen_merge)(*args, _lib.stream_of(dev))
         if rc != _lib.OK:

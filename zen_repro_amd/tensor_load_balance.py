@@ -404,12 +404,12 @@ class TensorPartition:
             rc = L.zen_load_balance(*args, _lib.stream_of(dev))
         else:
             rc = L.zen_load_balance_sizes(*args, words.ptr, words.words, _lib.stream_of(dev))
-        if rc != _lib.OK:
-            table.zero_()  # a call that failed half way may have left entries behind
-        _lib.check(rc, "load_balance")
         if words is not None:
             _lib.scratch.left_running(dev, f"load_balance/{slot}")
             kept.left_running(dev)
+        if rc != _lib.OK:
+            table.zero_()  # a call that failed half way may have left entries behind
+        _lib.check(rc, "load_balance")
         self._after_call(flat, int(k), capacity, slot, mode | flags, used)
         return out_idx, out_val, splits, status
 
