@@ -16,6 +16,13 @@
  *     kernels with atomic-or; the caller zeroes it and reads it after a sync);
  *   - `workspace` is caller-provided scratch of at least the size the matching
  *     `*_workspace` function returns; contents are undefined on return;
+ *   - a call that takes host words returns when what it tells the host is
+ *     known.  Everything else about it is complete in the order of `stream`
+ *     only, as with any other call: its outputs, its use of workspace and table,
+ *     and the reading of `input` by zen_load_balance_sizes and of `input` and
+ *     `thr` by zen_select_count (the others have read their inputs).  Whoever goes on
+ *     elsewhere (another stream, memory given back to something that is not in
+ *     the order of `stream`) waits for `stream` first;
  *   - indices are int32 (N < 2^31) as in the reference (functions_cuda.cpp:25-26
  *     narrows numel() to int).
  *
@@ -242,7 +249,7 @@ int zen_select(const void *input, int dtype, int64_t n, const uint32_t *thr,
  * zen_select that returns when the count and *status are in the host words 1
  * and 2, `host` and `words` from zen_host_words_alloc (at least 3).  The
  * entries are complete on the stream, as always, and so is the use of the
- * workspace.
+ * workspace; until then `input` and `thr` may still be read.
  */
 int zen_select_count(const void *input, int dtype, int64_t n, const uint32_t *thr,
                      void *out_idx, int idx64, void *out_val, int64_t capacity,
@@ -293,7 +300,8 @@ int zen_load_balance(const void *input, int dtype, int64_t n, int64_t m,
  * host[1 + partitions] = *status are there, of `words` words from
  * zen_host_words_alloc (at least partitions + 2; one call at a time on a set of
  * words).  The entries themselves are complete on the stream, as always, and
- * may still be on their way to their places when the call returns.
+ * may still be on their way to their places when the call returns, some of them
+ * from `input`: it must not be overwritten but in the order of the stream.
  */
 int zen_load_balance_sizes(const void *input, int dtype, int64_t n, int64_t m,
                            int partitions, int rehash, const uint32_t *thr, int64_t k,

@@ -433,7 +433,7 @@ def test_calls_that_return_early_leave_their_buffers_marked(monkeypatch, call, c
     class Words:
         ptr, words, view = 0, 64, [0] * 64
 
-    waits, now = [], [1]
+    waits, held, now = [], [], [1]
     streams = {h: Stream(h) for h in (1, 2)}
 
     def join(kept, stream, new=False):
@@ -450,6 +450,7 @@ def test_calls_that_return_early_leave_their_buffers_marked(monkeypatch, call, c
     monkeypatch.setattr(_lib, "scratch", _lib.Scratch())
     monkeypatch.setattr(_lib, "zeros", _lib.ZeroPool())
     monkeypatch.setattr(_lib.Kept, "join", join)
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, s: held.append((t.data_ptr(), s.cuda_stream)))
     lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
     dense, idx = torch.ones(64), torch.arange(8, dtype=torch.int32)
     run = {"load_balance": lambda: lba.tensor_partition.load_balance(dense, capacity=64),
@@ -464,6 +465,9 @@ def test_calls_that_return_early_leave_their_buffers_marked(monkeypatch, call, c
             run()
     buffers = 2 if call == "load_balance" else 1
     assert waits == [w for w in [(2, 1), (1, 2), (2, 1)] for _ in range(buffers)]
+    # two of them may still read their input, which the allocator is told of; the others are through with theirs
+    reads = call in ("load_balance", "encode_sparse_tensor")
+    assert held == ([(dense.data_ptr(), s) for s in (1, 1, 2, 2, 1, 2)] if reads else [])
 
 
 def test_compaction_kernels_keep_their_rows_in_registers(tmp_path):

@@ -236,12 +236,17 @@ class Kept:
             self.buf.record_stream(stream)
             self.seen.add(stream.cuda_stream)
 
-    def left_running(self, device):
+    def left_running(self, device, *inputs):
         """A call that waits for its sizes has returned while its last kernels may still use the buffer on the
-        current stream: every other stream waits for that at its next use, like for the making."""
+        current stream: every other stream waits for that at its next use, like for the making.  `inputs` (None:
+        not given): tensors those kernels still read, whose memory is not handed out before they have, also if it
+        belongs to another stream's pool and its owner drops it now."""
         if len(self.seen) > 1:  # else no stream but this one has used it
             self.maker = torch.cuda.current_stream(device)
             self.seen = {self.maker.cuda_stream}
+        for t in inputs:
+            if t is not None:
+                t.record_stream(self.maker)
 
 
 class Scratch:
@@ -280,9 +285,9 @@ class Scratch:
             kept.join(torch.cuda.current_stream(index) if stream is None else stream)
         return kept.buf
 
-    def left_running(self, device, name):
+    def left_running(self, device, name, *inputs):
         """See Kept.left_running."""
-        self._bufs()[device_index(device), name].left_running(device)
+        self._bufs()[device_index(device), name].left_running(device, *inputs)
 
     def drop(self):
         """Forget the calling thread's buffers."""

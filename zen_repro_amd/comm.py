@@ -28,7 +28,8 @@ class LocalGroup:
 def _select_raw(tensor, thr, idx64, capacity=None):
     """(indices, values, count, status bits) of the selected elements of a flat tensor, ascending; the count
     is that of all elements that pass, also beyond `capacity` (then the bits hold STAT_CAPACITY and the first
-    `capacity` entries are there).  Waits for the count; the entries are complete on the current stream."""
+    `capacity` entries are there).  Waits for the count; the entries are complete on the current stream, and the
+    tensor has been read then."""
     flat = tensor.reshape(-1)
     n = flat.numel()
     dev = flat.device
@@ -45,7 +46,7 @@ def _select_raw(tensor, thr, idx64, capacity=None):
     rc = L.zen_select_count(_lib.ptr(flat), code, n, _lib.ptr(thr), _lib.ptr(out_idx), 1 if idx64 else 0,
                             _lib.ptr(out_val), capacity, _lib.ptr(count), _lib.ptr(ws), ws.numel(),
                             _lib.ptr(status), words.ptr, words.words, _lib.stream_of(dev))
-    _lib.scratch.left_running(dev, "select")
+    _lib.scratch.left_running(dev, "select", flat, thr)
     _lib.check(rc, "select")
     host = words.view[1:3]
     kept = min(host[0], capacity)
@@ -102,7 +103,9 @@ class LoadBalanceAllreduce:
         tensor of the list is a strictly ascending index list (what the second
         exchange and method 1 deliver, comm.py:113-117, 142-145): the dense
         tensor is then built tile by tile without a sort; a list that is not
-        ascending after all only costs the time of the attempt."""
+        ascending after all only costs the time of the attempt.  The payloads
+        have been read when the call returns; the dense tensor is complete on the
+        current stream, for which another stream that reads it waits."""
         L = _lib.lib()
         if ascending:
             dense = self._decode_ascending(indices_tensors, values_tensors, alltoall_dense_size)
@@ -183,7 +186,10 @@ class LoadBalanceAllreduce:
         return [fast] + ([_lib.MODE_FAST | _lib.MODE_SLABS] if not fast & _lib.MODE_SLABS else []) + [_lib.MODE_GENERAL]
 
     def encode_sparse_tensor(self, tensor):
-        """(ascending int64 indices of the nonzeros, their values), comm.py:47-50."""
+        """(ascending int64 indices of the nonzeros, their values), comm.py:47-50.  Both are complete on the current
+        stream, and may still be on their way when the call returns (it waits for their number only); until then the
+        tensor is still read.  Another stream that reads them or overwrites the tensor waits for this one first
+        (dropping the tensor is safe)."""
         _lib.require_gpu(tensor, "input")
         idx, val, _ = _select(tensor, None, idx64=True)
         return idx, val
@@ -380,7 +386,8 @@ class LoadBalanceAllreduce:
     def merge_rounded(self, indices_tensors, values_tensors, dense_size, dtype):
         """merge_sparse followed by the rounding of round_merged_flat: (int64 indices, values of `dtype`), with
         one host synchronisation (the result's size) instead of three, and in one pass where the received values
-        have that type."""
+        have that type.  The payloads have been read when the call returns; the result is complete on the current
+        stream, for which another stream that reads it waits."""
         values_tensors = self.stack_tensors(values_tensors)
         rounded = values_tensors.dtype == dtype
         for mode in self._fast_then_general():

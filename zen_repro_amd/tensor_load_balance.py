@@ -406,7 +406,7 @@ class TensorPartition:
             rc = L.zen_load_balance_sizes(*args, words.ptr, words.words, _lib.stream_of(dev))
         if words is not None:
             _lib.scratch.left_running(dev, f"load_balance/{slot}")
-            kept.left_running(dev)
+            kept.left_running(dev, flat)
         if rc != _lib.OK:
             table.zero_()  # a call that failed half way may have left entries behind
         _lib.check(rc, "load_balance")
@@ -419,7 +419,9 @@ class TensorPartition:
         two contiguous buffers; slicing them needs the split sizes on the
         host, which is this call's only synchronisation: what they hold is
         complete on the current stream, and may still be on its way when the
-        call returns.  Without a `capacity`
+        call returns.  Until then the gradient is still read: another stream that
+        reads the result or overwrites the gradient waits for this one first
+        (dropping the gradient is safe).  Without a `capacity`
         one is worked out and the call is repeated with four times as much
         when the selection turns out larger; `grow=True` asks for the same
         with a capacity that is the caller's estimate."""
