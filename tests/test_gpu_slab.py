@@ -130,6 +130,11 @@ def test_slab_load_balance_odd_length_unaligned_and_empty(zen, oracle, dtype):
     (8, 21, 3),       # buckets of 131 075 slots: just past the narrowest width the bucket kernels come in
     (64, 100, 2),     # the second width
     (3000, 5000, 3),  # 333 333 slots: as many buckets as there may be, and wider than two workgroups to a unit allow
+    (1, 33, 3),       # 366 667 as the records call for: more buckets, so that their bitmaps fit
+    (1, 60, 2),       # 666 667, and too few records for more buckets: by comparisons, like the case before the last
+    (4, 60, 1),       # the same with one level: whoever loses it goes to the serial lists
+    (2500, 7400, 3),  # 592 000
+    (2049, 10800, 2),  # 1 047 600: the widest there is
 ])
 def test_slab_load_balance_at_every_bucket_width(zen, oracle, P, scale, rehash, dtype):
     from zen_repro_amd import _lib

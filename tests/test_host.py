@@ -66,6 +66,17 @@ def test_path_selection_is_host_only(L):
     assert L.zen_merge_path(1000, 1 << 20, 0) == 0
 
 
+@pytest.mark.parametrize("P", [1, 64, 511, 513, 600, 700, 1024, 1025, 1365, 1366, 2048, 2049, 2500, 3000, 4096])
+def test_the_widest_tables_stay_on_the_slabs(L, P):
+    """However badly the partitions fill the 4096 buckets there may be: the largest table has a slab geometry."""
+    from zen_repro_amd import _lib
+
+    m = (2 ** 31 - 1) // P * P
+    for dtype in (0, 1):
+        for k in (0, m // 1000):
+            assert L.zen_load_balance_path(m, m, dtype, m // 900, P, k, _lib.MODE_SLABS) == 2
+
+
 def test_bad_arguments_are_rejected_on_the_host(L):
     from zen_repro_amd import _lib
 

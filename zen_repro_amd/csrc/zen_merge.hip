@@ -440,7 +440,7 @@ SlabMergePlan plan_slab_merge(void *workspace, const SlabGeom &geo, int64_t r) {
 
 bool slab_merge_fits(int64_t r, int64_t dense_n, SlabGeom *geo) {
   SlabGeom g;
-  if (r < (1 << 15) || r > 0x7ffffffell || !slab_geometry(dense_n, 1, r, kMergeTarget, 0, 0, &g)) return false;
+  if (r < (1 << 15) || r > 0x7ffffffell || !slab_geometry(dense_n, 1, r, kMergeTarget, 0, &g)) return false;
   if (g.sub_shift + ceil_log2_u64((uint64_t)r) > 32) return false;  // (index inside a narrow range, arrival number) must fit a word
   if (geo) *geo = g;
   return true;

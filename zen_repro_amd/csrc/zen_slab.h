@@ -92,8 +92,7 @@ inline double slab_bucket_width(uint32_t bpp_mult) { return 4294967296.0 / (doub
 // Host side: geometry for `partitions` partitions of a key space of m keys (m a
 // multiple of partitions) expected to hold about `expected` records, its buckets
 // good_span keys wide or less where the number of buckets allows that (0: any
-// width).  Returns false if the slab layout does not suit these sizes or a bucket
-// would be wider than most_span keys.
+// width).  Returns false if the slab layout does not suit these sizes.
 inline float slab_inverse_below(uint32_t d) {
   const double want = (1.0 / (double)d) * (1.0 - 1.0 / 1048576.0);
   float f = (float)want;
@@ -101,8 +100,7 @@ inline float slab_inverse_below(uint32_t d) {
   return f;
 }
 
-inline bool slab_geometry(int64_t m, int partitions, int64_t expected, int target, int64_t good_span, int64_t most_span,
-                          SlabGeom *out) {
+inline bool slab_geometry(int64_t m, int partitions, int64_t expected, int target, int64_t good_span, SlabGeom *out) {
   if (m < (1ll << 22) || m > 0x7fffffffll || partitions < 1 || partitions > kSlabMaxBuckets || m % partitions != 0 ||
       expected < 1)
     return false;
@@ -133,7 +131,6 @@ inline bool slab_geometry(int64_t m, int partitions, int64_t expected, int targe
   g.bpp_mult = (uint32_t)(((uint64_t)bpp << 32) / (uint64_t)npp);
   g.nbuckets = (uint32_t)nb;
   const uint64_t width = ((1ull << 32) + g.bpp_mult - 1) / g.bpp_mult + 1;  // keys per bucket, at most
-  if (most_span > 0 && width > (uint64_t)most_span) return false;
   g.span = (uint32_t)width;
   g.sub_shift = 0;
   while ((width >> g.sub_shift) >= (uint64_t)kSlabSubs) ++g.sub_shift;
@@ -161,6 +158,7 @@ constexpr int kSlabQueueCap = kSlabCap - kSlabSubs - 1;  // large-group records 
 constexpr int kSlabInline = 4;                            // groups up to this size are ranked by their own threads
 constexpr int kSlabQueueMin = 256;                        // records in larger groups below which nothing is set aside
 struct SlabSortShared {
+  static constexpr bool kQueue = true;
   uint32_t key[kSlabCap];
   union {
     uint32_t tie[kSlabCap];
@@ -174,10 +172,23 @@ struct SlabSortShared {
 };
 static_assert(kSlabSubs + 1 <= kSlabCap, "the counters fit under the ties");
 
+// The same without the queue (whose code costs slab_rank registers).
+struct SlabSortSharedNoQueue {
+  static constexpr bool kQueue = false;
+  uint32_t key[kSlabCap];
+  union {
+    uint32_t tie[kSlabCap];
+    uint32_t cnt[kSlabSubs + 1];
+  };
+  uint32_t scan[kSlabMaxBlock / 64 + 1];
+  uint32_t bad;
+};
+
 // Number of words in sh.key[b0, b1) that are smaller than w.  The words are fetched four at a time (places past
 // the end are pulled back onto the last word and not counted): a loop that fetches one word per turn waits
 // for LDS once per word, and that wait is what such a loop spends its time on.
-__device__ inline uint32_t slab_count_less(const SlabSortShared &sh, uint32_t b0, uint32_t b1, uint32_t w) {
+template <typename Shared>
+__device__ inline uint32_t slab_count_less(const Shared &sh, uint32_t b0, uint32_t b1, uint32_t w) {
   uint32_t less = 0;
   const uint32_t last = b1 - 1u;
   for (uint32_t u = b0; u < b1; u += 4) {
@@ -197,15 +208,15 @@ __device__ inline uint32_t slab_count_less(const SlabSortShared &sh, uint32_t b0
 // inside its group every record counts the words smaller than its own: the first kSlabInline words of every
 // record's group are fetched in one go (all of them in flight together), which settles groups up to that size.
 // Where many records share a key (a merge of payloads that overlap) a few lanes of every wave would then walk
-// through groups of dozens while the others wait: records of groups larger
+// through groups of dozens while the others wait: with a Shared that has a queue, records of groups larger
 // than kSlabInline are set aside instead (their places in the queue follow from the same prefix sums as the
 // groups' places: the counters carry both, 16 bits each) and handed out again afterwards, one per lane, so
 // that the lanes of a wave walk through large groups together.  Returns false (for every thread) if a
 // group is too large for that; else rank[i] for live records and *n_out = number of live records.  On return
 // sh.key / sh.tie may be overwritten at once (sh.tie is not touched at all), and the low 16 bits of
 // sh.cnt[sub_place(s)] hold the sorted place of the first record of narrow range s.
-template <int BLOCK>
-__device__ inline bool slab_rank(SlabSortShared &sh, const SlabGeom &geo, int tie_bits,
+template <int BLOCK, typename Shared>
+__device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
                                  const uint32_t (&off)[kSlabCap / BLOCK], const uint32_t (&tie)[kSlabCap / BLOCK],
                                  uint32_t live, uint32_t (&rank)[kSlabCap / BLOCK], uint32_t *n_out) {
   static_assert(BLOCK <= kSlabMaxBlock && kSlabCap % BLOCK == 0 && kSlabSubs % BLOCK == 0, "workgroup size");
@@ -249,7 +260,7 @@ __device__ inline bool slab_rank(SlabSortShared &sh, const SlabGeom &geo, int ti
   if (sh.bad) return false;
   const uint32_t totals = sh.cnt[kSlabSubs];
   // a few large groups are not worth the extra barrier
-  const bool set_aside = (totals >> 16) >= (uint32_t)kSlabQueueMin;
+  const bool set_aside = Shared::kQueue && (totals >> 16) >= (uint32_t)kSlabQueueMin;
   constexpr uint32_t kSetAside = 0x80000000u;
   uint32_t g0[kItems], g1[kItems], word[kItems];
 #pragma unroll
@@ -261,12 +272,14 @@ __device__ inline bool slab_rank(SlabSortShared &sh, const SlabGeom &geo, int ti
       g1[i] = sh.cnt[sub_place<BLOCK>(sub[i] + 1)] & 0xffffu;
       word[i] = ((off[i] & low_mask) << tie_bits) | tie[i];
       sh.key[g0[i] + at[i]] = word[i];
-      static_assert(kSlabSubs <= (1 << 12) && kSlabGroupLimit <= (1 << 19), "a queue entry is one word");
-      const uint32_t q = (here >> 16) + at[i];
-      if (set_aside && g1[i] - g0[i] > (uint32_t)kSlabInline && q < (uint32_t)kSlabQueueCap) {
-        sh.queue[q] = sub[i] | (at[i] << 12);  // sub < 2^12, at < group size <= kSlabGroupLimit
-        rank[i] = kSetAside | q;
-        g1[i] = g0[i];  // nothing left to do for it below
+      if constexpr (Shared::kQueue) {
+        static_assert(kSlabSubs <= (1 << 12) && kSlabGroupLimit <= (1 << 19), "a queue entry is one word");
+        const uint32_t q = (here >> 16) + at[i];
+        if (set_aside && g1[i] - g0[i] > (uint32_t)kSlabInline && q < (uint32_t)kSlabQueueCap) {
+          sh.queue[q] = sub[i] | (at[i] << 12);  // sub < 2^12, at < group size <= kSlabGroupLimit
+          rank[i] = kSetAside | q;
+          g1[i] = g0[i];  // nothing left to do for it below
+        }
       }
     }
   }
@@ -303,20 +316,22 @@ __device__ inline bool slab_rank(SlabSortShared &sh, const SlabGeom &geo, int ti
       }
     }
   }
-  if (set_aside) {
-    const uint32_t queued = (totals >> 16) < (uint32_t)kSlabQueueCap ? (totals >> 16) : (uint32_t)kSlabQueueCap;
-    // the thread that takes a queue entry also overwrites it with the rank
+  if constexpr (Shared::kQueue) {
+    if (set_aside) {
+      const uint32_t queued = (totals >> 16) < (uint32_t)kSlabQueueCap ? (totals >> 16) : (uint32_t)kSlabQueueCap;
+      // the thread that takes a queue entry also overwrites it with the rank
 #pragma unroll 1
-    for (uint32_t q = threadIdx.x; q < queued; q += BLOCK) {
-      const uint32_t e = sh.queue[q];
-      const uint32_t b0 = sh.cnt[sub_place<BLOCK>(e & 4095u)] & 0xffffu;
-      const uint32_t b1 = sh.cnt[sub_place<BLOCK>((e & 4095u) + 1)] & 0xffffu;
-      sh.queue[q] = b0 + slab_count_less(sh, b0, b1, sh.key[b0 + (e >> 12)]);
-    }
-    __syncthreads();
+      for (uint32_t q = threadIdx.x; q < queued; q += BLOCK) {
+        const uint32_t e = sh.queue[q];
+        const uint32_t b0 = sh.cnt[sub_place<BLOCK>(e & 4095u)] & 0xffffu;
+        const uint32_t b1 = sh.cnt[sub_place<BLOCK>((e & 4095u) + 1)] & 0xffffu;
+        sh.queue[q] = b0 + slab_count_less(sh, b0, b1, sh.key[b0 + (e >> 12)]);
+      }
+      __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kItems; ++i)
-      if (rank[i] & kSetAside) rank[i] = sh.queue[rank[i] & ~kSetAside];
+      for (int i = 0; i < kItems; ++i)
+        if (rank[i] & kSetAside) rank[i] = sh.queue[rank[i] & ~kSetAside];
+    }
   }
   *n_out = totals & 0xffffu;
   __syncthreads();

@@ -9,9 +9,10 @@
 //   k_fine_scatter  the coarse slabs, filtered by the exact threshold, go to the
 //                   bucket slabs, so that every store belongs to a long run;
 //   k_slab_sort     one workgroup per bucket: puts the bucket in the order of its
-//                   level-1 slots by a bitmap of them in LDS; of the entries that
-//                   share a slot the one with the smallest index is its level-1
-//                   owner, the others lost level 1 and are logged;
+//                   level-1 slots by a bitmap of them in LDS (wide buckets: by
+//                   comparing entries); of the entries that share a slot the one
+//                   with the smallest index is its level-1 owner, the others lost
+//                   level 1 and are logged;
 //   k_slab_chains   levels 2 and 3 for the losers through a small hash map,
 //                   with the reference's rule executed in ascending index order
 //                   (a slot belongs to the smallest index that ever probes it;
@@ -35,8 +36,8 @@ namespace {
 struct SlabTables {
   uint32_t *cursor;     // [B * kCursorPad] records in the bucket's slab, at [b * kCursorPad]
   uint32_t *bucket_lo;  // [B] smallest level-1 slot of the bucket
-  uint32_t *bucket_n;   // [B] level-1 owners, sorted, in the slab
-  uint32_t *removed_n;  // [B] of which were pushed out of their slot
+  uint32_t *bucket_n;   // [B] sorted records in the slab: level-1 owners, in wide buckets the losers too
+  uint32_t *removed_n;  // [B] of which have lost their slot
   uint32_t *movein_n;   // [B * kMoveinPad] occupied cells of the bucket's part of the map
   uint32_t *serial_n;   // [P * kMoveinPad] entries that found no slot
   uint32_t *raw_idx;    // [B * kSlabCap] entries as they arrive: index ...
@@ -103,10 +104,17 @@ struct EncodeSink {
 
 // ------------------------------------------------------------ sort a bucket
 
-// Keys of a bucket: the three widths the per-bucket kernels come in.  Their bitmaps decide how much LDS a workgroup
-// takes: up to the second width two workgroups share a compute unit, and the number of buckets is raised to stay
-// within it (slab_geometry) until there are kSlabMaxBuckets of them.
-constexpr uint32_t kSlabSpan1 = 1u << 17, kSlabSpan2 = 5u << 16, kSlabSpan3 = 9u << 16;
+// Two ways to put a bucket in order.  By a bitmap of its slots (k_slab_sort, k_slab_place) the work goes with the slots:
+// these kernels come in two widths, with which two workgroups share a compute unit.  By comparing records
+// (k_slab_sort_wide, k_slab_place_wide) it goes with the records, whatever the width.  A bucket within the second width
+// takes the bitmap.  Where the buckets the records call for are wider, more of them are made for the bitmap's sake up
+// to kSlabSparse slots per record of the capacity.  bf16, sort + place + chains, bitmap and comparisons: 2^30 slots,
+// 10.7 M records 127 and 170 us, 7.5 M 111 and 113, 6.4 M 102 and 99, 5.4 M 100 and 82; 1 M on 1024 partitions 97 and
+// 44.  No number of buckets makes the widest tables fit (more than 1.34 G slots): a bitmap of nine 2^16 slots, one
+// workgroup to a compute unit, takes 216 us for 1.34 G slots and 6.7 M records, comparisons 106; 2.1 G slots and 4.3 M
+// records 216 and 75.
+constexpr uint32_t kSlabSpan1 = 1u << 17, kSlabSpan2 = 5u << 16;
+constexpr int64_t kSlabSparse = 128;
 
 constexpr int kSortBlock = 1024;
 constexpr int kSortItems = kSlabCap / kSortBlock;
@@ -129,8 +137,7 @@ struct SlabSortLds {
 // the 12 to 16 bytes a record moves: 62 M slots, 6.2 M bf16 records 48 us, 3.1 M 24.  (Grouped by narrow key ranges and ranked by comparing the words of a group, with
 // the owners found by walking the sorted runs: 64 and 33.)
 template <typename S, uint32_t SPAN>
-__global__ __launch_bounds__(kSortBlock, SPAN <= kSlabSpan2 ? 8 : 4) void k_slab_sort(SlabGeom geo, SlabTables tb,
-                                                                                  int32_t *status) {
+__global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabTables tb, int32_t *status) {
   __shared__ SlabSortLds<S, SPAN> sh;
   const uint32_t b = blockIdx.x;
   const size_t base = (size_t)b * kSlabCap;
@@ -234,6 +241,140 @@ __global__ __launch_bounds__(kSortBlock, SPAN <= kSlabSpan2 ? 8 : 4) void k_slab
         atomicOr(status, ZEN_STAT_RETRY);
       ++at;
     }
+  }
+}
+
+// The same for few records among many slots: grouped by narrow key ranges, ranked against the words of their group
+// (slab_rank), the owners found by walking the sorted runs.  Those that lost stay where they are, marked.  Bound by LDS
+// round trips: 1.48 G slots, 14.8 M bf16 records 107 us; 1.34 G and 6.7 M 54.
+template <typename S>
+__global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort_wide(SlabGeom geo, SlabTables tb, int32_t *status) {
+  // the ties take the place of the counters once the ranks are known: with 32-bit values the kernel would
+  // otherwise need 88 KB of LDS, one workgroup to a compute unit instead of two
+  __shared__ SlabSortSharedNoQueue sh;
+  __shared__ S s_val[kSlabCap];
+  __shared__ uint32_t s_lost, s_base;
+  const uint32_t b = blockIdx.x;
+  const size_t base = (size_t)b * kSlabCap;
+  uint32_t n_raw = tb.cursor[b * kCursorPad];
+  if (n_raw > (uint32_t)kSlabCap) n_raw = kSlabCap;  // the scatter flagged the overflow
+  const uint32_t lo = tb.bucket_lo[b];
+  S *slab_val = static_cast<S *>(tb.slab_val);
+  if (threadIdx.x == 0) s_lost = 0;
+  // the kernels before this one were the last to need these: back to zero, a slice per workgroup
+  for (uint32_t i = b * kSortBlock + threadIdx.x; i < kCoarseCursorWords; i += gridDim.x * kSortBlock)
+    tb.coarse_cursor[i] = 0;
+  if (tb.refine_hist)
+    for (uint32_t i = b * kSortBlock + threadIdx.x; i <= (uint32_t)kRefineBins; i += gridDim.x * kSortBlock)
+      tb.refine_hist[i] = 0;
+  uint32_t off[kSortItems], idx[kSortItems], pos[kSortItems], rank[kSortItems];
+  S val[kSortItems];
+  uint32_t live = 0;
+#pragma unroll
+  for (int i = 0; i < kSortItems; ++i) {
+    const uint32_t j = threadIdx.x + i * kSortBlock;
+    // no branch around the loads (places past the end are pulled back onto the slab's first record): they are
+    // all in flight together
+    const size_t from = base + (j < n_raw ? j : 0u);
+    idx[i] = tb.raw_idx[from];
+    val[i] = static_cast<const S *>(tb.raw_val)[from];
+    off[i] = pos[i] = 0;
+    if (j < n_raw) {
+      off[i] = geo.mod_m(poly(idx[i]) + kSeed1) - lo;  // the level-1 slot again: cheaper than carrying it along
+      pos[i] = j;
+      live |= 1u << i;
+    }
+  }
+  // ties between equal slots are broken by the record's place in the slab (13 bits, so a record is one word
+  // while it is ranked); the runs of equal slots, few and short, are put right afterwards
+  static_assert(kSlabCap <= (1 << 13), "slab places in 13 bits");
+  uint32_t n = 0;
+  if (!slab_rank<kSortBlock>(sh, geo, 13, off, pos, live, rank, &n)) {
+    if (threadIdx.x == 0) {
+      tb.cursor[b * kCursorPad] = 0;
+      atomicOr(status, ZEN_STAT_RETRY);
+      tb.bucket_n[b] = 0;
+      tb.removed_n[b] = 0;
+    }
+    for (int j = threadIdx.x; j < kSlabIndexLen; j += kSortBlock) tb.sub_index[(size_t)b * kSlabIndexLen + j] = 0;
+    return;
+  }
+  // every thread has read the slab's fill count (slab_rank synchronised); this workgroup was its only reader
+  if (threadIdx.x == 0) tb.cursor[b * kCursorPad] = 0;
+  // the counters hold where every narrow range starts in the sorted bucket: every kSlabIndexStep-th goes to
+  // the index (before the counters' memory is used for the ties below)
+  for (int j = threadIdx.x; j < kSlabIndexLen; j += kSortBlock)
+    tb.sub_index[(size_t)b * kSlabIndexLen + j] = (uint16_t)sh.cnt[sub_place<kSortBlock>((uint32_t)j * kSlabIndexStep)];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kSortItems; ++i) {
+    if (live & (1u << i)) {
+      sh.key[rank[i]] = off[i];
+      sh.tie[rank[i]] = idx[i];
+      s_val[rank[i]] = val[i];
+    }
+  }
+  __syncthreads();
+  // a run of equal slots gets its smallest index in front (the thread at the run's first place does it)
+  for (uint32_t p = threadIdx.x; p + 1 < n; p += kSortBlock) {
+    const uint32_t k = sh.key[p];
+    if (sh.key[p + 1] == k && (p == 0 || sh.key[p - 1] != k)) {
+      uint32_t best = p;
+      for (uint32_t u = p + 1; u < n && sh.key[u] == k; ++u)
+        if (sh.tie[u] < sh.tie[best]) best = u;
+      if (best != p) {
+        const uint32_t ti = sh.tie[p];
+        const S tv = s_val[p];
+        sh.tie[p] = sh.tie[best];
+        s_val[p] = s_val[best];
+        sh.tie[best] = ti;
+        s_val[best] = tv;
+      }
+    }
+  }
+  __syncthreads();
+  // In a run of equal slots the first entry has the smallest index: the slot's level-1 owner.  The others
+  // lost level 1.  Their places in the sorted slab are collected where the slots were, once every thread has
+  // looked at those (a bucket has at most kSlabSubs of them, else the call is declined).
+  uint32_t lost_mask = 0;
+#pragma unroll 1
+  for (int i = 0; i < kSortItems; ++i) {
+    const uint32_t p = threadIdx.x + (uint32_t)i * kSortBlock;
+    if (p < n) {
+      const uint32_t k = sh.key[p];
+      const bool lost = p > 0 && sh.key[p - 1] == k;
+      tb.slab_idx[base + p] = (int32_t)(sh.tie[p] | (lost ? kRemovedBit : 0u));
+      slab_val[base + p] = s_val[p];  // every thread has read its records: in place is safe
+      lost_mask |= lost ? 1u << i : 0u;
+    }
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int i = 0; i < kSortItems; ++i) {
+    if (lost_mask & (1u << i)) {
+      const uint32_t at = atomicAdd(&s_lost, 1u);
+      if (at < (uint32_t)kSlabSubs) sh.key[at] = threadIdx.x + (uint32_t)i * kSortBlock;
+    }
+  }
+  __syncthreads();
+  uint32_t lost_n = s_lost;
+  if (lost_n > (uint32_t)kSlabSubs) {
+    if (threadIdx.x == 0) atomicOr(status, ZEN_STAT_RETRY);
+    lost_n = kSlabSubs;
+  }
+  if (threadIdx.x == 0) {
+    tb.bucket_n[b] = n;
+    tb.removed_n[b] = lost_n;
+    s_base = lost_n ? atomicAdd(tb.losers, lost_n) : 0u;
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < lost_n; i += kSortBlock) {
+    const uint32_t at = s_base + i;
+    const uint32_t p = sh.key[i];
+    if (at < tb.log_cap)
+      tb.log_t[at] = sh.tie[p];
+    else
+      atomicOr(status, ZEN_STAT_RETRY);
   }
 }
 
@@ -452,7 +593,7 @@ struct SlabPlaceLds {
 };
 
 template <typename S, uint32_t SPAN>
-__global__ __launch_bounds__(kSlabBlock, SPAN <= kSlabSpan2 ? 6 : 2) void k_slab_place(SlabGeom geo, SlabTables tb, unsigned long long *cells,
+__global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, SlabTables tb, unsigned long long *cells,
                                                            const S *__restrict__ dense, int32_t *__restrict__ out_idx,
                                                            S *__restrict__ out_val, uint32_t capacity) {
   constexpr int kCells = (1 << kSlabPartLog2) / kSlabBlock;
@@ -554,6 +695,188 @@ __global__ __launch_bounds__(kSlabBlock, SPAN <= kSlabSpan2 ? 6 : 2) void k_slab
   }
 }
 
+// The same for buckets that k_slab_sort_wide has sorted.  A sorted slab is almost the bucket's part of the output
+// already: the entries that lost their slot drop out and the entries that moved in from elsewhere slip in between.  So
+// an entry at sorted place p goes to
+//     bucket start + p - (removed entries before p) + (moved-in entries in front of it).
+// A wave's 64 consecutive places are one stretch: how many of its entries in front of a lane's are removed is a
+// ballot, how many moved-in ones slip in there a prefix sum across the lanes, and the stretches' sums are chained
+// once per bucket.  Consecutive lanes read consecutive entries and write (almost) consecutive places.  (Both counts
+// as bisections of sorted lists: 100 us for 6.2 M entries of which 5 % had moved, this 63.)  1.48 G slots, 14.8 M bf16
+// records 61 us; 1.34 G and 6.7 M 32.
+template <typename S>
+__global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place_wide(SlabGeom geo, SlabTables tb,
+                                                                unsigned long long *cells,
+                                                                const S *__restrict__ dense,
+                                                                int32_t *__restrict__ out_idx,
+                                                                S *__restrict__ out_val, uint32_t capacity) {
+  constexpr int kStretches = kSlabCap / 64;
+  constexpr int kCells = (1 << kSlabPartLog2) / kSlabBlock;
+  static_assert(kStretches <= 128, "two stretches per lane of a wave");
+  __shared__ uint32_t s_key[kSlabCap];                 // sorted slots of the bucket
+  __shared__ uint32_t s_cnt[kSlabCap / 2 + 1];         // per sorted place, 16 bits each: the moved-in entries right in
+  uint16_t *s_front = reinterpret_cast<uint16_t *>(s_cnt);  // front of it, then those before it in its stretch
+  __shared__ uint32_t s_mk[1 << kSlabPartLog2];        // the moved-in entries' slots, by the place they slip in at
+  __shared__ uint64_t s_mask[kStretches];              // per stretch: its removed entries
+  __shared__ uint32_t s_mv[kStretches], s_rm[kStretches];  // moved-in and removed entries of the stretches before
+  __shared__ uint32_t s_nrm;
+  const uint32_t b = blockIdx.x;
+  const uint32_t B = geo.nbuckets;
+  const size_t base = (size_t)b * kSlabCap;
+  const S *slab_val = static_cast<const S *>(tb.slab_val);
+  const uint32_t *serial_n = tb.final_n + B;
+  const uint32_t n = tb.bucket_n[b];
+  // what the bucket's part of the map holds has moved in, and keeps to the thread that finds it; the part goes
+  // back empty
+  const uint32_t mv_n = tb.final_n[b];
+  const uint32_t out_base = tb.out_start[b];
+  const uint32_t out_n = tb.out_start[b + 1] - out_base;
+  unsigned long long *cell = cells + ((size_t)b << kSlabPartLog2) + threadIdx.x;
+  unsigned long long moved[kCells];
+#pragma unroll
+  for (int e = 0; e < kCells; ++e) moved[e] = mv_n ? cell[e * kSlabBlock] : 0ull;
+  // the thread's entries (sorted places threadIdx.x + i * kSlabBlock) stay in registers; the slots go to LDS
+  // for the searches
+  uint32_t idx[kSlabItems];
+  S val[kSlabItems];
+#pragma unroll
+  for (int i = 0; i < kSlabItems; ++i) {
+    const uint32_t p = threadIdx.x + i * kSlabBlock;
+    idx[i] = (uint32_t)tb.slab_idx[base + (p < n ? p : 0u)];
+    val[i] = slab_val[base + (p < n ? p : 0u)];
+  }
+  S mval[kCells];  // an entry is a copy of the element it stands for
+#pragma unroll
+  for (int e = 0; e < kCells; ++e) mval[e] = mv_n ? dense[(uint32_t)moved[e]] : S(0);
+  if (threadIdx.x == 0) s_nrm = 0;
+  for (int i = threadIdx.x; i < kSlabCap / 2 + 1; i += kSlabBlock) s_cnt[i] = 0;
+#pragma unroll
+  for (int i = 0; i < kSlabItems; ++i) {
+    const uint32_t p = threadIdx.x + i * kSlabBlock;
+    if (p < n) s_key[p] = geo.mod_m(poly(idx[i] & kIndexMask) + kSeed1);
+  }
+  __syncthreads();
+  // a moved-in entry's place: the sorted place in front of which it slips in, and its turn among those that slip
+  // in there too
+  uint32_t mplace[kCells], mturn[kCells];
+#pragma unroll
+  for (int e = 0; e < kCells; ++e) {
+    mplace[e] = mturn[e] = 0;
+    if (moved[e]) {
+      cell[e * kSlabBlock] = 0ull;
+      mplace[e] = lower_bound_u32(s_key, n, (uint32_t)(moved[e] >> 32) - 1u);
+      const uint32_t shift = 16u * (mplace[e] & 1u);
+      mturn[e] = (atomicAdd(&s_cnt[mplace[e] >> 1], 1u << shift) >> shift) & 0xffffu;
+    }
+  }
+  __syncthreads();
+  uint32_t in_front[kSlabItems];  // moved-in entries of the stretch that slip in at or before the entry's place
+  uint32_t removed = 0;           // bit i: entry i has lost its slot
+#pragma unroll
+  for (int i = 0; i < kSlabItems; ++i) {
+    const uint32_t p = threadIdx.x + i * kSlabBlock;
+    in_front[i] = 0;
+    if ((uint32_t)(i * kSlabBlock) > n) {  // the same for the whole workgroup: nothing beyond the entries
+      if (lane_id() == 63) s_mv[p >> 6] = s_rm[p >> 6] = 0;
+      continue;
+    }
+    const bool gone = p < n && (idx[i] & kRemovedBit);
+    const uint64_t m = __ballot(gone);
+    removed |= (gone ? 1u : 0u) << i;
+    if (mv_n) {
+      const uint32_t c = s_front[p];
+      in_front[i] = wave_inclusive_scan(c);
+      s_front[p] = (uint16_t)(in_front[i] - c);
+    }
+    if (lane_id() == 63) {
+      s_mask[p >> 6] = m;
+      s_mv[p >> 6] = in_front[i];
+      s_rm[p >> 6] = (uint32_t)__popcll(m);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const int l = threadIdx.x;
+    const uint32_t v0 = s_mv[l], v1 = l + 64 < kStretches ? s_mv[l + 64] : 0u;
+    const uint32_t r0 = s_rm[l], r1 = l + 64 < kStretches ? s_rm[l + 64] : 0u;
+    const uint32_t iv0 = wave_inclusive_scan(v0), iv1 = wave_inclusive_scan(v1);
+    const uint32_t ir0 = wave_inclusive_scan(r0), ir1 = wave_inclusive_scan(r1);
+    const uint32_t tv = __shfl(iv0, 63, 64), tr = __shfl(ir0, 63, 64);
+    s_mv[l] = iv0 - v0;
+    s_rm[l] = ir0 - r0;
+    if (l + 64 < kStretches) {
+      s_mv[l + 64] = tv + iv1 - v1;
+      s_rm[l + 64] = tr + ir1 - r1;
+    }
+    if (l == 63) s_nrm = tr + ir1;
+  }
+  __syncthreads();
+  // survivors
+#pragma unroll
+  for (int i = 0; i < kSlabItems; ++i) {
+    const uint32_t p = threadIdx.x + i * kSlabBlock;
+    if ((uint32_t)(i * kSlabBlock) >= n) break;
+    const uint64_t m = __ballot((removed >> i) & 1u);
+    if (p < n && !((removed >> i) & 1u)) {
+      const uint32_t before = (uint32_t)__popcll(m & lanes_below());
+      const uint32_t pos = out_base + p + s_mv[p >> 6] + in_front[i] - s_rm[p >> 6] - before;
+      if (pos < capacity) {
+        out_idx[pos] = (int32_t)idx[i];
+        out_val[pos] = val[i];
+      }
+    }
+  }
+  if (mv_n) {  // the same for the whole workgroup
+    // the moved-in entries by the place they slip in at; several at one place (two at times) by ascending slot
+    const auto front = [&](uint32_t p) -> uint32_t {  // moved-in entries before those of place p
+      return p < (uint32_t)kSlabCap ? s_mv[p >> 6] + s_front[p] : p > (uint32_t)kSlabCap ? mv_n : mv_n - s_front[kSlabCap];
+    };
+#pragma unroll
+    for (int e = 0; e < kCells; ++e)
+      if (moved[e]) s_mk[front(mplace[e]) + mturn[e]] = (uint32_t)(moved[e] >> 32) - 1u;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kCells; ++e) {
+      if (moved[e]) {
+        const uint32_t at = mplace[e], key = (uint32_t)(moved[e] >> 32) - 1u;
+        const uint32_t first = front(at), end = front(at + 1u);
+        uint32_t rank = first;
+        for (uint32_t u = first; u < end; ++u) rank += s_mk[u] < key;
+        const uint32_t gone =
+            at < n ? s_rm[at >> 6] + (uint32_t)__popcll(s_mask[at >> 6] & ((1ull << (at & 63u)) - 1ull)) : s_nrm;
+        const uint32_t pos = out_base + at + rank - gone;
+        if (pos < capacity) {
+          out_idx[pos] = (int32_t)(uint32_t)moved[e];
+          out_val[pos] = mval[e];
+        }
+      }
+    }
+  }
+  const uint32_t part = b / geo.bpp;
+  const bool last_of_part = b % geo.bpp == geo.bpp - 1;
+  uint32_t serial = 0;
+  if (last_of_part) {
+    serial = serial_n[part];
+    if (serial > (uint32_t)kSlabSerialCap) serial = kSlabSerialCap;
+  }
+  const uint32_t own_n = out_n - serial;  // survivors + moved-in
+  if (serial) {
+    // the partition's overflow entries in ascending index order (the reference hands its tickets to
+    // ascending thread ids, functions_cuda_kernel.cu:107-108), behind everything that found a slot
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < serial; i += kSlabBlock) s_key[i] = tb.ser_idx[(size_t)part * kSlabSerialCap + i];
+    __syncthreads();
+    sort_network(s_key, serial);
+    for (uint32_t i = threadIdx.x; i < serial; i += kSlabBlock) {
+      const uint32_t pos = out_base + own_n + i;
+      if (pos < capacity) {
+        out_idx[pos] = (int32_t)s_key[i];
+        out_val[pos] = dense[s_key[i]];
+      }
+    }
+  }
+}
+
 struct SlabPlan {
   SlabTables tb;
   uint32_t *sample_hist[2];  // sampled floor histogram (+ finished-block count); two sets, so that the sample of
@@ -614,6 +937,7 @@ SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partit
   return p;
 }
 
+// SPAN: keys a bucket's bitmap holds; 0: the kernels that compare.
 template <typename S, uint32_t SPAN>
 int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPlan &p, hipStream_t s) {
   const uint32_t B = geo.nbuckets;
@@ -629,7 +953,10 @@ int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPl
   }
   {
     ProfScope prof(kProfSlabSort, s);
-    k_slab_sort<S, SPAN><<<dim3(B), dim3(kSortBlock), 0, s>>>(geo, p.tb, a.status);
+    if constexpr (SPAN > 0)
+      k_slab_sort<S, SPAN><<<dim3(B), dim3(kSortBlock), 0, s>>>(geo, p.tb, a.status);
+    else
+      k_slab_sort_wide<S><<<dim3(B), dim3(kSortBlock), 0, s>>>(geo, p.tb, a.status);
     ZEN_LAUNCH_CHECK("k_slab_sort");
   }
   {
@@ -643,8 +970,12 @@ int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPl
   }
   {
     ProfScope prof(kProfSlabPlace, s);
-    k_slab_place<S, SPAN><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, dense, a.out_idx,
-                                                               static_cast<S *>(a.out_val), (uint32_t)a.capacity);
+    if constexpr (SPAN > 0)
+      k_slab_place<S, SPAN><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, dense, a.out_idx,
+                                                                 static_cast<S *>(a.out_val), (uint32_t)a.capacity);
+    else
+      k_slab_place_wide<S><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, dense, a.out_idx,
+                                                                static_cast<S *>(a.out_val), (uint32_t)a.capacity);
     ZEN_LAUNCH_CHECK("k_slab_place");
   }
   return ZEN_OK;
@@ -654,12 +985,19 @@ template <typename S>
 int slab_launch(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPlan &p, hipStream_t s) {
   if (geo.span <= kSlabSpan1) return slab_launch_span<S, kSlabSpan1>(a, geo, p, s);
   if (geo.span <= kSlabSpan2) return slab_launch_span<S, kSlabSpan2>(a, geo, p, s);
-  return slab_launch_span<S, kSlabSpan3>(a, geo, p, s);
+  return slab_launch_span<S, 0>(a, geo, p, s);
 }
 
+// The buckets the records call for; where those are too wide for a bitmap, more of them if the records are dense enough
+// and that makes them fit.
 bool encode_geometry(int64_t m, int partitions, int64_t capacity, SlabGeom *geo) {
+  if (!slab_geometry(m, partitions, capacity, kSlabTarget, 0, geo)) return false;
+  SlabGeom more;
   // (a few thousand keys below the width: the divisions round the buckets up)
-  return slab_geometry(m, partitions, capacity, kSlabTarget, (int64_t)kSlabSpan2 - 4096, kSlabSpan3, geo);
+  if (geo->span > kSlabSpan2 && m / kSlabSparse <= capacity &&
+      slab_geometry(m, partitions, capacity, kSlabTarget, (int64_t)kSlabSpan2 - 4096, &more) && more.span <= kSlabSpan2)
+    *geo = more;
+  return true;
 }
 
 }  // namespace
