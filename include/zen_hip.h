@@ -38,7 +38,21 @@
 extern "C" {
 #endif
 
-#define ZEN_ABI_VERSION 7 /* 2: zen_encode_merge (its argument struct), zen_sample_threshold, zen_round_compact, path code 3; 3: next_n .. next_table; 4: zen_read_back, zen_count, zen_merge_rounded, zen_decode_dense_lists, zen_bitmap_dense_lists; 5: zen_table_find, zen_table_gather; 6: ZEN_MODE_NO_SAMPLES; 7: zen_load_balance_sizes, zen_merge_rounded_count */
+/*
+ * 2: zen_encode_merge (its argument struct), zen_sample_threshold,
+ *    zen_round_compact, path code 3
+ * 3: next_n .. next_table
+ * 4: zen_read_back, zen_count, zen_merge_rounded, zen_decode_dense_lists,
+ *    zen_bitmap_dense_lists
+ * 5: zen_table_find, zen_table_gather
+ * 6: ZEN_MODE_NO_SAMPLES
+ * 7: zen_load_balance_sizes, zen_select_count, zen_merge_rounded_count,
+ *    zen_decode_dense_status, zen_table_find_sizes; the rank dictionary holds a
+ *    16-byte entry per 96 indices (zen_bitmap_rank_words), and the dense
+ *    dictionary is longer by a chunk of places (zen_bitmap_dense_dict_bytes):
+ *    both are built anew, not kept from an older library
+ */
+#define ZEN_ABI_VERSION 7
 
 #define ZEN_F32 0
 #define ZEN_BF16 1
@@ -596,8 +610,9 @@ size_t zen_table_lists_workspace(int64_t m, int partitions);
 int zen_table_find(const int32_t *table, int64_t m, int partitions, int64_t n, int64_t *splits, void *workspace,
                    size_t workspace_bytes, int32_t *status, void *stream);
 /*
- * zen_table_find, of at most ZEN_TABLE_SIZES_MOST partitions, that returns when the split sizes and then *status are in the host words [1, partitions + 2), `host`
- * and `words` from zen_host_words_alloc (at least partitions + 2).  marks: 2 * partitions + 66 zeroed device words.
+ * zen_table_find, of at most ZEN_TABLE_SIZES_MOST partitions, that returns when the split sizes and then *status are in
+ * the host words [1, partitions + 2), `host` and `words` from zen_host_words_alloc (at least partitions + 2).
+ * marks: 2 * partitions + 66 zeroed device words.
  */
 #define ZEN_TABLE_SIZES_MOST 1024
 int zen_table_find_sizes(const int32_t *table, int64_t m, int partitions, int64_t n, int64_t *splits, int64_t *marks,

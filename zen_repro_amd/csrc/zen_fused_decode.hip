@@ -162,7 +162,8 @@ inline uint32_t fd_groups(uint32_t tiles) { return (tiles + kFdGroup - 1) / kFdG
 // Per (group of tiles, list): set bits in each tile's bit range of the list's bitmap, summed up inside the
 // group.  A bitmap shorter than its list (the reference's mask would not fit the member list, comm.py:97-98)
 // raises ZEN_STAT_BAD_INDEX.
-constexpr int kFdCountAhead = 5;  // a tile's range of a list spans eight or nine words at sixteen ranks (268 M elements: 22 us with one, 16 with five)
+// A tile's range of a list spans eight or nine words at sixteen ranks (268 M elements: 22 us with one, 16 with five).
+constexpr int kFdCountAhead = 5;
 __global__ __launch_bounds__(kFdGroup) void k_fd_count(const uint32_t *__restrict__ below, uint32_t tiles, int P,
                                                        FdLists lists, uint32_t *__restrict__ vstart,
                                                        uint32_t *__restrict__ gsum, int32_t *status) {
@@ -194,7 +195,11 @@ __global__ __launch_bounds__(kFdGroupsMax) void k_fd_groups(uint32_t *__restrict
   if (threadIdx.x < groups) *at = before;
 }
 
-constexpr int kFdWords = 9;                  // words of a chunk: sixteen lists have 512 members in a tile, few more than 576
+// Words of a chunk: sixteen lists have 512 members in a tile, few more than 576.  Tile kernel with 8, 9 and 10 words, us,
+// 134 M bf16: 2 lists 171, 161 and 158, 3 185, 152 and 155, 4 176, 163 and 166, 8 184, 160 and 163, 16 190, 123 and 127,
+// 24 156, 159 and 166, 32 190, 193 and 202, 64 318, 324 and 340; 67 M fp32: 2 112, 109 and 108, 4 124, 112 and 114, 16
+// 132, 100 and 101, 64 195, 203 and 212.
+constexpr int kFdWords = 9;
 constexpr int kFdMembers = 64 * kFdWords;    // members of a chunk
 
 template <typename S>

@@ -134,8 +134,8 @@ struct SlabSortLds {
 // logged and not kept.  A bucket has a few to a few hundred slots per record, so the slots are marked in a bitmap: a
 // record's place is the number of marks below its own, and whoever finds its slot marked already is settled by the
 // smallest index afterwards.  Bound by the LDS round trips (six records a thread, two workgroups a compute unit) and by
-// the 12 to 16 bytes a record moves: 62 M slots, 6.2 M bf16 records 48 us, 3.1 M 24.  (Grouped by narrow key ranges and ranked by comparing the words of a group, with
-// the owners found by walking the sorted runs: 64 and 33.)
+// the 12 to 16 bytes a record moves: 62 M slots, 6.2 M bf16 records 48 us, 3.1 M 24.  (By comparisons, k_slab_sort_wide:
+// 64 and 33.)
 template <typename S, uint32_t SPAN>
 __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabTables tb, int32_t *status) {
   __shared__ SlabSortLds<S, SPAN> sh;
@@ -492,7 +492,9 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
   if (answer.host) {
     wait_global_acks();
     __syncthreads();
-    if (threadIdx.x == 0) host_store(answer.host + 1 + tb.partitions, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (threadIdx.x == 0)
+      host_store(answer.host + 1 + tb.partitions,
+                 (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     host_answered(answer);
   }
 }
@@ -501,8 +503,9 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
 // wave 15 us; a probe is four or five dependent trips to memory, the bucket's index, its records, the map) and by the
 // device-wide atomics, two or three a loser at 21 a nanosecond, when they are many (436 000: a wave 50 us).  Every loser
 // has a thread of its own on a full chip: with the scalar registers the compiler takes by itself three workgroups fit a
-// compute unit, and the last of 851 began when the first had ended (93 us, with four 83).  Nothing is counted in one place (62 M slots, 10 % taken, 300 000 losers: with one counter of the
-// map's claims and one log of the owners pushed out, whose entries another kernel classified afterwards, 338 + 220 us).
+// compute unit, and the last of 851 began when the first had ended (93 us, with four 83).  Nothing is counted in one
+// place (62 M slots, 10 % taken, 300 000 losers: with one counter of the map's claims and one log of the owners pushed
+// out, whose entries another kernel classified afterwards, 338 + 220 us).
 __global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Probe g, SlabTables tb, unsigned long long *cells,
                                                             int64_t spp, uint32_t capacity, int64_t *__restrict__ splits,
                                                             HostAnswer answer, int32_t *status) {
@@ -580,9 +583,8 @@ __global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Pro
 
 // A bucket's part of the output is its taken slots in order: the owners that nobody pushed out and the entries that moved
 // in.  Both are marked in a bitmap of the slots, and an entry goes to the bucket's start plus the number of marks below
-// its own.  Consecutive lanes read consecutive entries and write (almost) consecutive places.  (Removed and moved-in
-// entries counted per stretch of 64 sorted places, with a bisection for every moved-in one: 62 M slots, 6.2 M records, 5 %
-// moved: 63 us, now 48; both counts as bisections of sorted lists: 100.)
+// its own.  Consecutive lanes read consecutive entries and write (almost) consecutive places.  62 M slots, 6.2 M records,
+// 5 % moved: 48 us (k_slab_place_wide, which counts removed and moved-in entries: 63).
 template <uint32_t SPAN>
 struct SlabPlaceLds {
   union {

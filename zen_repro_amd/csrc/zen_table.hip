@@ -352,7 +352,8 @@ __global__ __launch_bounds__(kOneBlock) void k_table_one(const S *__restrict__ i
   if (answer.host) {
     wait_global_acks();
     __syncthreads();
-    if (threadIdx.x == 0) host_store(answer.host + 1 + parts, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (threadIdx.x == 0)
+      host_store(answer.host + 1 + parts, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     host_answered(answer);
   }
 }
