@@ -824,9 +824,10 @@ __device__ inline void stage_flush(uint32_t count, int32_t *st_idx, S *st_val, S
 // `fixed` tiles of kStageBig sub-tiles, tile i of workgroup b being number i * workgroups + b: no counter, and
 // the workgroups move through memory side by side (short tiles measured a little faster than long ones).
 // The rest of the tensor goes out in short tiles through ticket counters, so that workgroups that ran ahead take more
-// and all finish within one short tile of each other.  A device-wide counter serves about 90 tickets per microsecond, and 768 workgroups asking one
-// counter every few microseconds would queue up for it: the workgroups form kStageGroups groups (by number
-// modulo kStageGroups) with a counter each, and ticket t of group g is short tile number g + t * kStageGroups.
+// and all finish within one short tile of each other.  A device-wide counter serves about 90 tickets per microsecond,
+// and 768 workgroups asking one counter every few microseconds would queue up for it: the workgroups form kStageGroups
+// groups (by number modulo kStageGroups) with a counter each, and ticket t of group g is short tile number
+// g + t * kStageGroups.
 // The `late` first workgroups, which take the next call's sample first, go without the first `skip` of those
 // tiles: what the others read in the meantime.
 constexpr int kStageBig = 2;    // both tile lengths must be at least 2: the loads run two sub-tiles ahead
@@ -1262,11 +1263,13 @@ static int stage_launch(const StageArgs &a, hipStream_t stream) {
   int64_t blocks = (int64_t)device_cus() * ZEN_STAGE_WGS;
   const int64_t least = ceil_div(subs, kStageSmall);
   if (blocks > least) blocks = least;
-  // seven eighths of the tensor in counter-free tiles, the rest through tickets (measured on 1.5 GB: all
-  // tickets 280 us, two thirds fixed 252, seven eighths 247, everything fixed 258).  Half of it where a workgroup has few
-  // sub-tiles: one that a merge on another stream kept off its compute unit, or that took the next call's sample, is a
-  // larger part of the pass late then (twelve buckets of 62 M bf16 elements, ten sub-tiles each: 936 -> 920 us a pass,
-  // all tickets 933; 268 M, 42 each: 733 -> 738; 2^30 fp32, 341 each: 1105 -> 1155).
+  // Seven eighths of the tensor in counter-free tiles, the rest through tickets (measured on 1.5 GB: all tickets 280 us,
+  // two thirds fixed 252, seven eighths 247, everything fixed 258).  Half of it where a workgroup has few sub-tiles: one
+  // that a merge on another stream kept off its compute unit, or that took the next call's sample, is a larger part of
+  // the pass late then.  Four tensors in a row with their tails and merges, seven eighths and half, us: bf16, 13
+  // sub-tiles a workgroup 353 and 348, 16 381 and 376, 20 433 and 423, 25 484 and 486, 32 573 and 573, 43 663 and 676;
+  // fp32, 13 393 and 391, 16 418 and 416, 20 456 and 459, 25 516 and 523, 43 684 and 705; twelve bf16 tensors, ten each:
+  // 931 and 918 (all tickets 933).  A call by itself loses up to 2 % by it (ten each: 78.0 and 79.0).
   StageSched sch;
   const int64_t fixed_subs = subs < kStageFew * blocks ? subs / 2 : subs * 7 / 8;
   sch.fixed = (uint32_t)(fixed_subs / ((int64_t)kStageBig * blocks));
