@@ -143,6 +143,9 @@ class TensorPartition:
         few different sizes come round again and again (the hook is called per
         bucket, train.py:167-185), so a handful of tables is kept, least
         recently used first out."""
+        return self._kept_table(device, m, slot).buf
+
+    def _kept_table(self, device, m, slot):
         key = (device if isinstance(device, torch.device) else torch.device(device), m, slot)
         kept = self._tables.pop(key, None)
         if kept is None:
@@ -152,7 +155,7 @@ class TensorPartition:
         self._tables[key] = kept  # most recently used last
         if _lib.stream_handle(device) not in kept.seen:
             kept.join(torch.cuda.current_stream(device))
-        return kept.buf
+        return kept
 
     def _honest_capacity(self, flat, thr, k):
         """Room for the selection without guessing `numel` (which would take a
@@ -392,8 +395,8 @@ class TensorPartition:
         status = _lib.status_word(dev)
         nbytes = L.zen_load_balance_workspace(n, m, code, capacity, self.partitions)
         ws = _lib.scratch.get(dev, f"load_balance/{slot}", nbytes)
-        table = self._table(dev, m, slot)
-        kept = self._tables[dev, m, slot]
+        kept = self._kept_table(dev, m, slot)
+        table = kept.buf
         flags, used = self._take_ahead(flat, n, int(k), capacity, ws, slot, mode, thr, near)
         if near is not None and k > 0 and thr is None:
             thr, flags = near, flags | _lib.MODE_FLOOR
@@ -410,7 +413,8 @@ class TensorPartition:
         if rc != _lib.OK:
             table.zero_()  # a call that failed half way may have left entries behind
         _lib.check(rc, "load_balance")
-        self._after_call(flat, int(k), capacity, slot, mode | flags, used)
+        if self._ahead:  # (else no sample was ever taken ahead, and there is nothing to book)
+            self._after_call(flat, int(k), capacity, slot, mode | flags, used)
         return out_idx, out_val, splits, status
 
     def load_balance(self, tensor, thr=None, capacity=None, k=0, mode=None, grow=None):
