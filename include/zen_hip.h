@@ -347,8 +347,9 @@ int zen_load_balance_prepare(const void *input, int dtype, int64_t n, int64_t m,
  * general mode), 1 = the same in three launches or one (tables below 2^20 slots, up to 4 Mi slots with k == 0 and
  * ZEN_MODE_NO_SAMPLES) or sort-based owner resolution, 2 = bucket slabs (large inputs whose expected output is a
  * small fraction of the table: one streaming pass, then per-bucket sorts inside LDS), 3 = wide buckets (the same
- * for an expected output of up to a few million entries: at most 256 buckets, one resident workgroup each,
- * two launches).  No counterpart in the reference; tests and benchmarks use it to know what they measured.
+ * for an expected output of up to a few million entries, few of them on a slot that is taken: at most 256 buckets,
+ * one resident workgroup each, two launches; zen_load_balance_sizes takes path 2 there where the sizes allow it).  No
+ * counterpart in the reference; tests and benchmarks use it to know what they measured.
  */
 int zen_load_balance_path(int64_t n, int64_t m, int dtype, int64_t capacity, int partitions, int64_t k, int mode);
 

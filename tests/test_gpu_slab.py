@@ -92,6 +92,27 @@ def test_slab_load_balance_bit_exact(zen, oracle, n, P, density, rehash, dtype):
     assert not tp._table(d.device, m).any()
 
 
+@pytest.mark.parametrize("n,P,density,rehash,room", [
+    ((1 << 22) - 6, 3, 0.05, 3, 1.1),   # just below the smallest table of the slabs: the owner table
+    ((1 << 22) + 5, 2, 0.1, 3, 1.1),    # just above it, a tenth of the slots taken
+    ((1 << 22) + 5, 16, 0.001, 3, 1.1),
+    ((1 << 22) + 5, 2, 0.3, 2, 1.1),    # too dense for the slabs' buckets
+    (6000000, 3, 0.1, 2, 0.5),          # room for half: declined, and taken again with more
+])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_call_that_waits_gives_the_same_on_every_path(zen, oracle, n, P, density, rehash, room, dtype):
+    """load_balance waits for its sizes, which takes it off the wide buckets where the slabs fit."""
+    g = make_grad(oracle, n, density, dtype, seed=n + P)
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, rehash)
+    assert st_o == 0
+    tp = zen.TensorPartition(P, 1, rehash)
+    indices, values, splits = tp.load_balance(to_dev(g), capacity=int(len(idx_o) * room) + 1024, grow=True)
+    assert np.array_equal(to_np(splits), splits_o)
+    assert [len(i) for i in indices] == list(splits_o)
+    assert np.array_equal(to_np(torch.cat(indices)), idx_o) and np.array_equal(to_np(torch.cat(values)), val_o)
+    assert not tp._table(torch.device("cuda"), oracle.table_sizes(n, P, 1)[0]).any()
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 def test_slab_load_balance_odd_length_unaligned_and_empty(zen, oracle, dtype):
     """A tensor whose length is no multiple of anything and whose first element is not 16-byte aligned (the

@@ -380,12 +380,38 @@ size_t zen_load_balance_workspace(int64_t n, int64_t m, int dtype, int64_t capac
   return general > fast ? general : fast;
 }
 
+}  // extern "C"
+
+namespace {
+
+// Whether a call takes the wide buckets where both they and the bucket slabs fit.  The resident kernel of the wide
+// buckets is one launch where the slabs need four, but every workgroup of a partition looks at all of the partition's
+// collisions; the slabs' chains share them out over the chip.  A call that waits for its sizes has the host idle: the
+// slabs are the quicker throughout (us a call with a given threshold, wide and slabs: 4.3 M bf16 elements on 2
+// partitions, 0.5 % selected 71 and 63, 10 % 173 and 90; 36 M, 0.5 % 86 and 81, 3 % 157 and 96, 10 % 714 and 166; on 16
+// partitions 92 and 87, 134 and 109, 433 and 166; fp32 the same).  Calls that do not wait follow each other as fast as
+// the host enqueues them, and the wide buckets are the quicker while collisions are few, up to about 8192 of them or one
+// slot in 64 taken (three steps of 16 M bf16 elements on 16 partitions with their merges, top 0.5 % 245 and 265, 2 % 252
+// and 270, 5 % 317 and 279; of 36 M, 2 % 274 and 278, 3 % 342 and 288, 5 % 525 and 368; one of 743 M, 0.5 % 414 and 496;
+// three of 20 M with 0.5 % in whole rows, no threshold, 192 and 215).
+bool takes_wide(int64_t n, int64_t m, int partitions, int dtype, int64_t capacity, int64_t k, bool waits) {
+  using namespace zen;
+  if (!wide_balance_fits(m, partitions, capacity, k, wide_device_cus(), nullptr)) return false;
+  const int64_t most = k > 0 ? k : capacity;
+  const bool few = most <= m / 64 || (double)most * (double)most <= 2.0 * 8192.0 * (double)m;
+  return (few && !waits) || !slab_balance_fits(n, m, partitions, dtype, capacity, k, nullptr);
+}
+
+}  // namespace
+
+extern "C" {
+
 int zen_load_balance_path(int64_t n, int64_t m, int dtype, int64_t capacity, int partitions, int64_t k, int mode) {
   const bool slabs_only = (mode & ZEN_MODE_SLABS) != 0, no_samples = (mode & ZEN_MODE_NO_SAMPLES) != 0;
   mode &= 0xff;
   if (mode != ZEN_MODE_FAST || partitions <= 0 || m <= 0 || m % partitions != 0) return 0;
   if (!slabs_only && zen::table_balance_fits(n, m, partitions, k, no_samples)) return 1;
-  if (!slabs_only && zen::wide_balance_fits(m, partitions, capacity, k, zen::wide_device_cus(), nullptr)) return 3;
+  if (!slabs_only && takes_wide(n, m, partitions, dtype, capacity, k, false)) return 3;
   if (zen::slab_balance_fits(n, m, partitions, dtype, capacity, k, nullptr)) return 2;
   return m >= 4096 ? 1 : 0;
 }
@@ -483,7 +509,7 @@ int load_balance_call(const void *input, int dtype, int64_t n, int64_t m, int pa
   const bool small = mode == ZEN_MODE_FAST && !slabs_only && (reinterpret_cast<uintptr_t>(table) & 15u) == 0 &&
                      table_balance_fits(n, m, partitions, k, no_samples);
   const bool wide = mode == ZEN_MODE_FAST && !slabs_only && (reinterpret_cast<uintptr_t>(table) & 7u) == 0 &&
-                    wide_balance_fits(m, partitions, capacity, k, wide_device_cus(), nullptr);
+                    takes_wide(n, m, partitions, dtype, capacity, k, ask.answer.host != nullptr);
   if (small || wide || (mode == ZEN_MODE_FAST && (reinterpret_cast<uintptr_t>(table) & 7u) == 0 &&
                slab_balance_fits(n, m, partitions, dtype, capacity, k, nullptr))) {
     SlabBalanceArgs sa;

@@ -450,6 +450,10 @@ class TensorPartition:
                 self._table(tensor.device, m).zero_()
             if bits & _lib.STAT_RETRY:
                 modes.pop(0)
+                if modes and modes[0] & _lib.MODE_SLABS and _lib.lib().zen_load_balance_path(
+                        n, self.table_sizes(n)[0], _lib.dtype_code(flat), capacity, self.partitions, int(k),
+                        modes[0]) == 2:
+                    modes.pop(0)  # a call that waits for its sizes was on the slabs already
             elif bits & _lib.STAT_CAPACITY and grow and capacity < n:
                 # more passed than allowed for (a fast path short of room declines, so this is mostly the general
                 # mode speaking): with more room the fast modes get their turn again
