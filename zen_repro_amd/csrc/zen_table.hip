@@ -158,6 +158,15 @@ __global__ __launch_bounds__(kOutBlock) void k_table_out(const S *__restrict__ d
   uint4 q[kOutRows];
 #pragma unroll
   for (int r = 0; r < kOutRows; ++r) q[r] = load_slots(tb.slots, base + r * 256, m);
+  // The stretch's partitions, p_first to p_last.  Where it has several, their entries are counted in LDS (an add to the
+  // split sizes for every entry of such a stretch: some 6000 of them queue on one line, 1.8 M fp32 slots, 5 % taken, 16
+  // partitions 27 us, now 8).
+  const uint32_t lo = c * kStretch, hi = lo + kStretch < m ? lo + kStretch : m;  // lo < m
+  const uint32_t p_first = lo / npp, p_last = (hi - 1u) / npp;
+  uint32_t *held = buf;
+  static_assert(kMaxParts <= (int)kSerialLds, "a counter for every partition");
+  if (p_first != p_last)
+    for (uint32_t i = threadIdx.x; i <= p_last - p_first; i += kOutBlock) held[i] = 0;
   // entries in front of the stretch, and serial entries in front of every partition
   uint32_t sum = 0, front;
   for (uint32_t i = threadIdx.x; i < c; i += kOutBlock) sum += tb.found[i];
@@ -184,9 +193,6 @@ __global__ __launch_bounds__(kOutBlock) void k_table_out(const S *__restrict__ d
     at += w < wave ? smem[w] : 0u;
     all += smem[w];
   }
-  // The partitions of the stretch: p_first's entries from its beginning on, ...
-  const uint32_t lo = c * kStretch, hi = lo + kStretch < m ? lo + kStretch : m;  // lo < m
-  const uint32_t p_first = lo / npp, p_last = (hi - 1u) / npp;
 #pragma unroll
   for (int r = 0; r < kOutRows; ++r) {
     const uint32_t x = occupied(q[r]);
@@ -201,7 +207,7 @@ __global__ __launch_bounds__(kOutBlock) void k_table_out(const S *__restrict__ d
         out_idx[to] = (int32_t)t;
         out_val[to] = dense[t];
       }
-      if (p_first != p_last) atomicAdd(&tb.splits[p], 1ull);
+      if (p_first != p_last) atomicAdd(&held[p - p_first], 1u);
     }
     at += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
     if (x) {  // leave the table empty again
@@ -213,7 +219,13 @@ __global__ __launch_bounds__(kOutBlock) void k_table_out(const S *__restrict__ d
       }
     }
   }
-  if (p_first == p_last && threadIdx.x == 0 && all) atomicAdd(&tb.splits[p_first], (unsigned long long)all);
+  if (p_first == p_last) {
+    if (threadIdx.x == 0 && all) atomicAdd(&tb.splits[p_first], (unsigned long long)all);
+  } else {
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i <= p_last - p_first; i += kOutBlock)
+      if (held[i]) atomicAdd(&tb.splits[p_first + i], (unsigned long long)held[i]);
+  }
   if (c == stretches - 1 && threadIdx.x == 0 && front + all + carry > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
   // the serial tails of the partitions that end in this stretch, in ascending index order
   for (uint32_t p = p_first; p <= p_last; ++p) {
