@@ -181,6 +181,39 @@ def test_sparse_balance_tables_byte_identical(zen, oracle, n, P, density, scale,
         assert np.array_equal(to_np(ser), ser_o)
 
 
+@pytest.mark.parametrize("n,P,entries", [
+    (1 << 18, 1, 2), (1 << 18, 1, 8193),  # one turn of the region's sort: the smallest, many
+    (1 << 20, 1, 16384), (1 << 20, 1, 16385), (1 << 20, 1, 64512), (1 << 20, 1, 64513),  # one turn, two, as many as fit, one more
+    (1 << 22, 2, 40000),    # piled up at the end of the tensor
+    (60000, 1025, 600),     # more partitions than a workgroup collects for
+])
+def test_serial_regions_at_the_edges_of_their_sort(zen, oracle, n, P, entries):
+    """One level only, and `entries` indices more than there are slots taken: pairs of indices that share a slot."""
+    m, sn = oracle.table_sizes(n, P)
+    t = np.arange(n, dtype=np.uint32)
+    slot = (((np.uint32(573729859) * t + np.uint32(0xCC9E2D51)) * t + np.uint32(0x1B873593)) * t + np.uint32(10001861)) % np.uint32(m)
+    order = np.argsort(slot, kind="stable")[1:]
+    order = order[order != 0]
+    twin = order[1:][slot[order[1:]] == slot[order[:-1]]]  # every one loses its slot to the one in front of it
+    if n == 1 << 22:
+        twin = np.sort(twin)[-entries:]
+    chosen = np.random.default_rng(entries).permutation(twin)[:entries]
+    assert len(chosen) >= min(entries, 2)
+    g = np.zeros(n, np.float32)
+    g[chosen] = 1.0
+    place = np.empty(n, np.int64)
+    place[order] = np.arange(len(order))
+    g[order[place[chosen] - 1]] = 1.0
+    mem_o, ser_o, off_o, st_o = oracle.sparse_balance(g, m, sn, P, 1)
+    mem = torch.zeros(m, dtype=torch.int32, device="cuda")
+    ser = torch.zeros(sn, dtype=torch.int32, device="cuda")
+    zen.sparse_balance(to_dev(g), mem, ser, P, 1)
+    assert int(zen.last_status().status.item()) == st_o and np.array_equal(to_np(zen.last_status().offsets), off_o)
+    assert np.array_equal(to_np(mem), mem_o)
+    if st_o == 0:
+        assert np.array_equal(to_np(ser), ser_o)
+
+
 def test_sparse_balance_overflow_is_flagged_not_oob(zen, oracle):
     n, P = 40000, 4
     g = np.ones(n, np.float32)

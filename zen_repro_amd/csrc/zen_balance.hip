@@ -11,6 +11,8 @@
 // are needed.  In the library's own tables the winner is found with atomicMax on
 // the encoding 0 - index (so the empty marker 0 stays the smallest value).
 #include "zen_balance.h"
+#include "zen_hashmap.h"
+#include "zen_wide.h"
 
 namespace zen {
 namespace {
@@ -87,13 +89,35 @@ __device__ inline uint32_t insert_plain(uint32_t *table, const Probe &g, uint32_
 
 // Bound by the atomics, one or a few per index at random places: 21 a nanosecond.  (On 0 - index with a maximum, which
 // needed a second kernel that looked every index up again, wrote it as it is and found those without a slot: 16.8 M
-// bf16 elements, 5 % nonzero: 39 + 33 us.)
+// bf16 elements, 5 % nonzero: 39 + 33 us.)  The indices without a slot are collected per workgroup, and a wave asks for
+// the places of all partitions at once: the partitions' counters lie side by side, and one line carries out a request
+// every ten nanoseconds (a request per index, 2.3 M bf16 elements on 8 partitions, 10 % nonzero, one level: 151 us).
+constexpr int kDenseBlock = 512;
+constexpr uint32_t kDenseLost = 2048;   // indices without a slot a workgroup collects; the others ask one by one
+constexpr int kDenseParts = 1024;       // partitions up to which it collects
+
 template <typename S, bool ALIGNED>
-__global__ __launch_bounds__(256) void k_insert_dense(const S *__restrict__ in, int64_t n, uint32_t *table, Probe g,
-                                                      int32_t *serial, int64_t spp, int32_t *offset, int32_t *status) {
+__global__ __launch_bounds__(kDenseBlock) void k_insert_dense(const S *__restrict__ in, int64_t n, uint32_t *table, Probe g,
+                                                              int32_t *serial, int64_t spp, int32_t *offset, int partitions,
+                                                              int32_t *status) {
   constexpr int V = VecOf<S>::kN;
+  __shared__ uint32_t lost_t[kDenseLost], lost_at[kDenseLost];  // the index; partition << 16 | place among its partition's
+  __shared__ int32_t held[kDenseParts];                         // collected per partition, then where they go
+  __shared__ uint32_t lost_n;
+  static_assert(kDenseLost <= 65536, "a place in 16 bits");
+  const bool collect = partitions <= kDenseParts;
+  if (collect)
+    for (int p = threadIdx.x; p < partitions; p += kDenseBlock) held[p] = 0;
+  if (threadIdx.x == 0) lost_n = 0;
+  __syncthreads();
+  auto put = [&](uint32_t t, uint32_t part, int64_t ticket) {
+    if (ticket >= 0 && ticket < (int64_t)(part + 1) * spp)
+      serial[ticket] = (int32_t)t;
+    else
+      atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
+  };
   const int64_t nvec = (n + V - 1) / V;
-  for (int64_t v = blockIdx.x * (int64_t)256 + threadIdx.x; v < nvec; v += (int64_t)gridDim.x * 256) {
+  for (int64_t v = blockIdx.x * (int64_t)kDenseBlock + threadIdx.x; v < nvec; v += (int64_t)gridDim.x * kDenseBlock) {
     S e[V];
     const int live = load_vec<S, ALIGNED>(in, v * V, n, e);
 #pragma unroll
@@ -103,19 +127,100 @@ __global__ __launch_bounds__(256) void k_insert_dense(const S *__restrict__ in, 
       uint32_t part;
       const uint32_t left = insert_plain(table, g, t, &part);
       if (left == 0) continue;
-      const int64_t ticket = atomicAdd(&offset[part], 1);
-      if (ticket >= 0 && ticket < (int64_t)(part + 1) * spp)
-        serial[ticket] = (int32_t)left;
-      else
-        atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
+      const uint32_t at = collect ? atomicAdd(&lost_n, 1u) : kDenseLost;
+      if (at < kDenseLost) {
+        lost_t[at] = left;
+        lost_at[at] = (part << 16) | (uint32_t)atomicAdd(&held[part], 1);
+      } else {
+        put(left, part, atomicAdd(&offset[part], 1));
+      }
     }
+  }
+  __syncthreads();
+  const uint32_t lost = lost_n < kDenseLost ? lost_n : kDenseLost;
+  if (!collect || lost == 0) return;
+  for (int p = threadIdx.x; p < partitions; p += kDenseBlock)
+    if (held[p]) held[p] = atomicAdd(&offset[p], held[p]);
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < lost; i += kDenseBlock) {
+    const uint32_t part = lost_at[i] >> 16;
+    put(lost_t[i], part, (int64_t)held[part] + (lost_at[i] & 0xffffu));
   }
 }
 
 // Tickets are handed out in arrival order; the canonical order is ascending
 // index inside each partition's region, so each region is sorted in place.
-__global__ __launch_bounds__(256) void k_serial_sort(int32_t *serial, int64_t spp, const int32_t *offset) {
-  __shared__ uint32_t buf[kSerialLds];
+//
+// A region's indices lie anywhere in [0, n), spread as evenly as the nonzeros are: they are grouped by narrow index
+// ranges in LDS (WideCounters, zen_wide.h) and ranked against the few words of their range, a part of them at a time
+// and the rest in the workgroup's registers.  Bound by the LDS round trips, a dozen for every 16 384 entries: 4
+// regions of 5200 entries 12 us, 4 of 21 000 17 (the compare-exchange network: 68 and, in memory, several hundred).  Where the indices pile up, and
+// for more than 64 512, the network does it.
+constexpr int kSerialSortBlock = 1024;
+constexpr uint32_t kRangeSort = 8192;       // entries expected in one go where there are more than there is room for (16 384):
+                                            // the larger of two indices loses, so that the last range holds up to twice its share
+constexpr uint32_t kRangeGroup = 64;        // entries of a narrow range, at most
+struct SerialSortShared {
+  WideCounters cnt;
+  uint32_t key[kWideSubs];
+  uint32_t scan[kSerialSortBlock / 64 + 1];
+  uint32_t big;
+};
+
+// Whether the region's cnt <= ITEMS * kSerialSortBlock entries could be put in order (else they are as they were).
+template <int ITEMS>
+__device__ inline bool sort_spread(uint32_t *region, uint32_t cnt, uint32_t n, SerialSortShared &sh) {
+  const uint32_t tid = threadIdx.x;
+  uint32_t k[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const uint32_t j = tid + (uint32_t)(i * kSerialSortBlock);
+    k[i] = kNone;
+    if ((uint32_t)(i * kSerialSortBlock) < cnt) k[i] = j < cnt ? region[j] : kNone;
+  }
+  const uint32_t turns = cnt <= (uint32_t)kWideSubs ? 1u : (cnt + kRangeSort - 1u) / kRangeSort, width = (n - 1u) / turns + 1u;
+  uint32_t shift = 0, placed = 0;
+  while (((width - 1u) >> shift) >= (uint32_t)kWideSubs) ++shift;
+  bool ok = true;
+  for (uint32_t r = 0; r < turns; ++r) {
+    const uint32_t lo = r * width;  // (an entry's distance from it wraps around below)
+    sh.cnt.clear();
+    if (tid == 0) sh.big = 0;
+    __syncthreads();  // (and everybody holds the entries of the last turn in registers)
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i)
+      if ((uint32_t)(i * kSerialSortBlock) < cnt && k[i] != kNone && k[i] - lo < width) sh.cnt.count((k[i] - lo) >> shift);
+    __syncthreads();
+    const uint32_t here = sh.cnt.starts(sh.scan, kRangeGroup, &sh.big);
+    __syncthreads();
+    if (here > (uint32_t)kWideSubs || sh.big) {
+      ok = false;
+      break;
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i)
+      if ((uint32_t)(i * kSerialSortBlock) < cnt && k[i] != kNone && k[i] - lo < width) sh.key[sh.cnt.take((k[i] - lo) >> shift)] = k[i];
+    __syncthreads();
+    for (uint32_t j = tid; j < here; j += kSerialSortBlock) {
+      const uint32_t mine = sh.key[j], sub = (mine - lo) >> shift, end = sh.cnt.end_of(sub);
+      uint32_t at = sh.cnt.start_of(sub);
+      for (uint32_t u = at; u < end; ++u) at += sh.key[u] < mine;
+      region[placed + at] = mine;
+    }
+    placed += here;
+    __syncthreads();
+  }
+  if (ok) return true;
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i)
+    if (k[i] != kNone) region[tid + (uint32_t)(i * kSerialSortBlock)] = k[i];
+  __syncthreads();
+  return false;
+}
+
+__global__ __launch_bounds__(kSerialSortBlock) void k_serial_sort(int32_t *serial, int64_t spp, const int32_t *offset,
+                                                                  uint32_t n) {
+  __shared__ SerialSortShared sh;
   const int p = blockIdx.x;
   const int64_t begin = (int64_t)p * spp;
   int64_t end = offset[p];
@@ -123,12 +228,13 @@ __global__ __launch_bounds__(256) void k_serial_sort(int32_t *serial, int64_t sp
   if (end - begin < 2) return;
   const uint32_t cnt = (uint32_t)(end - begin);
   uint32_t *region = reinterpret_cast<uint32_t *>(serial + begin);
-  if (cnt <= kSerialLds) {
-    for (uint32_t i = threadIdx.x; i < cnt; i += blockDim.x) buf[i] = region[i];
+  if (cnt <= 16u * kSerialSortBlock) {
+    if (sort_spread<16>(region, cnt, n, sh)) return;
+    for (uint32_t i = threadIdx.x; i < cnt; i += kSerialSortBlock) sh.key[i] = region[i];
     __syncthreads();
-    sort_network(buf, cnt);
-    for (uint32_t i = threadIdx.x; i < cnt; i += blockDim.x) region[i] = buf[i];
-  } else {
+    sort_network(sh.key, cnt);
+    for (uint32_t i = threadIdx.x; i < cnt; i += kSerialSortBlock) region[i] = sh.key[i];
+  } else if (cnt > 63u * kSerialSortBlock || !sort_spread<63>(region, cnt, n, sh)) {  // (counts below 2^16)
     sort_network(region, cnt);
   }
 }
@@ -220,17 +326,17 @@ int sparse_balance_launch(const S *in, int64_t n, uint32_t *table, Probe g, int3
                           int32_t *offset, int partitions, int32_t *status, hipStream_t s) {
   constexpr int V = VecOf<S>::kN;
   const int64_t nvec = ceil_div(n, V);
-  int64_t blocks = ceil_div(nvec, 256);
-  if (blocks > 16384) blocks = 16384;
+  int64_t blocks = ceil_div(nvec, kDenseBlock);
+  if (blocks > 1024) blocks = 1024;  // as many as the chip holds
   const bool aligned = (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
   ProfScope prof(kProfInsertDense, s);
   if (aligned)
-    k_insert_dense<S, true><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(in, n, table, g, serial, spp, offset, status);
+    k_insert_dense<S, true><<<dim3((unsigned)blocks), dim3(kDenseBlock), 0, s>>>(in, n, table, g, serial, spp, offset, partitions, status);
   else
-    k_insert_dense<S, false><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(in, n, table, g, serial, spp, offset, status);
+    k_insert_dense<S, false><<<dim3((unsigned)blocks), dim3(kDenseBlock), 0, s>>>(in, n, table, g, serial, spp, offset, partitions, status);
   ZEN_LAUNCH_CHECK("k_insert_dense");
   if (spp > 0) {
-    k_serial_sort<<<dim3((unsigned)partitions), dim3(256), 0, s>>>(serial, spp, offset);
+    k_serial_sort<<<dim3((unsigned)partitions), dim3(kSerialSortBlock), 0, s>>>(serial, spp, offset, (uint32_t)n);
     ZEN_LAUNCH_CHECK("k_serial_sort");
   }
   return ZEN_OK;
