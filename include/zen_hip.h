@@ -51,8 +51,9 @@ extern "C" {
  *    16-byte entry per 96 indices (zen_bitmap_rank_words), and the dense
  *    dictionary is longer by a chunk of places (zen_bitmap_dense_dict_bytes):
  *    both are built anew, not kept from an older library
+ * 8: zen_balance_tables
  */
-#define ZEN_ABI_VERSION 7
+#define ZEN_ABI_VERSION 8
 
 #define ZEN_F32 0
 #define ZEN_BF16 1
@@ -192,6 +193,14 @@ int zen_sparse_balance(const void *input, int dtype, int64_t n,
                        int32_t *serial, int64_t serial_n,
                        int32_t *offset, int partitions, int rehash,
                        int32_t *status, void *stream);
+/*
+ * The same into tables of any content, which are cleared first; offset[partitions] is filled in.  Returns when
+ * everything is done, with the status word in host[1] (host: `words` >= 2 of zen_host_words_alloc).  What
+ * TensorPartition.balance_sparse_tensor does (tensor_load_balance.py:13-21).
+ */
+int zen_balance_tables(const void *input, int dtype, int64_t n, int32_t *memory, int64_t m, int32_t *serial,
+                       int64_t serial_n, int32_t *offset, int partitions, int rehash, int32_t *status,
+                       int64_t *host, int64_t words, void *stream);
 
 /* ---------------------------------------------------------------- select */
 

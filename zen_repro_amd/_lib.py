@@ -24,7 +24,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("ZEN_HIP_LIB") or os.path.join(_HERE, "csrc", "libzen_hip.so")
 
 # ZEN_ABI_VERSION of include/zen_hip.h this loader's signatures and structs are written for
-ABI_VERSION = 7
+ABI_VERSION = 8
 TABLE_SIZES_MOST = 1024  # ZEN_TABLE_SIZES_MOST
 
 _lib = None
@@ -80,6 +80,7 @@ def lib():
         "zen_bitmap_decode_workspace": (sz, [i64]),
         "zen_bitmap_decode": (i32, [vp, i64, vp, i64, vp, i64, vp, vp, sz, vp, vp]),
         "zen_sparse_balance": (i32, [vp, i32, i64, vp, i64, vp, i64, vp, i32, i32, vp, vp]),
+        "zen_balance_tables": (i32, [vp, i32, i64, vp, i64, vp, i64, vp, i32, i32, vp, vp, i64, vp]),
         "zen_encode_merge_samples_next": (i32, [i64, i64, i32, i64, i32, i64, i32]),
         "zen_topk_threshold_workspace": (sz, []),
         "zen_topk_threshold": (i32, [vp, i32, i64, i64, vp, vp, sz, vp]),

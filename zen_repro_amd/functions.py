@@ -19,11 +19,11 @@ def sparse_balance(tensor, memory, serial_memory, partitions, rehash):
     reference, float32 additionally.  Raises RuntimeError when a partition has
     more overflow entries than serial slots (the reference writes out of bounds).
     """
-    assert tensor.is_cuda and tensor.dtype in (torch.bfloat16, torch.float32)
+    _check_input(tensor)
     assert memory.is_cuda and memory.dtype == torch.int32
     assert serial_memory.is_cuda and serial_memory.dtype == torch.int32
-    for name, t in (("input", tensor), ("memory", memory), ("serial_memory", serial_memory)):
-        _lib.require_gpu(t, name)
+    _lib.require_gpu(memory, "memory")
+    _lib.require_gpu(serial_memory, "serial_memory")
     numel = serial_memory.numel()
     numel_per_part = numel // partitions
     # serial base offsets, extensions/cuda/functions.py:8-11
@@ -35,6 +35,32 @@ def sparse_balance(tensor, memory, serial_memory, partitions, rehash):
         _lib.ptr(offsets), partitions, rehash, _lib.ptr(status), _lib.stream_of(tensor.device))
     _lib.check(rc, "sparse_balance")
     _last.pending = _PendingStatus(status, offsets)  # the call itself returns None, like the reference's
+
+
+def fresh_tables(tensor, memory_size, serial_memory_size, partitions, rehash):
+    """sparse_balance into two new tables of these sizes, checked (last_status): (memory, serial_memory)."""
+    _check_input(tensor)
+    dev = tensor.device
+    memory = torch.empty(memory_size, dtype=torch.int32, device=dev)
+    serial_memory = torch.empty(serial_memory_size, dtype=torch.int32, device=dev)
+    offsets = torch.empty(partitions, dtype=torch.int32, device=dev)
+    status = _lib.status_word(dev)
+    words = _lib.host_words(1)
+    rc = _lib.lib().zen_balance_tables(
+        _lib.ptr(tensor), _lib.dtype_code(tensor), tensor.numel(), _lib.ptr(memory), memory_size,
+        _lib.ptr(serial_memory), serial_memory_size, _lib.ptr(offsets), partitions, rehash, _lib.ptr(status), words.ptr,
+        words.words, _lib.stream_of(dev))
+    _lib.check(rc, "sparse_balance")
+    bits = words.view[1]
+    _last.pending = _PendingStatus(status, offsets)
+    if bits:
+        raise RuntimeError("sparse_balance: " + _lib.describe_status(bits))
+    return memory, serial_memory
+
+
+def _check_input(tensor):
+    assert tensor.is_cuda and tensor.dtype in (torch.bfloat16, torch.float32)
+    _lib.require_gpu(tensor, "input")
 
 
 _last = threading.local()

@@ -6,7 +6,7 @@ import ctypes
 import torch
 
 from . import _lib
-from .functions import last_status, sparse_balance
+from .functions import fresh_tables
 
 
 class _Mark:
@@ -59,11 +59,7 @@ class TensorPartition:
         """Allocates and fills the two tables (tensor_load_balance.py:13-21)."""
         with _lib.annotate("balance_sparse_tensor"):  # tensor_load_balance.py:44
             memory_size, serial_memory_size = self.table_sizes(tensor.numel())
-            memory = torch.zeros(memory_size, dtype=torch.int32, device=tensor.device)
-            serial_memory = torch.zeros(serial_memory_size, dtype=torch.int32, device=tensor.device)
-            sparse_balance(tensor, memory, serial_memory, self.partitions, rehash=self.rehash)
-            last_status().check()
-            return memory, serial_memory
+            return fresh_tables(tensor, memory_size, serial_memory_size, self.partitions, self.rehash)
 
     def get_sub_sparse_tensors(self, tensor, memory):
         """Per-partition nonzero entries of a table and the values they point
