@@ -385,6 +385,29 @@ def test_slab_merge_bit_exact(zen, oracle, n, peers, per_peer, overlap, dtype, i
     assert np.array_equal(to_np(dense), oracle.f32_to_bf16_bits(f32) if dtype == "bf16" else f32)
 
 
+@pytest.mark.parametrize("r", [1 << 19, (1 << 19) + 1, 1900000, 128 * 15360 + 1])
+def test_merge_that_waits_gives_the_same_on_half_and_all_of_the_chip(zen, oracle, r):
+    """One list of r entries around the sizes where the number of wide buckets changes, against merge_sparse_flat."""
+    n = 20000000
+    gen = torch.Generator(device="cuda").manual_seed(r)
+    idx = torch.randint(0, n, (r,), generator=gen, device="cuda")
+    val = torch.randn(r, generator=gen, device="cuda").to(torch.bfloat16)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    w_idx, w_val = oracle.merge_sparse(to_np(idx), to_np(val), n)
+    dense = lba.decode_sparse_tensors(idx, val, n)
+    f_idx, f_val, count, status = lba.merge_sparse_flat(idx, val, n)
+    assert status.item() == 0 and count.item() == len(w_idx)
+    assert np.array_equal(to_np(f_idx)[:len(w_idx)], w_idx)
+    assert np.array_equal(to_np(f_val)[:len(w_idx)].view(np.uint32), w_val.view(np.uint32))
+    rounded = torch.from_numpy(w_val).to(torch.bfloat16)
+    kept = rounded != 0
+    want = torch.zeros(n, dtype=torch.bfloat16)
+    want[torch.from_numpy(w_idx.astype(np.int64))] = rounded
+    assert torch.equal(dense.cpu(), want)
+    m_idx, m_val = lba.merge_rounded(idx, val, n, torch.bfloat16)
+    assert np.array_equal(to_np(m_idx), w_idx[kept.numpy()]) and torch.equal(m_val.cpu(), rounded[kept])
+
+
 def test_slab_merge_bad_indices_cancellation_and_pile_up(zen, oracle):
     from zen_repro_amd import _lib
 

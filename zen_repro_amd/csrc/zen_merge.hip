@@ -545,7 +545,7 @@ int merge_launch(const void *idx, int idx64_in, const S *val, int64_t r, int64_t
     }
     WideList list;
     if (!wide_merge_list(idx, idx64_in, val, r, dense_n, cursor, static_cast<char *>(workspace) + kMergeZeroBytes,
-                         wide_device_cus(), status, &list))
+                         wide_device_cus(), status, &list, ask.answer.host != nullptr))
       return fail(ZEN_EINVAL, "zen_merge: sizes do not suit the wide buckets");
     return wide_merge(list, sizeof(S) == 2 ? ZEN_BF16 : ZEN_F32, out_idx, idx64_out, out_val,
                       sizeof(O) == 2 ? ZEN_BF16 : ZEN_F32, capacity, out_count, scan, s, ask);

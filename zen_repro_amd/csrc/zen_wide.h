@@ -31,16 +31,19 @@ constexpr uint32_t kWideCursorWords = kWideMaxBuckets * kWideSplit * kWidePad;
 // a chip of `cus` compute units; false if the layout does not suit these sizes.  The result is a SlabGeom
 // whose sub_shift refers to kWideSubs narrow ranges.  least_m: the encode keeps its counters in the caller's table
 // (4 MB or more: the map at its head takes at most half, the counters behind it less than 1 MB); least_width: keys of
-// a bucket, at least.
+// a bucket, at least; whole_chip: nothing runs beside the launch.
 inline bool wide_geometry(int64_t m, int partitions, int64_t expected, int cus, SlabGeom *out,
-                          int64_t least_m = 1ll << 20, int64_t least_width = 4ll * kWideSubs) {
+                          int64_t least_m = 1ll << 20, int64_t least_width = 4ll * kWideSubs, bool whole_chip = false) {
   if (m < least_m || m > 0x7fffffffll || partitions < 1 || partitions > kWideMaxBuckets || m % partitions != 0 ||
       expected < 1)
     return false;
   int64_t most = cus < kWideMaxBuckets ? cus : kWideMaxBuckets;
   // half the chip where that holds the records: a bucket's workgroup wants a compute unit to itself, and the
-  // encode's and the merge's workgroups of one step then find room side by side instead of one after the other
-  if (most >= 2 * partitions && expected <= most / 2 * (int64_t)kWideTarget) most /= 2;
+  // encode's and the merge's workgroups of one step then find room side by side instead of one after the other.  Where
+  // nothing runs beside it, all of it for more records than a bucket gets through in no time (merges that the host waits
+  // for, 128 and 256 buckets: 1.8 M bf16 entries 80 and 74 us dense, 82 and 76 sparse; 0.6 M 65 either way, fewer 0.5
+  // more with 256).
+  if (!(whole_chip && expected > most / 2 * 4096) && most >= 2 * partitions && expected <= most / 2 * (int64_t)kWideTarget) most /= 2;
   int64_t bpp = most / partitions;
   const int64_t npp = m / partitions;
   if (bpp > npp / least_width) bpp = npp / least_width;
@@ -287,10 +290,11 @@ int wide_line_leave(hipStream_t stream);
 int wide_device_cus();
 
 // zen_wide_merge.hip
-bool wide_merge_fits(int64_t r, int64_t dense_n, int cus, SlabGeom *geo);
+// alone: nothing runs beside the merge (a call that waits for its answer).
+bool wide_merge_fits(int64_t r, int64_t dense_n, int cus, SlabGeom *geo, bool alone = false);
 size_t wide_merge_bytes(int64_t r, int64_t dense_n, int cus);
 bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, int64_t dense_n, uint32_t *cursor,
-                     void *rest, int cus, int32_t *status, WideList *list);
+                     void *rest, int cus, int32_t *status, WideList *list, bool alone);
 // One workgroup straight from the list, for up to wide_merge_one_max() entries (kWideCap would fit; from about here
 // on the scatter's launch costs less than the longer chains of one workgroup): no slabs, no zeroed memory.
 constexpr int64_t wide_merge_one_max() { return 4096; }

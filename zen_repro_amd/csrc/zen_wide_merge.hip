@@ -442,7 +442,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
 
 }  // namespace
 
-bool wide_merge_fits(int64_t r, int64_t dense_n, int cus, SlabGeom *geo) {
+bool wide_merge_fits(int64_t r, int64_t dense_n, int cus, SlabGeom *geo, bool alone) {
   SlabGeom g;
   // (shorter lists: wide_merge_one)
   if (r <= wide_merge_one_max() || r > 0x7ffffffell || cus <= 0) return false;
@@ -452,7 +452,7 @@ bool wide_merge_fits(int64_t r, int64_t dense_n, int cus, SlabGeom *geo) {
   const int64_t least = ceil_div(r, (int64_t)8192) > 16 ? ceil_div(r, (int64_t)8192) : 16;
   int64_t width = dense_n / least < 4ll * kWideSubs ? dense_n / least : 4ll * kWideSubs;
   if (width < 1024) width = 1024;
-  if (!wide_geometry(dense_n, 1, r, cus, &g, 1ll << 14, width)) return false;
+  if (!wide_geometry(dense_n, 1, r, cus, &g, 1ll << 14, width, alone)) return false;
   if (g.sub_shift + ceil_log2_u64((uint64_t)r) > 32) return false;  // (index inside a narrow range, arrival number) must fit a word
   // a slab record carries the index's offset inside its bucket and the arrival number in fixed fields
   if ((uint64_t)g.sub_shift + 14 > kWmOffBits || (uint64_t)r >= (1ull << kWmArrBits)) return false;
@@ -464,18 +464,23 @@ static uint32_t wide_merge_part_cap(const SlabGeom &geo, int64_t r) { return wid
 
 // Workspace of the wide path behind the zero region at the head of zen_merge's workspace.
 size_t wide_merge_bytes(int64_t r, int64_t dense_n, int cus) {
-  SlabGeom geo;
-  if (!wide_merge_fits(r, dense_n, cus, &geo)) return 0;
-  const size_t entries = (size_t)geo.nbuckets * kWideSplit * wide_merge_part_cap(geo, r);
+  size_t entries = 0;
+  for (const bool alone : {false, true}) {
+    SlabGeom geo;
+    if (!wide_merge_fits(r, dense_n, cus, &geo, alone)) continue;
+    const size_t e = (size_t)geo.nbuckets * kWideSplit * wide_merge_part_cap(geo, r);
+    if (e > entries) entries = e;
+  }
+  if (!entries) return 0;
   return align_up(entries * sizeof(uint2), 256) + align_up(entries * sizeof(uint32_t), 256);
 }
 
 // The received entries as the scatter wants them: cursor: kCoarseCursorWords zeroed words (zero again when
 // k_wide_merge has run); rest: wide_merge_bytes(...) bytes.  False if the sizes do not suit the wide buckets.
 bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, int64_t dense_n, uint32_t *cursor,
-                     void *rest, int cus, int32_t *status, WideList *list) {
+                     void *rest, int cus, int32_t *status, WideList *list, bool alone) {
   SlabGeom geo;
-  if (!wide_merge_fits(r, dense_n, cus, &geo)) return false;
+  if (!wide_merge_fits(r, dense_n, cus, &geo, alone)) return false;
   WideSlabs slabs;
   slabs.part_cap = wide_merge_part_cap(geo, r);
   const size_t entries = (size_t)geo.nbuckets * kWideSplit * slabs.part_cap;
