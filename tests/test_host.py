@@ -481,6 +481,30 @@ def test_calls_that_return_early_leave_their_buffers_marked(monkeypatch, call, c
     assert held == ([(dense.data_ptr(), s) for s in (1, 1, 2, 2, 1, 2)] if reads else [])
 
 
+def test_every_call_gets_zeroed_words_of_its_own():
+    """Status words and split sizes are cut from blocks: none is handed out twice, also where a block ends, where a
+    piece is longer than a block, and where a stream starts afresh."""
+    from zen_repro_amd import _lib
+
+    zeros = _lib.host.Zeros()
+    flat, ws = torch.zeros(8, dtype=torch.bfloat16), torch.zeros(16, dtype=torch.uint8)
+    held, words = [], []
+    for call in range(3000):
+        parts, stream = (9000, 5) if call == 1500 else (5, 5 + call % 2)
+        rc, idx, val, splits, status = _lib.host.load_balance(
+            lambda *a: len(a), zeros, flat, 1, 8, parts, 3, None, 0, None, 4, 0, 0, ws, stream, 0, 0)
+        assert rc == 19 and idx.shape == val.shape == (4,) and splits.shape == (parts,) and status.shape == (1,)
+        assert not splits.any() and not status.any()
+        held += [splits, status]
+        words += [(t.data_ptr(), t.data_ptr() + t.numel() * t.element_size()) for t in (splits, status)]
+        splits.fill_(-1)
+        status.fill_(-1)
+        if call == 2000:
+            zeros.fresh(-1, 5)
+    words.sort()
+    assert all(a[1] <= b[0] and b[0] % 8 == 0 for a, b in zip(words, words[1:]))
+
+
 def test_compaction_kernels_keep_their_rows_in_registers(tmp_path):
     """The rows a wave has in flight are the kernels' speed: none of their registers may end up in memory, for
     aligned tensors and for views that begin at an odd element."""

@@ -9,6 +9,11 @@ import threading
 
 import torch  # first: makes the process use torch's HIP runtime for libzen_hip too
 
+try:
+    from . import _host as host  # zen_host.cpp: what the calls do around the library's functions
+except ImportError as e:  # not built, or for another torch: lib() says so
+    host, _host_error = None, e
+
 F32, BF16 = 0, 1
 OK, EINVAL, EHIP, EWORKSPACE = 0, -1, -2, -3
 STAT_SERIAL_OVERFLOW, STAT_CAPACITY, STAT_INTERNAL, STAT_BAD_INDEX, STAT_RETRY = 1, 2, 4, 8, 16
@@ -65,6 +70,9 @@ def lib():
         raise RuntimeError(
             f"{LIB_PATH} is missing: build it with `make -C zen_repro_amd/csrc` "
             "(or __graft_entry__.build()); there is no fallback path")
+    if host is None or host.ABI_VERSION != ABI_VERSION:
+        raise RuntimeError(f"zen_repro_amd/_host.so does not load or is of another version: build it with `make -C "
+                           f"zen_repro_amd/csrc` ({_host_error if host is None else host.ABI_VERSION})")
     L = ctypes.CDLL(LIB_PATH)
     vp, i32, i64, sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_size_t
     sig = {
@@ -106,8 +114,7 @@ def lib():
         "zen_encode_merge": (i32, [ctypes.POINTER(EncodeMergeArgs)]),
         "zen_merge_rounded": (i32, [vp, i32, vp, i32, i64, i64, vp, i32, vp, i64, vp, i32, vp, sz, vp, vp]),
         "zen_merge_rounded_count": (i32, [vp, i32, vp, i32, i64, i64, vp, i32, vp, i64, vp, i32, vp, sz, vp, vp, i64, vp]),
-        "zen_decode_dense_lists": (i32, [ctypes.POINTER(vp), i32, ctypes.POINTER(vp), i32, ctypes.POINTER(i64), i32, vp, i64, vp,
-                                         sz, vp, vp]),
+        "zen_decode_dense_lists": (i32, [vp, i32, vp, i32, vp, i32, vp, i64, vp, sz, vp, vp]),
         "zen_decode_dense_workspace": (sz, [i64, i64]),
         "zen_decode_dense": (i32, [vp, i32, vp, i32, i64, vp, i64, i32, vp, sz, vp, vp]),
         "zen_decode_dense_status": (i32, [vp, i32, vp, i32, i64, vp, i64, i32, vp, sz, vp, vp, i64, vp]),
@@ -118,8 +125,7 @@ def lib():
         "zen_bitmap_dense_workspace": (sz, [i64, i32]),
         "zen_bitmap_dense": (i32, [vp, i64, i32, vp, ctypes.POINTER(ctypes.c_int64), vp, i32,
                                    ctypes.POINTER(ctypes.c_int64), vp, vp, sz, vp, vp]),
-        "zen_bitmap_dense_lists": (i32, [vp, i64, i32, ctypes.POINTER(vp), ctypes.POINTER(i64), ctypes.POINTER(vp), i32,
-                                         ctypes.POINTER(i64), vp, vp, sz, vp, vp]),
+        "zen_bitmap_dense_lists": (i32, [vp, i64, i32, vp, vp, vp, i32, vp, vp, vp, sz, vp, vp]),
         "zen_sort_pairs_workspace": (sz, [i64]),
         "zen_sort_pairs": (i32, [vp, vp, i64, vp, i32, vp, sz, vp, vp]),
         "zen_bucket_sort_fits": (i32, [i64, ctypes.c_uint32]),
@@ -314,6 +320,14 @@ class ZeroPool:
     def __init__(self):
         self._local = threading.local()
 
+    def native(self):
+        """The same for this thread's calls through zen_host.cpp, whose blocks are their own."""
+        try:
+            return self._local.native
+        except AttributeError:
+            self._local.native = host.Zeros()
+            return self._local.native
+
     _SIZES = {torch.int32: 4, torch.int64: 8, torch.uint8: 1, torch.float32: 4}
 
     def _blocks(self):
@@ -371,6 +385,7 @@ class ZeroPool:
         key = (device_index(device), stream_handle(device))
         for k in [k for k in blocks if k[:2] == key]:
             del blocks[k]
+        self.native().fresh(*key)
 
 
 zeros = ZeroPool()

@@ -37,15 +37,10 @@ def _select_raw(tensor, thr, idx64, capacity=None):
         capacity = n
     L = _lib.lib()
     code = _lib.dtype_code(flat)
-    out_idx = torch.empty(capacity, dtype=torch.int64 if idx64 else torch.int32, device=dev)
-    out_val = torch.empty(capacity, dtype=flat.dtype, device=dev)
-    count = _lib.zeros.word(dev, torch.int64)
-    status = _lib.status_word(dev)
     ws = _lib.scratch.get(dev, "select", L.zen_select_workspace(n, code))
     words = _lib.host_words(2)
-    rc = L.zen_select_count(_lib.ptr(flat), code, n, _lib.ptr(thr), _lib.ptr(out_idx), 1 if idx64 else 0,
-                            _lib.ptr(out_val), capacity, _lib.ptr(count), _lib.ptr(ws), ws.numel(),
-                            _lib.ptr(status), words.ptr, words.words, _lib.stream_of(dev))
+    rc, out_idx, out_val = _lib.host.select_count(L.zen_select_count, _lib.zeros.native(), flat, code, _lib.ptr(thr), idx64,
+                                                  capacity, ws, _lib.stream_of(dev), words.ptr, words.words)
     _lib.scratch.left_running(dev, "select", flat, thr)
     _lib.check(rc, "select")
     host = words.view[1:3]
@@ -91,7 +86,7 @@ class LoadBalanceAllreduce:
         # comm.py:25-29; payloads that already sit back to back in one buffer
         # (what an all-to-all into a single flat buffer leaves) are not copied
         if isinstance(tensors, (list, tuple)):
-            flat = _as_one_buffer(tensors)
+            flat = _lib.host.one_buffer(tensors)
             return (flat if flat is not None else torch.cat(list(tensors))).reshape(shape)
         return tensors.reshape(shape)
 
@@ -122,12 +117,10 @@ class LoadBalanceAllreduce:
         # zeroed at first and left so by the calls, like merge_sparse_flat's
         ws = _lib.scratch.get(dev, "decode", L.zen_decode_dense_workspace(r, alltoall_dense_size), zero=True)
         for mode in self._fast_then_general():
-            status = _lib.status_word(dev)
             words = _lib.host_words(1)
-            rc = L.zen_decode_dense_status(_lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(values),
-                                           _lib.dtype_code(values), r, _lib.ptr(dense), alltoall_dense_size,
-                                           mode | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status),
-                                           words.ptr, words.words, _lib.stream_of(dev))
+            rc, _ = _lib.host.decode(L.zen_decode_dense_status, _lib.zeros.native(), indices, values,
+                                     _lib.dtype_code(values), dense, mode | _lib.MODE_ZEROED, ws, _lib.stream_of(dev),
+                                     words.ptr, words.words)
             _lib.scratch.left_running(dev, "decode")
             if rc != _lib.OK:
                 ws[:L.zen_merge_zero_bytes()].zero_()
@@ -151,8 +144,7 @@ class LoadBalanceAllreduce:
         if not 1 <= count <= 64 or not values:
             return None
         dev = values[0].device
-        if len(values) != count or not _plain_runs(lists) or not _plain_runs(values) or any(
-                i.numel() != v.numel() or i.get_device() != v.get_device() for i, v in zip(lists, values)):
+        if not _lib.host.matching_runs(lists, values):
             sizes = [t.numel() for t in lists]
             indices = self.stack_tensors(indices_tensors)
             values = self.stack_tensors(values_tensors)
@@ -163,15 +155,9 @@ class LoadBalanceAllreduce:
         _lib.require_gpu(values[0], "values")
         assert lists[0].dtype in (torch.int32, torch.int64)
         L = _lib.lib()
-        dense = torch.empty(dense_size, dtype=values[0].dtype, device=dev)
-        idx_at = (ctypes.c_void_p * count)(*[t.data_ptr() for t in lists])
-        val_at = (ctypes.c_void_p * count)(*[t.data_ptr() for t in values])
-        sizes = (ctypes.c_int64 * count)(*[t.numel() for t in lists])
         ws = _lib.scratch.get(dev, "decode_sorted", L.zen_decode_dense_sorted_workspace(dense_size, count))
-        status = _lib.status_word(dev)
-        rc = L.zen_decode_dense_lists(idx_at, int(lists[0].dtype == torch.int64), val_at, _lib.dtype_code(values[0]),
-                                      sizes, count, _lib.ptr(dense), dense_size, _lib.ptr(ws), ws.numel(),
-                                      _lib.ptr(status), _lib.stream_of(dev))
+        rc, dense, status = _lib.host.decode_lists(L.zen_decode_dense_lists, _lib.zeros.native(), lists, values,
+                                                   _lib.dtype_code(values[0]), dense_size, ws, _lib.stream_of(dev))
         _lib.check(rc, "decode_sparse_tensors")
         # the reference's scatter_add_ raises on a bad index, also a sync
         return None if _lib.read_back(status)[0] else dense
@@ -220,21 +206,15 @@ class LoadBalanceAllreduce:
             capacity = r
         if (mode & 0xff) == _lib.MODE_FAST:
             mode |= self.fast_flags
-        out_idx = torch.empty(capacity, dtype=torch.int64 if idx64 else torch.int32, device=dev)
-        out_val = torch.empty(capacity, dtype=values.dtype if rounded else torch.float32, device=dev)
-        count = _lib.zeros.word(dev, torch.int64)
-        status = _lib.status_word(dev)
         # The workspace is allocated zeroed and serves zen_merge only, which leaves its head (the counters
         # that must start at zero) zero again: no call spends a kernel on clearing it.
         ws = _lib.scratch.get(dev, f"merge/{slot}", L.zen_merge_workspace(r, dense_size), zero=True)
-        args = (_lib.ptr(indices), int(indices.dtype == torch.int64), _lib.ptr(values), _lib.dtype_code(values), r,
-                dense_size, _lib.ptr(out_idx), 1 if idx64 else 0, _lib.ptr(out_val), capacity, _lib.ptr(count),
-                mode | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status))
+        call = L.zen_merge_rounded_count if words is not None else L.zen_merge_rounded if rounded else L.zen_merge
+        rc, out_idx, out_val, count, status = _lib.host.merge(
+            call, _lib.zeros.native(), indices, values, _lib.dtype_code(values), dense_size, capacity, idx64, rounded,
+            mode | _lib.MODE_ZEROED, ws, _lib.stream_of(dev), *((words.ptr, words.words) if words is not None else (0, 0)))
         if words is not None:
-            rc = L.zen_merge_rounded_count(*args, words.ptr, words.words, _lib.stream_of(dev))
             _lib.scratch.left_running(dev, f"merge/{slot}")
-        else:
-            rc = (L.zen_merge_rounded if rounded else L.zen_merge)(*args, _lib.stream_of(dev))
         if rc != _lib.OK:
             ws[:L.zen_merge_zero_bytes()].zero_()
         _lib.check(rc, "merge_sparse")
@@ -279,14 +259,6 @@ class LoadBalanceAllreduce:
                                                L.zen_merge_workspace(r, dense_size), None)
         m, ws_bytes, mws_bytes = sizes[:3]
         mode = _lib.MODE_FAST | partition.fast_flags
-        out_idx = torch.empty(capacity, dtype=torch.int32, device=dev)
-        out_val = torch.empty(capacity, dtype=flat.dtype, device=dev)
-        m_idx = torch.empty(r, dtype=torch.int32, device=dev)
-        m_val = torch.empty(r, dtype=torch.float32, device=dev)
-        # split sizes, merged count, the two status words
-        small = _lib.zeros.take(dev, P + 2, torch.int64, merge_stream)
-        splits, count, status2 = small.split((P, 1, 1))
-        status, m_status = status2.view(torch.int32).split(1)
         if next_k is None:
             next_k = k
         if next_capacity is None:
@@ -317,35 +289,20 @@ class LoadBalanceAllreduce:
                                         r=r, dense_n=dense_size, merged_capacity=r)
             sizes = self._step_sizes[shape] = sizes[:3] + (base,)
         a = _lib.EncodeMergeArgs.from_buffer_copy(base)
-        a.input = flat.data_ptr()
+        encoded, merged, wait = _lib.host.step_buffers(
+            ctypes.addressof(a), _lib.zeros.native(), flat, indices, values, capacity, P, _lib.stream_handle(dev),
+            merge_stream.cuda_stream if merge_stream is not None else 0, ws, mws)
+        if wait:  # the fill of the words lies on the current stream
+            merge_stream.wait_stream(torch.cuda.current_stream(dev))
         a.rehash = partition.rehash
         if thr is not None:
             a.thr = thr.data_ptr()
         a.k = int(k)
         if thr_out is not None:
             a.thr_out = thr_out.data_ptr()
-        a.out_idx = out_idx.data_ptr()
-        a.out_val = out_val.data_ptr()
-        at = small.data_ptr()
-        a.splits = at
         a.table = table.data_ptr()
         a.mode = mode | flags | _lib.MODE_ZEROED
-        a.workspace = ws.data_ptr()
-        a.workspace_bytes = ws.numel()
-        a.status = at + 8 * (P + 1)
-        a.recv_idx = indices.data_ptr()
-        a.recv_idx64 = indices.dtype is torch.int64
-        a.recv_val = values.data_ptr()
-        a.merged_idx = m_idx.data_ptr()
-        a.merged_val = m_val.data_ptr()
-        a.merged_count = at + 8 * P
         a.merge_mode = _lib.MODE_FAST | self.fast_flags | _lib.MODE_ZEROED
-        a.merge_workspace = mws.data_ptr()
-        a.merge_workspace_bytes = mws.numel()
-        a.merge_status = at + 8 * (P + 1) + 4
-        a.stream = _lib.stream_handle(dev)
-        if merge_stream is not None:
-            a.merge_stream = merge_stream.cuda_stream
         if nxt is not None:
             a.next_input = nxt.data_ptr()
             a.next_k = int(next_k)
@@ -362,7 +319,7 @@ class LoadBalanceAllreduce:
         partition._after_call(flat, int(k), capacity, slot, mode | flags, used)
         if nxt is not None:
             partition._sample_taken(nxt, int(next_k), next_capacity, ws, slot, 1 - used)
-        return (out_idx, out_val, splits, status), (m_idx, m_val, count, m_status)
+        return encoded, merged
 
     def round_merged_flat(self, indices, sums, count, dtype):
         """What comm.py:125-127 hands to the second exchange, from merge_sparse_flat's output and without host
@@ -547,7 +504,7 @@ class LoadBalanceAllreduce:
         L = _lib.lib()
         values = list(values_tensors)
         dev = values[0].device
-        if not _plain_runs(values):
+        if not _lib.host.plain_runs(values):
             # lists that are no plain runs of one type: in one buffer, of the type that holds them all
             values = torch.split(self.stack_tensors(values), [t.numel() for t in values])
         _lib.require_gpu(values[0], "values")
@@ -561,16 +518,9 @@ class LoadBalanceAllreduce:
                        "decode_bitmaps_dense")
             self._dense_dicts[numel] = cached
         P = self.partitions
-        bm_at = (ctypes.c_void_p * P)(*[t.data_ptr() for t in bitmap_indices])
-        bm_bytes = (ctypes.c_int64 * P)(*[t.numel() for t in bitmap_indices])
-        v_at = (ctypes.c_void_p * P)(*[t.data_ptr() for t in values])
-        v_count = (ctypes.c_int64 * P)(*[t.numel() for t in values])
-        dense = torch.empty(numel, dtype=values[0].dtype, device=dev)
         ws = _lib.scratch.get(dev, "bitmap_dense", L.zen_bitmap_dense_workspace(numel, P))
-        status = _lib.status_word(dev)
-        rc = L.zen_bitmap_dense_lists(_lib.ptr(cached), numel, P, bm_at, bm_bytes, v_at, _lib.dtype_code(values[0]),
-                                      v_count, _lib.ptr(dense), _lib.ptr(ws), ws.numel(), _lib.ptr(status),
-                                      _lib.stream_of(dev))
+        rc, dense, status = _lib.host.bitmaps_dense(L.zen_bitmap_dense_lists, _lib.zeros.native(), bitmap_indices, values,
+                                                    _lib.dtype_code(values[0]), cached, numel, ws, _lib.stream_of(dev))
         _lib.check(rc, "decode_bitmaps_dense")
         bits = _lib.read_back(status)[0]  # the reference's masking and scatter_add_ raise on a mismatch, also a sync
         if bits & _lib.STAT_BAD_INDEX:
@@ -655,36 +605,7 @@ class LoadBalanceAllreduce:
             return self.decode_sparse_tensors(indices_tensors, values_tensors, numel, ascending=True)
 
 
-def _plain_runs(tensors):
-    """Whether the tensors are contiguous, of one type and on one device: what a kernel takes by their addresses."""
-    dtype, at = tensors[0].dtype, tensors[0].get_device()
-    for t in tensors:
-        if t.dtype is not dtype or t.get_device() != at or not t.is_contiguous():
-            return False
-    return True
-
-
 def _as_one_buffer(tensors):
     """If the 1-D tensors are consecutive views of one storage, the covering
     view; else None."""
-    if not tensors:
-        return None
-    first = tensors[0]
-    if first.dim() != 1 or not first.is_contiguous():
-        return None
-    dtype, base, size = first.dtype, first._base, first.element_size()
-    storage = None
-    at = first.data_ptr()
-    total = 0
-    for t in tensors:
-        if t.dtype != dtype or t.data_ptr() != at or t.dim() != 1 or not t.is_contiguous():
-            return None
-        if base is None or t._base is not base:  # not views of one tensor: of one storage all the same?
-            if storage is None:
-                storage = first.untyped_storage().data_ptr()
-            if t.untyped_storage().data_ptr() != storage:
-                return None
-        count = t.numel()
-        total += count
-        at += count * size
-    return torch.as_strided(first, (total,), (1,))
+    return _lib.host.one_buffer(tensors)

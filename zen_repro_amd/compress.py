@@ -35,13 +35,10 @@ def sample_threshold(tensor, sample_index, k):
         raise RuntimeError("sample_index must be int64")
     L = _lib.lib()
     dev = flat.device
-    s = sample_index.numel()
     code = _lib.dtype_code(flat)
-    thr = torch.empty(2, dtype=torch.int32, device=dev)
-    status = _lib.status_word(dev)
-    ws = _lib.scratch.get(dev, "sample_threshold", L.zen_sample_threshold_workspace(s, code))
-    rc = L.zen_sample_threshold(_lib.ptr(flat), code, flat.numel(), _lib.ptr(sample_index.reshape(-1)), s, int(k),
-                                _lib.ptr(thr), _lib.ptr(ws), ws.numel(), _lib.ptr(status), _lib.stream_of(dev))
+    ws = _lib.scratch.get(dev, "sample_threshold", L.zen_sample_threshold_workspace(sample_index.numel(), code))
+    rc, thr, status = _lib.host.sample_threshold(L.zen_sample_threshold, _lib.zeros.native(), flat, code, sample_index,
+                                                 int(k), ws, _lib.stream_of(dev))
     _lib.check(rc, "sample_threshold")
     return thr, status
 

@@ -40,16 +40,11 @@ def sparse_balance(tensor, memory, serial_memory, partitions, rehash):
 def fresh_tables(tensor, memory_size, serial_memory_size, partitions, rehash):
     """sparse_balance into two new tables of these sizes, checked (last_status): (memory, serial_memory)."""
     _check_input(tensor)
-    dev = tensor.device
-    memory = torch.empty(memory_size, dtype=torch.int32, device=dev)
-    serial_memory = torch.empty(serial_memory_size, dtype=torch.int32, device=dev)
-    offsets = torch.empty(partitions, dtype=torch.int32, device=dev)
-    status = _lib.status_word(dev)
+    L = _lib.lib()
     words = _lib.host_words(1)
-    rc = _lib.lib().zen_balance_tables(
-        _lib.ptr(tensor), _lib.dtype_code(tensor), tensor.numel(), _lib.ptr(memory), memory_size,
-        _lib.ptr(serial_memory), serial_memory_size, _lib.ptr(offsets), partitions, rehash, _lib.ptr(status), words.ptr,
-        words.words, _lib.stream_of(dev))
+    rc, memory, serial_memory, offsets, status = _lib.host.tables(
+        L.zen_balance_tables, _lib.zeros.native(), tensor, _lib.dtype_code(tensor), memory_size, serial_memory_size,
+        partitions, rehash, _lib.stream_of(tensor.device), words.ptr, words.words)
     _lib.check(rc, "sparse_balance")
     bits = words.view[1]
     _last.pending = _PendingStatus(status, offsets)

@@ -92,34 +92,23 @@ class TensorPartition:
 
     def _table_lists(self, flat, memory):
         L = _lib.lib()
-        dev = flat.device
         m, n = memory.numel(), flat.numel()
         parts = self.partitions
-        # beside the split sizes, the words in which the walk adds them up
-        splits, marks = _lib.zeros.take(dev, 3 * parts + 66, torch.int64).split((parts, 2 * parts + 66))
-        status = _lib.status_word(dev)
-        # not from the scratch cache: this thread may walk another table before these lists are used up
-        ws = torch.empty(L.zen_table_lists_workspace(m, parts), dtype=torch.uint8, device=dev)
-        if parts <= _lib.TABLE_SIZES_MOST:
-            words = _lib.host_words(parts + 1)
-            _lib.check(L.zen_table_find_sizes(_lib.ptr(memory), m, parts, n, _lib.ptr(splits), _lib.ptr(marks),
-                                              _lib.ptr(ws), ws.numel(), _lib.ptr(status), words.ptr, words.words,
-                                              _lib.stream_of(dev)), "table_find")
-            host = words.view[1:parts + 2]
-        else:
-            _lib.check(L.zen_table_find(_lib.ptr(memory), m, parts, n, _lib.ptr(splits), _lib.ptr(ws), ws.numel(),
-                                        _lib.ptr(status), _lib.stream_of(dev)), "table_find")
-            host = _lib.read_back(splits, status)
-        if host[-1]:
-            raise IndexError("get_sub_sparse_tensors: " + _lib.describe_status(host[-1]))
-        sizes = host[:-1]
-        total = sum(sizes)
-        idx = torch.empty(total, dtype=torch.int32, device=dev)
-        val = torch.empty(total, dtype=flat.dtype, device=dev)
-        _lib.check(L.zen_table_gather(_lib.ptr(memory), m, self.partitions, _lib.ptr(flat), _lib.dtype_code(flat), n,
-                                      _lib.ptr(idx), _lib.ptr(val), total, _lib.ptr(ws), ws.numel(),
-                                      _lib.stream_of(dev)), "table_gather")
-        return list(torch.split(idx, sizes)), list(torch.split(val, sizes)), splits
+        stream = _lib.stream_of(flat.device)
+        told = parts <= _lib.TABLE_SIZES_MOST
+        words = _lib.host_words(parts + 1) if told else None
+        rc, splits, status, ws = _lib.host.table_find(
+            L.zen_table_find_sizes if told else L.zen_table_find, _lib.zeros.native(), memory, parts, n,
+            L.zen_table_lists_workspace(m, parts), stream, *((words.ptr, words.words) if told else (0, 0)))
+        _lib.check(rc, "table_find")
+        host = words.view[1:parts + 2] if told else _lib.read_back(splits, status)
+        bits = host.pop()
+        if bits:
+            raise IndexError("get_sub_sparse_tensors: " + _lib.describe_status(bits))
+        rc, indices, values = _lib.host.table_gather(L.zen_table_gather, memory, flat, _lib.dtype_code(flat), host, ws,
+                                                     stream)
+        _lib.check(rc, "table_gather")
+        return indices, values, splits
 
     @staticmethod
     def _nonzero_int32(table):
@@ -385,10 +374,6 @@ class TensorPartition:
             mode |= self.fast_flags
         dev = flat.device
         L = _lib.lib()
-        out_idx = torch.empty(capacity, dtype=torch.int32, device=dev)
-        out_val = torch.empty(capacity, dtype=flat.dtype, device=dev)
-        splits = _lib.zeros.take(dev, self.partitions, torch.int64)
-        status = _lib.status_word(dev)
         nbytes = L.zen_load_balance_workspace(n, m, code, capacity, self.partitions)
         ws = _lib.scratch.get(dev, f"load_balance/{slot}", nbytes)
         kept = self._kept_table(dev, m, slot)
@@ -396,13 +381,10 @@ class TensorPartition:
         flags, used = self._take_ahead(flat, n, int(k), capacity, ws, slot, mode, thr, near)
         if near is not None and k > 0 and thr is None:
             thr, flags = near, flags | _lib.MODE_FLOOR
-        args = (_lib.ptr(flat), code, n, m, self.partitions, self.rehash, _lib.ptr(thr), int(k), _lib.ptr(thr_out),
-                _lib.ptr(out_idx), _lib.ptr(out_val), capacity, _lib.ptr(splits), _lib.ptr(table),
-                mode | flags | _lib.MODE_ZEROED, _lib.ptr(ws), ws.numel(), _lib.ptr(status))
-        if words is None:
-            rc = L.zen_load_balance(*args, _lib.stream_of(dev))
-        else:
-            rc = L.zen_load_balance_sizes(*args, words.ptr, words.words, _lib.stream_of(dev))
+        rc, out_idx, out_val, splits, status = _lib.host.load_balance(
+            L.zen_load_balance if words is None else L.zen_load_balance_sizes, _lib.zeros.native(), flat, code, m,
+            self.partitions, self.rehash, _lib.ptr(thr), int(k), _lib.ptr(thr_out), capacity, _lib.ptr(table),
+            mode | flags | _lib.MODE_ZEROED, ws, _lib.stream_of(dev), *((0, 0) if words is None else (words.ptr, words.words)))
         if words is not None:
             _lib.scratch.left_running(dev, f"load_balance/{slot}")
             kept.left_running(dev, flat)
@@ -438,8 +420,7 @@ class TensorPartition:
         while modes:
             words = _lib.host_words(self.partitions + 1)
             out_idx, out_val, splits, _ = self._fused(tensor, thr, capacity, k, modes[0], None, 0, None, words)
-            host = words.view[1:self.partitions + 2]
-            bits = host[-1]
+            bits = words.view[self.partitions + 1]
             if bits & (_lib.STAT_RETRY | _lib.STAT_INTERNAL):
                 # a declined or aborted call may leave entries and counters behind in the table
                 m, _ = self.table_sizes(n)
@@ -453,12 +434,11 @@ class TensorPartition:
             elif bits & _lib.STAT_CAPACITY and grow and capacity < n:
                 # more passed than allowed for (a fast path short of room declines, so this is mostly the general
                 # mode speaking): with more room the fast modes get their turn again
-                capacity = min(n, max(sum(host[:-1]) + 1024, capacity * 4))
+                capacity = min(n, max(sum(words.view[1:self.partitions + 1]) + 1024, capacity * 4))
                 modes = list(every)
             else:
                 break
         if bits:
             raise RuntimeError("load_balance: " + _lib.describe_status(bits))
-        sizes = host[:-1]
-        total = sum(sizes)
-        return list(torch.split(out_idx[:total], sizes)), list(torch.split(out_val[:total], sizes)), splits
+        indices, values = _lib.host.cut(out_idx, out_val, words.view[1:self.partitions + 1])
+        return indices, values, splits
