@@ -1024,6 +1024,57 @@ def test_load_balance_through_the_owner_table(zen, oracle, n, P, density, scale,
     assert not tp._table(d.device, m).any()
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("n,P,density,rehash", [
+    (9219, 4, 0.1, 3), (32768, 4, 0.6, 3),            # one workgroup: a list of selected indices, several of them
+    (49152, 3, 0.1, 3), (49151, 3, 0.1, 2),           # partitions that end with a stretch, and in front of its end
+    (1 << 18, 1000, 0.02, 3), (3000001, 16, 0.1, 1),  # dozens of partitions to a stretch; long serial tails
+])
+def test_owner_table_tells_the_host(zen, oracle, n, P, density, rehash, dtype):
+    """The calls that wait for the sizes, which the last kernel itself stores."""
+    g = make_grad(oracle, n, density, dtype, seed=n + 3 * P)
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, rehash)
+    assert st_o == 0
+    tp = zen.TensorPartition(P, 1, rehash)
+    d = to_dev(g)
+    for rep in range(2):
+        indices, values, splits = tp.load_balance(d)
+        assert [len(i) for i in indices] == list(splits_o) and np.array_equal(to_np(splits), splits_o)
+        assert np.array_equal(to_np(torch.cat(indices)), idx_o) and np.array_equal(to_np(torch.cat(values)), val_o)
+    with pytest.raises(RuntimeError, match="capacity"):
+        tp.load_balance(d, capacity=len(idx_o) - 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("r", [1, 1023, 1025, 4096, 6144, 6145])
+@pytest.mark.parametrize("n", [1, 1000, 262144, 262145, 2147483647])
+def test_merge_in_one_workgroup(zen, oracle, n, r, dtype):
+    """One workgroup up to 6144 entries, just beyond it the wide buckets or the sort; every entry on one index, few and many
+    of them; dense results of up to a megabyte, and longer ones."""
+    gen = torch.Generator().manual_seed(r + n % 1000)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    for spread in (1, min(n, 700), n):
+        idx = torch.randint(0, spread, (r,), generator=gen, dtype=torch.int64) * (n // spread) + (n - 1) % (n // spread)
+        val = (torch.randn(r, generator=gen) * 1e-3).to(dtype)
+        val[r // 2] = -0.0
+        which, place = np.unique(idx.numpy(), return_inverse=True)  # (the oracle's dense tensor: as long as needed)
+        w_idx, w_val = oracle.merge_sparse(place, to_np(val), len(which))
+        w_idx = which[w_idx]
+        d_idx, d_val = idx.cuda(), val.cuda()
+        m_idx, m_val = lba.merge_sparse(d_idx, d_val, n)
+        assert np.array_equal(to_np(m_idx), w_idx) and np.array_equal(to_np(m_val).view(np.uint32), w_val.view(np.uint32))
+        rounded = torch.from_numpy(w_val).to(dtype)
+        kept = rounded != 0
+        m_idx, m_val = lba.merge_rounded(d_idx.int(), d_val, n, dtype)
+        assert np.array_equal(to_np(m_idx), w_idx[kept.numpy()]) and torch.equal(m_val.cpu(), rounded[kept])
+        if n <= 262145:
+            want = torch.zeros(n, dtype=dtype)
+            want[torch.from_numpy(w_idx.astype(np.int64))] = rounded
+            assert torch.equal(lba.decode_sparse_tensors(d_idx, d_val, n).cpu(), want)
+            with pytest.raises(RuntimeError, match="range"):
+                lba.decode_sparse_tensors(torch.where(d_idx == d_idx[0], n, d_idx), d_val, n)
+
+
 @pytest.mark.parametrize("words", [1, 1023, 1024, (1 << 16) - 1, 1 << 16, (1 << 19) + 1])
 def test_read_back_of_any_length(zen, words):
     """Both types, a word and a list of `words` of them, up to and past what goes through the pinned buffer."""

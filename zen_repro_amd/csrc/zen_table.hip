@@ -8,23 +8,26 @@
 //                   smallest index that ever probes it; who takes a slot from a larger index continues that index's
 //                   probes, as in zen_balance.hip); an index that is out of levels takes a ticket of its partition's
 //                   serial region;
-//   k_table_count   occupied slots per stretch of the table;
-//   k_table_out     entries in slot order to their places, serial tails, split sizes; empties the table again.
+//   k_table_out     entries in slot order to their places (every stretch of the table says how many it holds, and adds up
+//                   what the ones before it said), serial tails, split sizes; empties the table again; tells the host.
 // Up to kOneSlots slots the table is kept in LDS and one workgroup does all of it (k_table_one).
-// Bound by latency: 1 Mi slots, 1 % selected: 5 + 3 + 5 us.
+// Bound by latency.
 #include "zen_balance.h"
 
 namespace zen {
 namespace {
 
 constexpr int kInsBlock = 512;
-constexpr int kOutBlock = 256;
+constexpr int kOutBlock = 1024;
 constexpr int kOutRows = 4;                                 // rows of 256 slots per wave
-constexpr uint32_t kStretch = kOutBlock / 64 * kOutRows * 256;  // slots per workgroup (4096)
+// Slots per workgroup: 16 384.  A workgroup draws a ticket, adds to a partition's size and counts itself as finished, all
+// on lines that take ten nanoseconds each time: with stretches of 4096 (256 threads) 4.1 M slots took 87 us, now 70.
+constexpr uint32_t kStretch = kOutBlock / 64 * kOutRows * 256;
 constexpr int kMaxParts = 1024;
 constexpr int kOneBlock = 1024;
 constexpr uint32_t kOneSlots = 32768;                       // 128 KB of LDS
 constexpr int kOneParts = 256;
+constexpr uint32_t kOneList = 4096;                         // selected indices side by side
 constexpr uint32_t kOneSerial = 3456;                       // more than a tenth of kOneSlots: more would be an overflow
 
 // Inserts index t.  Returns the index that ends up without a slot (0: none) and its partition.
@@ -58,22 +61,29 @@ struct Tables {
   uint32_t *slots;       // [m] the caller's table, zero between calls
   unsigned long long *splits;  // [P], zero: serial tickets in the upper halves while the indices are inserted
   uint32_t *serial;      // [P * ser_cap] indices without a slot
-  uint32_t *serial_n;    // [P]
-  uint32_t *found;       // [stretches]
+  unsigned long long *desc;  // [stretches] entries each holds, and behind them the words of `ticket` and `done`
+  uint32_t *ticket, *done;   // stretches taken, stretches finished
   uint32_t ser_cap;
   int parts;
   int64_t spp;           // serial slots of the reference's table, per partition
 };
 
+// Indices of partition p without a slot, as long as its tickets are in the upper half of its split size.
+__device__ inline uint32_t tickets(const Tables &tb, int p) {
+  const uint32_t s = (uint32_t)(__hip_atomic_load(&tb.splits[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32);
+  return s < tb.ser_cap ? s : tb.ser_cap;
+}
+
 template <typename S, bool ALIGNED>
 __global__ __launch_bounds__(kInsBlock) void k_table_insert(const S *__restrict__ in, int64_t n,
                                                             const uint32_t *__restrict__ thr, Probe g, Tables tb,
-                                                            int32_t *status) {
+                                                            uint32_t stretches, int32_t *status) {
   // the selected indices of the workgroup's stretch side by side, so that every thread has one to insert
   constexpr int V = VecOf<S>::kN;
   __shared__ uint32_t list[kInsBlock * V];
   __shared__ uint32_t count;
   if (threadIdx.x == 0) count = 0;
+  for (uint32_t i = blockIdx.x * kInsBlock + threadIdx.x; i <= stretches; i += gridDim.x * kInsBlock) tb.desc[i] = 0ull;
   const uint32_t least = least_key(thr, KeyOf<S>::kMask);
   const int64_t first = ((int64_t)blockIdx.x * kInsBlock + threadIdx.x) * V;
   S e[V];
@@ -121,94 +131,57 @@ __device__ inline uint32_t word_of(const uint4 &q, uint32_t e) {
   return e & 2u ? b : a;
 }
 
-__global__ __launch_bounds__(kOutBlock) void k_table_count(Tables tb, uint32_t m) {
-  __shared__ uint32_t part[kOutBlock / 64];
-  const uint32_t base = blockIdx.x * kStretch + (threadIdx.x >> 6) * (kOutRows * 256) + (uint32_t)lane_id() * 4;
-  uint32_t c = 0;
-#pragma unroll
-  for (int r = 0; r < kOutRows; ++r) c += (uint32_t)__popc(occupied(load_slots(tb.slots, base + r * 256, m)));
-  c = wave_sum(c);
-  if (lane_id() == 0) part[threadIdx.x >> 6] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t sum = 0;
-#pragma unroll
-    for (int w = 0; w < kOutBlock / 64; ++w) sum += part[w];
-    tb.found[blockIdx.x] = sum;
-  }
-  if (blockIdx.x == 0)  // the serial tickets leave the split sizes, which count the entries from here on
-    for (int p = threadIdx.x; p < tb.parts; p += kOutBlock) {
-      uint32_t s = (uint32_t)(tb.splits[p] >> 32);
-      if (s > tb.ser_cap) s = tb.ser_cap;
-      tb.serial_n[p] = s;
-      tb.splits[p] = s;
-    }
-}
-
+// Bound by the trips to memory: the slots, what the stretches before hold, the entries' values, the host.  The entries
+// are put side by side in LDS first, so that all of a stretch's values are on their way together (each thread's own
+// entries one after the other: 12 us for 145 000 bf16 slots, 10 % taken); with a kernel for the counts in front and one for
+// the host behind, a load balance of 300 000 bf16 elements took 46 us, of 2.2 M, 10 % selected, 74.
 template <typename S>
 __global__ __launch_bounds__(kOutBlock) void k_table_out(const S *__restrict__ dense, Tables tb, uint32_t m, uint32_t npp,
                                                          uint32_t stretches, int32_t *__restrict__ out_idx,
-                                                         S *__restrict__ out_val, uint32_t capacity, int32_t *status) {
+                                                         S *__restrict__ out_val, uint32_t capacity, HostAnswer answer,
+                                                         int32_t *status) {
   __shared__ uint32_t smem[kOutBlock / 64 + 1];
   __shared__ uint32_t before_part[kMaxParts + 1];  // serial entries of the partitions before
-  __shared__ uint32_t buf[kSerialLds];
+  __shared__ uint32_t buf[kStretch + kMaxParts];   // the stretch's entries and its partitions' counts, then a serial tail
   __shared__ uint32_t ends_at[kOutBlock];
-  const uint32_t c = blockIdx.x, wave = threadIdx.x >> 6, lane = (uint32_t)lane_id();
+  __shared__ uint32_t s_turn;
+  static_assert(kSerialLds <= kStretch + kMaxParts, "room for a tail");
+  uint32_t *held = buf + kStretch;
+  if (threadIdx.x == 0) s_turn = atomicAdd(tb.ticket, 1u);
+  __syncthreads();
+  const uint32_t c = s_turn;  // stretches are taken in order, so every earlier one already runs
+  if (c >= stretches) return;
+  const uint32_t wave = threadIdx.x >> 6, lane = (uint32_t)lane_id();
   const uint32_t base = c * kStretch + wave * (kOutRows * 256) + lane * 4;
   uint4 q[kOutRows];
 #pragma unroll
   for (int r = 0; r < kOutRows; ++r) q[r] = load_slots(tb.slots, base + r * 256, m);
   // The stretch's partitions, p_first to p_last.  Where it has several, their entries are counted in LDS (an add to the
   // split sizes for every entry of such a stretch: some 6000 of them queue on one line, 1.8 M fp32 slots, 5 % taken, 16
-  // partitions 27 us, now 8).
+  // partitions 27 us, then 8).
   const uint32_t lo = c * kStretch, hi = lo + kStretch < m ? lo + kStretch : m;  // lo < m
   const uint32_t p_first = lo / npp, p_last = (hi - 1u) / npp;
-  uint32_t *held = buf;
-  static_assert(kMaxParts <= (int)kSerialLds, "a counter for every partition");
   if (p_first != p_last)
     for (uint32_t i = threadIdx.x; i <= p_last - p_first; i += kOutBlock) held[i] = 0;
-  // entries in front of the stretch, and serial entries in front of every partition
-  uint32_t sum = 0, front;
-  for (uint32_t i = threadIdx.x; i < c; i += kOutBlock) sum += tb.found[i];
-  block_exclusive_scan<uint32_t, kOutBlock>(sum, smem, &front);
-  uint32_t carry = 0;
-  for (int p0 = 0; p0 < tb.parts; p0 += kOutBlock) {
-    const int p = p0 + (int)threadIdx.x;
-    const uint32_t s = p < tb.parts ? tb.serial_n[p] : 0u;
-    uint32_t total;
-    const uint32_t ex = block_exclusive_scan<uint32_t, kOutBlock>(s, smem, &total);
-    if (p < tb.parts) before_part[p] = carry + ex;
-    carry += total;
-  }
-  if (threadIdx.x == 0) before_part[tb.parts] = carry;
   uint32_t mine = 0;
 #pragma unroll
   for (int r = 0; r < kOutRows; ++r) mine += (uint32_t)__popc(occupied(q[r]));
   const uint32_t in_wave = wave_sum(mine);
   if (lane == 0) smem[wave] = in_wave;
   __syncthreads();
-  uint32_t at = front, all = 0;
+  uint32_t at = 0, all = 0;
 #pragma unroll
   for (uint32_t w = 0; w < kOutBlock / 64; ++w) {
     at += w < wave ? smem[w] : 0u;
     all += smem[w];
   }
+  if (threadIdx.x == 0) desc_store(&tb.desc[c], kDescAggregate | all);
 #pragma unroll
   for (int r = 0; r < kOutRows; ++r) {
     const uint32_t x = occupied(q[r]);
     const uint32_t n = (uint32_t)__popc(x), incl = wave_inclusive_scan(n);
     uint32_t pos = at + incl - n;
-    for (uint32_t bits = x; bits; bits &= bits - 1u, ++pos) {
-      const uint32_t e = (uint32_t)__ffs((int)bits) - 1u;
-      const uint32_t t = 0u - word_of(q[r], e);
-      const uint32_t p = p_first == p_last ? p_first : (base + r * 256 + e) / npp;
-      const uint32_t to = pos + before_part[p];
-      if (to < capacity) {
-        out_idx[to] = (int32_t)t;
-        out_val[to] = dense[t];
-      }
-      if (p_first != p_last) atomicAdd(&held[p - p_first], 1u);
-    }
+    for (uint32_t bits = x; bits; bits &= bits - 1u, ++pos) buf[pos] = 0u - word_of(q[r], (uint32_t)__ffs((int)bits) - 1u);
     at += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
     if (x) {  // leave the table empty again
       const uint32_t s0 = base + r * 256;
@@ -217,6 +190,48 @@ __global__ __launch_bounds__(kOutBlock) void k_table_out(const S *__restrict__ d
       } else {
         for (uint32_t i = 0; s0 + i < m; ++i) tb.slots[s0 + i] = 0;
       }
+    }
+  }
+  // entries in front of the stretch (bounded waits), and serial entries in front of every partition
+  uint32_t sum = 0, front;
+  for (uint32_t i = threadIdx.x; i < c; i += kOutBlock) {
+    uint64_t d = desc_load(&tb.desc[i]);
+    uint32_t spins = 0;
+    while ((d >> 62) == 0) {
+      if (++spins > kSpinLimit) {
+        atomicOr(status, ZEN_STAT_INTERNAL);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(2);
+      d = desc_load(&tb.desc[i]);
+    }
+    sum += (uint32_t)(d & kDescValue);
+  }
+  __syncthreads();  // (smem has been read)
+  block_exclusive_scan<uint32_t, kOutBlock>(sum, smem, &front);
+  uint32_t carry = 0;
+  for (int p0 = 0; p0 < tb.parts; p0 += kOutBlock) {
+    const int p = p0 + (int)threadIdx.x;
+    const uint32_t s = p < tb.parts ? tickets(tb, p) : 0u;
+    uint32_t total;
+    const uint32_t ex = block_exclusive_scan<uint32_t, kOutBlock>(s, smem, &total);
+    if (p < tb.parts) before_part[p] = carry + ex;
+    carry += total;
+  }
+  if (threadIdx.x == 0) before_part[tb.parts] = carry;
+  __syncthreads();
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < all; i += kOutBlock) {
+    const uint32_t t = buf[i];
+    uint32_t p = p_first;
+    if (p_first != p_last) {  // (an index stays in the partition of its first slot)
+      p = (poly(t) + kSeed1) % m / npp;
+      atomicAdd(&held[p - p_first], 1u);
+    }
+    const uint32_t to = front + i + before_part[p];
+    if (to < capacity) {
+      out_idx[to] = (int32_t)t;
+      out_val[to] = dense[t];
     }
   }
   if (p_first == p_last) {
@@ -254,6 +269,23 @@ __global__ __launch_bounds__(kOutBlock) void k_table_out(const S *__restrict__ d
       __syncthreads();
     }
   }
+  // the stretch that finishes last turns tickets and counts into the split sizes
+  wait_global_acks();
+  __syncthreads();
+  if (threadIdx.x == 0) s_turn = atomicAdd(tb.done, 1u);
+  __syncthreads();
+  if (s_turn != stretches - 1u) return;
+  for (int p = threadIdx.x; p < tb.parts; p += kOutBlock) {
+    const unsigned long long both = __hip_atomic_load(&tb.splits[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int64_t size = (int64_t)(both & 0xffffffffull) + (int64_t)tickets(tb, p);
+    tb.splits[p] = (unsigned long long)size;
+    if (answer.host) host_store(answer.host + 1 + p, size);
+  }
+  if (answer.host) {
+    if (threadIdx.x == 0)
+      host_store(answer.host + 1 + tb.parts, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    host_answered(answer);
+  }
 }
 
 template <typename S, bool ALIGNED>
@@ -267,6 +299,7 @@ __global__ __launch_bounds__(kOneBlock) void k_table_one(const S *__restrict__ i
   __shared__ uint32_t serial[kOneSerial];       // partition << 15 | index
   __shared__ uint32_t held[kOneParts], left[kOneParts], before_left[kOneParts];
   __shared__ uint32_t smem[kOneBlock / 64 + 1];
+  __shared__ uint16_t list[kOneList];
   __shared__ uint32_t serial_n;
   const uint32_t m = g.m;
   const uint32_t words = (m + 3u) / 4u * 4u;
@@ -274,29 +307,54 @@ __global__ __launch_bounds__(kOneBlock) void k_table_one(const S *__restrict__ i
   if (threadIdx.x < kOneParts) held[threadIdx.x] = left[threadIdx.x] = 0;
   if (threadIdx.x == 0) serial_n = 0;
   const uint32_t least = least_key(thr, KeyOf<S>::kMask);
-  __syncthreads();
-  for (uint32_t first = threadIdx.x * V; first < n; first += kOneBlock * V) {
-    S e[V];
-    load_vec<S, ALIGNED>(in, first, n, e);
-#pragma unroll 1
-    for (int i = 0; i < V; ++i) {
-      const uint32_t t = first + (uint32_t)i;
-      if ((uint32_t)(e[0] & KeyOf<S>::kMask) >= least && t != 0) {
-        uint32_t part;
-        const uint32_t out = insert(slots, g, t, &part);
-        if (out) {
-          const uint32_t at = atomicAdd(&serial_n, 1u);
-          if (at < kOneSerial) {
-            serial[at] = (part << 15) | out;
-            atomicAdd(&left[part], 1u);
-          } else {
-            atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);  // some partition has more than its tenth
-          }
+  // All of the tensor is asked for at once; then the selected indices side by side, so that every thread has one to insert
+  // (9219 bf16 elements, 10 % selected: 16 us, 7.7 of them here, with a round of this for every 4096 elements; 17.6 with
+  // every thread inserting its own elements one after the other).
+  constexpr int kRows = (int)(kOneSlots / (kOneBlock * V));
+  uint32_t flags[kRows];
+  uint32_t mine_n = 0;
+  {
+    S e[kRows][V];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      const uint32_t first = ((uint32_t)r * kOneBlock + threadIdx.x) * V;
+      if ((uint32_t)r * kOneBlock * V < n) load_vec<S, ALIGNED>(in, first, n, e[r]);  // (places past the end: zeros)
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      flags[r] = 0;
+      if ((uint32_t)r * kOneBlock * V < n) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) flags[r] |= (uint32_t)((uint32_t)(e[r][i] & KeyOf<S>::kMask) >= least) << i;
+      }
+      if (r == 0 && threadIdx.x == 0) flags[r] &= ~1u;  // index 0 is never transmitted
+      mine_n += (uint32_t)__popc(flags[r]);
+    }
+  }
+  uint32_t selected;
+  const uint32_t ahead = block_exclusive_scan<uint32_t, kOneBlock>(mine_n, smem, &selected);  // (its barriers: the slots are empty)
+  for (uint32_t from = 0; from < selected; from += kOneList) {
+    uint32_t at = ahead;
+#pragma unroll
+    for (int r = 0; r < kRows; ++r)
+      for (uint32_t bits = flags[r]; bits; bits &= bits - 1u, ++at)
+        if (at - from < kOneList) list[at - from] = (uint16_t)(((uint32_t)r * kOneBlock + threadIdx.x) * V + (uint32_t)__ffs((int)bits) - 1u);
+    __syncthreads();
+    const uint32_t listed = selected - from < kOneList ? selected - from : kOneList;
+    for (uint32_t i = threadIdx.x; i < listed; i += kOneBlock) {
+      uint32_t part;
+      const uint32_t out = insert(slots, g, list[i], &part);
+      if (out) {
+        const uint32_t place = atomicAdd(&serial_n, 1u);
+        if (place < kOneSerial) {
+          serial[place] = (part << 15) | out;
+          atomicAdd(&left[part], 1u);
+        } else {
+          atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);  // some partition has more than its tenth
         }
       }
-#pragma unroll
-      for (int j = 0; j + 1 < V; ++j) e[j] = e[j + 1];  // (the loop's body once, not once per element)
     }
+    __syncthreads();
   }
   __syncthreads();
   const uint32_t total_left = serial_n < kOneSerial ? serial_n : kOneSerial;
@@ -324,22 +382,26 @@ __global__ __launch_bounds__(kOneBlock) void k_table_one(const S *__restrict__ i
     at += w < wave ? smem[w] : 0u;
     all += smem[w];
   }
+  // a wave puts its entries side by side at the head of its own slots (which it has read by then), ...
+  uint32_t put = 0;
   for (uint32_t r = 0; r < rows; ++r) {
     const uint32_t s0 = base + r * 256;
     const uint4 q = s0 < words ? *reinterpret_cast<const uint4 *>(slots + s0) : make_uint4(0, 0, 0, 0);
     const uint32_t x = occupied(q), c = (uint32_t)__popc(x), incl = wave_inclusive_scan(c);
-    uint32_t pos = at + incl - c;
-    for (uint32_t bits = x; bits; bits &= bits - 1u, ++pos) {
-      const uint32_t e = (uint32_t)__ffs((int)bits) - 1u;
-      const uint32_t t = 0u - word_of(q, e), p = (s0 + e) / g.npp;
-      atomicAdd(&held[p], 1u);
-      const uint32_t to = pos + before_left[p];
-      if (to < capacity) {
-        out_idx[to] = (int32_t)t;
-        out_val[to] = in[t];
-      }
+    uint32_t pos = wave * rows * 256 + put + incl - c;
+    __builtin_amdgcn_wave_barrier();  // (the row is read by all lanes before any of them writes)
+    for (uint32_t bits = x; bits; bits &= bits - 1u, ++pos) slots[pos] = 0u - word_of(q, (uint32_t)__ffs((int)bits) - 1u);
+    put += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+  }
+  // ... and takes them to their places, all values on their way together
+  for (uint32_t i = lane; i < in_wave; i += 64) {
+    const uint32_t t = slots[wave * rows * 256 + i], p = (poly(t) + kSeed1) % m / g.npp;  // (it stays in its first slot's partition)
+    atomicAdd(&held[p], 1u);
+    const uint32_t to = at + i + before_left[p];
+    if (to < capacity) {
+      out_idx[to] = (int32_t)t;
+      out_val[to] = in[t];
     }
-    at += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
   }
   __syncthreads();
   {
@@ -386,8 +448,9 @@ TablePlan plan_table(void *workspace, int64_t n, int64_t m, int dtype, int parti
   const int64_t spp = n / partitions / 10;
   p.tb.ser_cap = (uint32_t)(spp > 64 ? spp : 64);
   p.tb.serial = cv.take<uint32_t>((size_t)p.tb.ser_cap * partitions);
-  p.tb.serial_n = cv.take<uint32_t>((size_t)partitions);
-  p.tb.found = cv.take<uint32_t>(p.stretches);
+  p.tb.desc = cv.take<unsigned long long>((size_t)p.stretches + 1);
+  p.tb.ticket = reinterpret_cast<uint32_t *>(p.tb.desc + p.stretches);
+  p.tb.done = p.tb.ticket + 1;
   p.topk = cv.take<char>(topk_whole_bytes(n, dtype));
   p.tb.parts = partitions;
   p.tb.spp = spp;
@@ -409,13 +472,12 @@ int table_launch(const SlabBalanceArgs &a, const TablePlan &p, const uint32_t *t
   }
   if (!zeroed) launch_fill<int64_t>(a.splits, 0, (size_t)a.partitions, s);
   const int64_t blocks = ceil_div(a.n, (int64_t)kInsBlock * VecOf<S>::kN);
-  k_table_insert<S, ALIGNED><<<dim3((unsigned)blocks), dim3(kInsBlock), 0, s>>>(in, a.n, thr, a.g, p.tb, a.status);
+  k_table_insert<S, ALIGNED><<<dim3((unsigned)blocks), dim3(kInsBlock), 0, s>>>(in, a.n, thr, a.g, p.tb, p.stretches, a.status);
   ZEN_LAUNCH_CHECK("k_table_insert");
-  k_table_count<<<dim3(p.stretches), dim3(kOutBlock), 0, s>>>(p.tb, a.g.m);
-  ZEN_LAUNCH_CHECK("k_table_count");
   k_table_out<S><<<dim3(p.stretches), dim3(kOutBlock), 0, s>>>(in, p.tb, a.g.m, a.g.npp, p.stretches, a.out_idx, out_val,
-                                                              (uint32_t)a.capacity, a.status);
+                                                              (uint32_t)a.capacity, a.ask.answer, a.status);
   ZEN_LAUNCH_CHECK("k_table_out");
+  if (a.ask.answer.host) *a.ask.answered = true;
   return ZEN_OK;
 }
 
