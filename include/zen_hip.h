@@ -376,7 +376,7 @@ int zen_load_balance_path(int64_t n, int64_t m, int dtype, int64_t capacity, int
  */
 size_t zen_merge_workspace(int64_t r, int64_t dense_n);
 size_t zen_merge_zero_bytes(void); /* see ZEN_MODE_ZEROED; the same for every r and dense_n */
-/* 0 = radix sort (general mode) or, in the fast mode, one workgroup for lists of up to 4096 entries, 1 = one bucket
+/* 0 = radix sort (general mode) or, in the fast mode, one workgroup for lists of up to 6144 entries, 1 = one bucket
    pass + per-range sorts, 2 = bucket slabs, 3 = wide buckets; see zen_load_balance_path */
 int zen_merge_path(int64_t r, int64_t dense_n, int mode);
 int zen_merge(const void *idx, int idx64_in, const void *val, int dtype,

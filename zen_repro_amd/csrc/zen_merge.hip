@@ -201,6 +201,77 @@ struct MergeSink {
   }
 };
 
+// The sums of a workgroup's n sorted records (indices in sh.key, value bits in sh.tie), in registers: record q of a thread
+// ends a run of equal indices, whose sum is kept, where bit q of the answer is set.
+template <typename O, typename Shared>
+__device__ inline uint32_t sum_runs(const Shared &sh, uint32_t n, uint32_t (&k)[kMergeItems], float (&sum)[kMergeItems]) {
+  // Thread t owns the sorted places [t * per, (t + 1) * per): as few per thread as cover the bucket (and an odd
+  // number, which keeps the lanes of a wave on different LDS banks).  It fetches them all at once and walks
+  // through them in registers.  A run of equal indices is summed in arrival order from +0 (like the dense
+  // tensor of comm.py:35) and belongs to the thread that holds its last record; where that run began before
+  // the thread's first place (rare: runs are short next to `per`, long ones come from payloads that overlap),
+  // the part in front is summed first, from the run's head on.
+  const uint32_t per = ((n + kMergeBlock - 1) / kMergeBlock) | 1u;  // <= kMergeItems
+  const uint32_t first = threadIdx.x * per;
+  uint32_t keep = 0;
+  {
+    constexpr uint32_t kNoKey = 0xffffffffu;  // offsets are below the bucket width
+    float v[kMergeItems];
+#pragma unroll
+    for (int q = 0; q < kMergeItems; ++q) {
+      const uint32_t p = first + q;
+      const bool have = (uint32_t)q < per && p < n;
+      const uint32_t from = have ? p : 0u;
+      k[q] = sh.key[from];
+      v[q] = __uint_as_float(sh.tie[from]);
+      if (!have) k[q] = kNoKey;
+    }
+    const uint32_t before_k = first > 0 && first < n ? sh.key[first - 1] : kNoKey;
+    const uint32_t after_k = first + per < n ? sh.key[first + per] : kNoKey;
+    float acc = 0.0f;
+    if (first < n && before_k == k[0]) {
+      // the run began before this thread's places: find its head, sum up to the place in front of `first`
+      uint32_t head = first - 1;
+      while (head > 0) {
+        const uint32_t a0 = sh.key[head - 1];
+        const uint32_t a1 = sh.key[head >= 2 ? head - 2 : 0u];
+        const uint32_t a2 = sh.key[head >= 3 ? head - 3 : 0u];
+        const uint32_t a3 = sh.key[head >= 4 ? head - 4 : 0u];
+        if (a0 != before_k) break;
+        if (head < 2 || a1 != before_k) { head -= 1; break; }
+        if (head < 3 || a2 != before_k) { head -= 2; break; }
+        if (head < 4 || a3 != before_k) { head -= 3; break; }
+        head -= 4;
+      }
+      for (uint32_t u = head; u < first; u += 4) {
+        const float f0 = __uint_as_float(sh.tie[u]);
+        const float f1 = __uint_as_float(sh.tie[u + 1 < first ? u + 1 : u]);
+        const float f2 = __uint_as_float(sh.tie[u + 2 < first ? u + 2 : u]);
+        const float f3 = __uint_as_float(sh.tie[u + 3 < first ? u + 3 : u]);
+        acc += f0;
+        if (u + 1 < first) acc += f1;
+        if (u + 2 < first) acc += f2;
+        if (u + 3 < first) acc += f3;
+      }
+    }
+    uint32_t prev = before_k;
+#pragma unroll
+    for (int q = 0; q < kMergeItems; ++q) {
+      const uint32_t next = q + 1 < kMergeItems ? ((uint32_t)(q + 1) < per ? k[q + 1] : after_k) : after_k;
+      if (k[q] != kNoKey) {
+        if (k[q] != prev) acc = 0.0f;
+        acc += v[q];
+        prev = k[q];
+        sum[q] = acc;
+        if (k[q] != next && SumAs<O>::kept(acc)) keep |= 1u << q;
+      } else {
+        sum[q] = 0.0f;
+      }
+    }
+  }
+  return keep;
+}
+
 template <typename I, typename S, typename O>
 __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, uint32_t *__restrict__ cursor,
                                                              uint32_t *__restrict__ coarse_cursor,
@@ -264,72 +335,9 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
     }
   }
   __syncthreads();
-  // Thread t owns the sorted places [t * per, (t + 1) * per): as few per thread as cover the bucket (and an odd
-  // number, which keeps the lanes of a wave on different LDS banks).  It fetches them all at once and walks
-  // through them in registers.  A run of equal indices is summed in arrival order from +0 (like the dense
-  // tensor of comm.py:35) and belongs to the thread that holds its last record; where that run began before
-  // the thread's first place (rare: runs are short next to `per`, long ones come from payloads that overlap),
-  // the part in front is summed first, from the run's head on.
-  const uint32_t per = ((n + kMergeBlock - 1) / kMergeBlock) | 1u;  // <= kMergeItems
-  const uint32_t first = threadIdx.x * per;
   uint32_t k[kMergeItems];
   float sum[kMergeItems];
-  uint32_t keep = 0;
-  {
-    constexpr uint32_t kNoKey = 0xffffffffu;  // offsets are below the bucket width
-    float v[kMergeItems];
-#pragma unroll
-    for (int q = 0; q < kMergeItems; ++q) {
-      const uint32_t p = first + q;
-      const bool have = (uint32_t)q < per && p < n;
-      const uint32_t from = have ? p : 0u;
-      k[q] = sh.key[from];
-      v[q] = __uint_as_float(sh.tie[from]);
-      if (!have) k[q] = kNoKey;
-    }
-    const uint32_t before_k = first > 0 && first < n ? sh.key[first - 1] : kNoKey;
-    const uint32_t after_k = first + per < n ? sh.key[first + per] : kNoKey;
-    float acc = 0.0f;
-    if (first < n && before_k == k[0]) {
-      // the run began before this thread's places: find its head, sum up to the place in front of `first`
-      uint32_t head = first - 1;
-      while (head > 0) {
-        const uint32_t a0 = sh.key[head - 1];
-        const uint32_t a1 = sh.key[head >= 2 ? head - 2 : 0u];
-        const uint32_t a2 = sh.key[head >= 3 ? head - 3 : 0u];
-        const uint32_t a3 = sh.key[head >= 4 ? head - 4 : 0u];
-        if (a0 != before_k) break;
-        if (head < 2 || a1 != before_k) { head -= 1; break; }
-        if (head < 3 || a2 != before_k) { head -= 2; break; }
-        if (head < 4 || a3 != before_k) { head -= 3; break; }
-        head -= 4;
-      }
-      for (uint32_t u = head; u < first; u += 4) {
-        const float f0 = __uint_as_float(sh.tie[u]);
-        const float f1 = __uint_as_float(sh.tie[u + 1 < first ? u + 1 : u]);
-        const float f2 = __uint_as_float(sh.tie[u + 2 < first ? u + 2 : u]);
-        const float f3 = __uint_as_float(sh.tie[u + 3 < first ? u + 3 : u]);
-        acc += f0;
-        if (u + 1 < first) acc += f1;
-        if (u + 2 < first) acc += f2;
-        if (u + 3 < first) acc += f3;
-      }
-    }
-    uint32_t prev = before_k;
-#pragma unroll
-    for (int q = 0; q < kMergeItems; ++q) {
-      const uint32_t next = q + 1 < kMergeItems ? ((uint32_t)(q + 1) < per ? k[q + 1] : after_k) : after_k;
-      if (k[q] != kNoKey) {
-        if (k[q] != prev) acc = 0.0f;
-        acc += v[q];
-        prev = k[q];
-        sum[q] = acc;
-        if (k[q] != next && SumAs<O>::kept(acc)) keep |= 1u << q;
-      } else {
-        sum[q] = 0.0f;
-      }
-    }
-  }
+  const uint32_t keep = sum_runs<O>(sh, n, k, sum);
   uint32_t total;
   const uint32_t before = block_exclusive_scan<uint32_t, kMergeBlock>((uint32_t)__popc(keep), sh.scan, &total);
   // where this bucket's output starts: the sum of what all earlier buckets keep.  Every thread asks for a
@@ -399,6 +407,137 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
     }
     host_answer_count(answer, out_count, status);
   }
+}
+
+// A short list in one workgroup, straight from where it lies: no slabs, no zeroed memory, any indices (a narrow range takes
+// whatever comes).  DENSE: out_val is the dense tensor, written whole.  Bound by the chain of its phases, LDS round trips
+// and three trips to memory: a rounded merge of 1000 entries 27 us a call (38 on the tables of the wide buckets, which are
+// laid out for 16 384).
+struct MergeOneShared : SlabSortShared {
+  static constexpr uint32_t kLimit = kSlabCap;
+};
+
+template <typename I, typename S, typename O, bool DENSE>
+__global__ __launch_bounds__(kMergeBlock) void k_merge_one(SlabGeom geo, const void *__restrict__ idx, int idx64,
+                                                           const S *__restrict__ val, uint32_t r, uint32_t dense_n,
+                                                           I *__restrict__ out_idx, O *__restrict__ out_val, int64_t capacity,
+                                                           int tie_bits, int64_t *out_count, HostAnswer answer, int32_t *status) {
+  __shared__ MergeOneShared sh;
+  uint32_t off[kMergeRecs], arr[kMergeRecs], rank[kMergeRecs];
+  S v[kMergeRecs];
+  uint32_t live = 0;
+  {
+    int64_t at[kMergeRecs];
+#pragma unroll
+    for (int i = 0; i < kMergeRecs; ++i) {
+      const uint32_t j = threadIdx.x + i * kMergeBlock;
+      at[i] = 0;
+      v[i] = 0;
+      if ((uint32_t)(i * kMergeBlock) >= r) continue;  // the same for the whole workgroup
+      const uint32_t e = j < r ? j : 0u;
+      at[i] = idx64 ? static_cast<const int64_t *>(idx)[e] : (int64_t)static_cast<const int32_t *>(idx)[e];
+      v[i] = val[e];
+    }
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kMergeRecs; ++i) {
+      const uint32_t j = threadIdx.x + i * kMergeBlock;
+      const bool good = at[i] >= 0 && at[i] < (int64_t)dense_n;
+      off[i] = good ? (uint32_t)at[i] : 0u;
+      arr[i] = j;
+      if (j < r && good) live |= 1u << i;
+      bad |= j < r && !good;
+    }
+    if (bad) atomicOr(status, ZEN_STAT_BAD_INDEX);  // skipped
+  }
+  if (DENSE) {  // zeros, while the records are ranked
+    constexpr uint32_t V = 16 / sizeof(O);
+    const uint32_t skew = (uint32_t)((reinterpret_cast<uintptr_t>(out_val) & 15u) / sizeof(O));
+    uint32_t head = (V - skew) % V;
+    if (head > dense_n) head = dense_n;
+    const uint32_t vecs = (dense_n - head) / V;
+    const u32x4 zero = {0, 0, 0, 0};
+    u32x4 *to = reinterpret_cast<u32x4 *>(out_val + head);
+    for (uint32_t i = threadIdx.x; i < vecs; i += kMergeBlock) to[i] = zero;
+    if (threadIdx.x < head) out_val[threadIdx.x] = O(0);
+    for (uint32_t i = head + vecs * V + threadIdx.x; i < dense_n; i += kMergeBlock) out_val[i] = O(0);
+  }
+  uint32_t n = 0;
+  (void)slab_rank<kMergeBlock>(sh, geo, tie_bits, off, arr, live, rank, &n);  // (never declined: no group is beyond the limit)
+#pragma unroll
+  for (int i = 0; i < kMergeRecs; ++i) {
+    if (live & (1u << i)) {
+      sh.key[rank[i]] = off[i];
+      sh.tie[rank[i]] = __float_as_uint(KeyOf<S>::to_f32(v[i]));
+    }
+  }
+  __syncthreads();
+  uint32_t k[kMergeItems];
+  float sum[kMergeItems];
+  // (a dense tensor takes every sum that is not zero, also one that rounds to -0)
+  const uint32_t keep = DENSE ? sum_runs<float>(sh, n, k, sum) : sum_runs<O>(sh, n, k, sum);
+  uint32_t total;
+  if (DENSE) wait_global_acks();  // this wave's zeros are written (the scan's barriers: everybody's)
+  uint32_t at = block_exclusive_scan<uint32_t, kMergeBlock>((uint32_t)__popc(keep), sh.scan, &total);
+#pragma unroll
+  for (int q = 0; q < kMergeItems; ++q) {
+    if (keep & (1u << q)) {
+      if (DENSE) {
+        out_val[k[q]] = SumAs<O>::of(sum[q]);
+      } else {
+        sh.key[at] = k[q];
+        sh.tie[at] = __float_as_uint(sum[q]);
+        ++at;
+      }
+    }
+  }
+  if (!DENSE) {
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < total; i += kMergeBlock) {
+      if ((int64_t)i < capacity) {
+        out_idx[i] = (I)sh.key[i];
+        out_val[i] = SumAs<O>::of(__uint_as_float(sh.tie[i]));
+      }
+    }
+    if (threadIdx.x == 0) {
+      *out_count = (int64_t)total;
+      if ((int64_t)total > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
+    }
+  }
+  if (answer.host) {
+    wait_global_acks();  // its share of the status word, and the count
+    __syncthreads();
+    host_answer_count(answer, DENSE ? nullptr : out_count, status);
+  }
+}
+
+// Entries up to which one workgroup does it all: as many as fit (6144 of them 28 to 36 us a dense call, in the wide
+// buckets' two launches 39).
+constexpr int64_t kMergeOneMax = merge_one_max();
+static_assert(kMergeOneMax <= kSlabCap, "the records fit");
+
+template <typename S, typename O>
+int merge_one_launch(const void *idx, int idx64_in, const S *val, int64_t r, int64_t dense_n, void *out_idx, int idx64_out,
+                     O *out_val, int64_t capacity, int64_t *out_count, int32_t *status, hipStream_t s, const HostAsk &ask) {
+  SlabGeom geo{};
+  while ((dense_n >> geo.sub_shift) >= kSlabSubs) ++geo.sub_shift;  // 19 at most: with 13 bits of arrival number a word
+  const int tie_bits = ceil_log2_u64((uint64_t)r);
+  const dim3 grid(1), block(kMergeBlock);
+  ProfScope prof(kProfWideMerge, s);
+#define ZEN_ONE(I, DENSE)                                                                                             \
+  k_merge_one<I, S, O, DENSE><<<grid, block, 0, s>>>(geo, idx, idx64_in, val, (uint32_t)r, (uint32_t)dense_n,         \
+                                                     static_cast<I *>(out_idx), out_val, capacity, tie_bits, out_count, \
+                                                     ask.answer, status)
+  if (!out_idx)
+    ZEN_ONE(int32_t, true);
+  else if (idx64_out)
+    ZEN_ONE(int64_t, false);
+  else
+    ZEN_ONE(int32_t, false);
+#undef ZEN_ONE
+  ZEN_LAUNCH_CHECK("k_merge_one");
+  if (ask.answer.host) *ask.answered = true;
+  return ZEN_OK;
 }
 
 // Memory that must be zero when a merge starts: the prefix state over the buckets and the scatter kernels'
@@ -512,7 +651,7 @@ MergePlan plan_merge(void *workspace, int64_t r, int64_t dense_n) {
 }
 
 // Whether a call with these sizes goes to one workgroup, to the wide buckets.
-bool takes_one(int64_t r, int mode) { return (mode & 0xff) == ZEN_MODE_FAST && r <= wide_merge_one_max(); }
+bool takes_one(int64_t r, int mode) { return (mode & 0xff) == ZEN_MODE_FAST && r <= kMergeOneMax; }
 bool takes_wide(int64_t r, int64_t dense_n, int mode) {
   return (mode & ~ZEN_MODE_ZEROED) == ZEN_MODE_FAST && wide_merge_fits(r, dense_n, wide_device_cus(), nullptr);
 }
@@ -529,8 +668,7 @@ int merge_launch(const void *idx, int idx64_in, const S *val, int64_t r, int64_t
                  int32_t *status, hipStream_t s, const HostAsk &ask = {}) {
   const bool zeroed = (mode & ZEN_MODE_ZEROED) != 0;
   if (takes_one(r, mode))
-    return wide_merge_one(idx, idx64_in, val, sizeof(S) == 2 ? ZEN_BF16 : ZEN_F32, r, dense_n, out_idx, idx64_out, out_val,
-                          sizeof(O) == 2 ? ZEN_BF16 : ZEN_F32, capacity, out_count, status, s, ask);
+    return merge_one_launch(idx, idx64_in, val, r, dense_n, out_idx, idx64_out, out_val, capacity, out_count, status, s, ask);
   const bool wide = takes_wide(r, dense_n, mode);
   mode &= ~(ZEN_MODE_ZEROED | ZEN_MODE_SLABS);
   SlabGeom geo;

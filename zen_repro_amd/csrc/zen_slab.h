@@ -159,6 +159,7 @@ constexpr int kSlabInline = 4;                            // groups up to this s
 constexpr int kSlabQueueMin = 256;                        // records in larger groups below which nothing is set aside
 struct SlabSortShared {
   static constexpr bool kQueue = true;
+  static constexpr uint32_t kLimit = kSlabGroupLimit;
   uint32_t key[kSlabCap];
   union {
     uint32_t tie[kSlabCap];
@@ -175,6 +176,7 @@ static_assert(kSlabSubs + 1 <= kSlabCap, "the counters fit under the ties");
 // The same without the queue (whose code costs slab_rank registers).
 struct SlabSortSharedNoQueue {
   static constexpr bool kQueue = false;
+  static constexpr uint32_t kLimit = kSlabGroupLimit;
   uint32_t key[kSlabCap];
   union {
     uint32_t tie[kSlabCap];
@@ -244,7 +246,7 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
     for (int e = 0; e < kSubsPer; ++e) {
       c[e] = sh.cnt[e * BLOCK + threadIdx.x];
       sum += c[e] + (c[e] > (uint32_t)kSlabInline ? c[e] << 16 : 0u);
-      big |= c[e] > (uint32_t)kSlabGroupLimit;
+      big |= c[e] > Shared::kLimit;
     }
     if (big) sh.bad = 1;
     uint32_t total;
@@ -273,7 +275,7 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
       word[i] = ((off[i] & low_mask) << tie_bits) | tie[i];
       sh.key[g0[i] + at[i]] = word[i];
       if constexpr (Shared::kQueue) {
-        static_assert(kSlabSubs <= (1 << 12) && kSlabGroupLimit <= (1 << 19), "a queue entry is one word");
+        static_assert(kSlabSubs <= (1 << 12) && Shared::kLimit <= (1u << 19), "a queue entry is one word");
         const uint32_t q = (here >> 16) + at[i];
         if (set_aside && g1[i] - g0[i] > (uint32_t)kSlabInline && q < (uint32_t)kSlabQueueCap) {
           sh.queue[q] = sub[i] | (at[i] << 12);  // sub < 2^12, at < group size <= kSlabGroupLimit

@@ -295,12 +295,8 @@ bool wide_merge_fits(int64_t r, int64_t dense_n, int cus, SlabGeom *geo, bool al
 size_t wide_merge_bytes(int64_t r, int64_t dense_n, int cus);
 bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, int64_t dense_n, uint32_t *cursor,
                      void *rest, int cus, int32_t *status, WideList *list, bool alone);
-// One workgroup straight from the list, for up to wide_merge_one_max() entries (kWideCap would fit; from about here
-// on the scatter's launch costs less than the longer chains of one workgroup): no slabs, no zeroed memory.
-constexpr int64_t wide_merge_one_max() { return 4096; }
-int wide_merge_one(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n, void *out_idx,
-                   int idx64_out, void *out_val, int out_dtype, int64_t capacity, int64_t *out_count, int32_t *status,
-                   hipStream_t s, const HostAsk &ask = {});
+// Lists up to this long take one workgroup (zen_merge.hip).
+constexpr int64_t merge_one_max() { return 6144; }
 int wide_merge(const WideList &list, int dtype, void *out_idx, int idx64_out, void *out_val, int out_dtype,
                int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s, const HostAsk &ask = {});
 

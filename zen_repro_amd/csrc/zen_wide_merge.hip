@@ -66,8 +66,7 @@ struct WideMergeShared {
 // end (62 M bf16 elements, 3.1 M entries: 60 us; 69 with the zeros in front of the records' loads, which then wait for
 // them to be written; the fill and scatter kernels in front of and behind a sparse merge took 18 + 21 us.  Workgroups
 // of k_wide_scatter that do nothing else cost that kernel the 17 us they save this one).
-// DIRECT: the launch is one workgroup and one bucket, and the records are the list's entries themselves.
-template <typename I, typename S, typename O, bool DENSE, bool DIRECT>
+template <typename I, typename S, typename O, bool DENSE>
 __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__restrict__ out_idx,
                                                            O *__restrict__ out_val, int64_t capacity,
                                                            ScanState st, int tie_bits, int64_t *out_count,
@@ -79,15 +78,15 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
   int32_t *const status = list.status;
   const uint32_t tid = threadIdx.x;
   if (tid == 0) {
-    sh.tile = DIRECT ? 0 : (int)atomicAdd(st.ticket, 1u);
+    sh.tile = (int)atomicAdd(st.ticket, 1u);
     sh.qn = sh.big = 0;
   }
   sh.cnt.clear();
   __syncthreads();
   const uint32_t b = (uint32_t)sh.tile;  // buckets are taken in order, so every earlier bucket already runs
-  const uint32_t nb = DIRECT ? 1u : geo.nbuckets;
+  const uint32_t nb = geo.nbuckets;
   if (b >= nb) return;
-  const uint32_t lo = DIRECT ? 0u : geo.first_key(b);
+  const uint32_t lo = geo.first_key(b);
   // The bucket's range of a dense tensor: elements up to the first multiple of 16 bytes, vectors, elements.  The
   // vectors' zeros are stored a few at a time between the steps of the ranking loops, whose LDS round trips leave the
   // memory idle.
@@ -114,11 +113,10 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
   uint32_t longest = 0;
 #pragma unroll
   for (int q = 0; q < kWideSplit; ++q) {
-    pcount[q] = DIRECT ? 0u : in.cursor[(b * kWideSplit + q) * kWmPad];
-    if (!DIRECT && pcount[q] > in.part_cap) pcount[q] = in.part_cap;  // the scatter flagged the overflow
+    pcount[q] = in.cursor[(b * kWideSplit + q) * kWmPad];
+    if (pcount[q] > in.part_cap) pcount[q] = in.part_cap;  // the scatter flagged the overflow
     longest = pcount[q] > longest ? pcount[q] : longest;
   }
-  if (DIRECT) longest = (list.r + kWideSplit - 1) / kWideSplit;  // entry (r * kWideSplit + q) * kWideBlock + tid is item q of round r
   bool declined = false;
   if (longest > (uint32_t)kWmPartMax) {
     declined = true;
@@ -141,26 +139,10 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
     if ((uint32_t)r * kWideBlock < longest) {
 #pragma unroll
       for (int q = 0; q < kWideSplit; ++q) {
-        uint32_t off, arr;
-        bool live;
-        if (DIRECT) {
-          arr = (uint32_t)(r * kWideSplit + q) * kWideBlock + tid;
-          live = arr < list.r;
-          const uint32_t e = live ? arr : 0u;
-          const int64_t v = list.idx64 ? static_cast<const int64_t *>(list.idx)[e]
-                                       : (int64_t)static_cast<const int32_t *>(list.idx)[e];
-          if (live && (v < 0 || v >= (int64_t)dense_n)) {
-            atomicOr(status, ZEN_STAT_BAD_INDEX);  // skipped
-            live = false;
-          }
-          off = (uint32_t)v;
-        } else {
-          const uint32_t e = tid + (uint32_t)r * kWideBlock;
-          live = e < pcount[q];
-          const uint2 rec = rec_plane[(size_t)q * in.part_cap + (live ? e : 0u)];
-          off = wm_off(rec);
-          arr = wm_arr(rec);
-        }
+        const uint32_t e = tid + (uint32_t)r * kWideBlock;
+        const bool live = e < pcount[q];
+        const uint2 rec = rec_plane[(size_t)q * in.part_cap + (live ? e : 0u)];
+        const uint32_t off = wm_off(rec), arr = wm_arr(rec);
         if (live) {
           w[r * kWideSplit + q] = ((off & low_mask) << tie_bits) | arr;
           ps[r * kWideSplit + q] = off >> shift;  // the narrow range, for now
@@ -174,7 +156,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
   __syncthreads();
   uint32_t n = sh.cnt.starts(sh.scan, (uint32_t)kWmGroupLimit, &sh.big);
   __syncthreads();
-  if (!DIRECT && (n > (uint32_t)kWideCap || sh.big)) {  // more than fits, or keys piled on a few values: another path answers
+  if (n > (uint32_t)kWideCap || sh.big) {  // more than fits, or keys piled on a few values: another path answers
     declined = true;
     __syncthreads();
     sh.cnt.clear();
@@ -186,7 +168,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
   }
   if (declined && tid == 0) atomicOr(status, ZEN_STAT_RETRY);
   // this workgroup was the only reader of its part cursors: back to zero for the next call
-  if (!DIRECT && tid < (uint32_t)kWideSplit) in.cursor[(b * kWideSplit + tid) * kWmPad] = 0;
+  if (tid < (uint32_t)kWideSplit) in.cursor[(b * kWideSplit + tid) * kWmPad] = 0;
 
   // The thread's records are worked through in steps of kWmLanes, by loops whose body handles the first
   // kWmLanes registers of a set and then rotates the set (the body written out for all records would not fit
@@ -303,14 +285,9 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
 #pragma unroll
       for (int q = 0; q < kWideSplit; ++q) {
         const bool live = rk[r * kWideSplit + q] != kInvalid;
-        if (DIRECT) {
-          const uint32_t e = (uint32_t)(r * kWideSplit + q) * kWideBlock + tid;
-          v[q] = (uint32_t) static_cast<const S *>(list.val)[live ? e : 0u];
-        } else {
-          const uint32_t e = tid + (uint32_t)r * kWideBlock;
-          const size_t at = (size_t)q * in.part_cap + (live ? e : 0u);
-          v[q] = sizeof(S) == 2 ? rec_plane[at].y >> 16 : val_plane[at];
-        }
+        const uint32_t e = tid + (uint32_t)r * kWideBlock;
+        const size_t at = (size_t)q * in.part_cap + (live ? e : 0u);
+        v[q] = sizeof(S) == 2 ? rec_plane[at].y >> 16 : val_plane[at];
       }
 #pragma unroll
       for (int q = 0; q < kWideSplit; ++q) {
@@ -376,7 +353,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
   // where this bucket's output starts: the sum of what all earlier buckets keep.  Every thread asks for one of
   // them (bounded wait), nobody waits for a chain of prefixes; while the answers are on their way the kept
   // entries are gathered in LDS (everybody is past reading the sorted bucket: the scan synchronised).
-  if (!DENSE && !DIRECT && tid == 0) desc_store(&st.desc[b], kDescAggregate | total);
+  if (!DENSE && tid == 0) desc_store(&st.desc[b], kDescAggregate | total);
   uint64_t d = !DENSE && tid < b ? desc_load(&st.desc[tid]) : kDescAggregate;
   uint32_t li = before;
 #pragma unroll
@@ -419,11 +396,6 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
     }
   }
   if (answer.host) wait_global_acks();  // its share of the status word, and the count
-  if (DIRECT) {
-    __syncthreads();
-    host_answer_count(answer, DENSE ? nullptr : out_count, status);
-    return;
-  }
   // every workgroup has read the descriptors it needs before it gets here: the last one to finish clears the
   // prefix state
   uint32_t *finished = reinterpret_cast<uint32_t *>(st.desc + nb + 1);
@@ -444,8 +416,8 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
 
 bool wide_merge_fits(int64_t r, int64_t dense_n, int cus, SlabGeom *geo, bool alone) {
   SlabGeom g;
-  // (shorter lists: wide_merge_one)
-  if (r <= wide_merge_one_max() || r > 0x7ffffffell || cus <= 0) return false;
+  // (shorter lists: one workgroup, zen_merge.hip)
+  if (r <= merge_one_max() || r > 0x7ffffffell || cus <= 0) return false;
   // Sixteen buckets for small index ranges, more only for lists that need them: a bucket's workgroup takes a compute
   // unit, and 128 of them for ten thousand entries keep the encode beside them waiting (a step of 1 Mi elements
   // took 106 us instead of 85).
@@ -501,53 +473,32 @@ bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, 
 
 uint32_t wide_scatter_batches(const WideList &list, int batch) { return (uint32_t)ceil_div((int64_t)list.r, batch); }
 
-template <typename S, typename O, bool DIRECT>
+template <typename S, typename O>
 static void wide_merge_launch(const WideList &list, void *out_idx, int idx64_out, O *out_val, int64_t capacity,
                               int64_t *out_count, unsigned long long *scan, hipStream_t s, const HostAsk &ask) {
   const ScanState st = scan_state(scan, (int64_t)list.geo.nbuckets);
   const int tie_bits = ceil_log2_u64((uint64_t)list.r);  // arrival numbers are < r
-  const dim3 grid(DIRECT ? 1u : list.geo.nbuckets), block(kWideBlock);
+  const dim3 grid(list.geo.nbuckets), block(kWideBlock);
   if (!out_idx)
-    k_wide_merge<int32_t, S, O, true, DIRECT><<<grid, block, 0, s>>>(list, nullptr, out_val, capacity, st, tie_bits, out_count,
+    k_wide_merge<int32_t, S, O, true><<<grid, block, 0, s>>>(list, nullptr, out_val, capacity, st, tie_bits, out_count,
                                                                          ask.answer);
   else if (idx64_out)
-    k_wide_merge<int64_t, S, O, false, DIRECT><<<grid, block, 0, s>>>(list, static_cast<int64_t *>(out_idx), out_val, capacity,
+    k_wide_merge<int64_t, S, O, false><<<grid, block, 0, s>>>(list, static_cast<int64_t *>(out_idx), out_val, capacity,
                                                                      st, tie_bits, out_count, ask.answer);
   else
-    k_wide_merge<int32_t, S, O, false, DIRECT><<<grid, block, 0, s>>>(list, static_cast<int32_t *>(out_idx), out_val, capacity,
+    k_wide_merge<int32_t, S, O, false><<<grid, block, 0, s>>>(list, static_cast<int32_t *>(out_idx), out_val, capacity,
                                                                      st, tie_bits, out_count, ask.answer);
 }
 
-template <bool DIRECT>
 static void wide_merge_typed(const WideList &list, int dtype, void *out_idx, int idx64_out, void *out_val, int out_dtype,
                              int64_t capacity, int64_t *out_count, unsigned long long *scan, hipStream_t s,
                              const HostAsk &ask) {
   if (dtype == ZEN_F32)
-    wide_merge_launch<uint32_t, float, DIRECT>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s, ask);
+    wide_merge_launch<uint32_t, float>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s, ask);
   else if (out_dtype == ZEN_BF16)
-    wide_merge_launch<uint16_t, uint16_t, DIRECT>(list, out_idx, idx64_out, static_cast<uint16_t *>(out_val), capacity, out_count, scan, s, ask);
+    wide_merge_launch<uint16_t, uint16_t>(list, out_idx, idx64_out, static_cast<uint16_t *>(out_val), capacity, out_count, scan, s, ask);
   else
-    wide_merge_launch<uint16_t, float, DIRECT>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s, ask);
-}
-
-// out_dtype and out_idx as for wide_merge below.  Any indices: a narrow range takes whatever comes.
-int wide_merge_one(const void *idx, int idx64_in, const void *val, int dtype, int64_t r, int64_t dense_n, void *out_idx,
-                   int idx64_out, void *out_val, int out_dtype, int64_t capacity, int64_t *out_count, int32_t *status,
-                   hipStream_t s, const HostAsk &ask) {
-  WideList list{};
-  while ((dense_n >> list.geo.sub_shift) >= kWideSubs) ++list.geo.sub_shift;  // 17 at most: with 14 bits of arrival number a word
-  list.geo.nbuckets = 1;
-  list.idx = idx;
-  list.val = val;
-  list.r = (uint32_t)r;
-  list.dense_n = (uint32_t)dense_n;
-  list.idx64 = idx64_in;
-  list.status = status;
-  ProfScope prof(kProfWideMerge, s);
-  wide_merge_typed<true>(list, dtype, out_idx, idx64_out, out_val, out_dtype, capacity, out_count, nullptr, s, ask);
-  ZEN_LAUNCH_CHECK("k_wide_merge");
-  if (ask.answer.host) *ask.answered = true;
-  return ZEN_OK;
+    wide_merge_launch<uint16_t, float>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s, ask);
 }
 
 // The two launches.  scan: zeroed prefix state for 256 buckets (descriptors, ticket, finished count), zero again
@@ -564,7 +515,7 @@ int wide_merge(const WideList &list, int dtype, void *out_idx, int idx64_out, vo
     ZEN_LAUNCH_CHECK("k_wide_scatter");
   }
   ProfScope prof(kProfWideMerge, s);
-  wide_merge_typed<false>(list, dtype, out_idx, idx64_out, out_val, out_dtype, capacity, out_count, scan, s, ask);
+  wide_merge_typed(list, dtype, out_idx, idx64_out, out_val, out_dtype, capacity, out_count, scan, s, ask);
   ZEN_LAUNCH_CHECK("k_wide_merge");
   if (ask.answer.host) *ask.answered = true;
   return ZEN_OK;
