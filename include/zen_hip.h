@@ -99,7 +99,7 @@ extern "C" {
 #define ZEN_MODE_SLABS 0x2000
 /* OR-ed into the `mode` of zen_load_balance with k == 0: the caller vouches that no sample taken ahead
    (zen_load_balance_prepare, zen_encode_merge's next_input) waits in `table`, that every word of it is zero.  Tables of
-   2^20 to 4 Mi slots then serve as owner tables, the quickest way at those sizes; without the flag such a call takes
+   2^20 to 6 or 10 Mi slots then serve as owner tables, the quickest way at those sizes; without the flag such a call takes
    a path that leaves waiting samples alone.  Smaller tables never hold a sample. */
 #define ZEN_MODE_NO_SAMPLES 0x4000
 
@@ -304,7 +304,7 @@ int zen_select_count(const void *input, int dtype, int64_t n, const uint32_t *th
  * raised ZEN_STAT_RETRY or ZEN_STAT_INTERNAL, or returned an error code, its
  * contents are undefined and the caller clears it.  ZEN_MODE_GENERAL keeps the owner of every probed slot in
  * it, like the reference, and so does ZEN_MODE_FAST where the table is small
- * (below 2^20 slots; up to 4 Mi slots with k == 0 and ZEN_MODE_NO_SAMPLES; tables of up to 32768 slots are kept in
+ * (below 2^20 slots; up to 10 Mi slots with k == 0 and ZEN_MODE_NO_SAMPLES; tables of up to 32768 slots are kept in
  * LDS).  Otherwise ZEN_MODE_FAST sorts the selected entries by their level-1 slot and borrows at most half of the
  * table as a hash map for the few entries that collide (ZEN_STAT_RETRY if there are too many), and the megabyte
  * behind it for its counters and the samples.
@@ -353,8 +353,8 @@ int zen_load_balance_prepare(const void *input, int dtype, int64_t n, int64_t m,
 
 /*
  * Which implementation a zen_load_balance call with these sizes and this mode takes: 0 = owner table (the
- * general mode), 1 = the same in three launches or one (tables below 2^20 slots, up to 4 Mi slots with k == 0 and
- * ZEN_MODE_NO_SAMPLES) or sort-based owner resolution, 2 = bucket slabs (large inputs whose expected output is a
+ * general mode), 1 = the same in two launches or one (tables below 2^20 slots, up to 6 Mi slots, 10 Mi with a
+ * capacity of at most a 32nd of them, with k == 0 and ZEN_MODE_NO_SAMPLES) or sort-based owner resolution, 2 = bucket slabs (large inputs whose expected output is a
  * small fraction of the table: one streaming pass, then per-bucket sorts inside LDS), 3 = wide buckets (the same
  * for an expected output of up to a few million entries, few of them on a slot that is taken: at most 256 buckets,
  * one resident workgroup each, two launches; zen_load_balance_sizes takes path 2 there where the sizes allow it).  No

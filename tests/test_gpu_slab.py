@@ -93,11 +93,12 @@ def test_slab_load_balance_bit_exact(zen, oracle, n, P, density, rehash, dtype):
 
 
 @pytest.mark.parametrize("n,P,density,rehash,room", [
-    ((1 << 22) - 6, 3, 0.05, 3, 1.1),   # just below the smallest table of the slabs: the owner table
-    ((1 << 22) + 5, 2, 0.1, 3, 1.1),    # just above it, a tenth of the slots taken
-    ((1 << 22) + 5, 16, 0.001, 3, 1.1),
-    ((1 << 22) + 5, 2, 0.3, 2, 1.1),    # too dense for the slabs' buckets
-    (6000000, 3, 0.1, 2, 0.5),          # room for half: declined, and taken again with more
+    ((6 << 20) - 3, 3, 0.05, 3, 1.1),   # the largest owner tables, a tenth selected and little
+    ((10 << 20) - 6, 16, 0.001, 3, 1.1),
+    ((6 << 20) + 2, 2, 0.1, 3, 1.1),    # just beyond them: the slabs
+    ((10 << 20) + 16, 16, 0.001, 3, 1.1),
+    ((6 << 20) + 5, 2, 0.3, 2, 1.1),    # too dense for the slabs' buckets
+    (7000000, 3, 0.1, 2, 0.5),          # room for half: declined, and taken again with more
 ])
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 def test_call_that_waits_gives_the_same_on_every_path(zen, oracle, n, P, density, rehash, room, dtype):

@@ -167,8 +167,8 @@ int wide_device_cus();  // compute units of the current device (0: no device)
 
 // Load balance through the owner table (zen_table.hip), for up to a few million slots.  a.hash is the caller's table
 // (16-byte aligned); splits_zero: a.splits is zero already.  no_samples: no sample taken ahead waits in the table.
-bool table_balance_fits(int64_t n, int64_t m, int partitions, int64_t k, bool no_samples);
-size_t table_balance_bytes(int64_t n, int64_t m, int dtype, int partitions);
+bool table_balance_fits(int64_t n, int64_t m, int partitions, int64_t capacity, int64_t k, bool no_samples);
+size_t table_balance_bytes(int64_t n, int64_t m, int dtype, int partitions, int64_t capacity);
 int table_load_balance(const SlabBalanceArgs &a, bool splits_zero, hipStream_t stream);
 
 size_t resolve_scratch_bytes(int64_t list_cap, uint64_t key_limit);  // key_limit = P * (m / P + 1) + 1

@@ -519,7 +519,7 @@ size_t zen_load_balance_workspace(int64_t n, int64_t m, int dtype, int64_t capac
   const size_t wide = partitions > 0 && m % partitions == 0
                           ? zen::wide_balance_bytes(m, partitions, dtype, capacity, zen::wide_device_cus())
                           : 0;
-  const size_t table = partitions > 0 && m % partitions == 0 ? zen::table_balance_bytes(n, m, dtype, partitions) : 0;
+  const size_t table = partitions > 0 && m % partitions == 0 ? zen::table_balance_bytes(n, m, dtype, partitions, capacity) : 0;
   const size_t buckets = slabs > wide ? slabs : wide;
   const size_t fast = buckets > table ? buckets : table;
   return general > fast ? general : fast;
@@ -555,7 +555,7 @@ int zen_load_balance_path(int64_t n, int64_t m, int dtype, int64_t capacity, int
   const bool slabs_only = (mode & ZEN_MODE_SLABS) != 0, no_samples = (mode & ZEN_MODE_NO_SAMPLES) != 0;
   mode &= 0xff;
   if (mode != ZEN_MODE_FAST || partitions <= 0 || m <= 0 || m % partitions != 0) return 0;
-  if (!slabs_only && zen::table_balance_fits(n, m, partitions, k, no_samples)) return 1;
+  if (!slabs_only && zen::table_balance_fits(n, m, partitions, capacity, k, no_samples)) return 1;
   if (!slabs_only && takes_wide(n, m, partitions, dtype, capacity, k, false)) return 3;
   if (zen::slab_balance_fits(n, m, partitions, dtype, capacity, k, nullptr)) return 2;
   return m >= 4096 ? 1 : 0;
@@ -585,7 +585,7 @@ int zen_load_balance_prepare(const void *input, int dtype, int64_t n, int64_t m,
     return fail(ZEN_EWORKSPACE, "zen_load_balance_prepare: workspace too small");
   const int second = (mode & ZEN_MODE_SECOND) != 0;
   if ((mode & 0xff) != ZEN_MODE_FAST || k == 0 || (reinterpret_cast<uintptr_t>(table) & 7u) != 0 ||
-      (!(mode & ZEN_MODE_SLABS) && table_balance_fits(n, m, partitions, k, false)) ||
+      (!(mode & ZEN_MODE_SLABS) && table_balance_fits(n, m, partitions, capacity, k, false)) ||
       (!slab_balance_fits(n, m, partitions, dtype, capacity, k, nullptr) &&
        !wide_balance_fits(m, partitions, capacity, k, wide_device_cus(), nullptr)))
     return ZEN_OK;  // nothing to take ahead on the other paths
@@ -652,7 +652,7 @@ int load_balance_call(const void *input, int dtype, int64_t n, int64_t m, int pa
   const uint32_t drop_key = (uint32_t)partitions * (g.npp + 1u);
   const int bits = ceil_log2_u64(drop_key);
   const bool small = mode == ZEN_MODE_FAST && !slabs_only && (reinterpret_cast<uintptr_t>(table) & 15u) == 0 &&
-                     table_balance_fits(n, m, partitions, k, no_samples);
+                     table_balance_fits(n, m, partitions, capacity, k, no_samples);
   const bool wide = mode == ZEN_MODE_FAST && !slabs_only && (reinterpret_cast<uintptr_t>(table) & 7u) == 0 &&
                     takes_wide(n, m, partitions, dtype, capacity, k, ask.answer.host != nullptr);
   if (small || wide || (mode == ZEN_MODE_FAST && (reinterpret_cast<uintptr_t>(table) & 7u) == 0 &&

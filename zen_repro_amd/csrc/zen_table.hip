@@ -483,17 +483,20 @@ int table_launch(const SlabBalanceArgs &a, const TablePlan &p, const uint32_t *t
 
 }  // namespace
 
-// Tables of up to 4 Mi slots (16 MB: two readings of it cost less than the wide buckets' resident kernel, 30 us);
-// a top-k selection, whose threshold takes launches of its own here, only where the wide buckets do not apply.  Every
-// word of the table is a slot here, and a sample taken ahead waits in its call's table, in tables of 2^20 slots or more
-// (wide_geometry, slab_geometry): those are taken only if there is none, the others hold none.
-bool table_balance_fits(int64_t n, int64_t m, int partitions, int64_t k, bool no_samples) {
-  const int64_t most = k > 0 || !no_samples ? (1ll << 20) - 1 : 1ll << 22;
-  return n <= (1ll << 22) && m <= most && partitions <= kMaxParts;
+// A selection by a given threshold, or of the nonzeros: the atomics and two readings of the table cost less than the bucket
+// slabs' five launches up to 6 Mi slots, up to 10 Mi where little is selected (a call that waits, 2 partitions, us here and
+// on the slabs: 6 M bf16 elements 0.5 % selected 50 and 62, 5 % 67 and 74, 10 % 90 and 88; 9 M 58 and 63, 1.5 % 62 and 65,
+// 5 % 85 and 77; 16 M 71 and 67, 5 % 113 and 90).  A top-k selection, whose threshold takes launches of its own here, only
+// where the wide buckets do not apply.  Every word of the table is a slot here, and a sample taken ahead waits in its call's
+// table, in tables of 2^20 slots or more (wide_geometry, slab_geometry): those are taken only if there is none, the others
+// hold none.
+bool table_balance_fits(int64_t n, int64_t m, int partitions, int64_t capacity, int64_t k, bool no_samples) {
+  const int64_t most = k > 0 || !no_samples ? (1ll << 20) - 1 : capacity <= m / 32 ? 10ll << 20 : 6ll << 20;
+  return n <= (10ll << 20) && m <= most && partitions <= kMaxParts;
 }
 
-size_t table_balance_bytes(int64_t n, int64_t m, int dtype, int partitions) {
-  return table_balance_fits(n, m, partitions, 0, true) ? plan_table(nullptr, n, m, dtype, partitions).bytes : 0;
+size_t table_balance_bytes(int64_t n, int64_t m, int dtype, int partitions, int64_t capacity) {
+  return table_balance_fits(n, m, partitions, capacity, 0, true) ? plan_table(nullptr, n, m, dtype, partitions).bytes : 0;
 }
 
 int table_load_balance(const SlabBalanceArgs &a, bool splits_zero, hipStream_t s) {
