@@ -51,7 +51,8 @@ extern "C" {
  *    16-byte entry per 96 indices (zen_bitmap_rank_words), and the dense
  *    dictionary is longer by a chunk of places (zen_bitmap_dense_dict_bytes):
  *    both are built anew, not kept from an older library
- * 8: zen_balance_tables
+ * 8: zen_balance_tables, zen_decode_dense_lists_status,
+ *    zen_bitmap_dense_lists_status, zen_bitmap_encode_status
  */
 #define ZEN_ABI_VERSION 8
 
@@ -168,6 +169,10 @@ int zen_bitmap_ranks(const int64_t *mapping_p, int64_t mapping_n, int64_t numel,
 int zen_bitmap_encode(const int64_t *mapping_p, int64_t mapping_n, const void *idx, int idx64, int64_t idx_n,
                       const int64_t *idx_n_dev, const uint32_t *rank_at, int64_t numel, uint32_t *bitmap_words,
                       int32_t *status, void *stream);
+/* Returns when it is done, with the status word in host[1] (host: `words` >= 2 of zen_host_words_alloc). */
+int zen_bitmap_encode_status(const int64_t *mapping_p, int64_t mapping_n, const void *idx, int idx64, int64_t idx_n,
+                             const int64_t *idx_n_dev, const uint32_t *rank_at, int64_t numel,
+                             uint32_t *bitmap_words, int32_t *status, int64_t *host, int64_t words, void *stream);
 size_t zen_bitmap_decode_workspace(int64_t mapping_n);
 int zen_bitmap_decode(const int64_t *mapping_p, int64_t mapping_n, const uint8_t *bitmap, int64_t bitmap_bytes,
                       int64_t *out, int64_t capacity, int64_t *out_count, void *workspace, size_t workspace_bytes,
@@ -523,6 +528,12 @@ size_t zen_decode_dense_sorted_workspace(int64_t dense_n, int nlists);
 int zen_decode_dense_lists(const void *const *idx, int idx64_in, const void *const *val, int dtype,
                            const int64_t *len, int nlists, void *dense, int64_t dense_n,
                            void *workspace, size_t workspace_bytes, int32_t *status, void *stream);
+/* Returns when every entry has been read, with the status word in host[1] (host: `words` >= 2 of
+   zen_host_words_alloc); the dense tensor is complete in the order of `stream`. */
+int zen_decode_dense_lists_status(const void *const *idx, int idx64_in, const void *const *val, int dtype,
+                                  const int64_t *len, int nlists, void *dense, int64_t dense_n,
+                                  void *workspace, size_t workspace_bytes, int32_t *status,
+                                  int64_t *host, int64_t words, void *stream);
 int zen_decode_dense_sorted(const void *idx, int idx64_in, const void *val, int dtype,
                             const int64_t *list_start, int nlists, void *dense, int64_t dense_n,
                             void *workspace, size_t workspace_bytes, int32_t *status, void *stream);
@@ -557,6 +568,12 @@ int zen_bitmap_dense_lists(const void *dict, int64_t numel, int partitions, cons
                            const int64_t *bitmap_bytes, const void *const *values, int dtype,
                            const int64_t *value_count, void *dense, void *workspace, size_t workspace_bytes,
                            int32_t *status, void *stream);
+/* Returns when the status is known, with it in host[1] (host: `words` >= 2 of zen_host_words_alloc): the tensor, for
+   which bitmaps, values, dictionary and workspace are still read, is complete in the order of `stream`. */
+int zen_bitmap_dense_lists_status(const void *dict, int64_t numel, int partitions, const uint8_t *const *bitmaps,
+                                  const int64_t *bitmap_bytes, const void *const *values, int dtype,
+                                  const int64_t *value_count, void *dense, void *workspace, size_t workspace_bytes,
+                                  int32_t *status, int64_t *host, int64_t words, void *stream);
 
 /* --------------------------------------------------------------- utility */
 

@@ -85,6 +85,7 @@ def lib():
         "zen_bitmap_rank_words": (sz, [i64]),
         "zen_bitmap_ranks": (i32, [vp, i64, i64, vp, vp]),
         "zen_bitmap_encode": (i32, [vp, i64, vp, i32, i64, vp, vp, i64, vp, vp, vp]),
+        "zen_bitmap_encode_status": (i32, [vp, i64, vp, i32, i64, vp, vp, i64, vp, vp, vp, i64, vp]),
         "zen_bitmap_decode_workspace": (sz, [i64]),
         "zen_bitmap_decode": (i32, [vp, i64, vp, i64, vp, i64, vp, vp, sz, vp, vp]),
         "zen_sparse_balance": (i32, [vp, i32, i64, vp, i64, vp, i64, vp, i32, i32, vp, vp]),
@@ -114,6 +115,7 @@ def lib():
         "zen_encode_merge": (i32, [ctypes.POINTER(EncodeMergeArgs)]),
         "zen_merge_rounded": (i32, [vp, i32, vp, i32, i64, i64, vp, i32, vp, i64, vp, i32, vp, sz, vp, vp]),
         "zen_merge_rounded_count": (i32, [vp, i32, vp, i32, i64, i64, vp, i32, vp, i64, vp, i32, vp, sz, vp, vp, i64, vp]),
+        "zen_decode_dense_lists_status": (i32, [vp, i32, vp, i32, vp, i32, vp, i64, vp, sz, vp, vp, i64, vp]),
         "zen_decode_dense_lists": (i32, [vp, i32, vp, i32, vp, i32, vp, i64, vp, sz, vp, vp]),
         "zen_decode_dense_workspace": (sz, [i64, i64]),
         "zen_decode_dense": (i32, [vp, i32, vp, i32, i64, vp, i64, i32, vp, sz, vp, vp]),
@@ -125,6 +127,7 @@ def lib():
         "zen_bitmap_dense_workspace": (sz, [i64, i32]),
         "zen_bitmap_dense": (i32, [vp, i64, i32, vp, ctypes.POINTER(ctypes.c_int64), vp, i32,
                                    ctypes.POINTER(ctypes.c_int64), vp, vp, sz, vp, vp]),
+        "zen_bitmap_dense_lists_status": (i32, [vp, i64, i32, vp, vp, vp, i32, vp, vp, vp, sz, vp, vp, i64, vp]),
         "zen_bitmap_dense_lists": (i32, [vp, i64, i32, vp, vp, vp, i32, vp, vp, vp, sz, vp, vp]),
         "zen_sort_pairs_workspace": (sz, [i64]),
         "zen_sort_pairs": (i32, [vp, vp, i64, vp, i32, vp, sz, vp, vp]),

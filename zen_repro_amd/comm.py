@@ -156,11 +156,13 @@ class LoadBalanceAllreduce:
         assert lists[0].dtype in (torch.int32, torch.int64)
         L = _lib.lib()
         ws = _lib.scratch.get(dev, "decode_sorted", L.zen_decode_dense_sorted_workspace(dense_size, count))
-        rc, dense, status = _lib.host.decode_lists(L.zen_decode_dense_lists, _lib.zeros.native(), lists, values,
-                                                   _lib.dtype_code(values[0]), dense_size, ws, _lib.stream_of(dev))
+        words = _lib.host_words(1)
+        rc, dense = _lib.host.decode_lists(L.zen_decode_dense_lists_status, _lib.zeros.native(), lists, values,
+                                           _lib.dtype_code(values[0]), dense_size, ws, _lib.stream_of(dev), words.ptr,
+                                           words.words)
         _lib.check(rc, "decode_sparse_tensors")
         # the reference's scatter_add_ raises on a bad index, also a sync
-        return None if _lib.read_back(status)[0] else dense
+        return None if words.view[1] else dense
 
     # OR-ed into the mode of every fast-mode call (_lib.MODE_SLABS keeps the calls off the wide buckets)
     fast_flags = 0
@@ -414,35 +416,48 @@ class LoadBalanceAllreduce:
         """encode_bitmap without host synchronisation: (uint8 bitmap, status
         int32[1]).  `count` (int64[1] on the device) limits the indices that
         are looked at to the first `count`."""
-        mapping = self.mapping[numel][self.local_rank]
-        _lib.require_gpu(sparse_indices, "sparse_indices")
-        if sparse_indices.dtype not in (torch.int32, torch.int64):
-            raise RuntimeError("sparse_indices must be int32 or int64")
+        mapping, ranks = self._ranks(sparse_indices, numel)
         dev = sparse_indices.device
         L = _lib.lib()
         members = mapping.numel()
         words = torch.empty(max(1, L.zen_bitmap_words(members)), dtype=torch.int32, device=dev)
         status = _lib.status_word(dev)
-        # the rank table lives next to the mapping it belongs to (same cache, same lifetime)
-        cached = self._bitmap_ranks.get(numel)
-        if cached is None or cached[0] is not mapping:
-            rank_at = torch.empty(L.zen_bitmap_rank_words(numel), dtype=torch.int32, device=dev)
-            _lib.check(L.zen_bitmap_ranks(_lib.ptr(mapping), members, numel, _lib.ptr(rank_at),
-                                          _lib.stream_of(dev)), "encode_bitmap")
-            cached = self._bitmap_ranks[numel] = (mapping, rank_at)
         rc = L.zen_bitmap_encode(_lib.ptr(mapping), members, _lib.ptr(sparse_indices),
                                  int(sparse_indices.dtype == torch.int64), sparse_indices.numel(),
-                                 _lib.ptr(count) if count is not None else None, _lib.ptr(cached[1]), numel,
+                                 _lib.ptr(count) if count is not None else None, _lib.ptr(ranks), numel,
                                  _lib.ptr(words), _lib.ptr(status), _lib.stream_of(dev))
         _lib.check(rc, "encode_bitmap")
         return words.view(torch.uint8)[:(members + 7) // 8], status
+
+    def _ranks(self, sparse_indices, numel):
+        """This rank's mapping list and its rank table, which lives next to the mapping it belongs to (same cache,
+        same lifetime)."""
+        mapping = self.mapping[numel][self.local_rank]
+        _lib.require_gpu(sparse_indices, "sparse_indices")
+        if sparse_indices.dtype not in (torch.int32, torch.int64):
+            raise RuntimeError("sparse_indices must be int32 or int64")
+        cached = self._bitmap_ranks.get(numel)
+        if cached is None or cached[0] is not mapping:
+            L = _lib.lib()
+            dev = sparse_indices.device
+            rank_at = torch.empty(L.zen_bitmap_rank_words(numel), dtype=torch.int32, device=dev)
+            _lib.check(L.zen_bitmap_ranks(_lib.ptr(mapping), mapping.numel(), numel, _lib.ptr(rank_at),
+                                          _lib.stream_of(dev)), "encode_bitmap")
+            cached = self._bitmap_ranks[numel] = (mapping, rank_at)
+        return cached
 
     def encode_bitmap(self, sparse_indices, numel):
         """One bit per member of this rank's mapping list, set where the member
         is among sparse_indices; least significant bit first, padded to a whole
         byte (comm.py:59-85).  self.mapping[numel] must exist (comm.py:135)."""
-        bitmap, status = self.encode_bitmap_flat(sparse_indices, numel)
-        bits = _lib.read_back(status)[0]
+        mapping, ranks = self._ranks(sparse_indices, numel)
+        L = _lib.lib()
+        words = _lib.host_words(1)
+        rc, bitmap = _lib.host.bitmap_encode(L.zen_bitmap_encode_status, _lib.zeros.native(), mapping, sparse_indices,
+                                             ranks, numel, L.zen_bitmap_words(mapping.numel()),
+                                             _lib.stream_of(sparse_indices.device), words.ptr, words.words)
+        _lib.check(rc, "encode_bitmap")
+        bits = words.view[1]
         if bits & _lib.STAT_BAD_INDEX:  # result[indices] = 1 with an index == len(result), comm.py:63
             raise IndexError("encode_bitmap: an index lies beyond the last member of the mapping")
         if bits:
@@ -494,7 +509,11 @@ class LoadBalanceAllreduce:
         dictionary of two bytes per element (per tile of the dense tensor, the
         places of its indices ordered by partition) is built on first use of a
         `numel` and cached like the reference caches the mapping
-        (comm.py:132-134)."""
+        (comm.py:132-134).  The call waits until it is known whether bitmaps and
+        values agree; the dense tensor is complete on the current stream, and the
+        bitmaps and values are still read until then: another stream that reads the
+        result or overwrites them waits for this one first (dropping them is
+        safe)."""
         if len(bitmap_indices) != self.partitions or len(values_tensors) != self.partitions:
             raise RuntimeError("decode_bitmaps_dense: one bitmap and one value list per rank")
         for t in bitmap_indices:
@@ -519,10 +538,13 @@ class LoadBalanceAllreduce:
             self._dense_dicts[numel] = cached
         P = self.partitions
         ws = _lib.scratch.get(dev, "bitmap_dense", L.zen_bitmap_dense_workspace(numel, P))
-        rc, dense, status = _lib.host.bitmaps_dense(L.zen_bitmap_dense_lists, _lib.zeros.native(), bitmap_indices, values,
-                                                    _lib.dtype_code(values[0]), cached, numel, ws, _lib.stream_of(dev))
+        words = _lib.host_words(1)
+        rc, dense = _lib.host.bitmaps_dense(L.zen_bitmap_dense_lists_status, _lib.zeros.native(), bitmap_indices, values,
+                                            _lib.dtype_code(values[0]), cached, numel, ws, _lib.stream_of(dev), words.ptr,
+                                            words.words)
+        _lib.scratch.left_running(dev, "bitmap_dense")
         _lib.check(rc, "decode_bitmaps_dense")
-        bits = _lib.read_back(status)[0]  # the reference's masking and scatter_add_ raise on a mismatch, also a sync
+        bits = words.view[1]  # the reference's masking and scatter_add_ raise on a mismatch, also a sync
         if bits & _lib.STAT_BAD_INDEX:
             raise IndexError("decode_bitmaps_dense: a bitmap is shorter than its partition's index list, or has "
                              "more set bits than values came with it")

@@ -333,6 +333,19 @@ int zen_bitmap_encode(const int64_t *mapping_p, int64_t mapping_n, const void *i
   return ZEN_OK;
 }
 
+int zen_bitmap_encode_status(const int64_t *mapping_p, int64_t mapping_n, const void *idx, int idx64, int64_t idx_n,
+                             const int64_t *idx_n_dev, const uint32_t *rank_at, int64_t numel, uint32_t *bitmap_words,
+                             int32_t *status, int64_t *host, int64_t words, void *stream) {
+  using namespace zen;
+  HostAnswer answer;
+  int rc = host_ask(host, words, 1, &answer);
+  if (rc != ZEN_OK) return rc;
+  rc = zen_bitmap_encode(mapping_p, mapping_n, idx, idx64, idx_n, idx_n_dev, rank_at, numel, bitmap_words, status, stream);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (rc == ZEN_OK) rc = host_answer_launch(answer, nullptr, 0, status, 1, s);
+  return rc == ZEN_OK ? host_wait(answer, s) : rc;
+}
+
 size_t zen_bitmap_decode_workspace(int64_t mapping_n) {
   return zen::align_up((size_t)zen::decode_blocks(mapping_n) * sizeof(uint32_t), 256);
 }

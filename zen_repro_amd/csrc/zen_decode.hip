@@ -33,8 +33,8 @@ struct DecLists {
   int n;
 };
 
-// starts[l * (ntiles + 1) + t] = number of entries of list l with index < t * kDecTile (by a search that assumes
-// the list ascending; the tile kernel checks that it is).  Bound by the memory lines it asks for, one for nearly
+// Number of entries of the list with index < t * kDecTile (by a search that assumes the list ascending; the tile kernel
+// checks that it is).  Bound by the memory lines it asks for, one for nearly
 // every probe: a list that a hash chose is spread evenly, so the place is guessed from the key and then from what
 // was found at the guess, a little further than needed so that the answer gets bracketed from both sides; a
 // handful of probes leaves a stretch inside a line or two, which is bisected (any list is, after kDecGuesses
@@ -42,13 +42,7 @@ struct DecLists {
 constexpr int kDecGuesses = 6;
 constexpr uint32_t kDecNear = 16;
 template <typename I>
-__global__ __launch_bounds__(256) void k_decode_starts(DecLists lists, int64_t ntiles, int64_t dense_n,
-                                                       uint32_t *__restrict__ starts) {
-  const int l = blockIdx.y;
-  const int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
-  if (t > ntiles) return;
-  const I *list = static_cast<const I *>(lists.idx[l]);
-  const uint32_t len = lists.len[l];
+__device__ inline uint32_t decode_start(const I *__restrict__ list, uint32_t len, int64_t t, int64_t ntiles, int64_t dense_n) {
   uint32_t lo = 0, hi = len;  // the answer lies in [lo, hi]
   if (t == 0 || len == 0) {
     hi = 0;
@@ -72,7 +66,26 @@ __global__ __launch_bounds__(256) void k_decode_starts(DecLists lists, int64_t n
       if ((int64_t)list[mid] < key) lo = mid + 1u; else hi = mid;
     }
   }
-  starts[(int64_t)l * (ntiles + 1) + t] = lo;
+  return lo;
+}
+
+// Tiles that have looked at their entries, counted for the host: a line takes ten nanoseconds for an add, so the tiles
+// form groups with a counter each.  Few tiles search for themselves and count in the status word, above its flags.
+constexpr int kDecGroups = 64, kDecPad = 32;
+constexpr int kDecCounters = (kDecGroups + 1) * kDecPad;
+constexpr int64_t kDecFew = 256;
+constexpr int kDecFlags = 8;
+
+// starts[l * (ntiles + 1) + t]: decode_start of list l.
+template <typename I>
+__global__ __launch_bounds__(256) void k_decode_starts(DecLists lists, int64_t ntiles, int64_t dense_n,
+                                                       uint32_t *__restrict__ starts, uint32_t *__restrict__ counters) {
+  const int l = blockIdx.y;
+  const int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (blockIdx.x == 0 && l == 0 && threadIdx.x <= kDecGroups) counters[threadIdx.x * kDecPad] = 0;
+  if (t > ntiles) return;
+  starts[(int64_t)l * (ntiles + 1) + t] =
+      decode_start(static_cast<const I *>(lists.idx[l]), lists.len[l], t, ntiles, dense_n);
 }
 
 // The value a dense element gets from one entry: +0 + v in fp32, rounded to the tensor's type (-0 becomes +0,
@@ -106,10 +119,13 @@ __device__ inline void store_vec(const S (&e)[16 / sizeof(S)], S *__restrict__ d
 // flight and no entry has to look for its list.  (Entries numbered through and dealt to threads one by one, each
 // bisecting for its list and waiting for its own load: 182 us for 28.7 M entries of sixteen lists into 62 M bf16
 // elements, now 80.)
-template <typename I, typename S>
+// The host is told by the tile that is the last to have looked at its entries: what is left then are stores.  FEW: the
+// tile finds its stretches itself, two waves for both ends (a launch less, a chain of probes more).
+template <typename I, typename S, bool FEW>
 __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int64_t ntiles,
-                                                            const uint32_t *__restrict__ starts, S *__restrict__ dense,
-                                                            int64_t dense_n, int32_t *status) {
+                                                            const uint32_t *__restrict__ starts,
+                                                            uint32_t *__restrict__ counters, S *__restrict__ dense,
+                                                            int64_t dense_n, HostAnswer answer, int32_t *status) {
   // the tile in the tensor's own type or, where lists meet, as fp32 sums
   __shared__ __attribute__((aligned(16))) float acc[kDecTile];
   __shared__ uint32_t occ[kDecTile / 32];
@@ -121,8 +137,32 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t t = blockIdx.x;
   const int64_t first = t * (int64_t)kDecTile;
+  __shared__ uint32_t s_ends[FEW ? 2 : 1][64];
+  // one thread, when the workgroup's flags are in the status word: counts the tile; true for the last of all
+  auto counted = [&]() {
+    if (FEW) return (uint32_t)atomicAdd(status, 1 << kDecFlags);
+    return atomicAdd(&counters[(t % kDecGroups) * kDecPad], 1u);
+  };
+  auto tell = [&](uint32_t before) {
+    if (FEW) {
+      if ((before >> kDecFlags) != (uint32_t)ntiles - 1u) return;
+      const int32_t flags = (int32_t)(before & ((1u << kDecFlags) - 1u));
+      __hip_atomic_store(status, flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      host_store(answer.host + 1, (int64_t)flags);
+    } else {
+      const uint32_t g = (uint32_t)(t % kDecGroups), groups = ntiles < kDecGroups ? (uint32_t)ntiles : (uint32_t)kDecGroups;
+      if (before != (uint32_t)((ntiles - g + kDecGroups - 1) / kDecGroups) - 1u) return;
+      if (atomicAdd(&counters[kDecGroups * kDecPad], 1u) != groups - 1u) return;
+      host_store(answer.host + 1, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    }
+    wait_global_acks();
+    host_store(answer.host, answer.ticket);
+  };
   uint32_t a = 0, b = 0;  // asked for first: the answer is on its way while the tile is cleared
-  if (lane < lists.n) {
+  if (FEW) {
+    if (wave < 2 && lane < lists.n)
+      s_ends[wave][lane] = decode_start(static_cast<const I *>(lists.idx[lane]), lists.len[lane], t + wave, ntiles, dense_n);
+  } else if (lane < lists.n) {
     const uint32_t *at = starts + (int64_t)lane * (ntiles + 1) + t;
     a = at[0];
     b = at[1];
@@ -131,6 +171,13 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
     reinterpret_cast<uint4 *>(acc)[j] = make_uint4(0, 0, 0, 0);
   if (tid < kDecTile / 32) occ[tid] = 0;
   if (tid == 0) s_count = s_wrong = 0;
+  if (FEW) {
+    __syncthreads();
+    if (lane < lists.n) {
+      a = s_ends[0][lane];
+      b = s_ends[FEW ? 1 : 0][lane];
+    }
+  }
   bool wrong = b < a;  // the search went astray: the list is not ascending
   const uint32_t len = wrong ? 0u : b - a;
   const uint32_t chunks = (len + kDecChunk - 1) / kDecChunk;
@@ -176,7 +223,11 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
   if (wrong) s_wrong = 1;
   __syncthreads();
   if (s_wrong) {
-    if (tid == 0) atomicOr(status, ZEN_STAT_RETRY);
+    if (tid == 0) {
+      atomicOr(status, ZEN_STAT_RETRY);
+      wait_global_acks();
+      if (answer.host) tell(counted());
+    }
     return;  // the caller repeats the whole call: what this tile holds does not matter
   }
   {  // as many different elements as entries?
@@ -185,13 +236,16 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
   }
   __syncthreads();
   const bool aligned = (reinterpret_cast<uintptr_t>(dense + first) & 15u) == 0;
+  uint32_t before = 0;
   if (s_count == total) {
+    if (answer.host && tid == 0) before = counted();  // (on its way while the tile is written)
     for (int j = tid * V; j < kDecTile; j += kDecBlock * V) {
       S e[V];
       const uint4 q = *reinterpret_cast<const uint4 *>(tile + j);
       __builtin_memcpy(e, &q, 16);
       store_vec<S>(e, dense, first + j, dense_n, aligned);
     }
+    if (answer.host && tid == 0) tell(before);
     return;
   }
   // Two lists share an index here: fp32 sums, the lists one after the other (inside a list every index occurs
@@ -200,6 +254,9 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
   for (int j = tid; j < kDecTile / 4; j += kDecBlock) reinterpret_cast<uint4 *>(acc)[j] = make_uint4(0, 0, 0, 0);
   __syncthreads();
   constexpr int kAhead = 8;
+  // (an entry of some list, for lists with nothing in the tile)
+  const int other = __ffsll((unsigned long long)__ballot(a < b)) - 1;
+  const uint32_t other_at = (uint32_t)__builtin_amdgcn_readlane((int)a, other);
   for (int l0 = 0; l0 < lists.n; l0 += kAhead) {
     // an entry of each list per thread, in no branch (a list with nothing for this thread reads some entry), so
     // that all are in flight together
@@ -211,8 +268,8 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
       const uint32_t la = (uint32_t)__builtin_amdgcn_readlane((int)a, l);
       const uint32_t lb = (uint32_t)__builtin_amdgcn_readlane((int)b, l);
       const bool some = la < lb;
-      const I *idx = some ? static_cast<const I *>(lists.idx[l]) + la : reinterpret_cast<const I *>(starts);
-      const S *val = some ? static_cast<const S *>(lists.val[l]) + la : reinterpret_cast<const S *>(starts);
+      const I *idx = some ? static_cast<const I *>(lists.idx[l]) + la : static_cast<const I *>(lists.idx[other]) + other_at;
+      const S *val = some ? static_cast<const S *>(lists.val[l]) + la : static_cast<const S *>(lists.val[other]) + other_at;
       const uint32_t e = la + (uint32_t)tid < lb ? (uint32_t)tid : 0u;
       k[i] = idx[e];
       v[i] = val[e];
@@ -230,23 +287,32 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
       }
     }
   }
+  if (answer.host && tid == 0) before = counted();
   for (int j = tid * V; j < kDecTile; j += kDecBlock * V) {
     S e[V];
 #pragma unroll
     for (int q = 0; q < V; ++q) e[q] = rounded(acc[j + q], S(0));
     store_vec<S>(e, dense, first + j, dense_n, aligned);
   }
+  if (answer.host && tid == 0) tell(before);
 }
 
 template <typename I, typename S>
-int decode_sorted_launch(const DecLists &lists, void *dense, int64_t dense_n, uint32_t *starts, int32_t *status,
-                         hipStream_t s) {
+int decode_sorted_launch(const DecLists &lists, void *dense, int64_t dense_n, uint32_t *workspace, int32_t *status,
+                         hipStream_t s, const HostAnswer &answer) {
   const int64_t ntiles = ceil_div(dense_n, (int64_t)kDecTile);
-  k_decode_starts<I><<<dim3((unsigned)ceil_div(ntiles + 1, (int64_t)256), (unsigned)lists.n), dim3(256), 0, s>>>(
-      lists, ntiles, dense_n, starts);
-  ZEN_LAUNCH_CHECK("k_decode_starts");
-  k_decode_tiles<I, S><<<dim3((unsigned)ntiles), dim3(kDecBlock), 0, s>>>(lists, ntiles, starts,
-                                                                          static_cast<S *>(dense), dense_n, status);
+  S *out = static_cast<S *>(dense);
+  if (ntiles <= kDecFew) {
+    k_decode_tiles<I, S, true><<<dim3((unsigned)ntiles), dim3(kDecBlock), 0, s>>>(lists, ntiles, nullptr, nullptr, out,
+                                                                                 dense_n, answer, status);
+  } else {
+    uint32_t *counters = workspace, *starts = workspace + kDecCounters;
+    k_decode_starts<I><<<dim3((unsigned)ceil_div(ntiles + 1, (int64_t)256), (unsigned)lists.n), dim3(256), 0, s>>>(
+        lists, ntiles, dense_n, starts, counters);
+    ZEN_LAUNCH_CHECK("k_decode_starts");
+    k_decode_tiles<I, S, false><<<dim3((unsigned)ntiles), dim3(kDecBlock), 0, s>>>(lists, ntiles, starts, counters, out,
+                                                                                  dense_n, answer, status);
+  }
   ZEN_LAUNCH_CHECK("k_decode_tiles");
   return ZEN_OK;
 }
@@ -259,12 +325,12 @@ extern "C" {
 size_t zen_decode_dense_sorted_workspace(int64_t dense_n, int nlists) {
   if (dense_n <= 0 || nlists <= 0) return 256;
   const int64_t ntiles = zen::ceil_div(dense_n, (int64_t)zen::kDecTile);
-  return (size_t)((ntiles + 1) * nlists) * sizeof(uint32_t) + 256;
+  return ((size_t)((ntiles + 1) * nlists) + zen::kDecCounters) * sizeof(uint32_t) + 256;
 }
 
-int zen_decode_dense_lists(const void *const *idx, int idx64_in, const void *const *val, int dtype, const int64_t *len,
-                           int nlists, void *dense, int64_t dense_n, void *workspace, size_t workspace_bytes,
-                           int32_t *status, void *stream) {
+static int decode_lists_call(const void *const *idx, int idx64_in, const void *const *val, int dtype, const int64_t *len,
+                             int nlists, void *dense, int64_t dense_n, void *workspace, size_t workspace_bytes,
+                             int32_t *status, void *stream, const zen::HostAnswer &answer) {
   using namespace zen;
   if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_decode_dense_lists: bad dtype");
   if (!dense || !status || !idx || !val || !len || !workspace)
@@ -284,12 +350,29 @@ int zen_decode_dense_lists(const void *const *idx, int idx64_in, const void *con
   if (workspace_bytes < zen_decode_dense_sorted_workspace(dense_n, nlists))
     return fail(ZEN_EWORKSPACE, "zen_decode_dense_lists: workspace too small");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  uint32_t *starts = static_cast<uint32_t *>(workspace);
+  uint32_t *ws = static_cast<uint32_t *>(workspace);
   if (dtype == ZEN_BF16)
-    return idx64_in ? decode_sorted_launch<int64_t, uint16_t>(lists, dense, dense_n, starts, status, s)
-                    : decode_sorted_launch<int32_t, uint16_t>(lists, dense, dense_n, starts, status, s);
-  return idx64_in ? decode_sorted_launch<int64_t, uint32_t>(lists, dense, dense_n, starts, status, s)
-                  : decode_sorted_launch<int32_t, uint32_t>(lists, dense, dense_n, starts, status, s);
+    return idx64_in ? decode_sorted_launch<int64_t, uint16_t>(lists, dense, dense_n, ws, status, s, answer)
+                    : decode_sorted_launch<int32_t, uint16_t>(lists, dense, dense_n, ws, status, s, answer);
+  return idx64_in ? decode_sorted_launch<int64_t, uint32_t>(lists, dense, dense_n, ws, status, s, answer)
+                  : decode_sorted_launch<int32_t, uint32_t>(lists, dense, dense_n, ws, status, s, answer);
+}
+
+int zen_decode_dense_lists(const void *const *idx, int idx64_in, const void *const *val, int dtype, const int64_t *len,
+                           int nlists, void *dense, int64_t dense_n, void *workspace, size_t workspace_bytes,
+                           int32_t *status, void *stream) {
+  return decode_lists_call(idx, idx64_in, val, dtype, len, nlists, dense, dense_n, workspace, workspace_bytes, status, stream, {});
+}
+
+int zen_decode_dense_lists_status(const void *const *idx, int idx64_in, const void *const *val, int dtype, const int64_t *len,
+                                  int nlists, void *dense, int64_t dense_n, void *workspace, size_t workspace_bytes,
+                                  int32_t *status, int64_t *host, int64_t words, void *stream) {
+  using namespace zen;
+  HostAnswer answer;
+  int rc = host_ask(host, words, 1, &answer);
+  if (rc != ZEN_OK) return rc;
+  rc = decode_lists_call(idx, idx64_in, val, dtype, len, nlists, dense, dense_n, workspace, workspace_bytes, status, stream, answer);
+  return rc == ZEN_OK ? host_wait(answer, static_cast<hipStream_t>(stream)) : rc;
 }
 
 int zen_decode_dense_sorted(const void *idx, int idx64_in, const void *val, int dtype, const int64_t *list_start,

@@ -5,6 +5,7 @@
 //
 // A library function arrives as the ctypes object that stands for it, so that whoever replaces the library replaces it
 // here too; ctypes lets other threads run while the function does.
+#include <c10/core/impl/DeviceGuardImplInterface.h>
 #include <torch/extension.h>
 
 #include <algorithm>
@@ -181,22 +182,41 @@ bool matching_runs(const std::vector<Tensor> &indices, const std::vector<Tensor>
 }
 
 py::tuple decode_lists(const py::object &fn, Zeros &zeros, const std::vector<Tensor> &indices,
-                        const std::vector<Tensor> &values, int code, int64_t dense_size, const Tensor &ws, int64_t stream) {
+                       const std::vector<Tensor> &values, int code, int64_t dense_size, const Tensor &ws, int64_t stream,
+                       int64_t host, int64_t words) {
   const Tensor dense = room(values[0], dense_size, values[0].scalar_type()), status = zeros.status(values[0], stream);
   const Lists i(indices), v(values);
   const py::object rc = fn(i.addresses(), indices[0].scalar_type() == at::kLong ? 1 : 0, v.addresses(), code, i.counts(),
-                           indices.size(), address(dense), dense_size, address(ws), ws.numel(), address(status), stream);
-  return py::make_tuple(rc, dense, status);
+                           indices.size(), address(dense), dense_size, address(ws), ws.numel(), address(status), host, words,
+                           stream);
+  return py::make_tuple(rc, dense);
 }
 
 py::tuple bitmaps_dense(const py::object &fn, Zeros &zeros, const std::vector<Tensor> &bitmaps,
                         const std::vector<Tensor> &values, int code, const Tensor &dict, int64_t numel, const Tensor &ws,
-                        int64_t stream) {
+                        int64_t stream, int64_t host, int64_t words) {
   const Tensor dense = room(values[0], numel, values[0].scalar_type()), status = zeros.status(values[0], stream);
   const Lists b(bitmaps), v(values);
   const py::object rc = fn(address(dict), numel, bitmaps.size(), b.addresses(), b.counts(), v.addresses(), code, v.counts(),
-                           address(dense), address(ws), ws.numel(), address(status), stream);
-  return py::make_tuple(rc, dense, status);
+                           address(dense), address(ws), ws.numel(), address(status), host, words, stream);
+  // the call returns while its last kernel reads these: their memory is not handed out before that, also if it belongs to
+  // another stream's pool and its owner drops it now
+  if (dense.is_cuda()) {
+    const c10::Stream now = c10::impl::getDeviceGuardImpl(dense.device().type())->getStream(dense.device());
+    for (const auto *list : {&bitmaps, &values})
+      for (const Tensor &t : *list) t.record_stream(now);
+    dict.record_stream(now);
+  }
+  return py::make_tuple(rc, dense);
+}
+
+py::tuple bitmap_encode(const py::object &fn, Zeros &zeros, const Tensor &mapping, const Tensor &indices, const Tensor &ranks,
+                        int64_t numel, int64_t count, int64_t stream, int64_t host, int64_t words) {
+  const Tensor bitmap = room(indices, std::max<int64_t>(count, 1) * 4, at::kByte), status = zeros.status(indices, stream);
+  const py::object rc = fn(address(mapping), mapping.numel(), address(indices), indices.scalar_type() == at::kLong ? 1 : 0,
+                           indices.numel(), py::none(), address(ranks), numel, address(bitmap), address(status), host, words,
+                           stream);
+  return py::make_tuple(rc, bitmap.narrow(0, 0, (mapping.numel() + 7) / 8));
 }
 
 py::tuple tables(const py::object &fn, Zeros &zeros, const Tensor &input, int code, int64_t m, int64_t serial_n,
@@ -284,6 +304,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("matching_runs", &matching_runs);
   m.def("decode_lists", &decode_lists);
   m.def("bitmaps_dense", &bitmaps_dense);
+  m.def("bitmap_encode", &bitmap_encode);
   m.def("tables", &tables);
   m.def("table_find", &table_find);
   m.def("table_gather", &table_gather);
