@@ -343,6 +343,29 @@ def test_two_slots_in_flight_give_the_same_answer(zen, oracle):
 # ------------------------------------------------------------------ merge
 
 
+def test_resident_launches_on_streams_that_take_turns(zen, oracle):
+    """Calls on the default stream and on two others in every order, none waited for, each with a slot of its own."""
+    n, P, k = 3 << 20, 8, 20000
+    rng = np.random.default_rng(77)
+    tp = zen.TensorPartition(P, 1, 3)
+    streams = [torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.Stream()]
+    cases = []
+    for slot in range(4):
+        g = (rng.standard_normal(n) * 1e-3).astype(np.float32)
+        masked, _ = oracle.mask_dense(g, oracle.kth_key(g, k))
+        cases.append((to_dev(g), oracle.load_balance(masked, P, 1, 3)))
+    torch.cuda.synchronize()
+    got = []
+    for call, which in enumerate([0, 0, 1, 1, 0, 2, 1, 0, 0, 2, 2, 0]):
+        with torch.cuda.stream(streams[which]):
+            got.append(tp.load_balance_flat(cases[call % 4][0], capacity=2 * k, k=k, slot=call))
+    torch.cuda.synchronize()
+    for call, (oi, ov, splits, status) in enumerate(got):
+        idx_o, val_o, splits_o, _ = cases[call % 4][1]
+        assert status.item() == 0 and np.array_equal(to_np(splits), splits_o)
+        assert np.array_equal(to_np(oi)[:len(idx_o)], idx_o) and np.array_equal(to_np(ov)[:len(idx_o)], val_o)
+
+
 def payloads(oracle, rng, n, peers, per_peer, overlap, dtype):
     pool = rng.choice(n, max(1, int(per_peer * overlap) * 2), replace=False)
     idx, val = [], []
