@@ -115,6 +115,29 @@ def test_call_that_waits_gives_the_same_on_every_path(zen, oracle, n, P, density
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("P,per_part", [(4, 800), (4, 960), (4, 1000), (2, 1024), (16, 1024)])
+def test_slab_load_balance_at_a_round_of_records(zen, oracle, P, per_part, dtype):
+    """Wide buckets whose slabs' parts hold fewer records than the workgroup has threads, more, or some of each: it keeps
+    them in registers in the first case and loads them round by round in the others.  Hundreds lose their slot."""
+    if FLAGS:
+        pytest.skip("covered by the other run")
+    n = 1 << 20
+    k = per_part * 8 * 16
+    x = (np.random.default_rng(P * per_part).standard_normal(n) * 1e-3).astype(np.float32)
+    x[0] = 0
+    g = x if dtype == "f32" else (x.view(np.uint32) >> 16).astype(np.uint16)
+    masked, kept = oracle.mask_dense(g, int(oracle.kth_key(g, k)))
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(masked, P, 1, 3)
+    capacity = kept + 1024
+    assert st_o == 0 and lb_path(zen, n, P, dtype, capacity, k=k) == WIDE
+    tp = zen.TensorPartition(P, 1, 3)
+    oi, ov, splits, status = tp.load_balance_flat(to_dev(g), capacity=capacity, k=k)
+    assert status.item() == 0 and np.array_equal(to_np(splits), splits_o)
+    assert np.array_equal(to_np(oi)[:kept], idx_o) and np.array_equal(to_np(ov)[:kept], val_o)
+    assert not tp._table(torch.device("cuda"), n).any()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
 def test_slab_load_balance_odd_length_unaligned_and_empty(zen, oracle, dtype):
     """A tensor whose length is no multiple of anything and whose first element is not 16-byte aligned (the
     streaming kernel's element-wise loads and its ragged last tile), and a tensor of zeros."""

@@ -107,7 +107,6 @@ int wide_device_cus() {
 namespace {
 
 constexpr int kWideRounds = 3;                          // a part of a bucket's slab is read in rounds of kWideBlock records
-constexpr int kWideItems = kWideSplit * kWideRounds;    // raw records per thread (candidates below the threshold included)
 constexpr int kWidePartMax = kWideBlock * kWideRounds;  // raw records of one part, at most
 constexpr int kWideMove = 1024;                         // entries that may move into one bucket from elsewhere
 constexpr int kWideRemoved = 1024;                      // entries of a bucket that may lose their level-1 slot
@@ -117,7 +116,6 @@ constexpr int kWideGroupLimit = 512;                    // records in one narrow
 constexpr int kWideIndexStep = 4;                       // every 4th narrow range has its first sorted place written down
 constexpr int kWideIndexLen = kWideSubs / kWideIndexStep;
 constexpr int kWideCtrPad = 8;                          // words between two per-partition counters
-constexpr int kWideSteps = kWideSplit * kWideRounds / 4;  // = kWideItems / kWideLanes
 constexpr int kWideProbeLimit = 512;                    // probes in the map before it counts as full
 constexpr uint32_t kInvalid = 0xffffffffu;
 // a record's raw place: part * 4096 + place inside the part
@@ -171,6 +169,7 @@ struct WideShared {
       uint32_t q_range[kWideQueue];  // where its narrow range starts | where it ends << 16
     };
   };
+  uint32_t gone[kWideRemoved];  // sorted places of the entries that lost their slot, as they come up
   int32_t delta[kWideCap / 64];
   uint32_t scan[kWideBlock / 64 + 1];
   uint64_t scan64[kWideBlock / 64 + 1];
@@ -255,58 +254,30 @@ __device__ unsigned long long g_wide_dbg[256 * 32];
 #define WIDE_MARK(k) do { } while (0)
 #endif
 
-template <typename S>
-__global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g, WideTables tb,
-                                                          const uint32_t *__restrict__ filter,
-                                                          unsigned long long *cells, int64_t spp,
-                                                          const S *__restrict__ dense, int32_t *__restrict__ out_idx,
-                                                          S *__restrict__ out_val, uint32_t capacity,
-                                                          int64_t *__restrict__ splits, uint32_t *clear,
-                                                          uint32_t clear_words, uint32_t *clear_too,
-                                                          uint32_t clear_too_words, HostAnswer answer, int32_t *status) {
-  __shared__ WideShared<S> sh;
-  const uint32_t b = blockIdx.x, B = geo.nbuckets, bpp = geo.bpp;
-  const uint32_t part = b / bpp;
+// Puts the bucket's records that reach the threshold in order of (level-1 slot, index): indices to sh.idx, values to sh.val
+// (the losers of a slot marked, their places and indices noted in sh.gone and sh.rm), the narrow ranges' first places to
+// memory for the look-ups of other workgroups.  Returns how many there are.  ROUNDS: of kWideBlock records of every part.
+// One round, up to eight records a thread, is written out, its records stay in registers from their load to the end; of
+// three the loops' bodies handle the first kWideLanes registers of a set and then rotate the set, and the records are
+// loaded again (written out, the code would no longer fit the instruction cache, and every workgroup runs it just once).
+// A chain of LDS and memory trips bounds it, not a rate.  Written out, with the records held and the removed places noted
+// instead of searched for, the launch takes 31 us where the loops took 36 (62 M bf16 elements, 0.5 %, 128 workgroups) and
+// 24 where they took 28 (1 M fp32, 1 %, 16 workgroups).
+template <typename S, int ROUNDS>
+__device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, const WideTables &tb, const uint2 *records,
+                                     const uint2 (&first_round)[kWideSplit], const uint32_t (&pcount)[kWideSplit],
+                                     uint32_t longest, uint32_t thr_key, bool declined, uint32_t b, int32_t *status) {
+  constexpr int kItems = kWideSplit * ROUNDS, kSteps = kItems / kWideLanes;
+  constexpr bool kHeld = ROUNDS == 1;
   const uint32_t tid = threadIdx.x;
-  WIDE_MARK(0);
-  // counters of the kernels before this one that nobody needs any more: back to zero, a slice per workgroup
-  for (uint32_t i = b * kWideBlock + tid; i < clear_words; i += B * kWideBlock) clear[i] = 0;
-  for (uint32_t i = b * kWideBlock + tid; i < clear_too_words; i += B * kWideBlock) clear_too[i] = 0;  // fp32: the refinement's histogram
-  if (tid == 0) {
-    sh.lo = geo.first_key(b);
-    sh.lost_n = sh.nrm = sh.mv_n = sh.ser_n = sh.big = 0;
-  }
-  sh.cnt.clear();
-  // the bucket's candidates sit in kWideSplit parts; item r * kWideSplit + q of a thread is the record at
-  // place tid + r * kWideBlock of part q
-  uint32_t pcount[kWideSplit];
-  uint32_t longest = 0;
-#pragma unroll
-  for (int q = 0; q < kWideSplit; ++q) {
-    pcount[q] = tb.cursor[(b * kWideSplit + q) * kWidePad];
-    if (pcount[q] > tb.part_cap) pcount[q] = tb.part_cap;  // the producer flagged the overflow
-    longest = pcount[q] > longest ? pcount[q] : longest;
-  }
-  bool declined = false;
-  if (longest > (uint32_t)kWidePartMax) {  // more candidates than the workgroup looks at: another path answers
-    declined = true;
-#pragma unroll
-    for (int q = 0; q < kWideSplit; ++q) pcount[q] = 0;
-    longest = 0;
-  }
-  const uint32_t thr_key = filter ? filter[0] : 0u;
-  // the bucket's records: (index, value bits), kWideSplit parts of part_cap records
-  const uint2 *records = reinterpret_cast<const uint2 *>(tb.words) + (size_t)b * kWideSplit * tb.part_cap;
-  __syncthreads();
   const uint32_t lo = sh.lo;
   const int shift = geo.sub_shift;
   const uint32_t low_mask = (1u << shift) - 1u;
-
   // ---- slot offsets in registers; loads in no branch (places past a part's end are pulled back onto its
   // first record), so that all are in flight together
-  uint32_t off[kWideItems];
+  uint32_t off[kItems];
 #pragma unroll
-  for (int r = 0; r < kWideRounds; ++r) {
+  for (int r = 0; r < ROUNDS; ++r) {
 #pragma unroll
     for (int q = 0; q < kWideSplit; ++q) off[r * kWideSplit + q] = kInvalid;
     if ((uint32_t)r * kWideBlock < longest) {
@@ -314,7 +285,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
       for (int q = 0; q < kWideSplit; ++q) {
         const uint32_t e = tid + (uint32_t)r * kWideBlock;
         const size_t at = (size_t)q * tb.part_cap + (e < pcount[q] ? e : 0u);
-        const uint2 rec = records[at];
+        const uint2 rec = r == 0 ? first_round[q] : records[at];
         const uint32_t slot = geo.mod_m(poly(rec.x) + kSeed1);  // the level-1 slot: a dozen instructions, not a plane of its own
         const bool keep = e < pcount[q] && (rec.y & KeyOf<S>::kMask) >= thr_key;
         off[r * kWideSplit + q] = keep ? slot - lo : kInvalid;
@@ -323,7 +294,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   }
   WIDE_MARK(1);
 #pragma unroll
-  for (int i = 0; i < kWideItems; ++i)
+  for (int i = 0; i < kItems; ++i)
     if (off[i] != kInvalid) sh.cnt.count(off[i] >> shift);
   __syncthreads();
   // a narrow range that holds hundreds of records (keys piled on a few values) would keep the rank loop busy
@@ -335,23 +306,20 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
     __syncthreads();
     sh.cnt.clear();
 #pragma unroll
-    for (int i = 0; i < kWideItems; ++i) off[i] = kInvalid;
+    for (int i = 0; i < kItems; ++i) off[i] = kInvalid;
     n = 0;
     __syncthreads();
   }
   if (declined && tid == 0) atomicOr(status, ZEN_STAT_RETRY);
-  // From here on a thread's records are worked through in kWideSteps steps of kWideLanes records, by a loop
-  // whose body always handles the first kWideLanes registers of the set and then rotates the set: with the
-  // body written out for all records the kernel's code no longer fits the instruction cache, and every
-  // workgroup runs it just once.
-  auto rotate = [](uint32_t (&a)[kWideItems]) {
+  auto rotate = [](uint32_t (&a)[kItems]) {
+    if (kHeld) return;
     uint32_t head[kWideLanes];
 #pragma unroll
     for (int k = 0; k < kWideLanes; ++k) head[k] = a[k];
 #pragma unroll
-    for (int i = 0; i + kWideLanes < kWideItems; ++i) a[i] = a[i + kWideLanes];
+    for (int i = 0; i + kWideLanes < kItems; ++i) a[i] = a[i + kWideLanes];
 #pragma unroll
-    for (int k = 0; k < kWideLanes; ++k) a[kWideItems - kWideLanes + k] = head[k];
+    for (int k = 0; k < kWideLanes; ++k) a[kItems - kWideLanes + k] = head[k];
   };
   // raw place of the record in lane k of step s: part * 4096 + place inside the part
   auto raw_place = [&](int s, int k) {
@@ -360,40 +328,43 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   };
   // steps of rounds that no part of the slab reaches hold nothing: the loops stop short of them
   const int steps = longest == 0 ? 0 : (int)((longest + kWideBlock - 1) / kWideBlock) * (kWideSplit / kWideLanes);
-#pragma unroll 1
-  for (int s = 0; s < kWideSteps; ++s) {
-    if (s < steps) {
+  auto take_step = [&](int s, int from) {
 #pragma unroll
-      for (int k = 0; k < kWideLanes; ++k) {
-        if (off[k] != kInvalid) {
-          const uint32_t p = sh.cnt.take(off[k] >> shift);
-          sh.word[p] = ((off[k] & low_mask) << 15) | raw_place(s, k);
-        }
+    for (int k = 0; k < kWideLanes; ++k) {
+      if (off[from + k] != kInvalid) {
+        const uint32_t p = sh.cnt.take(off[from + k] >> shift);
+        sh.word[p] = ((off[from + k] & low_mask) << 15) | raw_place(s, k);
       }
     }
-    rotate(off);
+  };
+  if (kHeld) {
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) take_step(s, s * kWideLanes);
+  } else {
+#pragma unroll 1
+    for (int s = 0; s < kSteps; ++s) {
+      if (s < steps) take_step(s, 0);
+      rotate(off);
+    }
   }
   __syncthreads();
   WIDE_MARK(2);
   // rank = records of the bucket with a smaller (slot, index): the records of the narrow ranges before it,
   // plus those of its own range with a smaller slot, plus (rare) those with its slot and a smaller index.
-  // A round's eight records at a time: first where every record's range starts and ends, then the range's
-  // first three words of each (most ranges hold no more), all in flight together.
-  uint32_t rk[kWideItems];
+  // A step's records together: first where every record's range starts and ends, then the range's
+  // first four words of each (most ranges hold no more), all in flight together.
+  uint32_t rk[kItems];
   auto raw_at = [&](uint32_t j) { return (size_t)(j >> 12) * tb.part_cap + (j & 4095u); };
 #pragma unroll
-  for (int i = 0; i < kWideItems; ++i) rk[i] = kInvalid;
-#pragma unroll 1
-  for (int s = 0; s < kWideSteps; ++s) {
+  for (int i = 0; i < kItems; ++i) rk[i] = kInvalid;
+  auto rank_step = [&](int s, int from, uint32_t (&out)[kWideLanes]) {
     constexpr int kAhead = 4;
-    uint32_t out[kWideLanes];
 #pragma unroll
     for (int k = 0; k < kWideLanes; ++k) out[k] = kInvalid;
-    if (s < steps) {
     uint32_t g0[kWideLanes], g1[kWideLanes], a[kWideLanes][kAhead];
 #pragma unroll
     for (int k = 0; k < kWideLanes; ++k) {
-      const uint32_t sub = off[k] != kInvalid ? off[k] >> shift : 0u;
+      const uint32_t sub = off[from + k] != kInvalid ? off[from + k] >> shift : 0u;
       g0[k] = sh.cnt.start_of(sub);
       g1[k] = sh.cnt.end_of(sub);
     }
@@ -405,8 +376,8 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
     }
 #pragma unroll
     for (int k = 0; k < kWideLanes; ++k) {
-      if (off[k] != kInvalid) {
-        const uint32_t key = off[k] & low_mask;
+      if (off[from + k] != kInvalid) {
+        const uint32_t key = off[from + k] & low_mask;
         const uint32_t my = (key << 15) | raw_place(s, k);
         uint32_t less = 0, twins = 0;
 #pragma unroll
@@ -432,17 +403,31 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
         out[k] = x;
       }
     }
-    }
-    rotate(off);
-    rotate(rk);  // the step's ranks enter at the end: after the last step rank i belongs to record i
+  };
+  if (kHeld) {
 #pragma unroll
-    for (int k = 0; k < kWideLanes; ++k) rk[kWideItems - kWideLanes + k] = out[k];
-    WIDE_MARK(16 + s);
+    for (int s = 0; s < kSteps; ++s) {
+      uint32_t out[kWideLanes];
+      rank_step(s, s * kWideLanes, out);
+#pragma unroll
+      for (int k = 0; k < kWideLanes; ++k) rk[s * kWideLanes + k] = out[k];
+    }
+  } else {
+#pragma unroll 1
+    for (int s = 0; s < kSteps; ++s) {
+      uint32_t out[kWideLanes];
+#pragma unroll
+      for (int k = 0; k < kWideLanes; ++k) out[k] = kInvalid;
+      if (s < steps) rank_step(s, 0, out);
+      rotate(off);
+      rotate(rk);  // the step's ranks enter at the end: after the last step rank i belongs to record i
+#pragma unroll
+      for (int k = 0; k < kWideLanes; ++k) rk[kItems - kWideLanes + k] = out[k];
+    }
   }
   WIDE_MARK(22);
   __syncthreads();
   {
-    WIDE_MARK(23);
     uint32_t pending = sh.lost_n;
     if (pending > (uint32_t)kWideQueue) {
       if (tid == 0) atomicOr(status, ZEN_STAT_RETRY);
@@ -467,27 +452,24 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
       }
       sh.q_word[e] = (g0 + less + lost) | (lost ? kRemovedBit : 0u);  // the entry's thread is its only reader
     }
-    WIDE_MARK(24);
+    // the narrow ranges' first places go to memory for the other workgroups' look-ups before the values take
+    // the counters' place
+    for (uint32_t j = tid; j < (uint32_t)kWideIndexLen; j += kWideBlock) {
+      const uint32_t s0 = j * kWideIndexStep;
+      store_agent(&tb.sub_index[(size_t)b * kWideIndexLen + j],
+                  sh.cnt.start_of(s0) | (sh.cnt.end_of(s0 + kWideIndexStep - 1) << 16));
+    }
     __syncthreads();
-    WIDE_MARK(25);
 #pragma unroll
-    for (int i = 0; i < kWideItems; ++i)
+    for (int i = 0; i < kItems; ++i)
       if (rk[i] != kInvalid && (rk[i] & kRemovedBit)) rk[i] = sh.q_word[rk[i] & kIndexMask];
     __syncthreads();  // the queue's memory serves other lists from here on
     if (tid == 0) sh.lost_n = 0;
   }
   __syncthreads();
   WIDE_MARK(3);
-  // the narrow ranges' first places go to memory for the other workgroups' look-ups before the values take
-  // the counters' place
-  for (uint32_t j = tid; j < (uint32_t)kWideIndexLen; j += kWideBlock) {
-    const uint32_t s0 = j * kWideIndexStep;
-    store_agent(&tb.sub_index[(size_t)b * kWideIndexLen + j],
-                sh.cnt.start_of(s0) | (sh.cnt.end_of(s0 + kWideIndexStep - 1) << 16));
-  }
-  __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kWideRounds; ++r) {
+  for (int r = 0; r < ROUNDS; ++r) {
     if ((uint32_t)r * kWideBlock < longest) {
       uint32_t t[kWideSplit];
       S v[kWideSplit];
@@ -495,7 +477,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
       for (int q = 0; q < kWideSplit; ++q) {
         const uint32_t e = tid + (uint32_t)r * kWideBlock;
         const size_t at = (size_t)q * tb.part_cap + (rk[r * kWideSplit + q] != kInvalid ? e : 0u);
-        const uint2 rec = records[at];
+        const uint2 rec = kHeld ? first_round[q] : records[at];
         t[q] = rec.x;
         v[q] = (S)rec.y;
       }
@@ -508,7 +490,10 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
           sh.val[p] = v[q];
           if (x & kRemovedBit) {
             const uint32_t at = atomicAdd(&sh.lost_n, 1u);
-            if (at < (uint32_t)kWideRemoved) sh.rm[at] = t[q];
+            if (at < (uint32_t)kWideRemoved) {
+              sh.rm[at] = t[q];
+              sh.gone[at] = p;
+            }
           }
         }
       }
@@ -516,12 +501,67 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   }
   __syncthreads();
   WIDE_MARK(4);
+  return n;
+}
+
+template <typename S>
+__global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g, WideTables tb,
+                                                          const uint32_t *__restrict__ filter,
+                                                          unsigned long long *cells, int64_t spp,
+                                                          const S *__restrict__ dense, int32_t *__restrict__ out_idx,
+                                                          S *__restrict__ out_val, uint32_t capacity,
+                                                          int64_t *__restrict__ splits, uint32_t *clear,
+                                                          uint32_t clear_words, uint32_t *clear_too,
+                                                          uint32_t clear_too_words, HostAnswer answer, int32_t *status) {
+  __shared__ WideShared<S> sh;
+  const uint32_t b = blockIdx.x, B = geo.nbuckets, bpp = geo.bpp;
+  const uint32_t part = b / bpp;
+  const uint32_t tid = threadIdx.x;
+  WIDE_MARK(0);
+  // the bucket's records: (index, value bits), kWideSplit parts of part_cap records; item r * kWideSplit + q of a thread is
+  // the record at place tid + r * kWideBlock of part q.  The first round is asked for before it is known how many there
+  // are (a part has room for more than a round): a trip to memory less.
+  const uint2 *records = reinterpret_cast<const uint2 *>(tb.words) + (size_t)b * kWideSplit * tb.part_cap;
+  uint2 first_round[kWideSplit];
+#pragma unroll
+  for (int q = 0; q < kWideSplit; ++q) first_round[q] = records[(size_t)q * tb.part_cap + tid];
+  // counters of the kernels before this one that nobody needs any more: back to zero, a slice per workgroup
+  for (uint32_t i = b * kWideBlock + tid; i < clear_words; i += B * kWideBlock) clear[i] = 0;
+  for (uint32_t i = b * kWideBlock + tid; i < clear_too_words; i += B * kWideBlock) clear_too[i] = 0;  // fp32: the refinement's histogram
+  if (tid == 0) {
+    sh.lo = geo.first_key(b);
+    sh.lost_n = sh.nrm = sh.mv_n = sh.ser_n = sh.big = 0;
+  }
+  sh.cnt.clear();
+  uint32_t pcount[kWideSplit];
+  uint32_t longest = 0;
+#pragma unroll
+  for (int q = 0; q < kWideSplit; ++q) {
+    pcount[q] = tb.cursor[(b * kWideSplit + q) * kWidePad];
+    if (pcount[q] > tb.part_cap) pcount[q] = tb.part_cap;  // the producer flagged the overflow
+    longest = pcount[q] > longest ? pcount[q] : longest;
+  }
+  bool declined = false;
+  if (longest > (uint32_t)kWidePartMax) {  // more candidates than the workgroup looks at: another path answers
+    declined = true;
+#pragma unroll
+    for (int q = 0; q < kWideSplit; ++q) pcount[q] = 0;
+    longest = 0;
+  }
+  const uint32_t thr_key = filter ? filter[0] : 0u;
+  __syncthreads();
+  const uint32_t n = longest <= (uint32_t)kWideBlock
+                         ? wide_sort<S, 1>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, status)
+                         : wide_sort<S, kWideRounds>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, status);
   uint32_t lost_n = sh.lost_n;
   if (lost_n > (uint32_t)kWideRemoved) {
     if (tid == 0) atomicOr(status, ZEN_STAT_RETRY);
     lost_n = kWideRemoved;
   }
-  if (tid == 0) sh.base = lost_n ? atomicAdd(&tb.log_n[part * kWideCtrPad], lost_n) : 0u;
+  if (tid == 0) {
+    sh.base = lost_n ? atomicAdd(&tb.log_n[part * kWideCtrPad], lost_n) : 0u;
+    sh.nrm = lost_n;  // (their places are the first of sh.gone)
+  }
   for (uint32_t p = tid; p < n; p += kWideBlock) store_agent(&tb.slab_idx[(size_t)b * kWideCap + p], sh.idx[p]);
   __syncthreads();
   for (uint32_t i = tid; i < lost_n; i += kWideBlock) {
@@ -607,7 +647,11 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
     const size_t at_log = (size_t)part * tb.log_cap + (first ? i : i - losers);
     const uint32_t t = load_agent(first ? &tb.log_t[at_log] : &tb.dlog_t[at_log]);
     const uint32_t from = first ? 0u : load_agent(&tb.dlog_at[at_log]);
-    if (!first && (from >> 16) == b && (from & 0xffffu) < n) sh.idx[from & 0xffffu] |= kRemovedBit;  // pushed out once
+    if (!first && (from >> 16) == b && (from & 0xffffu) < n) {  // pushed out, once
+      sh.idx[from & 0xffffu] |= kRemovedBit;
+      const uint32_t at = atomicAdd(&sh.nrm, 1u);
+      if (at < (uint32_t)kWideRemoved) sh.gone[at] = from & 0xffffu;
+    }
     uint32_t prt = 0, cell = kNone, slot = kNone;
     for (int lv = 1; lv < g.levels && slot == kNone; ++lv) {
       const uint32_t s = probe_slot(g, t, lv, &prt);
@@ -645,13 +689,6 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
     if (tid == 0) atomicOr(status, (int64_t)kSlabSerialCap >= spp ? ZEN_STAT_SERIAL_OVERFLOW : ZEN_STAT_RETRY);
     serial = kSlabSerialCap;
   }
-  for (uint32_t p = tid; p < n; p += kWideBlock) {
-    if (sh.idx[p] & kRemovedBit) {
-      const uint32_t at = atomicAdd(&sh.nrm, 1u);
-      if (at < (uint32_t)kWideRemoved) sh.rm[at] = p;
-    }
-  }
-  __syncthreads();
   uint32_t rm_n = sh.nrm;
   if (rm_n > (uint32_t)kWideRemoved) {  // more collisions than this path carries
     if (tid == 0) atomicOr(status, ZEN_STAT_RETRY);
@@ -667,8 +704,8 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
     // the bucket, whose slots are hashed again)
     uint32_t x = 0, xr = 0;
     if (tid < rm_n) {
-      x = sh.rm[tid];
-      for (uint32_t u = 0; u < rm_n; ++u) xr += sh.rm[u] < x;
+      x = sh.gone[tid];
+      for (uint32_t u = 0; u < rm_n; ++u) xr += sh.gone[u] < x;
     }
     uint32_t mj = 0, mplace = 0;
     if (tid < mv_n) {
