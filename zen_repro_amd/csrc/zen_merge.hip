@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
   const int nb = (int)geo.nbuckets;
   if (b >= nb) return;
   const size_t base = (size_t)b * kSlabCap;
-  uint32_t n_raw = cursor[b * kCursorPad];
+  uint32_t n_raw = cursor[b];
   if (n_raw > (uint32_t)kSlabCap) n_raw = kSlabCap;  // the scatter flagged the overflow
   const uint32_t lo = bucket_lo[b];
   // The counters of the scatter kernels go back to zero (this workgroup was the only reader of its slab's
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
   }
   uint32_t n = 0;
   const bool ranked = slab_rank<kMergeBlock>(sh, geo, tie_bits, off, arr, live, rank, &n);
-  if (threadIdx.x == 0) cursor[b * kCursorPad] = 0;  // every thread has read it: slab_rank synchronised
+  if (threadIdx.x == 0) cursor[b] = 0;  // every thread has read it: slab_rank synchronised
   if (!ranked) {
     if (threadIdx.x == 0) atomicOr(status, ZEN_STAT_RETRY);
     n = 0;  // the bucket contributes nothing; the prefix protocol still gets its (empty) tile
@@ -546,7 +546,7 @@ int merge_one_launch(const void *idx, int idx64_in, const S *val, int64_t r, int
 // kernel that would clear it.
 constexpr size_t kMergeZeroBytes =
     ((scan_words_c(kSlabMaxBuckets) * sizeof(unsigned long long) + 255) / 256 * 256) +
-    (size_t)kCoarseCursorWords * sizeof(uint32_t) + (size_t)kSlabMaxBuckets * kCursorPad * sizeof(uint32_t);
+    (size_t)kCoarseCursorWords * sizeof(uint32_t) + (size_t)kSlabMaxBuckets * sizeof(uint32_t);
 
 struct SlabMergePlan {
   unsigned long long *scan;  // prefix state over the buckets (zeroed before use)
@@ -564,7 +564,7 @@ SlabMergePlan plan_slab_merge(void *workspace, const SlabGeom &geo, int64_t r) {
   const size_t B = geo.nbuckets;
   p.scan = cv.take<unsigned long long>(scan_words((int64_t)B));
   p.feed.coarse_cursor = cv.take<uint32_t>(feed_coarse_cursor_words());
-  p.feed.cursor = cv.take<uint32_t>(B * kCursorPad);
+  p.feed.cursor = cv.take<uint32_t>(B);
   p.zero_bytes = cv.used;
   cv.used = kMergeZeroBytes;  // whatever the geometry, the rest starts behind the largest zero region
   p.feed.bucket_lo = cv.take<uint32_t>(B);

@@ -33,7 +33,7 @@ __global__ __launch_bounds__(kRefineBlock) void k_refine_threshold(CoarseGeom cg
   // a workgroup takes several parts: every workgroup ends with an atomic on one counter, and a thousand of
   // those stand in line for 11 us
   for (uint32_t part = blockIdx.x; part < parts; part += gridDim.x) {
-    uint32_t count = coarse_cursor[part * kCoarsePad];
+    uint32_t count = coarse_cursor[coarse_cursor_at(part / kCoarseSplit, part % kCoarseSplit)];
     if (count > cg.cap) count = cg.cap;
     const uint32_t *vals = val_plane < 0 ? coarse_words + (size_t)part * cg.cap * 2 + 1
                                          : coarse_words + (size_t)val_plane * plane + (size_t)part * cg.cap;

@@ -779,7 +779,7 @@ __device__ inline void stage_flush(uint32_t count, int32_t *st_idx, S *st_val, S
     const uint32_t before = block_exclusive_scan<uint32_t, kSelBlock>(c, fl.scan, &total);
     if (threadIdx.x < ndst) {
       fl.pref[threadIdx.x] = before;
-      fl.gbase[threadIdx.x] = c ? atomicAdd(&out.cursor[(threadIdx.x * kCoarseSplit + part) * kCoarsePad], c) : 0u;
+      fl.gbase[threadIdx.x] = c ? atomicAdd(&out.cursor[coarse_cursor_at(threadIdx.x, part)], c) : 0u;
     }
     if (threadIdx.x == 0) fl.pref[ndst] = total;
   }

@@ -34,7 +34,7 @@ namespace zen {
 namespace {
 
 struct SlabTables {
-  uint32_t *cursor;     // [B * kCursorPad] records in the bucket's slab, at [b * kCursorPad]
+  uint32_t *cursor;     // [B] records in the bucket's slab
   uint32_t *bucket_lo;  // [B] smallest level-1 slot of the bucket
   uint32_t *bucket_n;   // [B] sorted records in the slab: level-1 owners, in wide buckets the losers too
   uint32_t *removed_n;  // [B] of which have lost their slot
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabT
   const uint32_t b = blockIdx.x;
   const size_t base = (size_t)b * kSlabCap;
   const uint32_t words = (geo.span + 63u) / 64u;
-  uint32_t n_raw = tb.cursor[b * kCursorPad];
+  uint32_t n_raw = tb.cursor[b];
   if (n_raw > (uint32_t)kSlabCap) n_raw = kSlabCap;  // the scatter flagged the overflow
   const uint32_t lo = tb.bucket_lo[b];
   S *slab_val = static_cast<S *>(tb.slab_val);
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabT
     if (j < n_raw) live |= 1u << i;
   }
   __syncthreads();  // the bitmap is clear, and everybody has read the slab's fill count
-  if (threadIdx.x == 0) tb.cursor[b * kCursorPad] = 0;
+  if (threadIdx.x == 0) tb.cursor[b] = 0;
   // no branch around a wave's marks either: a lane without a record marks nothing
 #pragma unroll
   for (int i = 0; i < kSortItems; ++i) {
@@ -256,7 +256,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort_wide(SlabGeom geo, 
   __shared__ uint32_t s_lost, s_base;
   const uint32_t b = blockIdx.x;
   const size_t base = (size_t)b * kSlabCap;
-  uint32_t n_raw = tb.cursor[b * kCursorPad];
+  uint32_t n_raw = tb.cursor[b];
   if (n_raw > (uint32_t)kSlabCap) n_raw = kSlabCap;  // the scatter flagged the overflow
   const uint32_t lo = tb.bucket_lo[b];
   S *slab_val = static_cast<S *>(tb.slab_val);
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort_wide(SlabGeom geo, 
   uint32_t n = 0;
   if (!slab_rank<kSortBlock>(sh, geo, 13, off, pos, live, rank, &n)) {
     if (threadIdx.x == 0) {
-      tb.cursor[b * kCursorPad] = 0;
+      tb.cursor[b] = 0;
       atomicOr(status, ZEN_STAT_RETRY);
       tb.bucket_n[b] = 0;
       tb.removed_n[b] = 0;
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort_wide(SlabGeom geo, 
     return;
   }
   // every thread has read the slab's fill count (slab_rank synchronised); this workgroup was its only reader
-  if (threadIdx.x == 0) tb.cursor[b * kCursorPad] = 0;
+  if (threadIdx.x == 0) tb.cursor[b] = 0;
   // the counters hold where every narrow range starts in the sorted bucket: every kSlabIndexStep-th goes to
   // the index (before the counters' memory is used for the ties below)
   for (int j = threadIdx.x; j < kSlabIndexLen; j += kSortBlock)
@@ -904,7 +904,7 @@ SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partit
     p.sample_hist[1] = cv.take<uint32_t>(sampled_floor_zero_bytes() / sizeof(uint32_t));
     p.cand_hist = cv.take<uint32_t>((size_t)kCandHistWords);
     p.ticket = cv.take<uint32_t>(select_stage_ticket_words());
-    p.tb.cursor = cv.take<uint32_t>(B * kCursorPad);
+    p.tb.cursor = cv.take<uint32_t>(B);
     p.feed.coarse_cursor = cv.take<uint32_t>(feed_coarse_cursor_words());
     p.tb.movein_n = cv.take<uint32_t>(B * kMoveinPad);
     p.tb.serial_n = cv.take<uint32_t>((size_t)partitions * kMoveinPad);

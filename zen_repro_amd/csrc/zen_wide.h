@@ -24,8 +24,7 @@ constexpr int kWideSubs = 16384;                    // narrow key ranges inside 
 constexpr int kWideTarget = 15360;                  // records a bucket is sized for
 constexpr int kWideMaxBuckets = 256;
 constexpr int kWideSplit = kCoarseSplit;            // parts of a bucket's slab
-constexpr int kWidePad = kCoarsePad;                // words between two part cursors
-constexpr uint32_t kWideCursorWords = kWideMaxBuckets * kWideSplit * kWidePad;
+static_assert(kWideMaxBuckets <= kCoarseRow, "a part cursor for every bucket");
 
 // Buckets for `partitions` partitions of a key space of m keys expected to hold about `expected` records, on
 // a chip of `cus` compute units; false if the layout does not suit these sizes.  The result is a SlabGeom
@@ -163,9 +162,8 @@ __device__ inline uint32_t load_agent(const uint32_t *p) {
 // 2^23) in bits 0-22, the arrival number (below 2^25) in bits 23-47 and, for bf16, the value in bits 48-63;
 // fp32 values travel in a word plane of their own.  One store per record, and a run of eight fills a line.
 constexpr uint32_t kWmOffBits = 23, kWmArrBits = 25;
-constexpr int kWmPad = 8;  // words between two part cursors
 struct WideSlabs {
-  uint32_t *cursor;    // [nbuckets * kWideSplit * kWmPad], zero before the scatter; the bucket's workgroup puts them back
+  uint32_t *cursor;    // [kCoarseCursorWords], zero before the scatter; the bucket's workgroup puts its own back
   uint2 *rec;          // [nbuckets * kWideSplit * part_cap]
   uint32_t *val32;     // fp32 values (unused for bf16)
   uint32_t part_cap;
@@ -248,7 +246,7 @@ __device__ inline void wide_scatter_batch(const WideList &a, uint32_t batch, uin
     const uint32_t before = total + block_exclusive_scan<uint32_t, BLOCK>(c, sh.scan, &turn);
     if (b < nb) {
       sh.pref[b] = before;
-      sh.gbase[b] = c ? atomicAdd(&a.out.cursor[(b * kWideSplit + part) * kWmPad], c) : 0u;
+      sh.gbase[b] = c ? atomicAdd(&a.out.cursor[coarse_cursor_at(b, part)], c) : 0u;
     }
     total += turn;
   }

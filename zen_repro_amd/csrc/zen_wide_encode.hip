@@ -115,6 +115,7 @@ constexpr int kWideLanes = 4;                           // records a thread hand
 constexpr int kWideGroupLimit = 512;                    // records in one narrow range: bounds the rank loop
 constexpr int kWideIndexStep = 4;                       // every 4th narrow range has its first sorted place written down
 constexpr int kWideIndexLen = kWideSubs / kWideIndexStep;
+constexpr int kWidePad = 32;                            // words between two barrier counters
 constexpr int kWideCtrPad = 8;                          // words between two per-partition counters
 constexpr int kWideProbeLimit = 512;                    // probes in the map before it counts as full
 constexpr uint32_t kInvalid = 0xffffffffu;
@@ -126,7 +127,7 @@ static_assert(kWideMove < (1 << 12) && kWideRemoved < (1 << 12), "two counts in 
 
 struct WideTables {
   // zero between calls (kept in the caller's zero table, behind the hash map)
-  uint32_t *cursor;            // [B * kWideSplit * kWidePad] part cursors
+  uint32_t *cursor;            // [kCoarseCursorWords] part cursors
   uint32_t *gbar;              // [P * kWidePad] barrier counters of the partitions' workgroups
   uint32_t *pdone;             // [P * kWidePad] workgroups of the partition that have finished
   uint32_t *log_n;             // [P * kWideCtrPad] entries that lost level 1, per partition
@@ -537,7 +538,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   uint32_t longest = 0;
 #pragma unroll
   for (int q = 0; q < kWideSplit; ++q) {
-    pcount[q] = tb.cursor[(b * kWideSplit + q) * kWidePad];
+    pcount[q] = tb.cursor[coarse_cursor_at(b, q)];
     if (pcount[q] > tb.part_cap) pcount[q] = tb.part_cap;  // the producer flagged the overflow
     longest = pcount[q] > longest ? pcount[q] : longest;
   }
@@ -819,7 +820,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   // the partition's workgroup that finishes last (all of them are through with the map and the logs then)
   // empties the cells the partition holds and clears its counters; the launch's last workgroup clears what
   // the buckets published.
-  if (tid < (uint32_t)kWideSplit) tb.cursor[(b * kWideSplit + tid) * kWidePad] = 0;
+  if (tid < (uint32_t)kWideSplit) tb.cursor[coarse_cursor_at(b, tid)] = 0;
   wait_global_acks();
   __syncthreads();
   if (tid == 0) {
@@ -877,7 +878,7 @@ WidePlan plan_wide(void *workspace, void *state, const SlabGeom &geo, int partit
     p.sample_hist[1] = cv.take<uint32_t>(sampled_floor_zero_bytes() / sizeof(uint32_t));
     p.cand_hist = cv.take<uint32_t>((size_t)kCandHistWords);
     p.ticket = cv.take<uint32_t>(select_stage_ticket_words());
-    p.tb.cursor = cv.take<uint32_t>(B * kWideSplit * kWidePad);
+    p.tb.cursor = cv.take<uint32_t>(kCoarseCursorWords);
     p.tb.gbar = cv.take<uint32_t>(P * kWidePad);
     p.tb.pdone = cv.take<uint32_t>(P * kWidePad);
     p.tb.log_n = cv.take<uint32_t>(P * kWideCtrPad);

@@ -14,8 +14,6 @@
 namespace zen {
 namespace {
 
-constexpr uint32_t kWmCursorWords = kWideMaxBuckets * kWideSplit * kWmPad;
-static_assert(kWmCursorWords <= kCoarseCursorWords, "the cursors fit the zero region of the slab path's coarse cursors");
 constexpr int kWmRounds = 3;                               // a part of a bucket's slab is read in rounds of kWideBlock records
 constexpr int kWmItems = kWideSplit * kWmRounds;           // records per thread
 constexpr int kWmPartMax = kWideBlock * kWmRounds;         // records of one part, at most
@@ -113,7 +111,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
   uint32_t longest = 0;
 #pragma unroll
   for (int q = 0; q < kWideSplit; ++q) {
-    pcount[q] = in.cursor[(b * kWideSplit + q) * kWmPad];
+    pcount[q] = in.cursor[coarse_cursor_at(b, q)];
     if (pcount[q] > in.part_cap) pcount[q] = in.part_cap;  // the scatter flagged the overflow
     longest = pcount[q] > longest ? pcount[q] : longest;
   }
@@ -168,7 +166,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
   }
   if (declined && tid == 0) atomicOr(status, ZEN_STAT_RETRY);
   // this workgroup was the only reader of its part cursors: back to zero for the next call
-  if (tid < (uint32_t)kWideSplit) in.cursor[(b * kWideSplit + tid) * kWmPad] = 0;
+  if (tid < (uint32_t)kWideSplit) in.cursor[coarse_cursor_at(b, tid)] = 0;
 
   // The thread's records are worked through in steps of kWmLanes, by loops whose body handles the first
   // kWmLanes registers of a set and then rotates the set (the body written out for all records would not fit
