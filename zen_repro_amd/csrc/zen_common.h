@@ -181,6 +181,19 @@ __device__ inline uint32_t load_fresh(const uint32_t *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Counts workgroup `index` of `total` as finished (by one thread of it, once what the last one is to find has been carried
+// out); true for the last of them.  A word takes one add after the other, ten nanoseconds each, and workgroups that end
+// together would stand in line for it: they count in kDoneGroups words, and the last of each group in one more (the select
+// kernel's 768 workgroups on 62 M bf16 elements 35.2 us with one word, 31.8 so; 1536 of k_merge_bucket 87.8 and 79.4).
+// words: kDoneWords of them, zero, each counter in a memory line of its own.
+constexpr uint32_t kDoneGroups = 16, kDonePad = 32;
+constexpr uint32_t kDoneWords = (kDoneGroups + 1) * kDonePad;
+__device__ inline bool done_last(uint32_t *words, uint32_t index, uint32_t total) {
+  const uint32_t g = index % kDoneGroups, groups = total < kDoneGroups ? total : kDoneGroups;
+  if (atomicAdd(&words[g * kDonePad], 1u) != (total - g + kDoneGroups - 1u) / kDoneGroups - 1u) return false;
+  return atomicAdd(&words[kDoneGroups * kDonePad], 1u) == groups - 1u;
+}
+
 // Where the host waits for what a call has to know there (zen_readback.hip): pinned words, of which word 0 takes the
 // ticket once the others hold the answer.  The kernel that knows the answer stores it, where that is one of the call's
 // own: no launch for it, and what is left of the call's work runs while the host goes on.

@@ -280,7 +280,7 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
                                                              const uint32_t *__restrict__ slab_arr,
                                                              const S *__restrict__ slab_val,
                                                              I *__restrict__ out_idx, O *__restrict__ out_val,
-                                                             int64_t capacity, ScanState st, int tie_bits,
+                                                             int64_t capacity, ScanState st, uint32_t *done, int tie_bits,
                                                              int64_t *out_count, HostAnswer answer, int32_t *status) {
   __shared__ SlabSortShared sh;  // the values take the counters' place once the ranks are known
   __shared__ uint64_t s_scan64[kMergeBlock / 64 + 1];
@@ -394,17 +394,14 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
     }
   }
   // every workgroup has read the descriptors it needs before it gets here
-  uint32_t *finished = reinterpret_cast<uint32_t *>(st.desc + nb + 1);
   if (answer.host) wait_global_acks();  // its share of the status word, and the count
   __syncthreads();
-  if (threadIdx.x == 0) s_tile = atomicAdd(finished, 1u) == (uint32_t)nb - 1u;
+  if (threadIdx.x == 0) s_tile = done_last(done, (uint32_t)b, (uint32_t)nb);
   __syncthreads();
   if (s_tile) {
     for (int i = threadIdx.x; i < nb; i += kMergeBlock) st.desc[i] = 0ull;
-    if (threadIdx.x == 0) {
-      *st.ticket = 0;
-      *finished = 0;
-    }
+    for (uint32_t i = threadIdx.x; i < kDoneWords; i += kMergeBlock) done[i] = 0;
+    if (threadIdx.x == 0) *st.ticket = 0;
     host_answer_count(answer, out_count, status);
   }
 }
@@ -544,12 +541,14 @@ int merge_one_launch(const void *idx, int idx64_in, const S *val, int64_t r, int
 // counters, for the largest geometry.  It sits at the head of the workspace whatever path a call takes, and a
 // call on bucket slabs leaves it zero again, so that a caller who vouches for it (ZEN_MODE_ZEROED) saves the
 // kernel that would clear it.
+constexpr size_t kDoneBytes = (kDoneWords * sizeof(uint32_t) + 255) / 256 * 256;
 constexpr size_t kMergeZeroBytes =
     ((scan_words_c(kSlabMaxBuckets) * sizeof(unsigned long long) + 255) / 256 * 256) +
-    (size_t)kCoarseCursorWords * sizeof(uint32_t) + (size_t)kSlabMaxBuckets * sizeof(uint32_t);
+    (size_t)kCoarseCursorWords * sizeof(uint32_t) + kDoneBytes + (size_t)kSlabMaxBuckets * sizeof(uint32_t);
 
 struct SlabMergePlan {
   unsigned long long *scan;  // prefix state over the buckets (zeroed before use)
+  uint32_t *done;            // [kDoneWords] buckets merged (the same)
   CoarseGeom cg;
   FeedBuffers feed;
   uint32_t *slab_idx, *slab_arr;
@@ -564,6 +563,7 @@ SlabMergePlan plan_slab_merge(void *workspace, const SlabGeom &geo, int64_t r) {
   const size_t B = geo.nbuckets;
   p.scan = cv.take<unsigned long long>(scan_words((int64_t)B));
   p.feed.coarse_cursor = cv.take<uint32_t>(feed_coarse_cursor_words());
+  p.done = cv.take<uint32_t>(kDoneWords);
   p.feed.cursor = cv.take<uint32_t>(B);
   p.zero_bytes = cv.used;
   cv.used = kMergeZeroBytes;  // whatever the geometry, the rest starts behind the largest zero region
@@ -607,13 +607,13 @@ int slab_merge_launch(const SlabGeom &geo, const I *idx, const S *val, int64_t r
   if (idx64_out)
     k_merge_bucket<int64_t, S, O><<<dim3(geo.nbuckets), dim3(kMergeBlock), 0, s>>>(
         geo, p.feed.cursor, p.feed.coarse_cursor, p.feed.bucket_lo, p.slab_idx, p.slab_arr,
-        static_cast<const S *>(p.slab_val), static_cast<int64_t *>(out_idx), out_val, capacity, st, tie_bits, out_count,
-        ask.answer, status);
+        static_cast<const S *>(p.slab_val), static_cast<int64_t *>(out_idx), out_val, capacity, st, p.done, tie_bits,
+        out_count, ask.answer, status);
   else
     k_merge_bucket<int32_t, S, O><<<dim3(geo.nbuckets), dim3(kMergeBlock), 0, s>>>(
         geo, p.feed.cursor, p.feed.coarse_cursor, p.feed.bucket_lo, p.slab_idx, p.slab_arr,
-        static_cast<const S *>(p.slab_val), static_cast<int32_t *>(out_idx), out_val, capacity, st, tie_bits, out_count,
-        ask.answer, status);
+        static_cast<const S *>(p.slab_val), static_cast<int32_t *>(out_idx), out_val, capacity, st, p.done, tie_bits,
+        out_count, ask.answer, status);
   ZEN_LAUNCH_CHECK("k_merge_bucket");
   if (ask.answer.host) *ask.answered = true;
   return ZEN_OK;
@@ -677,12 +677,13 @@ int merge_launch(const void *idx, int idx64_in, const S *val, int64_t r, int64_t
     Carver cv(workspace);
     unsigned long long *scan = cv.take<unsigned long long>(scan_words((int64_t)kSlabMaxBuckets));
     uint32_t *cursor = cv.take<uint32_t>(feed_coarse_cursor_words());
+    uint32_t *done = cv.take<uint32_t>(kDoneWords);
     if (!zeroed) {
       launch_fill<unsigned long long>(scan, 0ull, kMergeZeroBytes / sizeof(unsigned long long), s);
       ZEN_LAUNCH_CHECK("merge: clear prefix state");
     }
     WideList list;
-    if (!wide_merge_list(idx, idx64_in, val, r, dense_n, cursor, static_cast<char *>(workspace) + kMergeZeroBytes,
+    if (!wide_merge_list(idx, idx64_in, val, r, dense_n, cursor, done, static_cast<char *>(workspace) + kMergeZeroBytes,
                          wide_device_cus(), status, &list, ask.answer.host != nullptr))
       return fail(ZEN_EINVAL, "zen_merge: sizes do not suit the wide buckets");
     return wide_merge(list, sizeof(S) == 2 ? ZEN_BF16 : ZEN_F32, out_idx, idx64_out, out_val,

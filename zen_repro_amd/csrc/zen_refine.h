@@ -10,6 +10,7 @@ namespace {
 // --------------------------------------------- fp32: the threshold's last 16 bits
 
 constexpr int kRefineBins = 65536;
+constexpr int kRefineWords = kRefineBins + (int)kDoneWords;  // (and the count of finished workgroups)
 constexpr int kRefineBlock = 512;
 
 // The candidates' histogram resolves the 15 leading bits of an fp32 key: after the select kernel thr[0] is
@@ -18,7 +19,7 @@ constexpr int kRefineBlock = 512;
 // bin (they sit in word plane `val_plane` of the coarse slabs, or with val_plane < 0 in the second word of the
 // wide buckets' two-word records; element 0, which is never handed on, is looked at in the tensor), and the
 // workgroup that finishes last replaces thr[0..1] by the exact key and the number of elements at or above it.
-// Grid: any number of workgroups, which take the parts of the coarse slabs in turn.  hist: kRefineBins + 1 zeroed words.
+// Grid: any number of workgroups, which take the parts of the coarse slabs in turn.  hist: kRefineWords zeroed words.
 __global__ __launch_bounds__(kRefineBlock) void k_refine_threshold(CoarseGeom cg, int val_plane,
                                                                    const uint32_t *__restrict__ coarse_cursor,
                                                                    const uint32_t *__restrict__ coarse_words,
@@ -49,7 +50,7 @@ __global__ __launch_bounds__(kRefineBlock) void k_refine_threshold(CoarseGeom cg
   }
   wait_global_acks();
   __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(&hist[kRefineBins], 1u) == gridDim.x - 1u;
+  if (threadIdx.x == 0) s_last = done_last(&hist[kRefineBins], blockIdx.x, gridDim.x);
   __syncthreads();
   if (!s_last) return;
   // from the top down: thread t owns the kPer bins below kRefineBins - t * kPer.  The counts were raised

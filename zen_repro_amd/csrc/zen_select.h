@@ -87,7 +87,7 @@ int topk_sampled_floor(const void *in, int dtype, int64_t n, int64_t k, uint32_t
 size_t sampled_floor_zero_bytes();  // leading part of the scratch that must be zero (scratch_is_zero: the caller did it)
 constexpr int kCandBins = 512;   // four octaves of 15-bit magnitudes above the floor; the rest shares the last bin
 constexpr int kCandRows = 8;   // partial candidate histograms (blocks spread over them)
-constexpr int kCandHistWords = kCandRows * kCandBins + 1;
+constexpr int kCandHistWords = kCandRows * kCandBins + (int)kDoneWords;  // (and the count of finished workgroups)
 
 // One pass over a dense tensor, by persistent workgroups, that hands every element with key >= max(thr[0], 1)
 // (thr == nullptr: the nonzero ones) except element 0 to the coarse slabs of zen_slab_feed.h, as (index,

@@ -153,6 +153,8 @@ __global__ __launch_bounds__(kHistBlock) void k_topk_pick(TopkState *st, uint32_
 // 16-bit counters packed two per word; a block never sees more than 65535
 // sample elements, so they cannot overflow into each other.
 constexpr int kFineBins = 32768;
+constexpr int kSampleTop = kFineBins + (int)kDoneWords;  // behind the bins: the count of finished blocks, the highest populated bin
+constexpr size_t kSampleWords = kSampleTop + 1;
 constexpr int kSampleBlock = 1024;
 
 // Device-wide atomics on one 128-byte line are carried out one after the other (about 10 ns each), and the
@@ -164,13 +166,13 @@ __device__ inline uint32_t fine_place(uint32_t bin) { return ((bin & 63u) << 9) 
 // such that `rank` sample elements lie in bins >= b; floor_out[0] = lowest key
 // of that bin (0 if the sample is too small).
 
-// Walks down from the highest populated bin (hist[kFineBins + 1]) in windows of one bin per thread, with
+// Walks down from the highest populated bin (hist[kSampleTop]) in windows of one bin per thread, with
 // consecutive lanes on consecutive words (one workgroup fetching 32768 scattered words past the caches would
 // take tens of microseconds), until `rank` sample elements lie at or above a bin.
 template <int BLOCK>
 __device__ inline void sample_pick_block(const uint32_t *hist, uint32_t rank, int key_shift, uint32_t *floor_out,
                                          uint32_t *smem) {
-  int base = (int)load_fresh(&hist[kFineBins + 1]);
+  int base = (int)load_fresh(&hist[kSampleTop]);
   if (base > kFineBins - 1) base = kFineBins - 1;
   uint32_t cum = 0;
   for (;; base -= BLOCK) {
@@ -248,7 +250,7 @@ __global__ __launch_bounds__(kSampleBlock) void k_sample_hist(const S *__restric
         if (c[j] & 0xffffu) top = 2 * w;
         if (c[j] >> 16) top = 2 * w + 1;
       }
-      atomicMax(&hist[kFineBins + 1], (uint32_t)top);
+      atomicMax(&hist[kSampleTop], (uint32_t)top);
     }
 #pragma unroll
     for (int j = 0; j < kWords; ++j) {
@@ -260,14 +262,14 @@ __global__ __launch_bounds__(kSampleBlock) void k_sample_hist(const S *__restric
       above += lo;
     }
   }
-  // The block that finishes last reads the threshold off the complete histogram (hist[kFineBins] counts
+  // The block that finishes last reads the threshold off the complete histogram (hist[kFineBins] on count
   // finished blocks).  The adds above return nothing, so they are all in flight together.  They are carried
   // out where device-wide atomics are carried out; every wave waits until its own have been acknowledged
   // (a device-scope fence would also write the whole L2 back, once per wave) before this block's count goes
   // up, and the reader loads from that same place (load_fresh).
   wait_global_acks();
   __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(&hist[kFineBins], 1u) == gridDim.x - 1;
+  if (threadIdx.x == 0) s_last = done_last(&hist[kFineBins], blockIdx.x, gridDim.x);
   __syncthreads();
   if (!s_last) return;
   sample_pick_block<kSampleBlock>(hist, rank, kShift, floor_out, smem);
@@ -570,13 +572,13 @@ __global__ __launch_bounds__(kSelBlock) void k_select_compact(
     }
     if (pick_thr) {
       // The block that finishes last reads the exact threshold off the complete histogram
-      // (cand_hist[kCandRows * kCandBins] counts finished blocks).
+      // (behind the rows: the count of finished blocks).
       __shared__ bool s_last;
       // the adds are carried out (where device-wide atomics are) before the count goes up; no device-scope
       // fence: that would write the L2 back once per wave
       wait_global_acks();
       __syncthreads();
-      if (threadIdx.x == 0) s_last = atomicAdd(&cand_hist[kCandRows * kCandBins], 1u) == (uint32_t)ntiles - 1u;
+      if (threadIdx.x == 0) s_last = done_last(&cand_hist[kCandRows * kCandBins], blockIdx.x, (uint32_t)ntiles);
       __syncthreads();
       if (s_last) {
         cand_pick_block<kSelBlock>(cand_hist, floor_key, pick_k, KeyOf<S>::kBits == 15 ? 0 : 16, pick_thr, status,
@@ -959,7 +961,7 @@ __device__ inline void stage_sample_next(const StageSample &smp, uint32_t *windo
     }
     uint32_t total;
     uint32_t above = block_exclusive_scan<uint32_t, kSelBlock>(mine, smem, &total);
-    if (threadIdx.x == 0 && total) atomicMax(&smp.hist[kFineBins + 1], hi_bin);
+    if (threadIdx.x == 0 && total) atomicMax(&smp.hist[kSampleTop], hi_bin);
 #pragma unroll
     for (int j = 0; j < kWords; ++j) {
       const int w = kSampleWindow / 2 - 1 - (threadIdx.x * kWords + j);
@@ -973,7 +975,7 @@ __device__ inline void stage_sample_next(const StageSample &smp, uint32_t *windo
   // the adds are carried out before the workgroup counts itself as finished (see k_sample_hist)
   wait_global_acks();
   __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(&smp.hist[kFineBins], 1u) == smp.wgs - 1u;
+  if (threadIdx.x == 0) s_last = done_last(&smp.hist[kFineBins], blockIdx.x, smp.wgs);
   __syncthreads();
   if (s_last) sample_pick_block<kSelBlock>(smp.hist, smp.rank, kShift, smp.floor_out, smem);
 }
@@ -1224,7 +1226,7 @@ __global__ __launch_bounds__(kSelBlock, 3) void k_select_stage(
       // fence: that would write the L2 back once per wave
       wait_global_acks();
       __syncthreads();
-      if (threadIdx.x == 0) s_last = atomicAdd(&cand_hist[kCandRows * kCandBins], 1u) == gridDim.x - 1u;
+      if (threadIdx.x == 0) s_last = done_last(&cand_hist[kCandRows * kCandBins], blockIdx.x, gridDim.x);
       __syncthreads();
       if (s_last) {
         cand_pick_block<kSelBlock>(cand_hist, floor_key, pick_k, KeyOf<S>::kBits == 15 ? 0 : 16, pick_thr, status,
@@ -1363,7 +1365,7 @@ int sample_launch(const S *in, int64_t n, int64_t k, uint32_t *thr_lo, void *wor
   const int64_t nblocks = sp.nblocks;
   const uint32_t rank = sp.rank;
   if (!is_zero) {
-    launch_fill<uint32_t>(hist, 0u, kFineBins + 2, stream);
+    launch_fill<uint32_t>(hist, 0u, kSampleWords, stream);
     ZEN_LAUNCH_CHECK("sample: clear histogram");
   }
   // every block must see fewer than 65536 sample elements (16-bit LDS counters)
@@ -1404,7 +1406,7 @@ int compress_launch(const S *in, int64_t n, const uint32_t *thr, S *out, hipStre
 
 size_t topk_scratch_bytes() {
   const size_t exact = align_up(sizeof(TopkState), 256) + align_up(kHistBins * sizeof(uint32_t), 256);
-  const size_t sampled = align_up((kFineBins + 2) * sizeof(uint32_t), 256);
+  const size_t sampled = align_up(kSampleWords * sizeof(uint32_t), 256);
   return exact > sampled ? exact : sampled;
 }
 
@@ -1422,7 +1424,7 @@ int topk_sampled_floor(const void *in, int dtype, int64_t n, int64_t k, uint32_t
   return sample_launch(static_cast<const uint32_t *>(in), n, k, thr_lo, scratch, stream, scratch_is_zero);
 }
 
-size_t sampled_floor_zero_bytes() { return (kFineBins + 2) * sizeof(uint32_t); }
+size_t sampled_floor_zero_bytes() { return kSampleWords * sizeof(uint32_t); }
 
 }  // namespace zen
 

@@ -50,7 +50,7 @@ struct SlabTables {
   uint32_t *ser_idx;    // [P * kSlabSerialCap]
   uint32_t *log_t;      // [log_cap] indices that lost level 1
   uint32_t *out_start;  // [B + 1] where every bucket starts in the output
-  uint32_t *done;       // [1] workgroups of k_slab_chains that have finished
+  uint32_t *done;       // [kDoneWords] workgroups of k_slab_chains that have finished
   uint32_t *final_n;    // [B + P] what k_slab_place needs of the counters above, copied by the last workgroup of
                         // k_slab_chains before it puts them back to zero: moved-in entries per bucket, serial
                         // entries per partition
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabT
   for (uint32_t i = b * kSortBlock + threadIdx.x; i < kCoarseCursorWords; i += gridDim.x * kSortBlock)
     tb.coarse_cursor[i] = 0;
   if (tb.refine_hist)
-    for (uint32_t i = b * kSortBlock + threadIdx.x; i <= (uint32_t)kRefineBins; i += gridDim.x * kSortBlock)
+    for (uint32_t i = b * kSortBlock + threadIdx.x; i < (uint32_t)kRefineWords; i += gridDim.x * kSortBlock)
       tb.refine_hist[i] = 0;
   uint32_t off[kSortItems], idx[kSortItems], rank[kSortItems];
   S val[kSortItems];
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort_wide(SlabGeom geo, 
   for (uint32_t i = b * kSortBlock + threadIdx.x; i < kCoarseCursorWords; i += gridDim.x * kSortBlock)
     tb.coarse_cursor[i] = 0;
   if (tb.refine_hist)
-    for (uint32_t i = b * kSortBlock + threadIdx.x; i <= (uint32_t)kRefineBins; i += gridDim.x * kSortBlock)
+    for (uint32_t i = b * kSortBlock + threadIdx.x; i < (uint32_t)kRefineWords; i += gridDim.x * kSortBlock)
       tb.refine_hist[i] = 0;
   uint32_t off[kSortItems], idx[kSortItems], pos[kSortItems], rank[kSortItems];
   S val[kSortItems];
@@ -438,65 +438,74 @@ __device__ inline uint32_t part_min(unsigned long long *cells, const SlabTables 
 // behind its last bucket.  Run by one workgroup of kSlabBlock threads once all counts are final: it is the last
 // to need the counters the chains raised with atomics, hands what k_slab_place still wants of them on in final_n
 // and puts them back to zero.  What the status word can come to is known here too (k_slab_place adds nothing).
-__device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables &tb, uint32_t *s_scan, int64_t spp,
-                                          uint32_t capacity, int64_t *splits, const HostAnswer &answer, int32_t *status) {
-  constexpr int kPer = kSlabMaxBuckets / kSlabBlock;
-  const uint32_t B = geo.nbuckets;
-  uint32_t c[kPer], mv[kPer], rm[kPer];
-  uint32_t sum = 0;
+// The chip waits for this one workgroup: one trip to memory for all counts, and what the host asked for is put together in
+// LDS (s_start: kSlabMaxBuckets + 1 words).
+__device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables &tb, uint32_t *s_scan, uint32_t *s_start,
+                                          int64_t spp, uint32_t capacity, int64_t *splits, const HostAnswer &answer,
+                                          int32_t *status) {
+  constexpr uint32_t kPer = kSlabMaxBuckets / kSlabBlock;
+  const uint32_t B = geo.nbuckets, per = (B + (uint32_t)kSlabBlock - 1u) / (uint32_t)kSlabBlock, x0 = threadIdx.x * per;
+  uint32_t c[kPer], mv[kPer], rm[kPer], sn[kPer];
 #pragma unroll
-  for (int e = 0; e < kPer; ++e) {  // no branch around the loads: all in flight together
-    const uint32_t x = threadIdx.x * kPer + e, at = x < B ? x : 0u;
-    mv[e] = load_fresh(&tb.movein_n[at * kMoveinPad]);
-    rm[e] = load_fresh(&tb.removed_n[at]);
-    c[e] = tb.bucket_n[at];
+  for (uint32_t e = 0; e < kPer; ++e) {
+    if (e < per) {  // the same for all threads; no other branch around the loads: all in flight together
+      const uint32_t at = x0 + e < B ? x0 + e : 0u;
+      mv[e] = load_fresh(&tb.movein_n[at * kMoveinPad]);
+      rm[e] = load_fresh(&tb.removed_n[at]);
+      sn[e] = load_fresh(&tb.serial_n[at / geo.bpp * kMoveinPad]);
+      c[e] = tb.bucket_n[at];
+    }
   }
+  uint32_t sum = 0;
+  bool overflow = false;
 #pragma unroll
-  for (int e = 0; e < kPer; ++e) {
-    const uint32_t x = threadIdx.x * kPer + e;
-    c[e] = x < B ? c[e] - rm[e] + mv[e] : 0u;
-    if (x < B) {
+  for (uint32_t e = 0; e < kPer; ++e) {
+    const uint32_t x = x0 + e;
+    if (e < per && x < B) {
+      c[e] += mv[e] - rm[e];
       tb.final_n[x] = mv[e];
       if (x % geo.bpp == geo.bpp - 1) {
-        const uint32_t sn_raw = load_fresh(&tb.serial_n[x / geo.bpp * kMoveinPad]);
-        tb.final_n[B + x / geo.bpp] = sn_raw;
-        c[e] += sn_raw > (uint32_t)kSlabSerialCap ? (uint32_t)kSlabSerialCap : sn_raw;
+        tb.final_n[B + x / geo.bpp] = sn[e];
+        overflow |= (int64_t)sn[e] > spp;
+        c[e] += sn[e] > (uint32_t)kSlabSerialCap ? (uint32_t)kSlabSerialCap : sn[e];
       }
+      sum += c[e];
     }
-    sum += c[e];
   }
   uint32_t total;
   uint32_t running = block_exclusive_scan<uint32_t, kSlabBlock>(sum, s_scan, &total);
 #pragma unroll
-  for (int e = 0; e < kPer; ++e) {
-    const uint32_t x = threadIdx.x * kPer + e;
-    if (x <= B) tb.out_start[x] = running;
-    running += c[e];
+  for (uint32_t e = 0; e < kPer; ++e) {
+    const uint32_t x = x0 + e;
+    if (e < per && x < B) {
+      tb.out_start[x] = running;
+      if (x % geo.bpp == 0) s_start[x / geo.bpp] = running;
+      running += c[e];
+    }
   }
-  if (B == (uint32_t)kSlabMaxBuckets && threadIdx.x == kSlabBlock - 1) tb.out_start[B] = running;
-  for (uint32_t x = threadIdx.x; x < B; x += kSlabBlock) tb.movein_n[x * kMoveinPad] = 0;
-  for (uint32_t x = threadIdx.x; x < (uint32_t)tb.partitions; x += kSlabBlock) tb.serial_n[x * kMoveinPad] = 0;
   if (threadIdx.x == 0) {
-    *tb.losers = 0;
-    *tb.done = 0;
+    tb.out_start[B] = s_start[tb.partitions] = total;
+    if (total > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
   }
-  // the split sizes: the host has them while the entries are still on their way to their places
+  if (overflow) atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
+  if (answer.host) wait_global_acks();
   __syncthreads();
+  // the split sizes: the host has them while the entries are still on their way to their places
   for (uint32_t p = threadIdx.x; p < (uint32_t)tb.partitions; p += kSlabBlock) {
-    const int64_t size = (int64_t)(tb.out_start[(p + 1u) * geo.bpp] - tb.out_start[p * geo.bpp]);
+    const int64_t size = (int64_t)(s_start[p + 1u] - s_start[p]);
     splits[p] = size;
     if (answer.host) host_store(answer.host + 1 + p, size);
-    if ((int64_t)tb.final_n[B + p] > spp) atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
   }
-  if (threadIdx.x == 0 && tb.out_start[B] > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
   if (answer.host) {
-    wait_global_acks();
-    __syncthreads();
     if (threadIdx.x == 0)
       host_store(answer.host + 1 + tb.partitions,
                  (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     host_answered(answer);
   }
+  for (uint32_t x = threadIdx.x; x < B; x += kSlabBlock) tb.movein_n[x * kMoveinPad] = 0;
+  for (uint32_t x = threadIdx.x; x < (uint32_t)tb.partitions; x += kSlabBlock) tb.serial_n[x * kMoveinPad] = 0;
+  for (uint32_t x = threadIdx.x; x < kDoneWords; x += kSlabBlock) tb.done[x] = 0;
+  if (threadIdx.x == 0) *tb.losers = 0;
 }
 
 // Levels 2 and 3 for the indices that lost level 1, one per thread.  Bound by latency while losers are few (110 000: a
@@ -510,6 +519,7 @@ __global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Pro
                                                             int64_t spp, uint32_t capacity, int64_t *__restrict__ splits,
                                                             HostAnswer answer, int32_t *status) {
   __shared__ uint32_t s_scan[kSlabBlock / 64 + 1];
+  __shared__ uint32_t s_start[kSlabMaxBuckets + 1];
   __shared__ bool s_last;
   uint32_t losers = load_fresh(tb.losers);
   if (losers > tb.log_cap) losers = tb.log_cap;
@@ -574,9 +584,9 @@ __global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Pro
   // the workgroup that finishes last knows every count and lays out the output
   wait_global_acks();
   __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(tb.done, 1u) == working - 1u;
+  if (threadIdx.x == 0) s_last = done_last(tb.done, blockIdx.x, working);
   __syncthreads();
-  if (s_last) slab_output_starts(geo, tb, s_scan, spp, capacity, splits, answer, status);
+  if (s_last) slab_output_starts(geo, tb, s_scan, s_start, spp, capacity, splits, answer, status);
 }
 
 // ------------------------------------------------------------------ place
@@ -909,8 +919,8 @@ SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partit
     p.tb.movein_n = cv.take<uint32_t>(B * kMoveinPad);
     p.tb.serial_n = cv.take<uint32_t>((size_t)partitions * kMoveinPad);
     p.tb.losers = cv.take<uint32_t>(1);
-    p.tb.done = cv.take<uint32_t>(1);
-    p.refine_hist = cv.take<uint32_t>(dtype == ZEN_BF16 ? 1 : (size_t)kRefineBins + 1);
+    p.tb.done = cv.take<uint32_t>(kDoneWords);
+    p.refine_hist = cv.take<uint32_t>(dtype == ZEN_BF16 ? 1 : (size_t)kRefineWords);
     p.state_bytes = cv.used;
   }
   Carver cv(workspace);

@@ -194,6 +194,7 @@ struct WideList {
   uint32_t r, dense_n;
   int idx64;
   WideSlabs out;
+  uint32_t *done;      // [kDoneWords], zero between calls: buckets merged
   int32_t *status;     // BAD_INDEX, RETRY
 };
 
@@ -292,7 +293,7 @@ int wide_device_cus();
 bool wide_merge_fits(int64_t r, int64_t dense_n, int cus, SlabGeom *geo, bool alone = false);
 size_t wide_merge_bytes(int64_t r, int64_t dense_n, int cus);
 bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, int64_t dense_n, uint32_t *cursor,
-                     void *rest, int cus, int32_t *status, WideList *list, bool alone);
+                     uint32_t *done, void *rest, int cus, int32_t *status, WideList *list, bool alone);
 // Lists up to this long take one workgroup (zen_merge.hip).
 constexpr int64_t merge_one_max() { return 6144; }
 int wide_merge(const WideList &list, int dtype, void *out_idx, int idx64_out, void *out_val, int out_dtype,

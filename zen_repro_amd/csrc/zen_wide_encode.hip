@@ -133,7 +133,7 @@ struct WideTables {
   uint32_t *log_n;             // [P * kWideCtrPad] entries that lost level 1, per partition
   uint32_t *dlog_n;            // [P * kWideCtrPad] level-1 owners pushed out by a level-2/3 prober, per partition
   unsigned long long *desc;    // [B] what every bucket contributes to the output (flag + count)
-  uint32_t *done;              // [1] workgroups that have finished
+  uint32_t *done;              // [1] partitions whose workgroups have finished
   Counters *ctr;               // [P] (the claims of the partition's map)
   // workspace
   uint32_t *words;             // [B * kWideSplit * part_cap] raw candidates, two words each: index, value bits
@@ -824,8 +824,8 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   wait_global_acks();
   __syncthreads();
   if (tid == 0) {
-    const uint32_t here = atomicAdd(&tb.pdone[part * kWidePad], 1u), all = atomicAdd(tb.done, 1u);
-    sh.flag = (here == bpp - 1u ? 1u : 0u) | (all == B - 1u ? 2u : 0u);
+    const bool here = atomicAdd(&tb.pdone[part * kWidePad], 1u) == bpp - 1u;
+    sh.flag = !here ? 0u : atomicAdd(tb.done, 1u) == (uint32_t)tb.partitions - 1u ? 3u : 1u;
   }
   __syncthreads();
   WIDE_MARK(13);
@@ -886,7 +886,7 @@ WidePlan plan_wide(void *workspace, void *state, const SlabGeom &geo, int partit
     p.tb.desc = cv.take<unsigned long long>(B);
     p.tb.done = cv.take<uint32_t>(1);
     p.tb.ctr = cv.take<Counters>(P);
-    p.refine_hist = cv.take<uint32_t>(dtype == ZEN_BF16 ? 1 : (size_t)kRefineBins + 1);
+    p.refine_hist = cv.take<uint32_t>(dtype == ZEN_BF16 ? 1 : (size_t)kRefineWords);
     p.state_bytes = cv.used;
   }
   Carver cv(workspace);
@@ -1009,7 +1009,7 @@ int wide_load_balance(const SlabBalanceArgs &a, size_t state_offset, hipStream_t
   }
   const uint32_t *filter = a.k > 0 ? p.thr : nullptr;
   uint32_t *clear_too = refine ? p.refine_hist : nullptr;
-  const uint32_t clear_too_words = refine ? (uint32_t)kRefineBins + 1u : 0u;
+  const uint32_t clear_too_words = refine ? (uint32_t)kRefineWords : 0u;
   if ((rc = wide_line_enter(s)) != ZEN_OK) return rc;
   {
     ProfScope prof(kProfWideTail, s);

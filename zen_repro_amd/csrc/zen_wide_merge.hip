@@ -396,16 +396,13 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
   if (answer.host) wait_global_acks();  // its share of the status word, and the count
   // every workgroup has read the descriptors it needs before it gets here: the last one to finish clears the
   // prefix state
-  uint32_t *finished = reinterpret_cast<uint32_t *>(st.desc + nb + 1);
   __syncthreads();
-  if (tid == 0) sh.tile = atomicAdd(finished, 1u) == nb - 1u;
+  if (tid == 0) sh.tile = done_last(list.done, b, nb);
   __syncthreads();
   if (sh.tile) {
     for (uint32_t i = tid; i < nb; i += kWideBlock) st.desc[i] = 0ull;
-    if (tid == 0) {
-      *st.ticket = 0;
-      *finished = 0;
-    }
+    if (tid < kDoneWords) list.done[tid] = 0;
+    if (tid == 0) *st.ticket = 0;
     host_answer_count(answer, DENSE ? nullptr : out_count, status);
   }
 }
@@ -446,9 +443,9 @@ size_t wide_merge_bytes(int64_t r, int64_t dense_n, int cus) {
 }
 
 // The received entries as the scatter wants them: cursor: kCoarseCursorWords zeroed words (zero again when
-// k_wide_merge has run); rest: wide_merge_bytes(...) bytes.  False if the sizes do not suit the wide buckets.
+// k_wide_merge has run); done: kDoneWords of the same kind; rest: wide_merge_bytes(...) bytes.  False if the sizes do not suit the wide buckets.
 bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, int64_t dense_n, uint32_t *cursor,
-                     void *rest, int cus, int32_t *status, WideList *list, bool alone) {
+                     uint32_t *done, void *rest, int cus, int32_t *status, WideList *list, bool alone) {
   SlabGeom geo;
   if (!wide_merge_fits(r, dense_n, cus, &geo, alone)) return false;
   WideSlabs slabs;
@@ -465,6 +462,7 @@ bool wide_merge_list(const void *idx, int idx64_in, const void *val, int64_t r, 
   list->dense_n = (uint32_t)dense_n;
   list->idx64 = idx64_in;
   list->out = slabs;
+  list->done = done;
   list->status = status;
   return true;
 }
@@ -499,7 +497,7 @@ static void wide_merge_typed(const WideList &list, int dtype, void *out_idx, int
     wide_merge_launch<uint16_t, float>(list, out_idx, idx64_out, static_cast<float *>(out_val), capacity, out_count, scan, s, ask);
 }
 
-// The two launches.  scan: zeroed prefix state for 256 buckets (descriptors, ticket, finished count), zero again
+// The two launches.  scan: zeroed prefix state for 256 buckets (descriptors, ticket), zero again
 // when the second ends.  out_dtype: ZEN_F32 (the sums; the only choice for fp32 values) or ZEN_BF16 (rounded).
 // out_idx == nullptr: out_val is the dense tensor.
 int wide_merge(const WideList &list, int dtype, void *out_idx, int idx64_out, void *out_val, int out_dtype,
