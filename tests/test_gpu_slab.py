@@ -455,6 +455,35 @@ def test_merge_that_waits_gives_the_same_on_half_and_all_of_the_chip(zen, oracle
     assert np.array_equal(to_np(m_idx), w_idx[kept.numpy()]) and torch.equal(m_val.cpu(), rounded[kept])
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("piled", [1000, 1024, 1025, 2047, 2049, 3072, 3200])
+def test_merge_at_a_round_of_records(zen, oracle, piled, dtype):
+    """The first of 128 wide buckets gets all its records from every eighth batch of 4096 entries, which is one part of its
+    slab: up to one and two records a thread, more, and more than the workgroup takes."""
+    from zen_repro_amd import _lib
+
+    n, batches = 1 << 24, 336
+    rng = np.random.default_rng(piled)
+    ci = rng.integers(n // 128, n, batches * 4096)
+    at = rng.choice(batches // 8 * 4096, piled, replace=False)
+    ci[at // 4096 * 8 * 4096 + at % 4096] = rng.integers(0, n // 128, piled)
+    cv = (rng.standard_normal(len(ci)) * 1e-3).astype(np.float32)
+    if dtype == "bf16":
+        cv = oracle.f32_to_bf16_bits(cv)
+    want_i, want_v = oracle.merge_sparse(ci, cv, n)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    gi, gv, cnt, st = lba.merge_sparse_flat(to_dev(ci), to_dev(cv), n, mode=_lib.MODE_FAST)
+    if piled > 3072 and not FLAGS:
+        assert st.item() == _lib.STAT_RETRY
+    else:
+        assert st.item() == 0 and cnt.item() == len(want_i)
+        assert np.array_equal(to_np(gi)[:len(want_i)], want_i.astype(np.int32))
+        assert np.array_equal(to_np(gv)[:len(want_i)].view(np.uint32), want_v.view(np.uint32))
+    dense = lba.decode_sparse_tensors(to_dev(ci), to_dev(cv), n)
+    f32 = oracle.decode(ci, cv, n, "f32acc")
+    assert np.array_equal(to_np(dense), oracle.f32_to_bf16_bits(f32) if dtype == "bf16" else f32)
+
+
 def test_slab_merge_bad_indices_cancellation_and_pile_up(zen, oracle):
     from zen_repro_amd import _lib
 

@@ -15,10 +15,8 @@ namespace zen {
 namespace {
 
 constexpr int kWmRounds = 3;                               // a part of a bucket's slab is read in rounds of kWideBlock records
-constexpr int kWmItems = kWideSplit * kWmRounds;           // records per thread
 constexpr int kWmPartMax = kWideBlock * kWmRounds;         // records of one part, at most
 constexpr int kWmLanes = 4;                                // records a thread handles per step of the ranking loops
-constexpr int kWmSteps = kWmItems / kWmLanes;
 constexpr int kWmQueue = 6144;                             // records of large groups set aside while ranking
 constexpr int kWmGroupLimit = 2048;                        // records in one narrow range: bounds the rank loop
 constexpr int kWmSumItems = 17;                            // sorted records per thread while summing (odd: no LDS bank conflicts)
@@ -59,9 +57,252 @@ struct WideMergeShared {
   int tile;
 };
 
+// Puts the bucket's records in order of (index, arrival number): indices (minus the bucket's first) to sh.key, values to
+// sh.val.  Returns how many there are.  ROUNDS: of kWideBlock records of every part.  Up to two are written out, a thread's
+// (at most sixteen) records stay in registers from their load to the end, and all loads are in flight together; of three
+// the loops' bodies handle the first kWmLanes registers of a set and then rotate the set, and the values are loaded at the
+// end (written out for 24 records the code would not fit the instruction cache, and every workgroup runs it once).  A
+// chain of trips to LDS and memory: 62 M bf16, 3.1 M entries, 256 buckets of two rounds 42.6 us to index lists and 55.0
+// dense, with the loops for those too 48.2 and 59.0; 9 M, 0.9 M entries, one round 26.8 and 32.4.
+template <typename S, int ROUNDS, typename Zero>
+__device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &geo, const WideSlabs &in, uint32_t b,
+                                           const uint32_t (&pcount)[kWideSplit], uint32_t longest, bool declined,
+                                           int tie_bits, int32_t *status, Zero zero_some) {
+  constexpr int kItems = kWideSplit * ROUNDS, kSteps = kItems / kWmLanes;
+  constexpr bool kHeld = ROUNDS <= 2;
+  const uint32_t tid = threadIdx.x;
+  const uint2 *rec_plane = in.rec + (size_t)b * kWideSplit * in.part_cap;
+  const uint32_t *val_plane = in.val32 + (size_t)b * kWideSplit * in.part_cap;
+  const int shift = geo.sub_shift;
+  const uint32_t low_mask = (1u << shift) - 1u;
+
+  // item r * kWideSplit + q of a thread is the record at place tid + r * kWideBlock of part q; loads in no
+  // branch, so that all are in flight together
+  uint32_t w[kItems], ps[kItems];  // the record's word; then its place in `word` | narrow range << 14
+  uint32_t v[kHeld ? kItems : 1];
+  if (kHeld) {
+    uint2 rec[kItems];
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      const uint32_t e = tid + (uint32_t)(i / kWideSplit) * kWideBlock;
+      const size_t at = (size_t)(i % kWideSplit) * in.part_cap + (e < pcount[i % kWideSplit] ? e : 0u);
+      rec[i] = rec_plane[at];
+      v[kHeld ? i : 0] = sizeof(S) == 2 ? 0u : val_plane[at];
+    }
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      const bool live = tid + (uint32_t)(i / kWideSplit) * kWideBlock < pcount[i % kWideSplit];
+      const uint32_t off = wm_off(rec[i]), arr = wm_arr(rec[i]);
+      w[i] = live ? ((off & low_mask) << tie_bits) | arr : kInvalid;
+      ps[i] = live ? off >> shift : kInvalid;  // the narrow range, for now
+      if (sizeof(S) == 2) v[kHeld ? i : 0] = rec[i].y >> 16;
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+#pragma unroll
+      for (int q = 0; q < kWideSplit; ++q) w[r * kWideSplit + q] = ps[r * kWideSplit + q] = kInvalid;
+      if ((uint32_t)r * kWideBlock < longest) {
+#pragma unroll
+        for (int q = 0; q < kWideSplit; ++q) {
+          const uint32_t e = tid + (uint32_t)r * kWideBlock;
+          const bool live = e < pcount[q];
+          const uint2 rec = rec_plane[(size_t)q * in.part_cap + (live ? e : 0u)];
+          const uint32_t off = wm_off(rec), arr = wm_arr(rec);
+          if (live) {
+            w[r * kWideSplit + q] = ((off & low_mask) << tie_bits) | arr;
+            ps[r * kWideSplit + q] = off >> shift;
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kItems; ++i)
+    if (ps[i] != kInvalid) sh.cnt.count(ps[i]);
+  __syncthreads();
+  uint32_t n = sh.cnt.starts(sh.scan, (uint32_t)kWmGroupLimit, &sh.big);
+  __syncthreads();
+  if (n > (uint32_t)kWideCap || sh.big) {  // more than fits, or keys piled on a few values: another path answers
+    declined = true;
+    __syncthreads();
+    sh.cnt.clear();
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) w[i] = ps[i] = kInvalid;
+    n = 0;
+    longest = 0;
+    __syncthreads();
+  }
+  if (declined && tid == 0) atomicOr(status, ZEN_STAT_RETRY);
+  // this workgroup was the only reader of its part cursors: back to zero for the next call
+  if (tid < (uint32_t)kWideSplit) in.cursor[coarse_cursor_at(b, tid)] = 0;
+
+  auto rotate = [](uint32_t (&a)[kItems]) {
+    uint32_t head[kWmLanes];
+#pragma unroll
+    for (int k = 0; k < kWmLanes; ++k) head[k] = a[k];
+#pragma unroll
+    for (int i = 0; i + kWmLanes < kItems; ++i) a[i] = a[i + kWmLanes];
+#pragma unroll
+    for (int k = 0; k < kWmLanes; ++k) a[kItems - kWmLanes + k] = head[k];
+  };
+  const int steps = longest == 0 ? 0 : (int)((longest + kWideBlock - 1) / kWideBlock) * (kWideSplit / kWmLanes);
+  auto take_step = [&](int from) {
+#pragma unroll
+    for (int k = 0; k < kWmLanes; ++k) {
+      if (ps[from + k] != kInvalid) {
+        const uint32_t p = sh.cnt.take(ps[from + k]);
+        sh.word[p] = w[from + k];
+        ps[from + k] = p | (ps[from + k] << 14);
+      }
+    }
+  };
+  if (kHeld) {
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      if (s < steps) take_step(s * kWmLanes);
+      zero_some();
+    }
+  } else {
+#pragma unroll 1
+    for (int s = 0; s < kSteps; ++s) {
+      if (s < steps) take_step(0);
+      rotate(w);
+      rotate(ps);
+      zero_some();
+    }
+  }
+  __syncthreads();
+  // rank = records of the bucket with a smaller (index, arrival number): those of the narrow ranges before,
+  // plus those of the record's own range with a smaller word.  The range's first four words are fetched in one
+  // go, which settles ranges up to that size; where many records share an index (payloads that overlap) a few
+  // lanes of every wave would walk through dozens of words while the others wait: records of larger ranges
+  // are set aside and handed out again afterwards, one per thread.
+  uint32_t rk[kItems];
+#pragma unroll
+  for (int i = 0; i < kItems; ++i) rk[i] = kInvalid;
+  auto rank_step = [&](int from, uint32_t (&out)[kWmLanes]) {
+    constexpr int kAhead = 4;
+    uint32_t g0[kWmLanes], g1[kWmLanes], a[kWmLanes][kAhead];
+#pragma unroll
+    for (int k = 0; k < kWmLanes; ++k) {
+      const uint32_t sub = ps[from + k] != kInvalid ? ps[from + k] >> 14 : 0u;
+      g0[k] = sh.cnt.start_of(sub);
+      g1[k] = sh.cnt.end_of(sub);
+    }
+#pragma unroll
+    for (int k = 0; k < kWmLanes; ++k) {
+      const uint32_t last = g1[k] > g0[k] ? g1[k] - 1u : g0[k];
+#pragma unroll
+      for (int e = 0; e < kAhead; ++e) a[k][e] = sh.word[g0[k] + e < last ? g0[k] + e : last];
+    }
+#pragma unroll
+    for (int k = 0; k < kWmLanes; ++k) {
+      if (ps[from + k] != kInvalid) {
+        uint32_t less = 0;
+#pragma unroll
+        for (int e = 0; e < kAhead; ++e) less += g0[k] + e < g1[k] && a[k][e] < w[from + k];
+        uint32_t x = g0[k] + less;
+        if (g1[k] - g0[k] > (uint32_t)kAhead) {
+          const uint32_t at = atomicAdd(&sh.qn, 1u);
+          if (at < (uint32_t)kWmQueue) {
+            sh.queue[at] = ps[from + k];
+            x = 0x80000000u | at;  // pending: place in the queue
+          } else {  // no room to set it aside: walked through here
+            for (uint32_t u = g0[k] + kAhead; u < g1[k]; ++u) x += sh.word[u] < w[from + k];
+          }
+        }
+        out[k] = x;
+      }
+    }
+  };
+  if (kHeld) {
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      uint32_t out[kWmLanes];
+#pragma unroll
+      for (int k = 0; k < kWmLanes; ++k) out[k] = kInvalid;
+      if (s < steps) rank_step(s * kWmLanes, out);
+#pragma unroll
+      for (int k = 0; k < kWmLanes; ++k) rk[s * kWmLanes + k] = out[k];
+      zero_some();
+    }
+  } else {
+#pragma unroll 1
+    for (int s = 0; s < kSteps; ++s) {
+      uint32_t out[kWmLanes];
+#pragma unroll
+      for (int k = 0; k < kWmLanes; ++k) out[k] = kInvalid;
+      if (s < steps) rank_step(0, out);
+      rotate(w);
+      rotate(ps);
+      rotate(rk);  // the step's ranks enter at the end: after the last step rank i belongs to record i
+#pragma unroll
+      for (int k = 0; k < kWmLanes; ++k) rk[kItems - kWmLanes + k] = out[k];
+      zero_some();
+    }
+  }
+  __syncthreads();
+  {
+    uint32_t pending = sh.qn;
+    if (pending > (uint32_t)kWmQueue) pending = kWmQueue;
+    for (uint32_t e = tid; e < pending; e += kWideBlock) {
+      const uint32_t p = sh.queue[e] & 0x3fffu, sub = sh.queue[e] >> 14;
+      const uint32_t g0 = sh.cnt.start_of(sub), g1 = sh.cnt.end_of(sub);
+      const uint32_t my = sh.word[p];
+      uint32_t less = 0;
+      for (uint32_t u = g0; u < g1; u += 4) {
+        const uint32_t last = g1 - 1u;
+        const uint32_t a0 = sh.word[u], a1 = sh.word[u + 1 < last ? u + 1 : last];
+        const uint32_t a2 = sh.word[u + 2 < last ? u + 2 : last], a3 = sh.word[u + 3 < last ? u + 3 : last];
+        less += (a0 < my) + (u + 1 < g1 && a1 < my) + (u + 2 < g1 && a2 < my) + (u + 3 < g1 && a3 < my);
+      }
+      sh.queue[e] = g0 + less;  // the entry's thread is its only reader
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kItems; ++i)
+      if (rk[i] != kInvalid && (rk[i] & 0x80000000u)) rk[i] = sh.queue[rk[i] & 0x7fffffffu];
+  }
+  __syncthreads();  // everybody is through with the words and the counters: the sorted records take their place
+  if (kHeld) {
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      if (rk[i] != kInvalid) {
+        sh.key[rk[i]] = ((ps[i] >> 14) << shift) | (w[i] >> tie_bits);
+        sh.val[rk[i]] = KeyOf<S>::to_f32((S)v[kHeld ? i : 0]);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+      if ((uint32_t)r * kWideBlock < longest) {
+        uint32_t u[kWideSplit];
+#pragma unroll
+        for (int q = 0; q < kWideSplit; ++q) {
+          const bool live = rk[r * kWideSplit + q] != kInvalid;
+          const uint32_t e = tid + (uint32_t)r * kWideBlock;
+          const size_t at = (size_t)q * in.part_cap + (live ? e : 0u);
+          u[q] = sizeof(S) == 2 ? rec_plane[at].y >> 16 : val_plane[at];
+        }
+#pragma unroll
+        for (int q = 0; q < kWideSplit; ++q) {
+          const int i = r * kWideSplit + q;
+          if (rk[i] != kInvalid) {
+            sh.key[rk[i]] = ((ps[i] >> 14) << shift) | (w[i] >> tie_bits);
+            sh.val[rk[i]] = KeyOf<S>::to_f32((S)u[q]);
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();
+  return n;
+}
+
 // O: what is written for a sum (zen_common.h).  DENSE: out_val is the dense tensor [0, dense_n); the workgroup
 // writes its bucket's range of it whole, zeros between the steps of the ranking loops, the sums behind them at the
-// end (62 M bf16 elements, 3.1 M entries: 60 us; 69 with the zeros in front of the records' loads, which then wait for
+// end (62 M bf16 elements, 3.1 M entries: 55 us; nine more with the zeros in front of the records' loads, which then wait for
 // them to be written; the fill and scatter kernels in front of and behind a sparse merge took 18 + 21 us.  Workgroups
 // of k_wide_scatter that do nothing else cost that kernel the 17 us they save this one).
 template <typename I, typename S, typename O, bool DENSE>
@@ -98,7 +339,6 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
     if (head > end - lo) head = end - lo;
     zero_vecs = (end - lo - head) / V;
     zero_to = reinterpret_cast<u32x4 *>(out_val + lo + head);
-    zero_each = (zero_vecs + kWideBlock * 2 * kWmSteps - 1) / (kWideBlock * 2 * kWmSteps);
     for (uint32_t i = tid; i < head; i += kWideBlock) out_val[lo + i] = O(0);
     for (uint32_t i = lo + head + zero_vecs * V + tid; i < end; i += kWideBlock) out_val[i] = O(0);
   }
@@ -115,6 +355,10 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
     if (pcount[q] > in.part_cap) pcount[q] = in.part_cap;  // the scatter flagged the overflow
     longest = pcount[q] > longest ? pcount[q] : longest;
   }
+  if (DENSE) {  // two pauses in every step
+    const uint32_t pauses = (longest <= (uint32_t)kWideBlock ? 1u : longest <= 2u * kWideBlock ? 2u : (uint32_t)kWmRounds) * (2u * kWideSplit / kWmLanes);
+    zero_each = (zero_vecs + kWideBlock * pauses - 1u) / (kWideBlock * pauses);
+  }
   bool declined = false;
   if (longest > (uint32_t)kWmPartMax) {
     declined = true;
@@ -122,182 +366,10 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
     for (int q = 0; q < kWideSplit; ++q) pcount[q] = 0;
     longest = 0;
   }
-  const uint2 *rec_plane = in.rec + (size_t)b * kWideSplit * in.part_cap;
-  const uint32_t *val_plane = in.val32 + (size_t)b * kWideSplit * in.part_cap;
-  const int shift = geo.sub_shift;
-  const uint32_t low_mask = (1u << shift) - 1u;
-
-  // item r * kWideSplit + q of a thread is the record at place tid + r * kWideBlock of part q; loads in no
-  // branch, so that all are in flight together
-  uint32_t w[kWmItems], ps[kWmItems];  // the record's word; then its place in `word` | narrow range << 14
-#pragma unroll
-  for (int r = 0; r < kWmRounds; ++r) {
-#pragma unroll
-    for (int q = 0; q < kWideSplit; ++q) w[r * kWideSplit + q] = ps[r * kWideSplit + q] = kInvalid;
-    if ((uint32_t)r * kWideBlock < longest) {
-#pragma unroll
-      for (int q = 0; q < kWideSplit; ++q) {
-        const uint32_t e = tid + (uint32_t)r * kWideBlock;
-        const bool live = e < pcount[q];
-        const uint2 rec = rec_plane[(size_t)q * in.part_cap + (live ? e : 0u)];
-        const uint32_t off = wm_off(rec), arr = wm_arr(rec);
-        if (live) {
-          w[r * kWideSplit + q] = ((off & low_mask) << tie_bits) | arr;
-          ps[r * kWideSplit + q] = off >> shift;  // the narrow range, for now
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < kWmItems; ++i)
-    if (ps[i] != kInvalid) sh.cnt.count(ps[i]);
-  __syncthreads();
-  uint32_t n = sh.cnt.starts(sh.scan, (uint32_t)kWmGroupLimit, &sh.big);
-  __syncthreads();
-  if (n > (uint32_t)kWideCap || sh.big) {  // more than fits, or keys piled on a few values: another path answers
-    declined = true;
-    __syncthreads();
-    sh.cnt.clear();
-#pragma unroll
-    for (int i = 0; i < kWmItems; ++i) w[i] = ps[i] = kInvalid;
-    n = 0;
-    longest = 0;
-    __syncthreads();
-  }
-  if (declined && tid == 0) atomicOr(status, ZEN_STAT_RETRY);
-  // this workgroup was the only reader of its part cursors: back to zero for the next call
-  if (tid < (uint32_t)kWideSplit) in.cursor[coarse_cursor_at(b, tid)] = 0;
-
-  // The thread's records are worked through in steps of kWmLanes, by loops whose body handles the first
-  // kWmLanes registers of a set and then rotates the set (the body written out for all records would not fit
-  // the instruction cache, and every workgroup runs it once).
-  auto rotate = [](uint32_t (&a)[kWmItems]) {
-    uint32_t head[kWmLanes];
-#pragma unroll
-    for (int k = 0; k < kWmLanes; ++k) head[k] = a[k];
-#pragma unroll
-    for (int i = 0; i + kWmLanes < kWmItems; ++i) a[i] = a[i + kWmLanes];
-#pragma unroll
-    for (int k = 0; k < kWmLanes; ++k) a[kWmItems - kWmLanes + k] = head[k];
-  };
-  const int steps = longest == 0 ? 0 : (int)((longest + kWideBlock - 1) / kWideBlock) * (kWideSplit / kWmLanes);
-#pragma unroll 1
-  for (int s = 0; s < kWmSteps; ++s) {
-    if (s < steps) {
-#pragma unroll
-      for (int k = 0; k < kWmLanes; ++k) {
-        if (ps[k] != kInvalid) {
-          const uint32_t p = sh.cnt.take(ps[k]);
-          sh.word[p] = w[k];
-          ps[k] = p | (ps[k] << 14);
-        }
-      }
-    }
-    rotate(w);
-    rotate(ps);
-    zero_some();
-  }
-  __syncthreads();
-  // rank = records of the bucket with a smaller (index, arrival number): those of the narrow ranges before,
-  // plus those of the record's own range with a smaller word.  The range's first four words are fetched in one
-  // go, which settles ranges up to that size; where many records share an index (payloads that overlap) a few
-  // lanes of every wave would walk through dozens of words while the others wait: records of larger ranges
-  // are set aside and handed out again afterwards, one per thread.
-  uint32_t rk[kWmItems];
-#pragma unroll
-  for (int i = 0; i < kWmItems; ++i) rk[i] = kInvalid;
-#pragma unroll 1
-  for (int s = 0; s < kWmSteps; ++s) {
-    constexpr int kAhead = 4;
-    uint32_t out[kWmLanes];
-#pragma unroll
-    for (int k = 0; k < kWmLanes; ++k) out[k] = kInvalid;
-    if (s < steps) {
-      uint32_t g0[kWmLanes], g1[kWmLanes], a[kWmLanes][kAhead];
-#pragma unroll
-      for (int k = 0; k < kWmLanes; ++k) {
-        const uint32_t sub = ps[k] != kInvalid ? ps[k] >> 14 : 0u;
-        g0[k] = sh.cnt.start_of(sub);
-        g1[k] = sh.cnt.end_of(sub);
-      }
-#pragma unroll
-      for (int k = 0; k < kWmLanes; ++k) {
-        const uint32_t last = g1[k] > g0[k] ? g1[k] - 1u : g0[k];
-#pragma unroll
-        for (int e = 0; e < kAhead; ++e) a[k][e] = sh.word[g0[k] + e < last ? g0[k] + e : last];
-      }
-#pragma unroll
-      for (int k = 0; k < kWmLanes; ++k) {
-        if (ps[k] != kInvalid) {
-          uint32_t less = 0;
-#pragma unroll
-          for (int e = 0; e < kAhead; ++e) less += g0[k] + e < g1[k] && a[k][e] < w[k];
-          uint32_t x = g0[k] + less;
-          if (g1[k] - g0[k] > (uint32_t)kAhead) {
-            const uint32_t at = atomicAdd(&sh.qn, 1u);
-            if (at < (uint32_t)kWmQueue) {
-              sh.queue[at] = ps[k];
-              x = 0x80000000u | at;  // pending: place in the queue
-            } else {  // no room to set it aside: walked through here
-              for (uint32_t u = g0[k] + kAhead; u < g1[k]; ++u) x += sh.word[u] < w[k];
-            }
-          }
-          out[k] = x;
-        }
-      }
-    }
-    rotate(w);
-    rotate(ps);
-    rotate(rk);  // the step's ranks enter at the end: after the last step rank i belongs to record i
-#pragma unroll
-    for (int k = 0; k < kWmLanes; ++k) rk[kWmItems - kWmLanes + k] = out[k];
-    zero_some();
-  }
-  __syncthreads();
-  {
-    uint32_t pending = sh.qn;
-    if (pending > (uint32_t)kWmQueue) pending = kWmQueue;
-    for (uint32_t e = tid; e < pending; e += kWideBlock) {
-      const uint32_t p = sh.queue[e] & 0x3fffu, sub = sh.queue[e] >> 14;
-      const uint32_t g0 = sh.cnt.start_of(sub), g1 = sh.cnt.end_of(sub);
-      const uint32_t my = sh.word[p];
-      uint32_t less = 0;
-      for (uint32_t u = g0; u < g1; u += 4) {
-        const uint32_t last = g1 - 1u;
-        const uint32_t a0 = sh.word[u], a1 = sh.word[u + 1 < last ? u + 1 : last];
-        const uint32_t a2 = sh.word[u + 2 < last ? u + 2 : last], a3 = sh.word[u + 3 < last ? u + 3 : last];
-        less += (a0 < my) + (u + 1 < g1 && a1 < my) + (u + 2 < g1 && a2 < my) + (u + 3 < g1 && a3 < my);
-      }
-      sh.queue[e] = g0 + less;  // the entry's thread is its only reader
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kWmItems; ++i)
-      if (rk[i] != kInvalid && (rk[i] & 0x80000000u)) rk[i] = sh.queue[rk[i] & 0x7fffffffu];
-  }
-  __syncthreads();  // everybody is through with the words and the counters: the sorted records take their place
-#pragma unroll
-  for (int r = 0; r < kWmRounds; ++r) {
-    if ((uint32_t)r * kWideBlock < longest) {
-      uint32_t v[kWideSplit];
-#pragma unroll
-      for (int q = 0; q < kWideSplit; ++q) {
-        const bool live = rk[r * kWideSplit + q] != kInvalid;
-        const uint32_t e = tid + (uint32_t)r * kWideBlock;
-        const size_t at = (size_t)q * in.part_cap + (live ? e : 0u);
-        v[q] = sizeof(S) == 2 ? rec_plane[at].y >> 16 : val_plane[at];
-      }
-#pragma unroll
-      for (int q = 0; q < kWideSplit; ++q) {
-        const int i = r * kWideSplit + q;
-        if (rk[i] != kInvalid) {
-          sh.key[rk[i]] = ((ps[i] >> 14) << shift) | (w[i] >> tie_bits);
-          sh.val[rk[i]] = KeyOf<S>::to_f32((S)v[q]);
-        }
-      }
-    }
-  }
-  __syncthreads();
+  const uint32_t n =
+      longest <= (uint32_t)kWideBlock ? wide_merge_sort<S, 1>(sh, geo, in, b, pcount, longest, declined, tie_bits, status, zero_some)
+      : longest <= 2u * kWideBlock ? wide_merge_sort<S, 2>(sh, geo, in, b, pcount, longest, declined, tie_bits, status, zero_some)
+                                   : wide_merge_sort<S, kWmRounds>(sh, geo, in, b, pcount, longest, declined, tie_bits, status, zero_some);
   // Thread t owns the sorted places [t * per, (t + 1) * per): as few per thread as cover the bucket (and an odd
   // number, which keeps the lanes of a wave on different LDS banks).  It fetches them all at once and walks
   // through them in registers.  A run of equal indices is summed in arrival order from +0 (like the dense
