@@ -262,7 +262,7 @@ __device__ unsigned long long g_wide_dbg[256 * 32];
 // three the loops' bodies handle the first kWideLanes registers of a set and then rotate the set, and the records are
 // loaded again (written out, the code would no longer fit the instruction cache, and every workgroup runs it just once).
 // A chain of LDS and memory trips bounds it, not a rate.  Written out, with the records held and the removed places noted
-// instead of searched for, the launch takes 31 us where the loops took 36 (62 M bf16 elements, 0.5 %, 128 workgroups) and
+// instead of searched for, the launch took 31 us where the loops took 36 (62 M bf16 elements, 0.5 %, 128 workgroups) and
 // 24 where they took 28 (1 M fp32, 1 %, 16 workgroups).
 template <typename S, int ROUNDS>
 __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, const WideTables &tb, const uint2 *records,
@@ -284,7 +284,7 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
     if ((uint32_t)r * kWideBlock < longest) {
 #pragma unroll
       for (int q = 0; q < kWideSplit; ++q) {
-        const uint32_t e = tid + (uint32_t)r * kWideBlock;
+        const uint32_t e = wide_place(q) + (uint32_t)r * kWideBlock;
         const size_t at = (size_t)q * tb.part_cap + (e < pcount[q] ? e : 0u);
         const uint2 rec = r == 0 ? first_round[q] : records[at];
         const uint32_t slot = geo.mod_m(poly(rec.x) + kSeed1);  // the level-1 slot: a dozen instructions, not a plane of its own
@@ -325,7 +325,8 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
   // raw place of the record in lane k of step s: part * 4096 + place inside the part
   auto raw_place = [&](int s, int k) {
     constexpr int kPer = kWideSplit / kWideLanes;  // steps per round
-    return (uint32_t)((s % kPer) * kWideLanes + k) * 4096u + tid + (uint32_t)(s / kPer) * kWideBlock;
+    const uint32_t q = (uint32_t)((s % kPer) * kWideLanes + k);
+    return q * 4096u + wide_place(q) + (uint32_t)(s / kPer) * kWideBlock;
   };
   // steps of rounds that no part of the slab reaches hold nothing: the loops stop short of them
   const int steps = longest == 0 ? 0 : (int)((longest + kWideBlock - 1) / kWideBlock) * (kWideSplit / kWideLanes);
@@ -362,6 +363,10 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
     constexpr int kAhead = 4;
 #pragma unroll
     for (int k = 0; k < kWideLanes; ++k) out[k] = kInvalid;
+    bool some = false;
+#pragma unroll
+    for (int k = 0; k < kWideLanes; ++k) some |= off[from + k] != kInvalid;
+    if (!__any(some)) return;
     uint32_t g0[kWideLanes], g1[kWideLanes], a[kWideLanes][kAhead];
 #pragma unroll
     for (int k = 0; k < kWideLanes; ++k) {
@@ -476,7 +481,7 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
       S v[kWideSplit];
 #pragma unroll
       for (int q = 0; q < kWideSplit; ++q) {
-        const uint32_t e = tid + (uint32_t)r * kWideBlock;
+        const uint32_t e = wide_place(q) + (uint32_t)r * kWideBlock;
         const size_t at = (size_t)q * tb.part_cap + (rk[r * kWideSplit + q] != kInvalid ? e : 0u);
         const uint2 rec = kHeld ? first_round[q] : records[at];
         t[q] = rec.x;
@@ -520,12 +525,12 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   const uint32_t tid = threadIdx.x;
   WIDE_MARK(0);
   // the bucket's records: (index, value bits), kWideSplit parts of part_cap records; item r * kWideSplit + q of a thread is
-  // the record at place tid + r * kWideBlock of part q.  The first round is asked for before it is known how many there
+  // the record at place wide_place(q) + r * kWideBlock of part q.  The first round is asked for before it is known how many there
   // are (a part has room for more than a round): a trip to memory less.
   const uint2 *records = reinterpret_cast<const uint2 *>(tb.words) + (size_t)b * kWideSplit * tb.part_cap;
   uint2 first_round[kWideSplit];
 #pragma unroll
-  for (int q = 0; q < kWideSplit; ++q) first_round[q] = records[(size_t)q * tb.part_cap + tid];
+  for (int q = 0; q < kWideSplit; ++q) first_round[q] = records[(size_t)q * tb.part_cap + wide_place(q)];
   // counters of the kernels before this one that nobody needs any more: back to zero, a slice per workgroup
   for (uint32_t i = b * kWideBlock + tid; i < clear_words; i += B * kWideBlock) clear[i] = 0;
   for (uint32_t i = b * kWideBlock + tid; i < clear_too_words; i += B * kWideBlock) clear_too[i] = 0;  // fp32: the refinement's histogram

@@ -76,7 +76,7 @@ __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &
   const int shift = geo.sub_shift;
   const uint32_t low_mask = (1u << shift) - 1u;
 
-  // item r * kWideSplit + q of a thread is the record at place tid + r * kWideBlock of part q; loads in no
+  // item r * kWideSplit + q of a thread is the record at place wide_place(q) + r * kWideBlock of part q; loads in no
   // branch, so that all are in flight together
   uint32_t w[kItems], ps[kItems];  // the record's word; then its place in `word` | narrow range << 14
   uint32_t v[kHeld ? kItems : 1];
@@ -84,14 +84,14 @@ __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &
     uint2 rec[kItems];
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
-      const uint32_t e = tid + (uint32_t)(i / kWideSplit) * kWideBlock;
+      const uint32_t e = wide_place(i % kWideSplit) + (uint32_t)(i / kWideSplit) * kWideBlock;
       const size_t at = (size_t)(i % kWideSplit) * in.part_cap + (e < pcount[i % kWideSplit] ? e : 0u);
       rec[i] = rec_plane[at];
       v[kHeld ? i : 0] = sizeof(S) == 2 ? 0u : val_plane[at];
     }
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
-      const bool live = tid + (uint32_t)(i / kWideSplit) * kWideBlock < pcount[i % kWideSplit];
+      const bool live = wide_place(i % kWideSplit) + (uint32_t)(i / kWideSplit) * kWideBlock < pcount[i % kWideSplit];
       const uint32_t off = wm_off(rec[i]), arr = wm_arr(rec[i]);
       w[i] = live ? ((off & low_mask) << tie_bits) | arr : kInvalid;
       ps[i] = live ? off >> shift : kInvalid;  // the narrow range, for now
@@ -105,7 +105,7 @@ __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &
       if ((uint32_t)r * kWideBlock < longest) {
 #pragma unroll
         for (int q = 0; q < kWideSplit; ++q) {
-          const uint32_t e = tid + (uint32_t)r * kWideBlock;
+          const uint32_t e = wide_place(q) + (uint32_t)r * kWideBlock;
           const bool live = e < pcount[q];
           const uint2 rec = rec_plane[(size_t)q * in.part_cap + (live ? e : 0u)];
           const uint32_t off = wm_off(rec), arr = wm_arr(rec);
@@ -183,6 +183,10 @@ __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &
   for (int i = 0; i < kItems; ++i) rk[i] = kInvalid;
   auto rank_step = [&](int from, uint32_t (&out)[kWmLanes]) {
     constexpr int kAhead = 4;
+    bool some = false;
+#pragma unroll
+    for (int k = 0; k < kWmLanes; ++k) some |= ps[from + k] != kInvalid;
+    if (!__any(some)) return;
     uint32_t g0[kWmLanes], g1[kWmLanes], a[kWmLanes][kAhead];
 #pragma unroll
     for (int k = 0; k < kWmLanes; ++k) {
@@ -281,7 +285,7 @@ __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &
 #pragma unroll
         for (int q = 0; q < kWideSplit; ++q) {
           const bool live = rk[r * kWideSplit + q] != kInvalid;
-          const uint32_t e = tid + (uint32_t)r * kWideBlock;
+          const uint32_t e = wide_place(q) + (uint32_t)r * kWideBlock;
           const size_t at = (size_t)q * in.part_cap + (live ? e : 0u);
           u[q] = sizeof(S) == 2 ? rec_plane[at].y >> 16 : val_plane[at];
         }
