@@ -137,6 +137,26 @@ def test_slab_load_balance_at_a_round_of_records(zen, oracle, P, per_part, dtype
     assert not tp._table(torch.device("cuda"), n).any()
 
 
+@pytest.mark.parametrize("rehash", [1, 2, 3])
+@pytest.mark.parametrize("P,k", [(4, 400), (4, 30000), (4, 45000), (4, 46300), (4, 48000), (1, 23000), (16, 92000), (3, 60000)])
+def test_slab_load_balance_of_few_losers(zen, oracle, P, k, rehash):
+    """Partitions with fewer and more entries that lose their first slot than their workgroups work out by themselves."""
+    if FLAGS:
+        pytest.skip("covered by the other run")
+    n = -(-(1 << 20) // P) * P
+    x = (np.random.default_rng(P * k).standard_normal(n) * 1e-3).astype(np.float32)
+    x[0] = 0
+    masked, kept = oracle.mask_dense(x, int(oracle.kth_key(x, k)))
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(masked, P, 1, rehash)
+    assert st_o == 0 and lb_path(zen, n, P, "f32", kept + 1024, k=k) == WIDE
+    tp = zen.TensorPartition(P, 1, rehash)
+    for _ in range(2):
+        oi, ov, splits, status = tp.load_balance_flat(to_dev(x), capacity=kept + 1024, k=k)
+        assert status.item() == 0 and np.array_equal(to_np(splits), splits_o)
+        assert np.array_equal(to_np(oi)[:kept], idx_o) and np.array_equal(to_np(ov)[:kept], val_o)
+    assert not tp._table(torch.device("cuda"), n).any()
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 def test_slab_load_balance_odd_length_unaligned_and_empty(zen, oracle, dtype):
     """A tensor whose length is no multiple of anything and whose first element is not 16-byte aligned (the

@@ -118,6 +118,12 @@ constexpr int kWideIndexLen = kWideSubs / kWideIndexStep;
 constexpr int kWidePad = 32;                            // words between two barrier counters
 constexpr int kWideCtrPad = 8;                          // words between two per-partition counters
 constexpr int kWideProbeLimit = 512;                    // probes in the map before it counts as full
+// Up to here every workgroup of a partition works out the chains of all the partition's losers by itself, in a map of its
+// own in LDS: who holds a slot in the end does not depend on the order, so they all find the same.  That takes a barrier
+// of the partition's workgroups and the trips to the map in memory out of the launch (62 M bf16 elements, 0.5 %, 48 losers
+// a partition: 29.6 and 26.3 us; 1 M fp32, 1 %, 14: 22.3 and 19.9).  The map has room for four times as many claims (the
+// claims of one loser's chain go down with the table's density), the list of owners pushed out for as many.
+constexpr int kWideOwnChains = 256, kWideOwnLog2 = 10, kWideOwnPushed = 256;
 constexpr uint32_t kInvalid = 0xffffffffu;
 // a record's raw place: part * 4096 + place inside the part
 static_assert(kWidePartMax <= 4096 && kWideSplit * 4096 <= (1 << 15), "raw places in 15 bits");
@@ -162,8 +168,13 @@ struct WideShared {
     struct {
       uint32_t mk[kWideMove];     // slots of the moved-in entries
       uint32_t mi[kWideMove];     // their indices
-      uint32_t mp[kWideMove];     // sorted place in front of which each slips in, by ascending slot
-      uint32_t rm[kWideRemoved];  // losers' indices while they are logged, then the sorted places of the removed entries
+      union {
+        struct {
+          uint32_t mp[kWideMove];     // sorted place in front of which each slips in, by ascending slot
+          uint32_t rm[kWideRemoved];  // losers' indices while they are logged, then the sorted places of the removed entries
+        };
+        unsigned long long own[1 << kWideOwnLog2];  // in between: the map of slots taken at level 2 or 3 (few losers)
+      };
     };
     struct {                      // while ranking: the records set aside
       uint32_t q_word[kWideQueue];   // the record's word, then its rank (| kRemovedBit)
@@ -171,10 +182,13 @@ struct WideShared {
     };
   };
   uint32_t gone[kWideRemoved];  // sorted places of the entries that lost their slot, as they come up
-  int32_t delta[kWideCap / 64];
+  union {
+    int32_t delta[kWideCap / 64];
+    uint32_t pushed[kWideOwnPushed];  // before: the level-1 owners pushed out (few losers)
+  };
   uint32_t scan[kWideBlock / 64 + 1];
   uint64_t scan64[kWideBlock / 64 + 1];
-  uint32_t lo, lost_n, nrm, mv_n, ser_n, base, flag, big;
+  uint32_t lo, lost_n, nrm, mv_n, ser_n, pushed_n, base, flag, big;
 };
 
 __device__ inline unsigned long long cell_fresh(const unsigned long long *p) {
@@ -184,6 +198,7 @@ __device__ inline unsigned long long cell_fresh(const unsigned long long *p) {
 // map_min (zen_hashmap.h) with one trip to memory where the slot is met for the first time: the cell is
 // claimed with a compare-and-swap straight away, and the count of claims is raised without waiting for it (a
 // map that fills up shows in the length of the probe sequences instead).
+// (ctr: null for a map that nobody counts the claims of)
 __device__ inline uint32_t map_min_claim(unsigned long long *cells, uint32_t log2, uint32_t slot, uint32_t t,
                                          Counters *ctr, bool *full) {
   const uint32_t mask = (1u << log2) - 1u;
@@ -192,7 +207,7 @@ __device__ inline uint32_t map_min_claim(unsigned long long *cells, uint32_t log
   for (uint32_t probes = 0; probes <= mask && probes < (uint32_t)kWideProbeLimit; ++probes, h = (h + 1u) & mask) {
     const unsigned long long cur = atomicCAS(&cells[h], 0ull, mine);
     if (cur == 0ull) {
-      atomicAdd(&ctr->claims, 1u);
+      if (ctr) atomicAdd(&ctr->claims, 1u);
       return kNone;
     }
     if ((uint32_t)(cur >> 32) == slot + 1u) return (uint32_t)atomicMin(&cells[h], mine);
@@ -536,7 +551,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   for (uint32_t i = b * kWideBlock + tid; i < clear_too_words; i += B * kWideBlock) clear_too[i] = 0;  // fp32: the refinement's histogram
   if (tid == 0) {
     sh.lo = geo.first_key(b);
-    sh.lost_n = sh.nrm = sh.mv_n = sh.ser_n = sh.big = 0;
+    sh.lost_n = sh.nrm = sh.mv_n = sh.ser_n = sh.pushed_n = sh.big = 0;
   }
   sh.cnt.clear();
   uint32_t pcount[kWideSplit];
@@ -582,15 +597,18 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   group_barrier(gbar, bpp, 1, status);
   WIDE_MARK(6);
 
-  // ---- levels 2 and 3 for the partition's losers: loser i is the business of workgroup i % bpp, thread
-  // i / bpp (more than bpp * 1024 of them: in rounds)
+  // ---- levels 2 and 3 for the partition's losers
   unsigned long long *pcells = cells + ((size_t)part << tb.map_log2);
   Counters *pctr = &tb.ctr[part];
   const uint32_t local = b - part * bpp;
+  const bool last_of_part = local == bpp - 1;
   uint32_t losers = load_agent(&tb.log_n[part * kWideCtrPad]);
   if (losers > tb.log_cap) losers = tb.log_cap;
-  for (uint32_t i = tid * bpp + local; i < losers; i += bpp * kWideBlock) {
-    uint32_t cur = load_agent(&tb.log_t[(size_t)part * tb.log_cap + i]);
+  const bool own = losers <= (uint32_t)kWideOwnChains;
+  uint32_t pushed = 0;
+  // cur loses level 1: claim(slot, t): t's entry in the map (map_min_claim); push(t, bucket, place): t, the level-1 owner at
+  // that place, is pushed out
+  auto chain = [&](uint32_t cur, auto claim, auto push) {
     int lv = 1;
     bool full = false;
     for (uint32_t steps = 0; lv < g.levels; ++steps) {
@@ -606,7 +624,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
         ++lv;
         continue;
       }
-      const uint32_t old = map_min_claim(pcells, tb.map_log2, slot, cur, pctr, &full);
+      const uint32_t old = claim(slot, cur, &full);
       if (full) {
         atomicOr(status, ZEN_STAT_RETRY);
         break;
@@ -618,13 +636,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
       if (old == kNone) {
         // first level-2/3 prober of this slot: its level-1 owner (a larger index, if any) is pushed out
         if (head == kNone) break;
-        const uint32_t at = atomicAdd(&tb.dlog_n[part * kWideCtrPad], 1u);
-        if (at < tb.log_cap) {
-          store_agent(&tb.dlog_t[(size_t)part * tb.log_cap + at], head);
-          store_agent(&tb.dlog_at[(size_t)part * tb.log_cap + at], (head_bucket << 16) | head_place);
-        } else {
-          atomicOr(status, ZEN_STAT_RETRY);
-        }
+        push(head, head_bucket, head_place);
         cur = head;
         lv = 1;
         continue;
@@ -636,38 +648,10 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
       cur = old;
       lv = lw + 1;
     }
-  }
-  WIDE_MARK(7);
-  group_barrier(gbar, bpp, 2, status);
-  WIDE_MARK(8);
-
-  // ---- every workgroup of the partition looks at every logged entry: where it finally sits (the level-2/3
-  // slot it holds in the map, or nowhere), and keeps what concerns its bucket: entries whose final slot lies
-  // in it move in, its own owners that were pushed out drop out; the partition's last bucket also gathers the
-  // entries that found no slot
-  const bool last_of_part = local == bpp - 1;
-  uint32_t pushed = load_agent(&tb.dlog_n[part * kWideCtrPad]);
-  if (pushed > tb.log_cap) pushed = tb.log_cap;
-  for (uint32_t i = tid; i < losers + pushed; i += kWideBlock) {
-    const bool first = i < losers;
-    const size_t at_log = (size_t)part * tb.log_cap + (first ? i : i - losers);
-    const uint32_t t = load_agent(first ? &tb.log_t[at_log] : &tb.dlog_t[at_log]);
-    const uint32_t from = first ? 0u : load_agent(&tb.dlog_at[at_log]);
-    if (!first && (from >> 16) == b && (from & 0xffffu) < n) {  // pushed out, once
-      sh.idx[from & 0xffffu] |= kRemovedBit;
-      const uint32_t at = atomicAdd(&sh.nrm, 1u);
-      if (at < (uint32_t)kWideRemoved) sh.gone[at] = from & 0xffffu;
-    }
-    uint32_t prt = 0, cell = kNone, slot = kNone;
-    for (int lv = 1; lv < g.levels && slot == kNone; ++lv) {
-      const uint32_t s = probe_slot(g, t, lv, &prt);
-      uint32_t at = 0;
-      if (map_find_fresh(pcells, tb.map_log2, s, &at) == t) {
-        slot = s;
-        cell = at;
-      }
-    }
-    if (i % bpp == local) store_agent(first ? &tb.log_cell[at_log] : &tb.dlog_cell[at_log], cell);
+  };
+  // entry t ends in `slot` (kNone: in none): it moves in if the slot is one of the bucket's, and the partition's last
+  // bucket also gathers the entries that found no slot
+  auto settle = [&](uint32_t t, uint32_t slot) {
     if (slot != kNone) {
       if (geo.bucket_of(slot) == b) {
         const uint32_t at = atomicAdd(&sh.mv_n, 1u);
@@ -679,6 +663,83 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
     } else if (last_of_part) {
       const uint32_t at = atomicAdd(&sh.ser_n, 1u);
       if (at < (uint32_t)kSlabSerialCap) store_agent(&tb.ser_idx[(size_t)part * kSlabSerialCap + at], t);
+    }
+  };
+  auto removed = [&](uint32_t bucket, uint32_t place) {  // an owner pushed out (once) is one of the bucket's
+    if (bucket == b && place < n) {
+      sh.idx[place] |= kRemovedBit;
+      const uint32_t at = atomicAdd(&sh.nrm, 1u);
+      if (at < (uint32_t)kWideRemoved) sh.gone[at] = place;
+    }
+  };
+  if (own) {
+    for (uint32_t i = tid; i < (1u << kWideOwnLog2); i += kWideBlock) sh.own[i] = 0ull;
+    const uint32_t loser = tid < losers ? load_agent(&tb.log_t[(size_t)part * tb.log_cap + tid]) : 0u;
+    __syncthreads();
+    if (tid < losers)
+      chain(
+          loser,
+          [&](uint32_t slot, uint32_t t, bool *full) { return map_min_claim(sh.own, kWideOwnLog2, slot, t, nullptr, full); },
+          [&](uint32_t t, uint32_t bucket, uint32_t place) {
+            removed(bucket, place);
+            const uint32_t at = atomicAdd(&sh.pushed_n, 1u);
+            if (at < (uint32_t)kWideOwnPushed)
+              sh.pushed[at] = t;
+            else
+              atomicOr(status, ZEN_STAT_RETRY);
+          });
+    WIDE_MARK(7);
+    __syncthreads();
+    WIDE_MARK(8);
+    const uint32_t more = sh.pushed_n < (uint32_t)kWideOwnPushed ? sh.pushed_n : (uint32_t)kWideOwnPushed;
+    if (tid < losers + more) {
+      const uint32_t t = tid < losers ? loser : sh.pushed[tid - losers];
+      uint32_t prt = 0, cell = 0, slot = kNone;
+      for (int lv = 1; lv < g.levels && slot == kNone; ++lv) {
+        const uint32_t at = probe_slot(g, t, lv, &prt);
+        if (map_find_fresh(sh.own, kWideOwnLog2, at, &cell) == t) slot = at;
+      }
+      settle(t, slot);
+    }
+  } else {
+    // loser i is the business of workgroup i % bpp, thread i / bpp (more than bpp * 1024 of them: in rounds)
+    for (uint32_t i = tid * bpp + local; i < losers; i += bpp * kWideBlock)
+      chain(
+          load_agent(&tb.log_t[(size_t)part * tb.log_cap + i]),
+          [&](uint32_t slot, uint32_t t, bool *full) { return map_min_claim(pcells, tb.map_log2, slot, t, pctr, full); },
+          [&](uint32_t t, uint32_t bucket, uint32_t place) {
+            const uint32_t at = atomicAdd(&tb.dlog_n[part * kWideCtrPad], 1u);
+            if (at < tb.log_cap) {
+              store_agent(&tb.dlog_t[(size_t)part * tb.log_cap + at], t);
+              store_agent(&tb.dlog_at[(size_t)part * tb.log_cap + at], (bucket << 16) | place);
+            } else {
+              atomicOr(status, ZEN_STAT_RETRY);
+            }
+          });
+    WIDE_MARK(7);
+    group_barrier(gbar, bpp, 2, status);
+    WIDE_MARK(8);
+    // every workgroup of the partition looks at every logged entry: where it finally sits (the level-2/3 slot it holds in
+    // the map, or nowhere), and keeps what concerns its bucket
+    pushed = load_agent(&tb.dlog_n[part * kWideCtrPad]);
+    if (pushed > tb.log_cap) pushed = tb.log_cap;
+    for (uint32_t i = tid; i < losers + pushed; i += kWideBlock) {
+      const bool first = i < losers;
+      const size_t at_log = (size_t)part * tb.log_cap + (first ? i : i - losers);
+      const uint32_t t = load_agent(first ? &tb.log_t[at_log] : &tb.dlog_t[at_log]);
+      const uint32_t from = first ? 0u : load_agent(&tb.dlog_at[at_log]);
+      if (!first) removed(from >> 16, from & 0xffffu);
+      uint32_t prt = 0, cell = kNone, slot = kNone;
+      for (int lv = 1; lv < g.levels && slot == kNone; ++lv) {
+        const uint32_t s = probe_slot(g, t, lv, &prt);
+        uint32_t at = 0;
+        if (map_find_fresh(pcells, tb.map_log2, s, &at) == t) {
+          slot = s;
+          cell = at;
+        }
+      }
+      if (i % bpp == local) store_agent(first ? &tb.log_cell[at_log] : &tb.dlog_cell[at_log], cell);
+      settle(t, slot);
     }
   }
   __syncthreads();
@@ -836,7 +897,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   WIDE_MARK(13);
   if (sh.flag & 1u) {
     // every occupied cell ends with the index that finally holds its slot, and that index's cell was recorded
-    for (uint32_t i = tid; i < losers + pushed; i += kWideBlock) {
+    for (uint32_t i = own ? losers : tid; i < losers + pushed; i += kWideBlock) {
       const size_t at = (size_t)part * tb.log_cap + (i < losers ? i : i - losers);
       const uint32_t cell = load_agent(i < losers ? &tb.log_cell[at] : &tb.dlog_cell[at]);
       if (cell != kNone) pcells[cell] = 0ull;
