@@ -532,13 +532,14 @@ namespace {
 // Whether a call takes the wide buckets where both they and the bucket slabs fit.  The resident kernel of the wide
 // buckets is one launch where the slabs need four, but every workgroup of a partition looks at all of the partition's
 // collisions; the slabs' chains share them out over the chip.  A call that waits for its sizes has the host idle: the
-// slabs are the quicker throughout (us a call with a given threshold, wide and slabs: 4.3 M bf16 elements on 2
-// partitions, 0.5 % selected 71 and 63, 10 % 173 and 90; 36 M, 0.5 % 86 and 81, 3 % 157 and 96, 10 % 714 and 166; on 16
-// partitions 92 and 87, 134 and 109, 433 and 166; fp32 the same).  Calls that do not wait follow each other as fast as
-// the host enqueues them, and the wide buckets are the quicker while collisions are few, up to about 8192 of them or one
-// slot in 64 taken (three steps of 16 M bf16 elements on 16 partitions with their merges, top 0.5 % 245 and 265, 2 % 252
-// and 270, 5 % 317 and 279; of 36 M, 2 % 274 and 278, 3 % 342 and 288, 5 % 525 and 368; one of 743 M, 0.5 % 414 and 496;
-// three of 20 M with 0.5 % in whole rows, no threshold, 192 and 215).
+// slabs, which know the sizes before the entries are in place, are the quicker (compress and load balance of the top 1 %,
+// us, wide and slabs: 4.3 M bf16 elements on 2 partitions 131 and 128; 8 M fp32 on 16 166 and 162; 36 M bf16 on 2 193 and
+// 181; the hook on 130 M fp32 elements, 4 ranks, 596 and 570; densely the more, a load balance of 36 M with 10 % 714 and
+// 166).  Calls that do not wait follow each other as fast as the host enqueues them, and the wide buckets are the quicker
+// while collisions are few, up to about 8192 of them or one slot in 64 taken (three steps of 16 M bf16 elements on 16
+// partitions with their merges, top 0.5 % 228 and 259, 2 % 259 and 273, 3.5 % 297 and 300, 5 % 350 and 325; of 36 M, 2 %
+// 306 and 311, 3 % 383 and 343, 5 % 554 and 417; one of 743 M, 0.5 %, 392 and 493; three of 20 M with 0.5 % in whole rows,
+// no threshold, 192 and 215).
 bool takes_wide(int64_t n, int64_t m, int partitions, int dtype, int64_t capacity, int64_t k, bool waits) {
   using namespace zen;
   if (!wide_balance_fits(m, partitions, capacity, k, wide_device_cus(), nullptr)) return false;
