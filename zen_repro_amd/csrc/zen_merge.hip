@@ -174,8 +174,9 @@ struct MergeSrc {
   using Last = S;
   static constexpr int kStaged = 2;
   __device__ inline uint32_t late(const uint32_t (&w)[3], int) const { return (uint32_t)val[w[1]]; }
-  __device__ inline bool load(uint32_t e, uint32_t (&w)[3], uint32_t *bucket) const {
-    const I k = idx[e];
+  using Raw = I;
+  __device__ inline I fetch(uint32_t e) const { return idx[e]; }
+  __device__ inline bool load(I k, uint32_t e, uint32_t (&w)[3], uint32_t *bucket) const {
     if (k < 0 || (uint64_t)k >= (uint64_t)dense_n) {
       atomicOr(status, ZEN_STAT_BAD_INDEX);  // skipped, like everything behind the good ones in the general path
       return false;

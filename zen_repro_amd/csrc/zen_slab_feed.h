@@ -18,7 +18,8 @@
 //
 // An entry travels as W 32-bit words, the last of which is kept in memory as the narrower type Src::Last (a
 // bf16 value takes two bytes on its way, not four).  What they are comes from two small functor types:
-//   Src:   bool load(uint32_t e, uint32_t (&w)[W], uint32_t *bucket)   words and bucket of list entry e;
+//   Src:   Raw fetch(uint32_t e)                                       what has to be read for list entry e
+//          bool load(Raw, uint32_t e, uint32_t (&w)[W], uint32_t *bucket)   its words and bucket;
 //                                                                      false: the entry is dropped
 //          kStaged, uint32_t late(const uint32_t (&w)[W], int q)       only the first kStaged words go through
 //                                                                      LDS in the first step; word q >= kStaged
@@ -131,12 +132,18 @@ __global__ __launch_bounds__(kSlabBlock) void k_coarse_scatter(SlabGeom geo, Coa
   if (batch >= count) return;
   const uint32_t part = blockIdx.x % kCoarseSplit;
   uint32_t w[kFeedItems][W], dst[kFeedItems], rank[kFeedItems];
+  typename Src::Raw raw[kFeedItems];
+#pragma unroll
+  for (int i = 0; i < kFeedItems; ++i) {  // in no branch (places past the end read the batch's first entry): all in flight together
+    const uint32_t e = batch + threadIdx.x + i * kSlabBlock;
+    raw[i] = src.fetch(e < count ? e : batch);
+  }
 #pragma unroll
   for (int i = 0; i < kFeedItems; ++i) {
     const uint32_t e = batch + threadIdx.x + i * kSlabBlock;
     dst[i] = 0xffu;
     uint32_t bucket = 0;
-    if (e < count && src.load(e, w[i], &bucket)) {
+    if (e < count && src.load(raw[i], e, w[i], &bucket)) {
       uint32_t rem;
       dst[i] = SlabGeom::div_small(bucket, cg.per, cg.inv_per, &rem);
     }
@@ -206,13 +213,11 @@ __global__ __launch_bounds__(kSlabBlock) void k_fine_scatter(SlabGeom geo, Coars
 #pragma unroll
   for (int i = 0; i < kFeedItems; ++i) {
     const uint32_t e = batch + threadIdx.x + i * kSlabBlock;
-    dst[i] = 0xffu;
-    if (e < count) {
+    const uint32_t at = e < count ? e : 0u;  // no branch around the loads: all in flight together
 #pragma unroll
-      for (int q = 0; q < W - 1; ++q) w[i][q] = from[q * plane + e];
-      w[i][W - 1] = (uint32_t)from_last[e];
-      dst[i] = 0;
-    }
+    for (int q = 0; q < W - 1; ++q) w[i][q] = from[q * plane + at];
+    w[i][W - 1] = (uint32_t)from_last[at];
+    dst[i] = e < count ? 0u : 0xffu;
   }
 #pragma unroll
   for (int i = 0; i < kFeedItems; ++i)
