@@ -1124,7 +1124,7 @@ int slab_load_balance(const SlabBalanceArgs &a, hipStream_t s) {
   if ((rc = select_stage_slabs(sc, s)) != ZEN_OK) return rc;
   if (refine) {
     const uint32_t refine_parts = p.cg.groups * (uint32_t)kCoarseSplit;
-    k_refine_threshold<<<dim3(refine_parts < 128u ? refine_parts : 128u), dim3(kRefineBlock), 0, s>>>(
+    k_refine_threshold<<<dim3(refine_grid(refine_parts)), dim3(kRefineBlock), 0, s>>>(
         p.cg, 1, p.feed.coarse_cursor, p.feed.coarse_words, static_cast<const uint32_t *>(a.input), p.thr,
         p.thr + 4, (uint32_t)a.k, p.refine_hist, a.thr_out, a.status);
     ZEN_LAUNCH_CHECK("k_refine_threshold");

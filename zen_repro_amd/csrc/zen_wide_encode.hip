@@ -1068,7 +1068,7 @@ int wide_load_balance(const SlabBalanceArgs &a, size_t state_offset, hipStream_t
   uint32_t clear_words = (uint32_t)(reinterpret_cast<char *>(p.tb.cursor) - reinterpret_cast<char *>(p.cand_hist)) / 4u;
   if (refine) {
     const uint32_t refine_parts = p.cg.groups * (uint32_t)kCoarseSplit;
-    k_refine_threshold<<<dim3(refine_parts < 128u ? refine_parts : 128u), dim3(kRefineBlock), 0, s>>>(
+    k_refine_threshold<<<dim3(refine_grid(refine_parts)), dim3(kRefineBlock), 0, s>>>(
         p.cg, -1, p.tb.cursor, p.tb.words, static_cast<const uint32_t *>(a.input), p.thr, p.thr + 4, (uint32_t)a.k,
         p.refine_hist, a.thr_out, a.status);
     ZEN_LAUNCH_CHECK("k_refine_threshold");
