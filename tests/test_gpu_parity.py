@@ -770,6 +770,22 @@ def test_decode_ascending_lists_without_a_sort(zen, oracle, n, nlists, per_list,
     assert np.array_equal(to_np(dense).view(want.dtype), want)
 
 
+@pytest.mark.parametrize("n", [256 * 8192, 256 * 8192 + 1, 4096 * 8192, 4096 * 8192 + 1])
+def test_decode_ascending_tells_the_host(zen, oracle, n):
+    """The sizes at which another kernel tells the host (tiles that search for themselves, tiles that count, a kernel
+    behind them): right lists bit for bit, a descent seen, and the call after it right again."""
+    rng = np.random.default_rng(n)
+    idx, val = ascending_lists(oracle, rng, n, 4, 20000, 0.1, "bf16", np.int64)
+    want = oracle.f32_to_bf16_bits(oracle.decode(np.concatenate(idx), np.concatenate(val), n, "f32acc"))
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    d_idx, d_val = [to_dev(i) for i in idx], [to_dev(v) for v in val]
+    swapped = [i.copy() for i in idx]
+    swapped[3][[-2, -1]] = swapped[3][[-1, -2]]
+    for _ in range(2):
+        assert np.array_equal(to_np(lba._decode_ascending(d_idx, d_val, n)).view(want.dtype), want)
+        assert lba._decode_ascending([to_dev(i) for i in swapped], d_val, n) is None
+
+
 def test_decode_ascending_declines_what_is_not_ascending(zen, oracle):
     """A list with a descent, a repeated index inside one list or an index outside the dense tensor raise
     ZEN_STAT_RETRY; decode_sparse_tensors then answers through the general entry point (or raises, for the
