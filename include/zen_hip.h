@@ -53,8 +53,9 @@ extern "C" {
  *    both are built anew, not kept from an older library
  * 8: zen_balance_tables, zen_decode_dense_lists_status,
  *    zen_bitmap_dense_lists_status, zen_bitmap_encode_status
+ * 9: ZEN_MODE_WIDE
  */
-#define ZEN_ABI_VERSION 8
+#define ZEN_ABI_VERSION 9
 
 #define ZEN_F32 0
 #define ZEN_BF16 1
@@ -103,6 +104,9 @@ extern "C" {
    2^20 to 6 or 10 Mi slots then serve as owner tables, the quickest way at those sizes; without the flag such a call takes
    a path that leaves waiting samples alone.  Smaller tables never hold a sample. */
 #define ZEN_MODE_NO_SAMPLES 0x4000
+/* zen_load_balance: with ZEN_MODE_FAST, take the wide buckets wherever they fit, also where an owner table or the
+   bucket slabs are the quicker (ZEN_MODE_SLABS goes before this one).  Results are the same. */
+#define ZEN_MODE_WIDE 0x8000
 
 int zen_abi_version(void);
 

@@ -1042,6 +1042,55 @@ def test_load_balance_through_the_owner_table(zen, oracle, n, P, density, scale,
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("n,P,density,rehash", [
+    (1 << 21, 16, 0.15, 3),          # thousands of level-2/3 moves
+    (1 << 21, 16, 0.15, 2),          # two levels: serial entries in every partition
+    ((1 << 21) + 1237, 16, 0.03, 3),  # a length that is no multiple of anything, and a table that is none of 4096
+    ((1 << 20) + 2, 3, 0.05, 1),     # one level: whoever loses its slot ends in the serial list
+    (1 << 21, 4, 0.2, 1),            # more of those than a partition carries: declined
+])
+def test_nonzeros_on_the_wide_buckets_while_a_sample_waits(zen, oracle, n, P, density, rehash, dtype):
+    """A sample waits in the table of its call, which then is no owner table, and tables of 2^20 to 2^22 slots are too
+    small for the bucket slabs: selections of any density on the wide buckets, from tensors that begin on 16 bytes and
+    between, and from one without nonzeros.  The call the sample was taken for finds it untouched."""
+    from zen_repro_amd import _lib
+
+    g = make_grad(oracle, n, density, dtype, seed=n + rehash)
+    g[-1] = 0x3F80 if dtype == "bf16" else 1.0
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, rehash)
+    x = (np.random.default_rng(n).standard_normal(n) * 1e-3).astype(np.float32)
+    x[0] = 0
+    if dtype == "bf16":
+        x = (x.view(np.uint32) >> 16).astype(np.uint16)
+    k, capacity = 4000, len(idx_o) + 1024
+    masked, kept = oracle.mask_dense(x, int(oracle.kth_key(x, k)))
+    tp = zen.TensorPartition(P, 1, rehash)
+    m, _ = tp.table_sizes(n)
+    sampled = to_dev(x)
+    tp.prepare(sampled, k, 2 * k)
+    assert tp._ahead_state(sampled.device, 0)["pending"]
+    code = _lib.BF16 if dtype == "bf16" else _lib.F32
+    assert _lib.lib().zen_load_balance_path(n, m, code, capacity, P, 0, _lib.MODE_FAST) == 3
+    buf = to_dev(np.concatenate([g[:3], g]))
+    for d in (to_dev(g), buf[3:]):
+        oi, ov, splits, status = tp.load_balance_flat(d, capacity=capacity)
+        if (density, rehash) == (0.2, 1):
+            assert status.item() & _lib.STAT_RETRY
+            return
+        assert st_o == 0 and status.item() == 0 and np.array_equal(to_np(splits), splits_o)
+        assert np.array_equal(to_np(oi)[:len(idx_o)], idx_o) and np.array_equal(to_np(ov)[:len(idx_o)], val_o)
+    _, _, splits, status = tp.load_balance_flat(torch.zeros_like(buf[3:]), capacity=capacity)
+    assert status.item() == 0 and not splits.any()
+    assert tp._ahead_state(sampled.device, 0)["pending"]
+    idx_o, val_o, splits_o, _ = oracle.load_balance(masked, P, 1, rehash)
+    oi, ov, splits, status = tp.load_balance_flat(sampled, capacity=2 * k, k=k)
+    assert not tp._ahead_state(sampled.device, 0)["pending"]
+    assert status.item() == 0 and np.array_equal(to_np(splits), splits_o)
+    assert np.array_equal(to_np(oi)[:kept], idx_o) and np.array_equal(to_np(ov)[:kept], val_o)
+    assert not tp._table(sampled.device, m).any()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("n,P,density,rehash", [
     (9219, 4, 0.1, 3), (32768, 4, 0.6, 3),            # one workgroup: a list of selected indices, several of them
     (49152, 3, 0.1, 3), (49151, 3, 0.1, 2),           # partitions that end with a stretch, and in front of its end
     (1 << 18, 1000, 0.02, 3), (3000001, 16, 0.1, 1),  # dozens of partitions to a stretch; long serial tails

@@ -14,34 +14,38 @@ pytestmark = pytest.mark.gpu
 
 SLAB = 2
 WIDE = 3
-FLAGS = 0  # OR-ed into the fast mode of every call and path query of this module (set per run, below)
+FLAGS = 0  # OR-ed into the fast mode of every merge and its path query in this module (set per run, below)
+BALANCE_FLAGS = 0  # the same for the load balances
 
 
 @pytest.fixture(scope="module", autouse=True, params=["wide", "slabs"])
 def fast_path(request):
-    """Every test of this module runs twice: on the wide buckets (where the sizes suit them) and with
-    MODE_SLABS, which keeps the calls on the bucket slabs."""
-    global FLAGS
+    """Every test of this module runs twice: on the wide buckets (MODE_WIDE takes load balances there wherever they
+    fit) and with MODE_SLABS, which keeps the calls on the bucket slabs."""
+    global FLAGS, BALANCE_FLAGS
     import zen_repro_amd
     from zen_repro_amd import _lib
 
     FLAGS = _lib.MODE_SLABS if request.param == "slabs" else 0
-    zen_repro_amd.TensorPartition.fast_flags = FLAGS
+    BALANCE_FLAGS = FLAGS or _lib.MODE_WIDE
+    zen_repro_amd.TensorPartition.fast_flags = BALANCE_FLAGS
     zen_repro_amd.LoadBalanceAllreduce.fast_flags = FLAGS
     yield request.param
-    FLAGS = 0
+    FLAGS = BALANCE_FLAGS = 0
     zen_repro_amd.TensorPartition.fast_flags = 0
     zen_repro_amd.LoadBalanceAllreduce.fast_flags = 0
 
 
 def on_fast_path(code):
-    """Whether a zen_*_path answer is the path this run is about: the bucket slabs with MODE_SLABS, else the
-    wide buckets (sizes that take the bucket slabs either way are covered by the other run)."""
-    if FLAGS:
-        return code == SLAB
-    if code == SLAB:
-        pytest.skip("these sizes take the bucket slabs with or without MODE_SLABS: covered by the other run")
-    return code == WIDE
+    """Whether a zen_*_path answer is the path this run is about."""
+    return code == (SLAB if FLAGS else WIDE)
+
+
+def balance_mode(k):
+    """The mode of a load_balance_flat call of this run on whose slot no sample waits."""
+    from zen_repro_amd import _lib
+
+    return _lib.MODE_FAST | BALANCE_FLAGS | (0 if k else _lib.MODE_NO_SAMPLES)
 
 
 @pytest.fixture(scope="module")
@@ -58,7 +62,7 @@ def lb_path(zen, n, P, dtype, capacity, k=0, mode=0, scale=1):
     from zen_repro_amd import _lib
 
     m = int(n * scale // P * P)
-    return _lib.lib().zen_load_balance_path(n, m, 1 if dtype == "bf16" else 0, capacity, P, k, mode | FLAGS)
+    return _lib.lib().zen_load_balance_path(n, m, 1 if dtype == "bf16" else 0, capacity, P, k, mode | balance_mode(k))
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
@@ -101,8 +105,10 @@ def test_slab_load_balance_bit_exact(zen, oracle, n, P, density, rehash, dtype):
     (7000000, 3, 0.1, 2, 0.5),          # room for half: declined, and taken again with more
 ])
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
-def test_call_that_waits_gives_the_same_on_every_path(zen, oracle, n, P, density, rehash, room, dtype):
-    """load_balance waits for its sizes, which takes it off the wide buckets where the slabs fit."""
+def test_call_that_waits_gives_the_same_on_every_path(zen, oracle, n, P, density, rehash, room, dtype, monkeypatch):
+    """load_balance waits for its sizes, which takes it off the wide buckets where the slabs fit (and nothing asks for
+    them)."""
+    monkeypatch.setattr(zen.TensorPartition, "fast_flags", FLAGS)
     g = make_grad(oracle, n, density, dtype, seed=n + P)
     idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, rehash)
     assert st_o == 0
@@ -559,7 +565,7 @@ def test_table_and_merge_workspace_are_zero_again_after_every_call(zen, oracle):
         else:
             masked, cap = x_np, int(np.count_nonzero(x)) + 1024
         m, _ = tp.table_sizes(n)
-        assert on_fast_path(L.zen_load_balance_path(n, m, _lib.dtype_code(grad), cap, P, k, _lib.MODE_FAST | FLAGS))
+        assert on_fast_path(L.zen_load_balance_path(n, m, _lib.dtype_code(grad), cap, P, k, balance_mode(k)))
         idx, val, splits, st = tp.load_balance_flat(grad, None, cap, k=k)
         idx_o, val_o, splits_o, st_o = oracle.load_balance(masked, P, 1, 3)
         assert int(st.item()) == 0 and st_o == 0
@@ -600,7 +606,7 @@ def test_load_balance_without_a_capacity_takes_the_slab_path(zen, oracle):
     cap = tp._honest_capacity(grad, None, 0)
     m, _ = tp.table_sizes(n)
     assert cap < n // 100
-    assert on_fast_path(L.zen_load_balance_path(n, m, _lib.BF16, cap, P, 0, _lib.MODE_FAST | FLAGS))
+    assert on_fast_path(L.zen_load_balance_path(n, m, _lib.BF16, cap, P, 0, balance_mode(0)))
     assert L.zen_load_balance_workspace(n, m, _lib.BF16, cap, P) < 1 << 28
     indices, values, splits = tp.load_balance(grad)
     idx_o, val_o, splits_o, st_o = oracle.load_balance(g_np, P, 1, 3)
@@ -637,7 +643,7 @@ def test_sample_taken_ahead_gives_the_same_result(zen, oracle):
         wants.append(oracle.load_balance(masked, P, 1, 3))
     torch.cuda.synchronize()
     m, _ = tp.table_sizes(n)
-    assert on_fast_path(_lib.lib().zen_load_balance_path(n, m, _lib.BF16, grads[0][2], P, grads[0][1], _lib.MODE_FAST | FLAGS))
+    assert on_fast_path(_lib.lib().zen_load_balance_path(n, m, _lib.BF16, grads[0][2], P, grads[0][1], balance_mode(grads[0][1])))
 
     def check(out, want):
         idx, val, splits, st = out
@@ -835,7 +841,7 @@ def test_step_replayed_from_a_captured_graph(zen, oracle):
     tp = zen.TensorPartition(P, 1, 3)
     lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P), None, None)
     m, _ = tp.table_sizes(n)
-    assert on_fast_path(_lib.lib().zen_load_balance_path(n, m, _lib.BF16, cap, P, k, _lib.MODE_FAST | FLAGS))
+    assert on_fast_path(_lib.lib().zen_load_balance_path(n, m, _lib.BF16, cap, P, k, balance_mode(k)))
     assert on_fast_path(_lib.lib().zen_merge_path(flat_i.size, n, _lib.MODE_FAST | FLAGS))
 
     def check(enc, mrg):
@@ -896,7 +902,7 @@ def test_threshold_of_an_earlier_call_replaces_the_sample(zen, oracle, dtype):
     tp = zen.TensorPartition(P, 1, 3)
     m, _ = tp.table_sizes(n)
     code = _lib.BF16 if dtype == "bf16" else _lib.F32
-    assert on_fast_path(_lib.lib().zen_load_balance_path(n, m, code, cap, P, k, _lib.MODE_FAST | FLAGS))
+    assert on_fast_path(_lib.lib().zen_load_balance_path(n, m, code, cap, P, k, balance_mode(k)))
 
     def bits(x):
         return oracle.f32_to_bf16_bits(x) if dtype == "bf16" else x
@@ -1000,7 +1006,7 @@ def test_sample_taken_along_by_the_call_before(zen, oracle, dtype):
     lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P), None, None)
     for s_, k_, c_ in zip(sizes, ks, caps):
         m, _ = oracle.table_sizes(s_, P, 1)
-        assert on_fast_path(_lib.lib().zen_load_balance_path(s_, m, _lib.dtype_code(ds[0]), c_, P, k_, _lib.MODE_FAST | FLAGS))
+        assert on_fast_path(_lib.lib().zen_load_balance_path(s_, m, _lib.dtype_code(ds[0]), c_, P, k_, balance_mode(k_)))
     want_m = oracle.merge_sparse(ci, cv, n)
     _lib.profile_enable(True)
     outs = []

@@ -23,13 +23,14 @@ MODE_PREPARED, MODE_SECOND, MODE_DISCARD = 0x200, 0x400, 0x800  # zen_load_balan
 MODE_FLOOR = 0x1000  # zen_load_balance with k > 0: thr holds a key close to the threshold, no sample is taken
 MODE_SLABS = 0x2000  # fast mode without the wide-bucket path (bucket slabs where they fit)
 MODE_NO_SAMPLES = 0x4000  # zen_load_balance with k == 0: no sample taken ahead waits in the table
+MODE_WIDE = 0x8000  # fast mode on the wide buckets wherever they fit (zen_load_balance)
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # ZEN_HIP_LIB names another build of the library (a debug build, a build with other compile-time settings)
 LIB_PATH = os.environ.get("ZEN_HIP_LIB") or os.path.join(_HERE, "csrc", "libzen_hip.so")
 
 # ZEN_ABI_VERSION of include/zen_hip.h this loader's signatures and structs are written for
-ABI_VERSION = 8
+ABI_VERSION = 9
 TABLE_SIZES_MOST = 1024  # ZEN_TABLE_SIZES_MOST
 
 _lib = None

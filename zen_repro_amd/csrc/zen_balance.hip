@@ -539,10 +539,11 @@ namespace {
 // while collisions are few, up to about 8192 of them or one slot in 64 taken (three steps of 16 M bf16 elements on 16
 // partitions with their merges, top 0.5 % 228 and 259, 2 % 259 and 273, 3.5 % 297 and 300, 5 % 350 and 325; of 36 M, 2 %
 // 306 and 311, 3 % 383 and 343, 5 % 554 and 417; one of 743 M, 0.5 %, 392 and 493; three of 20 M with 0.5 % in whole rows,
-// no threshold, 192 and 215).
-bool takes_wide(int64_t n, int64_t m, int partitions, int dtype, int64_t capacity, int64_t k, bool waits) {
+// no threshold, 192 and 215).  asked: ZEN_MODE_WIDE.
+bool takes_wide(int64_t n, int64_t m, int partitions, int dtype, int64_t capacity, int64_t k, bool waits, bool asked) {
   using namespace zen;
   if (!wide_balance_fits(m, partitions, capacity, k, wide_device_cus(), nullptr)) return false;
+  if (asked) return true;
   const int64_t most = k > 0 ? k : capacity;
   const bool few = most <= m / 64 || (double)most * (double)most <= 2.0 * 8192.0 * (double)m;
   return (few && !waits) || !slab_balance_fits(n, m, partitions, dtype, capacity, k, nullptr);
@@ -554,10 +555,12 @@ extern "C" {
 
 int zen_load_balance_path(int64_t n, int64_t m, int dtype, int64_t capacity, int partitions, int64_t k, int mode) {
   const bool slabs_only = (mode & ZEN_MODE_SLABS) != 0, no_samples = (mode & ZEN_MODE_NO_SAMPLES) != 0;
+  const bool ask_wide = (mode & ZEN_MODE_WIDE) != 0;
   mode &= 0xff;
   if (mode != ZEN_MODE_FAST || partitions <= 0 || m <= 0 || m % partitions != 0) return 0;
-  if (!slabs_only && zen::table_balance_fits(n, m, partitions, capacity, k, no_samples)) return 1;
-  if (!slabs_only && takes_wide(n, m, partitions, dtype, capacity, k, false)) return 3;
+  const bool wide = !slabs_only && takes_wide(n, m, partitions, dtype, capacity, k, false, ask_wide);
+  if (!slabs_only && !(wide && ask_wide) && zen::table_balance_fits(n, m, partitions, capacity, k, no_samples)) return 1;
+  if (wide) return 3;
   if (zen::slab_balance_fits(n, m, partitions, dtype, capacity, k, nullptr)) return 2;
   return m >= 4096 ? 1 : 0;
 }
@@ -633,7 +636,9 @@ int load_balance_call(const void *input, int dtype, int64_t n, int64_t m, int pa
   const bool slabs_only = (mode & ZEN_MODE_SLABS) != 0;
   const bool splits_zero = (mode & ZEN_MODE_ZEROED) != 0;
   const bool no_samples = (mode & ZEN_MODE_NO_SAMPLES) != 0;
-  mode &= ~(ZEN_MODE_PREPARED | ZEN_MODE_SECOND | ZEN_MODE_FLOOR | ZEN_MODE_SLABS | ZEN_MODE_ZEROED | ZEN_MODE_NO_SAMPLES);
+  const bool ask_wide = (mode & ZEN_MODE_WIDE) != 0;
+  mode &= ~(ZEN_MODE_PREPARED | ZEN_MODE_SECOND | ZEN_MODE_FLOOR | ZEN_MODE_SLABS | ZEN_MODE_ZEROED | ZEN_MODE_NO_SAMPLES |
+            ZEN_MODE_WIDE);
   if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_load_balance: bad dtype");
   if (mode != ZEN_MODE_FAST && mode != ZEN_MODE_GENERAL) return fail(ZEN_EINVAL, "zen_load_balance: bad mode");
   if (n <= 0 || n > 0x7fffffffll || m <= 0 || m > 0x7fffffffll || partitions <= 0 || partitions > 65535 ||
@@ -652,10 +657,11 @@ int load_balance_call(const void *input, int dtype, int64_t n, int64_t m, int pa
   const int64_t spp = n / partitions / 10;  // tensor_load_balance.py:18
   const uint32_t drop_key = (uint32_t)partitions * (g.npp + 1u);
   const int bits = ceil_log2_u64(drop_key);
-  const bool small = mode == ZEN_MODE_FAST && !slabs_only && (reinterpret_cast<uintptr_t>(table) & 15u) == 0 &&
-                     table_balance_fits(n, m, partitions, capacity, k, no_samples);
   const bool wide = mode == ZEN_MODE_FAST && !slabs_only && (reinterpret_cast<uintptr_t>(table) & 7u) == 0 &&
-                    takes_wide(n, m, partitions, dtype, capacity, k, ask.answer.host != nullptr);
+                    takes_wide(n, m, partitions, dtype, capacity, k, ask.answer.host != nullptr, ask_wide);
+  const bool small = mode == ZEN_MODE_FAST && !slabs_only && !(wide && ask_wide) &&
+                     (reinterpret_cast<uintptr_t>(table) & 15u) == 0 &&
+                     table_balance_fits(n, m, partitions, capacity, k, no_samples);
   if (small || wide || (mode == ZEN_MODE_FAST && (reinterpret_cast<uintptr_t>(table) & 7u) == 0 &&
                slab_balance_fits(n, m, partitions, dtype, capacity, k, nullptr))) {
     SlabBalanceArgs sa;

@@ -227,7 +227,7 @@ class TensorPartition:
             return None, None
         n, n2 = flat.numel(), nxt.numel()
         key = (n, n2, flat.dtype, k, capacity, next_capacity, next_k,
-               mode & (0xff | _lib.MODE_SLABS | _lib.MODE_NO_SAMPLES))
+               mode & (0xff | _lib.MODE_SLABS | _lib.MODE_WIDE | _lib.MODE_NO_SAMPLES))
         able = self._samples_next.get(key)
         if able is None:
             L = _lib.lib()
@@ -262,7 +262,8 @@ class TensorPartition:
     def _leaves_samples(self, flat, k, capacity, mode):
         """Whether a call leaves the samples that wait on its slot alone.  The bucket paths do; the others take the
         floors' place in the workspace, and the owner-table paths every word of the table."""
-        key = (flat.numel(), flat.dtype, k, capacity, mode & (0xff | _lib.MODE_SLABS | _lib.MODE_NO_SAMPLES))
+        key = (flat.numel(), flat.dtype, k, capacity,
+               mode & (0xff | _lib.MODE_SLABS | _lib.MODE_WIDE | _lib.MODE_NO_SAMPLES))
         able = self._on_buckets.get(key)
         if able is None:
             if len(self._on_buckets) >= 256:  # capacities may differ from call to call
@@ -426,8 +427,8 @@ class TensorPartition:
                 m, _ = self.table_sizes(n)
                 self._table(tensor.device, m).zero_()
             if bits & _lib.STAT_RETRY:
-                modes.pop(0)
-                if modes and modes[0] & _lib.MODE_SLABS and _lib.lib().zen_load_balance_path(
+                tried = modes.pop(0)
+                if modes and modes[0] & _lib.MODE_SLABS and not tried & _lib.MODE_WIDE and _lib.lib().zen_load_balance_path(
                         n, self.table_sizes(n)[0], _lib.dtype_code(flat), capacity, self.partitions, int(k),
                         modes[0]) == 2:
                     modes.pop(0)  # a call that waits for its sizes was on the slabs already
