@@ -122,11 +122,10 @@ def test_call_that_waits_gives_the_same_on_every_path(zen, oracle, n, P, density
 
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("P,per_part", [(4, 800), (4, 960), (4, 1000), (2, 1024), (16, 1024)])
+@pytest.mark.parametrize("fast_path", ["wide"], indirect=True)  # (the slabs have neither)
 def test_slab_load_balance_at_a_round_of_records(zen, oracle, P, per_part, dtype):
     """Wide buckets whose slabs' parts hold fewer records than the workgroup has threads, more, or some of each: it keeps
     them in registers in the first case and loads them round by round in the others.  Hundreds lose their slot."""
-    if FLAGS:
-        pytest.skip("covered by the other run")
     n = 1 << 20
     k = per_part * 8 * 16
     x = (np.random.default_rng(P * per_part).standard_normal(n) * 1e-3).astype(np.float32)
@@ -145,10 +144,9 @@ def test_slab_load_balance_at_a_round_of_records(zen, oracle, P, per_part, dtype
 
 @pytest.mark.parametrize("rehash", [1, 2, 3])
 @pytest.mark.parametrize("P,k", [(4, 400), (4, 30000), (4, 45000), (4, 46300), (4, 48000), (1, 23000), (16, 92000), (3, 60000)])
+@pytest.mark.parametrize("fast_path", ["wide"], indirect=True)  # (the slabs have neither)
 def test_slab_load_balance_of_few_losers(zen, oracle, P, k, rehash):
     """Partitions with fewer and more entries that lose their first slot than their workgroups work out by themselves."""
-    if FLAGS:
-        pytest.skip("covered by the other run")
     n = -(-(1 << 20) // P) * P
     x = (np.random.default_rng(P * k).standard_normal(n) * 1e-3).astype(np.float32)
     x[0] = 0
