@@ -3,8 +3,11 @@ declares, argument validation happens on the host, the host-side helpers and
 the synthetic workloads behave, and the CPU baseline restatement agrees with
 the oracle.  No kernel is launched here."""
 import ctypes
+import json
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -479,6 +482,80 @@ def test_calls_that_return_early_leave_their_buffers_marked(monkeypatch, call, c
     # two of them may still read their input, which the allocator is told of; the others are through with theirs
     reads = call in ("load_balance", "encode_sparse_tensor")
     assert held == ([(dense.data_ptr(), s) for s in (1, 1, 2, 2, 1, 2)] if reads else [])
+
+
+@pytest.fixture(scope="module")
+def deviceless(tmp_path_factory, L):
+    """(name, fail_at, arguments) -> (return code, what was launched and waited for): the library's calls on a HIP
+    runtime without a device (fake_hip.py)."""
+    from zen_repro_amd import _lib
+
+    here = os.path.dirname(os.path.abspath(__file__))
+    fake = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", os.path.join(here, "fake_hip.cpp"), "-o", fake], check=True)
+    child = subprocess.Popen([sys.executable, os.path.join(here, "fake_hip.py"), fake, _lib.LIB_PATH],
+                             stdin=subprocess.PIPE, stdout=subprocess.PIPE, text=True)
+
+    def call(name, fail_at, args):
+        child.stdin.write(json.dumps([name, fail_at, args]) + "\n")
+        child.stdin.flush()
+        return json.loads(child.stdout.readline())
+
+    yield call
+    child.stdin.close()
+    child.wait(timeout=60)
+
+
+PTR, ROOM, STREAM = 4096, 1 << 50, 77  # an address nothing looks at, a workspace of any size, a stream
+WAITING_CALLS = {
+    "zen_balance_tables": [PTR, 1, 4096, PTR, 4096, PTR, 400, PTR, 4, 3, PTR, "host", 64, STREAM],
+    "zen_bitmap_encode_status": [PTR, 1000, PTR, 1, 100, None, PTR, 4000, PTR, PTR, "host", 64, STREAM],
+    "zen_select_count": [PTR, 1, 1 << 20, None, PTR, 1, PTR, 1 << 20, PTR, PTR, ROOM, PTR, "host", 64, STREAM],
+    "zen_table_find_sizes": [PTR, 4096, 4, 4096, PTR, PTR, PTR, ROOM, PTR, "host", 64, STREAM],
+    "zen_load_balance_sizes, one workgroup": [PTR, 1, 9000, 9000, 4, 3, None, 0, None, PTR, PTR, 1000, PTR, PTR, 0x4100, PTR, ROOM,
+                                              PTR, "host", 64, STREAM],
+    "zen_load_balance_sizes, owner table": [PTR, 1, 1 << 21, 1 << 21, 4, 3, None, 0, None, PTR, PTR, 1000, PTR, PTR, 0x4100, PTR,
+                                            ROOM, PTR, "host", 64, STREAM],
+    "zen_load_balance_sizes, slabs": [PTR, 0, 1 << 24, 1 << 24, 4, 3, None, 1000, None, PTR, PTR, 2000, PTR, PTR, 0x100, PTR, ROOM,
+                                      PTR, "host", 64, STREAM],
+    "zen_load_balance_sizes, wide buckets": [PTR, 0, 1 << 24, 1 << 24, 4, 3, None, 1000, None, PTR, PTR, 2000, PTR, PTR, 0x8100, PTR,
+                                             ROOM, PTR, "host", 64, STREAM],
+    "zen_load_balance_sizes, general": [PTR, 0, 1 << 16, 1 << 16, 4, 3, None, 0, None, PTR, PTR, 2000, PTR, PTR, 1, PTR, ROOM, PTR,
+                                        "host", 64, STREAM],
+    "zen_merge_rounded_count, one workgroup": [PTR, 0, PTR, 1, 1000, 1 << 20, PTR, 0, PTR, 1000, PTR, 0x100, PTR, ROOM, PTR, "host",
+                                               64, STREAM],
+    "zen_merge_rounded_count, wide buckets": [PTR, 0, PTR, 1, 100000, 1 << 24, PTR, 0, PTR, 1000, PTR, 0x100, PTR, ROOM, PTR, "host",
+                                              64, STREAM],
+    "zen_merge_rounded_count, slabs": [PTR, 0, PTR, 1, 400000, 1 << 26, PTR, 0, PTR, 1000, PTR, 0x2100, PTR, ROOM, PTR, "host", 64,
+                                       STREAM],
+    "zen_merge_rounded_count, general": [PTR, 0, PTR, 1, 10000, 1 << 24, PTR, 0, PTR, 1000, PTR, 1, PTR, ROOM, PTR, "host", 64, STREAM],
+    "zen_decode_dense_status": [PTR, 1, PTR, 0, 100000, PTR, 1 << 24, 0x100, PTR, ROOM, PTR, "host", 64, STREAM],
+    "zen_decode_dense_lists_status": [[PTR, PTR], 1, [PTR, PTR], 1, [50, 60], 2, PTR, 1 << 20, PTR, ROOM, PTR, "host", 64, STREAM],
+    "zen_decode_dense_lists_status, many tiles": [[PTR, PTR], 1, [PTR, PTR], 1, [50, 60], 2, PTR, 1 << 26, PTR, ROOM, PTR, "host", 64,
+                                                  STREAM],
+    "zen_bitmap_dense_lists_status": [PTR, 1 << 20, 2, [PTR, PTR], [1 << 16, 1 << 16], [PTR, PTR], 1, [50, 60], PTR, PTR, ROOM, PTR,
+                                      "host", 64, STREAM],
+    "zen_read_back": [PTR, 3, 1, None, 0, 0, None, 0, 0, "host", 64, STREAM],
+}
+
+
+@pytest.mark.parametrize("what", list(WAITING_CALLS))
+def test_a_failed_call_leaves_no_answer_on_its_way(deviceless, what):
+    """A call that waits draws the ticket of its answer from the host's words, where a call that fails leaves them as
+    they were: the next one would take a late answer of this one for its own.  So whichever launch fails, the stream has
+    been waited for when the call returns."""
+    from zen_repro_amd import _lib
+
+    name, args = what.split(",")[0], WAITING_CALLS[what]
+    _, log = deviceless(name, 0, args)
+    launches = [line for line in log if line.startswith("launch")]
+    assert launches and all(line.endswith(f" {STREAM}") for line in launches)
+    for fail_at in range(1, 40):
+        rc, log = deviceless(name, fail_at, args)
+        if "fail" not in log:  # fewer checks than that
+            break
+        assert rc == _lib.EHIP and log[-2:] == ["fail", f"wait {STREAM}"]
+    assert fail_at > 1 and log == launches
 
 
 def test_every_call_gets_zeroed_words_of_its_own():

@@ -506,10 +506,11 @@ int zen_balance_tables(const void *input, int dtype, int64_t n, int32_t *memory,
   k_new_tables<<<dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(256), 0, s>>>(
       reinterpret_cast<uint32_t *>(memory), m, reinterpret_cast<uint32_t *>(serial), serial_n, offset, partitions,
       serial_n / partitions);
-  ZEN_LAUNCH_CHECK("k_new_tables");
-  rc = zen_sparse_balance(input, dtype, n, memory, m, serial, serial_n, offset, partitions, rehash, status, stream);
+  const hipError_t e = hipGetLastError();
+  rc = e == hipSuccess ? zen_sparse_balance(input, dtype, n, memory, m, serial, serial_n, offset, partitions, rehash, status, stream)
+                       : hip_fail(e, "k_new_tables");
   if (rc == ZEN_OK) rc = host_answer_launch(answer, nullptr, 0, status, 1, s);
-  return rc == ZEN_OK ? host_wait(answer, s) : rc;
+  return host_finish(rc, answer, s);
 }
 
 size_t zen_load_balance_workspace(int64_t n, int64_t m, int dtype, int64_t capacity, int partitions) {
@@ -824,9 +825,7 @@ int zen_load_balance_sizes(const void *input, int dtype, int64_t n, int64_t m, i
   rc = load_balance_call(input, dtype, n, m, partitions, rehash, thr, k, thr_out, out_idx, out_val, capacity, splits, table,
                          mode, workspace, workspace_bytes, status, stream, nullptr, 0, 0, 0, 0, nullptr, HostAsk{answer, &answered});
   if (rc == ZEN_OK && !answered) rc = host_answer_launch(answer, splits, partitions, status, 1, s);
-  if (rc == ZEN_OK) return host_wait(answer, s);
-  if (answered) (void)hipStreamSynchronize(s);  // an answer may be on its way: not into a later call's words
-  return rc;
+  return host_finish(rc, answer, s);
 }
 
 int zen_encode_merge_samples_next(int64_t n, int64_t m, int dtype, int64_t capacity, int partitions, int64_t k,

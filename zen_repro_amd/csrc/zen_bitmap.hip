@@ -343,7 +343,7 @@ int zen_bitmap_encode_status(const int64_t *mapping_p, int64_t mapping_n, const 
   rc = zen_bitmap_encode(mapping_p, mapping_n, idx, idx64, idx_n, idx_n_dev, rank_at, numel, bitmap_words, status, stream);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (rc == ZEN_OK) rc = host_answer_launch(answer, nullptr, 0, status, 1, s);
-  return rc == ZEN_OK ? host_wait(answer, s) : rc;
+  return host_finish(rc, answer, s);
 }
 
 size_t zen_bitmap_decode_workspace(int64_t mapping_n) {

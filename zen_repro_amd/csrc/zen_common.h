@@ -421,7 +421,8 @@ int bucket_sort_pairs(uint32_t *keys_a, uint32_t *vals_a, uint32_t *keys_b, uint
 int host_ask(int64_t *host, int64_t words, int64_t need, HostAnswer *answer);
 // One kernel that answers with the words two arrays hold, for calls whose kernels do not.
 int host_answer_launch(const HostAnswer &answer, const int64_t *first, int n0, const int32_t *second, int n1, hipStream_t s);
-// Returns when the answer is there, or with the stream's error.
-int host_wait(const HostAnswer &answer, hipStream_t s);
+// The end of a call that asked, `rc` of its launches: returns when the answer is there, or with an error (the stream's
+// among them) when no answer to this call can come any more.
+int host_finish(int rc, const HostAnswer &answer, hipStream_t s);
 
 }  // namespace zen

@@ -439,7 +439,7 @@ int zen_select_count(const void *input, int dtype, int64_t n, const uint32_t *th
   rc = select_call(input, dtype, n, thr, out_idx, idx64, out_val, capacity, out_count, workspace, workspace_bytes,
                    status, stream, answer);
   if (rc == ZEN_OK && n == 0) rc = host_answer_launch(answer, out_count, 1, status, 1, s);
-  return rc == ZEN_OK ? host_wait(answer, s) : rc;
+  return host_finish(rc, answer, s);
 }
 
 }  // extern "C"

@@ -383,7 +383,7 @@ int zen_decode_dense_lists_status(const void *const *idx, int idx64_in, const vo
   int rc = host_ask(host, words, 1, &answer);
   if (rc != ZEN_OK) return rc;
   rc = decode_lists_call(idx, idx64_in, val, dtype, len, nlists, dense, dense_n, workspace, workspace_bytes, status, stream, answer);
-  return rc == ZEN_OK ? host_wait(answer, static_cast<hipStream_t>(stream)) : rc;
+  return host_finish(rc, answer, static_cast<hipStream_t>(stream));
 }
 
 int zen_decode_dense_sorted(const void *idx, int idx64_in, const void *val, int dtype, const int64_t *list_start,

@@ -548,7 +548,7 @@ int zen_bitmap_dense_lists_status(const void *dict, int64_t numel, int partition
   if (rc != ZEN_OK) return rc;
   rc = bitmap_dense_call(dict, numel, partitions, bitmaps, bitmap_bytes, values, dtype, value_count, dense, workspace,
                          workspace_bytes, status, stream, answer);
-  return rc == ZEN_OK ? host_wait(answer, static_cast<hipStream_t>(stream)) : rc;
+  return host_finish(rc, answer, static_cast<hipStream_t>(stream));
 }
 
 int zen_bitmap_dense(const void *dict, int64_t numel, int partitions, const uint8_t *bitmaps,

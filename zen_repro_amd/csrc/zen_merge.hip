@@ -836,9 +836,7 @@ int zen_merge_rounded_count(const void *idx, int idx64_in, const void *val, int 
   rc = merge_call(idx, idx64_in, val, dtype, r, dense_n, out_idx, idx64_out, out_val, true, capacity, out_count, mode,
                   workspace, workspace_bytes, status, stream, HostAsk{answer, &answered});
   if (rc == ZEN_OK && !answered) rc = host_answer_launch(answer, out_count, 1, status, 1, s);
-  if (rc == ZEN_OK) return host_wait(answer, s);
-  if (answered) (void)hipStreamSynchronize(s);  // an answer may be on its way: not into a later call's words
-  return rc;
+  return host_finish(rc, answer, s);
 }
 
 size_t zen_decode_dense_workspace(int64_t r, int64_t dense_n) {
@@ -925,9 +923,7 @@ int zen_decode_dense_status(const void *idx, int idx64_in, const void *val, int 
   rc = decode_call(idx, idx64_in, val, dtype, r, dense, dense_n, mode, workspace, workspace_bytes, status, stream,
                    HostAsk{answer, &answered});
   if (rc == ZEN_OK && !answered) rc = host_answer_launch(answer, nullptr, 0, status, 1, s);
-  if (rc == ZEN_OK) return host_wait(answer, s);
-  if (answered) (void)hipStreamSynchronize(s);  // an answer may be on its way: not into a later call's words
-  return rc;
+  return host_finish(rc, answer, s);
 }
 
 }  // extern "C"

@@ -97,14 +97,17 @@ int host_ask(int64_t *host, int64_t words, int64_t need, HostAnswer *answer) {
   return ZEN_OK;
 }
 
-int host_answer_launch(const HostAnswer &answer, const int64_t *first, int n0, const int32_t *second, int n1, hipStream_t s) {
-  const ReadBack r{{first, second, nullptr}, {n0, n1, 0}, {1, 0, 0}};
+static int read_back_launch(const ReadBack &r, const HostAnswer &answer, hipStream_t s) {
   k_read_back<<<dim3(1), dim3(64), 0, s>>>(r, answer.host, answer.ticket);
   ZEN_LAUNCH_CHECK("k_read_back");
   return ZEN_OK;
 }
 
-int host_wait(const HostAnswer &answer, hipStream_t s) {
+int host_answer_launch(const HostAnswer &answer, const int64_t *first, int n0, const int32_t *second, int n1, hipStream_t s) {
+  return read_back_launch(ReadBack{{first, second, nullptr}, {n0, n1, 0}, {1, 0, 0}}, answer, s);
+}
+
+static int host_wait(const HostAnswer &answer, hipStream_t s) {
   // The waits of a call are short: this core watches for the answer.  A longer one is for what the stream has to wait
   // for itself (an exchange, other ranks): then the core is left to others, for a sixteenth of the time waited so far
   // and a millisecond at most, and the stream is asked every time, which says when something on it has failed.  (The
@@ -127,6 +130,14 @@ int host_wait(const HostAnswer &answer, hipStream_t s) {
                ? ZEN_OK
                : fail(ZEN_EHIP, "zen_read_back: the stream ended without an answer");
   }
+}
+
+int host_finish(int rc, const HostAnswer &answer, hipStream_t s) {
+  if (rc == ZEN_OK) return host_wait(answer, s);
+  // The kernel with the answer may have been launched all the same (one behind it failed, or the error was an older
+  // one): its ticket is the next call's too, so it has to be there before this one returns.
+  if (rc == ZEN_EHIP) (void)hipStreamSynchronize(s);
+  return rc;
 }
 
 }  // namespace zen
@@ -160,10 +171,8 @@ int zen_read_back(const void *p0, int n0, int wide0, const void *p1, int n1, int
   }
   if (!host || total > words) return fail(ZEN_EINVAL, "zen_read_back: host buffer missing or too small");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t ticket = host[0] + 1;
-  k_read_back<<<dim3(1), dim3(64), 0, s>>>(r, host, ticket);
-  ZEN_LAUNCH_CHECK("k_read_back");
-  return host_wait(HostAnswer{host, ticket}, s);
+  const HostAnswer answer{host, host[0] + 1};
+  return host_finish(read_back_launch(r, answer, s), answer, s);
 }
 
 int zen_count(const void *input, int dtype, int64_t n, const uint32_t *thr, int64_t *count, void *stream) {

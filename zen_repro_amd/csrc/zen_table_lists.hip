@@ -347,8 +347,8 @@ int zen_table_find_sizes(const int32_t *table, int64_t m, int partitions, int64_
   tm.part = tm.group + (size_t)tm.groups * tm.parts;
   tm.done = reinterpret_cast<uint32_t *>(tm.part + tm.parts);
   k_table_walk<true><<<dim3(tm.per_part * tm.parts), dim3(kBlock), 0, s>>>(table, n, tp, tm, splits, answer, status);
-  ZEN_LAUNCH_CHECK("k_table_walk");
-  return host_wait(answer, s);
+  const hipError_t e = hipGetLastError();
+  return host_finish(e == hipSuccess ? ZEN_OK : hip_fail(e, "k_table_walk"), answer, s);
 }
 
 int zen_table_gather(const int32_t *table, int64_t m, int partitions, const void *input, int dtype, int64_t n,
