@@ -572,8 +572,8 @@ int zen_bitmap_dense_lists(const void *dict, int64_t numel, int partitions, cons
                            const int64_t *bitmap_bytes, const void *const *values, int dtype,
                            const int64_t *value_count, void *dense, void *workspace, size_t workspace_bytes,
                            int32_t *status, void *stream);
-/* Returns when the status is known, with it in host[1] (host: `words` >= 2 of zen_host_words_alloc): the tensor, for
-   which bitmaps, values, dictionary and workspace are still read, is complete in the order of `stream`. */
+/* Returns when the tensor is complete, with the status word in host[1] (host: `words` >= 2 of
+   zen_host_words_alloc). */
 int zen_bitmap_dense_lists_status(const void *dict, int64_t numel, int partitions, const uint8_t *const *bitmaps,
                                   const int64_t *bitmap_bytes, const void *const *values, int dtype,
                                   const int64_t *value_count, void *dense, void *workspace, size_t workspace_bytes,

@@ -331,6 +331,28 @@ def test_bitmaps_to_dense_with_values_in_any_layout(zen, oracle, form):
     assert got.dtype == torch.float32 and np.array_equal(to_np(got), _dense_truth(oracle, n, idx, val))
 
 
+def test_bitmaps_to_dense_is_complete_for_every_stream(zen):
+    """When the call has returned another stream may overwrite bitmaps and values and read the tensor, without a wait."""
+    n, P = 1 << 26, 16
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    room = n // P + 8192  # (a partition's members: about n / P)
+    bitmaps = [torch.randint(0, 256, (room // 8,), generator=gen, device="cuda", dtype=torch.uint8) for _ in range(P)]
+    values = [torch.randn(room, generator=gen, device="cuda").bfloat16() for _ in range(P)]
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P, 0), None, None)
+    want = lba.decode_bitmaps_dense(bitmaps, values, n)
+    side = torch.cuda.Stream()
+    for _ in range(3):
+        b, v = [t.clone() for t in bitmaps], [t.clone() for t in values]
+        torch.cuda.synchronize()
+        got = lba.decode_bitmaps_dense(b, v, n)
+        with torch.cuda.stream(side):
+            seen = got.clone()
+            for t in b + v:
+                t.zero_()
+        torch.cuda.synchronize()
+        assert torch.equal(seen, want) and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("special", range(12))
 @pytest.mark.parametrize("n, P", [(8192, 1), (24576 + 80, 1), (3 * 8192 + 17, 3), (1 << 17, 16)])
 def test_bitmaps_to_dense_special_values(zen, oracle, n, P, special):

@@ -509,11 +509,9 @@ class LoadBalanceAllreduce:
         dictionary of two bytes per element (per tile of the dense tensor, the
         places of its indices ordered by partition) is built on first use of a
         `numel` and cached like the reference caches the mapping
-        (comm.py:132-134).  The call waits until it is known whether bitmaps and
-        values agree; the dense tensor is complete on the current stream, and the
-        bitmaps and values are still read until then: another stream that reads the
-        result or overwrites them waits for this one first (dropping them is
-        safe)."""
+        (comm.py:132-134).  The call waits for the dense tensor and for what is
+        said about bitmaps and values that do not agree: any stream may read the
+        result and overwrite what it came from when the call has returned."""
         if len(bitmap_indices) != self.partitions or len(values_tensors) != self.partitions:
             raise RuntimeError("decode_bitmaps_dense: one bitmap and one value list per rank")
         for t in bitmap_indices:
@@ -542,7 +540,6 @@ class LoadBalanceAllreduce:
         rc, dense = _lib.host.bitmaps_dense(L.zen_bitmap_dense_lists_status, _lib.zeros.native(), bitmap_indices, values,
                                             _lib.dtype_code(values[0]), cached, numel, ws, _lib.stream_of(dev), words.ptr,
                                             words.words)
-        _lib.scratch.left_running(dev, "bitmap_dense")
         _lib.check(rc, "decode_bitmaps_dense")
         bits = words.view[1]  # the reference's masking and scatter_add_ raise on a mismatch, also a sync
         if bits & _lib.STAT_BAD_INDEX:

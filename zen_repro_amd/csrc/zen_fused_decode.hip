@@ -185,32 +185,17 @@ __global__ __launch_bounds__(kFdGroup) void k_fd_count(const uint32_t *__restric
 }
 
 // Per list (blockIdx.x): exclusive prefix over the groups' sums, in place (a tensor of 2^31 elements has 1024 groups).
-// What the status word can come to is known here: a list with more set bits than values raises ZEN_STAT_BAD_INDEX, and
-// the last of the lists tells the host, which goes on while the tiles are written (the lists count themselves in the
-// status word, above its flags).
+// A list with more set bits than values raises ZEN_STAT_BAD_INDEX.
 constexpr int kFdGroupsMax = 1024;
-constexpr int kFdFlags = 8;
 __global__ __launch_bounds__(kFdGroupsMax) void k_fd_groups(uint32_t *__restrict__ gsum, uint32_t groups, int P, FdLists lists,
-                                                            HostAnswer answer, int32_t *status) {
+                                                            int32_t *status) {
   __shared__ uint32_t s_scan[kFdGroupsMax / 64 + 1];
   uint32_t *at = gsum + (size_t)threadIdx.x * P + blockIdx.x;
   const uint32_t v = threadIdx.x < groups ? *at : 0u;
   uint32_t total;
   const uint32_t before = block_exclusive_scan<uint32_t, kFdGroupsMax>(v, s_scan, &total);
   if (threadIdx.x < groups) *at = before;
-  if (threadIdx.x != 0) return;
-  if (total > lists.vals[blockIdx.x]) {
-    atomicOr(status, ZEN_STAT_BAD_INDEX);
-    wait_global_acks();
-  }
-  if (!answer.host) return;
-  const uint32_t word = (uint32_t)atomicAdd(status, 1 << kFdFlags);
-  if ((word >> kFdFlags) != (uint32_t)P - 1u) return;
-  const int32_t flags = (int32_t)(word & ((1u << kFdFlags) - 1u));
-  __hip_atomic_store(status, flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  host_store(answer.host + 1, (int64_t)flags);
-  wait_global_acks();
-  host_store(answer.host, answer.ticket);
+  if (threadIdx.x == 0 && total > lists.vals[blockIdx.x]) atomicOr(status, ZEN_STAT_BAD_INDEX);
 }
 
 // Words of a chunk: sixteen lists have 512 members in a tile, few more than 576.  Tile kernel with 8, 9 and 10 words, us,
@@ -484,10 +469,10 @@ size_t zen_bitmap_dense_workspace(int64_t numel, int partitions) {
   return zen::fd_vstart_bytes(numel, partitions) + zen::fd_gsum_bytes(numel, partitions);
 }
 
-static int bitmap_dense_call(const void *dict, int64_t numel, int partitions, const uint8_t *const *bitmaps,
-                             const int64_t *bitmap_bytes, const void *const *values, int dtype,
-                             const int64_t *value_count, void *dense, void *workspace, size_t workspace_bytes,
-                             int32_t *status, void *stream, const zen::HostAnswer &answer) {
+int zen_bitmap_dense_lists(const void *dict, int64_t numel, int partitions, const uint8_t *const *bitmaps,
+                           const int64_t *bitmap_bytes, const void *const *values, int dtype,
+                           const int64_t *value_count, void *dense, void *workspace, size_t workspace_bytes,
+                           int32_t *status, void *stream) {
   using namespace zen;
   const int rc = fd_check(numel, partitions);
   if (rc != ZEN_OK) return rc;
@@ -518,7 +503,7 @@ static int bitmap_dense_call(const void *dict, int64_t numel, int partitions, co
   k_fd_count<<<dim3(groups, (unsigned)partitions), dim3(kFdGroup), 0, s>>>(below, tiles, partitions, lists, vstart, gsum,
                                                                        status);
   ZEN_LAUNCH_CHECK("k_fd_count");
-  k_fd_groups<<<dim3((unsigned)partitions), dim3(kFdGroupsMax), 0, s>>>(gsum, groups, partitions, lists, answer, status);
+  k_fd_groups<<<dim3((unsigned)partitions), dim3(kFdGroupsMax), 0, s>>>(gsum, groups, partitions, lists, status);
   ZEN_LAUNCH_CHECK("k_fd_groups");
   if (dtype == ZEN_BF16)
     k_fd_tiles<uint16_t><<<dim3(tiles), dim3(fd_tile_block<uint16_t>()), 0, s>>>(order, below, vstart, gsum, partitions, (uint32_t)numel,
@@ -530,14 +515,6 @@ static int bitmap_dense_call(const void *dict, int64_t numel, int partitions, co
   return ZEN_OK;
 }
 
-int zen_bitmap_dense_lists(const void *dict, int64_t numel, int partitions, const uint8_t *const *bitmaps,
-                           const int64_t *bitmap_bytes, const void *const *values, int dtype,
-                           const int64_t *value_count, void *dense, void *workspace, size_t workspace_bytes,
-                           int32_t *status, void *stream) {
-  return bitmap_dense_call(dict, numel, partitions, bitmaps, bitmap_bytes, values, dtype, value_count, dense, workspace,
-                           workspace_bytes, status, stream, {});
-}
-
 int zen_bitmap_dense_lists_status(const void *dict, int64_t numel, int partitions, const uint8_t *const *bitmaps,
                                   const int64_t *bitmap_bytes, const void *const *values, int dtype,
                                   const int64_t *value_count, void *dense, void *workspace, size_t workspace_bytes,
@@ -546,9 +523,11 @@ int zen_bitmap_dense_lists_status(const void *dict, int64_t numel, int partition
   HostAnswer answer;
   int rc = host_ask(host, words, 1, &answer);
   if (rc != ZEN_OK) return rc;
-  rc = bitmap_dense_call(dict, numel, partitions, bitmaps, bitmap_bytes, values, dtype, value_count, dense, workspace,
-                         workspace_bytes, status, stream, answer);
-  return host_finish(rc, answer, static_cast<hipStream_t>(stream));
+  rc = zen_bitmap_dense_lists(dict, numel, partitions, bitmaps, bitmap_bytes, values, dtype, value_count, dense, workspace,
+                              workspace_bytes, status, stream);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (rc == ZEN_OK) rc = host_answer_launch(answer, nullptr, 0, status, 1, s);
+  return host_finish(rc, answer, s);
 }
 
 int zen_bitmap_dense(const void *dict, int64_t numel, int partitions, const uint8_t *bitmaps,

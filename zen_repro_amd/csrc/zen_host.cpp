@@ -5,7 +5,6 @@
 //
 // A library function arrives as the ctypes object that stands for it, so that whoever replaces the library replaces it
 // here too; ctypes lets other threads run while the function does.
-#include <c10/core/impl/DeviceGuardImplInterface.h>
 #include <torch/extension.h>
 
 #include <algorithm>
@@ -199,14 +198,6 @@ py::tuple bitmaps_dense(const py::object &fn, Zeros &zeros, const std::vector<Te
   const Lists b(bitmaps), v(values);
   const py::object rc = fn(address(dict), numel, bitmaps.size(), b.addresses(), b.counts(), v.addresses(), code, v.counts(),
                            address(dense), address(ws), ws.numel(), address(status), host, words, stream);
-  // the call returns while its last kernel reads these: their memory is not handed out before that, also if it belongs to
-  // another stream's pool and its owner drops it now
-  if (dense.is_cuda()) {
-    const c10::Stream now = c10::impl::getDeviceGuardImpl(dense.device().type())->getStream(dense.device());
-    for (const auto *list : {&bitmaps, &values})
-      for (const Tensor &t : *list) t.record_stream(now);
-    dict.record_stream(now);
-  }
   return py::make_tuple(rc, dense);
 }
 
