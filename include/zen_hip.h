@@ -532,8 +532,8 @@ size_t zen_decode_dense_sorted_workspace(int64_t dense_n, int nlists);
 int zen_decode_dense_lists(const void *const *idx, int idx64_in, const void *const *val, int dtype,
                            const int64_t *len, int nlists, void *dense, int64_t dense_n,
                            void *workspace, size_t workspace_bytes, int32_t *status, void *stream);
-/* Returns when every entry has been read, with the status word in host[1] (host: `words` >= 2 of
-   zen_host_words_alloc); the dense tensor is complete in the order of `stream`. */
+/* Returns when the tensor is complete, with the status word in host[1] (host: `words` >= 2 of
+   zen_host_words_alloc). */
 int zen_decode_dense_lists_status(const void *const *idx, int idx64_in, const void *const *val, int dtype,
                                   const int64_t *len, int nlists, void *dense, int64_t dense_n,
                                   void *workspace, size_t workspace_bytes, int32_t *status,

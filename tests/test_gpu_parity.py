@@ -772,8 +772,8 @@ def test_decode_ascending_lists_without_a_sort(zen, oracle, n, nlists, per_list,
 
 @pytest.mark.parametrize("n", [256 * 8192, 256 * 8192 + 1, 4096 * 8192, 4096 * 8192 + 1])
 def test_decode_ascending_tells_the_host(zen, oracle, n):
-    """The sizes at which another kernel tells the host (tiles that search for themselves, tiles that count, a kernel
-    behind them): right lists bit for bit, a descent seen, and the call after it right again."""
+    """Tiles that search for themselves, up to the last size that does, and tiles with a kernel in front: right lists bit
+    for bit, a descent seen, and the call after it right again."""
     rng = np.random.default_rng(n)
     idx, val = ascending_lists(oracle, rng, n, 4, 20000, 0.1, "bf16", np.int64)
     want = oracle.f32_to_bf16_bits(oracle.decode(np.concatenate(idx), np.concatenate(val), n, "f32acc"))
@@ -784,6 +784,27 @@ def test_decode_ascending_tells_the_host(zen, oracle, n):
     for _ in range(2):
         assert np.array_equal(to_np(lba._decode_ascending(d_idx, d_val, n)).view(want.dtype), want)
         assert lba._decode_ascending([to_dev(i) for i in swapped], d_val, n) is None
+
+
+@pytest.mark.parametrize("n", [200000, 20000000, 100000000])
+def test_decode_ascending_is_complete_for_every_stream(zen, n):
+    """When the call has returned another stream may overwrite the lists and read the tensor, without a wait."""
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    idx = [torch.nonzero(torch.rand(n, generator=gen, device="cuda") < 0.02).view(-1) for _ in range(3)]
+    val = [torch.randn(i.numel(), generator=gen, device="cuda").bfloat16() for i in idx]
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(3), None, None)
+    want = lba._decode_ascending(idx, val, n)
+    side = torch.cuda.Stream()
+    for _ in range(3):
+        i, v = [t.clone() for t in idx], [t.clone() for t in val]
+        torch.cuda.synchronize()
+        got = lba._decode_ascending(i, v, n)
+        with torch.cuda.stream(side):
+            seen = got.clone()
+            for t in i + v:
+                t.zero_()
+        torch.cuda.synchronize()
+        assert torch.equal(seen, want) and torch.equal(got, want)
 
 
 def test_decode_ascending_declines_what_is_not_ascending(zen, oracle):

@@ -558,11 +558,16 @@ def test_a_failed_call_leaves_no_answer_on_its_way(deviceless, what):
     assert fail_at > 1 and log == launches
 
 
-def test_the_bitmap_decode_is_done_when_its_status_is_known(deviceless):
-    """The host is told by a kernel behind the tiles: nobody reads bitmaps and values any more when the call returns, the
-    tensor is there for every stream, and what a tile has to say about the dictionary is in the status."""
-    rc, log = deviceless("zen_bitmap_dense_lists_status", 0, WAITING_CALLS["zen_bitmap_dense_lists_status"])
-    assert rc == 0 and "k_fd_tiles" in log[-2] and "k_read_back" in log[-1]
+@pytest.mark.parametrize("what,tiles", [
+    ("zen_bitmap_dense_lists_status", "k_fd_tiles"),
+    ("zen_decode_dense_lists_status", "k_decode_tiles"),
+    ("zen_decode_dense_lists_status, many tiles", "k_decode_tiles"),
+])
+def test_a_decode_is_done_when_its_status_is_known(deviceless, what, tiles):
+    """The host is told by a kernel behind the tiles: nobody reads the lists any more when the call returns, the tensor is
+    there for every stream, and what a tile has to say about the bitmaps' dictionary is in the status."""
+    rc, log = deviceless(what.split(",")[0], 0, WAITING_CALLS[what])
+    assert rc == 0 and tiles in log[-2] and "k_read_back" in log[-1]
 
 
 def test_every_call_gets_zeroed_words_of_its_own():

@@ -69,25 +69,17 @@ __device__ inline uint32_t decode_start(const I *__restrict__ list, uint32_t len
   return lo;
 }
 
-// Tiles that have looked at their entries, counted for the host: a line takes ten nanoseconds for an add, so the tiles
-// form groups with a counter each.  Few tiles search for themselves and count in the status word, above its flags.
-constexpr int kDecGroups = 64, kDecPad = 32;
-constexpr int kDecCounters = (kDecGroups + 1) * kDecPad;
+// Up to so many tiles, one to a compute unit, search for themselves: a launch less, for a chain of probes in every tile
+// (bf16, a call with the search in the tiles / in a kernel in front: two lists into 9000 elements 22.2 / 25.2 us, four
+// into a million 24.2 / 26.2, sixteen of a tenth of two million 44.7 / 47.8).
 constexpr int64_t kDecFew = 256;
-// Up to so many tiles the host is told by the last one; beyond, by a kernel behind them: a tile that counts stays on its
-// compute unit until the count is back, some 0.4 us of its 7, which the launch it saves makes up for while the tiles are
-// few rounds.  Sixteen lists of 0.4 % of the elements each into bf16, told by the tiles / by a kernel behind them, a call:
-// 454 tiles 26.7 / 27.8 us, 1890 34.5 / 35.3, 5672 55.8 / 56.2, 11 344 87.4 / 86.0, 22 688 165 / 160, 90 752 783 / 756.
-constexpr int64_t kDecTold = 4096;
-constexpr int kDecFlags = 8;
 
 // starts[l * (ntiles + 1) + t]: decode_start of list l.
 template <typename I>
 __global__ __launch_bounds__(256) void k_decode_starts(DecLists lists, int64_t ntiles, int64_t dense_n,
-                                                       uint32_t *__restrict__ starts, uint32_t *__restrict__ counters) {
+                                                       uint32_t *__restrict__ starts) {
   const int l = blockIdx.y;
   const int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
-  if (blockIdx.x == 0 && l == 0 && threadIdx.x <= kDecGroups) counters[threadIdx.x * kDecPad] = 0;
   if (t > ntiles) return;
   starts[(int64_t)l * (ntiles + 1) + t] =
       decode_start(static_cast<const I *>(lists.idx[l]), lists.len[l], t, ntiles, dense_n);
@@ -124,14 +116,11 @@ __device__ inline void store_vec(const S (&e)[16 / sizeof(S)], S *__restrict__ d
 // flight and no entry has to look for its list.  (Entries numbered through and dealt to threads one by one, each
 // bisecting for its list and waiting for its own load: 182 us for 28.7 M entries of sixteen lists into 62 M bf16
 // elements, now 80.)
-// The host is told (if it asks: answer.host) by the tile that is the last to have looked at its entries: what is left
-// then are stores.  FEW: the
-// tile finds its stretches itself, two waves for both ends (a launch less, a chain of probes more).
+// FEW: the tile finds its stretches itself, two waves for both ends.
 template <typename I, typename S, bool FEW>
 __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int64_t ntiles,
                                                             const uint32_t *__restrict__ starts,
-                                                            uint32_t *__restrict__ counters, S *__restrict__ dense,
-                                                            int64_t dense_n, HostAnswer answer, int32_t *status) {
+                                                            S *__restrict__ dense, int64_t dense_n, int32_t *status) {
   // the tile in the tensor's own type or, where lists meet, as fp32 sums
   __shared__ __attribute__((aligned(16))) float acc[kDecTile];
   __shared__ uint32_t occ[kDecTile / 32];
@@ -144,26 +133,6 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
   const int64_t t = blockIdx.x;
   const int64_t first = t * (int64_t)kDecTile;
   __shared__ uint32_t s_ends[FEW ? 2 : 1][64];
-  // one thread, when the workgroup's flags are in the status word: counts the tile; true for the last of all
-  auto counted = [&]() {
-    if (FEW) return (uint32_t)atomicAdd(status, 1 << kDecFlags);
-    return atomicAdd(&counters[(t % kDecGroups) * kDecPad], 1u);
-  };
-  auto tell = [&](uint32_t before) {
-    if (FEW) {
-      if ((before >> kDecFlags) != (uint32_t)ntiles - 1u) return;
-      const int32_t flags = (int32_t)(before & ((1u << kDecFlags) - 1u));
-      __hip_atomic_store(status, flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      host_store(answer.host + 1, (int64_t)flags);
-    } else {
-      const uint32_t g = (uint32_t)(t % kDecGroups), groups = ntiles < kDecGroups ? (uint32_t)ntiles : (uint32_t)kDecGroups;
-      if (before != (uint32_t)((ntiles - g + kDecGroups - 1) / kDecGroups) - 1u) return;
-      if (atomicAdd(&counters[kDecGroups * kDecPad], 1u) != groups - 1u) return;
-      host_store(answer.host + 1, (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    }
-    wait_global_acks();
-    host_store(answer.host, answer.ticket);
-  };
   uint32_t a = 0, b = 0;  // asked for first: the answer is on its way while the tile is cleared
   if (FEW) {
     if (wave < 2 && lane < lists.n)
@@ -229,11 +198,7 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
   if (wrong) s_wrong = 1;
   __syncthreads();
   if (s_wrong) {
-    if (tid == 0) {
-      atomicOr(status, ZEN_STAT_RETRY);
-      wait_global_acks();
-      if (answer.host) tell(counted());
-    }
+    if (tid == 0) atomicOr(status, ZEN_STAT_RETRY);
     return;  // the caller repeats the whole call: what this tile holds does not matter
   }
   {  // as many different elements as entries?
@@ -242,16 +207,13 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
   }
   __syncthreads();
   const bool aligned = (reinterpret_cast<uintptr_t>(dense + first) & 15u) == 0;
-  uint32_t before = 0;
   if (s_count == total) {
-    if (answer.host && tid == 0) before = counted();  // (on its way while the tile is written)
     for (int j = tid * V; j < kDecTile; j += kDecBlock * V) {
       S e[V];
       const uint4 q = *reinterpret_cast<const uint4 *>(tile + j);
       __builtin_memcpy(e, &q, 16);
       store_vec<S>(e, dense, first + j, dense_n, aligned);
     }
-    if (answer.host && tid == 0) tell(before);
     return;
   }
   // Two lists share an index here: fp32 sums, the lists one after the other (inside a list every index occurs
@@ -293,36 +255,26 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
       }
     }
   }
-  if (answer.host && tid == 0) before = counted();
   for (int j = tid * V; j < kDecTile; j += kDecBlock * V) {
     S e[V];
 #pragma unroll
     for (int q = 0; q < V; ++q) e[q] = rounded(acc[j + q], S(0));
     store_vec<S>(e, dense, first + j, dense_n, aligned);
   }
-  if (answer.host && tid == 0) tell(before);
 }
 
 template <typename I, typename S>
-int decode_sorted_launch(const DecLists &lists, void *dense, int64_t dense_n, uint32_t *workspace, int32_t *status,
-                         hipStream_t s, const HostAnswer &answer) {
+int decode_sorted_launch(const DecLists &lists, void *dense, int64_t dense_n, uint32_t *starts, int32_t *status,
+                         hipStream_t s) {
   const int64_t ntiles = ceil_div(dense_n, (int64_t)kDecTile);
   S *out = static_cast<S *>(dense);
   if (ntiles <= kDecFew) {
-    k_decode_tiles<I, S, true><<<dim3((unsigned)ntiles), dim3(kDecBlock), 0, s>>>(lists, ntiles, nullptr, nullptr, out,
-                                                                                 dense_n, answer, status);
+    k_decode_tiles<I, S, true><<<dim3((unsigned)ntiles), dim3(kDecBlock), 0, s>>>(lists, ntiles, nullptr, out, dense_n, status);
   } else {
-    const bool told = ntiles <= kDecTold;
-    uint32_t *counters = workspace, *starts = workspace + kDecCounters;
     k_decode_starts<I><<<dim3((unsigned)ceil_div(ntiles + 1, (int64_t)256), (unsigned)lists.n), dim3(256), 0, s>>>(
-        lists, ntiles, dense_n, starts, counters);
+        lists, ntiles, dense_n, starts);
     ZEN_LAUNCH_CHECK("k_decode_starts");
-    k_decode_tiles<I, S, false><<<dim3((unsigned)ntiles), dim3(kDecBlock), 0, s>>>(lists, ntiles, starts, counters, out,
-                                                                                  dense_n, told ? answer : HostAnswer{}, status);
-    if (answer.host && !told) {
-      ZEN_LAUNCH_CHECK("k_decode_tiles");
-      return host_answer_launch(answer, nullptr, 0, status, 1, s);
-    }
+    k_decode_tiles<I, S, false><<<dim3((unsigned)ntiles), dim3(kDecBlock), 0, s>>>(lists, ntiles, starts, out, dense_n, status);
   }
   ZEN_LAUNCH_CHECK("k_decode_tiles");
   return ZEN_OK;
@@ -336,12 +288,12 @@ extern "C" {
 size_t zen_decode_dense_sorted_workspace(int64_t dense_n, int nlists) {
   if (dense_n <= 0 || nlists <= 0) return 256;
   const int64_t ntiles = zen::ceil_div(dense_n, (int64_t)zen::kDecTile);
-  return ((size_t)((ntiles + 1) * nlists) + zen::kDecCounters) * sizeof(uint32_t) + 256;
+  return (size_t)((ntiles + 1) * nlists) * sizeof(uint32_t) + 256;
 }
 
-static int decode_lists_call(const void *const *idx, int idx64_in, const void *const *val, int dtype, const int64_t *len,
-                             int nlists, void *dense, int64_t dense_n, void *workspace, size_t workspace_bytes,
-                             int32_t *status, void *stream, const zen::HostAnswer &answer) {
+int zen_decode_dense_lists(const void *const *idx, int idx64_in, const void *const *val, int dtype, const int64_t *len,
+                           int nlists, void *dense, int64_t dense_n, void *workspace, size_t workspace_bytes,
+                           int32_t *status, void *stream) {
   using namespace zen;
   if (dtype != ZEN_F32 && dtype != ZEN_BF16) return fail(ZEN_EINVAL, "zen_decode_dense_lists: bad dtype");
   if (!dense || !status || !idx || !val || !len || !workspace)
@@ -361,18 +313,12 @@ static int decode_lists_call(const void *const *idx, int idx64_in, const void *c
   if (workspace_bytes < zen_decode_dense_sorted_workspace(dense_n, nlists))
     return fail(ZEN_EWORKSPACE, "zen_decode_dense_lists: workspace too small");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  uint32_t *ws = static_cast<uint32_t *>(workspace);
+  uint32_t *starts = static_cast<uint32_t *>(workspace);
   if (dtype == ZEN_BF16)
-    return idx64_in ? decode_sorted_launch<int64_t, uint16_t>(lists, dense, dense_n, ws, status, s, answer)
-                    : decode_sorted_launch<int32_t, uint16_t>(lists, dense, dense_n, ws, status, s, answer);
-  return idx64_in ? decode_sorted_launch<int64_t, uint32_t>(lists, dense, dense_n, ws, status, s, answer)
-                  : decode_sorted_launch<int32_t, uint32_t>(lists, dense, dense_n, ws, status, s, answer);
-}
-
-int zen_decode_dense_lists(const void *const *idx, int idx64_in, const void *const *val, int dtype, const int64_t *len,
-                           int nlists, void *dense, int64_t dense_n, void *workspace, size_t workspace_bytes,
-                           int32_t *status, void *stream) {
-  return decode_lists_call(idx, idx64_in, val, dtype, len, nlists, dense, dense_n, workspace, workspace_bytes, status, stream, {});
+    return idx64_in ? decode_sorted_launch<int64_t, uint16_t>(lists, dense, dense_n, starts, status, s)
+                    : decode_sorted_launch<int32_t, uint16_t>(lists, dense, dense_n, starts, status, s);
+  return idx64_in ? decode_sorted_launch<int64_t, uint32_t>(lists, dense, dense_n, starts, status, s)
+                  : decode_sorted_launch<int32_t, uint32_t>(lists, dense, dense_n, starts, status, s);
 }
 
 int zen_decode_dense_lists_status(const void *const *idx, int idx64_in, const void *const *val, int dtype, const int64_t *len,
@@ -382,8 +328,10 @@ int zen_decode_dense_lists_status(const void *const *idx, int idx64_in, const vo
   HostAnswer answer;
   int rc = host_ask(host, words, 1, &answer);
   if (rc != ZEN_OK) return rc;
-  rc = decode_lists_call(idx, idx64_in, val, dtype, len, nlists, dense, dense_n, workspace, workspace_bytes, status, stream, answer);
-  return host_finish(rc, answer, static_cast<hipStream_t>(stream));
+  rc = zen_decode_dense_lists(idx, idx64_in, val, dtype, len, nlists, dense, dense_n, workspace, workspace_bytes, status, stream);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (rc == ZEN_OK) rc = host_answer_launch(answer, nullptr, 0, status, 1, s);
+  return host_finish(rc, answer, s);
 }
 
 int zen_decode_dense_sorted(const void *idx, int idx64_in, const void *val, int dtype, const int64_t *list_start,
