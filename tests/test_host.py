@@ -570,6 +570,33 @@ def test_a_decode_is_done_when_its_status_is_known(deviceless, what, tiles):
     assert rc == 0 and tiles in log[-2] and "k_read_back" in log[-1]
 
 
+def test_other_threads_run_while_a_call_allocates():
+    """The native side lets go of the interpreter while it makes a call's tensors (long zeros here), as
+    torch's own functions do: another thread goes on meanwhile."""
+    import threading
+    import time
+
+    from zen_repro_amd import _lib
+
+    memory, began, ended, seen = torch.zeros(8, dtype=torch.int32), [], [], []
+    done = threading.Event()
+
+    def watch():
+        while not done.is_set():
+            seen.append(time.perf_counter())
+            time.sleep(1e-4)
+
+    parts = 1 << 25  # 0.8 GB of words
+    other = threading.Thread(target=watch)
+    other.start()
+    began.append(time.perf_counter())
+    _lib.host.table_find(lambda *a: ended.append(time.perf_counter()) or 0, _lib.host.Zeros(), memory, parts, 8, 16, 0, 0, 0)
+    done.set()
+    other.join()
+    inside = [began[0]] + [t for t in seen if began[0] < t < ended[0]] + [ended[0]]
+    assert max(b - a for a, b in zip(inside, inside[1:])) < 0.5 * (ended[0] - began[0])
+
+
 def test_every_call_gets_zeroed_words_of_its_own():
     """Status words and split sizes are cut from blocks: none is handed out twice, also where a block ends, where a
     piece is longer than a block, and where a stream starts afresh."""

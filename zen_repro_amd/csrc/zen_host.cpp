@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <map>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -24,6 +25,18 @@ int64_t address(const Tensor &t) { return reinterpret_cast<int64_t>(t.data_ptr()
 Tensor room(const Tensor &like, int64_t count, at::ScalarType type) {
   return at::empty({count}, like.options().dtype(type).requires_grad(false));
 }
+
+// What `make` returns, a call's new tensors, while other threads may hold the interpreter: an allocator that has to go to
+// the device, or free memory first, takes its time (torch's own bindings let go of it too).
+template <typename Make>
+auto made(Make make) {
+  py::gil_scoped_release others;
+  return make();
+}
+using Two = std::tuple<Tensor, Tensor>;  // (in braces: made in this order)
+using Three = std::tuple<Tensor, Tensor, Tensor>;
+using Four = std::tuple<Tensor, Tensor, Tensor, Tensor>;
+using Five = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor>;
 
 // Zeroed words for status words, counters and split sizes, cut from blocks that one fill zeroed.  Every piece is handed
 // out once, in the order of the stream its block was made on.  One object to a host thread.
@@ -121,8 +134,10 @@ py::tuple cut(const Tensor &indices, const Tensor &values, const std::vector<int
 py::tuple load_balance(const py::object &fn, Zeros &zeros, const Tensor &flat, int code, int64_t m, int64_t partitions,
                        int rehash, const py::object &thr, int64_t k, const py::object &thr_out, int64_t capacity,
                        int64_t table, int64_t mode, const Tensor &ws, int64_t stream, int64_t host, int64_t words) {
-  const Tensor idx = room(flat, capacity, at::kInt), val = room(flat, capacity, flat.scalar_type());
-  const Tensor splits = zeros.words(flat, stream, partitions), status = zeros.status(flat, stream);
+  const auto [idx, val, splits, status] = made([&] {
+    return Four{room(flat, capacity, at::kInt), room(flat, capacity, flat.scalar_type()), zeros.words(flat, stream, partitions),
+                zeros.status(flat, stream)};
+  });
   const py::object rc =
       host ? fn(address(flat), code, flat.numel(), m, partitions, rehash, thr, k, thr_out, address(idx), address(val),
                 capacity, address(splits), table, mode, address(ws), ws.numel(), address(status), host, words, stream)
@@ -134,9 +149,10 @@ py::tuple load_balance(const py::object &fn, Zeros &zeros, const Tensor &flat, i
 py::tuple merge(const py::object &fn, Zeros &zeros, const Tensor &indices, const Tensor &values, int code, int64_t dense_size,
                 int64_t capacity, bool idx64, bool rounded, int64_t mode, const Tensor &ws, int64_t stream, int64_t host,
                 int64_t words) {
-  const Tensor idx = room(values, capacity, idx64 ? at::kLong : at::kInt);
-  const Tensor val = room(values, capacity, rounded ? values.scalar_type() : at::kFloat);
-  const Tensor count = zeros.words(values, stream, 1), status = zeros.status(values, stream);
+  const auto [idx, val, count, status] = made([&] {
+    return Four{room(values, capacity, idx64 ? at::kLong : at::kInt), room(values, capacity, rounded ? values.scalar_type() : at::kFloat),
+                zeros.words(values, stream, 1), zeros.status(values, stream)};
+  });
   const int from64 = indices.scalar_type() == at::kLong;
   const py::object rc =
       host ? fn(address(indices), from64, address(values), code, indices.numel(), dense_size, address(idx), idx64 ? 1 : 0,
@@ -148,8 +164,10 @@ py::tuple merge(const py::object &fn, Zeros &zeros, const Tensor &indices, const
 
 py::tuple select_count(const py::object &fn, Zeros &zeros, const Tensor &flat, int code, const py::object &thr, bool idx64,
                  int64_t capacity, const Tensor &ws, int64_t stream, int64_t host, int64_t words) {
-  const Tensor idx = room(flat, capacity, idx64 ? at::kLong : at::kInt), val = room(flat, capacity, flat.scalar_type());
-  const Tensor count = zeros.words(flat, stream, 1), status = zeros.status(flat, stream);
+  const auto [idx, val, count, status] = made([&] {
+    return Four{room(flat, capacity, idx64 ? at::kLong : at::kInt), room(flat, capacity, flat.scalar_type()),
+                zeros.words(flat, stream, 1), zeros.status(flat, stream)};
+  });
   const py::object rc = fn(address(flat), code, flat.numel(), thr, address(idx), idx64 ? 1 : 0, address(val), capacity,
                            address(count), address(ws), ws.numel(), address(status), host, words, stream);
   return py::make_tuple(rc, idx, val);
@@ -157,7 +175,7 @@ py::tuple select_count(const py::object &fn, Zeros &zeros, const Tensor &flat, i
 
 py::tuple sample_threshold(const py::object &fn, Zeros &zeros, const Tensor &flat, int code, const Tensor &index, int64_t k,
                            const Tensor &ws, int64_t stream) {
-  const Tensor thr = room(flat, 2, at::kInt), status = zeros.status(flat, stream);
+  const auto [thr, status] = made([&] { return Two{room(flat, 2, at::kInt), zeros.status(flat, stream)}; });
   const py::object rc = fn(address(flat), code, flat.numel(), address(index), index.numel(), k, address(thr), address(ws),
                            ws.numel(), address(status), stream);
   return py::make_tuple(rc, thr, status);
@@ -165,7 +183,7 @@ py::tuple sample_threshold(const py::object &fn, Zeros &zeros, const Tensor &fla
 
 py::tuple decode(const py::object &fn, Zeros &zeros, const Tensor &indices, const Tensor &values, int code, const Tensor &dense,
                  int64_t mode, const Tensor &ws, int64_t stream, int64_t host, int64_t words) {
-  const Tensor status = zeros.status(values, stream);
+  const Tensor status = made([&] { return zeros.status(values, stream); });
   const py::object rc = fn(address(indices), indices.scalar_type() == at::kLong ? 1 : 0, address(values), code,
                            indices.numel(), address(dense), dense.numel(), mode, address(ws), ws.numel(), address(status),
                            host, words, stream);
@@ -183,7 +201,8 @@ bool matching_runs(const std::vector<Tensor> &indices, const std::vector<Tensor>
 py::tuple decode_lists(const py::object &fn, Zeros &zeros, const std::vector<Tensor> &indices,
                        const std::vector<Tensor> &values, int code, int64_t dense_size, const Tensor &ws, int64_t stream,
                        int64_t host, int64_t words) {
-  const Tensor dense = room(values[0], dense_size, values[0].scalar_type()), status = zeros.status(values[0], stream);
+  const auto [dense, status] =
+      made([&] { return Two{room(values[0], dense_size, values[0].scalar_type()), zeros.status(values[0], stream)}; });
   const Lists i(indices), v(values);
   const py::object rc = fn(i.addresses(), indices[0].scalar_type() == at::kLong ? 1 : 0, v.addresses(), code, i.counts(),
                            indices.size(), address(dense), dense_size, address(ws), ws.numel(), address(status), host, words,
@@ -194,7 +213,8 @@ py::tuple decode_lists(const py::object &fn, Zeros &zeros, const std::vector<Ten
 py::tuple bitmaps_dense(const py::object &fn, Zeros &zeros, const std::vector<Tensor> &bitmaps,
                         const std::vector<Tensor> &values, int code, const Tensor &dict, int64_t numel, const Tensor &ws,
                         int64_t stream, int64_t host, int64_t words) {
-  const Tensor dense = room(values[0], numel, values[0].scalar_type()), status = zeros.status(values[0], stream);
+  const auto [dense, status] =
+      made([&] { return Two{room(values[0], numel, values[0].scalar_type()), zeros.status(values[0], stream)}; });
   const Lists b(bitmaps), v(values);
   const py::object rc = fn(address(dict), numel, bitmaps.size(), b.addresses(), b.counts(), v.addresses(), code, v.counts(),
                            address(dense), address(ws), ws.numel(), address(status), host, words, stream);
@@ -203,7 +223,8 @@ py::tuple bitmaps_dense(const py::object &fn, Zeros &zeros, const std::vector<Te
 
 py::tuple bitmap_encode(const py::object &fn, Zeros &zeros, const Tensor &mapping, const Tensor &indices, const Tensor &ranks,
                         int64_t numel, int64_t count, int64_t stream, int64_t host, int64_t words) {
-  const Tensor bitmap = room(indices, std::max<int64_t>(count, 1) * 4, at::kByte), status = zeros.status(indices, stream);
+  const auto [bitmap, status] =
+      made([&] { return Two{room(indices, std::max<int64_t>(count, 1) * 4, at::kByte), zeros.status(indices, stream)}; });
   const py::object rc = fn(address(mapping), mapping.numel(), address(indices), indices.scalar_type() == at::kLong ? 1 : 0,
                            indices.numel(), py::none(), address(ranks), numel, address(bitmap), address(status), host, words,
                            stream);
@@ -212,8 +233,9 @@ py::tuple bitmap_encode(const py::object &fn, Zeros &zeros, const Tensor &mappin
 
 py::tuple tables(const py::object &fn, Zeros &zeros, const Tensor &input, int code, int64_t m, int64_t serial_n,
                  int64_t partitions, int rehash, int64_t stream, int64_t host, int64_t words) {
-  const Tensor memory = room(input, m, at::kInt), serial = room(input, serial_n, at::kInt);
-  const Tensor offsets = room(input, partitions, at::kInt), status = zeros.status(input, stream);
+  const auto [memory, serial, offsets, status] = made([&] {
+    return Four{room(input, m, at::kInt), room(input, serial_n, at::kInt), room(input, partitions, at::kInt), zeros.status(input, stream)};
+  });
   const py::object rc = fn(address(input), code, input.numel(), address(memory), m, address(serial), serial_n,
                            address(offsets), partitions, rehash, address(status), host, words, stream);
   return py::make_tuple(rc, memory, serial, offsets, status);
@@ -223,8 +245,10 @@ py::tuple table_find(const py::object &fn, Zeros &zeros, const Tensor &memory, i
                      int64_t stream, int64_t host, int64_t words) {
   // beside the split sizes, the words in which the walk adds them up; no workspace that is kept from call to call: the
   // thread may walk another table before these lists are used up
-  const Tensor all = zeros.words(memory, stream, 3 * partitions + 66), splits = all.narrow(0, 0, partitions);
-  const Tensor status = zeros.status(memory, stream), ws = room(memory, ws_bytes, at::kByte);
+  const auto [all, status, ws] = made([&] {
+    return Three{zeros.words(memory, stream, 3 * partitions + 66), zeros.status(memory, stream), room(memory, ws_bytes, at::kByte)};
+  });
+  const Tensor splits = all.narrow(0, 0, partitions);
   const py::object rc =
       host ? fn(address(memory), memory.numel(), partitions, n, address(splits), address(all) + 8 * partitions, address(ws),
                 ws_bytes, address(status), host, words, stream)
@@ -236,7 +260,7 @@ py::tuple table_gather(const py::object &fn, const Tensor &memory, const Tensor 
                        const std::vector<int64_t> &sizes, const Tensor &ws, int64_t stream) {
   int64_t total = 0;
   for (int64_t s : sizes) total += s;
-  const Tensor idx = room(flat, total, at::kInt), val = room(flat, total, flat.scalar_type());
+  const auto [idx, val] = made([&] { return Two{room(flat, total, at::kInt), room(flat, total, flat.scalar_type())}; });
   const py::object rc = fn(address(memory), memory.numel(), sizes.size(), address(flat), code, flat.numel(), address(idx),
                            address(val), total, address(ws), ws.numel(), stream);
   return py::make_tuple(rc, at::split_with_sizes(idx, sizes), at::split_with_sizes(val, sizes));
@@ -249,12 +273,14 @@ py::tuple step_buffers(int64_t args, Zeros &zeros, const Tensor &flat, const Ten
                        const Tensor &merge_ws) {
   zen_encode_merge_args *a = reinterpret_cast<zen_encode_merge_args *>(args);
   const int64_t r = indices.numel();
-  const Tensor idx = room(flat, capacity, at::kInt), val = room(flat, capacity, flat.scalar_type());
-  const Tensor m_idx = room(flat, r, at::kInt), m_val = room(flat, r, at::kFloat);
   bool wait = false;
-  // split sizes, merged count, the two status words
-  const Tensor small = merge_stream ? zeros.words_for(flat, stream, partitions + 2, merge_stream, &wait)
-                                    : zeros.words(flat, stream, partitions + 2);
+  // small: split sizes, merged count, the two status words
+  const auto [idx, val, m_idx, m_val, small] = made([&] {
+    return Five{room(flat, capacity, at::kInt), room(flat, capacity, flat.scalar_type()), room(flat, r, at::kInt),
+                room(flat, r, at::kFloat),
+                merge_stream ? zeros.words_for(flat, stream, partitions + 2, merge_stream, &wait)
+                             : zeros.words(flat, stream, partitions + 2)};
+  });
   const Tensor splits = small.narrow(0, 0, partitions), count = small.narrow(0, partitions, 1);
   const Tensor both = small.narrow(0, partitions + 1, 1).view(at::kInt);
   const Tensor status = both.narrow(0, 0, 1), m_status = both.narrow(0, 1, 1);
