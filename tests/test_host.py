@@ -137,6 +137,22 @@ def test_missing_library_fails_loudly(monkeypatch):
         _lib.lib()
 
 
+def test_missing_native_host_side_fails_loudly():
+    """Whatever is called first says what is to be built, also where the library itself has not been asked for."""
+    code = ("import sys; sys.modules['zen_repro_amd._host'] = None\n"
+            "import torch, zen_repro_amd as zen\n"
+            "from zen_repro_amd import _lib\n"
+            "lba = zen.LoadBalanceAllreduce.__new__(zen.LoadBalanceAllreduce)\n"
+            "for call in (lambda: lba.stack_tensors([torch.zeros(2), torch.zeros(3)]), _lib.lib, _lib.zeros.native):\n"
+            "    try:\n"
+            "        call()\n"
+            "    except RuntimeError as e:\n"
+            "        assert 'make -C zen_repro_amd/csrc' in str(e) and 'no fallback' in str(e)\n"
+            "        print('told')\n")
+    out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert out.stdout.split() == ["told"] * 3, out.stderr
+
+
 def test_table_sizes_follow_the_reference(oracle):
     from zen_repro_amd.tensor_load_balance import TensorPartition
 

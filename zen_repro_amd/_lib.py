@@ -9,10 +9,22 @@ import threading
 
 import torch  # first: makes the process use torch's HIP runtime for libzen_hip too
 
+
+class _Unbuilt:
+    """Stands for zen_host.cpp's module where that does not load: whoever comes to use it is told."""
+
+    def __init__(self, why):
+        self._why = why
+
+    def __getattr__(self, name):
+        raise RuntimeError("zen_repro_amd/_host.so does not load: build it with `make -C zen_repro_amd/csrc` "
+                           f"(or __graft_entry__.build()); there is no fallback path ({self._why})")
+
+
 try:
     from . import _host as host  # zen_host.cpp: what the calls do around the library's functions
-except ImportError as e:  # not built, or for another torch: lib() says so
-    host, _host_error = None, e
+except ImportError as e:  # not built, or for another torch
+    host = _Unbuilt(str(e))
 
 F32, BF16 = 0, 1
 OK, EINVAL, EHIP, EWORKSPACE = 0, -1, -2, -3
@@ -71,9 +83,8 @@ def lib():
         raise RuntimeError(
             f"{LIB_PATH} is missing: build it with `make -C zen_repro_amd/csrc` "
             "(or __graft_entry__.build()); there is no fallback path")
-    if host is None or host.ABI_VERSION != ABI_VERSION:
-        raise RuntimeError(f"zen_repro_amd/_host.so does not load or is of another version: build it with `make -C "
-                           f"zen_repro_amd/csrc` ({_host_error if host is None else host.ABI_VERSION})")
+    if host.ABI_VERSION != ABI_VERSION:
+        raise RuntimeError("zen_repro_amd/_host.so is of another version: build it with `make -C zen_repro_amd/csrc`")
     L = ctypes.CDLL(LIB_PATH)
     vp, i32, i64, sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_size_t
     sig = {
