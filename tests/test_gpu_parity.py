@@ -1161,6 +1161,53 @@ def test_merge_in_one_workgroup(zen, oracle, n, r, dtype):
                 lba.decode_sparse_tensors(torch.where(d_idx == d_idx[0], n, d_idx), d_val, n)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("r", [64, 65, 1025, 2048, 4097, 6143, 6144])
+@pytest.mark.parametrize("kind", ["narrow", "run", "eight of each", "half narrow", "half on one"])
+def test_merge_in_one_workgroup_of_indices_that_pile_up(zen, oracle, kind, r, dtype):
+    """Lists whose indices lie in few of the ranges they are sorted by, some outside the tensor among them: sums, order and
+    flags as ever, and a time that does not go with the square of the length (it was fifty times that of a spread list;
+    the sum of many values of one index is a chain of its own)."""
+    from zen_repro_amd import _lib
+
+    n = 1 << 30
+    gen = torch.Generator().manual_seed(r)
+    idx = {"narrow": lambda: torch.randint(0, 1 << 18, (r,), generator=gen),
+           "run": lambda: torch.randperm(r, generator=gen),
+           "eight of each": lambda: torch.randint(0, max(1, r // 8), (r,), generator=gen),
+           "half narrow": lambda: torch.where(torch.arange(r) % 2 == 0, torch.randint(0, n // 4, (r,), generator=gen),
+                                              torch.randint(0, 1 << 18, (r,), generator=gen)),
+           "half on one": lambda: torch.where(torch.arange(r) % 2 == 0, torch.randint(0, n // 4, (r,), generator=gen), 7)}[kind]()
+    idx = idx + n // 2
+    spread = torch.randint(0, n, (r,), generator=gen).cuda()
+    val = (torch.randn(r, generator=gen) * 1e-3).to(dtype)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    d_val = val.cuda()
+    for bad in (0, 3):
+        idx[torch.randperm(r, generator=gen)[:bad]] = torch.tensor([-1, n, 1 << 40])[:bad]
+        good = ((idx >= 0) & (idx < n)).numpy()
+        which, place = np.unique(idx.numpy()[good], return_inverse=True)
+        w_idx, w_val = oracle.merge_sparse(place, to_np(val)[good], len(which))
+        m_idx, m_val, count, status = lba.merge_sparse_flat(idx.cuda(), d_val, n)
+        assert status.item() == (_lib.STAT_BAD_INDEX if bad else 0) and count.item() == len(w_idx)
+        assert np.array_equal(to_np(m_idx)[:len(w_idx)], which[w_idx])
+        assert np.array_equal(to_np(m_val)[:len(w_idx)].view(np.uint32), w_val.view(np.uint32))
+    d_idx = idx.cuda()
+
+    def quickest(i):
+        times = []
+        for _ in range(20):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            lba.merge_sparse_flat(i, d_val, n)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+
+    assert kind == "half on one" or quickest(d_idx) < 10 * quickest(spread)
+
+
 @pytest.mark.parametrize("words", [1, 1023, 1024, (1 << 16) - 1, 1 << 16, (1 << 19) + 1])
 def test_read_back_of_any_length(zen, words):
     """Both types, a word and a list of `words` of them, up to and past what goes through the pinned buffer."""

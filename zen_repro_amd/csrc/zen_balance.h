@@ -8,38 +8,6 @@ namespace zen {
 
 constexpr uint32_t kSerialLds = 8192;  // serial tails up to this size are sorted in LDS
 
-// Ascending compare-exchange network (bitonic with mirrored first step), valid
-// for any n: positions >= n act as +infinity and never move.
-__device__ inline void sort_network(uint32_t *a, uint32_t n) {
-  uint32_t n2 = 1;
-  while (n2 < n) n2 <<= 1;
-  const uint32_t half = n2 >> 1;
-  for (uint32_t k = 2; k <= n2; k <<= 1) {
-    const uint32_t hk = k >> 1;
-    for (uint32_t q = threadIdx.x; q < half; q += blockDim.x) {
-      const uint32_t blk = q / hk, r = q % hk;
-      const uint32_t i = blk * k + r, l = blk * k + (k - 1 - r);
-      if (l < n) {
-        const uint32_t x = a[i], y = a[l];
-        if (x > y) { a[i] = y; a[l] = x; }
-      }
-    }
-    __syncthreads();
-    for (uint32_t j = hk >> 1; j > 0; j >>= 1) {
-      for (uint32_t q = threadIdx.x; q < half; q += blockDim.x) {
-        const uint32_t i = (q / j) * 2 * j + (q % j), l = i + j;
-        if (l < n) {
-          const uint32_t x = a[i], y = a[l];
-          if (x > y) { a[i] = y; a[l] = x; }
-        }
-      }
-      __syncthreads();
-    }
-  }
-}
-
-
-
 __device__ inline uint32_t lower_bound_u32(const uint32_t *a, uint32_t n, uint32_t x) {
   uint32_t lo = 0, hi = n;
   while (lo < hi) {

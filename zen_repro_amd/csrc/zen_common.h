@@ -194,6 +194,37 @@ __device__ inline bool done_last(uint32_t *words, uint32_t index, uint32_t total
   return atomicAdd(&words[kDoneGroups * kDonePad], 1u) == groups - 1u;
 }
 
+// Ascending compare-exchange network (bitonic with mirrored first step), valid for any n: positions >= n act as
+// +infinity and never move.  By the whole workgroup.
+template <typename T>
+__device__ inline void sort_network(T *a, uint32_t n) {
+  uint32_t steps = 0;
+  while ((1u << steps) < n) ++steps;
+  const uint32_t half = (1u << steps) >> 1;
+  auto exchange = [&](uint32_t i, uint32_t l) {
+    if (l >= n) return;
+    const T x = a[i], y = a[l];
+    if (x > y) {
+      a[i] = y;
+      a[l] = x;
+    }
+  };
+  for (uint32_t k = 0; k < steps; ++k) {  // sorted runs of 2^k become runs of 2^(k + 1)
+    for (uint32_t q = threadIdx.x; q < half; q += blockDim.x) {
+      const uint32_t first = q >> k << (k + 1), r = q & ((1u << k) - 1u);
+      exchange(first + r, first + (2u << k) - 1u - r);
+    }
+    __syncthreads();
+    for (uint32_t j = k; j-- > 0;) {
+      for (uint32_t q = threadIdx.x; q < half; q += blockDim.x) {
+        const uint32_t i = (q >> j << (j + 1)) + (q & ((1u << j) - 1u));
+        exchange(i, i + (1u << j));
+      }
+      __syncthreads();
+    }
+  }
+}
+
 // Where the host waits for what a call has to know there (zen_readback.hip): pinned words, of which word 0 takes the
 // ticket once the others hold the answer.  The kernel that knows the answer stores it, where that is one of the call's
 // own: no launch for it, and what is left of the call's work runs while the host goes on.

@@ -230,8 +230,8 @@ __device__ inline uint32_t sum_runs(const Shared &sh, uint32_t n, uint32_t (&k)[
     const uint32_t before_k = first > 0 && first < n ? sh.key[first - 1] : kNoKey;
     const uint32_t after_k = first + per < n ? sh.key[first + per] : kNoKey;
     float acc = 0.0f;
-    if (first < n && before_k == k[0]) {
-      // the run began before this thread's places: find its head, sum up to the place in front of `first`
+    if (first < n && before_k == k[0] && after_k != before_k) {
+      // the run began before this thread's places and ends here: find its head, sum up to the place in front of `first`
       uint32_t head = first - 1;
       while (head > 0) {
         const uint32_t a0 = sh.key[head - 1];
@@ -407,20 +407,32 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
   }
 }
 
-// A short list in one workgroup, straight from where it lies: no slabs, no zeroed memory, any indices (a narrow range takes
-// whatever comes).  DENSE: out_val is the dense tensor, written whole.  Bound by the chain of its phases, LDS round trips
-// and three trips to memory: a rounded merge of 1000 entries 27 us a call (38 on the tables of the wide buckets, which are
-// laid out for 16 384).
+// A short list in one workgroup, straight from where it lies: no slabs, no zeroed memory, any indices.  DENSE: out_val is
+// the dense tensor, written whole.  Bound by the chain of its phases, LDS round trips and three trips to memory: a rounded
+// merge of 1000 entries spread over the range 27 us a call (38 on the tables of the wide buckets, which are laid out for
+// 16 384).  Indices that pile up in few of the narrow ranges would be compared pair by pair, some 8000 pairs a microsecond:
+// beyond kMergeOnePairs for every entry a compare-exchange network sorts them, which takes about as long as that many
+// (6144 entries in a 4096th of a range of 2^30, a call: 2020 us and now 99; 1000 of them 73 and 42).
+constexpr uint32_t kMergeOnePairs = 64;
 struct MergeOneShared : SlabSortShared {
-  static constexpr uint32_t kLimit = kSlabCap;
+  static constexpr bool kPairs = true;
+  uint32_t pairs, pairs_most;
 };
+static_assert(offsetof(SlabSortShared, scan) >= kSlabCap * sizeof(uint64_t), "an index and an arrival number for every entry");
+constexpr int kMergeOneArrBits = 13;
+static_assert(kSlabCap <= (1 << kMergeOneArrBits), "an arrival number");
 
 template <typename I, typename S, typename O, bool DENSE>
 __global__ __launch_bounds__(kMergeBlock) void k_merge_one(SlabGeom geo, const void *__restrict__ idx, int idx64,
                                                            const S *__restrict__ val, uint32_t r, uint32_t dense_n,
                                                            I *__restrict__ out_idx, O *__restrict__ out_val, int64_t capacity,
                                                            int tie_bits, int64_t *out_count, HostAnswer answer, int32_t *status) {
-  __shared__ MergeOneShared sh;
+  __shared__ union {
+    MergeOneShared sh;
+    uint64_t both[kSlabCap];  // in the place of the keys and ties
+  } s_all;
+  MergeOneShared &sh = s_all.sh;
+  if (threadIdx.x == 0) sh.pairs_most = kMergeOnePairs * r;
   uint32_t off[kMergeRecs], arr[kMergeRecs], rank[kMergeRecs];
   S v[kMergeRecs];
   uint32_t live = 0;
@@ -461,12 +473,33 @@ __global__ __launch_bounds__(kMergeBlock) void k_merge_one(SlabGeom geo, const v
     for (uint32_t i = head + vecs * V + threadIdx.x; i < dense_n; i += kMergeBlock) out_val[i] = O(0);
   }
   uint32_t n = 0;
-  (void)slab_rank<kMergeBlock>(sh, geo, tie_bits, off, arr, live, rank, &n);  // (never declined: no group is beyond the limit)
+  if (slab_rank<kMergeBlock>(sh, geo, tie_bits, off, arr, live, rank, &n)) {
 #pragma unroll
-  for (int i = 0; i < kMergeRecs; ++i) {
-    if (live & (1u << i)) {
-      sh.key[rank[i]] = off[i];
-      sh.tie[rank[i]] = __float_as_uint(KeyOf<S>::to_f32(v[i]));
+    for (int i = 0; i < kMergeRecs; ++i) {
+      if (live & (1u << i)) {
+        sh.key[rank[i]] = off[i];
+        sh.tie[rank[i]] = __float_as_uint(KeyOf<S>::to_f32(v[i]));
+      }
+    }
+  } else {
+    (void)block_exclusive_scan<uint32_t, kMergeBlock>((uint32_t)__popc(live), sh.scan, &n);
+#pragma unroll
+    for (int i = 0; i < kMergeRecs; ++i)
+      if (arr[i] < r) s_all.both[arr[i]] = live & (1u << i) ? ((uint64_t)off[i] << kMergeOneArrBits) | arr[i] : ~0ull;
+    __syncthreads();
+    sort_network(s_all.both, r);  // entries that are skipped come last
+    uint64_t e[kMergeRecs];
+#pragma unroll
+    for (int i = 0; i < kMergeRecs; ++i) e[i] = arr[i] < n ? s_all.both[arr[i]] : 0ull;
+#pragma unroll
+    for (int i = 0; i < kMergeRecs; ++i) v[i] = val[(uint32_t)e[i] & ((1u << kMergeOneArrBits) - 1u)];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kMergeRecs; ++i) {
+      if (arr[i] < n) {
+        sh.key[arr[i]] = (uint32_t)(e[i] >> kMergeOneArrBits);
+        sh.tie[arr[i]] = __float_as_uint(KeyOf<S>::to_f32(v[i]));
+      }
     }
   }
   __syncthreads();
@@ -509,8 +542,8 @@ __global__ __launch_bounds__(kMergeBlock) void k_merge_one(SlabGeom geo, const v
   }
 }
 
-// Entries up to which one workgroup does it all: as many as fit (6144 of them 28 to 36 us a dense call, in the wide
-// buckets' two launches 39).
+// Entries up to which one workgroup does it all: as many as fit (6144 of them spread over the range 28 to 36 us a dense
+// call, in the wide buckets' two launches 39).
 constexpr int64_t kMergeOneMax = merge_one_max();
 static_assert(kMergeOneMax <= kSlabCap, "the records fit");
 

@@ -156,10 +156,11 @@ __device__ inline uint32_t sub_place(uint32_t s) {
 // LDS decides how many workgroups share a compute unit.
 constexpr int kSlabQueueCap = kSlabCap - kSlabSubs - 1;  // large-group records a workgroup sets aside
 constexpr int kSlabInline = 4;                            // groups up to this size are ranked by their own threads
+constexpr int kSlabPairsFrom = 16;                        // groups up to this size are not counted as pairs
 constexpr int kSlabQueueMin = 256;                        // records in larger groups below which nothing is set aside
 struct SlabSortShared {
   static constexpr bool kQueue = true;
-  static constexpr uint32_t kLimit = kSlabGroupLimit;
+  static constexpr bool kPairs = false;
   uint32_t key[kSlabCap];
   union {
     uint32_t tie[kSlabCap];
@@ -176,7 +177,7 @@ static_assert(kSlabSubs + 1 <= kSlabCap, "the counters fit under the ties");
 // The same without the queue (whose code costs slab_rank registers).
 struct SlabSortSharedNoQueue {
   static constexpr bool kQueue = false;
-  static constexpr uint32_t kLimit = kSlabGroupLimit;
+  static constexpr bool kPairs = false;
   uint32_t key[kSlabCap];
   union {
     uint32_t tie[kSlabCap];
@@ -214,7 +215,8 @@ __device__ inline uint32_t slab_count_less(const Shared &sh, uint32_t b0, uint32
 // than kSlabInline are set aside instead (their places in the queue follow from the same prefix sums as the
 // groups' places: the counters carry both, 16 bits each) and handed out again afterwards, one per lane, so
 // that the lanes of a wave walk through large groups together.  Returns false (for every thread) if a
-// group is too large for that; else rank[i] for live records and *n_out = number of live records.  On return
+// group is too large for that (kSlabGroupLimit; with a Shared that counts pairs: if the records have more than
+// sh.pairs_most of others to be compared with, all of them together); else rank[i] for live records and *n_out = number of live records.  On return
 // sh.key / sh.tie may be overwritten at once (sh.tie is not touched at all), and the low 16 bits of
 // sh.cnt[sub_place(s)] hold the sorted place of the first record of narrow range s.
 template <int BLOCK, typename Shared>
@@ -226,7 +228,10 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
   constexpr int kItems = kSlabCap / BLOCK;
   constexpr int kSubsPer = kSlabSubs / BLOCK;
   for (int d = threadIdx.x; d <= kSlabSubs; d += BLOCK) sh.cnt[d] = 0;
-  if (threadIdx.x == 0) sh.bad = 0;
+  if (threadIdx.x == 0) {
+    sh.bad = 0;
+    if constexpr (Shared::kPairs) sh.pairs = 0;
+  }
   __syncthreads();
   const uint32_t low_mask = (1u << geo.sub_shift) - 1u;
   uint32_t sub[kItems], at[kItems];
@@ -241,14 +246,20 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
   __syncthreads();
   {
     uint32_t c[kSubsPer];
-    uint32_t sum = 0, big = 0;  // sum: records in the low half, records of groups larger than kSlabInline in the high half
+    uint32_t sum = 0, big = 0, pairs = 0;  // sum: records in the low half, records of groups larger than kSlabInline in the high half
 #pragma unroll
     for (int e = 0; e < kSubsPer; ++e) {
       c[e] = sh.cnt[e * BLOCK + threadIdx.x];
       sum += c[e] + (c[e] > (uint32_t)kSlabInline ? c[e] << 16 : 0u);
-      big |= c[e] > Shared::kLimit;
+      if constexpr (Shared::kPairs)
+        pairs += c[e] > (uint32_t)kSlabPairsFrom ? c[e] * c[e] : 0u;
+      else
+        big |= c[e] > (uint32_t)kSlabGroupLimit;
     }
     if (big) sh.bad = 1;
+    if constexpr (Shared::kPairs) {
+      if (pairs) atomicAdd(&sh.pairs, pairs);
+    }
     uint32_t total;
     uint32_t running = block_exclusive_scan<uint32_t, BLOCK>(sum, sh.scan, &total);
 #pragma unroll
@@ -260,6 +271,9 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
   }
   __syncthreads();
   if (sh.bad) return false;
+  if constexpr (Shared::kPairs) {
+    if (sh.pairs > sh.pairs_most) return false;
+  }
   const uint32_t totals = sh.cnt[kSlabSubs];
   // a few large groups are not worth the extra barrier
   const bool set_aside = Shared::kQueue && (totals >> 16) >= (uint32_t)kSlabQueueMin;
@@ -275,7 +289,7 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
       word[i] = ((off[i] & low_mask) << tie_bits) | tie[i];
       sh.key[g0[i] + at[i]] = word[i];
       if constexpr (Shared::kQueue) {
-        static_assert(kSlabSubs <= (1 << 12) && Shared::kLimit <= (1u << 19), "a queue entry is one word");
+        static_assert(kSlabSubs <= (1 << 12) && kSlabGroupLimit <= (1 << 19) && kSlabCap <= (1 << 19), "a queue entry is one word");
         const uint32_t q = (here >> 16) + at[i];
         if (set_aside && g1[i] - g0[i] > (uint32_t)kSlabInline && q < (uint32_t)kSlabQueueCap) {
           sh.queue[q] = sub[i] | (at[i] << 12);  // sub < 2^12, at < group size <= kSlabGroupLimit
