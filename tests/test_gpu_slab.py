@@ -298,8 +298,8 @@ def test_slab_load_balance_fused_topk_fp32(zen, oracle):
 
 def test_fused_topk_fp32_wherever_the_kth_key_lies_in_its_bin(zen, oracle, fast_path):
     """The fp32 threshold's last 16 bits for a k-th key at the top, the bottom and the middle of the threshold's
-    bin of 65536 keys, at even and odd keys and either side of a multiple of 128 (the refinement's last
-    workgroup gives a thread 128 keys and a lane of its first wave two of them)."""
+    bin of 65536 keys, at even and odd keys and either side of multiples of 128 and 256 (the refinement's last
+    workgroup finds the 256 keys that hold the rank, then the key among them)."""
     n, P = (1 << 20) if fast_path == "wide" else (1 << 24), 4
     rng = np.random.default_rng(5)
     x = (rng.standard_normal(n) * 0.2).astype(np.float32)
@@ -307,7 +307,7 @@ def test_fused_topk_fp32_wherever_the_kth_key_lies_in_its_bin(zen, oracle, fast_
     keys = x.view(np.uint32) & 0x7FFFFFFF
     x[(keys >> 16) == (base >> 16)] = 0.3  # nobody else in that bin
     x[0] = 0.25
-    lows = [65535, 65534, 65409, 65408, 65407, 32769, 32768, 129, 128, 127, 1, 0]
+    lows = [65535, 65534, 65409, 65408, 65407, 65280, 65279, 32769, 32768, 32767, 257, 256, 255, 129, 128, 127, 1, 0]
     at = rng.choice(np.arange(1, n), 3 * len(lows), replace=False)
     sign = np.where(rng.random(len(at)) < 0.5, 0x80000000, 0).astype(np.uint32)
     x.view(np.uint32)[at] = (np.repeat(np.array(lows, np.uint32), 3) + np.uint32(base)) | sign  # three of each
@@ -592,7 +592,7 @@ def test_table_and_merge_workspace_are_zero_again_after_every_call(zen, oracle):
 
 def test_load_balance_without_a_capacity_takes_the_slab_path(zen, oracle):
     """TensorPartition.load_balance(tensor) as the reference calls it (tensor_load_balance.py:43): the capacity
-    it works out for itself keeps a bucket-sized, sparse tensor on the bucket-slab path, and the result is the
+    it works out for itself keeps a bucket-sized, sparse tensor on the fast paths, and the result is the
     oracle's."""
     from zen_repro_amd import _lib
 

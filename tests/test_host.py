@@ -620,13 +620,14 @@ def test_every_call_gets_zeroed_words_of_its_own():
 
     zeros = _lib.host.Zeros()
     flat, ws = torch.zeros(8, dtype=torch.bfloat16), torch.zeros(16, dtype=torch.uint8)
-    held, words = [], []
+    held, words = [], []  # (pieces begin at 16 bytes, those of status words at 8)
     for call in range(3000):
         parts, stream = (9000, 5) if call == 1500 else (5, 5 + call % 2)
         rc, idx, val, splits, status = _lib.host.load_balance(
             lambda *a: len(a), zeros, flat, 1, 8, parts, 3, None, 0, None, 4, 0, 0, ws, stream, 0, 0)
         assert rc == 19 and idx.shape == val.shape == (4,) and splits.shape == (parts,) and status.shape == (1,)
         assert not splits.any() and not status.any()
+        assert splits.data_ptr() % 16 == 0 and status.data_ptr() % 8 == 0
         held += [splits, status]
         words += [(t.data_ptr(), t.data_ptr() + t.numel() * t.element_size()) for t in (splits, status)]
         splits.fill_(-1)

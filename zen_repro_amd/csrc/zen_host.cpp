@@ -43,7 +43,7 @@ using Five = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor>;
 class Zeros {
  public:
   static constexpr int64_t kWords = 8192;
-  static constexpr int64_t kSplit = 2;  // pieces begin at multiples of 16 bytes
+  static constexpr int64_t kSplit = 2;  // pieces begin at multiples of so many words: of 16 bytes, status words of 8
 
   Tensor words(const Tensor &like, int64_t stream, int64_t count) { return take(blocks_, like, stream, count, at::kLong, 0, nullptr); }
   Tensor status(const Tensor &like, int64_t stream) { return take(narrow_, like, stream, 1, at::kInt, 0, nullptr); }
