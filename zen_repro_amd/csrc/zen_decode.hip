@@ -222,9 +222,16 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
   for (int j = tid; j < kDecTile / 4; j += kDecBlock) reinterpret_cast<uint4 *>(acc)[j] = make_uint4(0, 0, 0, 0);
   __syncthreads();
   constexpr int kAhead = 8;
-  // (an entry of some list, for lists with nothing in the tile)
-  const int other = __ffsll((unsigned long long)__ballot(a < b)) - 1;
-  const uint32_t other_at = (uint32_t)__builtin_amdgcn_readlane((int)a, other);
+  // What lists with nothing in the tile read: the tiles' starts, or where there are none an entry of some list (which has to
+  // be found first: 250 M bf16 elements, four lists of 1 %, 241 us instead of 231; 89 M, eight of 5 %, 154 and 145).
+  const I *no_idx = reinterpret_cast<const I *>(starts);
+  const S *no_val = reinterpret_cast<const S *>(starts);
+  if (FEW) {
+    const int other = __ffsll((unsigned long long)__ballot(a < b)) - 1;
+    const uint32_t other_at = (uint32_t)__builtin_amdgcn_readlane((int)a, other);
+    no_idx = static_cast<const I *>(lists.idx[other]) + other_at;
+    no_val = static_cast<const S *>(lists.val[other]) + other_at;
+  }
   for (int l0 = 0; l0 < lists.n; l0 += kAhead) {
     // an entry of each list per thread, in no branch (a list with nothing for this thread reads some entry), so
     // that all are in flight together
@@ -236,8 +243,8 @@ __global__ __launch_bounds__(kDecBlock) void k_decode_tiles(DecLists lists, int6
       const uint32_t la = (uint32_t)__builtin_amdgcn_readlane((int)a, l);
       const uint32_t lb = (uint32_t)__builtin_amdgcn_readlane((int)b, l);
       const bool some = la < lb;
-      const I *idx = some ? static_cast<const I *>(lists.idx[l]) + la : static_cast<const I *>(lists.idx[other]) + other_at;
-      const S *val = some ? static_cast<const S *>(lists.val[l]) + la : static_cast<const S *>(lists.val[other]) + other_at;
+      const I *idx = some ? static_cast<const I *>(lists.idx[l]) + la : no_idx;
+      const S *val = some ? static_cast<const S *>(lists.val[l]) + la : no_val;
       const uint32_t e = la + (uint32_t)tid < lb ? (uint32_t)tid : 0u;
       k[i] = idx[e];
       v[i] = val[e];
