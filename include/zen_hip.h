@@ -54,8 +54,11 @@ extern "C" {
  * 8: zen_balance_tables, zen_decode_dense_lists_status,
  *    zen_bitmap_dense_lists_status, zen_bitmap_encode_status
  * 9: ZEN_MODE_WIDE
+ * 10: the dense dictionary of up to sixteen partitions holds a byte per
+ *    element (zen_bitmap_dense_dict_bytes): built anew, not kept from an older
+ *    library
  */
-#define ZEN_ABI_VERSION 9
+#define ZEN_ABI_VERSION 10
 
 #define ZEN_F32 0
 #define ZEN_BF16 1
@@ -548,9 +551,9 @@ int zen_decode_dense_sorted(const void *idx, int idx64_in, const void *val, int 
  * all ranks followed by decode_sparse_tensors (comm.py:87-99, 136-145) without the indices, the member lists
  * (mapping) or a cleared dense tensor in between.
  *   zen_bitmap_dense_dict builds, once per (numel, partitions), what stands in for the mapping the reference
- * caches (comm.py:132-134): per tile of 8192 indices the places of the tile's indices ordered by partition (16
- * bits each) and the members of every partition below the tile (zen_bitmap_dense_dict_bytes bytes, a little
- * over two per element, 16-byte aligned).  members, if not
+ * caches (comm.py:132-134): per tile of indices the places of the tile's indices ordered by partition (a byte
+ * each for up to sixteen partitions, else 16 bits) and the members of every partition below the tile
+ * (zen_bitmap_dense_dict_bytes bytes, a little over one or two per element, 16-byte aligned).  members, if not
  * NULL, is a HOST array that receives the partitions' list lengths (this synchronises on the stream).
  *   zen_bitmap_dense: bitmaps / values hold the lists back to back, list p at byte bitmap_start[p] (of
  * bitmap_start[p + 1] - bitmap_start[p] bytes) and element value_start[p]; both offset arrays are HOST arrays

@@ -313,6 +313,32 @@ def test_bitmaps_to_dense_in_one_pass_matches_oracle(zen, oracle, n, P, frac, dt
     assert np.array_equal(to_np(got), _dense_truth(oracle, n, idx, val))
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("n, P", [
+    (7679, 1), (7168, 2), (7681, 3), (2 * 7168 + 1, 16), (8191, 16), (8193, 17), (3 * 7168 - 1, 15),  # edges of the tiles
+    (1030, 2), (16 * 8 + 5, 16), (100, 16),                      # lists of a chunk of 512 and a few more; of a few members
+    (83381, 16), (141040, 16), (167428, 15),                     # a list with two members 256 or more elements apart
+])
+def test_bitmaps_to_dense_at_the_edges_of_the_dictionary(zen, oracle, n, P, dtype):
+    """Every member set (lists end with their values), every other one, few and none, exact."""
+    mp = oracle.mapping(n, P)
+    rng = np.random.default_rng(n)
+    if n > 80000:
+        tile = [m // 7168 for m in mp]
+        far = [np.diff(np.concatenate([[-1], m % 7168 if len(m) else m])) for m in mp]
+        same = [np.concatenate([[True], np.diff(t) == 0]) for t in tile]
+        assert any((f[s] > 255).any() for f, s in zip(far, same))
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P, 0), None, None)
+    for share in (1.0, 0.5, 0.03, 0.0):
+        idx = [m[rng.random(len(m)) < share] if share < 1 else m for m in mp]
+        val = [(rng.standard_normal(len(i)) * 1e-3 + 1.0).astype(np.float32) for i in idx]
+        if dtype == "bf16":
+            val = [oracle.f32_to_bf16_bits(v) for v in val]
+        bitmaps = [oracle.bitmap_encode(m, i) for m, i in zip(mp, idx)]
+        got = lba.decode_bitmaps_dense([to_dev(b) for b in bitmaps], [to_dev(v) for v in val], n)
+        assert np.array_equal(to_np(got), _dense_truth(oracle, n, idx, val)), share
+
+
 @pytest.mark.parametrize("form", ["strided values", "two value types"])
 def test_bitmaps_to_dense_with_values_in_any_layout(zen, oracle, form):
     """Value lists that are not contiguous, or of two types (the dense tensor then has the one that holds both)."""

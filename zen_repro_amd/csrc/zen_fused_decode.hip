@@ -3,14 +3,16 @@
 // into int64 indices by masking the cached member list (comm.py:87-99, 136-141) and scatter-adds all
 // (index, value) lists into a zeroed dense tensor (comm.py:142-145, 32-44).  Neither the indices nor the
 // member lists are needed for that: which partition an index belongs to is a hash away, and bit j of
-// partition p's bitmap stands for the j-th index of that partition.  So the dense tensor is cut into tiles of
-// 8192 indices; a dictionary built once per (numel, partitions) holds, per tile, the places of the tile's
-// indices ordered by partition (16 bits each: partition 0's members in ascending order, then partition 1's,
-// ...) and, per partition and tile, how many members lie below the tile.  A call first counts, per tile and
-// partition, the set bits of the tile's bit range (which gives where the tile's values start in every value
-// list); then a workgroup per tile brings the tile's bit ranges and values into LDS, looks up the place of
-// every SET bit's member in the dictionary, and writes the tile once, zeros included: the dense tensor is
-// never cleared, nothing is scattered in memory, and of the dictionary only the set bits' entries are read.
+// partition p's bitmap stands for the j-th index of that partition.  So the dense tensor is cut into tiles; a
+// dictionary built once per (numel, partitions) holds, per tile, the places of the tile's indices ordered by
+// partition (partition 0's members in ascending order, then partition 1's, ...; up to sixteen partitions a byte
+// each, the distance from the member in front, else 16 bits) and, per partition and tile, how many members lie
+// below the tile.  A call first counts, per tile and partition, the set bits of the tile's bit range (which gives
+// where the tile's values start in every value list); then a workgroup per tile puts the values in their members'
+// places in LDS and writes the tile once, zeros included: the dense tensor is never cleared and nothing is
+// scattered in memory.
+#include <type_traits>
+
 #include "zen_common.h"
 
 namespace zen {
@@ -18,12 +20,29 @@ namespace {
 
 constexpr int kFdTile = 8192;
 constexpr int kFdBlock = 512;
-constexpr int kFdPer = kFdTile / kFdBlock;   // consecutive indices per thread (16)
 constexpr int kFdMaxLists = 64;
+
+// Dictionaries of bytes: a member's place is that of the member in front of it in its list plus a byte, which takes half
+// the memory of places of 16 bits.  The members of a list lie as far apart as there are lists, give or take: up to
+// sixteen lists one distance in ten million does not fit a byte (a chunk with such a one is marked, and its places are
+// found by hashing), at 32 lists one in three thousand and at 64 one in fifty, so that nearly every tile would have
+// some.  A lane takes eight members, a chunk is what a wave takes, and seven eighths of 8192 elements to a tile
+// keep the lists' shares under whole chunks: at sixteen lists 448 members, give or take 20.
+constexpr int kFdByteLists = 16;
+constexpr int kFdByteTile = 7168;
+constexpr int kFdLane = 8;                               // members a lane takes
+constexpr int kFdByteChunk = 64 * kFdLane;
+constexpr int kFdByteRow = kFdByteTile + kFdLane * kFdByteLists;  // bytes of a tile: lists begin at multiples of kFdLane
+constexpr int kFdByteChunks = 32;                        // 16-bit words of a tile's chunk table
+constexpr uint32_t kFdHashed = 0x8000u;                  // in a chunk's word: its places are found by hashing
+static_assert(kFdByteTile / kFdByteChunk + kFdByteLists <= kFdByteChunks, "every chunk of a tile has a word");
+static_assert(kFdByteTile % (16 * kFdBlock / 64) == 0 && kFdByteTile < (1 << 14) && kFdByteRow % 16 == 0, "tile layout");
 constexpr int kFdChunk = 16;                  // thread columns whose counts one thread adds up
 constexpr int kFdChunks = kFdBlock / kFdChunk;
 constexpr int kFdChunkRow = kFdChunks + 8;   // 16-bit words per list in the chunk table (rows stay 16-byte aligned)
 static_assert(kFdChunks == 32, "a wave's lower half scans the chunk sums");
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 struct FdLists {
   const uint8_t *bitmap[kFdMaxLists];
@@ -31,29 +50,65 @@ struct FdLists {
   uint32_t bytes[kFdMaxLists], vals[kFdMaxLists];  // of the bitmap (2^28 at most: its bits fit 32 bits); values
 };
 
-__device__ inline uint32_t part_of(uint32_t t, uint32_t n, uint32_t npp) {
-  return ((poly(t) + kSeed1) % n) / npp;  // functions_cuda_kernel.cu:172-175
+// Division by a number known to the host: its inverse, rounded down, gives the quotient or one less.
+struct FdDivisor {
+  uint32_t d, inverse;  // floor(2^32 / d), or 2^32 - 1
+};
+inline FdDivisor fd_divisor(uint32_t d) { return {d, d > 1 ? (uint32_t)((1ull << 32) / d) : 0xffffffffu}; }
+__device__ inline uint32_t part_of(uint32_t t, FdDivisor n, FdDivisor npp) {  // hash % n / npp, functions_cuda_kernel.cu:172-175
+  const uint32_t h = poly(t) + kSeed1;
+  uint32_t rem = h - __umulhi(h, n.inverse) * n.d;  // below 2 n
+  if (rem >= n.d) rem -= n.d;
+  const uint32_t part = __umulhi(rem, npp.inverse);
+  return part + (rem - part * npp.d >= npp.d ? 1u : 0u);
 }
 
 // Dictionary, step 1: per tile the places of its indices ordered by partition, and the number of indices of
-// every partition.  Dynamic LDS: P * (kFdBlock + kFdChunkRow) 16-bit counters.  Every thread counts, for its 16
-// consecutive indices, how many belong to each list; prefix sums over the threads, in two levels (chunks of
-// 16 threads, then the 32 chunks), give every index its rank inside its list.
-__global__ __launch_bounds__(kFdBlock) void k_fd_order(uint32_t n, uint32_t npp, int P, uint16_t *__restrict__ order,
-                                                      uint32_t *__restrict__ below) {
+// every partition.  Every thread counts, for its consecutive indices, how many belong to each list; prefix sums over
+// the threads, in two levels (chunks of 16 threads, then the 32 chunks), give every index its rank inside its list.
+// BYTES: `order` holds distances (kFdByteRow bytes a tile, lists padded to whole lanes) and chunk_at, per chunk of a
+// list's members, the first place behind the member in front of the chunk, with kFdHashed where a distance does not
+// fit.  Else 16-bit places, kFdTile a tile.  Dynamic LDS: fd_order_lds.
+template <bool BYTES>
+__global__ __launch_bounds__(kFdBlock) void k_fd_order(FdDivisor n, FdDivisor npp, int P, void *__restrict__ order,
+                                                      uint16_t *__restrict__ chunk_at, uint32_t *__restrict__ below) {
+  constexpr int kTile = BYTES ? kFdByteTile : kFdTile;
+  constexpr int kPer = kTile / kFdBlock;  // consecutive indices per thread
   extern __shared__ __attribute__((aligned(16))) uint16_t s_cnt[];  // [P][kFdBlock]
   uint16_t (*s_chunk)[kFdChunkRow] = reinterpret_cast<uint16_t (*)[kFdChunkRow]>(s_cnt + P * kFdBlock);  // [32]: the tile's total
-  __shared__ uint32_t s_base[kFdMaxLists];  // members of lower lists in the tile
-  const uint32_t tile_base = blockIdx.x * (uint32_t)kFdTile;
-  const uint32_t base = tile_base + threadIdx.x * (uint32_t)kFdPer;
-  uint32_t part[kFdPer];
+  __shared__ uint32_t s_base[kFdMaxLists];   // where a list begins in the tile's row
+  __shared__ uint32_t s_first[kFdMaxLists];  // BYTES: chunks of lower lists
+  const uint32_t tile_base = blockIdx.x * (uint32_t)kTile;
+  const uint32_t base = tile_base + threadIdx.x * (uint32_t)kPer;
+  uint32_t part[kPer];
 #pragma unroll
-  for (int e = 0; e < kFdPer; ++e) part[e] = base + e < n ? part_of(base + e, n, npp) : 0xffu;
-  for (int p = 0; p < P; ++p) {
-    uint32_t c = 0;
+  for (int e = 0; e < kPer; ++e) part[e] = base + e < n.d ? part_of(base + e, n, npp) : 0xffu;
+  uint32_t rank[kPer];  // among the thread's own, for now
+  if constexpr (BYTES) {
+    // four bits a list (268 M elements on sixteen lists: 810 us with a comparison per element and list and per pair of
+    // elements, and with the compiler's divisions; 570 so)
+    static_assert(kPer < 16 && kFdByteLists <= 16, "counters of four bits");
+    uint64_t count = 0;
 #pragma unroll
-    for (int e = 0; e < kFdPer; ++e) c += part[e] == (uint32_t)p;
-    s_cnt[p * kFdBlock + threadIdx.x] = (uint16_t)c;
+    for (int e = 0; e < kPer; ++e) {
+      const uint32_t at = part[e] * 4u & 63u;
+      rank[e] = (uint32_t)(count >> at) & 15u;
+      count += (uint64_t)(part[e] < (uint32_t)P ? 1u : 0u) << at;
+    }
+    for (int p = 0; p < P; ++p) s_cnt[p * kFdBlock + threadIdx.x] = (uint16_t)((uint32_t)(count >> (4 * p)) & 15u);
+  } else {
+    for (int p = 0; p < P; ++p) {
+      uint32_t c = 0;
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) c += part[e] == (uint32_t)p;
+      s_cnt[p * kFdBlock + threadIdx.x] = (uint16_t)c;
+    }
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+      rank[e] = 0;
+#pragma unroll
+      for (int f = 0; f < e; ++f) rank[e] += part[f] == part[e];
+    }
   }
   __syncthreads();
   for (int q = threadIdx.x; q < P * kFdChunks; q += kFdBlock) {
@@ -78,21 +133,50 @@ __global__ __launch_bounds__(kFdBlock) void k_fd_order(uint32_t n, uint32_t npp,
   __syncthreads();
   if (threadIdx.x < 64) {
     const uint32_t total = threadIdx.x < (uint32_t)P ? s_chunk[threadIdx.x][kFdChunks] : 0u;
-    const uint32_t incl = wave_inclusive_scan(total);
+    const uint32_t room = BYTES ? (total + kFdLane - 1) / kFdLane * kFdLane : total;
+    const uint32_t chunks = (total + kFdByteChunk - 1) / kFdByteChunk;
+    const uint32_t incl = wave_inclusive_scan(room), cincl = wave_inclusive_scan(chunks);
     if (threadIdx.x < (uint32_t)P) {
-      s_base[threadIdx.x] = incl - total;
+      s_base[threadIdx.x] = incl - room;
+      s_first[threadIdx.x] = cincl - chunks;
       below[(size_t)blockIdx.x * P + threadIdx.x] = total;
     }
   }
   __syncthreads();
 #pragma unroll
-  for (int e = 0; e < kFdPer; ++e) {
+  for (int e = 0; e < kPer; ++e) {
     const uint32_t p = part[e];
     if (p >= (uint32_t)P) continue;  // past the end of the tensor
-    uint32_t rank = s_base[p] + s_chunk[p][threadIdx.x / kFdChunk] + s_cnt[p * kFdBlock + threadIdx.x];
+    rank[e] += s_chunk[p][threadIdx.x / kFdChunk] + s_cnt[p * kFdBlock + threadIdx.x];
+    if (!BYTES) static_cast<uint16_t *>(order)[tile_base + s_base[p] + rank[e]] = (uint16_t)(threadIdx.x * kPer + e);
+  }
+  if constexpr (BYTES) {
+    uint16_t *s_place = &s_chunk[P][0];                                   // [kFdByteRow]
+    uint8_t *s_byte = reinterpret_cast<uint8_t *>(s_place + kFdByteRow);  // [kFdByteRow]
+    __shared__ uint32_t s_at[kFdByteChunks];
+    if (threadIdx.x < kFdByteChunks) s_at[threadIdx.x] = 0;
+    // what pads a list to whole lanes belongs to nobody
+    for (int i = threadIdx.x; i < kFdByteRow / 4; i += kFdBlock) reinterpret_cast<uint32_t *>(s_byte)[i] = 0x01010101u;
 #pragma unroll
-    for (int f = 0; f < e; ++f) rank += part[f] == p;
-    order[tile_base + rank] = (uint16_t)(threadIdx.x * kFdPer + e);
+    for (int e = 0; e < kPer; ++e)
+      if (part[e] < (uint32_t)P) s_place[s_base[part[e]] + rank[e]] = (uint16_t)(threadIdx.x * kPer + e);
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+      const uint32_t p = part[e];
+      if (p >= (uint32_t)P) continue;
+      const uint32_t at = s_base[p] + rank[e], place = threadIdx.x * kPer + e;
+      const uint32_t from = rank[e] ? s_place[at - 1] + 1u : 0u;  // the first place it could have had
+      const uint32_t chunk = s_first[p] + rank[e] / kFdByteChunk;
+      const uint32_t far = place - from > 254u ? kFdHashed : 0u;
+      s_byte[at] = (uint8_t)(far ? 0u : place - from + 1u);
+      const uint32_t word = far | (rank[e] % kFdByteChunk == 0 ? from : 0u);
+      if (word) atomicOr(&s_at[chunk], word);
+    }
+    __syncthreads();
+    uint4 *row = reinterpret_cast<uint4 *>(static_cast<uint8_t *>(order) + (size_t)blockIdx.x * kFdByteRow);
+    for (int i = threadIdx.x; i < kFdByteRow / 16; i += kFdBlock) row[i] = reinterpret_cast<const uint4 *>(s_byte)[i];
+    if (threadIdx.x < kFdByteChunks) chunk_at[(size_t)blockIdx.x * kFdByteChunks + threadIdx.x] = (uint16_t)s_at[threadIdx.x];
   }
 }
 
@@ -272,6 +356,43 @@ __device__ inline unsigned long long fd_chunk_bits(const uint8_t *bitmap, uint32
   return bits;
 }
 
+// 0.0f + v for a tile put together in LDS, and out with it in 16-byte pieces, consecutive threads consecutive pieces:
+// every store instruction fills whole lines.  By the whole workgroup; fix: some of the values may need the sum.
+template <typename S, int TILE, int BLOCK>
+__device__ inline void fd_write_tile(const S *s_tile, uint32_t tile_base, uint32_t n, bool fix, S *__restrict__ dense) {
+  if ((reinterpret_cast<uintptr_t>(dense) & 15u) == 0 && tile_base + (uint32_t)TILE <= n) {
+    constexpr int kAll = (int)(TILE * sizeof(S) / 16);
+    constexpr int kPieces = (kAll + BLOCK - 1) / BLOCK;
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(s_tile);
+    u32x4 *dst = reinterpret_cast<u32x4 *>(dense + tile_base);
+    u32x4 piece[kPieces];
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int at = i * BLOCK + (int)threadIdx.x;
+      piece[i] = src[(i + 1) * BLOCK <= kAll || at < kAll ? at : 0];
+    }
+    if (fix) fd_values(piece, S(0));
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int at = i * BLOCK + (int)threadIdx.x;
+      if ((i + 1) * BLOCK <= kAll || at < kAll) __builtin_nontemporal_store(piece[i], dst + at);
+    }
+  } else {
+    for (uint32_t e = threadIdx.x; e < (uint32_t)TILE && tile_base + e < n; e += BLOCK)
+      dense[tile_base + e] = fd_value<S>(s_tile[e]);
+  }
+}
+
+template <typename S, int TILE, int BLOCK>
+__device__ inline void fd_clear_tile(S *s_tile) {
+  uint4 *z = reinterpret_cast<uint4 *>(s_tile);
+#pragma unroll
+  for (int i = 0; i * BLOCK < (int)(TILE * sizeof(S) / 16); ++i) {
+    const int at = i * BLOCK + (int)threadIdx.x;
+    if ((i + 1) * BLOCK <= (int)(TILE * sizeof(S) / 16) || at < (int)(TILE * sizeof(S) / 16)) z[at] = make_uint4(0, 0, 0, 0);
+  }
+}
+
 // One workgroup per tile.  Lane p of every wave knows list p's members in the tile, the first bit of their range
 // and where its values start; the lists' members are cut into chunks of 576, dealt to the waves in turn.  A
 // wave gets the chunk's bits as nine 64-bit words in scalar registers: the word is the mask of the lanes whose
@@ -314,11 +435,7 @@ __global__ __launch_bounds__(fd_tile_block<S>(), sizeof(S) == 2 ? 6 : 8) void k_
     b1 = below[at + P];
     v0 = vstart[at] + gpre[(size_t)(tile / kFdGroup) * P + lane];
   }
-  {
-    uint4 *z = reinterpret_cast<uint4 *>(s_tile);
-#pragma unroll
-    for (int i = 0; i < (int)(kFdTile * sizeof(S) / 16) / kBlock; ++i) z[i * kBlock + threadIdx.x] = make_uint4(0, 0, 0, 0);
-  }
+  fd_clear_tile<S, kFdTile, kBlock>(s_tile);
   uint32_t cnt = b1 - b0;
   if (cnt > (uint32_t)kFdTile) cnt = 0;  // cannot be with a table this library built
   const uint32_t chunks = (cnt + kFdMembers - 1) / kFdMembers;
@@ -393,37 +510,220 @@ __global__ __launch_bounds__(fd_tile_block<S>(), sizeof(S) == 2 ? 6 : 8) void k_
       if (__builtin_amdgcn_inverse_ballot_w64(word[i])) s_tile[place[i] & (uint32_t)(kFdTile - 1)] = v[i];
   }
   __syncthreads();
-  // written out in 16-byte pieces, consecutive threads consecutive pieces: every store instruction fills whole lines
-  if ((reinterpret_cast<uintptr_t>(dense) & 15u) == 0 && tile_base + (uint32_t)kFdTile <= n) {
-    constexpr int kPieces = (int)(kFdTile * sizeof(S) / 16) / kBlock;
-    const u32x4 *src = reinterpret_cast<const u32x4 *>(s_tile);
-    u32x4 *dst = reinterpret_cast<u32x4 *>(dense + tile_base);
-    u32x4 piece[kPieces];
-#pragma unroll
-    for (int i = 0; i < kPieces; ++i) piece[i] = src[i * kBlock + threadIdx.x];
-    fd_values(piece, S(0));
-#pragma unroll
-    for (int i = 0; i < kPieces; ++i) __builtin_nontemporal_store(piece[i], dst + i * kBlock + threadIdx.x);
-  } else {
-    for (uint32_t e = threadIdx.x; e < (uint32_t)kFdTile && tile_base + e < n; e += kBlock)
-      dense[tile_base + e] = fd_value<S>(s_tile[e]);
-  }
+  fd_write_tile<S, kFdTile, kBlock>(s_tile, tile_base, n, true, dense);
   if (odd && lane == 0) atomicOr(status, ZEN_STAT_BAD_INDEX);
 }
 
-inline uint32_t fd_tiles(int64_t numel) { return (uint32_t)ceil_div(numel, kFdTile); }
-// (a chunk's places are read as if it were full)
-inline size_t fd_order_bytes(int64_t numel) {
-  return align_up(((size_t)fd_tiles(numel) * kFdTile + kFdMembers) * sizeof(uint16_t), 256);
+// The kernel for dictionaries of bytes.  A wave takes a chunk of a list's members, a lane eight of them: their distances
+// are one 8-byte load, their bits of the bitmap two bytes, and one prefix sum across the lanes gives every lane both the
+// place in front of its first member and the number of its first value.  The lanes list the places of their members that
+// have a value, in LDS, and the values go there with consecutive lanes on consecutive values.
+// Bound by the vector instructions (two thirds of the kernel's time) and by the three trips to memory of a tile; of the
+// bytes (0.86 GB for the 268 M elements below) it moves 4.1 TB a second.  bf16, sixteen lists, with places of 16 bits and
+// so, us: 268 M elements, 11 % set 245 and 209; the calls of 62 M, 71 % set 110 and 99; four lists, 134 M, 10 % 198 and 184;
+// fp32, sixteen lists, 67 M 119 and 120.  Slower: a lane that fetches the values of its own members (eight loads that
+// touch the same lines; 268 M: 316); tiles of 7680 elements, whose lists of 480 members go beyond a chunk in one case of
+// fifteen, and one of a tile's four waves takes five chunks where the others take four; 512 threads (40 more); four chunks
+// of a wave under way together, all their loads in front (registers: 209 at six waves a SIMD, 20 more at eight).
+template <typename S>
+__global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
+    const uint8_t *__restrict__ order, const uint16_t *__restrict__ chunk_at, const uint32_t *__restrict__ below,
+    const uint32_t *__restrict__ vstart, const uint32_t *__restrict__ gpre, int P, FdDivisor n, FdDivisor npp, FdLists lists,
+    S *__restrict__ dense, int32_t *status) {
+  constexpr int kBlock = fd_tile_block<S>();
+  __shared__ __attribute__((aligned(16))) S s_tile[kFdByteTile];
+  __shared__ uint16_t s_list[kBlock / 64][kFdByteChunk];
+  __shared__ uint32_t s_special;  // a value that 0.0f + v changes: -0 or a NaN
+  const uint32_t tile = blockIdx.x;
+  const uint32_t tile_base = tile * (uint32_t)kFdByteTile;
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  uint32_t b0 = 0, b1 = 0, v0 = 0;
+  if (lane < P) {
+    const size_t at = (size_t)tile * P + lane;
+    b0 = below[at];
+    b1 = below[at + P];
+    v0 = vstart[at] + gpre[(size_t)(tile / kFdGroup) * P + lane];
+  }
+  const uint32_t starts = lane < kFdByteChunks ? chunk_at[(size_t)tile * kFdByteChunks + lane] : 0u;
+  fd_clear_tile<S, kFdByteTile, kBlock>(s_tile);
+  if (threadIdx.x == 0) s_special = 0;
+  uint32_t cnt = b1 - b0;
+  if (cnt > (uint32_t)kFdByteTile) cnt = 0;  // cannot be with a table this library built
+  const uint32_t room = (cnt + kFdLane - 1) / kFdLane * kFdLane, chunks = (cnt + kFdByteChunk - 1) / kFdByteChunk;
+  const uint32_t incl = wave_inclusive_scan(room), cincl = wave_inclusive_scan(chunks);
+  const uint32_t nchunks = (uint32_t)__builtin_amdgcn_readlane((int)cincl, 63);
+  const bool odd = __builtin_amdgcn_readlane((int)incl, 63) > kFdByteRow || nchunks > (uint32_t)kFdByteChunks;  // cannot be either
+  const uint8_t *row = order + (size_t)tile * kFdByteRow;
+  uint16_t *list = s_list[wave];
+  __syncthreads();
+  // What a chunk asks memory for: its distances, and for every lane the byte of the bitmap that holds its first bit and
+  // the one behind that.  The next chunk's are asked for while this one's are worked on.
+  // (so are the list's pointers and lengths: a wave would wait for the constants' cache in front of every use)
+  struct Asked {
+    int p;
+    uint32_t j0, bytes, have;
+    const uint8_t *bitmap;
+    const char *val;
+    uint8_t lo, hi;
+    u32x2 far;
+  };
+  auto ask = [&](uint32_t c) {
+    Asked a;
+    a.p = (int)__popcll(__ballot(cincl <= c));  // the chunk's list
+    a.j0 = (c - (uint32_t)__builtin_amdgcn_readlane((int)(cincl - chunks), a.p)) * kFdByteChunk;
+    // (past the members: the next list's distances, or what follows the last)
+    a.far = __builtin_nontemporal_load(reinterpret_cast<const u32x2 *>(
+        row + (uint32_t)__builtin_amdgcn_readlane((int)(incl - room), a.p) + a.j0 + lane * kFdLane));
+    a.bytes = lists.bytes[a.p];
+    a.bitmap = lists.bitmap[a.p];  // of a list without one: readable all the same
+    a.have = lists.vals[a.p];
+    a.val = static_cast<const char *>(lists.val[a.p]);
+    const uint32_t last = a.bytes ? a.bytes - 1u : 0u;
+    const uint32_t at = (((uint32_t)__builtin_amdgcn_readlane((int)b0, a.p) + a.j0) >> 3) + (uint32_t)lane;
+    const uint32_t at0 = at < last ? at : last, at1 = at + 1u < last ? at + 1u : last;
+    a.lo = a.bitmap[at0];
+    a.hi = a.bitmap[at1];
+    return a;
+  };
+  Asked next{};
+  if ((uint32_t)wave < nchunks && !odd) next = ask((uint32_t)wave);
+#pragma unroll 1
+  for (uint32_t c = (uint32_t)wave; c < nchunks && !odd; c += kBlock / 64) {
+    const Asked now = next;
+    next = ask(c + kBlock / 64 < nchunks ? c + kBlock / 64 : c);
+    const int p = now.p;
+    const uint32_t j0 = now.j0;
+    const u32x2 far = now.far;
+    const uint32_t members = (uint32_t)__builtin_amdgcn_readlane((int)cnt, p) - j0;  // from here on, > 0
+    const uint32_t bit0 = (uint32_t)__builtin_amdgcn_readlane((int)b0, p) + j0;
+    const uint32_t start = (uint32_t)__builtin_amdgcn_readlane((int)starts, (int)c);
+    // the members' bits; those past the members and past the bitmap's end are zero
+    const uint32_t before = (uint32_t)lane * kFdLane;
+    uint32_t bits;
+    {
+      const uint32_t limit = now.bytes * 8u;
+      const uint32_t has = bit0 < limit ? limit - bit0 : 0u;  // bits the bitmap has from the chunk's first on
+      const uint32_t end = has < members ? has : members;
+      const uint32_t left = end > before ? end - before : 0u;
+      bits = __builtin_amdgcn_ubfe((uint32_t)now.lo | (uint32_t)now.hi << 8, bit0 & 7u, left < (uint32_t)kFdLane ? left : (uint32_t)kFdLane);
+    }
+    // set bits of the tile's range in front of the chunk: the list's earlier chunks in this tile
+    uint32_t nth = (uint32_t)__builtin_amdgcn_readlane((int)v0, p);
+    if (j0) {  // 128 bits per lane
+      const uint32_t from = bit0 - j0 + (uint32_t)lane * (kFdTile / 64);
+      const uint32_t to = from + kFdTile / 64;
+      nth += wave_sum(from < bit0 ? popcount_range<1>(now.bitmap, now.bytes, from, to < bit0 ? to : bit0) : 0u);
+    }
+    nth = (uint32_t)__builtin_amdgcn_readfirstlane((int)nth);
+    // Both prefix sums in one word: places (below 2^14; those of lanes past the members stay below 2^18) in the low 18 bits,
+    // values above.
+    const uint32_t mine = __builtin_amdgcn_sad_u8(far.x, 0u, __builtin_amdgcn_sad_u8(far.y, 0u, (uint32_t)__popc(bits) << 18));
+    const uint32_t all = wave_inclusive_scan(mine);
+    uint32_t set = (uint32_t)__builtin_amdgcn_readlane((int)all, 63) >> 18;
+    const uint32_t k = (all - mine) >> 18;
+    const uint32_t have = now.have;
+    if (nth + set > have) {  // more set bits than values: the missing ones count as unset
+      set = have > nth ? have - nth : 0u;
+      while (bits && k + (uint32_t)__popc(bits) > set) bits &= ~(0x80000000u >> __clz((int)bits));
+    }
+    if (set == 0) continue;
+    const char *val = now.val + (size_t)nth * sizeof(S);
+    if (start & kFdHashed) {  // a distance that does not fit its byte: whose the places are is hashed out
+      uint32_t seen = 0;
+      for (uint32_t t0 = 0; t0 < (uint32_t)kFdByteTile; t0 += 64) {
+        const uint32_t t = t0 + (uint32_t)lane;
+        const bool member = tile_base + t < n.d && part_of(tile_base + t, n, npp) == (uint32_t)p;
+        const unsigned long long who = __ballot(member);
+        const uint32_t j = seen + __builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0u)) - j0;
+        seen += (uint32_t)__popcll(who);
+        const uint32_t theirs = (uint32_t)__shfl((int)bits, (int)(j / kFdLane) & 63, 64);
+        const uint32_t front = (uint32_t)__shfl((int)k, (int)(j / kFdLane) & 63, 64);
+        const uint32_t bit = j % kFdLane;
+        if (member && j < (uint32_t)kFdByteChunk && ((theirs >> bit) & 1u))
+          s_special = 1, s_tile[t] = reinterpret_cast<const S *>(val)[front + (uint32_t)__popc(theirs & ((1u << bit) - 1u))];
+      }
+      continue;
+    }
+    // The places of those that have a value are listed in its order, and the values go there with consecutive lanes on
+    // consecutive values: a lane that fetches its own members' reads the same lines as its neighbours eight times over.
+    const uint32_t front = (start & (kFdHashed - 1u)) + ((all - mine) & 0x3ffffu) - 1u;
+    auto put = [&](auto rows) {
+      constexpr int kRows = decltype(rows)::value;
+      S v[kRows];
+#pragma unroll
+      for (int i = 0; i < kRows; ++i) {
+        const uint32_t at = (uint32_t)(i * 64 + lane);
+        v[i] = *reinterpret_cast<const S *>(val + (uint32_t)((at < set ? at : set - 1u) * sizeof(S)));
+      }
+      uint32_t place = front;
+      int mark = (int)__brev(bits);
+      uint16_t *to = list + k;
+#pragma unroll
+      for (int i = 0; i < kFdLane; ++i) {
+        place += ((i < 4 ? far.x : far.y) >> (8 * (i & 3))) & 0xffu;
+        if (mark < 0) *to++ = (uint16_t)place;
+        mark <<= 1;
+      }
+      __builtin_amdgcn_wave_barrier();
+      bool special = false;
+#pragma unroll
+      for (int i = 0; i < kRows; ++i) special |= __builtin_amdgcn_classf(KeyOf<S>::to_f32(v[i]), 0x23);
+      if (special) s_special = 1;
+#pragma unroll
+      for (int i = 0; i < kRows; ++i) {
+        const uint32_t at = (uint32_t)(i * 64 + lane);
+        if (at < set) s_tile[list[at]] = v[i];
+      }
+      __builtin_amdgcn_wave_barrier();
+    };
+    if (set <= 64u)
+      put(std::integral_constant<int, 1>{});
+    else if (set <= 128u)
+      put(std::integral_constant<int, 2>{});
+    else
+      put(std::integral_constant<int, kFdLane>{});
+  }
+  __syncthreads();
+  fd_write_tile<S, kFdByteTile, kBlock>(s_tile, tile_base, n.d, s_special != 0, dense);
+  if (odd && lane == 0) atomicOr(status, ZEN_STAT_BAD_INDEX);
 }
-inline size_t fd_table_bytes(int64_t numel, int P) { return align_up(((size_t)fd_tiles(numel) + 1) * P * sizeof(uint32_t), 256); }
-inline size_t fd_vstart_bytes(int64_t numel, int P) { return align_up((size_t)fd_tiles(numel) * P * sizeof(uint32_t), 256); }
-inline size_t fd_gsum_bytes(int64_t numel, int P) { return align_up((size_t)fd_groups(fd_tiles(numel)) * P * sizeof(uint32_t), 256); }
+
+// Dictionaries of bytes (see kFdByteLists), as long as their tiles' groups have a thread each in k_fd_groups (1.88e9 elements).
+inline bool fd_of_bytes(int64_t numel, int P) {
+  return P <= kFdByteLists && ceil_div(numel, kFdByteTile) <= (int64_t)kFdGroupsMax * kFdGroup;
+}
+inline uint32_t fd_tiles(int64_t numel, int P) { return (uint32_t)ceil_div(numel, fd_of_bytes(numel, P) ? kFdByteTile : kFdTile); }
+// (a chunk's places are read as if it were full)
+inline size_t fd_order_bytes(int64_t numel, int P) {
+  const size_t tiles = fd_tiles(numel, P);
+  return align_up(fd_of_bytes(numel, P) ? tiles * kFdByteRow + kFdByteChunk : (tiles * kFdTile + kFdMembers) * sizeof(uint16_t), 256);
+}
+inline size_t fd_chunk_bytes(int64_t numel, int P) {
+  return fd_of_bytes(numel, P) ? align_up((size_t)fd_tiles(numel, P) * kFdByteChunks * sizeof(uint16_t), 256) : 0;
+}
+inline size_t fd_table_bytes(int64_t numel, int P) { return align_up(((size_t)fd_tiles(numel, P) + 1) * P * sizeof(uint32_t), 256); }
+inline size_t fd_vstart_bytes(int64_t numel, int P) { return align_up((size_t)fd_tiles(numel, P) * P * sizeof(uint32_t), 256); }
+inline size_t fd_gsum_bytes(int64_t numel, int P) { return align_up((size_t)fd_groups(fd_tiles(numel, P)) * P * sizeof(uint32_t), 256); }
 
 int fd_check(int64_t numel, int partitions) {
   if (numel <= 0 || numel > 0x7fffffffll || partitions < 1 || partitions > kFdMaxLists || numel / partitions == 0)
     return fail(ZEN_EINVAL, "zen_bitmap_dense: need 0 < partitions <= 64 and partitions <= numel < 2^31");
   return ZEN_OK;
+}
+
+template <typename S>
+void fd_launch_tiles(const void *dict, const uint8_t *chunk_at, const uint32_t *below, const uint32_t *vstart,
+                     const uint32_t *gsum, uint32_t tiles, int P, int64_t numel, const FdLists &lists, void *dense,
+                     int32_t *status, hipStream_t s) {
+  const dim3 grid(tiles), block(fd_tile_block<S>());
+  if (fd_of_bytes(numel, P))
+    k_fd_tiles_bytes<S><<<grid, block, 0, s>>>(static_cast<const uint8_t *>(dict), reinterpret_cast<const uint16_t *>(chunk_at),
+                                               below, vstart, gsum, P, fd_divisor((uint32_t)numel), fd_divisor((uint32_t)(numel / P)), lists,
+                                               static_cast<S *>(dense), status);
+  else
+    k_fd_tiles<S><<<grid, block, 0, s>>>(static_cast<const uint16_t *>(dict), below, vstart, gsum, P, (uint32_t)numel, lists,
+                                         static_cast<S *>(dense), status);
 }
 
 }  // namespace
@@ -433,7 +733,7 @@ extern "C" {
 
 size_t zen_bitmap_dense_dict_bytes(int64_t numel, int partitions) {
   if (zen::fd_check(numel, partitions) != ZEN_OK) return 0;
-  return zen::fd_order_bytes(numel) + zen::fd_table_bytes(numel, partitions);
+  return zen::fd_order_bytes(numel, partitions) + zen::fd_chunk_bytes(numel, partitions) + zen::fd_table_bytes(numel, partitions);
 }
 
 int zen_bitmap_dense_dict(int64_t numel, int partitions, void *dict, int64_t *members, void *stream) {
@@ -442,13 +742,16 @@ int zen_bitmap_dense_dict(int64_t numel, int partitions, void *dict, int64_t *me
   if (rc != ZEN_OK) return rc;
   if (!dict || (reinterpret_cast<uintptr_t>(dict) & 15u)) return fail(ZEN_EINVAL, "zen_bitmap_dense_dict: null or unaligned dictionary");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  uint16_t *order = static_cast<uint16_t *>(dict);
-  uint32_t *below = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(dict) + fd_order_bytes(numel));
-  const uint32_t tiles = fd_tiles(numel);
-  const size_t lds = (size_t)partitions * (kFdBlock + kFdChunkRow) * sizeof(uint16_t);
+  const bool of_bytes = fd_of_bytes(numel, partitions);
+  uint8_t *chunk_at = static_cast<uint8_t *>(dict) + fd_order_bytes(numel, partitions);
+  uint32_t *below = reinterpret_cast<uint32_t *>(chunk_at + fd_chunk_bytes(numel, partitions));
+  const uint32_t tiles = fd_tiles(numel, partitions);
+  const size_t lds = (size_t)partitions * (kFdBlock + kFdChunkRow) * sizeof(uint16_t) + (of_bytes ? kFdByteRow * 3u : 0u);
+  const auto fill = of_bytes ? k_fd_order<true> : k_fd_order<false>;
   if (lds > 32768)  // beyond what a launch may ask for without saying so first
-    ZEN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fd_order), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  k_fd_order<<<dim3(tiles), dim3(kFdBlock), lds, s>>>((uint32_t)numel, (uint32_t)(numel / partitions), partitions, order, below);
+    ZEN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(fill), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  fill<<<dim3(tiles), dim3(kFdBlock), lds, s>>>(fd_divisor((uint32_t)numel), fd_divisor((uint32_t)(numel / partitions)), partitions, dict,
+                                                reinterpret_cast<uint16_t *>(chunk_at), below);
   ZEN_LAUNCH_CHECK("k_fd_order");
   k_fd_scan<<<dim3((unsigned)partitions), dim3(kFdScanBlock), 0, s>>>(below, tiles, partitions);
   ZEN_LAUNCH_CHECK("k_fd_scan");
@@ -487,17 +790,17 @@ int zen_bitmap_dense_lists(const void *dict, int64_t numel, int partitions, cons
     if ((bitmap_bytes[p] > 0 && !bitmaps[p]) || (value_count[p] > 0 && !values[p]))
       return fail(ZEN_EINVAL, "zen_bitmap_dense: null pointer");
     // what lies beyond the members a list can have is never looked at
-    lists.bitmap[p] = bitmaps[p];
+    lists.bitmap[p] = bitmap_bytes[p] ? bitmaps[p] : static_cast<const uint8_t *>(dict);
     lists.bytes[p] = (uint32_t)(bitmap_bytes[p] < (1ll << 28) ? bitmap_bytes[p] : 1ll << 28);
     lists.val[p] = values[p];
     lists.vals[p] = (uint32_t)(value_count[p] < (1ll << 31) ? value_count[p] : 1ll << 31);
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const uint16_t *order = static_cast<const uint16_t *>(dict);
-  const uint32_t *below = reinterpret_cast<const uint32_t *>(static_cast<const uint8_t *>(dict) + fd_order_bytes(numel));
+  const uint8_t *chunk_at = static_cast<const uint8_t *>(dict) + fd_order_bytes(numel, partitions);
+  const uint32_t *below = reinterpret_cast<const uint32_t *>(chunk_at + fd_chunk_bytes(numel, partitions));
   uint32_t *vstart = static_cast<uint32_t *>(workspace);
   uint32_t *gsum = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(workspace) + fd_vstart_bytes(numel, partitions));
-  const uint32_t tiles = fd_tiles(numel);
+  const uint32_t tiles = fd_tiles(numel, partitions);
   const uint32_t groups = fd_groups(tiles);
   ProfScope prof(kProfDecodeFused, s);
   k_fd_count<<<dim3(groups, (unsigned)partitions), dim3(kFdGroup), 0, s>>>(below, tiles, partitions, lists, vstart, gsum,
@@ -506,11 +809,9 @@ int zen_bitmap_dense_lists(const void *dict, int64_t numel, int partitions, cons
   k_fd_groups<<<dim3((unsigned)partitions), dim3(kFdGroupsMax), 0, s>>>(gsum, groups, partitions, lists, status);
   ZEN_LAUNCH_CHECK("k_fd_groups");
   if (dtype == ZEN_BF16)
-    k_fd_tiles<uint16_t><<<dim3(tiles), dim3(fd_tile_block<uint16_t>()), 0, s>>>(order, below, vstart, gsum, partitions, (uint32_t)numel,
-                                                                lists, static_cast<uint16_t *>(dense), status);
+    fd_launch_tiles<uint16_t>(dict, chunk_at, below, vstart, gsum, tiles, partitions, numel, lists, dense, status, s);
   else
-    k_fd_tiles<uint32_t><<<dim3(tiles), dim3(fd_tile_block<uint32_t>()), 0, s>>>(order, below, vstart, gsum, partitions, (uint32_t)numel,
-                                                                lists, static_cast<uint32_t *>(dense), status);
+    fd_launch_tiles<uint32_t>(dict, chunk_at, below, vstart, gsum, tiles, partitions, numel, lists, dense, status, s);
   ZEN_LAUNCH_CHECK("k_fd_tiles");
   return ZEN_OK;
 }
