@@ -246,13 +246,16 @@ inline uint32_t fd_groups(uint32_t tiles) { return (tiles + kFdGroup - 1) / kFdG
 // Per (group of tiles, list): set bits in each tile's bit range of the list's bitmap, summed up inside the
 // group.  A bitmap shorter than its list (the reference's mask would not fit the member list, comm.py:97-98)
 // raises ZEN_STAT_BAD_INDEX.
-// A tile's range of a list spans eight or nine words at sixteen ranks (268 M elements: 22 us with one, 16 with five).
+// The lists of a group share the lines of the tables, so a group's workgroups belong on one die: the grid is as many groups
+// wide as make a multiple of the eight dies that workgroups are dealt to in turn (268 M elements, sixteen lists, 147 groups:
+// 18.5 us, with 152 12.5).  A tile's range of a list spans eight words there (22 us with one, 16 with five, and with eight 2 us more).
 constexpr int kFdCountAhead = 5;
 __global__ __launch_bounds__(kFdGroup) void k_fd_count(const uint32_t *__restrict__ below, uint32_t tiles, int P,
                                                        FdLists lists, uint32_t *__restrict__ vstart,
                                                        uint32_t *__restrict__ gsum, int32_t *status) {
   __shared__ uint32_t s_scan[kFdGroup / 64 + 1];
   const uint32_t tile = blockIdx.x * (uint32_t)kFdGroup + threadIdx.x;
+  if (blockIdx.x * (uint32_t)kFdGroup >= tiles) return;
   const int p = blockIdx.y;
   uint32_t cnt = 0;
   if (tile < tiles) {
@@ -803,7 +806,7 @@ int zen_bitmap_dense_lists(const void *dict, int64_t numel, int partitions, cons
   const uint32_t tiles = fd_tiles(numel, partitions);
   const uint32_t groups = fd_groups(tiles);
   ProfScope prof(kProfDecodeFused, s);
-  k_fd_count<<<dim3(groups, (unsigned)partitions), dim3(kFdGroup), 0, s>>>(below, tiles, partitions, lists, vstart, gsum,
+  k_fd_count<<<dim3((groups + 7u) / 8u * 8u, (unsigned)partitions), dim3(kFdGroup), 0, s>>>(below, tiles, partitions, lists, vstart, gsum,
                                                                        status);
   ZEN_LAUNCH_CHECK("k_fd_count");
   k_fd_groups<<<dim3((unsigned)partitions), dim3(kFdGroupsMax), 0, s>>>(gsum, groups, partitions, lists, status);
