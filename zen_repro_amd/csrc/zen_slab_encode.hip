@@ -63,6 +63,10 @@ struct SlabTables {
 
 // Device-wide atomics on one 128-byte line are carried out one after the other: four counters to a line.
 constexpr uint32_t kMoveinPad = 8;
+// Losers beyond which the chains leave the moved-in entries to be counted from the map (k_slab_layout): a third of their
+// device-wide atomics less for 15 us of a launch that reads the map and lays out the output.  62 M slots, bf16: 436 000
+// losers 79 us, without the counting 49 and the launch 15; 110 000 losers 31 us, 18 of them latency that stays.
+constexpr uint32_t kUncountedFrom = 200000;
 
 // The counters and histograms that must be zero when a call starts live in memory that is zero between calls
 // (the part of the caller's table the hash map does not use), and every one of them is put back to zero by the
@@ -415,9 +419,9 @@ __device__ inline uint32_t slab_head(const SlabGeom &geo, const SlabTables &tb, 
 }
 
 // Enters t as a prober of `slot` in bucket b's part of the map; returns the smallest earlier prober (kNone: there was
-// none).  *full is set if the part has no room.
+// none).  *full is set if the part has no room.  counted: the part's entries are counted as they come.
 __device__ inline uint32_t part_min(unsigned long long *cells, const SlabTables &tb, uint32_t b, uint32_t slot, uint32_t t,
-                                    bool *full) {
+                                    bool counted, bool *full) {
   unsigned long long *part = cells + ((size_t)b << kSlabPartLog2);
   constexpr uint32_t mask = (1u << kSlabPartLog2) - 1u;
   const unsigned long long mine = ((unsigned long long)(slot + 1u) << 32) | t;
@@ -425,7 +429,7 @@ __device__ inline uint32_t part_min(unsigned long long *cells, const SlabTables 
   for (uint32_t probes = 0; probes <= mask; ++probes, h = (h + 1u) & mask) {
     const unsigned long long cur = atomicCAS(&part[h], 0ull, mine);
     if (cur == 0ull) {
-      atomicAdd(&tb.movein_n[b * kMoveinPad], 1u);
+      if (counted) atomicAdd(&tb.movein_n[b * kMoveinPad], 1u);
       return kNone;
     }
     if ((uint32_t)(cur >> 32) == slot + 1u) return (uint32_t)atomicMin(&part[h], mine);
@@ -510,18 +514,20 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
 
 // Levels 2 and 3 for the indices that lost level 1, one per thread.  Bound by latency while losers are few (110 000: a
 // wave 15 us; a probe is four or five dependent trips to memory, the bucket's index, its records, the map) and by the
-// device-wide atomics, two or three a loser at 21 a nanosecond, when they are many (436 000: a wave 50 us).  Every loser
+// device-wide atomics, one or two a loser (two or three while the moved-in entries are counted) at 21 a nanosecond, when they
+// are many (436 000: 49 us, counted 79).  Every loser
 // has a thread of its own on a full chip: with the scalar registers the compiler takes by itself three workgroups fit a
 // compute unit, and the last of 851 began when the first had ended (93 us, with four 83).  Nothing is counted in one
 // place (62 M slots, 10 % taken, 300 000 losers: with one counter of the map's claims and one log of the owners pushed
 // out, whose entries another kernel classified afterwards, 338 + 220 us).
 __global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Probe g, SlabTables tb, unsigned long long *cells,
                                                             int64_t spp, uint32_t capacity, int64_t *__restrict__ splits,
-                                                            HostAnswer answer, int32_t *status) {
+                                                            uint32_t count_up_to, HostAnswer answer, int32_t *status) {
   __shared__ uint32_t s_scan[kSlabBlock / 64 + 1];
   __shared__ uint32_t s_start[kSlabMaxBuckets + 1];
   __shared__ bool s_last;
   uint32_t losers = load_fresh(tb.losers);
+  const bool counted = losers <= count_up_to;
   if (losers > tb.log_cap) losers = tb.log_cap;
   // workgroups without a loser are not waited for (one that starts after the last of the others has put the count
   // back to zero sees none either)
@@ -555,7 +561,7 @@ __global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Pro
         ++lv;
         continue;
       }
-      const uint32_t old = part_min(cells, tb, bucket, slot, cur, &full);
+      const uint32_t old = part_min(cells, tb, bucket, slot, cur, counted, &full);
       if (full) {
         atomicOr(status, ZEN_STAT_RETRY);
         break;
@@ -581,10 +587,43 @@ __global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Pro
       lv = lw + 1;
     }
   }
+  if (!counted) return;  // k_slab_layout counts, and lays out the output
   // the workgroup that finishes last knows every count and lays out the output
   wait_global_acks();
   __syncthreads();
   if (threadIdx.x == 0) s_last = done_last(tb.done, blockIdx.x, working);
+  __syncthreads();
+  if (s_last) slab_output_starts(geo, tb, s_scan, s_start, spp, capacity, splits, answer, status);
+}
+
+// Where the chains left the moved-in entries uncounted: a wave to a bucket counts what its part of the map holds (8 KB, a
+// read of the whole map), the last workgroup lays out the output.  Launched behind the chains where the sizes allow that
+// many losers; returns at once if they were counted after all (the layout has put their number back to zero).
+constexpr int kLayoutBuckets = kSlabBlock / 64;
+__global__ __launch_bounds__(kSlabBlock) void k_slab_layout(SlabGeom geo, SlabTables tb,
+                                                            const unsigned long long *__restrict__ cells, int64_t spp,
+                                                            uint32_t capacity, int64_t *__restrict__ splits,
+                                                            uint32_t count_up_to, HostAnswer answer, int32_t *status) {
+  __shared__ uint32_t s_scan[kSlabBlock / 64 + 1];
+  __shared__ uint32_t s_start[kSlabMaxBuckets + 1];
+  __shared__ bool s_last;
+  if (load_fresh(tb.losers) <= count_up_to) return;  // (nobody resets the number before every workgroup has counted)
+  const uint32_t b = blockIdx.x * (uint32_t)kLayoutBuckets + (threadIdx.x >> 6);
+  if (b < geo.nbuckets) {
+    constexpr int kLoads = (1 << kSlabPartLog2) / 128;
+    const u32x4 *part = reinterpret_cast<const u32x4 *>(cells + ((size_t)b << kSlabPartLog2)) + lane_id();
+    u32x4 two[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) two[i] = part[i * 64];
+    uint32_t n = 0;  // (a taken cell's upper half is its slot and one)
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) n += (two[i].y != 0u) + (two[i].w != 0u);
+    n = wave_sum(n);
+    if (lane_id() == 0) __hip_atomic_store(&tb.movein_n[b * kMoveinPad], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  wait_global_acks();
+  __syncthreads();
+  if (threadIdx.x == 0) s_last = done_last(tb.done, blockIdx.x, gridDim.x);
   __syncthreads();
   if (s_last) slab_output_starts(geo, tb, s_scan, s_start, spp, capacity, splits, answer, status);
 }
@@ -975,9 +1014,16 @@ int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPl
     ProfScope prof(kProfSlabChains, s);
     // (as many workgroups as the chip holds; fewer where there can be few losers)
     const int64_t groups = ceil_div((int64_t)p.tb.log_cap / 4, (int64_t)kSlabBlock);
+    const bool many = (double)a.capacity * (double)a.capacity > 2.0 * (double)geo.m * kUncountedFrom;
+    const uint32_t count_up_to = many ? kUncountedFrom : 0xffffffffu;
     k_slab_chains<<<dim3((unsigned)(groups < 64 ? 64 : groups > 1024 ? 1024 : groups)), dim3(kSlabBlock), 0, s>>>(
-        geo, a.g, p.tb, a.hash, a.spp, (uint32_t)a.capacity, a.splits, a.ask.answer, a.status);
+        geo, a.g, p.tb, a.hash, a.spp, (uint32_t)a.capacity, a.splits, count_up_to, a.ask.answer, a.status);
     ZEN_LAUNCH_CHECK("k_slab_chains");
+    if (many) {
+      k_slab_layout<<<dim3((B + kLayoutBuckets - 1) / kLayoutBuckets), dim3(kSlabBlock), 0, s>>>(
+          geo, p.tb, a.hash, a.spp, (uint32_t)a.capacity, a.splits, count_up_to, a.ask.answer, a.status);
+      ZEN_LAUNCH_CHECK("k_slab_layout");
+    }
     if (a.ask.answer.host) *a.ask.answered = true;
   }
   {
