@@ -137,72 +137,54 @@ struct SlabSortLds {
 // Sorts a bucket's records by level-1 slot; of those that share a slot the smallest index owns it, the others are
 // logged and not kept.  A bucket has a few to a few hundred slots per record, so the slots are marked in a bitmap: a
 // record's place is the number of marks below its own, and whoever finds its slot marked already is settled by the
-// smallest index afterwards.  Bound by the LDS round trips (six records a thread, two workgroups a compute unit) and by
-// the 12 to 16 bytes a record moves: 62 M slots, 6.2 M bf16 records 48 us, 3.1 M 24.  (By comparisons, k_slab_sort_wide:
-// 64 and 33.)
-template <typename S, uint32_t SPAN>
-__global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabTables tb, int32_t *status) {
-  __shared__ SlabSortLds<S, SPAN> sh;
+// smallest index afterwards.  Bound by the vector instructions and the LDS round trips behind every phase's barrier (two
+// workgroups a compute unit).  ROWS: records of a thread (the last row may be cut short); the code is written out for
+// each number, so that all marks and all look-ups of a phase are on their way together (with one body for all numbers
+// and branches around the rows a wave waited for every single mark): 62 M slots, 6.2 M bf16 records 46 -> 42 us, 3.1 M
+// 23.7 -> 21.5.  (By comparisons, k_slab_sort_wide: 64 and 33.)
+template <int ROWS, typename S, uint32_t SPAN>
+__device__ __forceinline__ void slab_sort_rows(SlabSortLds<S, SPAN> &sh, const SlabGeom &geo, const SlabTables &tb,
+                                               uint32_t n_raw, int32_t *status) {
   const uint32_t b = blockIdx.x;
   const size_t base = (size_t)b * kSlabCap;
   const uint32_t words = (geo.span + 63u) / 64u;
-  uint32_t n_raw = tb.cursor[b];
-  if (n_raw > (uint32_t)kSlabCap) n_raw = kSlabCap;  // the scatter flagged the overflow
   const uint32_t lo = tb.bucket_lo[b];
-  S *slab_val = static_cast<S *>(tb.slab_val);
-  if (threadIdx.x == 0) sh.shared = sh.lost = 0;
-  sh.taken.template clear<kSortBlock>(words);
-  // the kernels before this one were the last to need these: back to zero, a slice per workgroup
-  for (uint32_t i = b * kSortBlock + threadIdx.x; i < kCoarseCursorWords; i += gridDim.x * kSortBlock)
-    tb.coarse_cursor[i] = 0;
-  if (tb.refine_hist)
-    for (uint32_t i = b * kSortBlock + threadIdx.x; i < (uint32_t)kRefineWords; i += gridDim.x * kSortBlock)
-      tb.refine_hist[i] = 0;
-  uint32_t off[kSortItems], idx[kSortItems], rank[kSortItems];
-  S val[kSortItems];
+  const char *raw_idx = reinterpret_cast<const char *>(tb.raw_idx + base);
+  const char *raw_val = reinterpret_cast<const char *>(static_cast<const S *>(tb.raw_val) + base);
+  uint32_t off[ROWS], idx[ROWS], rank[ROWS];
+  S val[ROWS];
   uint32_t live = 0, owner = 0;
-  // rows past the records are left out (the same for the whole workgroup): a bucket is seldom more than half full, and
-  // the instructions for the other half cost 24 of 72 us
-  auto row = [&](int i) { return (uint32_t)(i * kSortBlock) < n_raw; };
 #pragma unroll
-  for (int i = 0; i < kSortItems; ++i) {
+  for (int i = 0; i < ROWS; ++i) {
     const uint32_t j = threadIdx.x + i * kSortBlock;
-    idx[i] = 0;
-    val[i] = 0;
-    if (!row(i)) continue;
     // no branch around a wave's loads (places past the end are pulled back onto the slab's first record): they are
     // all in flight together
-    const size_t from = base + (j < n_raw ? j : 0u);
-    idx[i] = tb.raw_idx[from];
-    val[i] = static_cast<const S *>(tb.raw_val)[from];
-    if (j < n_raw) live |= 1u << i;
+    const uint32_t from = j < n_raw ? j : 0u;
+    idx[i] = *reinterpret_cast<const uint32_t *>(raw_idx + (uint32_t)(from * sizeof(uint32_t)));
+    val[i] = *reinterpret_cast<const S *>(raw_val + (uint32_t)(from * sizeof(S)));
+    live |= (j < n_raw ? 1u : 0u) << i;
   }
   __syncthreads();  // the bitmap is clear, and everybody has read the slab's fill count
   if (threadIdx.x == 0) tb.cursor[b] = 0;
   // no branch around a wave's marks either: a lane without a record marks nothing
 #pragma unroll
-  for (int i = 0; i < kSortItems; ++i) {
-    off[i] = rank[i] = 0;
-    if (row(i)) {
-      off[i] = geo.mod_m(poly(idx[i]) + kSeed1) - lo;  // the level-1 slot again: cheaper than carrying it along
-      if (!(live & (1u << i))) off[i] = 0;
-      rank[i] = sh.taken.take(off[i], (live >> i) & 1u);
-    }
+  for (int i = 0; i < ROWS; ++i) {
+    off[i] = geo.mod_m(poly(idx[i]) + kSeed1) - lo;  // the level-1 slot again: cheaper than carrying it along
+    if (!(live & (1u << i))) off[i] = 0;
+    rank[i] = sh.taken.take(off[i], (live >> i) & 1u);
   }
 #pragma unroll
-  for (int i = 0; i < kSortItems; ++i)
-    if ((live & (1u << i)) && !((rank[i] >> (off[i] & 31u)) & 1u)) owner |= 1u << i;  // the first to mark its slot
+  for (int i = 0; i < ROWS; ++i) owner |= (~(rank[i] >> (off[i] & 31u)) & 1u) << i;  // the first to mark its slot
+  owner &= live;
   if (owner != live) sh.shared = 1;
   __syncthreads();
   const uint32_t n = sh.taken.template count<kSortBlock>(words, sh.scan);
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kSortItems; ++i) {
-    if (row(i)) {
-      rank[i] = sh.taken.place(off[i]);
-      if (owner & (1u << i)) sh.idx[rank[i]] = idx[i];
-    }
-  }
+  for (int i = 0; i < ROWS; ++i) rank[i] = sh.taken.place(off[i]);
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i)
+    if (owner & (1u << i)) sh.idx[rank[i]] = idx[i];
   // every kSlabIndexStep-th narrow range's first sorted place goes to the index
   for (int j = threadIdx.x; j < kSlabIndexLen; j += kSortBlock) {
     const uint32_t first = (uint32_t)j * kSlabIndexStep << geo.sub_shift;
@@ -211,18 +193,21 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabT
   __syncthreads();
   if (sh.shared) {  // (the same for the whole workgroup)
 #pragma unroll
-    for (int i = 0; i < kSortItems; ++i)
+    for (int i = 0; i < ROWS; ++i)
       if ((live & ~owner) & (1u << i)) atomicMin(&sh.idx[rank[i]], idx[i]);
     __syncthreads();
+    uint32_t own[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) own[i] = sh.idx[rank[i]];
     owner = 0;
 #pragma unroll
-    for (int i = 0; i < kSortItems; ++i)
-      if ((live & (1u << i)) && sh.idx[rank[i]] == idx[i]) owner |= 1u << i;
+    for (int i = 0; i < ROWS; ++i) owner |= (own[i] == idx[i] ? 1u : 0u) << i;
+    owner &= live;
   }
   const uint32_t losers = live & ~owner;
   uint32_t at = losers ? atomicAdd(&sh.lost, (uint32_t)__popc(losers)) : 0u;
 #pragma unroll
-  for (int i = 0; i < kSortItems; ++i)
+  for (int i = 0; i < ROWS; ++i)
     if (owner & (1u << i)) sh.val[rank[i]] = val[i];  // (the bitmap has done its work)
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -230,14 +215,20 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabT
     tb.removed_n[b] = 0;
     sh.base = sh.lost ? atomicAdd(tb.losers, sh.lost) : 0u;
   }
-  for (uint32_t p = threadIdx.x; p < n; p += kSortBlock) {
-    tb.slab_idx[base + p] = (int32_t)sh.idx[p];
-    slab_val[base + p] = sh.val[p];
+  int32_t *slab_idx = tb.slab_idx + base;
+  S *slab_val = static_cast<S *>(tb.slab_val) + base;
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const uint32_t p = threadIdx.x + i * kSortBlock;
+    if (p < n) {
+      slab_idx[p] = (int32_t)sh.idx[p];
+      slab_val[p] = sh.val[p];
+    }
   }
   __syncthreads();
   at += sh.base;
 #pragma unroll
-  for (int i = 0; i < kSortItems; ++i) {
+  for (int i = 0; i < ROWS; ++i) {
     if (losers & (1u << i)) {
       if (at < tb.log_cap)
         tb.log_t[at] = idx[i];
@@ -245,6 +236,33 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabT
         atomicOr(status, ZEN_STAT_RETRY);
       ++at;
     }
+  }
+}
+
+template <typename S, uint32_t SPAN>
+__global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabTables tb, int32_t *status) {
+  __shared__ SlabSortLds<S, SPAN> sh;
+  const uint32_t b = blockIdx.x;
+  const uint32_t words = (geo.span + 63u) / 64u;
+  uint32_t n_raw = tb.cursor[b];
+  if (n_raw > (uint32_t)kSlabCap) n_raw = kSlabCap;  // the scatter flagged the overflow
+  if (threadIdx.x == 0) sh.shared = sh.lost = 0;
+  sh.taken.template clear<kSortBlock>(words);
+  // the kernels before this one were the last to need these: back to zero, a slice per workgroup
+  for (uint32_t i = b * kSortBlock + threadIdx.x; i < kCoarseCursorWords; i += gridDim.x * kSortBlock)
+    tb.coarse_cursor[i] = 0;
+  if (tb.refine_hist)
+    for (uint32_t i = b * kSortBlock + threadIdx.x; i < (uint32_t)kRefineWords; i += gridDim.x * kSortBlock)
+      tb.refine_hist[i] = 0;
+  static_assert(kSortItems == 6, "a case for every number of rows");
+  switch ((n_raw + kSortBlock - 1) / kSortBlock) {
+    case 0:
+    case 1: slab_sort_rows<1>(sh, geo, tb, n_raw, status); break;
+    case 2: slab_sort_rows<2>(sh, geo, tb, n_raw, status); break;
+    case 3: slab_sort_rows<3>(sh, geo, tb, n_raw, status); break;
+    case 4: slab_sort_rows<4>(sh, geo, tb, n_raw, status); break;
+    case 5: slab_sort_rows<5>(sh, geo, tb, n_raw, status); break;
+    default: slab_sort_rows<6>(sh, geo, tb, n_raw, status); break;
   }
 }
 
