@@ -651,7 +651,10 @@ __global__ __launch_bounds__(kSlabBlock) void k_slab_layout(SlabGeom geo, SlabTa
 // A bucket's part of the output is its taken slots in order: the owners that nobody pushed out and the entries that moved
 // in.  Both are marked in a bitmap of the slots, and an entry goes to the bucket's start plus the number of marks below
 // its own.  Consecutive lanes read consecutive entries and write (almost) consecutive places.  62 M slots, 6.2 M records,
-// 5 % moved: 48 us (k_slab_place_wide, which counts removed and moved-in entries: 63).
+// 7 % moved: 34 us (k_slab_place_wide, which counts removed and moved-in entries: 63).
+// A partition's overflow entries are a workgroup's own, the first of the launch: sorting them takes longer than placing a
+// bucket, and as a part of the partition's last bucket it kept the chip waiting (270 of them on each of 16 partitions, the
+// call below: 46 us).
 template <uint32_t SPAN>
 struct SlabPlaceLds {
   union {
@@ -661,18 +664,47 @@ struct SlabPlaceLds {
   uint32_t scan[kSlabBlock / 64 + 1];
 };
 
+// The workgroups in front of the buckets': one for every partition, to a multiple of the eight dies, so that a bucket
+// stays on the die that sorted it.
+__host__ __device__ inline uint32_t slab_place_lead(uint32_t partitions) { return (partitions + 7u) & ~7u; }
+
+// A partition's overflow entries in ascending index order (the reference hands its tickets to ascending thread ids,
+// functions_cuda_kernel.cu:107-108), behind everything that found a slot.
+template <typename S>
+__device__ inline void slab_place_serial(uint32_t *s_serial, const SlabGeom &geo, const SlabTables &tb, uint32_t part,
+                                         const S *__restrict__ dense, int32_t *__restrict__ out_idx,
+                                         S *__restrict__ out_val, uint32_t capacity) {
+  uint32_t serial = tb.final_n[geo.nbuckets + part];
+  if (serial > (uint32_t)kSlabSerialCap) serial = kSlabSerialCap;
+  if (serial == 0) return;
+  const uint32_t first = tb.out_start[(part + 1u) * geo.bpp] - serial;
+  for (uint32_t i = threadIdx.x; i < serial; i += kSlabBlock) s_serial[i] = tb.ser_idx[(size_t)part * kSlabSerialCap + i];
+  __syncthreads();
+  sort_network(s_serial, serial);
+  for (uint32_t i = threadIdx.x; i < serial; i += kSlabBlock) {
+    if (first + i < capacity) {
+      out_idx[first + i] = (int32_t)s_serial[i];
+      out_val[first + i] = dense[s_serial[i]];
+    }
+  }
+}
+
 template <typename S, uint32_t SPAN>
 __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, SlabTables tb, unsigned long long *cells,
                                                            const S *__restrict__ dense, int32_t *__restrict__ out_idx,
                                                            S *__restrict__ out_val, uint32_t capacity) {
   constexpr int kCells = (1 << kSlabPartLog2) / kSlabBlock;
   __shared__ SlabPlaceLds<SPAN> sh;
-  const uint32_t b = blockIdx.x;
-  const uint32_t B = geo.nbuckets;
+  const uint32_t lead = slab_place_lead((uint32_t)tb.partitions);
+  if (blockIdx.x < lead) {
+    if (blockIdx.x < (uint32_t)tb.partitions)
+      slab_place_serial(sh.serial, geo, tb, blockIdx.x, dense, out_idx, out_val, capacity);
+    return;
+  }
+  const uint32_t b = blockIdx.x - lead;
   const size_t base = (size_t)b * kSlabCap;
   const uint32_t words = (geo.span + 63u) / 64u;
   const S *slab_val = static_cast<const S *>(tb.slab_val);
-  const uint32_t *serial_n = tb.final_n + B;
   const uint32_t n = tb.bucket_n[b];
   // what the bucket's part of the map holds has moved in, and keeps to the thread that finds it; the part goes
   // back empty
@@ -719,7 +751,7 @@ __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, Slab
     }
   }
   __syncthreads();
-  const uint32_t own_n = sh.taken.template count<kSlabBlock>(words, sh.scan);  // survivors + moved-in
+  sh.taken.template count<kSlabBlock>(words, sh.scan);  // survivors + moved-in
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
@@ -738,27 +770,6 @@ __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, Slab
       if (pos < capacity) {
         out_idx[pos] = (int32_t)(uint32_t)moved[e];
         out_val[pos] = mval[e];
-      }
-    }
-  }
-  const uint32_t part = b / geo.bpp;
-  uint32_t serial = 0;
-  if (b % geo.bpp == geo.bpp - 1) {  // the partition's last bucket
-    serial = serial_n[part];
-    if (serial > (uint32_t)kSlabSerialCap) serial = kSlabSerialCap;
-  }
-  if (serial) {
-    // the partition's overflow entries in ascending index order (the reference hands its tickets to
-    // ascending thread ids, functions_cuda_kernel.cu:107-108), behind everything that found a slot
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < serial; i += kSlabBlock) sh.serial[i] = tb.ser_idx[(size_t)part * kSlabSerialCap + i];
-    __syncthreads();
-    sort_network(sh.serial, serial);
-    for (uint32_t i = threadIdx.x; i < serial; i += kSlabBlock) {
-      const uint32_t pos = out_base + own_n + i;
-      if (pos < capacity) {
-        out_idx[pos] = (int32_t)sh.serial[i];
-        out_val[pos] = dense[sh.serial[i]];
       }
     }
   }
@@ -1047,8 +1058,8 @@ int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPl
   {
     ProfScope prof(kProfSlabPlace, s);
     if constexpr (SPAN > 0)
-      k_slab_place<S, SPAN><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, dense, a.out_idx,
-                                                                 static_cast<S *>(a.out_val), (uint32_t)a.capacity);
+      k_slab_place<S, SPAN><<<dim3(slab_place_lead((uint32_t)p.tb.partitions) + B), dim3(kSlabBlock), 0, s>>>(
+          geo, p.tb, a.hash, dense, a.out_idx, static_cast<S *>(a.out_val), (uint32_t)a.capacity);
     else
       k_slab_place_wide<S><<<dim3(B), dim3(kSlabBlock), 0, s>>>(geo, p.tb, a.hash, dense, a.out_idx,
                                                                 static_cast<S *>(a.out_val), (uint32_t)a.capacity);
