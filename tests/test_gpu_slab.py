@@ -96,6 +96,35 @@ def test_slab_load_balance_bit_exact(zen, oracle, n, P, density, rehash, dtype):
     assert not tp._table(d.device, m).any()
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("P,density,room", [
+    (16, 0.2, 1.05),  # some 450 000 losers: the entries that moved in are counted behind the chains
+    (3, 0.16, 1.1),   # 203 000, just past the line
+    (16, 0.1, 2.0),   # 119 000 where the capacity has room for many: by the chains themselves
+])
+@pytest.mark.parametrize("fast_path", ["slabs"], indirect=True)
+def test_slab_load_balance_of_many_losers(zen, oracle, P, density, room, dtype):
+    from zen_repro_amd import _lib
+
+    n = ((1 << 24) + 160) // P * P  # (no power of two, where the hash has fewer collisions)
+    g = make_grad(oracle, n, density, dtype, seed=P)
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, 3)
+    capacity = int(len(idx_o) * room)
+    assert st_o == 0 and lb_path(zen, n, P, dtype, capacity) == SLAB
+    tp = zen.TensorPartition(P, 1, 3)
+    d = to_dev(g)
+    for rep in range(2):  # the second call finds the counters zero again
+        oi, ov, splits, status = tp.load_balance_flat(d, capacity=capacity, mode=_lib.MODE_FAST)
+        assert status.item() == 0
+        assert np.array_equal(to_np(splits), splits_o)
+        assert np.array_equal(to_np(oi)[:len(idx_o)], idx_o)
+        assert np.array_equal(to_np(ov)[:len(idx_o)], val_o)
+    indices, values, splits = tp.load_balance(d, capacity=capacity)  # the host is told by the last of these launches
+    assert np.array_equal(to_np(splits), splits_o)
+    assert np.array_equal(to_np(torch.cat(indices)), idx_o)
+    assert np.array_equal(to_np(torch.cat(values)), val_o)
+
+
 @pytest.mark.parametrize("n,P,density,rehash,room", [
     ((6 << 20) - 3, 3, 0.05, 3, 1.1),   # the largest owner tables, a tenth selected and little
     ((10 << 20) - 6, 16, 0.001, 3, 1.1),
