@@ -232,28 +232,7 @@ __device__ inline uint32_t sum_runs(const Shared &sh, uint32_t n, uint32_t (&k)[
     float acc = 0.0f;
     if (first < n && before_k == k[0] && after_k != before_k) {
       // the run began before this thread's places and ends here: find its head, sum up to the place in front of `first`
-      uint32_t head = first - 1;
-      while (head > 0) {
-        const uint32_t a0 = sh.key[head - 1];
-        const uint32_t a1 = sh.key[head >= 2 ? head - 2 : 0u];
-        const uint32_t a2 = sh.key[head >= 3 ? head - 3 : 0u];
-        const uint32_t a3 = sh.key[head >= 4 ? head - 4 : 0u];
-        if (a0 != before_k) break;
-        if (head < 2 || a1 != before_k) { head -= 1; break; }
-        if (head < 3 || a2 != before_k) { head -= 2; break; }
-        if (head < 4 || a3 != before_k) { head -= 3; break; }
-        head -= 4;
-      }
-      for (uint32_t u = head; u < first; u += 4) {
-        const float f0 = __uint_as_float(sh.tie[u]);
-        const float f1 = __uint_as_float(sh.tie[u + 1 < first ? u + 1 : u]);
-        const float f2 = __uint_as_float(sh.tie[u + 2 < first ? u + 2 : u]);
-        const float f3 = __uint_as_float(sh.tie[u + 3 < first ? u + 3 : u]);
-        acc += f0;
-        if (u + 1 < first) acc += f1;
-        if (u + 2 < first) acc += f2;
-        if (u + 3 < first) acc += f3;
-      }
+      acc = sum_run_before(sh.key, sh.tie, first, before_k);
     }
     uint32_t prev = before_k;
 #pragma unroll

@@ -62,8 +62,8 @@ struct WideMergeShared {
 // (at most sixteen) records stay in registers from their load to the end, and all loads are in flight together; of three
 // the loops' bodies handle the first kWmLanes registers of a set and then rotate the set, and the values are loaded at the
 // end (written out for 24 records the code would not fit the instruction cache, and every workgroup runs it once).  A
-// chain of trips to LDS and memory: 62 M bf16, 3.1 M entries, 256 buckets of two rounds 42.6 us to index lists and 55.0
-// dense, with the loops for those too 48.2 and 59.0; 9 M, 0.9 M entries, one round 26.8 and 32.4.
+// chain of trips to LDS and memory: 62 M bf16, 3.1 M entries, 256 buckets of two rounds 39.2 us to index lists and 52.1
+// dense (42.6 and 55.0 at the time, with the loops for those too 48.2 and 59.0); 9 M, 0.9 M entries, one round 26.8 and 32.4.
 template <typename S, int ROUNDS, typename Zero>
 __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &geo, const WideSlabs &in, uint32_t b,
                                            const uint32_t (&pcount)[kWideSplit], uint32_t longest, bool declined,
@@ -253,14 +253,7 @@ __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &
     for (uint32_t e = tid; e < pending; e += kWideBlock) {
       const uint32_t p = sh.queue[e] & 0x3fffu, sub = sh.queue[e] >> 14;
       const uint32_t g0 = sh.cnt.start_of(sub), g1 = sh.cnt.end_of(sub);
-      const uint32_t my = sh.word[p];
-      uint32_t less = 0;
-      for (uint32_t u = g0; u < g1; u += 4) {
-        const uint32_t last = g1 - 1u;
-        const uint32_t a0 = sh.word[u], a1 = sh.word[u + 1 < last ? u + 1 : last];
-        const uint32_t a2 = sh.word[u + 2 < last ? u + 2 : last], a3 = sh.word[u + 3 < last ? u + 3 : last];
-        less += (a0 < my) + (u + 1 < g1 && a1 < my) + (u + 2 < g1 && a2 < my) + (u + 3 < g1 && a3 < my);
-      }
+      const uint32_t less = count_less(sh.word, g0, g1, sh.word[p]);
       sh.queue[e] = g0 + less;  // the entry's thread is its only reader
     }
     __syncthreads();
@@ -402,9 +395,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
     float acc = 0.0f;
     if (first < n && before_k == k[0]) {
       // the run began before this thread's places: find its head, sum up to the place in front of `first`
-      uint32_t head = first - 1;
-      while (head > 0 && sh.key[head - 1] == before_k) --head;
-      for (uint32_t u = head; u < first; ++u) acc += sh.val[u];
+      acc = sum_run_before(sh.key, sh.val, first, before_k);
     }
     uint32_t prev = before_k;
 #pragma unroll
