@@ -485,6 +485,29 @@ def test_slab_merge_bit_exact(zen, oracle, n, peers, per_peer, overlap, dtype, i
     assert np.array_equal(to_np(dense), oracle.f32_to_bf16_bits(f32) if dtype == "bf16" else f32)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("times", [2, 3, 4, 5, 6, 7, 8, 9, 11, 16, 17, 37])
+def test_merge_of_groups_of_every_length(zen, oracle, times, dtype):
+    """Every index comes `times` times, and one in three once: groups are ranked, and runs that began in front of a
+    thread's records summed, four records at a time."""
+    from zen_repro_amd import _lib
+
+    n, r = (1 << 23) + 3, 200000
+    rng = np.random.default_rng(times)
+    ci = np.concatenate([np.tile(rng.integers(0, n, r * 2 // 3 // times), times), rng.integers(0, n, r // 3)])
+    rng.shuffle(ci)
+    cv = (rng.standard_normal(len(ci)) * 1e-3).astype(np.float32)
+    if dtype == "bf16":
+        cv = oracle.f32_to_bf16_bits(cv)
+    assert on_fast_path(_lib.lib().zen_merge_path(len(ci), n, _lib.MODE_FAST | FLAGS))
+    want_i, want_v = oracle.merge_sparse(ci, cv, n)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    gi, gv, cnt, st = lba.merge_sparse_flat(to_dev(ci), to_dev(cv), n, mode=_lib.MODE_FAST)
+    assert st.item() == 0 and cnt.item() == len(want_i)
+    assert np.array_equal(to_np(gi)[:len(want_i)], want_i.astype(np.int32))
+    assert np.array_equal(to_np(gv)[:len(want_i)].view(np.uint32), want_v.view(np.uint32))
+
+
 @pytest.mark.parametrize("r", [1 << 19, (1 << 19) + 1, 1900000, 128 * 15360 + 1])
 def test_merge_that_waits_gives_the_same_on_half_and_all_of_the_chip(zen, oracle, r):
     """One list of r entries around the sizes where the number of wide buckets changes, against merge_sparse_flat."""
