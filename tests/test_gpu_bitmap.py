@@ -339,6 +339,25 @@ def test_bitmaps_to_dense_at_the_edges_of_the_dictionary(zen, oracle, n, P, dtyp
         assert np.array_equal(to_np(got), _dense_truth(oracle, n, idx, val)), share
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_bitmaps_to_dense_with_a_dictionary_that_leaves_the_tile(zen, oracle, dtype):
+    """Distances that add up to places beyond the tile are refused, and nothing but the tensor suffers."""
+    n, P = 3 * 7168, 2
+    mp, idx, val = _shards(oracle, n, P, 0.4, dtype, seed=5)
+    bitmaps = [to_dev(oracle.bitmap_encode(mp[p], idx[p])) for p in range(P)]
+    values = [to_dev(v) for v in val]
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P, 0), None, None)
+    want = _dense_truth(oracle, n, idx, val)
+    assert np.array_equal(to_np(lba.decode_bitmaps_dense(bitmaps, values, n)), want)
+    dictionary = lba._dense_dicts[n]
+    kept = dictionary.clone()
+    dictionary[:n].fill_(255)  # the distances lie in front
+    with pytest.raises(IndexError):
+        lba.decode_bitmaps_dense(bitmaps, values, n)
+    dictionary.copy_(kept)
+    assert np.array_equal(to_np(lba.decode_bitmaps_dense(bitmaps, values, n)), want)
+
+
 @pytest.mark.parametrize("form", ["strided values", "two value types"])
 def test_bitmaps_to_dense_with_values_in_any_layout(zen, oracle, form):
     """Value lists that are not contiguous, or of two types (the dense tensor then has the one that holds both)."""

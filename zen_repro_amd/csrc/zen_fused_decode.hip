@@ -589,6 +589,14 @@ __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
     a.hi = a.bitmap[at1];
     return a;
   };
+  // Places are sums of the dictionary's distances, and the dictionary is the caller's memory: one that this library did not
+  // build for these sizes must not reach beyond the tile in LDS.  (134 M bf16 elements, sixteen lists, 10 % set: 117 us
+  // with and without.)
+  uint32_t last_place = 0;
+  auto put_one = [&](uint32_t place, S v) {
+    last_place = last_place > place ? last_place : place;
+    s_tile[place < (uint32_t)kFdByteTile ? place : 0u] = v;
+  };
   Asked next{};
   if ((uint32_t)wave < nchunks && !odd) next = ask((uint32_t)wave);
 #pragma unroll 1
@@ -676,7 +684,7 @@ __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
 #pragma unroll
       for (int i = 0; i < kRows; ++i) {
         const uint32_t at = (uint32_t)(i * 64 + lane);
-        if (at < set) s_tile[list[at]] = v[i];
+        if (at < set) put_one(list[at], v[i]);
       }
       __builtin_amdgcn_wave_barrier();
     };
@@ -689,7 +697,7 @@ __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
   }
   __syncthreads();
   fd_write_tile<S, kFdByteTile, kBlock>(s_tile, tile_base, n.d, s_special != 0, dense);
-  if (odd && lane == 0) atomicOr(status, ZEN_STAT_BAD_INDEX);
+  if ((odd && lane == 0) || last_place >= (uint32_t)kFdByteTile) atomicOr(status, ZEN_STAT_BAD_INDEX);
 }
 
 // Dictionaries of bytes (see kFdByteLists), as long as their tiles' groups have a thread each in k_fd_groups (1.88e9 elements).
