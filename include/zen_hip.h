@@ -57,8 +57,9 @@ extern "C" {
  * 10: the dense dictionary of up to sixteen partitions holds a byte per
  *    element (zen_bitmap_dense_dict_bytes): built anew, not kept from an older
  *    library
+ * 11: such a dictionary's chunk words have 32 bits: built anew
  */
-#define ZEN_ABI_VERSION 10
+#define ZEN_ABI_VERSION 11
 
 #define ZEN_F32 0
 #define ZEN_BF16 1

@@ -313,21 +313,60 @@ def test_bitmaps_to_dense_in_one_pass_matches_oracle(zen, oracle, n, P, frac, dt
     assert np.array_equal(to_np(got), _dense_truth(oracle, n, idx, val))
 
 
+def _far_members(mapping):
+    """(list, number in the list) of the members 256 or more elements behind the one in front of them in their tile."""
+    return [(p, int(j) + 1) for p, m in enumerate(mapping)
+            for j in np.flatnonzero((np.diff(m) > 255) & (np.diff(m // 7168) == 0))]
+
+
+@pytest.mark.parametrize("several", [False, True])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("n, P", [(52974, 16), (141040, 16), (101419, 14)])
+def test_bitmaps_to_dense_across_far_members(zen, oracle, n, P, dtype, several):
+    """-0, a NaN and ordinary values in front of, at and behind a distance that does not fit its byte; the same with every
+    chunk marked as one with several such distances, whose places are hashed out."""
+    mp = oracle.mapping(n, P)
+    p, j = _far_members(mp)[0]
+    rng = np.random.default_rng(n)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P, 0), None, None)
+    for at in (j - 1, j, j + 1):
+        for bits, quiet in ((0x80000000, 0), (0x7f810000, 0x7fc10000), (0xffc00000, 0xffc00000), (0x3f800000, 0x3f800000)):
+            for share in (1.0, 0.3, 0.02):
+                pick = [rng.random(len(m)) < share for m in mp]
+                pick[p][[j - 1, j, j + 1]] = at == np.array([j - 1, j, j + 1])
+                idx = [m[t] for m, t in zip(mp, pick)]
+                val = [(rng.standard_normal(len(i)) + 9.0).astype(np.float32).view(np.uint32) & 0xffff0000 for i in idx]
+                val[p][np.flatnonzero(idx[p] == mp[p][at])] = bits
+                want = np.zeros(n, np.uint32)
+                for i, v in zip(idx, val):
+                    want[i] = v
+                want[mp[p][at]] = quiet
+                bitmaps = [to_dev(oracle.bitmap_encode(m, i)) for m, i in zip(mp, idx)]
+                values = [torch.from_numpy(v.view(np.int32)).cuda().view(torch.float32) for v in val]
+                if dtype == "bf16":
+                    values = [torch.from_numpy((v >> 16).astype(np.uint16).view(np.int16)).cuda().view(torch.bfloat16) for v in val]
+                    want >>= 16
+                got = lba.decode_bitmaps_dense(bitmaps, values, n)
+                if several:
+                    words = lba._dense_dicts[n][(n + 7167) // 7168 * 7296 + 512 + 255 & -256:].view(torch.int32)
+                    words[:(n + 7167) // 7168 * 32].bitwise_or_(0xc000)
+                    got = lba.decode_bitmaps_dense(bitmaps, values, n)
+                got = got.view(torch.int32 if dtype == "f32" else torch.int16).cpu().numpy()
+                assert np.array_equal(got.view(np.uint32 if dtype == "f32" else np.uint16), want), (at - j, bits, share)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("n, P", [
     (7679, 1), (7168, 2), (7681, 3), (2 * 7168 + 1, 16), (8191, 16), (8193, 17), (3 * 7168 - 1, 15),  # edges of the tiles
     (1030, 2), (16 * 8 + 5, 16), (100, 16),                      # lists of a chunk of 512 and a few more; of a few members
-    (83381, 16), (141040, 16), (167428, 15),                     # a list with two members 256 or more elements apart
+    (52974, 16), (83381, 16), (141040, 16), (167428, 15),        # a list with two members 256 or more elements apart
 ])
 def test_bitmaps_to_dense_at_the_edges_of_the_dictionary(zen, oracle, n, P, dtype):
     """Every member set (lists end with their values), every other one, few and none, exact."""
     mp = oracle.mapping(n, P)
     rng = np.random.default_rng(n)
-    if n > 80000:
-        tile = [m // 7168 for m in mp]
-        far = [np.diff(np.concatenate([[-1], m % 7168 if len(m) else m])) for m in mp]
-        same = [np.concatenate([[True], np.diff(t) == 0]) for t in tile]
-        assert any((f[s] > 255).any() for f, s in zip(far, same))
+    if n > 50000:
+        assert _far_members(mp)
     lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P, 0), None, None)
     for share in (1.0, 0.5, 0.03, 0.0):
         idx = [m[rng.random(len(m)) < share] if share < 1 else m for m in mp]

@@ -42,7 +42,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("ZEN_HIP_LIB") or os.path.join(_HERE, "csrc", "libzen_hip.so")
 
 # ZEN_ABI_VERSION of include/zen_hip.h this loader's signatures and structs are written for
-ABI_VERSION = 10
+ABI_VERSION = 11
 TABLE_SIZES_MOST = 1024  # ZEN_TABLE_SIZES_MOST
 
 _lib = None

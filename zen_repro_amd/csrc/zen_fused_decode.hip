@@ -24,19 +24,21 @@ constexpr int kFdMaxLists = 64;
 
 // Dictionaries of bytes: a member's place is that of the member in front of it in its list plus a byte, which takes half
 // the memory of places of 16 bits.  The members of a list lie as far apart as there are lists, give or take: up to
-// sixteen lists one distance in ten million does not fit a byte (a chunk with such a one is marked, and its places are
-// found by hashing), at 32 lists one in three thousand and at 64 one in fifty, so that nearly every tile would have
-// some.  A lane takes eight members, a chunk is what a wave takes, and seven eighths of 8192 elements to a tile
-// keep the lists' shares under whole chunks: at sixteen lists 448 members, give or take 20.
+// sixteen lists one distance in ten million does not fit a byte (its chunk's word holds it), at 32 lists one in three
+// thousand and at 64 one in fifty, so that nearly every tile would have some.  A lane takes eight members, a chunk is
+// what a wave takes, and seven eighths of 8192 elements to a tile keep the lists' shares under whole chunks: at sixteen
+// lists 448 members, give or take 20.
 constexpr int kFdByteLists = 16;
 constexpr int kFdByteTile = 7168;
 constexpr int kFdLane = 8;                               // members a lane takes
 constexpr int kFdByteChunk = 64 * kFdLane;
 constexpr int kFdByteRow = kFdByteTile + kFdLane * kFdByteLists;  // bytes of a tile: lists begin at multiples of kFdLane
-constexpr int kFdByteChunks = 32;                        // 16-bit words of a tile's chunk table
-constexpr uint32_t kFdHashed = 0x8000u;                  // in a chunk's word: its places are found by hashing
+constexpr int kFdByteChunks = 32;                        // words of a tile's chunk table
+// A chunk's word: the place of its first member; kFdFar if another of its members lies 256 or more behind the one in front
+// of it (its byte is zero), and in the upper half how far; kFdSeveral if more than one does.
+constexpr uint32_t kFdPlace = 0x1fffu, kFdFar = 0x8000u, kFdSeveral = 0x4000u;
 static_assert(kFdByteTile / kFdByteChunk + kFdByteLists <= kFdByteChunks, "every chunk of a tile has a word");
-static_assert(kFdByteTile % (16 * kFdBlock / 64) == 0 && kFdByteTile < (1 << 14) && kFdByteRow % 16 == 0, "tile layout");
+static_assert(kFdByteTile % (16 * kFdBlock / 64) == 0 && kFdByteTile <= (int)kFdPlace + 1 && kFdByteRow % 16 == 0, "tile layout");
 constexpr int kFdChunk = 16;                  // thread columns whose counts one thread adds up
 constexpr int kFdChunks = kFdBlock / kFdChunk;
 constexpr int kFdChunkRow = kFdChunks + 8;   // 16-bit words per list in the chunk table (rows stay 16-byte aligned)
@@ -66,12 +68,11 @@ __device__ inline uint32_t part_of(uint32_t t, FdDivisor n, FdDivisor npp) {  //
 // Dictionary, step 1: per tile the places of its indices ordered by partition, and the number of indices of
 // every partition.  Every thread counts, for its consecutive indices, how many belong to each list; prefix sums over
 // the threads, in two levels (chunks of 16 threads, then the 32 chunks), give every index its rank inside its list.
-// BYTES: `order` holds distances (kFdByteRow bytes a tile, lists padded to whole lanes) and chunk_at, per chunk of a
-// list's members, the first place behind the member in front of the chunk, with kFdHashed where a distance does not
-// fit.  Else 16-bit places, kFdTile a tile.  Dynamic LDS: fd_order_lds.
+// BYTES: `order` holds distances (kFdByteRow bytes a tile, lists padded to whole lanes; a chunk's first is one) and
+// chunk_at a word per chunk of a list's members (kFdPlace).  Else 16-bit places, kFdTile a tile.  Dynamic LDS: fd_order_lds.
 template <bool BYTES>
 __global__ __launch_bounds__(kFdBlock) void k_fd_order(FdDivisor n, FdDivisor npp, int P, void *__restrict__ order,
-                                                      uint16_t *__restrict__ chunk_at, uint32_t *__restrict__ below) {
+                                                      uint32_t *__restrict__ chunk_at, uint32_t *__restrict__ below) {
   constexpr int kTile = BYTES ? kFdByteTile : kFdTile;
   constexpr int kPer = kTile / kFdBlock;  // consecutive indices per thread
   extern __shared__ __attribute__((aligned(16))) uint16_t s_cnt[];  // [P][kFdBlock]
@@ -153,8 +154,8 @@ __global__ __launch_bounds__(kFdBlock) void k_fd_order(FdDivisor n, FdDivisor np
   if constexpr (BYTES) {
     uint16_t *s_place = &s_chunk[P][0];                                   // [kFdByteRow]
     uint8_t *s_byte = reinterpret_cast<uint8_t *>(s_place + kFdByteRow);  // [kFdByteRow]
-    __shared__ uint32_t s_at[kFdByteChunks];
-    if (threadIdx.x < kFdByteChunks) s_at[threadIdx.x] = 0;
+    __shared__ uint32_t s_at[kFdByteChunks], s_far[kFdByteChunks];
+    if (threadIdx.x < kFdByteChunks) s_at[threadIdx.x] = s_far[threadIdx.x] = 0;
     // what pads a list to whole lanes belongs to nobody
     for (int i = threadIdx.x; i < kFdByteRow / 4; i += kFdBlock) reinterpret_cast<uint32_t *>(s_byte)[i] = 0x01010101u;
 #pragma unroll
@@ -166,17 +167,21 @@ __global__ __launch_bounds__(kFdBlock) void k_fd_order(FdDivisor n, FdDivisor np
       const uint32_t p = part[e];
       if (p >= (uint32_t)P) continue;
       const uint32_t at = s_base[p] + rank[e], place = threadIdx.x * kPer + e;
-      const uint32_t from = rank[e] ? s_place[at - 1] + 1u : 0u;  // the first place it could have had
       const uint32_t chunk = s_first[p] + rank[e] / kFdByteChunk;
-      const uint32_t far = place - from > 254u ? kFdHashed : 0u;
-      s_byte[at] = (uint8_t)(far ? 0u : place - from + 1u);
-      const uint32_t word = far | (rank[e] % kFdByteChunk == 0 ? from : 0u);
-      if (word) atomicOr(&s_at[chunk], word);
+      if (rank[e] % kFdByteChunk == 0) {
+        s_byte[at] = 1;
+        atomicOr(&s_at[chunk], place);
+        continue;
+      }
+      const uint32_t far = place - s_place[at - 1];
+      s_byte[at] = (uint8_t)(far < 256u ? far : 0u);
+      if (far >= 256u) atomicOr(&s_at[chunk], atomicCAS(&s_far[chunk], 0u, far) ? kFdFar | kFdSeveral : kFdFar);
     }
     __syncthreads();
     uint4 *row = reinterpret_cast<uint4 *>(static_cast<uint8_t *>(order) + (size_t)blockIdx.x * kFdByteRow);
     for (int i = threadIdx.x; i < kFdByteRow / 16; i += kFdBlock) row[i] = reinterpret_cast<const uint4 *>(s_byte)[i];
-    if (threadIdx.x < kFdByteChunks) chunk_at[(size_t)blockIdx.x * kFdByteChunks + threadIdx.x] = (uint16_t)s_at[threadIdx.x];
+    if (threadIdx.x < kFdByteChunks)
+      chunk_at[(size_t)blockIdx.x * kFdByteChunks + threadIdx.x] = s_at[threadIdx.x] | s_far[threadIdx.x] << 16;
   }
 }
 
@@ -530,7 +535,7 @@ __global__ __launch_bounds__(fd_tile_block<S>(), sizeof(S) == 2 ? 6 : 8) void k_
 // of a wave under way together, all their loads in front (registers: 209 at six waves a SIMD, 20 more at eight).
 template <typename S>
 __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
-    const uint8_t *__restrict__ order, const uint16_t *__restrict__ chunk_at, const uint32_t *__restrict__ below,
+    const uint8_t *__restrict__ order, const uint32_t *__restrict__ chunk_at, const uint32_t *__restrict__ below,
     const uint32_t *__restrict__ vstart, const uint32_t *__restrict__ gpre, int P, FdDivisor n, FdDivisor npp, FdLists lists,
     S *__restrict__ dense, int32_t *status) {
   constexpr int kBlock = fd_tile_block<S>();
@@ -640,7 +645,7 @@ __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
     }
     if (set == 0) continue;
     const char *val = now.val + (size_t)nth * sizeof(S);
-    if (start & kFdHashed) {  // a distance that does not fit its byte: whose the places are is hashed out
+    if (start & kFdSeveral) {  // several distances that do not fit their bytes: whose the places are is hashed out
       uint32_t seen = 0;
       for (uint32_t t0 = 0; t0 < (uint32_t)kFdByteTile; t0 += 64) {
         const uint32_t t = t0 + (uint32_t)lane;
@@ -656,9 +661,22 @@ __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
       }
       continue;
     }
+    // One that does not fit, of the member whose byte is zero: its lane adds the distance to the places that it has listed
+    // from there on, the lanes behind it begin that much further.  (Hashed out like several, one such chunk of a call cost
+    // 15 to 20 us where it came late: sixteen lists, 141 040 elements 35 us and 16 so, 16.8 M fp32 55 and 35, 134 M bf16
+    // with eight of them 118 and 107.)
+    auto far_member = [&] {  // kFdLane: none of this lane's
+      const uint32_t zx = (far.x - 0x01010101u) & ~far.x & 0x80808080u, zy = (far.y - 0x01010101u) & ~far.y & 0x80808080u;
+      const uint32_t i = zx ? (uint32_t)__ffs((int)zx) / 8u - 1u : zy ? (uint32_t)__ffs((int)zy) / 8u + 3u : (uint32_t)kFdLane;
+      return before + i < members ? i : (uint32_t)kFdLane;
+    };
+    uint32_t front = (start & kFdPlace) + ((all - mine) & 0x3ffffu) - 1u;
+    if (start & kFdFar) {
+      const int who = __ffsll(__ballot(far_member() < (uint32_t)kFdLane));  // and one
+      if (who && lane >= who) front += start >> 16;
+    }
     // The places of those that have a value are listed in its order, and the values go there with consecutive lanes on
     // consecutive values: a lane that fetches its own members' reads the same lines as its neighbours eight times over.
-    const uint32_t front = (start & (kFdHashed - 1u)) + ((all - mine) & 0x3ffffu) - 1u;
     auto put = [&](auto rows) {
       constexpr int kRows = decltype(rows)::value;
       S v[kRows];
@@ -676,6 +694,11 @@ __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
         if (mark < 0) *to++ = (uint16_t)place;
         mark <<= 1;
       }
+      if (kRows == kFdLane && (start & kFdFar)) {
+        const uint32_t i = far_member();
+        if (i < (uint32_t)kFdLane)
+          for (uint16_t *e = list + k + (uint32_t)__popc(bits & ((1u << i) - 1u)); e < to; ++e) *e = (uint16_t)(*e + (start >> 16));
+      }
       __builtin_amdgcn_wave_barrier();
       bool special = false;
 #pragma unroll
@@ -688,7 +711,9 @@ __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
       }
       __builtin_amdgcn_wave_barrier();
     };
-    if (set <= 64u)
+    if (start & kFdFar)
+      put(std::integral_constant<int, kFdLane>{});
+    else if (set <= 64u)
       put(std::integral_constant<int, 1>{});
     else if (set <= 128u)
       put(std::integral_constant<int, 2>{});
@@ -711,7 +736,7 @@ inline size_t fd_order_bytes(int64_t numel, int P) {
   return align_up(fd_of_bytes(numel, P) ? tiles * kFdByteRow + kFdByteChunk : (tiles * kFdTile + kFdMembers) * sizeof(uint16_t), 256);
 }
 inline size_t fd_chunk_bytes(int64_t numel, int P) {
-  return fd_of_bytes(numel, P) ? align_up((size_t)fd_tiles(numel, P) * kFdByteChunks * sizeof(uint16_t), 256) : 0;
+  return fd_of_bytes(numel, P) ? align_up((size_t)fd_tiles(numel, P) * kFdByteChunks * sizeof(uint32_t), 256) : 0;
 }
 inline size_t fd_table_bytes(int64_t numel, int P) { return align_up(((size_t)fd_tiles(numel, P) + 1) * P * sizeof(uint32_t), 256); }
 inline size_t fd_vstart_bytes(int64_t numel, int P) { return align_up((size_t)fd_tiles(numel, P) * P * sizeof(uint32_t), 256); }
@@ -729,7 +754,7 @@ void fd_launch_tiles(const void *dict, const uint8_t *chunk_at, const uint32_t *
                      int32_t *status, hipStream_t s) {
   const dim3 grid(tiles), block(fd_tile_block<S>());
   if (fd_of_bytes(numel, P))
-    k_fd_tiles_bytes<S><<<grid, block, 0, s>>>(static_cast<const uint8_t *>(dict), reinterpret_cast<const uint16_t *>(chunk_at),
+    k_fd_tiles_bytes<S><<<grid, block, 0, s>>>(static_cast<const uint8_t *>(dict), reinterpret_cast<const uint32_t *>(chunk_at),
                                                below, vstart, gsum, P, fd_divisor((uint32_t)numel), fd_divisor((uint32_t)(numel / P)), lists,
                                                static_cast<S *>(dense), status);
   else
@@ -762,7 +787,7 @@ int zen_bitmap_dense_dict(int64_t numel, int partitions, void *dict, int64_t *me
   if (lds > 32768)  // beyond what a launch may ask for without saying so first
     ZEN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(fill), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   fill<<<dim3(tiles), dim3(kFdBlock), lds, s>>>(fd_divisor((uint32_t)numel), fd_divisor((uint32_t)(numel / partitions)), partitions, dict,
-                                                reinterpret_cast<uint16_t *>(chunk_at), below);
+                                                reinterpret_cast<uint32_t *>(chunk_at), below);
   ZEN_LAUNCH_CHECK("k_fd_order");
   k_fd_scan<<<dim3((unsigned)partitions), dim3(kFdScanBlock), 0, s>>>(below, tiles, partitions);
   ZEN_LAUNCH_CHECK("k_fd_scan");
