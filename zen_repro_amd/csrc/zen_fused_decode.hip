@@ -717,6 +717,11 @@ __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
       put(std::integral_constant<int, 1>{});
     else if (set <= 128u)
       put(std::integral_constant<int, 2>{});
+    // (a quarter to half of a chunk set; by the eight rows of all those denser fp32 calls were slower than with places of
+    // 16 bits: 67 M fp32, us, with 16 bits, eight rows, four: sixteen lists, 45 % set 94, 98 and 94; eight, 48 % 111, 116
+    // and 114; four, 30 % 113, 118 and 116.  134 M bf16, sixteen lists, 45 %: 134, 124 and 118.)
+    else if (set <= 256u)
+      put(std::integral_constant<int, 4>{});
     else
       put(std::integral_constant<int, kFdLane>{});
   }
