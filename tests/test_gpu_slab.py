@@ -97,20 +97,28 @@ def test_slab_load_balance_bit_exact(zen, oracle, n, P, density, rehash, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
-@pytest.mark.parametrize("P,density,room", [
-    (16, 0.2, 1.05),  # some 450 000 losers: the entries that moved in are counted behind the chains
-    (3, 0.16, 1.1),   # 203 000, just past the line
-    (16, 0.1, 2.0),   # 119 000 where the capacity has room for many: by the chains themselves
+@pytest.mark.parametrize("P,density,room,losers", [
+    # where the entries that moved in are counted: by the chains up to 50 000 losers, behind them where there are more
+    # and the capacity has room for many
+    (16, 0.2, 1.05, 451039),
+    (3, 0.16, 1.1, 202997),
+    (16, 0.1, 2.0, 119306),
+    (3, 0.08, 2.0, 52072),    # just past the line
+    (3, 0.078, 2.1, 49630),   # just below it, with the launch behind the chains
+    (16, 0.1, 1.1, 119306),   # without it
 ])
 @pytest.mark.parametrize("fast_path", ["slabs"], indirect=True)
-def test_slab_load_balance_of_many_losers(zen, oracle, P, density, room, dtype):
+def test_slab_load_balance_of_many_losers(zen, oracle, P, density, room, losers, dtype):
     from zen_repro_amd import _lib
+    from zen_repro_amd.workloads import hash_slot
 
     n = ((1 << 24) + 160) // P * P  # (no power of two, where the hash has fewer collisions)
     g = make_grad(oracle, n, density, dtype, seed=P)
     idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, 3)
     capacity = int(len(idx_o) * room)
     assert st_o == 0 and lb_path(zen, n, P, dtype, capacity) == SLAB
+    assert len(idx_o) - torch.unique(hash_slot(torch.from_numpy(idx_o.astype(np.int64)), n)).numel() == losers
+    assert (capacity ** 2 / (2 * n) > 200000) == (room != 1.1 or P == 3)
     tp = zen.TensorPartition(P, 1, 3)
     d = to_dev(g)
     for rep in range(2):  # the second call finds the counters zero again

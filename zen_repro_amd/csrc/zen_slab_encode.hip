@@ -64,9 +64,15 @@ struct SlabTables {
 // Device-wide atomics on one 128-byte line are carried out one after the other: four counters to a line.
 constexpr uint32_t kMoveinPad = 8;
 // Losers beyond which the chains leave the moved-in entries to be counted from the map (k_slab_layout): a third of their
-// device-wide atomics less for 15 us of a launch that reads the map and lays out the output.  62 M slots, bf16: 436 000
-// losers 79 us, without the counting 49 and the launch 15; 110 000 losers 31 us, 18 of them latency that stays.
-constexpr uint32_t kUncountedFrom = 200000;
+// device-wide atomics less for a launch that reads the map and lays out the output.  62 M slots, bf16: 436 000 losers
+// 79 us, without the counting 49 and the launch 15.  Whole calls, counted by the chains and from the map, us: 62 M slots,
+// 45 000 losers 94 and 92, 100 000 122 and 119, 173 000 139 and 128, 394 000 200 and 183; 300 M, 71 000 losers 211 and
+// 211, 172 000 265 and 261; 1 G, 82 000 539 and 541.  (With the line at 200 000, calls of fewer losers had the
+// launch behind the chains and counted all the same: 1.3 to 2 us more than without it.)
+constexpr uint32_t kUncountedFrom = 50000;
+// The launch is there from this estimate of the losers on: n^2 / 2m of n = capacity entries in m slots.  The hash loses 1.4
+// times as many, at powers of two a third, and calls select from two thirds of their capacity to all of it.
+constexpr double kLayoutFrom = 200000;
 
 // The counters and histograms that must be zero when a call starts live in memory that is zero between calls
 // (the part of the caller's table the hash map does not use), and every one of them is put back to zero by the
@@ -615,8 +621,9 @@ __global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Pro
 }
 
 // Where the chains left the moved-in entries uncounted: a wave to a bucket counts what its part of the map holds (8 KB, a
-// read of the whole map), the last workgroup lays out the output.  Launched behind the chains where the sizes allow that
-// many losers; returns at once if they were counted after all (the layout has put their number back to zero).
+// read of the whole map), the last workgroup lays out the output.  Launched behind the chains where the capacity has room
+// for many losers (kLayoutFrom); returns at once if they were counted after all (the layout has put their number back
+// to zero).
 constexpr int kLayoutBuckets = kSlabBlock / 64;
 __global__ __launch_bounds__(kSlabBlock) void k_slab_layout(SlabGeom geo, SlabTables tb,
                                                             const unsigned long long *__restrict__ cells, int64_t spp,
@@ -1043,7 +1050,7 @@ int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPl
     ProfScope prof(kProfSlabChains, s);
     // (as many workgroups as the chip holds; fewer where there can be few losers)
     const int64_t groups = ceil_div((int64_t)p.tb.log_cap / 4, (int64_t)kSlabBlock);
-    const bool many = (double)a.capacity * (double)a.capacity > 2.0 * (double)geo.m * kUncountedFrom;
+    const bool many = (double)a.capacity * (double)a.capacity > 2.0 * (double)geo.m * kLayoutFrom;
     const uint32_t count_up_to = many ? kUncountedFrom : 0xffffffffu;
     k_slab_chains<<<dim3((unsigned)(groups < 64 ? 64 : groups > 1024 ? 1024 : groups)), dim3(kSlabBlock), 0, s>>>(
         geo, a.g, p.tb, a.hash, a.spp, (uint32_t)a.capacity, a.splits, count_up_to, a.ask.answer, a.status);
