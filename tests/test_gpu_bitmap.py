@@ -438,7 +438,8 @@ def test_bitmaps_to_dense_is_complete_for_every_stream(zen):
 
 
 @pytest.mark.parametrize("special", range(12))
-@pytest.mark.parametrize("n, P", [(8192, 1), (24576 + 80, 1), (3 * 8192 + 17, 3), (1 << 17, 16)])
+@pytest.mark.parametrize("n, P", [(8192, 1), (24576 + 80, 1), (3 * 8192 + 17, 3), (1 << 17, 16),
+                                  (3 * 8192 + 17, 17), (1 << 16, 64)])  # places of 16 bits
 def test_bitmaps_to_dense_special_values(zen, oracle, n, P, special):
     """0.0f + v for one element that needs it (-0, NaNs of either sign, quiet or not) and for those that do not, alone
     among ordinary ones, in whole tiles and in the last one; every member set, so that the values end with the list."""
@@ -458,8 +459,8 @@ def test_bitmaps_to_dense_special_values(zen, oracle, n, P, special):
     assert np.array_equal(got.view(torch.int16).cpu().numpy().view(np.uint16), want)
 
 
-def test_bitmaps_to_dense_edge_cases(zen, oracle):
-    n, P = 1 << 18, 8
+@pytest.mark.parametrize("n, P, n2, P2", [(1 << 18, 8, 100003, 4), (1 << 18, 32, 100003, 24), (8192 * 17, 17, 100003, 64)])
+def test_bitmaps_to_dense_edge_cases(zen, oracle, n, P, n2, P2):
     mp, idx, val = _shards(oracle, n, P, 0.1, "f32", seed=3)
     bitmaps = [oracle.bitmap_encode(mp[p], idx[p]) for p in range(P)]
     lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P, 0), None, None)
@@ -495,7 +496,6 @@ def test_bitmaps_to_dense_edge_cases(zen, oracle):
     with pytest.raises(IndexError):
         lba.decode_bitmaps_dense([to_dev(b) for b in bitmaps], [to_dev(v) for v in fewer], n)
     # n % P != 0: some indices belong to no list (hash_index gives P for them, functions_cuda_kernel.cu:172-175)
-    n2, P2 = 100003, 4
     part = oracle.hash_index(n2, P2)
     mp2 = oracle.mapping(n2, P2)
     rng = np.random.default_rng(8)
@@ -505,6 +505,46 @@ def test_bitmaps_to_dense_edge_cases(zen, oracle):
     lba2 = zen.LoadBalanceAllreduce(zen.LocalGroup(P2, 0), None, None)
     got = to_np(lba2.decode_bitmaps_dense([to_dev(b) for b in bm2], [to_dev(v) for v in val2], n2))
     assert np.array_equal(got, _dense_truth(oracle, n2, idx2, val2)) and (got[part == P2] == 0).all()
+
+
+@pytest.mark.parametrize("P", [1, 16])
+def test_bitmaps_to_dense_of_few_lists_beyond_the_bytes(zen, P):
+    """More elements than dictionaries of bytes serve: places of 16 bits, and at one list fifteen chunks to a tile, of
+    which the later ones begin behind what the earlier have set."""
+    from zen_repro_amd.workloads import hash_slot
+
+    n = (1024 * 256 * 7168 + 8192 + 40) // P * P
+    gen = torch.Generator(device="cuda").manual_seed(P)
+    step = 1 << 26
+    counts = [0] * P
+    where, bits, values = [[] for _ in range(P)], [[] for _ in range(P)], [[] for _ in range(P)]
+    for lo in range(0, n, step):
+        t = torch.arange(lo, min(n, lo + step), device="cuda")
+        part = hash_slot(t, n) // (n // P)
+        chosen = torch.rand(t.numel(), generator=gen, device="cuda") < 1e-6
+        if lo == 0 or lo + step >= n:  # three tiles in front, and the last ones, two thirds set
+            chosen |= (torch.rand(t.numel(), generator=gen, device="cuda") < 0.66) & ((t < 3 * 8192) | (t >= n - 2 * 8192 - 100))
+        for p in range(P):
+            mine = part == p
+            rank = torch.cumsum(mine, 0) - 1 + counts[p]
+            counts[p] += int(mine.sum())
+            at = mine & chosen
+            where[p].append(t[at])
+            bits[p].append(rank[at])
+        del t, part, chosen, mine, rank, at
+    bitmaps = []
+    for p in range(P):
+        where[p], rank = torch.cat(where[p]), torch.cat(bits[p]).cpu().numpy()
+        bitmap = np.zeros((counts[p] + 7) // 8, np.uint8)
+        np.bitwise_or.at(bitmap, rank >> 3, (1 << (rank & 7)).astype(np.uint8))
+        bitmaps.append(to_dev(bitmap))
+        values[p] = (torch.rand(where[p].numel(), generator=gen, device="cuda") + 1).to(torch.bfloat16)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P, 0), None, None)
+    got = lba.decode_bitmaps_dense(bitmaps, values, n)
+    assert got.numel() == n
+    for p in range(P):
+        assert torch.equal(got[where[p]], values[p])
+    assert sum(int(torch.count_nonzero(part)) for part in got.split(step)) == sum(v.numel() for v in values)
 
 
 # ---------------------------------------------------------- the DDP hook
