@@ -506,12 +506,13 @@ class LoadBalanceAllreduce:
         rank i's bitmap over partition i's index list and the values of its set
         bits in order; returns the dense tensor of `numel` elements in the
         values' dtype.  Neither the index lists nor self.mapping are needed: a
-        dictionary of two bytes per element (per tile of the dense tensor, the
-        places of its indices ordered by partition) is built on first use of a
-        `numel` and cached like the reference caches the mapping
-        (comm.py:132-134).  The call waits for the dense tensor and for what is
-        said about bitmaps and values that do not agree: any stream may read the
-        result and overwrite what it came from when the call has returned."""
+        dictionary of one byte per element, two for more than sixteen ranks
+        (per tile of the dense tensor, the places of its indices ordered by
+        partition), is built on first use of a `numel` and cached like the
+        reference caches the mapping (comm.py:132-134).  The call waits for the
+        dense tensor and for what is said about bitmaps and values that do not
+        agree: any stream may read the result and overwrite what it came from
+        when the call has returned."""
         if len(bitmap_indices) != self.partitions or len(values_tensors) != self.partitions:
             raise RuntimeError("decode_bitmaps_dense: one bitmap and one value list per rank")
         for t in bitmap_indices:

@@ -293,7 +293,8 @@ __global__ __launch_bounds__(kFdGroupsMax) void k_fd_groups(uint32_t *__restrict
 // Words of a chunk: sixteen lists have 512 members in a tile, few more than 576.  Tile kernel with 8, 9 and 10 words, us,
 // 134 M bf16: 2 lists 171, 161 and 158, 3 185, 152 and 155, 4 176, 163 and 166, 8 184, 160 and 163, 16 190, 123 and 127,
 // 24 156, 159 and 166, 32 190, 193 and 202, 64 318, 324 and 340; 67 M fp32: 2 112, 109 and 108, 4 124, 112 and 114, 16
-// 132, 100 and 101, 64 195, 203 and 212.
+// 132, 100 and 101, 64 195, 203 and 212.  (Up to sixteen lists come here beyond 1.88e9 elements only, fd_of_bytes: eight
+// words would gain 2 to 4 % from 24 lists on and lose 6 to 54 % there.)
 constexpr int kFdWords = 9;
 constexpr int kFdMembers = 64 * kFdWords;    // members of a chunk
 
@@ -407,16 +408,18 @@ __device__ inline void fd_clear_tile(S *s_tile) {
 // member has a value, a lane's value is the one numbered by the set bits below it, and its place in the tile is
 // the chunk's next entry of the dictionary, so that all loads are consecutive, nine of each kind in flight.  The
 // places written are put together in LDS and leave with full-width stores.
-// Bound by memory: two bytes of dictionary and one element of output per index, and the values.  62 M bf16 elements
-// on sixteen ranks, 71 % of them set, 0.34 GB: 73 us; 268 M elements, 11 % set, 1.13 GB: 241 us, 4.7 TB/s.
-// What a 64th of a chunk costs beside its loads counts too: places read without a look at the end of the list (the
+// For 17 to 64 lists, and fewer beyond 1.88e9 elements.  Bound by the work per chunk, of which more lists make more and
+// emptier ones: a decode of 134 M bf16 elements, 10 % set, takes 140 us with 17 lists (0.58 GB, 4.1 TB/s), 166 with 24, 201
+// with 32, 334 with 64; 67 M fp32 99, 113, 132 and 198.  The figures below are from the time when sixteen lists came here
+// too: 62 M bf16 elements, 71 % set, and 268 M, 11 % set (1.13 GB; 241 us in the end).
+// What a 64th of a chunk costs beside its loads counts: places read without a look at the end of the list (the
 // dictionary goes on behind it), values clamped only where they end, and 0.0f + v taken for what is written out as a
-// whole instead of each value: 260 -> 249 us; chunks of nine words instead of ten, of which two were past most lists'
-// ends, 241.  Slower: the bits by scalar loads (289; nine cache lines one after the other), the low bytes of the places
-// alone with the high ones counted from where they wrap (0.86 GB, 275: seven instructions more per word).
-// One SET bit per
-// thread and turn, looked up in staged copies of the tile's bytes and values, took 307 and 411 us; with each value's
-// load in a branch of its own, which makes the compiler wait for it there, this kernel took 129 and 428 (79 and 300 without).
+// whole instead of each value: 268 M 260 -> 249 us; chunks of nine words instead of ten, of which two were past most
+// lists' ends, 241.  Slower: the bits by scalar loads (289; nine cache lines one after the other), the low bytes of the
+// places alone with the high ones counted from where they wrap (0.86 GB, 275: seven instructions more per word).
+// One SET bit per thread and turn, looked up in staged copies of the tile's bytes and values, took 307 us for the 62 M
+// and 411 for the 268 M; with each value's load in a branch of its own, which makes the compiler wait for it there,
+// this kernel took 129 and 428 (79 and 300 without).
 // Waves of a workgroup meet at its two barriers, so small workgroups keep loads and stores going side by side as long
 // as their tiles' LDS lets a compute unit hold enough of them: 16 KB a tile for bf16, four waves (the all-reduce of
 // the 268 M elements 803 us; 837 with eight waves, 872 with two, 940 with sixteen), 32 KB for fp32, eight (200 M
@@ -526,13 +529,14 @@ __global__ __launch_bounds__(fd_tile_block<S>(), sizeof(S) == 2 ? 6 : 8) void k_
 // are one 8-byte load, their bits of the bitmap two bytes, and one prefix sum across the lanes gives every lane both the
 // place in front of its first member and the number of its first value.  The lanes list the places of their members that
 // have a value, in LDS, and the values go there with consecutive lanes on consecutive values.
-// Bound by the vector instructions (two thirds of the kernel's time) and by the three trips to memory of a tile; of the
-// bytes (0.86 GB for the 268 M elements below) it moves 4.1 TB a second.  bf16, sixteen lists, with places of 16 bits and
-// so, us: 268 M elements, 11 % set 245 and 209; the calls of 62 M, 71 % set 110 and 99; four lists, 134 M, 10 % 198 and 184;
-// fp32, sixteen lists, 67 M 119 and 120.  Slower: a lane that fetches the values of its own members (eight loads that
-// touch the same lines; 268 M: 316); tiles of 7680 elements, whose lists of 480 members go beyond a chunk in one case of
-// fifteen, and one of a tile's four waves takes five chunks where the others take four; 512 threads (40 more); four chunks
-// of a wave under way together, all their loads in front (registers: 209 at six waves a SIMD, 20 more at eight).
+// Bound by the three trips to memory of a tile, one after the other (743 M bf16 elements, sixteen lists, 6 % set: the
+// waves wait 60 % of their time), and by the vector instructions (475 a wave of a tile): 268 M bf16 elements, sixteen
+// lists, 11 % set, are 0.91 GB and a decode of 203 us, 4.5 TB a second (with places of 16 bits 249 us and 1.17 GB);
+// fd_of_bytes has more. Slower (figures from the kernel's first form, 209 us there): a lane that fetches the values of
+// its own members (eight loads that touch the same lines; 268 M: 316); tiles of 7680 elements, whose lists of 480
+// members go beyond a chunk in one case of fifteen, and one of a tile's four waves takes five chunks where the others
+// take four; 512 threads (40 more); four chunks of a wave under way together, all their loads in front (registers: 209
+// at six waves a SIMD, 20 more at eight).
 template <typename S>
 __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
     const uint8_t *__restrict__ order, const uint32_t *__restrict__ chunk_at, const uint32_t *__restrict__ below,
@@ -731,6 +735,13 @@ __global__ __launch_bounds__(fd_tile_block<S>(), 8) void k_fd_tiles_bytes(
 }
 
 // Dictionaries of bytes (see kFdByteLists), as long as their tiles' groups have a thread each in k_fd_groups (1.88e9 elements).
+// A decode with places of 16 bits and with bytes, us, 10 % and 70 % set.  134 M bf16: one list 167, 147 and 169, 164;
+// two 175, 154 and 177, 172; three 163, 144 and 165, 161; four 172, 155 and 175, 173; eight 169, 150 and 172, 168;
+// twelve 221, 192 and 224, 201; sixteen 132, 108 and 137, 129.  67 M fp32: one 117, 115 and 119, 124; two 116, 113 and
+// 118, 123; three 111, 110 and 114, 119; four 113, 112 and 116, 121; eight 109, 108 and 113, 117; twelve 137, 130 and
+// 139, 137; sixteen 89, 85 and 102, 102.  Up to 9 M elements bytes take 5 to 30 % less, and the dictionary is built in
+// three quarters to six sevenths of the time.  (fp32 of few lists with most of their members set loses up to 5 %: a
+// dictionary serves both types.)
 inline bool fd_of_bytes(int64_t numel, int P) {
   return P <= kFdByteLists && ceil_div(numel, kFdByteTile) <= (int64_t)kFdGroupsMax * kFdGroup;
 }

@@ -5,7 +5,7 @@
 // (functions_cuda_kernel.cu:97-167, tensor_load_balance.py:13-51).  Here the
 // select kernel leaves its candidates in 64 coarse slabs (a coarse slab = the
 // level-1 hash slots of a group of buckets; a bucket is a range of level-1
-// slots, zen_slab.h), and four short kernels finish the job:
+// slots, zen_slab.h), and four or five short kernels finish the job:
 //   k_fine_scatter  the coarse slabs, filtered by the exact threshold, go to the
 //                   bucket slabs, so that every store belongs to a long run;
 //   k_slab_sort     one workgroup per bucket: puts the bucket in the order of its
@@ -20,7 +20,10 @@
 //                   index's probe sequence).  Every bucket has a part of the map
 //                   of its own, so what finally moved into a bucket is what its
 //                   part holds; an index that ran out of levels goes to its
-//                   partition's serial list; split sizes;
+//                   partition's serial list; split sizes, unless the losers are
+//                   many:
+//   k_slab_layout   (where the capacity has room for many losers) counts what
+//                   moved into the buckets from the map; split sizes;
 //   k_slab_place    one workgroup per bucket: survivors and moved-in entries by
 //                   the same kind of bitmap to the bucket's place in the
 //                   partition-major output.
@@ -50,10 +53,10 @@ struct SlabTables {
   uint32_t *ser_idx;    // [P * kSlabSerialCap]
   uint32_t *log_t;      // [log_cap] indices that lost level 1
   uint32_t *out_start;  // [B + 1] where every bucket starts in the output
-  uint32_t *done;       // [kDoneWords] workgroups of k_slab_chains that have finished
+  uint32_t *done;       // [kDoneWords] workgroups of k_slab_chains (or k_slab_layout) that have finished
   uint32_t *final_n;    // [B + P] what k_slab_place needs of the counters above, copied by the last workgroup of
-                        // k_slab_chains before it puts them back to zero: moved-in entries per bucket, serial
-                        // entries per partition
+                        // k_slab_chains, or of k_slab_layout where that counts, before it puts them back to zero:
+                        // moved-in entries per bucket, serial entries per partition
   uint32_t *losers;     // [1] entries of log_t
   uint32_t *coarse_cursor;  // the feed's coarse cursors and, for an fp32 top-k, the refinement histogram (else
   uint32_t *refine_hist;    // null): k_slab_sort puts them back to zero
@@ -119,10 +122,10 @@ struct EncodeSink {
 // (k_slab_sort_wide, k_slab_place_wide) it goes with the records, whatever the width.  A bucket within the second width
 // takes the bitmap.  Where the buckets the records call for are wider, more of them are made for the bitmap's sake up
 // to kSlabSparse slots per record of the capacity.  bf16, sort + place + chains, bitmap and comparisons: 2^30 slots,
-// 10.7 M records 127 and 170 us, 7.5 M 111 and 113, 6.4 M 102 and 99, 5.4 M 100 and 82; 1 M on 1024 partitions 97 and
-// 44.  No number of buckets makes the widest tables fit (more than 1.34 G slots): a bitmap of nine 2^16 slots, one
-// workgroup to a compute unit, takes 216 us for 1.34 G slots and 6.7 M records, comparisons 106; 2.1 G slots and 4.3 M
-// records 216 and 75.
+// 10.7 M records 116 us and (at the time, the bitmap 127) 170, 7.5 M 104 and 104, 6.4 M 94 and 92, 5.4 M 91 and 78; 1 M on
+// 1024 partitions 87 and 40.  No number of buckets makes the widest tables fit (more than 1.34 G slots): a bitmap of nine
+// 2^16 slots, one workgroup to a compute unit, took 216 us for 1.34 G slots and 6.7 M records, comparisons 106 (99 now);
+// 2.1 G slots and 4.3 M records 216 and 75.
 constexpr uint32_t kSlabSpan1 = 1u << 17, kSlabSpan2 = 5u << 16;
 constexpr int64_t kSlabSparse = 128;
 
@@ -147,7 +150,7 @@ struct SlabSortLds {
 // workgroups a compute unit).  ROWS: records of a thread (the last row may be cut short); the code is written out for
 // each number, so that all marks and all look-ups of a phase are on their way together (with one body for all numbers
 // and branches around the rows a wave waited for every single mark): 62 M slots, 6.2 M bf16 records 46 -> 42 us, 3.1 M
-// 23.7 -> 21.5.  (By comparisons, k_slab_sort_wide: 64 and 33.)
+// 23.7 -> 21.5.  (By comparisons, k_slab_sort_wide: 64 and 33 at the time.)
 template <int ROWS, typename S, uint32_t SPAN>
 __device__ __forceinline__ void slab_sort_rows(SlabSortLds<S, SPAN> &sh, const SlabGeom &geo, const SlabTables &tb,
                                                uint32_t n_raw, int32_t *status) {
@@ -274,7 +277,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabT
 
 // The same for few records among many slots: grouped by narrow key ranges, ranked against the words of their group
 // (slab_rank), the owners found by walking the sorted runs.  Those that lost stay where they are, marked.  Bound by LDS
-// round trips: 1.48 G slots, 14.8 M bf16 records 107 us; 1.34 G and 6.7 M 54.
+// round trips: 1.48 G slots, 14.7 M bf16 records 98 us; 1.34 G and 6.7 M 50.
 template <typename S>
 __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort_wide(SlabGeom geo, SlabTables tb, int32_t *status) {
   // the ties take the place of the counters once the ranks are known: with 32-bit values the kernel would
@@ -672,7 +675,8 @@ struct SlabPlaceLds {
 };
 
 // The workgroups in front of the buckets': one for every partition, to a multiple of the eight dies, so that a bucket
-// stays on the die that sorted it.
+// stays on the die that sorted it.  Of 1024 partitions few have any: a call of 3 M entries takes 116.5 us with them and 117
+// with 256 workgroups of four partitions each; where all have some (one level, 106 000 entries) 112 and 122.
 __host__ __device__ inline uint32_t slab_place_lead(uint32_t partitions) { return (partitions + 7u) & ~7u; }
 
 // A partition's overflow entries in ascending index order (the reference hands its tickets to ascending thread ids,
