@@ -96,6 +96,37 @@ def test_slab_load_balance_bit_exact(zen, oracle, n, P, density, rehash, dtype):
     assert not tp._table(d.device, m).any()
 
 
+@pytest.mark.parametrize("P,log2,density,room,rehash,settled", [
+    # the losers of level 1: settled group by group where 0.7 capacity^2 / slots is above half a million
+    (16, 24, 0.25, 1.0, 3, True),
+    (128, 24, 0.27, 1.02, 2, True),   # nearly as full as buckets may be
+    (1, 26, 0.08, 1.35, 3, True),     # one partition of all groups
+    (7, 24, 0.22, 1.05, 3, True),     # the last group of a partition has fewer buckets
+    (300, 24, 0.22, 1.05, 3, False),  # too many partitions for lists
+    (16, 24, 0.2, 1.03, 3, False),    # just below the line
+])
+@pytest.mark.parametrize("fast_path", ["slabs"], indirect=True)
+def test_slab_load_balance_of_settled_losers(zen, oracle, P, log2, density, room, rehash, settled):
+    from zen_repro_amd import _lib
+
+    n = ((1 << log2) + 160) // P * P
+    g = make_grad(oracle, n, density, "bf16", seed=P + rehash)
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, rehash)
+    capacity = int(len(idx_o) * room)
+    assert st_o == 0 and lb_path(zen, n, P, "bf16", capacity) == SLAB
+    assert (0.7 * capacity ** 2 / n > 500000 and P < 256) == settled
+    tp = zen.TensorPartition(P, 1, rehash)
+    d = to_dev(g)
+    for rep in range(2):  # the second call finds the counters and the map zero again
+        oi, ov, splits, status = tp.load_balance_flat(d, capacity=capacity, mode=_lib.MODE_FAST)
+        assert status.item() == 0
+        assert np.array_equal(to_np(splits), splits_o)
+        assert np.array_equal(to_np(oi)[:len(idx_o)], idx_o)
+        assert np.array_equal(to_np(ov)[:len(idx_o)], val_o)
+    m, _ = oracle.table_sizes(n, P, 1)
+    assert not tp._table(d.device, m).any()
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("P,density,room,losers", [
     # where the entries that moved in are counted: by the chains up to 50 000 losers, behind them where there are more

@@ -43,6 +43,7 @@ struct SlabGeom {
   int sub_shift;      // key offset inside a bucket >> sub_shift = narrow range (fewer than kSlabSubs of them)
   float inv_m;        // (1 / m)(1 - 2^-20), rounded down
   float inv_npp;      // the same for npp
+  uint32_t npp_mult;  // floor(2^32 / npp)
   double width;       // 2^32 / bpp_mult: keys per bucket, to 53 bits
 
   // x / d for x < 2^32 and quotients below 2^11, without the long integer division sequence.  `inv` is
@@ -85,8 +86,24 @@ struct SlabGeom {
     *offset = local - first_local(sb);
     return part * bpp + sb;
   }
+  // Where index t looks at rehash level 1 or 2: as probe_slot, with the slot's bucket and its offset there, and without a
+  // division (x * npp_mult / 2^32 is the quotient or one less).
+  struct Spot {
+    uint32_t slot, bucket, offset;
+  };
+  __device__ inline Spot spot(uint32_t t, int level) const {
+    const uint32_t h = poly(t);
+    uint32_t first;
+    const uint32_t part = div_small(mod_m(h + kSeed1), npp, inv_npp, &first);
+    const uint32_t x = h + (level == 1 ? kSeed2 : kSeed3);
+    uint32_t local = x - __umulhi(x, npp_mult) * npp;
+    if (local >= npp) local -= npp;
+    const uint32_t sb = __umulhi(local, bpp_mult);
+    return Spot{part * npp + local, part * bpp + sb, local - first_local(sb)};
+  }
 };
 
+inline uint32_t slab_npp_mult(uint32_t npp) { return npp > 1u ? (uint32_t)((1ull << 32) / npp) : 0xffffffffu; }
 inline double slab_bucket_width(uint32_t bpp_mult) { return 4294967296.0 / (double)bpp_mult; }
 
 // Host side: geometry for `partitions` partitions of a key space of m keys (m a
@@ -135,6 +152,7 @@ inline bool slab_geometry(int64_t m, int partitions, int64_t expected, int targe
   g.sub_shift = 0;
   while ((width >> g.sub_shift) >= (uint64_t)kSlabSubs) ++g.sub_shift;
   g.width = slab_bucket_width(g.bpp_mult);
+  g.npp_mult = slab_npp_mult(g.npp);
   g.inv_m = slab_inverse_below(g.m);
   g.inv_npp = slab_inverse_below(g.npp);
   *out = g;

@@ -12,21 +12,22 @@
 //                   level-1 slots by a bitmap of them in LDS (wide buckets: by
 //                   comparing entries); of the entries that share a slot the one
 //                   with the smallest index is its level-1 owner, the others lost
-//                   level 1 and are logged;
-//   k_slab_chains   levels 2 and 3 for the losers through a small hash map,
-//                   with the reference's rule executed in ascending index order
-//                   (a slot belongs to the smallest index that ever probes it;
-//                   whoever takes a slot from a larger index continues that
-//                   index's probe sequence).  Every bucket has a part of the map
-//                   of its own, so what finally moved into a bucket is what its
-//                   part holds; an index that ran out of levels goes to its
-//                   partition's serial list; split sizes, unless the losers are
-//                   many:
-//   k_slab_layout   (where the capacity has room for many losers) counts what
-//                   moved into the buckets from the map; split sizes;
+//                   level 1;
+//   k_slab_settle   (where many losers are expected) their level-2 slots, a group
+//                   of buckets at a time in LDS;
+//   k_slab_chains   levels 2 and 3 for the losers that are left through a small
+//                   hash map, with the reference's rule executed in ascending
+//                   index order (a slot belongs to the smallest index that ever
+//                   probes it; whoever takes a slot from a larger index continues
+//                   that index's probe sequence).  Every bucket has a part of the
+//                   map of its own, so what finally moved into a bucket is what
+//                   its part holds; an index that ran out of levels goes to its
+//                   partition's serial list; split sizes;
 //   k_slab_place    one workgroup per bucket: survivors and moved-in entries by
 //                   the same kind of bitmap to the bucket's place in the
 //                   partition-major output.
+#include <algorithm>
+
 #include "zen_balance.h"
 #include "zen_hashmap.h"
 #include "zen_slab.h"
@@ -41,9 +42,9 @@ struct SlabTables {
   uint32_t *bucket_lo;  // [B] smallest level-1 slot of the bucket
   uint32_t *bucket_n;   // [B] sorted records in the slab: level-1 owners, in wide buckets the losers too
   uint32_t *removed_n;  // [B] of which have lost their slot
-  uint32_t *movein_n;   // [B * kMoveinPad] occupied cells of the bucket's part of the map
+  uint32_t *movein_n;   // [B * kMoveinPad] entries that moved in; a word behind: the part of the map has dead cells
   uint32_t *serial_n;   // [P * kMoveinPad] entries that found no slot
-  uint32_t *raw_idx;    // [B * kSlabCap] entries as they arrive: index ...
+  uint32_t *raw_idx;    // [B * kSlabCap] entries as they arrive: index (after the sort: losers, again_n of them) ...
   void *raw_val;        // ... and value
   int32_t *slab_idx;    // [B * kSlabCap] after the sort: index | kRemovedBit, by ascending level-1 slot (the slot
                         // itself is not kept: hashing the index again is cheaper than a trip to memory)
@@ -51,31 +52,51 @@ struct SlabTables {
   uint16_t *sub_index;  // [B * kSlabIndexLen] sorted place of the first record of every kSlabIndexStep-th narrow
                         // key range of the bucket (the last entry: the number of records)
   uint32_t *ser_idx;    // [P * kSlabSerialCap]
-  uint32_t *log_t;      // [log_cap] indices that lost level 1
+  uint32_t *again_n;    // [B] losers the bucket's sort found, but for those in the groups' lists
+  uint32_t *group_n;    // [P * group_pad] losers whose level-2 slot is one of the group's ...
+  uint32_t *group_list; // [groups * group_cap] ... and who they are
+  uint32_t *token_n;    // [groups] indices that k_slab_settle leaves to k_slab_chains ...
+  uint32_t *token;      // [groups * group_cap] ... and who they are (kAtLevel3: at which level)
   uint32_t *out_start;  // [B + 1] where every bucket starts in the output
-  uint32_t *done;       // [kDoneWords] workgroups of k_slab_chains (or k_slab_layout) that have finished
+  uint32_t *done;       // [kDoneWords] workgroups of k_slab_chains that have finished
   uint32_t *final_n;    // [B + P] what k_slab_place needs of the counters above, copied by the last workgroup of
-                        // k_slab_chains, or of k_slab_layout where that counts, before it puts them back to zero:
-                        // moved-in entries per bucket, serial entries per partition
-  uint32_t *losers;     // [1] entries of log_t
+                        // k_slab_chains before it puts them back to zero: moved-in entries per bucket (kHasDead: dead
+                        // cells too), serial entries per partition
   uint32_t *coarse_cursor;  // the feed's coarse cursors and, for an fp32 top-k, the refinement histogram (else
   uint32_t *refine_hist;    // null): k_slab_sort puts them back to zero
   int partitions;
-  uint32_t log_cap;
+  uint32_t gpp;         // groups in a partition ...
+  uint32_t per_group;   // ... of so many buckets
+  uint32_t group_pad;   // words from one partition's counters to the next's
+  uint32_t group_cap;   // losers in a group's list (0: no lists)
 };
 
 // Device-wide atomics on one 128-byte line are carried out one after the other: four counters to a line.
 constexpr uint32_t kMoveinPad = 8;
-// Losers beyond which the chains leave the moved-in entries to be counted from the map (k_slab_layout): a third of their
-// device-wide atomics less for a launch that reads the map and lays out the output.  62 M slots, bf16: 436 000 losers
-// 79 us, without the counting 49 and the launch 15.  Whole calls, counted by the chains and from the map, us: 62 M slots,
-// 45 000 losers 94 and 92, 100 000 122 and 119, 173 000 139 and 128, 394 000 200 and 183; 300 M, 71 000 losers 211 and
-// 211, 172 000 265 and 261; 1 G, 82 000 539 and 541.  (With the line at 200 000, calls of fewer losers had the
-// launch behind the chains and counted all the same: 1.3 to 2 us more than without it.)
-constexpr uint32_t kUncountedFrom = 50000;
-// The launch is there from this estimate of the losers on: n^2 / 2m of n = capacity entries in m slots.  The hash loses 1.4
-// times as many, at powers of two a third, and calls select from two thirds of their capacity to all of it.
-constexpr double kLayoutFrom = 200000;
+constexpr uint32_t kHasDead = 1u << 31;
+
+// A cell of the map: (slot + 1) << 32 | index, 0 if empty, of index kNone if nobody is left in it (dead).
+__device__ inline uint32_t cell_slot(unsigned long long cell) { return (uint32_t)(cell >> 32) - 1u; }
+// The index in a cell, 0 if there is none.
+__device__ inline uint32_t cell_index(unsigned long long cell) { return (uint32_t)cell == kNone ? 0u : (uint32_t)cell; }
+
+// Where many losers are expected a bucket's losers go to lists, by the group of buckets their level-2 slots lie in, and
+// k_slab_settle enters a group's list into its parts of the map in LDS: device-wide atomics are carried out at 25 a
+// nanosecond, and of an entry for each loser in the map and one to count it nine in ten fall away.  Where fewer are
+// expected each goes its way through memory (k_slab_chains), for the other way is a launch more and two barriers in the sort.
+// The line is an estimate from the capacity; the hash loses 1.4 times as many as evenly spread slots would.  Whole calls,
+// settled and not, 62 M slots, bf16, sixteen partitions: 436 000 losers (estimate 980 000) 554 and 570 us, 110 000 (240 000)
+// 416 and 413; 268 M, 18 000 (42 000) 643 and 637.
+constexpr double kSettleFrom = 500000;
+constexpr uint32_t kGroupBuckets = 12;         // of a group, at most: their parts of the map and indices fill 121 KB
+constexpr uint32_t kGroupLeast = 4, kGroupsWanted = 256;  // (a compute unit to each)
+constexpr uint32_t kMostGroups = 256;          // of a partition
+constexpr size_t kMostGroupWords = 8192;       // of all partitions' counters, a partition's in memory lines of their own
+constexpr int kSettleBlock = 1024;
+constexpr int kSettleRows = 6;                 // losers of a thread, at most
+constexpr uint32_t kGroupCap = kSettleBlock * kSettleRows;
+constexpr uint32_t kChainsResident = 1024;     // workgroups of k_slab_chains the chip holds at a time
+constexpr uint32_t kAtLevel3 = 1u << 31;       // in a list: the index goes on at level 3 (else at level 2)
 
 // The counters and histograms that must be zero when a call starts live in memory that is zero between calls
 // (the part of the caller's table the hash map does not use), and every one of them is put back to zero by the
@@ -88,8 +109,6 @@ constexpr double kLayoutFrom = 200000;
 constexpr int kSlabIndexStep = 4;
 constexpr int kSlabIndexLen = kSlabSubs / kSlabIndexStep + 1;
 static_assert(kSlabSubs % kSlabIndexStep == 0 && kSlabCap < 65536, "index layout");
-
-__device__ inline uint32_t level1_slot(const Probe &g, uint32_t t) { return (poly(t) + kSeed1) % g.m; }
 
 // ---------------------------------------------- coarse slabs -> bucket slabs
 
@@ -137,14 +156,17 @@ struct SlabSortLds {
   uint32_t idx[kSlabCap];  // the sorted indices
   union {
     SlabTaken<SPAN> taken;
-    S val[kSlabCap];       // once the ranks are known: the sorted values
+    struct {               // once the ranks are known:
+      S val[kSlabCap];         // the sorted values
+      uint32_t list[kSlabCap]; // the losers
+    };
   };
   uint32_t scan[kSortBlock / 64 + 1];
-  uint32_t shared, lost, base;
+  uint32_t shared, lost, again;
 };
 
 // Sorts a bucket's records by level-1 slot; of those that share a slot the smallest index owns it, the others are
-// logged and not kept.  A bucket has a few to a few hundred slots per record, so the slots are marked in a bitmap: a
+// listed and not kept.  A bucket has a few to a few hundred slots per record, so the slots are marked in a bitmap: a
 // record's place is the number of marks below its own, and whoever finds its slot marked already is settled by the
 // smallest index afterwards.  Bound by the vector instructions and the LDS round trips behind every phase's barrier (two
 // workgroups a compute unit).  ROWS: records of a thread (the last row may be cut short); the code is written out for
@@ -153,7 +175,7 @@ struct SlabSortLds {
 // 23.7 -> 21.5.  (By comparisons, k_slab_sort_wide: 64 and 33 at the time.)
 template <int ROWS, typename S, uint32_t SPAN>
 __device__ __forceinline__ void slab_sort_rows(SlabSortLds<S, SPAN> &sh, const SlabGeom &geo, const SlabTables &tb,
-                                               uint32_t n_raw, int32_t *status) {
+                                               uint32_t n_raw) {
   const uint32_t b = blockIdx.x;
   const size_t base = (size_t)b * kSlabCap;
   const uint32_t words = (geo.span + 63u) / 64u;
@@ -216,13 +238,14 @@ __device__ __forceinline__ void slab_sort_rows(SlabSortLds<S, SPAN> &sh, const S
   const uint32_t losers = live & ~owner;
   uint32_t at = losers ? atomicAdd(&sh.lost, (uint32_t)__popc(losers)) : 0u;
 #pragma unroll
-  for (int i = 0; i < ROWS; ++i)
+  for (int i = 0; i < ROWS; ++i) {
     if (owner & (1u << i)) sh.val[rank[i]] = val[i];  // (the bitmap has done its work)
+    if (losers & (1u << i)) sh.list[at++] = idx[i];
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
     tb.bucket_n[b] = n;
     tb.removed_n[b] = 0;
-    sh.base = sh.lost ? atomicAdd(tb.losers, sh.lost) : 0u;
   }
   int32_t *slab_idx = tb.slab_idx + base;
   S *slab_val = static_cast<S *>(tb.slab_val) + base;
@@ -234,28 +257,18 @@ __device__ __forceinline__ void slab_sort_rows(SlabSortLds<S, SPAN> &sh, const S
       slab_val[p] = sh.val[p];
     }
   }
-  __syncthreads();
-  at += sh.base;
-#pragma unroll
-  for (int i = 0; i < ROWS; ++i) {
-    if (losers & (1u << i)) {
-      if (at < tb.log_cap)
-        tb.log_t[at] = idx[i];
-      else
-        atomicOr(status, ZEN_STAT_RETRY);
-      ++at;
-    }
-  }
 }
 
-template <typename S, uint32_t SPAN>
-__global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabTables tb, int32_t *status) {
+// LISTS: the losers go to the groups' lists (a kernel of its own: beside the merge's workgroups the other one gets along
+// better without that code).
+template <typename S, uint32_t SPAN, bool LISTS>
+__global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabTables tb) {
   __shared__ SlabSortLds<S, SPAN> sh;
   const uint32_t b = blockIdx.x;
   const uint32_t words = (geo.span + 63u) / 64u;
   uint32_t n_raw = tb.cursor[b];
   if (n_raw > (uint32_t)kSlabCap) n_raw = kSlabCap;  // the scatter flagged the overflow
-  if (threadIdx.x == 0) sh.shared = sh.lost = 0;
+  if (threadIdx.x == 0) sh.shared = sh.lost = sh.again = 0;
   sh.taken.template clear<kSortBlock>(words);
   // the kernels before this one were the last to need these: back to zero, a slice per workgroup
   for (uint32_t i = b * kSortBlock + threadIdx.x; i < kCoarseCursorWords; i += gridDim.x * kSortBlock)
@@ -266,13 +279,52 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort(SlabGeom geo, SlabT
   static_assert(kSortItems == 6, "a case for every number of rows");
   switch ((n_raw + kSortBlock - 1) / kSortBlock) {
     case 0:
-    case 1: slab_sort_rows<1>(sh, geo, tb, n_raw, status); break;
-    case 2: slab_sort_rows<2>(sh, geo, tb, n_raw, status); break;
-    case 3: slab_sort_rows<3>(sh, geo, tb, n_raw, status); break;
-    case 4: slab_sort_rows<4>(sh, geo, tb, n_raw, status); break;
-    case 5: slab_sort_rows<5>(sh, geo, tb, n_raw, status); break;
-    default: slab_sort_rows<6>(sh, geo, tb, n_raw, status); break;
+    case 1: slab_sort_rows<1>(sh, geo, tb, n_raw); break;
+    case 2: slab_sort_rows<2>(sh, geo, tb, n_raw); break;
+    case 3: slab_sort_rows<3>(sh, geo, tb, n_raw); break;
+    case 4: slab_sort_rows<4>(sh, geo, tb, n_raw); break;
+    case 5: slab_sort_rows<5>(sh, geo, tb, n_raw); break;
+    default: slab_sort_rows<6>(sh, geo, tb, n_raw); break;
   }
+  // The losers, to the groups' lists a run of each (one atomic to a group), else to the bucket's own: that is the memory of
+  // the records' indices, which have been in registers since the first barrier.  (One log for all buckets, and its one
+  // counter, 11 ns a workgroup: 268 M slots, 2.7 M bf16 records in 1024 buckets 22.2 us, so 19.3.)
+  uint32_t *own = tb.raw_idx + (size_t)b * kSlabCap;
+  if constexpr (!LISTS) {
+    for (uint32_t i = threadIdx.x; i < sh.lost; i += kSortBlock) own[i] = sh.list[i];
+    if (threadIdx.x == 0) tb.again_n[b] = sh.lost;
+    return;
+  }
+  const uint32_t part = b / geo.bpp;
+  uint32_t *count = sh.idx;  // of every group (the sorted indices are on their way out)
+  static_assert(kMostGroups <= kSlabCap && kMostGroups <= kSortBlock, "a group per thread");
+  for (uint32_t i0 = 0; i0 < sh.lost; i0 += kSortBlock) {  // (one turn as a rule)
+    __syncthreads();
+    if (threadIdx.x < tb.gpp) count[threadIdx.x] = 0;
+    __syncthreads();
+    const bool one = i0 + threadIdx.x < sh.lost;
+    uint32_t t = 0, to = 0, at = 0;
+    if (one) {
+      t = sh.list[i0 + threadIdx.x];
+      to = (geo.spot(t, 1).bucket - part * geo.bpp) / tb.per_group;
+      at = atomicAdd(&count[to], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x < tb.gpp) {
+      const uint32_t n = count[threadIdx.x];
+      if (n) count[threadIdx.x] = atomicAdd(&tb.group_n[part * tb.group_pad + threadIdx.x], n);
+    }
+    __syncthreads();
+    if (one) {
+      at += count[to];
+      if (at < tb.group_cap)
+        tb.group_list[(size_t)(part * tb.gpp + to) * tb.group_cap + at] = t;
+      else
+        own[atomicAdd(&sh.again, 1u)] = t;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) tb.again_n[b] = sh.again;
 }
 
 // The same for few records among many slots: grouped by narrow key ranges, ranked against the words of their group
@@ -284,7 +336,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort_wide(SlabGeom geo, 
   // otherwise need 88 KB of LDS, one workgroup to a compute unit instead of two
   __shared__ SlabSortSharedNoQueue sh;
   __shared__ S s_val[kSlabCap];
-  __shared__ uint32_t s_lost, s_base;
+  __shared__ uint32_t s_lost;
   const uint32_t b = blockIdx.x;
   const size_t base = (size_t)b * kSlabCap;
   uint32_t n_raw = tb.cursor[b];
@@ -326,6 +378,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort_wide(SlabGeom geo, 
       atomicOr(status, ZEN_STAT_RETRY);
       tb.bucket_n[b] = 0;
       tb.removed_n[b] = 0;
+      tb.again_n[b] = 0;
     }
     for (int j = threadIdx.x; j < kSlabIndexLen; j += kSortBlock) tb.sub_index[(size_t)b * kSlabIndexLen + j] = 0;
     return;
@@ -393,36 +446,24 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort_wide(SlabGeom geo, 
     if (threadIdx.x == 0) atomicOr(status, ZEN_STAT_RETRY);
     lost_n = kSlabSubs;
   }
+  for (uint32_t i = threadIdx.x; i < lost_n; i += kSortBlock) tb.raw_idx[base + i] = sh.tie[sh.key[i]];
   if (threadIdx.x == 0) {
     tb.bucket_n[b] = n;
     tb.removed_n[b] = lost_n;
-    s_base = lost_n ? atomicAdd(tb.losers, lost_n) : 0u;
-  }
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < lost_n; i += kSortBlock) {
-    const uint32_t at = s_base + i;
-    const uint32_t p = sh.key[i];
-    if (at < tb.log_cap)
-      tb.log_t[at] = sh.tie[p];
-    else
-      atomicOr(status, ZEN_STAT_RETRY);
+    tb.again_n[b] = lost_n;
   }
 }
 
 // ------------------------------------------------------ levels 2 and 3
 
-// Smallest index whose level-1 slot is `slot` (kNone if nobody's), where it sits, and the slot's bucket.  The bucket's index
+// Smallest index whose level-1 slot is `at.slot` (kNone if nobody's) and where it sits.  The bucket's index
 // narrows the search to the records of kSlabIndexStep narrow ranges (three or four); they are fetched four at
 // a time and looked at in sorted order: by ascending slot, and in a run of equal slots the smallest index
 // comes first.
-__device__ inline uint32_t slab_head(const SlabGeom &geo, const SlabTables &tb, uint32_t slot, size_t *pos_out,
-                                     uint32_t *bucket_out) {
-  uint32_t off;
-  const uint32_t b = geo.bucket_and_offset(slot, &off);  // computed, not fetched: one trip less in the chain
-  *bucket_out = b;
-  const int32_t *idx = tb.slab_idx + (size_t)b * kSlabCap;
-  const uint32_t j = (off >> geo.sub_shift) / (uint32_t)kSlabIndexStep;
-  const uint16_t *index = tb.sub_index + (size_t)b * kSlabIndexLen;
+__device__ inline uint32_t slab_head(const SlabGeom &geo, const SlabTables &tb, const SlabGeom::Spot &at, size_t *pos_out) {
+  const int32_t *idx = tb.slab_idx + (size_t)at.bucket * kSlabCap;
+  const uint32_t j = (at.offset >> geo.sub_shift) / (uint32_t)kSlabIndexStep;
+  const uint16_t *index = tb.sub_index + (size_t)at.bucket * kSlabIndexLen;
   uint16_t range[2];  // one load each time: a wave's lanes all read other lines
   __builtin_memcpy(range, index + j, sizeof(range));
   const uint32_t end = range[1];
@@ -435,9 +476,9 @@ __device__ inline uint32_t slab_head(const SlabGeom &geo, const SlabTables &tb, 
     for (int q = 0; q < 4; ++q) {
       if (p + q >= end) return kNone;
       const uint32_t s1 = geo.mod_m(poly(t[q]) + kSeed1);
-      if (s1 > slot) return kNone;
-      if (s1 == slot) {
-        *pos_out = (size_t)b * kSlabCap + p + q;
+      if (s1 > at.slot) return kNone;
+      if (s1 == at.slot) {
+        *pos_out = (size_t)at.bucket * kSlabCap + p + q;
         return t[q];
       }
     }
@@ -446,20 +487,16 @@ __device__ inline uint32_t slab_head(const SlabGeom &geo, const SlabTables &tb, 
 }
 
 // Enters t as a prober of `slot` in bucket b's part of the map; returns the smallest earlier prober (kNone: there was
-// none).  *full is set if the part has no room.  counted: the part's entries are counted as they come.
-__device__ inline uint32_t part_min(unsigned long long *cells, const SlabTables &tb, uint32_t b, uint32_t slot, uint32_t t,
-                                    bool counted, bool *full) {
+// none, or the cell was dead).  *full is set if the part has no room.
+__device__ inline uint32_t part_min(unsigned long long *cells, uint32_t b, uint32_t slot, uint32_t t, bool *full) {
   unsigned long long *part = cells + ((size_t)b << kSlabPartLog2);
   constexpr uint32_t mask = (1u << kSlabPartLog2) - 1u;
   const unsigned long long mine = ((unsigned long long)(slot + 1u) << 32) | t;
   uint32_t h = cell_home(slot, kSlabPartLog2);
   for (uint32_t probes = 0; probes <= mask; ++probes, h = (h + 1u) & mask) {
     const unsigned long long cur = atomicCAS(&part[h], 0ull, mine);
-    if (cur == 0ull) {
-      if (counted) atomicAdd(&tb.movein_n[b * kMoveinPad], 1u);
-      return kNone;
-    }
-    if ((uint32_t)(cur >> 32) == slot + 1u) return (uint32_t)atomicMin(&part[h], mine);
+    if (cur == 0ull) return kNone;
+    if (cell_slot(cur) == slot) return (uint32_t)atomicMin(&part[h], mine);
   }
   *full = true;
   return 0u;  // pretend a smaller index owns it: the chain moves on and the call is retried anyway
@@ -469,61 +506,65 @@ __device__ inline uint32_t part_min(unsigned long long *cells, const SlabTables 
 // behind its last bucket.  Run by one workgroup of kSlabBlock threads once all counts are final: it is the last
 // to need the counters the chains raised with atomics, hands what k_slab_place still wants of them on in final_n
 // and puts them back to zero.  What the status word can come to is known here too (k_slab_place adds nothing).
-// The chip waits for this one workgroup: one trip to memory for all counts, and what the host asked for is put together in
-// LDS (s_start: kSlabMaxBuckets + 1 words).
+// The chip waits for this one workgroup: one trip to memory for all counts, by consecutive lanes, and prefixes in LDS
+// (s_start: kSlabMaxBuckets + 1 words).  A thread with neighbouring buckets of its own asked for a memory line a lane: 2560
+// buckets 9 us.
 __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables &tb, uint32_t *s_scan, uint32_t *s_start,
                                           int64_t spp, uint32_t capacity, int64_t *splits, const HostAnswer &answer,
                                           int32_t *status) {
   constexpr uint32_t kPer = kSlabMaxBuckets / kSlabBlock;
-  const uint32_t B = geo.nbuckets, per = (B + (uint32_t)kSlabBlock - 1u) / (uint32_t)kSlabBlock, x0 = threadIdx.x * per;
-  uint32_t c[kPer], mv[kPer], rm[kPer], sn[kPer];
+  const uint32_t B = geo.nbuckets, P = (uint32_t)tb.partitions;
+  unsigned long long *movein = reinterpret_cast<unsigned long long *>(tb.movein_n);
+  unsigned long long mv[kPer];
+  uint32_t rm[kPer], n[kPer], sn[kPer];
+#pragma unroll
+  for (uint32_t e = 0; e < kPer; ++e) {  // (the conditions are the same for all threads: all loads are in flight together)
+    const uint32_t x = threadIdx.x + e * (uint32_t)kSlabBlock;
+    if (e * (uint32_t)kSlabBlock < B) {
+      const uint32_t at = x < B ? x : 0u;
+      mv[e] = __hip_atomic_load(&movein[at * (kMoveinPad / 2)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      rm[e] = load_fresh(&tb.removed_n[at]);
+      n[e] = tb.bucket_n[at];
+    }
+    if (e * (uint32_t)kSlabBlock < P) sn[e] = load_fresh(&tb.serial_n[(x < P ? x : 0u) * kMoveinPad]);
+  }
 #pragma unroll
   for (uint32_t e = 0; e < kPer; ++e) {
-    if (e < per) {  // the same for all threads; no other branch around the loads: all in flight together
-      const uint32_t at = x0 + e < B ? x0 + e : 0u;
-      mv[e] = load_fresh(&tb.movein_n[at * kMoveinPad]);
-      rm[e] = load_fresh(&tb.removed_n[at]);
-      sn[e] = load_fresh(&tb.serial_n[at / geo.bpp * kMoveinPad]);
-      c[e] = tb.bucket_n[at];
-    }
+    const uint32_t x = threadIdx.x + e * (uint32_t)kSlabBlock;
+    if (x < B) s_start[x] = n[e] + (uint32_t)mv[e] - rm[e];
   }
-  uint32_t sum = 0;
+  __syncthreads();
   bool overflow = false;
 #pragma unroll
   for (uint32_t e = 0; e < kPer; ++e) {
-    const uint32_t x = x0 + e;
-    if (e < per && x < B) {
-      c[e] += mv[e] - rm[e];
-      tb.final_n[x] = mv[e];
-      if (x % geo.bpp == geo.bpp - 1) {
-        tb.final_n[B + x / geo.bpp] = sn[e];
-        overflow |= (int64_t)sn[e] > spp;
-        c[e] += sn[e] > (uint32_t)kSlabSerialCap ? (uint32_t)kSlabSerialCap : sn[e];
-      }
-      sum += c[e];
+    const uint32_t x = threadIdx.x + e * (uint32_t)kSlabBlock;
+    if (x < P) {
+      overflow |= (int64_t)sn[e] > spp;
+      s_start[x * geo.bpp + geo.bpp - 1u] += sn[e] > (uint32_t)kSlabSerialCap ? (uint32_t)kSlabSerialCap : sn[e];
     }
   }
+  __syncthreads();
+  const uint32_t per = (B + (uint32_t)kSlabBlock - 1u) / (uint32_t)kSlabBlock | 1u;  // odd: the lanes on different banks
+  const uint32_t first = threadIdx.x * per, end = first + per < B ? first + per : B;
+  uint32_t sum = 0;
+  for (uint32_t x = first; x < end; ++x) sum += s_start[x];
   uint32_t total;
   uint32_t running = block_exclusive_scan<uint32_t, kSlabBlock>(sum, s_scan, &total);
-#pragma unroll
-  for (uint32_t e = 0; e < kPer; ++e) {
-    const uint32_t x = x0 + e;
-    if (e < per && x < B) {
-      tb.out_start[x] = running;
-      if (x % geo.bpp == 0) s_start[x / geo.bpp] = running;
-      running += c[e];
-    }
+  for (uint32_t x = first; x < end; ++x) {
+    const uint32_t c = s_start[x];
+    s_start[x] = running;
+    running += c;
   }
   if (threadIdx.x == 0) {
-    tb.out_start[B] = s_start[tb.partitions] = total;
+    s_start[B] = total;
     if (total > capacity) atomicOr(status, ZEN_STAT_CAPACITY);
   }
   if (overflow) atomicOr(status, ZEN_STAT_SERIAL_OVERFLOW);
   if (answer.host) wait_global_acks();
   __syncthreads();
   // the split sizes: the host has them while the entries are still on their way to their places
-  for (uint32_t p = threadIdx.x; p < (uint32_t)tb.partitions; p += kSlabBlock) {
-    const int64_t size = (int64_t)(s_start[p + 1u] - s_start[p]);
+  for (uint32_t p = threadIdx.x; p < P; p += kSlabBlock) {
+    const int64_t size = (int64_t)(s_start[(p + 1u) * geo.bpp] - s_start[p * geo.bpp]);
     splits[p] = size;
     if (answer.host) host_store(answer.host + 1 + p, size);
   }
@@ -533,122 +574,268 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
                  (int64_t)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     host_answered(answer);
   }
-  for (uint32_t x = threadIdx.x; x < B; x += kSlabBlock) tb.movein_n[x * kMoveinPad] = 0;
-  for (uint32_t x = threadIdx.x; x < (uint32_t)tb.partitions; x += kSlabBlock) tb.serial_n[x * kMoveinPad] = 0;
-  for (uint32_t x = threadIdx.x; x < kDoneWords; x += kSlabBlock) tb.done[x] = 0;
-  if (threadIdx.x == 0) *tb.losers = 0;
-}
-
-// Levels 2 and 3 for the indices that lost level 1, one per thread.  Bound by latency while losers are few (110 000: a
-// wave 15 us; a probe is four or five dependent trips to memory, the bucket's index, its records, the map) and by the
-// device-wide atomics, one or two a loser (two or three while the moved-in entries are counted) at 21 a nanosecond, when they
-// are many (436 000: 49 us, counted 79).  Every loser
-// has a thread of its own on a full chip: with the scalar registers the compiler takes by itself three workgroups fit a
-// compute unit, and the last of 851 began when the first had ended (93 us, with four 83).  Nothing is counted in one
-// place (62 M slots, 10 % taken, 300 000 losers: with one counter of the map's claims and one log of the owners pushed
-// out, whose entries another kernel classified afterwards, 338 + 220 us).
-__global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Probe g, SlabTables tb, unsigned long long *cells,
-                                                            int64_t spp, uint32_t capacity, int64_t *__restrict__ splits,
-                                                            uint32_t count_up_to, HostAnswer answer, int32_t *status) {
-  __shared__ uint32_t s_scan[kSlabBlock / 64 + 1];
-  __shared__ uint32_t s_start[kSlabMaxBuckets + 1];
-  __shared__ bool s_last;
-  uint32_t losers = load_fresh(tb.losers);
-  const bool counted = losers <= count_up_to;
-  if (losers > tb.log_cap) losers = tb.log_cap;
-  // workgroups without a loser are not waited for (one that starts after the last of the others has put the count
-  // back to zero sees none either)
-  uint32_t working = (losers + kSlabBlock - 1u) / kSlabBlock;
-  working = working < 1u ? 1u : working > gridDim.x ? gridDim.x : working;
-  if (blockIdx.x >= working) return;
-  for (uint32_t i = blockIdx.x * (uint32_t)kSlabBlock + threadIdx.x; i < losers; i += gridDim.x * (uint32_t)kSlabBlock) {
-    uint32_t cur = tb.log_t[i];
-    int lv = 1;
-    bool full = false;
-    for (uint32_t steps = 0;; ++steps) {
-      if (lv >= g.levels) {  // out of levels: cur has no slot
-        const uint32_t part = level1_slot(g, cur) / g.npp;
-        const uint32_t at = atomicAdd(&tb.serial_n[part * kMoveinPad], 1u);
-        if (at < (uint32_t)kSlabSerialCap)
-          tb.ser_idx[(size_t)part * kSlabSerialCap + at] = cur;
-        else  // more than the partition's serial region holds is an overflow; more than this path carries, a retry
-          atomicOr(status, (int64_t)at >= spp ? ZEN_STAT_SERIAL_OVERFLOW : ZEN_STAT_RETRY);
-        break;
-      }
-      if (steps > kChainLimit) {
-        atomicOr(status, ZEN_STAT_INTERNAL);
-        break;
-      }
-      uint32_t part;
-      const uint32_t slot = probe_slot(g, cur, lv, &part);
-      size_t head_pos = 0;
-      uint32_t bucket = 0;
-      const uint32_t head = slab_head(geo, tb, slot, &head_pos, &bucket);
-      if (head < cur) {  // a smaller index probes this slot at level 1: cur moves on
-        ++lv;
-        continue;
-      }
-      const uint32_t old = part_min(cells, tb, bucket, slot, cur, counted, &full);
-      if (full) {
-        atomicOr(status, ZEN_STAT_RETRY);
-        break;
-      }
-      if (old < cur) {  // a smaller index got here at level 2 or 3
-        ++lv;
-        continue;
-      }
-      if (old == kNone) {
-        // first level-2/3 prober of this slot: its level-1 owner (a larger index, if any) is pushed out
-        if (head == kNone) break;
-        atomicOr(reinterpret_cast<uint32_t *>(&tb.slab_idx[head_pos]), kRemovedBit);
-        atomicAdd(&tb.removed_n[bucket], 1u);
-        cur = head;
-        lv = 1;
-        continue;
-      }
-      if (old == cur) break;
-      // took the slot from a larger index that held it at its first level mapping here
-      int lw = 1;
-      while (lw < g.levels && probe_slot(g, old, lw, &part) != slot) ++lw;
-      cur = old;
-      lv = lw + 1;
+#pragma unroll
+  for (uint32_t e = 0; e < kPer; ++e) {
+    const uint32_t x = threadIdx.x + e * (uint32_t)kSlabBlock;
+    if (x < B) {
+      tb.out_start[x] = s_start[x];
+      tb.final_n[x] = (uint32_t)mv[e] | (mv[e] >> 32 ? kHasDead : 0u);
+      movein[x * (kMoveinPad / 2)] = 0;
+    }
+    if (x < P) {
+      tb.final_n[B + x] = sn[e];
+      tb.serial_n[x * kMoveinPad] = 0;
     }
   }
-  if (!counted) return;  // k_slab_layout counts, and lays out the output
-  // the workgroup that finishes last knows every count and lays out the output
-  wait_global_acks();
-  __syncthreads();
-  if (threadIdx.x == 0) s_last = done_last(tb.done, blockIdx.x, working);
-  __syncthreads();
-  if (s_last) slab_output_starts(geo, tb, s_scan, s_start, spp, capacity, splits, answer, status);
+  if (threadIdx.x == 0) tb.out_start[B] = total;
+  for (uint32_t x = threadIdx.x; x < kDoneWords; x += kSlabBlock) tb.done[x] = 0;
 }
 
-// Where the chains left the moved-in entries uncounted: a wave to a bucket counts what its part of the map holds (8 KB, a
-// read of the whole map), the last workgroup lays out the output.  Launched behind the chains where the capacity has room
-// for many losers (kLayoutFrom); returns at once if they were counted after all (the layout has put their number back
-// to zero).
-constexpr int kLayoutBuckets = kSlabBlock / 64;
-__global__ __launch_bounds__(kSlabBlock) void k_slab_layout(SlabGeom geo, SlabTables tb,
-                                                            const unsigned long long *__restrict__ cells, int64_t spp,
-                                                            uint32_t capacity, int64_t *__restrict__ splits,
-                                                            uint32_t count_up_to, HostAnswer answer, int32_t *status) {
+// The way of one index from level `lv` + 1 on, and of those it sets in motion: whoever is pushed out of a slot goes on.
+// Those that find no slot are listed in LDS (`serial`, of which one call takes a word at most).
+__device__ inline void slab_chain(const SlabGeom &geo, const Probe &g, const SlabTables &tb, unsigned long long *cells,
+                                  uint32_t cur, int lv, uint32_t *serial, uint32_t *serial_n, int32_t *status) {
+  bool full = false;
+  for (uint32_t steps = 0;; ++steps) {
+    if (lv >= g.levels) {  // out of levels: cur has no slot
+      serial[atomicAdd(serial_n, 1u)] = cur;
+      break;
+    }
+    if (steps > kChainLimit) {
+      atomicOr(status, ZEN_STAT_INTERNAL);
+      break;
+    }
+    const SlabGeom::Spot spot = geo.spot(cur, lv);
+    const uint32_t bucket = spot.bucket;
+    size_t head_pos = 0;
+    const uint32_t head = slab_head(geo, tb, spot, &head_pos);
+    if (head < cur) {  // a smaller index probes this slot at level 1: cur moves on
+      ++lv;
+      continue;
+    }
+    const uint32_t old = part_min(cells, bucket, spot.slot, cur, &full);
+    if (full) {
+      atomicOr(status, ZEN_STAT_RETRY);
+      break;
+    }
+    if (old < cur) {  // a smaller index got here at level 2 or 3
+      ++lv;
+      continue;
+    }
+    if (old == kNone) {
+      // first level-2/3 prober of this slot that counts: its level-1 owner (a larger index, if any) is pushed out
+      atomicAdd(&tb.movein_n[bucket * kMoveinPad], 1u);
+      if (head == kNone) break;
+      atomicOr(reinterpret_cast<uint32_t *>(&tb.slab_idx[head_pos]), kRemovedBit);
+      atomicAdd(&tb.removed_n[bucket], 1u);
+      cur = head;
+      lv = 1;
+      continue;
+    }
+    if (old == cur) break;
+    // took the slot from a larger index that held it at its first level mapping here
+    int lw = 1;
+    while (lw < g.levels && geo.spot(old, lw).slot != spot.slot) ++lw;
+    cur = old;
+    lv = lw + 1;
+  }
+}
+
+// Level 2 for a group's list of losers.  All of them are entered in the group's parts of the map, which are put together in
+// LDS; whoever finds a smaller index there, or is pushed out by one, goes on at level 3.  Of those that are left one in
+// ten or so finds a level-1 owner: a smaller one sends it on (its cell stays, dead: entries behind it may have come past
+// it), a larger one is pushed out and goes on at level 2.  Nobody else touches the map while this kernel runs.  Bound by
+// latency (four or five trips to memory, as many phases in LDS) and instructions: a group to a compute unit, its losers to
+// all of the unit's waves.  62 M slots, 436 000 losers in 256 groups 19.5 us, the chains behind it 23 (without it the
+// chains 50, and 15 to count the entries that moved in).
+struct SlabSettleLds {
+  unsigned long long cells[kGroupBuckets << kSlabPartLog2];
+  uint16_t index[kGroupBuckets * kSlabIndexLen];  // the buckets' indices
+  uint32_t alive[kGroupBuckets], dead[kGroupBuckets], pushed[kGroupBuckets];
+  uint32_t tokens;
+};
+
+__global__ __launch_bounds__(kSettleBlock) void k_slab_settle(SlabGeom geo, SlabTables tb, unsigned long long *cells,
+                                                              int32_t *status) {
+  __shared__ SlabSettleLds sh;
+  constexpr uint32_t mask = (1u << kSlabPartLog2) - 1u;
+  const uint32_t group = blockIdx.x, part = group / tb.gpp, first = (group - part * tb.gpp) * tb.per_group;
+  const uint32_t b0 = part * geo.bpp + first;
+  const uint32_t buckets = geo.bpp - first < tb.per_group ? geo.bpp - first : tb.per_group;
+  uint32_t *counter = &tb.group_n[part * tb.group_pad + (group - part * tb.gpp)];
+  const uint32_t *list = tb.group_list + (size_t)group * tb.group_cap;
+  int32_t *slab_idx = tb.slab_idx + (size_t)b0 * kSlabCap;
+  uint32_t *token = tb.token + (size_t)group * tb.group_cap;  // (a loser leaves one at most)
+  uint32_t count = *counter;
+  const uint16_t *index = tb.sub_index + (size_t)b0 * kSlabIndexLen;
+  for (uint32_t i = threadIdx.x; i < buckets * kSlabIndexLen; i += kSettleBlock) sh.index[i] = index[i];
+  count = count < tb.group_cap ? count : tb.group_cap;
+  u32x4 *clear = reinterpret_cast<u32x4 *>(sh.cells);
+  for (uint32_t i = threadIdx.x; i < (buckets << kSlabPartLog2) / 2u; i += kSettleBlock) clear[i] = u32x4{0, 0, 0, 0};
+  if (threadIdx.x < kGroupBuckets) sh.alive[threadIdx.x] = sh.dead[threadIdx.x] = sh.pushed[threadIdx.x] = 0;
+  if (threadIdx.x == 0) sh.tokens = 0;
+  __syncthreads();
+  if (threadIdx.x == 0) *counter = 0;
+  // rows nobody has a loser in are skipped by the whole workgroup; the loads of a step are in flight together
+  uint32_t t[kSettleRows], cell[kSettleRows];
+  SlabGeom::Spot spot[kSettleRows];
+  uint32_t in = 0;  // bit r: row r has a loser for this thread; from the second barrier on, one that holds its cell
+#pragma unroll
+  for (int r = 0; r < kSettleRows; ++r) {
+    const uint32_t i = r * kSettleBlock + threadIdx.x;
+    if ((uint32_t)(r * kSettleBlock) < count) t[r] = list[i < count ? i : 0u];
+    in |= (i < count ? 1u : 0u) << r;
+  }
+#pragma unroll
+  for (int r = 0; r < kSettleRows; ++r) {
+    if ((uint32_t)(r * kSettleBlock) >= count) continue;
+    spot[r] = geo.spot(t[r], 1);
+    cell[r] = 0;
+    if (!(in & (1u << r))) continue;
+    const uint32_t at = (spot[r].bucket - b0) << kSlabPartLog2;
+    const unsigned long long mine = ((unsigned long long)(spot[r].slot + 1u) << 32) | t[r];
+    uint32_t h = cell_home(spot[r].slot, kSlabPartLog2), probes = 0;
+    for (; probes <= mask; ++probes, h = (h + 1u) & mask) {
+      const unsigned long long cur = atomicCAS(&sh.cells[at + h], 0ull, mine);
+      if (cur == 0ull) break;
+      if (cell_slot(cur) == spot[r].slot) {
+        const uint32_t old = (uint32_t)atomicMin(&sh.cells[at + h], mine);
+        token[atomicAdd(&sh.tokens, 1u)] = (old < t[r] ? t[r] : old) | kAtLevel3;
+        break;
+      }
+    }
+    cell[r] = at + h;
+    if (probes > mask) atomicOr(status, ZEN_STAT_RETRY);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kSettleRows; ++r)
+    if ((uint32_t)(r * kSettleBlock) < count && (uint32_t)sh.cells[cell[r]] != t[r]) in &= ~(1u << r);
+  // whose level-1 slot is it: the bucket's index narrows the search to a few records (see slab_head)
+  uint32_t head[kSettleRows], pos[kSettleRows], left[kSettleRows], near[kSettleRows][4];
+#pragma unroll
+  for (int r = 0; r < kSettleRows; ++r) {
+    if ((uint32_t)(r * kSettleBlock) >= count) continue;
+    const uint32_t local = spot[r].bucket - b0;
+    const uint32_t j = local * kSlabIndexLen + (spot[r].offset >> geo.sub_shift) / (uint32_t)kSlabIndexStep;
+    pos[r] = local * (uint32_t)kSlabCap + sh.index[j];
+    left[r] = (uint32_t)sh.index[j + 1u] - sh.index[j];
+    __builtin_memcpy(near[r], slab_idx + pos[r], sizeof(near[r]));  // (words past the range are not looked at)
+  }
+#pragma unroll
+  for (int r = 0; r < kSettleRows; ++r) {
+    head[r] = kNone;
+    if ((uint32_t)(r * kSettleBlock) >= count || !(in & (1u << r))) continue;
+    for (uint32_t at = pos[r];;) {
+      bool past = false;
+#pragma unroll
+      for (uint32_t q = 0; q < 4; ++q) {
+        const uint32_t v = near[r][q] & kIndexMask;
+        const uint32_t s1 = geo.mod_m(poly(v) + kSeed1);
+        if (q < left[r] && !past && s1 == spot[r].slot) {
+          head[r] = v;
+          pos[r] = at + q;
+        }
+        past |= q < left[r] && s1 >= spot[r].slot;
+      }
+      if (left[r] <= 4u || past) break;
+      left[r] -= 4u;
+      at += 4u;
+      __builtin_memcpy(near[r], slab_idx + at, sizeof(near[r]));
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < kSettleRows; ++r) {
+    if ((uint32_t)(r * kSettleBlock) >= count || !(in & (1u << r))) continue;
+    const uint32_t local = cell[r] >> kSlabPartLog2;
+    if (head[r] < t[r]) {
+      sh.cells[cell[r]] |= kNone;
+      sh.dead[local] = 1;
+      token[atomicAdd(&sh.tokens, 1u)] = t[r] | kAtLevel3;
+      continue;
+    }
+    atomicAdd(&sh.alive[local], 1u);
+    if (head[r] != kNone) {
+      slab_idx[pos[r]] = (int32_t)(head[r] | kRemovedBit);
+      atomicAdd(&sh.pushed[local], 1u);
+      token[atomicAdd(&sh.tokens, 1u)] = head[r];
+    }
+  }
+  __syncthreads();
+  u32x4 *out = reinterpret_cast<u32x4 *>(cells + ((size_t)b0 << kSlabPartLog2));
+  for (uint32_t i = threadIdx.x; i < (buckets << kSlabPartLog2) / 2u; i += kSettleBlock) {
+    const u32x4 q = clear[i];
+    if (q.y | q.w) out[i] = q;  // (the map is zero)
+  }
+  if (threadIdx.x < buckets) {
+    tb.movein_n[(b0 + threadIdx.x) * kMoveinPad] = sh.alive[threadIdx.x];
+    tb.movein_n[(b0 + threadIdx.x) * kMoveinPad + 1u] = sh.dead[threadIdx.x];
+    tb.removed_n[b0 + threadIdx.x] = sh.pushed[threadIdx.x];
+  }
+  if (threadIdx.x == 0) tb.token_n[group] = sh.tokens;
+}
+
+// Levels 2 and 3 for the losers on the buckets' lists and for what k_slab_settle has left, one index to a lane, `share`
+// workgroups to a group of buckets and as few lanes of a wave as that allows: a wave goes on until the last of them has
+// found its place.  Bound by latency: a probe is three or four dependent trips to memory (the bucket's index, its records,
+// the map), with a wave to its lanes 1.2 us, and by what all wait for in the end, the layout.  62 M slots, 110 000 losers
+// 29.6 -> 25.8 us, 268 M, 18 000 15.8 -> 14.1, 12.9 M, 900 14.9 -> 11.2 (dense waves, a log in one place, divisions, a
+// layout by lines of its own to a lane); 72 000 left of 436 000 settled ones 23.
+__global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Probe g, SlabTables tb, unsigned long long *cells,
+                                                            uint32_t share, int64_t spp, uint32_t capacity,
+                                                            int64_t *__restrict__ splits, HostAnswer answer,
+                                                            int32_t *status) {
   __shared__ uint32_t s_scan[kSlabBlock / 64 + 1];
   __shared__ uint32_t s_start[kSlabMaxBuckets + 1];
+  __shared__ uint32_t s_serial, s_first;
   __shared__ bool s_last;
-  if (load_fresh(tb.losers) <= count_up_to) return;  // (nobody resets the number before every workgroup has counted)
-  const uint32_t b = blockIdx.x * (uint32_t)kLayoutBuckets + (threadIdx.x >> 6);
-  if (b < geo.nbuckets) {
-    constexpr int kLoads = (1 << kSlabPartLog2) / 128;
-    const u32x4 *part = reinterpret_cast<const u32x4 *>(cells + ((size_t)b << kSlabPartLog2)) + lane_id();
-    u32x4 two[kLoads];
+  if (threadIdx.x == 0) s_serial = 0;
+  __syncthreads();
+  const uint32_t group = blockIdx.x / share, part = group / tb.gpp, first = (group - part * tb.gpp) * tb.per_group;
+  const uint32_t b0 = part * geo.bpp + first;
+  const uint32_t buckets = geo.bpp - first < tb.per_group ? geo.bpp - first : tb.per_group;
+  // lane l of every wave knows where bucket l's list begins among all that there is to do; the tokens come last
+  const uint32_t lane = lane_id();
+  uint32_t mine = lane < buckets ? tb.again_n[b0 + lane] : 0u;
+  if (lane == kGroupBuckets && tb.group_cap) mine = tb.token_n[group];
+  const uint32_t incl = wave_inclusive_scan(mine);
+  const uint32_t count = (uint32_t)__builtin_amdgcn_readlane((int)incl, kGroupBuckets);
+  const uint32_t waves = share * (kSlabBlock / 64), wave = (blockIdx.x - group * share) * (kSlabBlock / 64) + threadIdx.x / 64;
+  uint32_t lanes = (count + waves - 1u) / waves;
+  lanes = lanes < 64u ? lanes : 64u;
+  // (a round has an index to a thread at most: so many are listed at most when the next one begins)
+  for (uint32_t i0 = 0; i0 < count; i0 += waves * lanes) {
+    const uint32_t i = lane < lanes ? i0 + wave * lanes + lane : count;
+    uint32_t list = 0, before = 0;
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) two[i] = part[i * 64];
-    uint32_t n = 0;  // (a taken cell's upper half is its slot and one)
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) n += (two[i].y != 0u) + (two[i].w != 0u);
-    n = wave_sum(n);
-    if (lane_id() == 0) __hip_atomic_store(&tb.movein_n[b * kMoveinPad], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (uint32_t l = 0; l < kGroupBuckets; ++l) {
+      const uint32_t end = (uint32_t)__builtin_amdgcn_readlane((int)incl, (int)l);
+      if (i >= end) {
+        list = l + 1u;
+        before = end;
+      }
+    }
+    if (i < count) {
+      const uint32_t t = list < kGroupBuckets ? tb.raw_idx[(size_t)(b0 + list) * kSlabCap + (i - before)]
+                                              : tb.token[(size_t)group * tb.group_cap + (i - before)];
+      slab_chain(geo, g, tb, cells, t & ~kAtLevel3, t & kAtLevel3 ? 2 : 1, s_start, &s_serial, status);
+    }
+    __syncthreads();
+    // those that found no slot, to their partition's list: one atomic (with one each those of a partition stood in line)
+    const uint32_t serial = s_serial;
+    if (threadIdx.x == 0 && serial) s_first = atomicAdd(&tb.serial_n[part * kMoveinPad], serial);
+    __syncthreads();
+    if (threadIdx.x < serial) {
+      const uint32_t at = s_first + threadIdx.x;
+      if (at < (uint32_t)kSlabSerialCap)
+        tb.ser_idx[(size_t)part * kSlabSerialCap + at] = s_start[threadIdx.x];
+      else  // more than the partition's serial region holds is an overflow; more than this path carries, a retry
+        atomicOr(status, (int64_t)at >= spp ? ZEN_STAT_SERIAL_OVERFLOW : ZEN_STAT_RETRY);
+    }
+    if (threadIdx.x == 0) s_serial = 0;
+    __syncthreads();
   }
+  // the workgroup that finishes last knows every count and lays out the output
   wait_global_acks();
   __syncthreads();
   if (threadIdx.x == 0) s_last = done_last(tb.done, blockIdx.x, gridDim.x);
@@ -741,9 +928,10 @@ __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, Slab
   sh.taken.template clear<kSlabBlock>(words);
   S mval[kCells];  // an entry is a copy of the element it stands for
 #pragma unroll
-  for (int e = 0; e < kCells; ++e) mval[e] = mv_n ? dense[(uint32_t)moved[e]] : S(0);
+  for (int e = 0; e < kCells; ++e) mval[e] = mv_n ? dense[cell_index(moved[e])] : S(0);
   __syncthreads();
   uint32_t off[kSlabItems], moff[kCells];
+  uint32_t in = 0;  // bit e: the cell holds an entry (it is not dead)
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
     off[i] = 0;
@@ -755,9 +943,10 @@ __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, Slab
 #pragma unroll
   for (int e = 0; e < kCells; ++e) {
     moff[e] = 0;
-    if (moved[e]) {
-      cell[e * kSlabBlock] = 0ull;
-      moff[e] = (uint32_t)(moved[e] >> 32) - 1u - lo;
+    if (moved[e]) cell[e * kSlabBlock] = 0ull;
+    if (moved[e] && (uint32_t)moved[e] != kNone) {
+      in |= 1u << e;
+      moff[e] = cell_slot(moved[e]) - lo;
       sh.taken.take(moff[e], 1u);
     }
   }
@@ -776,7 +965,7 @@ __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, Slab
   }
 #pragma unroll
   for (int e = 0; e < kCells; ++e) {
-    if (moved[e]) {
+    if (in & (1u << e)) {
       const uint32_t pos = out_base + sh.taken.place(moff[e]);
       if (pos < capacity) {
         out_idx[pos] = (int32_t)(uint32_t)moved[e];
@@ -855,7 +1044,7 @@ __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place_wide(SlabGeom geo,
     mplace[e] = mturn[e] = 0;
     if (moved[e]) {
       cell[e * kSlabBlock] = 0ull;
-      mplace[e] = lower_bound_u32(s_key, n, (uint32_t)(moved[e] >> 32) - 1u);
+      mplace[e] = lower_bound_u32(s_key, n, cell_slot(moved[e]));
       const uint32_t shift = 16u * (mplace[e] & 1u);
       mturn[e] = (atomicAdd(&s_cnt[mplace[e] >> 1], 1u << shift) >> shift) & 0xffffu;
     }
@@ -924,12 +1113,12 @@ __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place_wide(SlabGeom geo,
     };
 #pragma unroll
     for (int e = 0; e < kCells; ++e)
-      if (moved[e]) s_mk[front(mplace[e]) + mturn[e]] = (uint32_t)(moved[e] >> 32) - 1u;
+      if (moved[e]) s_mk[front(mplace[e]) + mturn[e]] = cell_slot(moved[e]);
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < kCells; ++e) {
       if (moved[e]) {
-        const uint32_t at = mplace[e], key = (uint32_t)(moved[e] >> 32) - 1u;
+        const uint32_t at = mplace[e], key = cell_slot(moved[e]);
         const uint32_t first = front(at), end = front(at + 1u);
         uint32_t rank = first;
         for (uint32_t u = first; u < end; ++u) rank += s_mk[u] < key;
@@ -984,9 +1173,20 @@ struct SlabPlan {
 };
 
 // `state` is memory that is zero between calls (see above); everything else comes out of the workspace.
-SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partitions, int dtype, int64_t list_cap) {
+SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partitions, int dtype, int64_t capacity) {
   SlabPlan p;
   const size_t B = geo.nbuckets;
+  const int64_t list_cap = list_capacity(capacity);
+  // The hash loses 1.4 times as many as evenly spread slots would.
+  const double losers = 0.7 * (double)capacity * ((double)capacity / geo.m);
+  p.tb.per_group = std::min(std::max((geo.nbuckets + kGroupsWanted - 1u) / kGroupsWanted, kGroupLeast), kGroupBuckets);
+  p.tb.gpp = (geo.bpp + p.tb.per_group - 1u) / p.tb.per_group;
+  p.tb.group_pad = (p.tb.gpp + 31u) & ~31u;
+  const size_t groups = (size_t)p.tb.gpp * partitions;
+  p.tb.group_cap = 0;
+  if (losers > kSettleFrom && geo.span <= kSlabSpan2 && p.tb.gpp <= kMostGroups &&
+      (size_t)partitions * p.tb.group_pad <= kMostGroupWords)
+    p.tb.group_cap = std::min((uint32_t)(1.25 * losers / (double)groups) + 512u, kGroupCap);
   {
     Carver cv(state);
     p.sample_hist[0] = cv.take<uint32_t>(sampled_floor_zero_bytes() / sizeof(uint32_t));
@@ -997,8 +1197,8 @@ SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partit
     p.feed.coarse_cursor = cv.take<uint32_t>(feed_coarse_cursor_words());
     p.tb.movein_n = cv.take<uint32_t>(B * kMoveinPad);
     p.tb.serial_n = cv.take<uint32_t>((size_t)partitions * kMoveinPad);
-    p.tb.losers = cv.take<uint32_t>(1);
     p.tb.done = cv.take<uint32_t>(kDoneWords);
+    p.tb.group_n = cv.take<uint32_t>(p.tb.group_cap ? (size_t)partitions * p.tb.group_pad : 1);
     p.refine_hist = cv.take<uint32_t>(dtype == ZEN_BF16 ? 1 : (size_t)kRefineWords);
     p.state_bytes = cv.used;
   }
@@ -1022,8 +1222,10 @@ SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partit
   p.tb.slab_val = cv.take<char>(B * kSlabCap * (dtype == ZEN_BF16 ? 2 : 4));
   p.tb.sub_index = cv.take<uint16_t>(B * kSlabIndexLen);
   p.tb.ser_idx = cv.take<uint32_t>((size_t)partitions * kSlabSerialCap);
-  p.tb.log_cap = (uint32_t)(list_cap / 4 + 1024);
-  p.tb.log_t = cv.take<uint32_t>(p.tb.log_cap);
+  p.tb.again_n = cv.take<uint32_t>(B);
+  p.tb.group_list = cv.take<uint32_t>(groups * p.tb.group_cap);
+  p.tb.token_n = cv.take<uint32_t>(groups);
+  p.tb.token = cv.take<uint32_t>(groups * p.tb.group_cap);
   p.bytes = cv.used;
   return p;
 }
@@ -1034,6 +1236,8 @@ int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPl
   const uint32_t B = geo.nbuckets;
   const uint32_t *filter = a.k > 0 ? p.thr : nullptr;
   const S *dense = static_cast<const S *>(a.input);
+  SlabTables tb = p.tb;
+  if (a.g.levels < 2) tb.group_cap = 0;  // (nothing to settle)
   {
     ProfScope prof(kProfFeed, s);
     const EncodeSink<S> sink{geo, p.tb.raw_idx, static_cast<S *>(p.tb.raw_val), filter};
@@ -1045,25 +1249,22 @@ int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPl
   {
     ProfScope prof(kProfSlabSort, s);
     if constexpr (SPAN > 0)
-      k_slab_sort<S, SPAN><<<dim3(B), dim3(kSortBlock), 0, s>>>(geo, p.tb, a.status);
+      (tb.group_cap ? k_slab_sort<S, SPAN, true> : k_slab_sort<S, SPAN, false>)<<<dim3(B), dim3(kSortBlock), 0, s>>>(geo, tb);
     else
-      k_slab_sort_wide<S><<<dim3(B), dim3(kSortBlock), 0, s>>>(geo, p.tb, a.status);
+      k_slab_sort_wide<S><<<dim3(B), dim3(kSortBlock), 0, s>>>(geo, tb, a.status);
     ZEN_LAUNCH_CHECK("k_slab_sort");
   }
   {
     ProfScope prof(kProfSlabChains, s);
-    // (as many workgroups as the chip holds; fewer where there can be few losers)
-    const int64_t groups = ceil_div((int64_t)p.tb.log_cap / 4, (int64_t)kSlabBlock);
-    const bool many = (double)a.capacity * (double)a.capacity > 2.0 * (double)geo.m * kLayoutFrom;
-    const uint32_t count_up_to = many ? kUncountedFrom : 0xffffffffu;
-    k_slab_chains<<<dim3((unsigned)(groups < 64 ? 64 : groups > 1024 ? 1024 : groups)), dim3(kSlabBlock), 0, s>>>(
-        geo, a.g, p.tb, a.hash, a.spp, (uint32_t)a.capacity, a.splits, count_up_to, a.ask.answer, a.status);
-    ZEN_LAUNCH_CHECK("k_slab_chains");
-    if (many) {
-      k_slab_layout<<<dim3((B + kLayoutBuckets - 1) / kLayoutBuckets), dim3(kSlabBlock), 0, s>>>(
-          geo, p.tb, a.hash, a.spp, (uint32_t)a.capacity, a.splits, count_up_to, a.ask.answer, a.status);
-      ZEN_LAUNCH_CHECK("k_slab_layout");
+    const uint32_t groups = tb.gpp * (uint32_t)tb.partitions;
+    if (tb.group_cap) {
+      k_slab_settle<<<dim3(groups), dim3(kSettleBlock), 0, s>>>(geo, tb, a.hash, a.status);
+      ZEN_LAUNCH_CHECK("k_slab_settle");
     }
+    const uint32_t share = std::min(std::max(kChainsResident / groups, 1u), 16u);
+    k_slab_chains<<<dim3(groups * share), dim3(kSlabBlock), 0, s>>>(geo, a.g, tb, a.hash, share, a.spp, (uint32_t)a.capacity,
+                                                                    a.splits, a.ask.answer, a.status);
+    ZEN_LAUNCH_CHECK("k_slab_chains");
     if (a.ask.answer.host) *a.ask.answered = true;
   }
   {
@@ -1103,7 +1304,7 @@ bool encode_geometry(int64_t m, int partitions, int64_t capacity, SlabGeom *geo)
 size_t slab_balance_bytes(int64_t m, int partitions, int dtype, int64_t capacity) {
   SlabGeom geo;
   if (!encode_geometry(m, partitions, capacity, &geo)) return 0;
-  return plan_slab(nullptr, nullptr, geo, partitions, dtype, list_capacity(capacity)).bytes;
+  return plan_slab(nullptr, nullptr, geo, partitions, dtype, capacity).bytes;
 }
 
 // The hash map takes the first 8 << hash_log2 bytes of the caller's table (at most half of it: zen_load_balance
@@ -1149,7 +1350,7 @@ int slab_load_balance(const SlabBalanceArgs &a, hipStream_t s) {
   if (!slab_balance_fits(a.n, a.g.m, a.partitions, a.dtype, a.capacity, a.k, &geo))
     return fail(ZEN_EINVAL, "slab_load_balance: sizes do not suit the slab layout");
   char *state = reinterpret_cast<char *>(a.hash) + slab_state_offset(a.hash_log2);
-  SlabPlan p = plan_slab(a.workspace, state, geo, a.partitions, a.dtype, list_capacity(a.capacity));
+  SlabPlan p = plan_slab(a.workspace, state, geo, a.partitions, a.dtype, a.capacity);
   if (slab_state_offset(a.hash_log2) + p.state_bytes > (size_t)a.g.m * sizeof(int32_t))
     return fail(ZEN_EINVAL, "slab_load_balance: table too small for the counters");
   // never with the geometries slab_geometry gives: a bucket spans 16384 slots or more, and there is a cell for about

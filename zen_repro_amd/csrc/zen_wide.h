@@ -67,6 +67,7 @@ inline bool wide_geometry(int64_t m, int partitions, int64_t expected, int cus, 
   g.sub_shift = 0;
   while ((width >> g.sub_shift) >= (uint64_t)kWideSubs) ++g.sub_shift;
   g.width = slab_bucket_width(g.bpp_mult);
+  g.npp_mult = slab_npp_mult(g.npp);
   g.inv_m = slab_inverse_below(g.m);
   g.inv_npp = slab_inverse_below(g.npp);
   *out = g;
