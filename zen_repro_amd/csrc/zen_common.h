@@ -303,25 +303,52 @@ __device__ inline uint64_t wave_sum(uint64_t v) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-// Exclusive scan over the threads of a block (BLOCK a multiple of 64).
-// `total` receives the block sum in every thread.  smem needs BLOCK/64 + 1 T's.
+// The value lane `lane` (the same for the whole wave) holds.
+__device__ inline uint32_t wave_read(uint32_t v, int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)v, lane); }
+__device__ inline uint64_t wave_read(uint64_t v, int lane) {
+  return ((uint64_t)wave_read((uint32_t)(v >> 32), lane) << 32) | wave_read((uint32_t)v, lane);
+}
+
+// The inclusive scan's steps inside rows of sixteen lanes.
+__device__ inline uint32_t row_inclusive_scan(uint32_t x) {
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+  return x;
+}
+__device__ inline uint64_t row_inclusive_scan(uint64_t x) {
+#define ZEN_STEP(ctrl)                                                                                                   \
+  {                                                                                                                      \
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, ctrl, 0xf, 0xf, false);               \
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), ctrl, 0xf, 0xf, false);       \
+    x += ((uint64_t)hi << 32) | lo;                                                                                      \
+  }
+  ZEN_STEP(0x111)
+  ZEN_STEP(0x112)
+  ZEN_STEP(0x114)
+  ZEN_STEP(0x118)
+#undef ZEN_STEP
+  return x;
+}
+
+// Exclusive scan over the threads of a block (all of them active).  `total` receives the block sum in every thread.
+// smem needs BLOCK/64 + 1 T's.  The waves' sums are scanned by the lanes of every wave, a lane a sum (a row of sixteen
+// lanes holds them all): the kernels of a thousand threads that scan between their steps are bound by vector instructions
+// and by the chain of their phases, and a loop over sixteen sums in every thread is 64 instructions (@SCAN@).
 template <typename T, int BLOCK>
 __device__ inline T block_exclusive_scan(T v, T *smem, T *total) {
   constexpr int kWaves = BLOCK / 64;
-  const int wave = threadIdx.x >> 6;
+  static_assert(BLOCK % 64 == 0 && kWaves >= 1 && kWaves <= 16 && (kWaves & (kWaves - 1)) == 0, "a row of lanes holds the waves' sums");
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const T incl = wave_inclusive_scan(v);
   if (lane_id() == 63) smem[wave] = incl;
   __syncthreads();
-  T wave_base = 0, sum = 0;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    const T s = smem[w];
-    if (w < wave) wave_base += s;
-    sum += s;
-  }
+  const T own = smem[lane_id() & (kWaves - 1)];
+  const T upto = row_inclusive_scan(own);  // right in the first kWaves lanes
   __syncthreads();
-  *total = sum;
-  return wave_base + incl - v;
+  *total = wave_read(upto, kWaves - 1);
+  return wave_read(upto - own, wave) + incl - v;
 }
 
 // ------------------------------------------------ single-pass prefix over tiles

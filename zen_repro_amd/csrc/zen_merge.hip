@@ -204,22 +204,22 @@ struct MergeSink {
 
 // The sums of a workgroup's n sorted records (indices in sh.key, value bits in sh.tie), in registers: record q of a thread
 // ends a run of equal indices, whose sum is kept, where bit q of the answer is set.
-template <typename O, typename Shared>
-__device__ inline uint32_t sum_runs(const Shared &sh, uint32_t n, uint32_t (&k)[kMergeItems], float (&sum)[kMergeItems]) {
+template <typename O, typename Shared, int ITEMS>
+__device__ inline uint32_t sum_runs(const Shared &sh, uint32_t n, uint32_t (&k)[ITEMS], float (&sum)[ITEMS]) {
   // Thread t owns the sorted places [t * per, (t + 1) * per): as few per thread as cover the bucket (and an odd
   // number, which keeps the lanes of a wave on different LDS banks).  It fetches them all at once and walks
   // through them in registers.  A run of equal indices is summed in arrival order from +0 (like the dense
   // tensor of comm.py:35) and belongs to the thread that holds its last record; where that run began before
   // the thread's first place (rare: runs are short next to `per`, long ones come from payloads that overlap),
   // the part in front is summed first, from the run's head on.
-  const uint32_t per = ((n + kMergeBlock - 1) / kMergeBlock) | 1u;  // <= kMergeItems
+  const uint32_t per = ((n + kMergeBlock - 1) / kMergeBlock) | 1u;  // <= ITEMS
   const uint32_t first = threadIdx.x * per;
   uint32_t keep = 0;
   {
     constexpr uint32_t kNoKey = 0xffffffffu;  // offsets are below the bucket width
-    float v[kMergeItems];
+    float v[ITEMS];
 #pragma unroll
-    for (int q = 0; q < kMergeItems; ++q) {
+    for (int q = 0; q < ITEMS; ++q) {
       const uint32_t p = first + q;
       const bool have = (uint32_t)q < per && p < n;
       const uint32_t from = have ? p : 0u;
@@ -236,8 +236,8 @@ __device__ inline uint32_t sum_runs(const Shared &sh, uint32_t n, uint32_t (&k)[
     }
     uint32_t prev = before_k;
 #pragma unroll
-    for (int q = 0; q < kMergeItems; ++q) {
-      const uint32_t next = q + 1 < kMergeItems ? ((uint32_t)(q + 1) < per ? k[q + 1] : after_k) : after_k;
+    for (int q = 0; q < ITEMS; ++q) {
+      const uint32_t next = q + 1 < ITEMS ? ((uint32_t)(q + 1) < per ? k[q + 1] : after_k) : after_k;
       if (k[q] != kNoKey) {
         if (k[q] != prev) acc = 0.0f;
         acc += v[q];

@@ -257,7 +257,7 @@ __device__ inline float sum_run_before(const uint32_t *key, const V *val, uint32
   return acc;
 }
 
-// Ranks the live records of a workgroup of BLOCK threads (kSlabCap / BLOCK records each) by (key offset, tie);
+// Ranks the live records of a workgroup of BLOCK threads (ITEMS records each) by (key offset, tie);
 // tie < 2^tie_bits, the pair unique, and
 // geo.sub_shift + tie_bits <= 32.  off[i] < bucket width.  The records are first grouped by narrow key range
 // with one LDS atomic each; a record is then one word, (offset inside the range) << tie_bits | tie, and
@@ -272,13 +272,13 @@ __device__ inline float sum_run_before(const uint32_t *key, const V *val, uint32
 // sh.pairs_most of others to be compared with, all of them together); else rank[i] for live records and *n_out = number of live records.  On return
 // sh.key / sh.tie may be overwritten at once (sh.tie is not touched at all), and the low 16 bits of
 // sh.cnt[sub_place(s)] hold the sorted place of the first record of narrow range s.
-template <int BLOCK, typename Shared>
+template <int BLOCK, typename Shared, int ITEMS>
 __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
-                                 const uint32_t (&off)[kSlabCap / BLOCK], const uint32_t (&tie)[kSlabCap / BLOCK],
-                                 uint32_t live, uint32_t (&rank)[kSlabCap / BLOCK], uint32_t *n_out) {
-  static_assert(BLOCK <= kSlabMaxBlock && kSlabCap % BLOCK == 0 && kSlabSubs % BLOCK == 0, "workgroup size");
+                                 const uint32_t (&off)[ITEMS], const uint32_t (&tie)[ITEMS],
+                                 uint32_t live, uint32_t (&rank)[ITEMS], uint32_t *n_out) {
+  static_assert(BLOCK <= kSlabMaxBlock && BLOCK * ITEMS <= kSlabCap && kSlabSubs % BLOCK == 0, "workgroup size");
   static_assert(kSlabCap < 65536, "two prefixes in one word");
-  constexpr int kItems = kSlabCap / BLOCK;
+  constexpr int kItems = ITEMS;
   constexpr int kSubsPer = kSlabSubs / BLOCK;
   for (int d = threadIdx.x; d <= kSlabSubs; d += BLOCK) sh.cnt[d] = 0;
   if (threadIdx.x == 0) {
