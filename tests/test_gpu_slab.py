@@ -547,6 +547,33 @@ def test_merge_of_groups_of_every_length(zen, oracle, times, dtype):
     assert np.array_equal(to_np(gv)[:len(want_i)].view(np.uint32), want_v.view(np.uint32))
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("piled", [3072, 3073, 4096, 4097, 5120, 5121, 6143, 6144])
+def test_slab_merge_at_a_row_of_records(zen, oracle, piled, dtype):
+    """The first of fourteen bucket slabs holds exactly `piled` records, a quarter of them on 64 indices, the others some
+    2800: the merge is written out for every number of rows of 1024 records, up to the slab's room."""
+    from zen_repro_amd import _lib
+
+    n, r, width = 14 << 19, 43000, 1 << 19
+    rng = np.random.default_rng(piled)
+    ci = rng.integers(width + 64, n, r)
+    first = rng.integers(0, width - 64, piled)
+    few = rng.choice(piled, piled // 4, replace=False)
+    first[few] = rng.choice(first, 64)[rng.integers(0, 64, len(few))]
+    ci[rng.choice(r, piled, replace=False)] = first
+    cv = (rng.standard_normal(r) * 1e-3).astype(np.float32)
+    if dtype == "bf16":
+        cv = oracle.f32_to_bf16_bits(cv)
+    want_i, want_v = oracle.merge_sparse(ci, cv, n)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    lba.fast_flags = _lib.MODE_SLABS
+    assert _lib.lib().zen_merge_path(r, n, _lib.MODE_FAST | _lib.MODE_SLABS) == 2
+    gi, gv, cnt, st = lba.merge_sparse_flat(to_dev(ci), to_dev(cv), n, mode=_lib.MODE_FAST)
+    assert st.item() == 0 and cnt.item() == len(want_i)
+    assert np.array_equal(to_np(gi)[:len(want_i)], want_i.astype(np.int32))
+    assert np.array_equal(to_np(gv)[:len(want_i)].view(np.uint32), want_v.view(np.uint32))
+
+
 @pytest.mark.parametrize("r", [1 << 19, (1 << 19) + 1, 1900000, 128 * 15360 + 1])
 def test_merge_that_waits_gives_the_same_on_half_and_all_of_the_chip(zen, oracle, r):
     """One list of r entries around the sizes where the number of wide buckets changes, against merge_sparse_flat."""

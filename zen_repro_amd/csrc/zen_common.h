@@ -168,7 +168,8 @@ struct SumAs<float> {
 template <>
 struct SumAs<uint16_t> {
   static __device__ inline uint16_t of(float v) { return f32_to_bf16_rne(v); }
-  static __device__ inline bool kept(float v) { return (f32_to_bf16_rne(v) & 0x7fffu) != 0; }
+  // (half of the smallest bf16 rounds to even, that is to zero; NaN is kept)
+  static __device__ inline bool kept(float v) { return (__float_as_uint(v) & 0x7fffffffu) > 0x8000u; }
 };
 
 // Waits until the global memory operations this wave has issued, stores and atomics without a return value
@@ -335,7 +336,8 @@ __device__ inline uint64_t row_inclusive_scan(uint64_t x) {
 // Exclusive scan over the threads of a block (all of them active).  `total` receives the block sum in every thread.
 // smem needs BLOCK/64 + 1 T's.  The waves' sums are scanned by the lanes of every wave, a lane a sum (a row of sixteen
 // lanes holds them all): the kernels of a thousand threads that scan between their steps are bound by vector instructions
-// and by the chain of their phases, and a loop over sixteen sums in every thread is 64 instructions (@SCAN@).
+// and by the chain of their phases, and a loop over sixteen sums in every thread is 64 instructions (k_slab_sort of 3.1 M
+// bf16 records 17.9 us, 17.0 so; k_wide_merge of as many 39.9 and 38.0).
 template <typename T, int BLOCK>
 __device__ inline T block_exclusive_scan(T v, T *smem, T *total) {
   constexpr int kWaves = BLOCK / 64;

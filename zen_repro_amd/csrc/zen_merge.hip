@@ -203,53 +203,112 @@ struct MergeSink {
 };
 
 // The sums of a workgroup's n sorted records (indices in sh.key, value bits in sh.tie), in registers: record q of a thread
-// ends a run of equal indices, whose sum is kept, where bit q of the answer is set.
+// ends a run of equal indices, whose sum is kept, where bit q of the answer is set.  Thread t owns the sorted places
+// [t * per, (t + 1) * per), per <= ITEMS odd, which keeps the lanes of a wave on different LDS banks.
 template <typename O, typename Shared, int ITEMS>
-__device__ inline uint32_t sum_runs(const Shared &sh, uint32_t n, uint32_t (&k)[ITEMS], float (&sum)[ITEMS]) {
-  // Thread t owns the sorted places [t * per, (t + 1) * per): as few per thread as cover the bucket (and an odd
-  // number, which keeps the lanes of a wave on different LDS banks).  It fetches them all at once and walks
-  // through them in registers.  A run of equal indices is summed in arrival order from +0 (like the dense
+__device__ inline uint32_t sum_runs(const Shared &sh, uint32_t n, uint32_t per, uint32_t (&k)[ITEMS], float (&sum)[ITEMS]) {
+  // It fetches them all at once (also what lies behind the last one, up to kSlabPad words past the slab, which counts for
+  // nothing) and walks through them in registers.  A run of equal indices is summed in arrival order from +0 (like the dense
   // tensor of comm.py:35) and belongs to the thread that holds its last record; where that run began before
   // the thread's first place (rare: runs are short next to `per`, long ones come from payloads that overlap),
   // the part in front is summed first, from the run's head on.
-  const uint32_t per = ((n + kMergeBlock - 1) / kMergeBlock) | 1u;  // <= ITEMS
+  static_assert(ITEMS <= kSlabPad, "words behind the records");
+  constexpr uint32_t kNoKey = 0xffffffffu;  // offsets are below the bucket width
   const uint32_t first = threadIdx.x * per;
+  const uint32_t left = first < n ? n - first : 0u;
+  const uint32_t own = left < per ? left : per;
+  const uint32_t from = first < (uint32_t)kSlabCap ? first : (uint32_t)kSlabCap;
+  float v[ITEMS];
+#pragma unroll
+  for (int q = 0; q < ITEMS; ++q) {
+    k[q] = sh.key[from + q];
+    v[q] = __uint_as_float(sh.tie[from + q]);
+  }
+  const uint32_t before = sh.key[from > 0 ? from - 1u : 0u], after = sh.key[first + per < n ? first + per : 0u];
+#pragma unroll
+  for (int q = 0; q < ITEMS; ++q) k[q] = (uint32_t)q < own ? k[q] : kNoKey;
+  const uint32_t before_k = first > 0 ? before : kNoKey;
+  const uint32_t after_k = first + per < n ? after : kNoKey;
+  float acc = 0.0f;
+  if (own && before_k == k[0] && after_k != before_k) {
+    // the run began before this thread's places and ends here: find its head, sum up to the place in front of `first`
+    acc = sum_run_before(sh.key, sh.tie, first, before_k);
+  }
   uint32_t keep = 0;
-  {
-    constexpr uint32_t kNoKey = 0xffffffffu;  // offsets are below the bucket width
-    float v[ITEMS];
 #pragma unroll
-    for (int q = 0; q < ITEMS; ++q) {
-      const uint32_t p = first + q;
-      const bool have = (uint32_t)q < per && p < n;
-      const uint32_t from = have ? p : 0u;
-      k[q] = sh.key[from];
-      v[q] = __uint_as_float(sh.tie[from]);
-      if (!have) k[q] = kNoKey;
-    }
-    const uint32_t before_k = first > 0 && first < n ? sh.key[first - 1] : kNoKey;
-    const uint32_t after_k = first + per < n ? sh.key[first + per] : kNoKey;
-    float acc = 0.0f;
-    if (first < n && before_k == k[0] && after_k != before_k) {
-      // the run began before this thread's places and ends here: find its head, sum up to the place in front of `first`
-      acc = sum_run_before(sh.key, sh.tie, first, before_k);
-    }
-    uint32_t prev = before_k;
-#pragma unroll
-    for (int q = 0; q < ITEMS; ++q) {
-      const uint32_t next = q + 1 < ITEMS ? ((uint32_t)(q + 1) < per ? k[q + 1] : after_k) : after_k;
-      if (k[q] != kNoKey) {
-        if (k[q] != prev) acc = 0.0f;
-        acc += v[q];
-        prev = k[q];
-        sum[q] = acc;
-        if (k[q] != next && SumAs<O>::kept(acc)) keep |= 1u << q;
-      } else {
-        sum[q] = 0.0f;
-      }
-    }
+  for (int q = 0; q < ITEMS; ++q) {
+    const uint32_t prev = q > 0 ? k[q > 0 ? q - 1 : 0] : before_k;
+    const uint32_t next = q + 1 < ITEMS ? ((uint32_t)(q + 1) < per ? k[q + 1 < ITEMS ? q + 1 : q] : after_k) : after_k;
+    acc = (k[q] != prev ? 0.0f : acc) + v[q];
+    sum[q] = acc;
+    keep |= ((uint32_t)q < own) & (k[q] != next) & SumAs<O>::kept(acc) ? 1u << q : 0u;
   }
   return keep;
+}
+
+// The first rows of a slab, loaded beside the number of its records (what lies behind the last one is read and not looked
+// at: the slab's memory is there), in no branch, so that all loads are in flight together.
+constexpr int kMergeAhead = 4;
+struct MergeAhead {
+  uint32_t idx[kMergeAhead], arr[kMergeAhead];
+};
+
+// A bucket's slab (`idx`, `arr`, `val`: n_raw records; indices from `lo` on): sorted, summed, and what is kept put side by
+// side to sh.key / sh.tie (visible behind a barrier).  Returns how many entries that are; false in *ranked if the indices
+// pile up.  ROWS records of a thread before the sort, ITEMS after it: written out for the numbers that occur, since what
+// bounds the kernel is vector instructions (with six rows and seven places for every bucket, addresses of 64 bits for every
+// access and counters in an order that took five instructions to find, 318 for every 64 records, 174 so): 6.2 M bf16 entries
+// of sixteen lists 74 -> 64 us, 10.7 M fp32 entries beside the encode's kernels 149 -> 137.
+template <typename S, typename O, int ROWS, int ITEMS>
+__device__ __forceinline__ uint32_t merge_rows(SlabSortShared &sh, const SlabGeom &geo, int tie_bits,
+                                               const MergeAhead &ahead, const uint32_t *__restrict__ idx,
+                                               const uint32_t *__restrict__ arr, const S *__restrict__ val, uint32_t n_raw,
+                                               uint32_t lo, bool *ranked) {
+  static_assert(kMergeBlock * ROWS <= kSlabCap && ITEMS % 2 == 1 && ROWS <= ITEMS, "the slab is there, every sorted place has an owner");
+  uint32_t off[ROWS], tie[ROWS], rank[ROWS];
+  uint32_t live = 0;
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const uint32_t j = threadIdx.x + i * kMergeBlock;
+    off[i] = i < kMergeAhead ? ahead.idx[i < kMergeAhead ? i : 0] : idx[j];
+    tie[i] = i < kMergeAhead ? ahead.arr[i < kMergeAhead ? i : 0] : arr[j];
+  }
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    off[i] -= lo;
+    live |= (threadIdx.x + i * kMergeBlock < n_raw ? 1u : 0u) << i;
+  }
+  uint32_t n = 0;
+  *ranked = slab_rank<kMergeBlock>(sh, geo, tie_bits, off, tie, live, rank, &n);
+  if (!*ranked) return 0;
+  // the values only now: kept across the ranking they cost registers that two workgroups a compute unit do not
+  // have (6.2 M records: 67 us instead of 64)
+  S v[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) v[i] = val[threadIdx.x + i * kMergeBlock];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    if (live & (1u << i)) {
+      sh.key[rank[i]] = off[i];
+      sh.tie[rank[i]] = __float_as_uint(KeyOf<S>::to_f32(v[i]));  // the arrival numbers have done their work: their place takes the values
+    }
+  }
+  __syncthreads();
+  uint32_t k[ITEMS];
+  float sum[ITEMS];
+  const uint32_t keep = sum_runs<O>(sh, n, (uint32_t)ITEMS, k, sum);
+  uint32_t total;
+  uint32_t at = block_exclusive_scan<uint32_t, kMergeBlock>((uint32_t)__popc(keep), sh.scan, &total);
+  // everybody is past reading the sorted bucket: the scan synchronised
+#pragma unroll
+  for (int q = 0; q < ITEMS; ++q) {
+    if (keep & (1u << q)) {
+      sh.key[at] = k[q] + lo;
+      sh.tie[at] = __float_as_uint(sum[q]);
+      ++at;
+    }
+  }
+  return total;
 }
 
 template <typename I, typename S, typename O>
@@ -263,87 +322,60 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
                                                              int64_t capacity, ScanState st, uint32_t *done, int tie_bits,
                                                              int64_t *out_count, HostAnswer answer, int32_t *status) {
   __shared__ SlabSortShared sh;  // the values take the counters' place once the ranks are known
-  __shared__ uint64_t s_scan64[kMergeBlock / 64 + 1];
   __shared__ int s_tile;
   if (threadIdx.x == 0) s_tile = (int)atomicAdd(st.ticket, 1u);
   __syncthreads();
-  const int b = s_tile;  // buckets are taken in order, so every earlier bucket already runs
+  const int b = __builtin_amdgcn_readfirstlane(s_tile);  // buckets are taken in order, so every earlier bucket already runs
   const int nb = (int)geo.nbuckets;
   if (b >= nb) return;
   const size_t base = (size_t)b * kSlabCap;
+  const uint32_t *idx = slab_idx + base, *arr = slab_arr + base;
+  const S *val = slab_val + base;
   uint32_t n_raw = cursor[b];
-  if (n_raw > (uint32_t)kSlabCap) n_raw = kSlabCap;  // the scatter flagged the overflow
   const uint32_t lo = bucket_lo[b];
+  MergeAhead ahead;
+#pragma unroll
+  for (int i = 0; i < kMergeAhead; ++i) {
+    ahead.idx[i] = idx[threadIdx.x + i * kMergeBlock];
+    ahead.arr[i] = arr[threadIdx.x + i * kMergeBlock];
+  }
+  if (n_raw > (uint32_t)kSlabCap) n_raw = kSlabCap;  // the scatter flagged the overflow
   // The counters of the scatter kernels go back to zero (this workgroup was the only reader of its slab's
   // count; the coarse cursors a slice per workgroup), and the last workgroup to finish clears the prefix
   // state: the memory that must be zero when a call starts is zero again when it ends.
   for (uint32_t i = (uint32_t)b * kMergeBlock + threadIdx.x; i < kCoarseCursorWords; i += (uint32_t)nb * kMergeBlock)
     coarse_cursor[i] = 0;
-  uint32_t off[kMergeRecs], arr[kMergeRecs], rank[kMergeRecs];
-  uint32_t live = 0;
-  // the loads sit in no branch (places past the end are pulled back onto the slab's first record), so that
-  // they are all in flight together
-#pragma unroll
-  for (int i = 0; i < kMergeRecs; ++i) {
-    const uint32_t j = threadIdx.x + i * kMergeBlock;
-    const size_t from = base + (j < n_raw ? j : 0u);
-    off[i] = slab_idx[from] - lo;
-    arr[i] = slab_arr[from];
-    if (j < n_raw) live |= 1u << i;
-  }
-  uint32_t n = 0;
-  const bool ranked = slab_rank<kMergeBlock>(sh, geo, tie_bits, off, arr, live, rank, &n);
-  if (threadIdx.x == 0) cursor[b] = 0;  // every thread has read it: slab_rank synchronised
-  if (!ranked) {
-    if (threadIdx.x == 0) atomicOr(status, ZEN_STAT_RETRY);
-    n = 0;  // the bucket contributes nothing; the prefix protocol still gets its (empty) tile
-  } else {
-    // the values only now: kept across the ranking they cost registers that two workgroups a compute unit do not
-    // have (5.8 M records: 101 us instead of 96)
-    S val[kMergeRecs];
-#pragma unroll
-    for (int i = 0; i < kMergeRecs; ++i) {
-      const uint32_t j = threadIdx.x + i * kMergeBlock;
-      val[i] = slab_val[base + (j < n_raw ? j : 0u)];
-    }
-#pragma unroll
-    for (int i = 0; i < kMergeRecs; ++i) {
-      if (live & (1u << i)) {
-        sh.key[rank[i]] = off[i];
-        sh.tie[rank[i]] = __float_as_uint(KeyOf<S>::to_f32(val[i]));  // the arrival numbers have done their work: their place takes the values
-      }
-    }
-  }
-  __syncthreads();
-  uint32_t k[kMergeItems];
-  float sum[kMergeItems];
-  const uint32_t keep = sum_runs<O>(sh, n, k, sum);
+  bool ranked;
   uint32_t total;
-  const uint32_t before = block_exclusive_scan<uint32_t, kMergeBlock>((uint32_t)__popc(keep), sh.scan, &total);
-  // where this bucket's output starts: the sum of what all earlier buckets keep.  Every thread asks for a
-  // few of them (bounded wait), nobody waits for a chain of prefixes; while the answers are on their way the
-  // kept entries are gathered in LDS (everybody is past reading the sorted bucket: the scan synchronised).
-  if (threadIdx.x == 0) desc_store(&st.desc[b], kDescAggregate | total);
+  if (n_raw <= 3u * kMergeBlock)
+    total = merge_rows<S, O, 3, 3>(sh, geo, tie_bits, ahead, idx, arr, val, n_raw, lo, &ranked);
+  else if (n_raw <= 4u * kMergeBlock)
+    total = merge_rows<S, O, 4, 5>(sh, geo, tie_bits, ahead, idx, arr, val, n_raw, lo, &ranked);
+  else if (n_raw <= 5u * kMergeBlock)
+    total = merge_rows<S, O, 5, 5>(sh, geo, tie_bits, ahead, idx, arr, val, n_raw, lo, &ranked);
+  else
+    total = merge_rows<S, O, kMergeRecs, kMergeItems>(sh, geo, tie_bits, ahead, idx, arr, val, n_raw, lo, &ranked);
+  if (threadIdx.x == 0) {
+    // where the next bucket's output starts: the sum of what all earlier buckets keep.  A bucket that was not ranked
+    // contributes nothing; the prefix protocol still gets its (empty) tile
+    desc_store(&st.desc[b], kDescAggregate | total);
+    cursor[b] = 0;  // every thread has read it: slab_rank synchronised
+    if (!ranked) atomicOr(status, ZEN_STAT_RETRY);
+  }
+  // Every thread asks for a few of the earlier buckets' counts (bounded wait), nobody waits for a chain of prefixes.
   constexpr int kAsk = kSlabMaxBuckets / kMergeBlock;
   uint64_t d[kAsk];
 #pragma unroll
   for (int e = 0; e < kAsk; ++e) {
     const int p = (int)threadIdx.x + e * kMergeBlock;
-    d[e] = p < b ? desc_load(&st.desc[p]) : kDescAggregate;
+    d[e] = kDescAggregate;
+    if (e * kMergeBlock < b && p < b) d[e] = desc_load(&st.desc[p]);
   }
-  uint32_t li = before;
-#pragma unroll
-  for (int q = 0; q < kMergeItems; ++q) {
-    if (keep & (1u << q)) {
-      sh.key[li] = k[q] + lo;
-      sh.tie[li] = __float_as_uint(sum[q]);
-      ++li;
-    }
-  }
-  uint64_t mine = 0;
+  uint32_t mine = 0;  // (fewer than 2^31 entries in all)
   bool gave_up = false;
 #pragma unroll
   for (int e = 0; e < kAsk; ++e) {
+    if (e * kMergeBlock >= b) break;
     const int p = (int)threadIdx.x + e * kMergeBlock;
     uint32_t spins = 0;
     while ((d[e] >> 62) == 0) {
@@ -354,24 +386,24 @@ __global__ __launch_bounds__(kMergeBlock, 8) void k_merge_bucket(SlabGeom geo, u
       __builtin_amdgcn_s_sleep(2);
       d[e] = desc_load(&st.desc[p]);
     }
-    mine += d[e] & kDescValue;
+    mine += (uint32_t)d[e];
   }
   if (gave_up) atomicOr(status, ZEN_STAT_INTERNAL);
-  uint64_t all_before;
-  block_exclusive_scan<uint64_t, kMergeBlock>(mine, s_scan64, &all_before);  // its barriers also publish the gathered entries
-  const uint64_t tile_start = all_before;
+  uint32_t tile_start;
+  block_exclusive_scan<uint32_t, kMergeBlock>(mine, sh.scan, &tile_start);  // its barriers also publish the gathered entries
   if (b == nb - 1 && threadIdx.x == 0) {
-    const uint64_t all = tile_start + total;
+    const uint64_t all = (uint64_t)tile_start + total;
     // (for the launch's last workgroup to read, on another die maybe)
     __hip_atomic_store(out_count, (int64_t)all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (all > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
   }
-  for (uint32_t i = threadIdx.x; i < total; i += kMergeBlock) {
-    const uint64_t pos = tile_start + i;
-    if (pos < (uint64_t)capacity) {
-      out_idx[pos] = (I)sh.key[i];
-      out_val[pos] = SumAs<O>::of(__uint_as_float(sh.tie[i]));
-    }
+  const uint64_t room = (uint64_t)capacity > tile_start ? (uint64_t)capacity - tile_start : 0;
+  const uint32_t fits = total < room ? total : (uint32_t)room;
+  I *const to_idx = out_idx + tile_start;
+  O *const to_val = out_val + tile_start;
+  for (uint32_t i = threadIdx.x; i < fits; i += kMergeBlock) {
+    to_idx[i] = (I)sh.key[i];
+    to_val[i] = SumAs<O>::of(__uint_as_float(sh.tie[i]));
   }
   // every workgroup has read the descriptors it needs before it gets here
   if (answer.host) wait_global_acks();  // its share of the status word, and the count
@@ -485,7 +517,8 @@ __global__ __launch_bounds__(kMergeBlock) void k_merge_one(SlabGeom geo, const v
   uint32_t k[kMergeItems];
   float sum[kMergeItems];
   // (a dense tensor takes every sum that is not zero, also one that rounds to -0)
-  const uint32_t keep = DENSE ? sum_runs<float>(sh, n, k, sum) : sum_runs<O>(sh, n, k, sum);
+  const uint32_t per = ((n + kMergeBlock - 1) / kMergeBlock) | 1u;  // as few places per thread as cover the list: <= kMergeItems
+  const uint32_t keep = DENSE ? sum_runs<float>(sh, n, per, k, sum) : sum_runs<O>(sh, n, per, k, sum);
   uint32_t total;
   if (DENSE) wait_global_acks();  // this wave's zeros are written (the scan's barriers: everybody's)
   uint32_t at = block_exclusive_scan<uint32_t, kMergeBlock>((uint32_t)__popc(keep), sh.scan, &total);

@@ -159,44 +159,35 @@ inline bool slab_geometry(int64_t m, int partitions, int64_t expected, int targe
   return true;
 }
 
-// Where the counter of narrow range s lives in SlabSortShared::cnt when BLOCK threads rank the slab: a thread
-// owns kSlabSubs / BLOCK consecutive ranges during the prefix step, and this keeps the lanes of a wave on
-// different LDS banks while they walk through their ranges.  Range kSlabSubs (the end marker) stays at index
-// kSlabSubs.
-template <int BLOCK>
-__device__ inline uint32_t sub_place(uint32_t s) {
-  constexpr uint32_t kPer = kSlabSubs / BLOCK;
-  return s < (uint32_t)kSlabSubs ? (s % kPer) * BLOCK + s / kPer : s;
-}
-
 // Shared memory of the in-LDS sort.  slab_rank does not touch `tie`: a caller fills it only after
 // slab_rank has returned and has no use for `cnt` from then on, so that the two share their memory:
 // LDS decides how many workgroups share a compute unit.
+constexpr int kSlabPad = 8;                               // words behind the records that may be read, not looked at
 constexpr int kSlabQueueCap = kSlabCap - kSlabSubs - 1;  // large-group records a workgroup sets aside
 constexpr int kSlabInline = 4;                            // groups up to this size are ranked by their own threads
 constexpr int kSlabPairsFrom = 16;                        // groups up to this size are not counted as pairs
 constexpr int kSlabQueueMin = 256;                        // records in larger groups below which nothing is set aside
-struct SlabSortShared {
+struct alignas(16) SlabSortShared {
   static constexpr bool kQueue = true;
   static constexpr bool kPairs = false;
-  uint32_t key[kSlabCap];
+  uint32_t key[kSlabCap + kSlabPad];
   union {
-    uint32_t tie[kSlabCap];
+    uint32_t tie[kSlabCap + kSlabPad];
     struct {
-      uint32_t cnt[kSlabSubs + 1];
+      uint32_t cnt[kSlabSubs + 1];  // at a multiple of 16 bytes
       uint32_t queue[kSlabQueueCap];  // the rest of the ties' memory: records of large groups (see slab_rank)
     };
   };
   uint32_t scan[kSlabMaxBlock / 64 + 1];
   uint32_t bad;
 };
-static_assert(kSlabSubs + 1 <= kSlabCap, "the counters fit under the ties");
+static_assert(kSlabSubs + 1 <= kSlabCap && (kSlabCap + kSlabPad) % 4 == 0, "the counters fit under the ties, and begin at a vector");
 
 // The same without the queue (whose code costs slab_rank registers).
-struct SlabSortSharedNoQueue {
+struct alignas(16) SlabSortSharedNoQueue {
   static constexpr bool kQueue = false;
   static constexpr bool kPairs = false;
-  uint32_t key[kSlabCap];
+  uint32_t key[kSlabCap + kSlabPad];
   union {
     uint32_t tie[kSlabCap];
     uint32_t cnt[kSlabSubs + 1];
@@ -271,39 +262,37 @@ __device__ inline float sum_run_before(const uint32_t *key, const V *val, uint32
 // group is too large for that (kSlabGroupLimit; with a Shared that counts pairs: if the records have more than
 // sh.pairs_most of others to be compared with, all of them together); else rank[i] for live records and *n_out = number of live records.  On return
 // sh.key / sh.tie may be overwritten at once (sh.tie is not touched at all), and the low 16 bits of
-// sh.cnt[sub_place(s)] hold the sorted place of the first record of narrow range s.
+// sh.cnt[s] hold the sorted place of the first record of narrow range s.
 template <int BLOCK, typename Shared, int ITEMS>
 __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
                                  const uint32_t (&off)[ITEMS], const uint32_t (&tie)[ITEMS],
                                  uint32_t live, uint32_t (&rank)[ITEMS], uint32_t *n_out) {
-  static_assert(BLOCK <= kSlabMaxBlock && BLOCK * ITEMS <= kSlabCap && kSlabSubs % BLOCK == 0, "workgroup size");
+  static_assert(BLOCK <= kSlabMaxBlock && BLOCK * ITEMS <= kSlabCap, "workgroup size");
+  static_assert(kSlabSubs == 4 * BLOCK, "a vector of counters to a thread");
   static_assert(kSlabCap < 65536, "two prefixes in one word");
-  constexpr int kItems = ITEMS;
-  constexpr int kSubsPer = kSlabSubs / BLOCK;
-  for (int d = threadIdx.x; d <= kSlabSubs; d += BLOCK) sh.cnt[d] = 0;
+  uint4 *const cnt4 = reinterpret_cast<uint4 *>(sh.cnt);
+  cnt4[threadIdx.x] = make_uint4(0, 0, 0, 0);
   if (threadIdx.x == 0) {
     sh.bad = 0;
     if constexpr (Shared::kPairs) sh.pairs = 0;
   }
   __syncthreads();
   const uint32_t low_mask = (1u << geo.sub_shift) - 1u;
-  uint32_t sub[kItems], at[kItems];
+  uint32_t at[ITEMS];
 #pragma unroll
-  for (int i = 0; i < kItems; ++i) {
-    sub[i] = at[i] = 0;
-    if (live & (1u << i)) {
-      sub[i] = off[i] >> geo.sub_shift;
-      at[i] = atomicAdd(&sh.cnt[sub_place<BLOCK>(sub[i])], 1u);
-    }
+  for (int i = 0; i < ITEMS; ++i) {
+    at[i] = 0;
+    if (live & (1u << i)) at[i] = atomicAdd(&sh.cnt[off[i] >> geo.sub_shift], 1u);
   }
   __syncthreads();
   {
-    uint32_t c[kSubsPer];
-    uint32_t sum = 0, big = 0, pairs = 0;  // sum: records in the low half, records of groups larger than kSlabInline in the high half
+    const uint4 q = cnt4[threadIdx.x];
+    const uint32_t c[4] = {q.x, q.y, q.z, q.w};
+    uint32_t add[4];  // records in the low half, records of groups larger than kSlabInline in the high half
+    uint32_t big = 0, pairs = 0;
 #pragma unroll
-    for (int e = 0; e < kSubsPer; ++e) {
-      c[e] = sh.cnt[e * BLOCK + threadIdx.x];
-      sum += c[e] + (c[e] > (uint32_t)kSlabInline ? c[e] << 16 : 0u);
+    for (int e = 0; e < 4; ++e) {
+      add[e] = c[e] | (c[e] > (uint32_t)kSlabInline ? c[e] << 16 : 0u);
       if constexpr (Shared::kPairs)
         pairs += c[e] > (uint32_t)kSlabPairsFrom ? c[e] * c[e] : 0u;
       else
@@ -314,72 +303,66 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
       if (pairs) atomicAdd(&sh.pairs, pairs);
     }
     uint32_t total;
-    uint32_t running = block_exclusive_scan<uint32_t, BLOCK>(sum, sh.scan, &total);
-#pragma unroll
-    for (int e = 0; e < kSubsPer; ++e) {
-      sh.cnt[e * BLOCK + threadIdx.x] = running;
-      running += c[e] + (c[e] > (uint32_t)kSlabInline ? c[e] << 16 : 0u);
-    }
-    if (threadIdx.x == BLOCK - 1) sh.cnt[kSlabSubs] = running;  // = total
+    const uint32_t b0 = block_exclusive_scan<uint32_t, BLOCK>(add[0] + add[1] + add[2] + add[3], sh.scan, &total);
+    const uint32_t b1 = b0 + add[0], b2 = b1 + add[1], b3 = b2 + add[2];
+    cnt4[threadIdx.x] = make_uint4(b0, b1, b2, b3);
+    if (threadIdx.x == BLOCK - 1) sh.cnt[kSlabSubs] = total;
   }
   __syncthreads();
   if (sh.bad) return false;
   if constexpr (Shared::kPairs) {
     if (sh.pairs > sh.pairs_most) return false;
   }
-  const uint32_t totals = sh.cnt[kSlabSubs];
+  const uint32_t totals = (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.cnt[kSlabSubs]);
   // a few large groups are not worth the extra barrier
   const bool set_aside = Shared::kQueue && (totals >> 16) >= (uint32_t)kSlabQueueMin;
   constexpr uint32_t kSetAside = 0x80000000u;
-  uint32_t g0[kItems], g1[kItems], word[kItems];
+  uint32_t g0[ITEMS], size[ITEMS], word[ITEMS];
 #pragma unroll
-  for (int i = 0; i < kItems; ++i) {
-    g0[i] = g1[i] = word[i] = rank[i] = 0;
+  for (int i = 0; i < ITEMS; ++i) {
+    g0[i] = size[i] = word[i] = rank[i] = 0;
     if (live & (1u << i)) {
-      const uint32_t here = sh.cnt[sub_place<BLOCK>(sub[i])];
+      const uint32_t sub = off[i] >> geo.sub_shift;
+      const uint32_t here = sh.cnt[sub], next = sh.cnt[sub + 1];
       g0[i] = here & 0xffffu;
-      g1[i] = sh.cnt[sub_place<BLOCK>(sub[i] + 1)] & 0xffffu;
+      size[i] = (next & 0xffffu) - g0[i];
       word[i] = ((off[i] & low_mask) << tie_bits) | tie[i];
       sh.key[g0[i] + at[i]] = word[i];
       if constexpr (Shared::kQueue) {
         static_assert(kSlabSubs <= (1 << 12) && kSlabGroupLimit <= (1 << 19) && kSlabCap <= (1 << 19), "a queue entry is one word");
-        const uint32_t q = (here >> 16) + at[i];
-        if (set_aside && g1[i] - g0[i] > (uint32_t)kSlabInline && q < (uint32_t)kSlabQueueCap) {
-          sh.queue[q] = sub[i] | (at[i] << 12);  // sub < 2^12, at < group size <= kSlabGroupLimit
-          rank[i] = kSetAside | q;
-          g1[i] = g0[i];  // nothing left to do for it below
+        if (set_aside) {
+          const uint32_t q = (here >> 16) + at[i];
+          if (size[i] > (uint32_t)kSlabInline && q < (uint32_t)kSlabQueueCap) {
+            sh.queue[q] = sub | (at[i] << 12);  // sub < 2^12, at < group size <= kSlabGroupLimit
+            rank[i] = kSetAside | q;
+            size[i] = 0;  // nothing left to do for it below
+          }
         }
       }
     }
   }
   __syncthreads();
-  // the first kRankAhead words of every record's group, those of kBatch records fetched before any is looked
-  // at (most groups are no larger); the rest of a group by count_less
-#ifndef ZEN_RANK_AHEAD
-#define ZEN_RANK_AHEAD 2
-#endif
-  constexpr int kRankAhead = ZEN_RANK_AHEAD;
-  constexpr int kBatch = kItems % 3 == 0 ? 3 : kItems;
+  // the first kAhead words of every record's group (what lies behind the group is read and not looked at), those of kBatch
+  // records fetched before any is looked at (most groups are no larger); the rest of a group by count_less
+  constexpr int kAhead = Shared::kQueue ? kSlabInline : 2;
+  constexpr int kBatch = ITEMS == 4 ? 2 : ITEMS < 3 ? ITEMS : 3;
+  static_assert(kAhead <= kSlabPad && kAhead <= 4, "words behind the records");
 #pragma unroll
-  for (int h = 0; h < kItems; h += kBatch) {
-    if (live >> h == 0) continue;
-    uint32_t a[kBatch][kRankAhead];
+  for (int h = 0; h < ITEMS; h += kBatch) {
+    uint32_t a[kBatch][kAhead];
 #pragma unroll
-    for (int i = 0; i < kBatch; ++i) {
-      const uint32_t last = g1[h + i] > g0[h + i] ? g1[h + i] - 1u : g0[h + i];
+    for (int i = 0; i < kBatch && h + i < ITEMS; ++i) {
 #pragma unroll
-      for (int j = 0; j < kRankAhead; ++j) a[i][j] = sh.key[g0[h + i] + j < last ? g0[h + i] + j : last];
+      for (int j = 0; j < kAhead; ++j) a[i][j] = sh.key[g0[h + i] + j];
     }
 #pragma unroll
-    for (int i = 0; i < kBatch; ++i) {
-      if (g1[h + i] > g0[h + i]) {
-        uint32_t less = 0;
+    for (int i = 0; i < kBatch && h + i < ITEMS; ++i) {
+      uint32_t less = a[i][0] < word[h + i] ? 1u : 0u;
 #pragma unroll
-        for (int j = 0; j < kRankAhead; ++j) less += g0[h + i] + j < g1[h + i] && a[i][j] < word[h + i];
-        const uint32_t size = g1[h + i] - g0[h + i];
-        if (size > (uint32_t)kRankAhead) less += count_less(sh.key, g0[h + i] + kRankAhead, g1[h + i], word[h + i]);
-        rank[h + i] = g0[h + i] + less;
-      }
+      for (int j = 1; j < kAhead; ++j) less += (size[h + i] > (uint32_t)j) & (a[i][j] < word[h + i]) ? 1u : 0u;
+      if (size[h + i] > (uint32_t)kAhead)
+        less += count_less(sh.key, g0[h + i] + kAhead, g0[h + i] + size[h + i], word[h + i]);
+      if (!Shared::kQueue || rank[h + i] == 0) rank[h + i] = g0[h + i] + less;
     }
   }
   if constexpr (Shared::kQueue) {
@@ -389,13 +372,13 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
 #pragma unroll 1
       for (uint32_t q = threadIdx.x; q < queued; q += BLOCK) {
         const uint32_t e = sh.queue[q];
-        const uint32_t b0 = sh.cnt[sub_place<BLOCK>(e & 4095u)] & 0xffffu;
-        const uint32_t b1 = sh.cnt[sub_place<BLOCK>((e & 4095u) + 1)] & 0xffffu;
+        const uint32_t b0 = sh.cnt[e & 4095u] & 0xffffu;
+        const uint32_t b1 = sh.cnt[(e & 4095u) + 1] & 0xffffu;
         sh.queue[q] = b0 + count_less(sh.key, b0, b1, sh.key[b0 + (e >> 12)]);
       }
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < kItems; ++i)
+      for (int i = 0; i < ITEMS; ++i)
         if (rank[i] & kSetAside) rank[i] = sh.queue[rank[i] & ~kSetAside];
     }
   }

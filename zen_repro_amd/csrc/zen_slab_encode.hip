@@ -388,7 +388,7 @@ __global__ __launch_bounds__(kSortBlock, 8) void k_slab_sort_wide(SlabGeom geo, 
   // the counters hold where every narrow range starts in the sorted bucket: every kSlabIndexStep-th goes to
   // the index (before the counters' memory is used for the ties below)
   for (int j = threadIdx.x; j < kSlabIndexLen; j += kSortBlock)
-    tb.sub_index[(size_t)b * kSlabIndexLen + j] = (uint16_t)sh.cnt[sub_place<kSortBlock>((uint32_t)j * kSlabIndexStep)];
+    tb.sub_index[(size_t)b * kSlabIndexLen + j] = (uint16_t)sh.cnt[j * kSlabIndexStep];
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kSortItems; ++i) {
