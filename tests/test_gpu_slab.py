@@ -574,6 +574,36 @@ def test_slab_merge_at_a_row_of_records(zen, oracle, piled, dtype):
     assert np.array_equal(to_np(gv)[:len(want_i)].view(np.uint32), want_v.view(np.uint32))
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("piled", [5120, 5121, 9216, 9217, 13312, 13313, 16383, 16384])
+def test_wide_merge_at_a_number_of_places(zen, oracle, piled, dtype):
+    """The first of 128 wide buckets holds exactly `piled` records, a quarter of them on 64 indices: the sums are written out
+    for 5, 9, 13 and 17 places a thread."""
+    from zen_repro_amd import _lib
+
+    n, r, width = 1 << 24, 128 * 8000, 1 << 17
+    rng = np.random.default_rng(piled)
+    ci = rng.integers(width + 64, n, r)
+    first = rng.integers(0, width - 64, piled)
+    few = rng.choice(piled, piled // 4, replace=False)
+    first[few] = rng.choice(first, 64)[rng.integers(0, 64, len(few))]
+    ci[rng.choice(r, piled, replace=False)] = first
+    cv = (rng.standard_normal(r) * 1e-3).astype(np.float32)
+    if dtype == "bf16":
+        cv = oracle.f32_to_bf16_bits(cv)
+    want_i, want_v = oracle.merge_sparse(ci, cv, n)
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    gi, gv, cnt, st = lba.merge_sparse_flat(to_dev(ci), to_dev(cv), n, mode=_lib.MODE_FAST)
+    # (on the slabs alone a bucket of a third of them is too much)
+    if not FLAGS:
+        assert st.item() == 0 and cnt.item() == len(want_i)
+        assert np.array_equal(to_np(gi)[:len(want_i)], want_i.astype(np.int32))
+        assert np.array_equal(to_np(gv)[:len(want_i)].view(np.uint32), want_v.view(np.uint32))
+    dense = lba.decode_sparse_tensors(to_dev(ci), to_dev(cv), n)
+    f32 = oracle.decode(ci, cv, n, "f32acc")
+    assert np.array_equal(to_np(dense), oracle.f32_to_bf16_bits(f32) if dtype == "bf16" else f32)
+
+
 @pytest.mark.parametrize("r", [1 << 19, (1 << 19) + 1, 1900000, 128 * 15360 + 1])
 def test_merge_that_waits_gives_the_same_on_half_and_all_of_the_chip(zen, oracle, r):
     """One list of r entries around the sizes where the number of wide buckets changes, against merge_sparse_flat."""

@@ -81,52 +81,58 @@ inline uint32_t wide_part_cap(const SlabGeom &geo, int64_t list_cap) {
   return (uint32_t)((share + share / 4 + 1024 + 63) / 64 * 64);
 }
 
-// Counters of the narrow ranges: 16 bits each, two to a word.  Thread t of the workgroup owns ranges
-// 16 t .. 16 t + 15 when the counts become running sums; range s is kept at place (s % 16) * 1024 + s / 16, so
-// that the lanes of a wave then walk through consecutive halfwords (and the atomics of the counting steps, on
-// ranges that a hash picks, spread over the banks whatever the layout).
+// Counters of the narrow ranges: 16 bits each, two to a word, in order.  Thread t of the workgroup owns ranges
+// 16 t .. 16 t + 15, two vectors, when the counts become running sums; where a range begins is where the one before it
+// ends, so that both are read at immediate distances of one address.  (Spread over the array, so that a thread's sixteen were
+// sixteen reads of consecutive halfwords, a range took five instructions to find: zen_wide_merge.hip has the figures.)
 struct alignas(16) WideCounters {
+  uint32_t none[4];  // in front of range 0: the last half is zero
   uint32_t word[kWideSubs / 2];
+  using Pair = uint16_t __attribute__((ext_vector_type(2)));
   static_assert(kWideSubs == 16 * kWideBlock, "sixteen ranges per thread");
-  __device__ static inline uint32_t place(uint32_t sub) { return ((sub & 15u) << 10) | (sub >> 4); }
+  __device__ inline uint16_t *half() { return reinterpret_cast<uint16_t *>(word); }
   __device__ inline const uint16_t *half() const { return reinterpret_cast<const uint16_t *>(word); }
   __device__ inline void clear() {
-    for (int i = threadIdx.x; i < kWideSubs / 2; i += kWideBlock) word[i] = 0;
+    uint4 *v = reinterpret_cast<uint4 *>(word);
+    v[threadIdx.x] = v[kWideBlock + threadIdx.x] = make_uint4(0, 0, 0, 0);
+    if (threadIdx.x == 0) none[3] = 0;
   }
-  __device__ inline void count(uint32_t sub) {
-    const uint32_t p = place(sub);
-    atomicAdd(&word[p >> 1], 1u << (16 * (p & 1u)));
-  }
+  __device__ inline void count(uint32_t sub) { atomicAdd(&word[sub >> 1], 1u << (16 * (sub & 1u))); }
   // takes the next place of range `sub` (after starts() the counters are running cursors)
   __device__ inline uint32_t take(uint32_t sub) {
-    const uint32_t p = place(sub), sh = 16 * (p & 1u);
-    return (atomicAdd(&word[p >> 1], 1u << sh) >> sh) & 0xffffu;
+    const uint32_t sh = 16 * (sub & 1u);
+    return (atomicAdd(&word[sub >> 1], 1u << sh) >> sh) & 0xffffu;
   }
   // once every record has taken its place the counter of range s holds where the range ends
-  __device__ inline uint32_t end_of(uint32_t sub) const { return half()[place(sub)]; }
-  __device__ inline uint32_t start_of(uint32_t sub) const { return sub ? half()[place(sub - 1u)] : 0u; }
+  __device__ inline uint32_t end_of(uint32_t sub) const { return half()[sub]; }
+  __device__ inline uint32_t start_of(uint32_t sub) const { return (half() + sub)[-1]; }
   // Counts -> exclusive starts, by the whole workgroup; returns the number of records counted and sets *big
   // (a word of LDS, zero before) if any range holds more than `limit` of them; the caller may read *big once
   // it has synchronised.  smem: kWideBlock / 64 + 1 words.
   __device__ inline uint32_t starts(uint32_t *smem, uint32_t limit, uint32_t *big) {
-    uint16_t *h = reinterpret_cast<uint16_t *>(word);
-    uint32_t c[16];
-    uint32_t sum = 0, over = 0;
+    uint4 *v = reinterpret_cast<uint4 *>(word) + 2 * threadIdx.x;
+    const uint4 lo = v[0], hi = v[1];
+    const uint32_t c[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    Pair sum = {0, 0}, most = {0, 0};  // fewer records than 2^16 in all
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      c[e] = h[e * kWideBlock + threadIdx.x];
-      sum += c[e];
-      over |= c[e] > limit;
+    for (int e = 0; e < 8; ++e) {
+      const Pair p = __builtin_bit_cast(Pair, c[e]);
+      sum += p;
+      most = __builtin_elementwise_max(most, p);
     }
+    if ((most.x > most.y ? most.x : most.y) > limit) *big = 1u;
     uint32_t total;
-    if (over) *big = 1u;
-    uint32_t run = block_exclusive_scan<uint32_t, kWideBlock>(sum, smem, &total);
+    uint32_t run = block_exclusive_scan<uint32_t, kWideBlock>((uint32_t)sum.x + sum.y, smem, &total);
     if (total <= 0xffffu) {  // more than the counters hold: the caller gives up anyway
+      uint32_t to[8];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        h[e * kWideBlock + threadIdx.x] = (uint16_t)run;
-        run += c[e];
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t second = run + (c[e] & 0xffffu);
+        to[e] = run | (second << 16);
+        run = second + (c[e] >> 16);
       }
+      v[0] = make_uint4(to[0], to[1], to[2], to[3]);
+      v[1] = make_uint4(to[4], to[5], to[6], to[7]);
     }
     return total;
   }

@@ -19,7 +19,8 @@ constexpr int kWmPartMax = kWideBlock * kWmRounds;         // records of one par
 constexpr int kWmLanes = 4;                                // records a thread handles per step of the ranking loops
 constexpr int kWmQueue = 6144;                             // records of large groups set aside while ranking
 constexpr int kWmGroupLimit = 2048;                        // records in one narrow range: bounds the rank loop
-constexpr int kWmSumItems = 17;                            // sorted records per thread while summing (odd: no LDS bank conflicts)
+constexpr int kWmSumItems = 17;                            // sorted records per thread while summing, at most (odd: no LDS bank conflicts)
+constexpr int kWmPad = 20;                                 // words behind the records that may be read, not looked at
 constexpr uint32_t kInvalid = 0xffffffffu;
 static_assert(kWideBlock * kWmSumItems >= kWideCap, "every sorted place needs an owner");
 static_assert(kWmQueue <= (1 << 14) && kWideCap <= (1 << 14) && kWideSubs <= (1 << 14), "queue entries in one word");
@@ -43,16 +44,15 @@ __global__ __launch_bounds__(kWsBlock) void k_wide_scatter(WideList list) {
 
 struct WideMergeShared {
   union {
-    uint32_t word[kWideCap];  // while ranking: (index inside its narrow range) << tie_bits | arrival number
-    uint32_t key[kWideCap];   // afterwards: the sorted indices (minus the bucket's first), then the kept ones
+    uint32_t word[kWideCap + kWmPad];  // while ranking: (index inside its narrow range) << tie_bits | arrival number
+    uint32_t key[kWideCap + kWmPad];   // afterwards: the sorted indices (minus the bucket's first), then the kept ones
   };
   union {
     WideCounters cnt;
-    float val[kWideCap];      // the sorted values, then the kept sums
+    float val[kWideCap + kWmPad];      // the sorted values, then the kept sums
   };
   uint32_t queue[kWmQueue];   // records set aside: place in `word` | narrow range << 14, then the rank
   uint32_t scan[kWideBlock / 64 + 1];
-  uint64_t scan64[kWideBlock / 64 + 1];
   uint32_t qn, big;
   int tile;
 };
@@ -63,7 +63,7 @@ struct WideMergeShared {
 // the loops' bodies handle the first kWmLanes registers of a set and then rotate the set, and the values are loaded at the
 // end (written out for 24 records the code would not fit the instruction cache, and every workgroup runs it once).  A
 // chain of trips to LDS and memory: 62 M bf16, 3.1 M entries, 256 buckets of two rounds 39.2 us to index lists and 52.1
-// dense (42.6 and 55.0 at the time, with the loops for those too 48.2 and 59.0); 9 M, 0.9 M entries, one round 26.8 and 32.4.
+// dense at the time (42.6 and 55.0 before, with the loops for those too 48.2 and 59.0); 9 M, 0.9 M entries, one round 26.8 and 32.4.
 template <typename S, int ROUNDS, typename Zero>
 __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &geo, const WideSlabs &in, uint32_t b,
                                            const uint32_t (&pcount)[kWideSplit], uint32_t longest, bool declined,
@@ -196,18 +196,18 @@ __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &
     }
 #pragma unroll
     for (int k = 0; k < kWmLanes; ++k) {
-      const uint32_t last = g1[k] > g0[k] ? g1[k] - 1u : g0[k];
 #pragma unroll
-      for (int e = 0; e < kAhead; ++e) a[k][e] = sh.word[g0[k] + e < last ? g0[k] + e : last];
+      for (int e = 0; e < kAhead; ++e) a[k][e] = sh.word[g0[k] + e];  // what lies behind the range is not looked at
     }
 #pragma unroll
     for (int k = 0; k < kWmLanes; ++k) {
       if (ps[from + k] != kInvalid) {
-        uint32_t less = 0;
+        const uint32_t size = g1[k] - g0[k];
+        uint32_t less = a[k][0] < w[from + k] ? 1u : 0u;
 #pragma unroll
-        for (int e = 0; e < kAhead; ++e) less += g0[k] + e < g1[k] && a[k][e] < w[from + k];
+        for (int e = 1; e < kAhead; ++e) less += (size > (uint32_t)e) & (a[k][e] < w[from + k]) ? 1u : 0u;
         uint32_t x = g0[k] + less;
-        if (g1[k] - g0[k] > (uint32_t)kAhead) {
+        if (size > (uint32_t)kAhead) {
           const uint32_t at = atomicAdd(&sh.qn, 1u);
           if (at < (uint32_t)kWmQueue) {
             sh.queue[at] = ps[from + k];
@@ -297,6 +297,69 @@ __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &
   return n;
 }
 
+// The sums of the n sorted records, what is kept of them put side by side to sh.key (plus `lo`) / sh.val (visible behind a
+// barrier); returns how many.  publish(total) is called before they are put there.  Thread t owns the sorted places
+// [t * ITEMS, (t + 1) * ITEMS), fetches them all at once (also what lies behind the last one, which counts for nothing) and
+// walks through them in registers.  A run of equal indices is summed in arrival order from +0 (like the dense
+// tensor of comm.py:35) and belongs to the thread that holds its last record; where that run began before
+// the thread's first place (rare: runs are short next to ITEMS, long ones come from payloads that overlap),
+// the part in front is summed first, from the run's head on.  Bound by vector instructions with four waves to a SIMD to
+// hide them: 218 for every record and lane with places for a full bucket in every one, checks on every word read ahead and
+// ranges that took five instructions to find; 62 M bf16, 3.1 M entries, 256 buckets of 12 000 records 38.0 -> 34.7 us, dense
+// 51.5 -> 48.8; 268 M, 2.7 M entries 36.6 -> 33.0; 0.3 M entries in 128 buckets beside the encode 17.4 -> 14.5.
+template <typename O, bool DENSE, int ITEMS, typename Publish>
+__device__ __forceinline__ uint32_t wide_merge_sums(WideMergeShared &sh, uint32_t n, uint32_t lo, Publish publish) {
+  static_assert(ITEMS <= kWmPad && ITEMS % 2 == 1, "words behind the records");
+  constexpr uint32_t kNoKey = 0xffffffffu;  // offsets are below the bucket width
+  const uint32_t first = threadIdx.x * (uint32_t)ITEMS;
+  const uint32_t left = first < n ? n - first : 0u;
+  const uint32_t own = left < (uint32_t)ITEMS ? left : (uint32_t)ITEMS;
+  const uint32_t from = first < (uint32_t)kWideCap ? first : (uint32_t)kWideCap;
+  uint32_t k[ITEMS];
+  float sum[ITEMS];
+  uint32_t keep = 0;
+  {
+    float v[ITEMS];
+#pragma unroll
+    for (int q = 0; q < ITEMS; ++q) {
+      k[q] = sh.key[from + q];
+      v[q] = sh.val[from + q];
+    }
+    const uint32_t before = sh.key[from > 0 ? from - 1u : 0u], after = sh.key[first + ITEMS < n ? first + ITEMS : 0u];
+#pragma unroll
+    for (int q = 0; q < ITEMS; ++q) k[q] = (uint32_t)q < own ? k[q] : kNoKey;
+    const uint32_t before_k = first > 0 ? before : kNoKey;
+    const uint32_t after_k = first + ITEMS < n ? after : kNoKey;
+    float acc = 0.0f;
+    if (own && before_k == k[0]) {
+      // the run began before this thread's places: find its head, sum up to the place in front of `first`
+      acc = sum_run_before(sh.key, sh.val, first, before_k);
+    }
+#pragma unroll
+    for (int q = 0; q < ITEMS; ++q) {
+      const uint32_t prev = q > 0 ? k[q > 0 ? q - 1 : 0] : before_k;
+      const uint32_t next = q + 1 < ITEMS ? k[q + 1 < ITEMS ? q + 1 : q] : after_k;
+      acc = (k[q] != prev ? 0.0f : acc) + v[q];
+      sum[q] = acc;
+      keep |= ((uint32_t)q < own) & (k[q] != next) & (DENSE ? acc != 0.0f : SumAs<O>::kept(acc)) ? 1u << q : 0u;
+    }
+  }
+  if (DENSE) wait_global_acks();  // this wave's zeros are written (the scan's barrier: everybody's)
+  uint32_t total;
+  uint32_t li = block_exclusive_scan<uint32_t, kWideBlock>((uint32_t)__popc(keep), sh.scan, &total);
+  publish(total);
+  // everybody is past reading the sorted bucket: the scan synchronised
+#pragma unroll
+  for (int q = 0; q < ITEMS; ++q) {
+    if (keep & (1u << q)) {
+      sh.key[li] = k[q] + lo;
+      sh.val[li] = sum[q];
+      ++li;
+    }
+  }
+  return total;
+}
+
 // O: what is written for a sum (zen_common.h).  DENSE: out_val is the dense tensor [0, dense_n); the workgroup
 // writes its bucket's range of it whole, zeros between the steps of the ranking loops, the sums behind them at the
 // end (62 M bf16 elements, 3.1 M entries: 55 us; nine more with the zeros in front of the records' loads, which then wait for
@@ -319,7 +382,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
   }
   sh.cnt.clear();
   __syncthreads();
-  const uint32_t b = (uint32_t)sh.tile;  // buckets are taken in order, so every earlier bucket already runs
+  const uint32_t b = (uint32_t)__builtin_amdgcn_readfirstlane(sh.tile);  // buckets are taken in order, so every earlier bucket already runs
   const uint32_t nb = geo.nbuckets;
   if (b >= nb) return;
   const uint32_t lo = geo.first_key(b);
@@ -367,68 +430,21 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
       longest <= (uint32_t)kWideBlock ? wide_merge_sort<S, 1>(sh, geo, in, b, pcount, longest, declined, tie_bits, status, zero_some)
       : longest <= 2u * kWideBlock ? wide_merge_sort<S, 2>(sh, geo, in, b, pcount, longest, declined, tie_bits, status, zero_some)
                                    : wide_merge_sort<S, kWmRounds>(sh, geo, in, b, pcount, longest, declined, tie_bits, status, zero_some);
-  // Thread t owns the sorted places [t * per, (t + 1) * per): as few per thread as cover the bucket (and an odd
-  // number, which keeps the lanes of a wave on different LDS banks).  It fetches them all at once and walks
-  // through them in registers.  A run of equal indices is summed in arrival order from +0 (like the dense
-  // tensor of comm.py:35) and belongs to the thread that holds its last record; where that run began before
-  // the thread's first place (rare: runs are short next to `per`, long ones come from payloads that overlap),
-  // the part in front is summed first, from the run's head on.
-  const uint32_t per = ((n + kWideBlock - 1) / kWideBlock) | 1u;  // <= kWmSumItems
-  const uint32_t first = tid * per;
-  uint32_t k[kWmSumItems];
-  float sum[kWmSumItems];
-  uint32_t keep = 0;
-  {
-    constexpr uint32_t kNoKey = 0xffffffffu;  // offsets are below the bucket width
-    float v[kWmSumItems];
-#pragma unroll
-    for (int q = 0; q < kWmSumItems; ++q) {
-      const uint32_t p = first + q;
-      const bool have = (uint32_t)q < per && p < n;
-      const uint32_t from = have ? p : 0u;
-      k[q] = sh.key[from];
-      v[q] = sh.val[from];
-      if (!have) k[q] = kNoKey;
-    }
-    const uint32_t before_k = first > 0 && first < n ? sh.key[first - 1] : kNoKey;
-    const uint32_t after_k = first + per < n ? sh.key[first + per] : kNoKey;
-    float acc = 0.0f;
-    if (first < n && before_k == k[0]) {
-      // the run began before this thread's places: find its head, sum up to the place in front of `first`
-      acc = sum_run_before(sh.key, sh.val, first, before_k);
-    }
-    uint32_t prev = before_k;
-#pragma unroll
-    for (int q = 0; q < kWmSumItems; ++q) {
-      const uint32_t next = q + 1 < kWmSumItems ? ((uint32_t)(q + 1) < per ? k[q + 1] : after_k) : after_k;
-      if (k[q] != kNoKey) {
-        if (k[q] != prev) acc = 0.0f;
-        acc += v[q];
-        prev = k[q];
-        sum[q] = acc;
-        if (k[q] != next && (DENSE ? acc != 0.0f : SumAs<O>::kept(acc))) keep |= 1u << q;
-      } else {
-        sum[q] = 0.0f;
-      }
-    }
-  }
-  if (DENSE) wait_global_acks();  // this wave's zeros are written (the scan's barrier: everybody's)
-  uint32_t total;
-  const uint32_t before = block_exclusive_scan<uint32_t, kWideBlock>((uint32_t)__popc(keep), sh.scan, &total);
   // where this bucket's output starts: the sum of what all earlier buckets keep.  Every thread asks for one of
   // them (bounded wait), nobody waits for a chain of prefixes; while the answers are on their way the kept
-  // entries are gathered in LDS (everybody is past reading the sorted bucket: the scan synchronised).
-  if (!DENSE && tid == 0) desc_store(&st.desc[b], kDescAggregate | total);
-  uint64_t d = !DENSE && tid < b ? desc_load(&st.desc[tid]) : kDescAggregate;
-  uint32_t li = before;
-#pragma unroll
-  for (int q = 0; q < kWmSumItems; ++q) {
-    if (keep & (1u << q)) {
-      sh.key[li] = k[q] + lo;
-      sh.val[li] = sum[q];
-      ++li;
-    }
-  }
+  // entries are gathered in LDS.
+  uint64_t d = kDescAggregate;
+  auto publish = [&](uint32_t kept) {
+    if (DENSE) return;
+    if (tid == 0) desc_store(&st.desc[b], kDescAggregate | kept);
+    if (tid < b) d = desc_load(&st.desc[tid]);
+  };
+  // written out for a few numbers of places a thread
+  static_assert(kWmSumItems == 17, "as many as a full bucket needs");
+  const uint32_t total = n <= 5u * kWideBlock    ? wide_merge_sums<O, DENSE, 5>(sh, n, lo, publish)
+                         : n <= 9u * kWideBlock  ? wide_merge_sums<O, DENSE, 9>(sh, n, lo, publish)
+                         : n <= 13u * kWideBlock ? wide_merge_sums<O, DENSE, 13>(sh, n, lo, publish)
+                                                 : wide_merge_sums<O, DENSE, kWmSumItems>(sh, n, lo, publish);
   {
     uint32_t spins = 0;
     while ((d >> 62) == 0) {
@@ -444,20 +460,21 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_merge(WideList list, I *__r
     __syncthreads();  // the gathered entries are there
     for (uint32_t i = tid; i < total; i += kWideBlock) out_val[sh.key[i]] = SumAs<O>::of(sh.val[i]);
   } else {
-    uint64_t all_before;
-    block_exclusive_scan<uint64_t, kWideBlock>(d & kDescValue, sh.scan64, &all_before);  // its barriers also publish the gathered entries
+    uint32_t all_before;  // (fewer than 2^31 entries in all)
+    block_exclusive_scan<uint32_t, kWideBlock>((uint32_t)d, sh.scan, &all_before);  // its barriers also publish the gathered entries
     if (b == nb - 1 && tid == 0) {
-      const uint64_t all = all_before + total;
+      const uint64_t all = (uint64_t)all_before + total;
       // (for the launch's last workgroup to read, on another die maybe)
       __hip_atomic_store(out_count, (int64_t)all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (all > (uint64_t)capacity) atomicOr(status, ZEN_STAT_CAPACITY);
     }
-    for (uint32_t i = tid; i < total; i += kWideBlock) {
-      const uint64_t pos = all_before + i;
-      if (pos < (uint64_t)capacity) {
-        out_idx[pos] = (I)sh.key[i];
-        out_val[pos] = SumAs<O>::of(sh.val[i]);
-      }
+    const uint64_t room = (uint64_t)capacity > all_before ? (uint64_t)capacity - all_before : 0;
+    const uint32_t fits = total < room ? total : (uint32_t)room;
+    I *const to_idx = out_idx + all_before;
+    O *const to_val = out_val + all_before;
+    for (uint32_t i = tid; i < fits; i += kWideBlock) {
+      to_idx[i] = (I)sh.key[i];
+      to_val[i] = SumAs<O>::of(sh.val[i]);
     }
   }
   if (answer.host) wait_global_acks();  // its share of the status word, and the count
