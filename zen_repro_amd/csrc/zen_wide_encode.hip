@@ -113,6 +113,7 @@ constexpr int kWideRemoved = 1024;                      // entries of a bucket t
 constexpr int kWideQueue = (2 * kWideMove + kWideMove + kWideRemoved) / 2;  // records set aside while ranking
 constexpr int kWideLanes = 4;                           // records a thread handles per step of the ranking loops
 constexpr int kWideGroupLimit = 512;                    // records in one narrow range: bounds the rank loop
+constexpr int kWidePast = 4;                            // words behind the records that may be read, not looked at
 constexpr int kWideIndexStep = 4;                       // every 4th narrow range has its first sorted place written down
 constexpr int kWideIndexLen = kWideSubs / kWideIndexStep;
 constexpr int kWidePad = 32;                            // words between two barrier counters
@@ -157,7 +158,7 @@ struct WideTables {
 template <typename S>
 struct WideShared {
   union {
-    uint32_t word[kWideCap];  // while ranking: (slot inside its narrow range) << 15 | raw place
+    uint32_t word[kWideCap + kWidePast];  // while ranking: (slot inside its narrow range) << 15 | raw place
     uint32_t idx[kWideCap];   // afterwards: the sorted indices (| kRemovedBit)
   };
   union {
@@ -284,7 +285,7 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
                                      const uint2 (&first_round)[kWideSplit], const uint32_t (&pcount)[kWideSplit],
                                      uint32_t longest, uint32_t thr_key, bool declined, uint32_t b, int32_t *status) {
   constexpr int kItems = kWideSplit * ROUNDS, kSteps = kItems / kWideLanes;
-  constexpr bool kHeld = ROUNDS == 1;
+  constexpr bool kHeld = ROUNDS <= 2;
   const uint32_t tid = threadIdx.x;
   const uint32_t lo = sh.lo;
   const int shift = geo.sub_shift;
@@ -292,16 +293,24 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
   // ---- slot offsets in registers; loads in no branch (places past a part's end are pulled back onto its
   // first record), so that all are in flight together
   uint32_t off[kItems];
+  uint2 second_round[ROUNDS == 2 ? kWideSplit : 1];
+  if (ROUNDS == 2) {
+#pragma unroll
+    for (int q = 0; q < kWideSplit; ++q) {
+      const uint32_t e = wide_place(q) + (uint32_t)kWideBlock;
+      second_round[ROUNDS == 2 ? q : 0] = records[(size_t)q * tb.part_cap + (e < pcount[q] ? e : 0u)];
+    }
+  }
 #pragma unroll
   for (int r = 0; r < ROUNDS; ++r) {
 #pragma unroll
     for (int q = 0; q < kWideSplit; ++q) off[r * kWideSplit + q] = kInvalid;
-    if ((uint32_t)r * kWideBlock < longest) {
+    if (kHeld || (uint32_t)r * kWideBlock < longest) {
 #pragma unroll
       for (int q = 0; q < kWideSplit; ++q) {
         const uint32_t e = wide_place(q) + (uint32_t)r * kWideBlock;
         const size_t at = (size_t)q * tb.part_cap + (e < pcount[q] ? e : 0u);
-        const uint2 rec = r == 0 ? first_round[q] : records[at];
+        const uint2 rec = r == 0 ? first_round[q] : ROUNDS == 2 ? second_round[ROUNDS == 2 ? q : 0] : records[at];
         const uint32_t slot = geo.mod_m(poly(rec.x) + kSeed1);  // the level-1 slot: a dozen instructions, not a plane of its own
         const bool keep = e < pcount[q] && (rec.y & KeyOf<S>::kMask) >= thr_key;
         off[r * kWideSplit + q] = keep ? slot - lo : kInvalid;
@@ -356,7 +365,8 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
   };
   if (kHeld) {
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) take_step(s, s * kWideLanes);
+    for (int s = 0; s < kSteps; ++s)
+      if (s < steps) take_step(s, s * kWideLanes);
   } else {
 #pragma unroll 1
     for (int s = 0; s < kSteps; ++s) {
@@ -391,25 +401,26 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
     }
 #pragma unroll
     for (int k = 0; k < kWideLanes; ++k) {
-      const uint32_t last = g1[k] > g0[k] ? g1[k] - 1u : g0[k];
 #pragma unroll
-      for (int e = 0; e < kAhead; ++e) a[k][e] = sh.word[g0[k] + e < last ? g0[k] + e : last];
+      for (int e = 0; e < kAhead; ++e) a[k][e] = sh.word[g0[k] + e];  // what lies behind the range is not looked at
     }
+    static_assert(kAhead <= kWidePast, "words behind the records");
 #pragma unroll
     for (int k = 0; k < kWideLanes; ++k) {
       if (off[from + k] != kInvalid) {
-        const uint32_t key = off[from + k] & low_mask;
-        const uint32_t my = (key << 15) | raw_place(s, k);
-        uint32_t less = 0, twins = 0;
+        const uint32_t key = (off[from + k] & low_mask) << 15;
+        const uint32_t my = key | raw_place(s, k);
+        const uint32_t size = g1[k] - g0[k];
+        uint32_t less = 0;
+        bool twins = false;
 #pragma unroll
         for (int e = 0; e < kAhead; ++e) {
-          if (g0[k] + e < g1[k]) {
-            less += (a[k][e] >> 15) < key;
-            twins += (a[k][e] >> 15) == key && a[k][e] != my;
-          }
+          const bool in = e == 0 || size > (uint32_t)e;
+          less += in & (a[k][e] < key) ? 1u : 0u;  // (a smaller slot: the raw place is below it)
+          twins |= in & ((a[k][e] ^ my) - 1u < 0x7fffu);  // the same slot, another record
         }
         uint32_t x = g0[k] + less;
-        if (twins || g1[k] - g0[k] > (uint32_t)kAhead) {
+        if (twins | (size > (uint32_t)kAhead)) {
           // A range of more than kAhead records, or another candidate with this very slot (the smaller
           // index then comes first, and comparing indices takes trips to memory): a wave would wait for
           // every lane that has one of these, at every record.  They are set aside and settled afterwards,
@@ -429,7 +440,9 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
       uint32_t out[kWideLanes];
-      rank_step(s, s * kWideLanes, out);
+#pragma unroll
+      for (int k = 0; k < kWideLanes; ++k) out[k] = kInvalid;
+      if (s < steps) rank_step(s, s * kWideLanes, out);
 #pragma unroll
       for (int k = 0; k < kWideLanes; ++k) rk[s * kWideLanes + k] = out[k];
     }
@@ -491,14 +504,14 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
   WIDE_MARK(3);
 #pragma unroll
   for (int r = 0; r < ROUNDS; ++r) {
-    if ((uint32_t)r * kWideBlock < longest) {
+    if (kHeld || (uint32_t)r * kWideBlock < longest) {
       uint32_t t[kWideSplit];
       S v[kWideSplit];
 #pragma unroll
       for (int q = 0; q < kWideSplit; ++q) {
         const uint32_t e = wide_place(q) + (uint32_t)r * kWideBlock;
         const size_t at = (size_t)q * tb.part_cap + (rk[r * kWideSplit + q] != kInvalid ? e : 0u);
-        const uint2 rec = kHeld ? first_round[q] : records[at];
+        const uint2 rec = !kHeld ? records[at] : r == 0 ? first_round[q] : second_round[ROUNDS == 2 ? q : 0];
         t[q] = rec.x;
         v[q] = (S)rec.y;
       }
@@ -573,6 +586,8 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   __syncthreads();
   const uint32_t n = longest <= (uint32_t)kWideBlock
                          ? wide_sort<S, 1>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, status)
+                     : longest <= 2u * kWideBlock
+                         ? wide_sort<S, 2>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, status)
                          : wide_sort<S, kWideRounds>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, status);
   uint32_t lost_n = sh.lost_n;
   if (lost_n > (uint32_t)kWideRemoved) {
