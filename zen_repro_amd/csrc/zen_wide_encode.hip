@@ -189,7 +189,7 @@ struct WideShared {
   };
   uint32_t scan[kWideBlock / 64 + 1];
   uint64_t scan64[kWideBlock / 64 + 1];
-  uint32_t lo, lost_n, nrm, mv_n, ser_n, pushed_n, base, flag, big;
+  uint32_t lo, queued, marked, lost_n, nrm, mv_n, ser_n, pushed_n, base, flag, big;
 };
 
 __device__ inline unsigned long long cell_fresh(const unsigned long long *p) {
@@ -283,9 +283,14 @@ __device__ unsigned long long g_wide_dbg[256 * 32];
 template <typename S, int ROUNDS>
 __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, const WideTables &tb, const uint2 *records,
                                      const uint2 (&first_round)[kWideSplit], const uint32_t (&pcount)[kWideSplit],
-                                     uint32_t longest, uint32_t thr_key, bool declined, uint32_t b, int32_t *status) {
+                                     uint32_t longest, uint32_t thr_key, bool declined, uint32_t b, uint32_t *log_n,
+                                     uint32_t &log_base, int32_t *status) {
   constexpr int kItems = kWideSplit * ROUNDS, kSteps = kItems / kWideLanes;
   constexpr bool kHeld = ROUNDS <= 2;
+  // of one round the words take half the room: the indices lie behind them, so that twins are settled without a trip to memory
+  constexpr bool kBeside = ROUNDS == 1;
+  constexpr uint32_t kRoom = kItems * kWideBlock;
+  static_assert(!kBeside || 2 * kRoom <= (uint32_t)kWideCap, "words and indices");
   const uint32_t tid = threadIdx.x;
   const uint32_t lo = sh.lo;
   const int shift = geo.sub_shift;
@@ -311,9 +316,9 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
         const uint32_t e = wide_place(q) + (uint32_t)r * kWideBlock;
         const size_t at = (size_t)q * tb.part_cap + (e < pcount[q] ? e : 0u);
         const uint2 rec = r == 0 ? first_round[q] : ROUNDS == 2 ? second_round[ROUNDS == 2 ? q : 0] : records[at];
-        const uint32_t slot = geo.mod_m(poly(rec.x) + kSeed1);  // the level-1 slot: a dozen instructions, not a plane of its own
-        const bool keep = e < pcount[q] && (rec.y & KeyOf<S>::kMask) >= thr_key;
-        off[r * kWideSplit + q] = keep ? slot - lo : kInvalid;
+        // the level-1 slot: a score of instructions, not a plane of its own; a wave without a record skips them
+        if (e < pcount[q] && (rec.y & KeyOf<S>::kMask) >= thr_key)
+          off[r * kWideSplit + q] = geo.mod_m(poly(rec.x) + kSeed1) - lo;
       }
     }
   }
@@ -360,6 +365,7 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
       if (off[from + k] != kInvalid) {
         const uint32_t p = sh.cnt.take(off[from + k] >> shift);
         sh.word[p] = ((off[from + k] & low_mask) << 15) | raw_place(s, k);
+        if (kBeside) sh.word[kRoom + p] = first_round[(s * kWideLanes + k) % kWideSplit].x;
       }
     }
   };
@@ -425,7 +431,7 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
           // index then comes first, and comparing indices takes trips to memory): a wave would wait for
           // every lane that has one of these, at every record.  They are set aside and settled afterwards,
           // one per thread.
-          const uint32_t at = atomicAdd(&sh.lost_n, 1u);
+          const uint32_t at = atomicAdd(&sh.queued, 1u);
           if (at < (uint32_t)kWideQueue) {
             sh.q_word[at] = my;
             sh.q_range[at] = g0[k] | (g1[k] << 16);
@@ -462,7 +468,7 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
   WIDE_MARK(22);
   __syncthreads();
   {
-    uint32_t pending = sh.lost_n;
+    uint32_t pending = sh.queued;
     if (pending > (uint32_t)kWideQueue) {
       if (tid == 0) atomicOr(status, ZEN_STAT_RETRY);
       pending = kWideQueue;
@@ -478,11 +484,18 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
       }
       uint32_t lost = 0;
       if (twins) {
-        const uint32_t mine = records[raw_at(my & 0x7fffu)].x;
+        uint32_t mine = 0;
+        if (kBeside) {
+          for (uint32_t u = g0; u < g1; ++u) mine = sh.word[u] == my ? sh.word[kRoom + u] : mine;
+        } else {
+          mine = records[raw_at(my & 0x7fffu)].x;
+        }
         for (uint32_t u = g0; u < g1; ++u) {
           const uint32_t w = sh.word[u];
-          if ((w >> 15) == key && w != my) lost += records[raw_at(w & 0x7fffu)].x < mine;
+          if ((w >> 15) == key && w != my)
+            lost += (kBeside ? sh.word[kRoom + u] : records[raw_at(w & 0x7fffu)].x) < mine;
         }
+        if (lost) atomicAdd(&sh.marked, 1u);
       }
       sh.q_word[e] = (g0 + less + lost) | (lost ? kRemovedBit : 0u);  // the entry's thread is its only reader
     }
@@ -494,13 +507,13 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
                   sh.cnt.start_of(s0) | (sh.cnt.end_of(s0 + kWideIndexStep - 1) << 16));
     }
     __syncthreads();
+    // room in the partition's log, on its way while the records are put in order
+    if (tid == 0 && sh.marked) log_base = atomicAdd(log_n, sh.marked < (uint32_t)kWideRemoved ? sh.marked : (uint32_t)kWideRemoved);
 #pragma unroll
     for (int i = 0; i < kItems; ++i)
       if (rk[i] != kInvalid && (rk[i] & kRemovedBit)) rk[i] = sh.q_word[rk[i] & kIndexMask];
-    __syncthreads();  // the queue's memory serves other lists from here on
-    if (tid == 0) sh.lost_n = 0;
   }
-  __syncthreads();
+  __syncthreads();  // the queue's memory serves other lists from here on
   WIDE_MARK(3);
 #pragma unroll
   for (int r = 0; r < ROUNDS; ++r) {
@@ -564,7 +577,7 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   for (uint32_t i = b * kWideBlock + tid; i < clear_too_words; i += B * kWideBlock) clear_too[i] = 0;  // fp32: the refinement's histogram
   if (tid == 0) {
     sh.lo = geo.first_key(b);
-    sh.lost_n = sh.nrm = sh.mv_n = sh.ser_n = sh.pushed_n = sh.big = 0;
+    sh.queued = sh.marked = sh.lost_n = sh.nrm = sh.mv_n = sh.ser_n = sh.pushed_n = sh.big = 0;
   }
   sh.cnt.clear();
   uint32_t pcount[kWideSplit];
@@ -584,18 +597,20 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   }
   const uint32_t thr_key = filter ? filter[0] : 0u;
   __syncthreads();
+  uint32_t *const log_n = &tb.log_n[part * kWideCtrPad];
+  uint32_t log_base = 0;  // thread 0: where the bucket's losers go in the partition's log
   const uint32_t n = longest <= (uint32_t)kWideBlock
-                         ? wide_sort<S, 1>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, status)
+                         ? wide_sort<S, 1>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, log_n, log_base, status)
                      : longest <= 2u * kWideBlock
-                         ? wide_sort<S, 2>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, status)
-                         : wide_sort<S, kWideRounds>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, status);
+                         ? wide_sort<S, 2>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, log_n, log_base, status)
+                         : wide_sort<S, kWideRounds>(sh, geo, tb, records, first_round, pcount, longest, thr_key, declined, b, log_n, log_base, status);
   uint32_t lost_n = sh.lost_n;
   if (lost_n > (uint32_t)kWideRemoved) {
     if (tid == 0) atomicOr(status, ZEN_STAT_RETRY);
     lost_n = kWideRemoved;
   }
   if (tid == 0) {
-    sh.base = lost_n ? atomicAdd(&tb.log_n[part * kWideCtrPad], lost_n) : 0u;
+    sh.base = log_base;
     sh.nrm = lost_n;  // (their places are the first of sh.gone)
   }
   for (uint32_t p = tid; p < n; p += kWideBlock) store_agent(&tb.slab_idx[(size_t)b * kWideCap + p], sh.idx[p]);
@@ -617,7 +632,9 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   Counters *pctr = &tb.ctr[part];
   const uint32_t local = b - part * bpp;
   const bool last_of_part = local == bpp - 1;
-  uint32_t losers = load_agent(&tb.log_n[part * kWideCtrPad]);
+  // the first losers beside their number: a trip to memory less (the log has room for more)
+  const uint32_t loser = tid < (uint32_t)kWideOwnChains ? load_agent(&tb.log_t[(size_t)part * tb.log_cap + tid]) : 0u;
+  uint32_t losers = load_agent(log_n);
   if (losers > tb.log_cap) losers = tb.log_cap;
   const bool own = losers <= (uint32_t)kWideOwnChains;
   uint32_t pushed = 0;
@@ -689,7 +706,6 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
   };
   if (own) {
     for (uint32_t i = tid; i < (1u << kWideOwnLog2); i += kWideBlock) sh.own[i] = 0ull;
-    const uint32_t loser = tid < losers ? load_agent(&tb.log_t[(size_t)part * tb.log_cap + tid]) : 0u;
     __syncthreads();
     if (tid < losers)
       chain(
@@ -789,8 +805,11 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
       x = sh.gone[tid];
       for (uint32_t u = 0; u < rm_n; ++u) xr += sh.gone[u] < x;
     }
-    uint32_t mj = 0, mplace = 0;
+    uint32_t mj = 0, mplace = 0, moved = 0;
+    S moved_val = 0;  // (on its way until the end)
     if (tid < mv_n) {
+      moved = sh.mi[tid];
+      moved_val = dense[moved];  // an entry is a copy of the element it stands for
       const uint32_t k = sh.mk[tid];
       for (uint32_t u = 0; u < mv_n; ++u) mj += sh.mk[u] < k;
       uint32_t p0 = 0, p1 = n;
@@ -867,9 +886,8 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
     if (tid < mv_n) {
       const uint32_t pos = out_base + mplace + mj - (rm_n ? lower_bound_u32(sh.rm, rm_n, mplace) : 0u);
       if (pos < capacity) {
-        const uint32_t t = sh.mi[tid];
-        out_idx[pos] = (int32_t)t;
-        out_val[pos] = dense[t];  // an entry is a copy of the element it stands for
+        out_idx[pos] = (int32_t)moved;
+        out_val[pos] = moved_val;
       }
     }
     if (serial) {
