@@ -812,22 +812,79 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
       moved_val = dense[moved];  // an entry is a copy of the element it stands for
       const uint32_t k = sh.mk[tid];
       for (uint32_t u = 0; u < mv_n; ++u) mj += sh.mk[u] < k;
+    }
+    auto slot_at = [&](uint32_t p) { return geo.mod_m(poly(sh.idx[p] & kIndexMask) + kSeed1); };
+    constexpr uint32_t kWaves = kWideBlock / 64, kMoveFew = 2 * kWaves;
+    if (mv_n <= kMoveFew) {  // a wave to an entry, which looks at 64 places at once (a thread's bisection: 12 trips to LDS and hashes)
+      for (uint32_t j = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)); j < mv_n; j += kWaves) {
+        const uint32_t k = sh.mk[j];
+        uint32_t p0 = 0, p1 = n;
+        while (p0 < p1) {
+          const uint32_t step = (p1 - p0 + 63u) / 64u, p = p0 + (uint32_t)lane_id() * step;
+          bool below = false;
+          if (p < p1) below = slot_at(p) < k;
+          const uint32_t c = (uint32_t)__popcll(__ballot(below));  // slots ascend: the first c of them
+          const uint32_t end = p0 + c * step;
+          if (end < p1) p1 = end;
+          if (c) p0 = end - step + 1u;
+        }
+        if (lane_id() == 0) sh.delta[j] = (int32_t)p0;
+      }
+    } else if (tid < mv_n) {
+      const uint32_t k = sh.mk[tid];
       uint32_t p0 = 0, p1 = n;
       while (p0 < p1) {
         const uint32_t mid = p0 + ((p1 - p0) >> 1);
-        if (geo.mod_m(poly(sh.idx[mid] & kIndexMask) + kSeed1) < k) p0 = mid + 1; else p1 = mid;
+        if (slot_at(mid) < k) p0 = mid + 1; else p1 = mid;
       }
       mplace = p0;
     }
     __syncthreads();
     if (tid < rm_n) sh.rm[xr] = x;
-    if (tid < mv_n) sh.mp[mj] = mplace;
+    if (tid < mv_n) {
+      if (mv_n <= kMoveFew) mplace = (uint32_t)sh.delta[tid];
+      sh.mp[mj] = mplace;
+    }
     __syncthreads();
     // where the bucket starts: the sum of what the earlier buckets publish (every workgroup of the launch is
-    // resident; the wait is bounded all the same)
+    // resident; the wait is bounded all the same), asked for now and waited for below
+    uint64_t d = tid < b ? desc_load(&tb.desc[tid]) : kDescAggregate;
+    // Most stretches of 64 consecutive sorted places contain neither a removed entry nor the place where a
+    // moved-in entry slips in: all their entries move by the same amount, found once per stretch.
+    // Per stretch of 64 consecutive sorted places: how many moved-in entries slip in at or before its first
+    // place and how many removed entries lie before it (12 bits each), and whether that holds for the whole
+    // stretch (most contain neither a removed entry nor a place where an entry slips in).
+    constexpr uint32_t kSame = 1u << 31;
+    for (uint32_t c = tid; c * 64u < n; c += kWideBlock) {
+      const uint32_t p0 = c * 64u, p1 = p0 + 63u < n ? p0 + 63u : n - 1u;
+      uint32_t mv0 = 0, mv1 = 0, r0 = 0, r1 = 0;
+      if (mv_n <= kMoveFew && rm_n <= kMoveFew) {  // counted, with no look waiting for the one before
+#pragma unroll 4
+        for (uint32_t u = 0; u < mv_n; ++u) {
+          const uint32_t at = sh.mp[u];
+          mv0 += at <= p0 ? 1u : 0u;
+          mv1 += at <= p1 ? 1u : 0u;
+        }
+#pragma unroll 4
+        for (uint32_t u = 0; u < rm_n; ++u) {
+          const uint32_t at = sh.rm[u];
+          r0 += at < p0 ? 1u : 0u;
+          r1 += at < p1 ? 1u : 0u;
+        }
+      } else {
+        if (mv_n) {
+          mv0 = upper_bound_u32(sh.mp, mv_n, p0);
+          mv1 = upper_bound_u32(sh.mp, mv_n, p1);
+        }
+        if (rm_n) {
+          r0 = lower_bound_u32(sh.rm, rm_n, p0);
+          r1 = lower_bound_u32(sh.rm, rm_n, p1);
+        }
+      }
+      sh.delta[c] = (int32_t)(mv0 | (r0 << 12) | ((mv0 == mv1 && r0 == r1) ? kSame : 0u));
+    }
     uint64_t before = 0;  // low half: entries of all earlier buckets; high half: of the partition's earlier buckets
     if (tid < b) {
-      uint64_t d = desc_load(&tb.desc[tid]);
       uint32_t spins = 0;
       while ((d >> 62) == 0) {
         if (++spins > kSpinLimit) {
@@ -842,28 +899,8 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_tail(SlabGeom geo, Probe g,
     }
     WIDE_MARK(10);
     uint64_t sums;
-    block_exclusive_scan<uint64_t, kWideBlock>(before, sh.scan64, &sums);
+    block_exclusive_scan<uint64_t, kWideBlock>(before, sh.scan64, &sums);  // its barriers also publish the stretches
     const uint32_t out_base = (uint32_t)sums, in_part = (uint32_t)(sums >> 32);
-    // Most stretches of 64 consecutive sorted places contain neither a removed entry nor the place where a
-    // moved-in entry slips in: all their entries move by the same amount, found once per stretch.
-    // Per stretch of 64 consecutive sorted places: how many moved-in entries slip in at or before its first
-    // place and how many removed entries lie before it (12 bits each), and whether that holds for the whole
-    // stretch (most contain neither a removed entry nor a place where an entry slips in).
-    constexpr uint32_t kSame = 1u << 31;
-    for (uint32_t c = tid; c * 64u < n; c += kWideBlock) {
-      const uint32_t p0 = c * 64u, p1 = p0 + 63u < n ? p0 + 63u : n - 1u;
-      uint32_t mv0 = 0, mv1 = 0, r0 = 0, r1 = 0;
-      if (mv_n) {
-        mv0 = upper_bound_u32(sh.mp, mv_n, p0);
-        mv1 = upper_bound_u32(sh.mp, mv_n, p1);
-      }
-      if (rm_n) {
-        r0 = lower_bound_u32(sh.rm, rm_n, p0);
-        r1 = lower_bound_u32(sh.rm, rm_n, p1);
-      }
-      sh.delta[c] = (int32_t)(mv0 | (r0 << 12) | ((mv0 == mv1 && r0 == r1) ? kSame : 0u));
-    }
-    __syncthreads();
     WIDE_MARK(11);
 #pragma unroll 4
     for (uint32_t p = tid; p < n; p += kWideBlock) {
