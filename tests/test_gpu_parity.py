@@ -1349,6 +1349,35 @@ def test_sample_threshold_of_every_size(zen, s, dtype):
             assert status.item() == 0
 
 
+@pytest.mark.parametrize("s", [128 * 1024, 128 * 1024 + 1, 255 * 1024 + 5, 256 * 4096 * 2, 256 * 4096 * 2 + 1, 256 * 4096 * 3 - 5,
+                               256 * 4096 * 5 + 9, 256 * 65535 + 1])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sample_threshold_in_rounds(zen, s, dtype):
+    """As many workgroups as the search sums up in one batch and one more; one to sixteen rounds of 4096 places a workgroup, whole
+    and cut off; more workgroups than compute units.  Places outside the tensor count as zero, in every round.  Exact."""
+    import importlib
+
+    from zen_repro_amd import _lib
+
+    C = importlib.import_module("zen_repro_amd.compress")
+    gen = torch.Generator(device="cuda").manual_seed(s)
+    n = 300007
+    t = torch.randn(n, generator=gen, device="cuda").to(dtype)
+    at = torch.randint(0, n, (s,), generator=gen, device="cuda")
+    for outside in (False, True):
+        if outside:
+            at[torch.randint(0, s, (1000,), generator=gen, device="cuda")] = n
+            at[s - 1] = -1
+        keys = torch.where((at >= 0) & (at < n), t[at.clamp(0, n - 1)], torch.zeros((), dtype=dtype, device="cuda"))
+        keys = keys.float().abs().view(torch.int32)
+        ordered = torch.sort(keys, descending=True)[0]
+        for k in (1, s // 20, s):
+            thr, status = C.sample_threshold(t, at, k)
+            want = ordered[k - 1].item()
+            assert thr.tolist() == [want >> 16 if dtype == torch.bfloat16 else want, (keys >= want).sum().item()]
+            assert int(status) == (_lib.STAT_BAD_INDEX if outside else 0)
+
+
 @pytest.mark.parametrize("shift", [0, 1])
 @pytest.mark.parametrize("n", [65537, 65536 + 2048, 65536 + 2049, 200001, 20000000])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

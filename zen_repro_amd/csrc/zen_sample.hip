@@ -187,31 +187,68 @@ struct SampleTables {
   uint32_t *state;   // fp32: [0] bin, [1] rank inside it, [2] elements above it, [3] members listed, [4] workgroups done
 };
 
-// Bound by the sample's lines: 2.7 M elements of a 537 MB tensor at random places are 344 MB of them, 62 us at the
-// rate of a copy.  The gather's loads are streamed (nontemporal): of a line one element is wanted, and a tensor of
-// gigabytes would only push others out.  The kernel alone 70 us with plain loads, 63.5 so; with the tensor cold in
-// every cache 120 and 72 a call.
+// Bound by the sample's lines: 2.7 M elements of a 537 MB tensor at random places are 344 MB of them, which come at 51 a
+// nanosecond at most, 53 us.  The gather's loads are streamed (nontemporal): of a line one element is wanted, and a tensor of
+// gigabytes would only push others out (with the tensor cold in every cache a call 72 us, 120 with plain loads).  Trips to
+// memory overlap: the first places are asked for in front of the clearing of the counters, a round's elements in front of the
+// counting of the round before, their places a round earlier still; and of the counters only groups that hold something are
+// written out, 64 KB a workgroup else.  One after the other and all written: 2.7 M bf16 elements 62.5 us, so 57.3; 620 000
+// 21.8 and 17.2; 129 000 fp32 11.9 and 7.4; 10 486 8.2 and 4.9.
 template <typename S>
 __global__ __launch_bounds__(kBlock) void k_sample_count(const S *__restrict__ in, int64_t n,
                                                          const int64_t *__restrict__ at, int64_t s, int64_t share,
                                                          SampleTables tb, int32_t *status) {
   __shared__ uint32_t hist[kHistWords];
   constexpr int kShift = KeyOf<S>::kBits - 15;
-  clear_hist(hist);
-  __syncthreads();
+  constexpr int64_t kStep = (int64_t)kRound * kBlock;
   const int64_t begin = (int64_t)blockIdx.x * share;
   const int64_t end = begin + share < s ? begin + share : s;
-  for (int64_t j0 = begin; j0 < end; j0 += (int64_t)kRound * kBlock) {
-    S v[kRound];
-    gather<S, kRound>(in, n, at, j0 + threadIdx.x, end, v, status);
+  int64_t pos[2][kRound];
+  S v[2][kRound];
+  uint32_t wrong[2], any = 0;  // bit i: element i's place is outside the tensor (element 0 is read, as zero)
+  auto ask_places = [&](int64_t j0, int64_t (&p)[kRound]) {
 #pragma unroll
     for (int i = 0; i < kRound; ++i) {
       const int64_t j = j0 + threadIdx.x + (int64_t)i * kBlock;
-      const uint32_t key = v[i] & KeyOf<S>::kMask;
+      p[i] = at ? __builtin_nontemporal_load(at + (j < end ? j : end - 1)) : (j < end ? j : end - 1);
+    }
+  };
+  auto ask_elements = [&](const int64_t (&p)[kRound], S (&e)[kRound], uint32_t &out) {
+    out = 0;
+#pragma unroll
+    for (int i = 0; i < kRound; ++i) {
+      const bool in_range = (uint64_t)p[i] < (uint64_t)n;
+      out |= in_range ? 0u : 1u << i;
+      e[i] = __builtin_nontemporal_load(in + (in_range ? p[i] : 0));
+    }
+    any |= out;
+  };
+  auto count = [&](int64_t j0, const S (&e)[kRound], uint32_t out) {
+#pragma unroll
+    for (int i = 0; i < kRound; ++i) {
+      const int64_t j = j0 + threadIdx.x + (int64_t)i * kBlock;
+      const uint32_t key = out & (1u << i) ? 0u : e[i] & KeyOf<S>::kMask;
       count_bin(hist, key >> kShift, j < end);
       if (sizeof(S) == 4 && j < end) tb.sample[j] = key;
     }
+  };
+  ask_places(begin, pos[0]);
+  if (begin + kStep < end) ask_places(begin + kStep, pos[1]);
+  clear_hist(hist);
+  ask_elements(pos[0], v[0], wrong[0]);
+  __syncthreads();
+  int64_t j0 = begin;
+  // a round's elements are asked for in front of the counting of the one before, its places a round earlier still
+  for (; j0 + kStep < end; j0 += 2 * kStep) {
+    ask_places(j0 + 2 * kStep, pos[0]);  // (past the end: the last place once more)
+    ask_elements(pos[1], v[1], wrong[1]);
+    count(j0, v[0], wrong[0]);
+    ask_places(j0 + 3 * kStep, pos[1]);
+    ask_elements(pos[0], v[0], wrong[0]);
+    count(j0 + kStep, v[1], wrong[1]);
   }
+  if (j0 < end) count(j0, v[0], wrong[0]);
+  if (any) atomicOr(status, ZEN_STAT_BAD_INDEX);
   __syncthreads();
   // thread t: 16 words = 32 bins, half a group
   uint32_t w[16];
@@ -221,32 +258,51 @@ __global__ __launch_bounds__(kBlock) void k_sample_count(const S *__restrict__ i
     w[j] = hist[hist_word((int)threadIdx.x * 16 + j)];
     sum += (w[j] & 0xffffu) + (w[j] >> 16);
   }
-  uint4 *bins = reinterpret_cast<uint4 *>(tb.bins + (size_t)blockIdx.x * kBins);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) bins[threadIdx.x * 4 + j] = make_uint4(w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]);
   sum += __shfl_xor(sum, 1, 64);
+  if (sum) {  // (nobody looks at the bins of a group without elements)
+    uint4 *bins = reinterpret_cast<uint4 *>(tb.bins + (size_t)blockIdx.x * kBins);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bins[threadIdx.x * 4 + j] = make_uint4(w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]);
+  }
   if ((threadIdx.x & 1u) == 0) tb.sums[(size_t)blockIdx.x * kGroups + threadIdx.x / 2] = (uint16_t)sum;
 }
 
-// Sums of 16-bit counters over the workgroups of the counting kernel: `words` columns of four counters, read by
-// kBlock / COLUMNS rows of threads side by side.  acc: [4 * COLUMNS] words of LDS, zeroed here.
-template <int COLUMNS>
-__device__ inline void sum_columns(const uint16_t *from, size_t stride, uint32_t rows, uint32_t *acc) {
-  if (threadIdx.x < 4 * COLUMNS) acc[threadIdx.x] = 0;
+// Sums of 16-bit counters over the workgroups of the counting kernel: COUNTERS of them, WORDS * 2 to a thread's load, by
+// rows of threads side by side, BATCH rows of a thread in flight together.  acc: [COUNTERS] words of LDS, zeroed here.  A row
+// counts where counted(row) says so.  (The rows that were left over from batches of eight were read one trip to memory after
+// the other: k_sample_pick with 152 rows 6.5 us, 256 rows 8.7.)
+template <int COUNTERS, int WORDS, int BATCH, typename Counted>
+__device__ inline void sum_columns(const uint16_t *from, size_t stride, uint32_t rows, uint32_t *acc, Counted counted) {
+  using Words = uint32_t __attribute__((ext_vector_type(WORDS)));
+  constexpr uint32_t kColumns = COUNTERS / (2 * WORDS), kRows = kBlock / kColumns;
+  for (int i = threadIdx.x; i < COUNTERS; i += kBlock) acc[i] = 0;
   __syncthreads();
-  const uint32_t col = threadIdx.x % COLUMNS, row = threadIdx.x / COLUMNS;
-  constexpr uint32_t kRows = kBlock / COLUMNS;
-  uint32_t c[4] = {0, 0, 0, 0};
-#pragma unroll 8
-  for (uint32_t r = row; r < rows; r += kRows) {
-    const uint2 q = *reinterpret_cast<const uint2 *>(from + (size_t)r * stride + col * 4);
-    c[0] += q.x & 0xffffu;
-    c[1] += q.x >> 16;
-    c[2] += q.y & 0xffffu;
-    c[3] += q.y >> 16;
+  const uint32_t col = threadIdx.x % kColumns, row = threadIdx.x / kColumns;
+  uint32_t c[2 * WORDS];
+#pragma unroll
+  for (int e = 0; e < 2 * WORDS; ++e) c[e] = 0;
+#pragma unroll 1
+  for (uint32_t r0 = row; r0 < rows; r0 += BATCH * kRows) {
+    Words q[BATCH];
+    bool in[BATCH];
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      const uint32_t r = r0 + i * kRows < rows ? r0 + i * kRows : row;
+      q[i] = *reinterpret_cast<const Words *>(from + (size_t)r * stride + col * 2 * WORDS);
+      in[i] = counted(r) && r0 + i * kRows < rows;
+    }
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i)
+#pragma unroll
+      for (int e = 0; e < WORDS; ++e) {
+        const uint32_t x = in[i] ? q[i][e] : 0u;
+        c[2 * e] += x & 0xffffu;
+        c[2 * e + 1] += x >> 16;
+      }
   }
 #pragma unroll
-  for (int e = 0; e < 4; ++e) atomicAdd(&acc[col * 4 + e], c[e]);
+  for (int e = 0; e < 2 * WORDS; ++e)
+    if (c[e]) atomicAdd(&acc[col * 2 * WORDS + e], c[e]);  // (most of a sample's bins are empty)
   __syncthreads();
 }
 
@@ -315,7 +371,7 @@ __global__ __launch_bounds__(kBlock) void k_sample_pick(SampleTables tb, uint32_
   __shared__ uint32_t acc[kGroups];
   __shared__ uint32_t smem[kBlock / 64 + 1];
   __shared__ uint32_t found[3];
-  sum_columns<kGroups / 4>(tb.sums, kGroups, rows, acc);
+  sum_columns<kGroups, 4, FEW ? 1 : 8>(tb.sums, kGroups, rows, acc, [](uint32_t) { return true; });
   {
     const uint32_t c = threadIdx.x < kGroups ? acc[kGroups - 1 - threadIdx.x] : 0u;
     uint32_t total;
@@ -327,7 +383,8 @@ __global__ __launch_bounds__(kBlock) void k_sample_pick(SampleTables tb, uint32_
   }
   __syncthreads();
   const uint32_t group = found[0], over = found[1];
-  sum_columns<kGroup / 4>(tb.bins + (size_t)group * kGroup, kBins, rows, acc);
+  sum_columns<kGroup, 2, FEW ? 1 : 4>(tb.bins + (size_t)group * kGroup, kBins, rows, acc,
+                          [&](uint32_t r) { return tb.sums[(size_t)r * kGroups + group] != 0; });
   {
     const uint32_t c = threadIdx.x < kGroup ? acc[kGroup - 1 - threadIdx.x] : 0u;
     uint32_t total;
@@ -402,16 +459,13 @@ __global__ __launch_bounds__(kBlock) void k_sample_members(SampleTables tb, int6
   });
 }
 
-// Workgroups of the counting kernel for a sample of s elements: up to 64, an element per thread (a call for 10 486
-// bf16 elements 14.0 us, with four per thread 18.8; 128 660 on 64 workgroups 19.6, on 32 22.1); beyond that a round
-// of four each, so that the picking kernel, which reads a row per workgroup, has fewer (619 534 elements: 151 rows
-// 29.5, 256 rows 31.4); one per compute unit at most, unless a share outgrew the counters.
-constexpr int64_t kSpread = 64;
+// Workgroups of the counting kernel for a sample of s elements: one per compute unit, an element per thread at least
+// (10 486 elements with four per thread 4.8 us more), more of them if a share outgrew the counters.  The picking kernel
+// reads a row per workgroup, which costs less than what the counting kernel gains: counting and picking with a workgroup to
+// each 4096 elements, 64 at least, and so, us: 128 660 fp32 elements on 64 and 126 workgroups 8.7 + 4.4 and 7.4 + 4.6,
+// 619 534 bf16 on 152 and 256 17.8 + 6.2 and 17.2 + 6.4.
 inline int64_t sample_groups(int64_t s) {
   int64_t g = ceil_div(s, (int64_t)kBlock);
-  if (g > kSpread) g = kSpread;
-  const int64_t full = ceil_div(s, (int64_t)kRound * kBlock);
-  if (g < full) g = full;
   if (g > 256) g = 256;
   const int64_t least = ceil_div(s, kShare);
   return g < least ? least : g;
