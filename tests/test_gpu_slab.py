@@ -1278,3 +1278,24 @@ def test_every_element_is_looked_at_once(zen, dtype, sub, more):
         want, total = torch.nonzero(passed).view(-1), int(splits.sum())
         order = torch.sort(idx[:total])
         assert torch.equal(order[0].long(), want) and torch.equal(val[:total][order[1]], grad[want])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("r", [8 * 4096, 8 * 4096 + 1, 8 * 4096 + 511, 8 * 4096 + 512, 8 * 4096 + 513, 9 * 4096 - 1])
+def test_slab_merge_of_cut_off_batches(zen, r, dtype):
+    """The last batch of a list has one entry, a little less than a row of a workgroup's threads, a row, a little more, all of
+    its entries but one; the coarse slabs' parts have a few.  Whole numbers: exact."""
+    from zen_repro_amd import _lib
+
+    n = 1 << 23
+    assert _lib.lib().zen_merge_path(r, n, _lib.MODE_FAST | _lib.MODE_SLABS) == SLAB
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(4), None, None)
+    lba.fast_flags = _lib.MODE_SLABS
+    gen = torch.Generator(device="cuda").manual_seed(r)
+    idx = torch.randint(0, n, (r,), generator=gen, device="cuda", dtype=torch.int32)
+    idx[-1], idx[-2] = 0, n - 1
+    val = torch.randint(1, 4, (r,), generator=gen, device="cuda").to(dtype)
+    want = torch.zeros(n, device="cuda").scatter_add_(0, idx.long(), val.float())
+    at = torch.nonzero(want).view(-1)
+    got_idx, got_val = lba.merge_rounded(idx, val, n, dtype)
+    assert torch.equal(got_idx, at) and torch.equal(got_val, want[at].to(dtype))

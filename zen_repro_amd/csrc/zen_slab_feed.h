@@ -161,20 +161,32 @@ __global__ __launch_bounds__(kSlabBlock) void k_coarse_scatter(SlabGeom geo, Coa
   }
   __syncthreads();
   const uint32_t total = s_pref[kCoarseMax];
+  if (total == 0) return;
   const size_t plane = (size_t)cg.groups * kCoarseSplit * cg.cap;  // words of one word plane
-  for (uint32_t p = threadIdx.x; p < total; p += kSlabBlock) {
+  // All of a thread's entries on their way together: with one look-up and fetch after the other a workgroup's last step was
+  // eight trips long (6.2 M bf16 entries k_coarse_scatter 34.6 us, so 32.6, k_fine_scatter 28.5 and 27.1; in the encode of
+  // 10.7 M fp32 entries, beside the merge, 115 and 97).
+  uint32_t rec[kFeedItems][W], at[kFeedItems], o[kFeedItems];
+#pragma unroll
+  for (int i = 0; i < kFeedItems; ++i) {
+    const uint32_t p = threadIdx.x + i * kSlabBlock < total ? threadIdx.x + i * kSlabBlock : total - 1u;
     const uint32_t d = s_dst[p];
-    const uint32_t at = s_gbase[d] + (p - s_pref[d]);
-    if (at < cg.cap) {
-      const size_t o = (size_t)(d * kCoarseSplit + part) * cg.cap + at;
-      uint32_t rec[W];
+    at[i] = s_gbase[d] + (p - s_pref[d]);
+    o[i] = (d * kCoarseSplit + part) * cg.cap + at[i];
 #pragma unroll
-      for (int q = 0; q < WS; ++q) rec[q] = s_word[q][p];
+    for (int q = 0; q < WS; ++q) rec[i][q] = s_word[q][p];
+  }
 #pragma unroll
-      for (int q = WS; q < W; ++q) rec[q] = src.late(rec, q);
+  for (int i = 0; i < kFeedItems; ++i)
 #pragma unroll
-      for (int q = 0; q < W - 1; ++q) coarse_words[q * plane + o] = rec[q];
-      reinterpret_cast<typename Src::Last *>(coarse_words + (size_t)(W - 1) * plane)[o] = (typename Src::Last)rec[W - 1];
+    for (int q = WS; q < W; ++q) rec[i][q] = src.late(rec[i], q);
+#pragma unroll
+  for (int i = 0; i < kFeedItems; ++i) {
+    if (threadIdx.x + i * kSlabBlock >= total) continue;
+    if (at[i] < cg.cap) {
+#pragma unroll
+      for (int q = 0; q < W - 1; ++q) coarse_words[q * plane + o[i]] = rec[i][q];
+      reinterpret_cast<typename Src::Last *>(coarse_words + (size_t)(W - 1) * plane)[o[i]] = (typename Src::Last)rec[i][W - 1];
     } else {
       atomicOr(status, ZEN_STAT_RETRY);  // a coarse slab is full: the general path answers
     }
@@ -236,18 +248,25 @@ __global__ __launch_bounds__(kSlabBlock) void k_fine_scatter(SlabGeom geo, Coars
   }
   __syncthreads();
   const uint32_t total = s_pref[kCoarsePer];
-  for (uint32_t p = threadIdx.x; p < total; p += kSlabBlock) {
-    const uint32_t d = s_dst[p];
-    const uint32_t at = s_gbase[d] + (p - s_pref[d]);
-    if (at < (uint32_t)kSlabCap) {
-      uint32_t rec[W];
+  if (total == 0) return;
+  uint32_t rec[kFeedItems][W], at[kFeedItems], o[kFeedItems];  // all on their way together, as above
 #pragma unroll
-      for (int q = 0; q < W - 1; ++q) rec[q] = s_word[q][p];
-      rec[W - 1] = (uint32_t)s_last[p];
-      sink.store((size_t)(first_bucket + d) * kSlabCap + at, rec);
-    } else {
+  for (int i = 0; i < kFeedItems; ++i) {
+    const uint32_t p = threadIdx.x + i * kSlabBlock < total ? threadIdx.x + i * kSlabBlock : total - 1u;
+    const uint32_t d = s_dst[p];
+    at[i] = s_gbase[d] + (p - s_pref[d]);
+    o[i] = (first_bucket + d) * (uint32_t)kSlabCap + at[i];
+#pragma unroll
+    for (int q = 0; q < W - 1; ++q) rec[i][q] = s_word[q][p];
+    rec[i][W - 1] = (uint32_t)s_last[p];
+  }
+#pragma unroll
+  for (int i = 0; i < kFeedItems; ++i) {
+    if (threadIdx.x + i * kSlabBlock >= total) continue;
+    if (at[i] < (uint32_t)kSlabCap)
+      sink.store(o[i], rec[i]);
+    else
       atomicOr(status, ZEN_STAT_RETRY);  // a slab is full: the general path answers
-    }
   }
 }
 
