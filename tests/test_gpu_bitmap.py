@@ -688,3 +688,50 @@ def test_comm_hook_needs_a_backend_for_more_than_one_rank(zen):
     hook(None, _StubBucket(grad))
     with pytest.raises(RuntimeError):
         hook(None, _StubBucket(grad))
+
+
+class _OneRank:
+    """The exchange of a rank that receives `idx` and whose peers send nothing else; `cut` values of the second exchange
+    are lost."""
+
+    def __init__(self, parts, idx, val, cut):
+        self.parts, self.idx, self.val, self.cut = parts, idx, val, cut
+
+    def allgather(self, tensor):
+        return [tensor]
+
+    def alltoallv(self, tensors, gather_splits):
+        return [self.idx if tensors[0].dtype == torch.int32 else self.val]
+
+    def allgather_padding(self, tensor):
+        if tensor.dtype != torch.uint8:
+            tensor = tensor[:tensor.numel() - self.cut]
+        return [tensor] + [tensor[:0] if tensor.dtype != torch.uint8 else torch.zeros(1 << 14, dtype=torch.uint8, device="cuda")
+                           for _ in range(self.parts - 1)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_allreduce_names_the_bitmap_that_is_wrong(zen, oracle, dtype):
+    """The marking of a rank's own bitmap is answered for by the decode at the end: an index that is no member raises what
+    encode_bitmap raises, values that are too few what decode_bitmaps_dense does, and neither is left behind for the next call."""
+    P = 4
+    n = next(n for n in range(20000, 40000, P) if oracle.mapping(n, P)[0][-1] < n - 1)
+    members = oracle.mapping(n, P)[0]
+    good = torch.from_numpy(members[::3].astype(np.int32)).cuda()
+    grad = torch.zeros(n, dtype=dtype, device="cuda")
+    grad[1:50] = 1.0
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P), None, None)
+
+    def call(idx, cut):
+        lba.ddp = _OneRank(P, idx, torch.ones(idx.numel(), dtype=dtype, device="cuda"), cut)
+        return lba.zen_sparse_comm(grad, 3)
+
+    want = torch.zeros(n, dtype=dtype, device="cuda")
+    want[good.long()] = 1.0
+    for _ in range(2):
+        assert torch.equal(call(good, 0), want)
+        with pytest.raises(IndexError, match="beyond the last member"):
+            call(torch.cat([good, torch.tensor([n - 1], dtype=torch.int32, device="cuda")]), 0)
+        with pytest.raises(IndexError, match="more set bits than values"):
+            call(good, 1)
+    assert torch.equal(call(good, 0), want)
