@@ -241,7 +241,7 @@ __device__ inline uint32_t sum_runs(const Shared &sh, uint32_t n, uint32_t per, 
     const uint32_t next = q + 1 < ITEMS ? ((uint32_t)(q + 1) < per ? k[q + 1 < ITEMS ? q + 1 : q] : after_k) : after_k;
     acc = (k[q] != prev ? 0.0f : acc) + v[q];
     sum[q] = acc;
-    keep |= ((uint32_t)q < own) & (k[q] != next) & SumAs<O>::kept(acc) ? 1u << q : 0u;
+    keep |= (((uint32_t)q < own) & (k[q] != next) & SumAs<O>::kept(acc)) ? 1u << q : 0u;
   }
   return keep;
 }

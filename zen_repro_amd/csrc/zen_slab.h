@@ -359,7 +359,7 @@ __device__ inline bool slab_rank(Shared &sh, const SlabGeom &geo, int tie_bits,
     for (int i = 0; i < kBatch && h + i < ITEMS; ++i) {
       uint32_t less = a[i][0] < word[h + i] ? 1u : 0u;
 #pragma unroll
-      for (int j = 1; j < kAhead; ++j) less += (size[h + i] > (uint32_t)j) & (a[i][j] < word[h + i]) ? 1u : 0u;
+      for (int j = 1; j < kAhead; ++j) less += ((size[h + i] > (uint32_t)j) & (a[i][j] < word[h + i])) ? 1u : 0u;
       if (size[h + i] > (uint32_t)kAhead)
         less += count_less(sh.key, g0[h + i] + kAhead, g0[h + i] + size[h + i], word[h + i]);
       if (!Shared::kQueue || rank[h + i] == 0) rank[h + i] = g0[h + i] + less;

@@ -422,7 +422,7 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
 #pragma unroll
         for (int e = 0; e < kAhead; ++e) {
           const bool in = e == 0 || size > (uint32_t)e;
-          less += in & (a[k][e] < key) ? 1u : 0u;  // (a smaller slot: the raw place is below it)
+          less += (in & (a[k][e] < key)) ? 1u : 0u;  // (a smaller slot: the raw place is below it)
           twins |= in & ((a[k][e] ^ my) - 1u < 0x7fffu);  // the same slot, another record
         }
         uint32_t x = g0[k] + less;

@@ -205,7 +205,7 @@ __device__ inline uint32_t wide_merge_sort(WideMergeShared &sh, const SlabGeom &
         const uint32_t size = g1[k] - g0[k];
         uint32_t less = a[k][0] < w[from + k] ? 1u : 0u;
 #pragma unroll
-        for (int e = 1; e < kAhead; ++e) less += (size > (uint32_t)e) & (a[k][e] < w[from + k]) ? 1u : 0u;
+        for (int e = 1; e < kAhead; ++e) less += ((size > (uint32_t)e) & (a[k][e] < w[from + k])) ? 1u : 0u;
         uint32_t x = g0[k] + less;
         if (size > (uint32_t)kAhead) {
           const uint32_t at = atomicAdd(&sh.qn, 1u);
@@ -341,7 +341,7 @@ __device__ __forceinline__ uint32_t wide_merge_sums(WideMergeShared &sh, uint32_
       const uint32_t next = q + 1 < ITEMS ? k[q + 1 < ITEMS ? q + 1 : q] : after_k;
       acc = (k[q] != prev ? 0.0f : acc) + v[q];
       sum[q] = acc;
-      keep |= ((uint32_t)q < own) & (k[q] != next) & (DENSE ? acc != 0.0f : SumAs<O>::kept(acc)) ? 1u << q : 0u;
+      keep |= (((uint32_t)q < own) & (k[q] != next) & (DENSE ? acc != 0.0f : SumAs<O>::kept(acc))) ? 1u << q : 0u;
     }
   }
   if (DENSE) wait_global_acks();  // this wave's zeros are written (the scan's barrier: everybody's)
