@@ -19,11 +19,11 @@ namespace {
 constexpr int kBins = 32768;       // 15 bits of the magnitude key
 constexpr int kBlock = 1024;
 // One workgroup as long as that is no slower than the two launches for larger samples: every 1024 elements cost it
-// 2.5 us, the gather of a single compute unit and its counting loop, and the other way costs a launch of the host's.  A
-// call in one launch and in two, us by events: bf16 1024 elements 9.8 and 13, 4096 17.8 and 13.6, 8192 28.8 and 14.0;
-// fp32 2048 elements 15.0 and 17, 4096 19.7 and 17.2, 10 486 39.0 and 17.1.  In front of a compress and a load balance,
-// which are bound by the host, one launch stays ahead a little longer: 4565 bf16 elements 100 and 104.5 us a pass, 4000
-// fp32 102.5 and 105, but 7000 bf16 106 and 103.
+// up to a microsecond, the gather of a single compute unit and its counting loop, and the other way costs a launch of the
+// host's.  A call on either side of the line, us by events: bf16 4096 elements 12.8, 5120 13.5, 5121 (two launches) 14.3,
+// 8192 14.4; fp32 4096 15.8, 5120 16.8, 5121 16.1, 8192 16.4.  In front of a compress and a load balance, which are bound by
+// the host, one launch stays ahead a little longer: 4565 bf16 elements 100 and 104.5 us a pass, 4000 fp32 102.5 and 105, but
+// 7000 bf16 106 and 103.
 constexpr int kOneItems = 5;
 constexpr int64_t kOneMax = kOneItems * kBlock;
 constexpr int kGroup = 64;         // bins per sum
