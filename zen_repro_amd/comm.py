@@ -450,25 +450,19 @@ class LoadBalanceAllreduce:
         """One bit per member of this rank's mapping list, set where the member
         is among sparse_indices; least significant bit first, padded to a whole
         byte (comm.py:59-85).  self.mapping[numel] must exist (comm.py:135)."""
+        mapping, ranks = self._ranks(sparse_indices, numel)
+        L = _lib.lib()
         words = _lib.host_words(1)
-        bitmap, _ = self._mark_bitmap(sparse_indices, numel, words)
+        rc, bitmap = _lib.host.bitmap_encode(L.zen_bitmap_encode_status, _lib.zeros.native(), mapping, sparse_indices,
+                                             ranks, numel, L.zen_bitmap_words(mapping.numel()),
+                                             _lib.stream_of(sparse_indices.device), words.ptr, words.words)
+        _lib.check(rc, "encode_bitmap")
         bits = words.view[1]
         if bits & _lib.STAT_BAD_INDEX:  # result[indices] = 1 with an index == len(result), comm.py:63
             raise IndexError("encode_bitmap: an index lies beyond the last member of the mapping")
         if bits:
             raise RuntimeError("encode_bitmap: " + _lib.describe_status(bits))
         return bitmap
-
-    def _mark_bitmap(self, sparse_indices, numel, words):
-        """(bitmap, status word on the device); waits for the status if `words` (of _lib.host_words) are there to take it."""
-        mapping, ranks = self._ranks(sparse_indices, numel)
-        L = _lib.lib()
-        rc, bitmap, status = _lib.host.bitmap_encode(
-            L.zen_bitmap_encode_status if words else L.zen_bitmap_encode, _lib.zeros.native(), mapping, sparse_indices, ranks,
-            numel, L.zen_bitmap_words(mapping.numel()), _lib.stream_of(sparse_indices.device),
-            *((words.ptr, words.words) if words else (0, 0)))
-        _lib.check(rc, "encode_bitmap")
-        return bitmap, status
 
     def decode_bitmap(self, bitmap_indices, numel):
         """For every rank i the members of mapping[numel][i] whose bit is set in
@@ -519,11 +513,6 @@ class LoadBalanceAllreduce:
         dense tensor and for what is said about bitmaps and values that do not
         agree: any stream may read the result and overwrite what it came from
         when the call has returned."""
-        return self._bitmaps_dense(bitmap_indices, values_tensors, numel)
-
-    def _bitmaps_dense(self, bitmap_indices, values_tensors, numel, marked=None):
-        """decode_bitmaps_dense; marked: (this rank's merged indices, the status
-        word their bitmap was marked with, which this call's wait answers for)."""
         if len(bitmap_indices) != self.partitions or len(values_tensors) != self.partitions:
             raise RuntimeError("decode_bitmaps_dense: one bitmap and one value list per rank")
         for t in bitmap_indices:
@@ -551,12 +540,10 @@ class LoadBalanceAllreduce:
         words = _lib.host_words(1)
         rc, dense = _lib.host.bitmaps_dense(L.zen_bitmap_dense_lists_status, _lib.zeros.native(), bitmap_indices, values,
                                             _lib.dtype_code(values[0]), cached, numel, ws, _lib.stream_of(dev), words.ptr,
-                                            words.words, marked[1] if marked else None)
+                                            words.words)
         _lib.check(rc, "decode_bitmaps_dense")
         bits = words.view[1]  # the reference's masking and scatter_add_ raise on a mismatch, also a sync
         if bits & _lib.STAT_BAD_INDEX:
-            if marked:
-                self.encode_bitmap(marked[0], numel)  # raises if it was an index of this rank's
             raise IndexError("decode_bitmaps_dense: a bitmap is shorter than its partition's index list, or has "
                              "more set bits than values came with it")
         if bits:
@@ -617,24 +604,17 @@ class LoadBalanceAllreduce:
             if numel not in self.mapping:
                 with ann("calculate_mapping"):
                     self.mapping[numel] = self.calculate_mapping(numel)
-            # With a decode behind it that waits, the marking is not waited for by itself: the host goes on to the exchange
-            # beside it, and the decode's answer says whether an index was no member.  A pass of the hook: 62 M bf16 on sixteen
-            # ranks, 10 %, 523 us and so 515; 268 M, 1 %, 611 and 600.
-            whole = self.partitions <= 64
             with ann("allgather_bitmap"):
                 with ann("encode_bitmap"):
-                    if whole:
-                        bitmap_indices, marked = self._mark_bitmap(sparse_indices, numel, None)
-                    else:
-                        bitmap_indices = self.encode_bitmap(sparse_indices, numel)
+                    bitmap_indices = self.encode_bitmap(sparse_indices, numel)
                 with ann("allgatherv"):
                     bitmap_indices_gather = ddp.allgather_padding(bitmap_indices)
             with ann("allgather indices"):
                 values_tensors = ddp.allgather_padding(sparse_values)
-            if whole:
+            if self.partitions <= 64:
                 # decode_bitmap + decode_sparse_tensors (comm.py:140-145) in one pass, without the indices
                 with ann("decode_bitmap"), ann("decode_sparse_tensors"):
-                    return self._bitmaps_dense(bitmap_indices_gather, values_tensors, numel, (sparse_indices, marked))
+                    return self.decode_bitmaps_dense(bitmap_indices_gather, values_tensors, numel)
             with ann("decode_bitmap"):
                 indices_tensors = self.decode_bitmap(bitmap_indices_gather, numel)
             with ann("decode_sparse_tensors"):
