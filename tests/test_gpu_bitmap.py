@@ -692,10 +692,11 @@ def test_comm_hook_needs_a_backend_for_more_than_one_rank(zen):
 
 class _OneRank:
     """The exchange of a rank that receives `idx` and whose peers send nothing else; `cut` values of the second exchange
-    are lost."""
+    are lost.  `sent`: what the second exchange was given, in copies taken on a stream that waits for no other."""
 
     def __init__(self, parts, idx, val, cut):
         self.parts, self.idx, self.val, self.cut = parts, idx, val, cut
+        self.sent, self.side = [], torch.cuda.Stream()
 
     def allgather(self, tensor):
         return [tensor]
@@ -704,6 +705,9 @@ class _OneRank:
         return [self.idx if tensors[0].dtype == torch.int32 else self.val]
 
     def allgather_padding(self, tensor):
+        with torch.cuda.stream(self.side):
+            self.sent.append(tensor.clone())
+        self.side.synchronize()
         if tensor.dtype != torch.uint8:
             tensor = tensor[:tensor.numel() - self.cut]
         return [tensor] + [tensor[:0] if tensor.dtype != torch.uint8 else torch.zeros(1 << 14, dtype=torch.uint8, device="cuda")
@@ -712,8 +716,8 @@ class _OneRank:
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_allreduce_names_the_bitmap_that_is_wrong(zen, oracle, dtype):
-    """The marking of a rank's own bitmap is answered for by the decode at the end: an index that is no member raises what
-    encode_bitmap raises, values that are too few what decode_bitmaps_dense does, and neither is left behind for the next call."""
+    """An index beyond the last member raises what encode_bitmap raises, values that are too few what decode_bitmaps_dense
+    does, and neither is left behind for the next call."""
     P = 4
     n = next(n for n in range(20000, 40000, P) if oracle.mapping(n, P)[0][-1] < n - 1)
     members = oracle.mapping(n, P)[0]
@@ -735,3 +739,47 @@ def test_allreduce_names_the_bitmap_that_is_wrong(zen, oracle, dtype):
         with pytest.raises(IndexError, match="more set bits than values"):
             call(good, 1)
     assert torch.equal(call(good, 0), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_allreduce_sends_no_bitmap_before_it_is_known_to_be_right(zen, oracle, dtype):
+    """An index beyond the last member raises in
+    front of the second exchange: its bitmap has fewer bits than there are values, which no peer would notice."""
+    n, P = 30001, 4
+    members = oracle.mapping(n, P)[0]
+    assert members[-1] < n - 1
+    idx = torch.from_numpy(np.append(members[::3], n - 1).astype(np.int32)).cuda()
+    grad = torch.zeros(n, dtype=dtype, device="cuda")
+    grad[1:50] = 1.0
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P), None, None)
+    lba.ddp = _OneRank(P, idx, torch.ones(idx.numel(), dtype=dtype, device="cuda"), 0)
+    with pytest.raises(IndexError, match="beyond the last member"):
+        lba.zen_sparse_comm(grad, 3)
+    assert not lba.ddp.sent
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_allreduce_sends_a_bitmap_that_is_there_for_every_stream(zen, oracle, dtype):
+    """The second exchange may read what it is given on any stream, whatever the call's own stream has in front of the
+    marking."""
+    n, P = 30000, 4
+    members = oracle.mapping(n, P)[0]
+    idx = torch.from_numpy(members[::3].astype(np.int32)).cuda()
+    grad = torch.zeros(n, dtype=dtype, device="cuda")
+    grad[1:50] = 1.0
+    lba = zen.LoadBalanceAllreduce(zen.LocalGroup(P), None, None)
+    lba.ddp = _OneRank(P, idx, torch.ones(idx.numel(), dtype=dtype, device="cuda"), 0)
+    calculate = lba.calculate_mapping
+
+    def slow(numel):  # called between the merge, which waits, and the marking
+        lists = calculate(numel)
+        torch.cuda._sleep(20000000)
+        return lists
+
+    lba.calculate_mapping = slow
+    want = torch.zeros(n, dtype=dtype, device="cuda")
+    want[idx.long()] = 1.0
+    assert torch.equal(lba.zen_sparse_comm(grad, 3), want)
+    bitmap, values = lba.ddp.sent
+    assert np.array_equal(to_np(bitmap), oracle.bitmap_encode(members, members[::3]))
+    assert torch.equal(values, torch.ones_like(values)) and values.numel() == idx.numel()
