@@ -100,6 +100,8 @@ def test_slab_load_balance_bit_exact(zen, oracle, n, P, density, rehash, dtype):
     # the losers of level 1: settled group by group where 0.7 capacity^2 / slots is above half a million
     (16, 24, 0.25, 1.0, 3, True),
     (128, 24, 0.27, 1.02, 2, True),   # nearly as full as buckets may be
+    (32, 24, 0.278, 1.0, 3, True),    # 943 of a part's 1024 cells taken, 1065 if losers with a smaller owner took one ...
+    (32, 24, 0.2812, 1.0, 3, True),   # ... 966 and 1091
     (1, 26, 0.08, 1.35, 3, True),     # one partition of all groups
     (7, 24, 0.22, 1.05, 3, True),     # the last group of a partition has fewer buckets
     (300, 24, 0.22, 1.05, 3, False),  # too many partitions for lists
@@ -125,6 +127,51 @@ def test_slab_load_balance_of_settled_losers(zen, oracle, P, log2, density, room
         assert np.array_equal(to_np(ov)[:len(idx_o)], val_o)
     m, _ = oracle.table_sizes(n, P, 1)
     assert not tp._table(d.device, m).any()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("rehash", [2, 3])
+@pytest.mark.parametrize("fast_path", ["slabs"], indirect=True)
+def test_slab_load_balance_of_losers_in_one_place(zen, oracle, rehash, dtype):
+    """More losers than a group's list takes (the rest go their way from their buckets' own lists, beside what the group has
+    left over), and a bucket with more losers than its workgroup has threads."""
+    from zen_repro_amd import _lib
+    from zen_repro_amd.workloads import hash_slot
+
+    n, P, capacity = (1 << 24) + 160, 16, 3500000
+    npp, bpp, per_group = n // P, 62, 4  # 3584 entries to a bucket; groups of at least four buckets, 256 of them
+    listed = int(1.25 * 0.7 * capacity * (capacity / n) / (P * 16)) + 512
+
+    def bucket(slot):  # of the partition
+        return slot % npp * ((bpp << 32) // npp) >> 32
+
+    t = torch.arange(1, n, device="cuda")
+    first = hash_slot(t, n)
+    second = (hash_slot(t, 1 << 32) - 10001861 + 100703) % (1 << 32) % npp
+    order = torch.argsort(first, stable=True)  # by slot, then index: whoever is not the first of its slot loses it
+    twin = torch.zeros(n - 1, dtype=torch.bool, device="cuda")
+    twin[order[1:]] = first[order[1:]] == first[order[:-1]]
+    mate = torch.zeros(n - 1, dtype=torch.int64, device="cuda")  # ... to the index in front of it
+    mate[order[1:]] = order[:-1]
+    to_group = twin & (first // npp == 5) & (bucket(second) // per_group == 3)
+    in_bucket = twin & (first // npp == 9) & (bucket(first) == 17)
+    chosen = torch.cat([torch.nonzero(to_group).view(-1)[:listed + 400], torch.nonzero(in_bucket).view(-1)[:1300]])
+    assert chosen.numel() == listed + 1700
+    g = make_grad(oracle, n, 0.03, dtype, seed=rehash)
+    at = torch.cat([chosen, mate[chosen]]).cpu().numpy() + 1
+    g[at] = 0x3F80 if dtype == "bf16" else 1.0
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, rehash)
+    assert st_o == 0 and len(idx_o) < capacity and lb_path(zen, n, P, dtype, capacity) == SLAB
+    assert 0.7 * capacity ** 2 / n > 500000
+    tp = zen.TensorPartition(P, 1, rehash)
+    d = to_dev(g)
+    for rep in range(2):  # the second call finds the counters and the map zero again
+        oi, ov, splits, status = tp.load_balance_flat(d, capacity=capacity, mode=_lib.MODE_FAST)
+        assert status.item() == 0
+        assert np.array_equal(to_np(splits), splits_o)
+        assert np.array_equal(to_np(oi)[:len(idx_o)], idx_o)
+        assert np.array_equal(to_np(ov)[:len(idx_o)], val_o)
+    assert not tp._table(d.device, n).any()
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])

@@ -42,7 +42,7 @@ struct SlabTables {
   uint32_t *bucket_lo;  // [B] smallest level-1 slot of the bucket
   uint32_t *bucket_n;   // [B] sorted records in the slab: level-1 owners, in wide buckets the losers too
   uint32_t *removed_n;  // [B] of which have lost their slot
-  uint32_t *movein_n;   // [B * kMoveinPad] entries that moved in; a word behind: the part of the map has dead cells
+  uint32_t *movein_n;   // [B * kMoveinPad] occupied cells of the bucket's part of the map: entries that moved in
   uint32_t *serial_n;   // [P * kMoveinPad] entries that found no slot
   uint32_t *raw_idx;    // [B * kSlabCap] entries as they arrive: index (after the sort: losers, again_n of them) ...
   void *raw_val;        // ... and value
@@ -60,8 +60,8 @@ struct SlabTables {
   uint32_t *out_start;  // [B + 1] where every bucket starts in the output
   uint32_t *done;       // [kDoneWords] workgroups of k_slab_chains that have finished
   uint32_t *final_n;    // [B + P] what k_slab_place needs of the counters above, copied by the last workgroup of
-                        // k_slab_chains before it puts them back to zero: moved-in entries per bucket (kHasDead: dead
-                        // cells too), serial entries per partition
+                        // k_slab_chains before it puts them back to zero: moved-in entries per bucket, serial entries
+                        // per partition
   uint32_t *coarse_cursor;  // the feed's coarse cursors and, for an fp32 top-k, the refinement histogram (else
   uint32_t *refine_hist;    // null): k_slab_sort puts them back to zero
   int partitions;
@@ -73,12 +73,9 @@ struct SlabTables {
 
 // Device-wide atomics on one 128-byte line are carried out one after the other: four counters to a line.
 constexpr uint32_t kMoveinPad = 8;
-constexpr uint32_t kHasDead = 1u << 31;
 
-// A cell of the map: (slot + 1) << 32 | index, 0 if empty, of index kNone if nobody is left in it (dead).
+// A cell of the map: (slot + 1) << 32 | index, 0 if empty.
 __device__ inline uint32_t cell_slot(unsigned long long cell) { return (uint32_t)(cell >> 32) - 1u; }
-// The index in a cell, 0 if there is none.
-__device__ inline uint32_t cell_index(unsigned long long cell) { return (uint32_t)cell == kNone ? 0u : (uint32_t)cell; }
 
 // Where many losers are expected a bucket's losers go to lists, by the group of buckets their level-2 slots lie in, and
 // k_slab_settle enters a group's list into its parts of the map in LDS: device-wide atomics are carried out at 25 a
@@ -487,7 +484,7 @@ __device__ inline uint32_t slab_head(const SlabGeom &geo, const SlabTables &tb, 
 }
 
 // Enters t as a prober of `slot` in bucket b's part of the map; returns the smallest earlier prober (kNone: there was
-// none, or the cell was dead).  *full is set if the part has no room.
+// none).  *full is set if the part has no room.
 __device__ inline uint32_t part_min(unsigned long long *cells, uint32_t b, uint32_t slot, uint32_t t, bool *full) {
   unsigned long long *part = cells + ((size_t)b << kSlabPartLog2);
   constexpr uint32_t mask = (1u << kSlabPartLog2) - 1u;
@@ -514,15 +511,13 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
                                           int32_t *status) {
   constexpr uint32_t kPer = kSlabMaxBuckets / kSlabBlock;
   const uint32_t B = geo.nbuckets, P = (uint32_t)tb.partitions;
-  unsigned long long *movein = reinterpret_cast<unsigned long long *>(tb.movein_n);
-  unsigned long long mv[kPer];
-  uint32_t rm[kPer], n[kPer], sn[kPer];
+  uint32_t mv[kPer], rm[kPer], n[kPer], sn[kPer];
 #pragma unroll
   for (uint32_t e = 0; e < kPer; ++e) {  // (the conditions are the same for all threads: all loads are in flight together)
     const uint32_t x = threadIdx.x + e * (uint32_t)kSlabBlock;
     if (e * (uint32_t)kSlabBlock < B) {
       const uint32_t at = x < B ? x : 0u;
-      mv[e] = __hip_atomic_load(&movein[at * (kMoveinPad / 2)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      mv[e] = load_fresh(&tb.movein_n[at * kMoveinPad]);
       rm[e] = load_fresh(&tb.removed_n[at]);
       n[e] = tb.bucket_n[at];
     }
@@ -531,7 +526,7 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
 #pragma unroll
   for (uint32_t e = 0; e < kPer; ++e) {
     const uint32_t x = threadIdx.x + e * (uint32_t)kSlabBlock;
-    if (x < B) s_start[x] = n[e] + (uint32_t)mv[e] - rm[e];
+    if (x < B) s_start[x] = n[e] + mv[e] - rm[e];
   }
   __syncthreads();
   bool overflow = false;
@@ -579,8 +574,8 @@ __device__ inline void slab_output_starts(const SlabGeom &geo, const SlabTables 
     const uint32_t x = threadIdx.x + e * (uint32_t)kSlabBlock;
     if (x < B) {
       tb.out_start[x] = s_start[x];
-      tb.final_n[x] = (uint32_t)mv[e] | (mv[e] >> 32 ? kHasDead : 0u);
-      movein[x * (kMoveinPad / 2)] = 0;
+      tb.final_n[x] = mv[e];
+      tb.movein_n[x * kMoveinPad] = 0;
     }
     if (x < P) {
       tb.final_n[B + x] = sn[e];
@@ -623,7 +618,7 @@ __device__ inline void slab_chain(const SlabGeom &geo, const Probe &g, const Sla
       continue;
     }
     if (old == kNone) {
-      // first level-2/3 prober of this slot that counts: its level-1 owner (a larger index, if any) is pushed out
+      // first level-2/3 prober of this slot: its level-1 owner (a larger index, if any) is pushed out
       atomicAdd(&tb.movein_n[bucket * kMoveinPad], 1u);
       if (head == kNone) break;
       atomicOr(reinterpret_cast<uint32_t *>(&tb.slab_idx[head_pos]), kRemovedBit);
@@ -641,17 +636,19 @@ __device__ inline void slab_chain(const SlabGeom &geo, const Probe &g, const Sla
   }
 }
 
-// Level 2 for a group's list of losers.  All of them are entered in the group's parts of the map, which are put together in
-// LDS; whoever finds a smaller index there, or is pushed out by one, goes on at level 3.  Of those that are left one in
-// ten or so finds a level-1 owner: a smaller one sends it on (its cell stays, dead: entries behind it may have come past
-// it), a larger one is pushed out and goes on at level 2.  Nobody else touches the map while this kernel runs.  Bound by
-// latency (four or five trips to memory, as many phases in LDS) and instructions: a group to a compute unit, its losers to
-// all of the unit's waves.  62 M slots, 436 000 losers in 256 groups 19.5 us, the chains behind it 23 (without it the
-// chains 50, and 15 to count the entries that moved in).
+// Level 2 for a group's list of losers.  One in ten or so finds a level-1 owner in its slot: a smaller one sends it on to
+// level 3.  The others are entered in the group's parts of the map, which are put together in LDS; whoever finds a smaller
+// index there, or is pushed out by one, goes on at level 3 too.  A larger level-1 owner is pushed out by the entry that holds
+// its slot in the end, and goes on at level 2.  The owner is asked for first, as a single chain does: a slot with a smaller
+// owner takes no cell, and the parts hold no more than the chains alone would put there (16.8 M slots, 27.8 % of them taken,
+// 32 partitions: 943 cells in the fullest part; entered first, 1065, more than there are).  Nobody else touches the map while this kernel
+// runs.  Bound by latency (four or five trips to memory, as many phases in LDS) and instructions: a group to a compute
+// unit, its losers to all of the unit's waves.  62 M slots, 436 000 losers in 256 groups 19.5 us, the chains behind it 23
+// (without it the chains 50, and 15 to count the entries that moved in).
 struct SlabSettleLds {
   unsigned long long cells[kGroupBuckets << kSlabPartLog2];
   uint16_t index[kGroupBuckets * kSlabIndexLen];  // the buckets' indices
-  uint32_t alive[kGroupBuckets], dead[kGroupBuckets], pushed[kGroupBuckets];
+  uint32_t in[kGroupBuckets], pushed[kGroupBuckets];  // entries that move in, level-1 owners pushed out
   uint32_t tokens;
 };
 
@@ -672,59 +669,37 @@ __global__ __launch_bounds__(kSettleBlock) void k_slab_settle(SlabGeom geo, Slab
   count = count < tb.group_cap ? count : tb.group_cap;
   u32x4 *clear = reinterpret_cast<u32x4 *>(sh.cells);
   for (uint32_t i = threadIdx.x; i < (buckets << kSlabPartLog2) / 2u; i += kSettleBlock) clear[i] = u32x4{0, 0, 0, 0};
-  if (threadIdx.x < kGroupBuckets) sh.alive[threadIdx.x] = sh.dead[threadIdx.x] = sh.pushed[threadIdx.x] = 0;
+  if (threadIdx.x < kGroupBuckets) sh.in[threadIdx.x] = sh.pushed[threadIdx.x] = 0;
   if (threadIdx.x == 0) sh.tokens = 0;
   __syncthreads();
   if (threadIdx.x == 0) *counter = 0;
   // rows nobody has a loser in are skipped by the whole workgroup; the loads of a step are in flight together
-  uint32_t t[kSettleRows], cell[kSettleRows];
+  uint32_t t[kSettleRows];
   SlabGeom::Spot spot[kSettleRows];
-  uint32_t in = 0;  // bit r: row r has a loser for this thread; from the second barrier on, one that holds its cell
+  uint32_t in = 0;  // bit r: row r has a loser for this thread that may hold its slot
 #pragma unroll
   for (int r = 0; r < kSettleRows; ++r) {
     const uint32_t i = r * kSettleBlock + threadIdx.x;
     if ((uint32_t)(r * kSettleBlock) < count) t[r] = list[i < count ? i : 0u];
     in |= (i < count ? 1u : 0u) << r;
   }
-#pragma unroll
-  for (int r = 0; r < kSettleRows; ++r) {
-    if ((uint32_t)(r * kSettleBlock) >= count) continue;
-    spot[r] = geo.spot(t[r], 1);
-    cell[r] = 0;
-    if (!(in & (1u << r))) continue;
-    const uint32_t at = (spot[r].bucket - b0) << kSlabPartLog2;
-    const unsigned long long mine = ((unsigned long long)(spot[r].slot + 1u) << 32) | t[r];
-    uint32_t h = cell_home(spot[r].slot, kSlabPartLog2), probes = 0;
-    for (; probes <= mask; ++probes, h = (h + 1u) & mask) {
-      const unsigned long long cur = atomicCAS(&sh.cells[at + h], 0ull, mine);
-      if (cur == 0ull) break;
-      if (cell_slot(cur) == spot[r].slot) {
-        const uint32_t old = (uint32_t)atomicMin(&sh.cells[at + h], mine);
-        token[atomicAdd(&sh.tokens, 1u)] = (old < t[r] ? t[r] : old) | kAtLevel3;
-        break;
-      }
-    }
-    cell[r] = at + h;
-    if (probes > mask) atomicOr(status, ZEN_STAT_RETRY);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < kSettleRows; ++r)
-    if ((uint32_t)(r * kSettleBlock) < count && (uint32_t)sh.cells[cell[r]] != t[r]) in &= ~(1u << r);
   // whose level-1 slot is it: the bucket's index narrows the search to a few records (see slab_head)
   uint32_t head[kSettleRows], pos[kSettleRows], left[kSettleRows], near[kSettleRows][4];
 #pragma unroll
   for (int r = 0; r < kSettleRows; ++r) {
     if ((uint32_t)(r * kSettleBlock) >= count) continue;
+    spot[r] = geo.spot(t[r], 1);
     const uint32_t local = spot[r].bucket - b0;
     const uint32_t j = local * kSlabIndexLen + (spot[r].offset >> geo.sub_shift) / (uint32_t)kSlabIndexStep;
     pos[r] = local * (uint32_t)kSlabCap + sh.index[j];
     left[r] = (uint32_t)sh.index[j + 1u] - sh.index[j];
     __builtin_memcpy(near[r], slab_idx + pos[r], sizeof(near[r]));  // (words past the range are not looked at)
   }
+  uint32_t cell[kSettleRows];
 #pragma unroll
   for (int r = 0; r < kSettleRows; ++r) {
     head[r] = kNone;
+    cell[r] = 0;
     if ((uint32_t)(r * kSettleBlock) >= count || !(in & (1u << r))) continue;
     for (uint32_t at = pos[r];;) {
       bool past = false;
@@ -743,18 +718,33 @@ __global__ __launch_bounds__(kSettleBlock) void k_slab_settle(SlabGeom geo, Slab
       at += 4u;
       __builtin_memcpy(near[r], slab_idx + at, sizeof(near[r]));
     }
-  }
-#pragma unroll
-  for (int r = 0; r < kSettleRows; ++r) {
-    if ((uint32_t)(r * kSettleBlock) >= count || !(in & (1u << r))) continue;
-    const uint32_t local = cell[r] >> kSlabPartLog2;
     if (head[r] < t[r]) {
-      sh.cells[cell[r]] |= kNone;
-      sh.dead[local] = 1;
+      in &= ~(1u << r);
       token[atomicAdd(&sh.tokens, 1u)] = t[r] | kAtLevel3;
       continue;
     }
-    atomicAdd(&sh.alive[local], 1u);
+    const uint32_t at = (spot[r].bucket - b0) << kSlabPartLog2;
+    const unsigned long long mine = ((unsigned long long)(spot[r].slot + 1u) << 32) | t[r];
+    uint32_t h = cell_home(spot[r].slot, kSlabPartLog2), probes = 0;
+    for (; probes <= mask; ++probes, h = (h + 1u) & mask) {
+      const unsigned long long cur = atomicCAS(&sh.cells[at + h], 0ull, mine);
+      if (cur == 0ull) break;
+      if (cell_slot(cur) == spot[r].slot) {
+        const uint32_t old = (uint32_t)atomicMin(&sh.cells[at + h], mine);
+        token[atomicAdd(&sh.tokens, 1u)] = (old < t[r] ? t[r] : old) | kAtLevel3;
+        break;
+      }
+    }
+    cell[r] = at + h;
+    if (probes > mask) atomicOr(status, ZEN_STAT_RETRY);
+  }
+  __syncthreads();
+  // everybody has entered: who holds the slot moves in, and pushes out a level-1 owner that is there
+#pragma unroll
+  for (int r = 0; r < kSettleRows; ++r) {
+    if ((uint32_t)(r * kSettleBlock) >= count || !(in & (1u << r)) || (uint32_t)sh.cells[cell[r]] != t[r]) continue;
+    const uint32_t local = cell[r] >> kSlabPartLog2;
+    atomicAdd(&sh.in[local], 1u);
     if (head[r] != kNone) {
       slab_idx[pos[r]] = (int32_t)(head[r] | kRemovedBit);
       atomicAdd(&sh.pushed[local], 1u);
@@ -768,8 +758,7 @@ __global__ __launch_bounds__(kSettleBlock) void k_slab_settle(SlabGeom geo, Slab
     if (q.y | q.w) out[i] = q;  // (the map is zero)
   }
   if (threadIdx.x < buckets) {
-    tb.movein_n[(b0 + threadIdx.x) * kMoveinPad] = sh.alive[threadIdx.x];
-    tb.movein_n[(b0 + threadIdx.x) * kMoveinPad + 1u] = sh.dead[threadIdx.x];
+    tb.movein_n[(b0 + threadIdx.x) * kMoveinPad] = sh.in[threadIdx.x];
     tb.removed_n[b0 + threadIdx.x] = sh.pushed[threadIdx.x];
   }
   if (threadIdx.x == 0) tb.token_n[group] = sh.tokens;
@@ -928,10 +917,9 @@ __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, Slab
   sh.taken.template clear<kSlabBlock>(words);
   S mval[kCells];  // an entry is a copy of the element it stands for
 #pragma unroll
-  for (int e = 0; e < kCells; ++e) mval[e] = mv_n ? dense[cell_index(moved[e])] : S(0);
+  for (int e = 0; e < kCells; ++e) mval[e] = mv_n ? dense[(uint32_t)moved[e]] : S(0);
   __syncthreads();
   uint32_t off[kSlabItems], moff[kCells];
-  uint32_t in = 0;  // bit e: the cell holds an entry (it is not dead)
 #pragma unroll
   for (int i = 0; i < kSlabItems; ++i) {
     off[i] = 0;
@@ -943,9 +931,8 @@ __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, Slab
 #pragma unroll
   for (int e = 0; e < kCells; ++e) {
     moff[e] = 0;
-    if (moved[e]) cell[e * kSlabBlock] = 0ull;
-    if (moved[e] && (uint32_t)moved[e] != kNone) {
-      in |= 1u << e;
+    if (moved[e]) {
+      cell[e * kSlabBlock] = 0ull;
       moff[e] = cell_slot(moved[e]) - lo;
       sh.taken.take(moff[e], 1u);
     }
@@ -965,7 +952,7 @@ __global__ __launch_bounds__(kSlabBlock, 6) void k_slab_place(SlabGeom geo, Slab
   }
 #pragma unroll
   for (int e = 0; e < kCells; ++e) {
-    if (in & (1u << e)) {
+    if (moved[e]) {
       const uint32_t pos = out_base + sh.taken.place(moff[e]);
       if (pos < capacity) {
         out_idx[pos] = (int32_t)(uint32_t)moved[e];
