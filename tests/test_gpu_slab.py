@@ -96,16 +96,32 @@ def test_slab_load_balance_bit_exact(zen, oracle, n, P, density, rehash, dtype):
     assert not tp._table(d.device, m).any()
 
 
+def slab_buckets(m, P, capacity):
+    """Buckets of a partition (slab_geometry): 3584 entries each, or fuller ones where that saves a round of 512."""
+    bpp = min(-(-capacity // (3584 * P)), 4096 // P)
+    fewer = (-(-bpp * P // 512) - 1) * 512 // P
+    return fewer if fewer and capacity // (fewer * P) <= 4608 else bpp
+
+
+def slab_settles(m, P, capacity):
+    """Whether the losers of level 1 are settled group by group (plan_slab)."""
+    losers = 0.5 * capacity ** 2 / m * (0.7 if m & (m - 1) == 0 else 1 if m % 4 else 1.4)
+    return losers > max(135 * slab_buckets(m, P, capacity) * P, 40000)
+
+
 @pytest.mark.parametrize("P,log2,density,room,rehash,settled", [
-    # the losers of level 1: settled group by group where 0.7 capacity^2 / slots is above half a million
     (16, 24, 0.25, 1.0, 3, True),
     (128, 24, 0.27, 1.02, 2, True),   # nearly as full as buckets may be
     (32, 24, 0.278, 1.0, 3, True),    # 943 of a part's 1024 cells taken, 1065 if losers with a smaller owner took one ...
     (32, 24, 0.2812, 1.0, 3, True),   # ... 966 and 1091
     (1, 26, 0.08, 1.35, 3, True),     # one partition of all groups
     (7, 24, 0.22, 1.05, 3, True),     # the last group of a partition has fewer buckets
-    (300, 24, 0.22, 1.05, 3, False),  # too many partitions for lists
-    (16, 24, 0.2, 1.03, 3, False),    # just below the line
+    (300, 24, 0.22, 1.05, 3, True),   # more partitions than groups are wanted: groups of three buckets
+    (1000, 24, 0.24, 1.02, 2, True),  # ... of one
+    (16, 24, 0.057, 1.0, 3, False),   # fewer than 40 000 losers
+    (16, 24, 0.06, 1.0, 3, True),
+    (257, 24, 0.09, 1.0, 3, False),   # fewer than 135 to a bucket
+    (257, 24, 0.093, 1.0, 3, True),
 ])
 @pytest.mark.parametrize("fast_path", ["slabs"], indirect=True)
 def test_slab_load_balance_of_settled_losers(zen, oracle, P, log2, density, room, rehash, settled):
@@ -116,7 +132,7 @@ def test_slab_load_balance_of_settled_losers(zen, oracle, P, log2, density, room
     idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, rehash)
     capacity = int(len(idx_o) * room)
     assert st_o == 0 and lb_path(zen, n, P, "bf16", capacity) == SLAB
-    assert (0.7 * capacity ** 2 / n > 500000 and P < 256) == settled
+    assert slab_settles(n, P, capacity) == settled
     tp = zen.TensorPartition(P, 1, rehash)
     d = to_dev(g)
     for rep in range(2):  # the second call finds the counters and the map zero again
@@ -162,7 +178,7 @@ def test_slab_load_balance_of_losers_in_one_place(zen, oracle, rehash, dtype):
     g[at] = 0x3F80 if dtype == "bf16" else 1.0
     idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, rehash)
     assert st_o == 0 and len(idx_o) < capacity and lb_path(zen, n, P, dtype, capacity) == SLAB
-    assert 0.7 * capacity ** 2 / n > 500000
+    assert slab_settles(n, P, capacity)
     tp = zen.TensorPartition(P, 1, rehash)
     d = to_dev(g)
     for rep in range(2):  # the second call finds the counters and the map zero again
@@ -175,18 +191,17 @@ def test_slab_load_balance_of_losers_in_one_place(zen, oracle, rehash, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
-@pytest.mark.parametrize("P,density,room,losers", [
-    # where the entries that moved in are counted: by the chains up to 50 000 losers, behind them where there are more
-    # and the capacity has room for many
-    (16, 0.2, 1.05, 451039),
-    (3, 0.16, 1.1, 202997),
-    (16, 0.1, 2.0, 119306),
-    (3, 0.08, 2.0, 52072),    # just past the line
-    (3, 0.078, 2.1, 49630),   # just below it, with the launch behind the chains
-    (16, 0.1, 1.1, 119306),   # without it
+@pytest.mark.parametrize("P,density,room,losers,settled", [
+    # losers that are settled group by group, and that each go their way
+    (16, 0.2, 1.05, 451039, True),
+    (3, 0.16, 1.1, 202997, True),
+    (16, 0.1, 2.0, 119306, True),
+    (16, 0.1, 1.1, 119306, True),
+    (3, 0.078, 1.0, 49630, True),   # just past the line
+    (3, 0.075, 1.0, 45974, False),  # just below it
 ])
 @pytest.mark.parametrize("fast_path", ["slabs"], indirect=True)
-def test_slab_load_balance_of_many_losers(zen, oracle, P, density, room, losers, dtype):
+def test_slab_load_balance_of_many_losers(zen, oracle, P, density, room, losers, settled, dtype):
     from zen_repro_amd import _lib
     from zen_repro_amd.workloads import hash_slot
 
@@ -196,7 +211,7 @@ def test_slab_load_balance_of_many_losers(zen, oracle, P, density, room, losers,
     capacity = int(len(idx_o) * room)
     assert st_o == 0 and lb_path(zen, n, P, dtype, capacity) == SLAB
     assert len(idx_o) - torch.unique(hash_slot(torch.from_numpy(idx_o.astype(np.int64)), n)).numel() == losers
-    assert (capacity ** 2 / (2 * n) > 200000) == (room != 1.1 or P == 3)
+    assert slab_settles(n, P, capacity) == settled
     tp = zen.TensorPartition(P, 1, 3)
     d = to_dev(g)
     for rep in range(2):  # the second call finds the counters zero again

@@ -68,7 +68,7 @@ struct SlabTables {
   uint32_t gpp;         // groups in a partition ...
   uint32_t per_group;   // ... of so many buckets
   uint32_t group_pad;   // words from one partition's counters to the next's
-  uint32_t group_cap;   // losers in a group's list (0: no lists)
+  uint32_t group_cap;   // losers in a group's list (0: no lists), at most kSettleRows to a thread of its workgroup
 };
 
 // Device-wide atomics on one 128-byte line are carried out one after the other: four counters to a line.
@@ -81,17 +81,24 @@ __device__ inline uint32_t cell_slot(unsigned long long cell) { return (uint32_t
 // k_slab_settle enters a group's list into its parts of the map in LDS: device-wide atomics are carried out at 25 a
 // nanosecond, and of an entry for each loser in the map and one to count it nine in ten fall away.  Where fewer are
 // expected each goes its way through memory (k_slab_chains), for the other way is a launch more and two barriers in the sort.
-// The line is an estimate from the capacity; the hash loses 1.4 times as many as evenly spread slots would.  Whole calls,
-// settled and not, 62 M slots, bf16, sixteen partitions: 436 000 losers (estimate 980 000) 554 and 570 us, 110 000 (240 000)
-// 416 and 413; 268 M, 18 000 (42 000) 643 and 637.
-constexpr double kSettleFrom = 500000;
+// What settling costs goes with the buckets, what it saves with the losers: it pays from about 135 expected losers to a
+// bucket and 40 000 in all.  Whole calls, bf16, 62 M slots, sixteen partitions, by losers to a bucket, unsettled and settled,
+// us: 120 115.2 and 114.5, 146 122.9 and 122.8, 195 127.0 and 123.4, 208 158.1 and 147.3, 325 202.9 and 180.3, 382 313.8 and
+// 255.5.  250 M: 117 254.6 and 254.2, 144 300.4 and 294.2.  62 M, an odd number: 105 118.4 and 120.9, 174 131.7 and 130.3, 206
+// 203.5 and 188.3.  2^26: 91 122.7 and 123.4, 162 149.0 and 146.5.  2^28: 84 307.1 and 314.6.  Few in all, 4 to 17 M slots:
+// 29 000 55.6 and 54.9, 55.7 and 56.8, 59.9 and 60.6; 39 000 66.6 and 67.4; 44 000 62.8 and 61.3, 61.7 and 60.1; 59 000 69.6
+// and 65.5, 74.7 and 74.5.
+constexpr double kSettleFrom = 135, kSettleLeast = 40000;
 constexpr uint32_t kGroupBuckets = 12;         // of a group, at most: their parts of the map and indices fill 121 KB
-constexpr uint32_t kGroupLeast = 4, kGroupsWanted = 256;  // (a compute unit to each)
-constexpr uint32_t kMostGroups = 256;          // of a partition
-constexpr size_t kMostGroupWords = 8192;       // of all partitions' counters, a partition's in memory lines of their own
+constexpr uint32_t kGroupLeast = 4, kGroupsMost = 256;  // (a compute unit to each)
+constexpr uint32_t kMostGroups = kSlabMaxBuckets / kGroupBuckets + 1;  // of a partition
 constexpr int kSettleBlock = 1024;
 constexpr int kSettleRows = 6;                 // losers of a thread, at most
-constexpr uint32_t kGroupCap = kSettleBlock * kSettleRows;
+// More partitions than kGroupsMost: groups of a few buckets, five to a compute unit (and the same line).  62 M slots, 300
+// partitions, by expected losers to a bucket: 99 105.9 and 106.7 us, 166 116.5 and 114.7, 199 157.9 and 147.4, 408 294 and 245; 1024:
+// 87 109.4 and 110.7, 146 126.8 and 123.7, 195 172 and 163; 3000: 99 176 and 179, 166 226 and 213, 326 324 and 271.
+constexpr uint32_t kFewBuckets = 3, kFewGroupsMost = 1280;
+constexpr int kFewBlock = 256;
 constexpr uint32_t kChainsResident = 1024;     // workgroups of k_slab_chains the chip holds at a time
 constexpr uint32_t kAtLevel3 = 1u << 31;       // in a list: the index goes on at level 3 (else at level 2)
 
@@ -645,16 +652,19 @@ __device__ inline void slab_chain(const SlabGeom &geo, const Probe &g, const Sla
 // runs.  Bound by latency (four or five trips to memory, as many phases in LDS) and instructions: a group to a compute
 // unit, its losers to all of the unit's waves.  62 M slots, 436 000 losers in 256 groups 19.5 us, the chains behind it 23
 // (without it the chains 50, and 15 to count the entries that moved in).
+template <uint32_t BUCKETS>
 struct SlabSettleLds {
-  unsigned long long cells[kGroupBuckets << kSlabPartLog2];
-  uint16_t index[kGroupBuckets * kSlabIndexLen];  // the buckets' indices
-  uint32_t in[kGroupBuckets], pushed[kGroupBuckets];  // entries that move in, level-1 owners pushed out
+  unsigned long long cells[BUCKETS << kSlabPartLog2];
+  uint16_t index[BUCKETS * kSlabIndexLen];  // the buckets' indices
+  uint32_t in[BUCKETS], pushed[BUCKETS];    // entries that move in, level-1 owners pushed out
   uint32_t tokens;
 };
 
-__global__ __launch_bounds__(kSettleBlock) void k_slab_settle(SlabGeom geo, SlabTables tb, unsigned long long *cells,
-                                                              int32_t *status) {
-  __shared__ SlabSettleLds sh;
+template <int BLOCK, uint32_t BUCKETS>
+__global__ __launch_bounds__(BLOCK) void k_slab_settle(SlabGeom geo, SlabTables tb, unsigned long long *cells,
+                                                       int32_t *status) {
+  static_assert(BUCKETS <= BLOCK, "a thread to a bucket");
+  __shared__ SlabSettleLds<BUCKETS> sh;
   constexpr uint32_t mask = (1u << kSlabPartLog2) - 1u;
   const uint32_t group = blockIdx.x, part = group / tb.gpp, first = (group - part * tb.gpp) * tb.per_group;
   const uint32_t b0 = part * geo.bpp + first;
@@ -665,11 +675,11 @@ __global__ __launch_bounds__(kSettleBlock) void k_slab_settle(SlabGeom geo, Slab
   uint32_t *token = tb.token + (size_t)group * tb.group_cap;  // (a loser leaves one at most)
   uint32_t count = *counter;
   const uint16_t *index = tb.sub_index + (size_t)b0 * kSlabIndexLen;
-  for (uint32_t i = threadIdx.x; i < buckets * kSlabIndexLen; i += kSettleBlock) sh.index[i] = index[i];
+  for (uint32_t i = threadIdx.x; i < buckets * kSlabIndexLen; i += BLOCK) sh.index[i] = index[i];
   count = count < tb.group_cap ? count : tb.group_cap;
   u32x4 *clear = reinterpret_cast<u32x4 *>(sh.cells);
-  for (uint32_t i = threadIdx.x; i < (buckets << kSlabPartLog2) / 2u; i += kSettleBlock) clear[i] = u32x4{0, 0, 0, 0};
-  if (threadIdx.x < kGroupBuckets) sh.in[threadIdx.x] = sh.pushed[threadIdx.x] = 0;
+  for (uint32_t i = threadIdx.x; i < (buckets << kSlabPartLog2) / 2u; i += BLOCK) clear[i] = u32x4{0, 0, 0, 0};
+  if (threadIdx.x < BUCKETS) sh.in[threadIdx.x] = sh.pushed[threadIdx.x] = 0;
   if (threadIdx.x == 0) sh.tokens = 0;
   __syncthreads();
   if (threadIdx.x == 0) *counter = 0;
@@ -679,15 +689,15 @@ __global__ __launch_bounds__(kSettleBlock) void k_slab_settle(SlabGeom geo, Slab
   uint32_t in = 0;  // bit r: row r has a loser for this thread that may hold its slot
 #pragma unroll
   for (int r = 0; r < kSettleRows; ++r) {
-    const uint32_t i = r * kSettleBlock + threadIdx.x;
-    if ((uint32_t)(r * kSettleBlock) < count) t[r] = list[i < count ? i : 0u];
+    const uint32_t i = r * BLOCK + threadIdx.x;
+    if ((uint32_t)(r * BLOCK) < count) t[r] = list[i < count ? i : 0u];
     in |= (i < count ? 1u : 0u) << r;
   }
   // whose level-1 slot is it: the bucket's index narrows the search to a few records (see slab_head)
   uint32_t head[kSettleRows], pos[kSettleRows], left[kSettleRows], near[kSettleRows][4];
 #pragma unroll
   for (int r = 0; r < kSettleRows; ++r) {
-    if ((uint32_t)(r * kSettleBlock) >= count) continue;
+    if ((uint32_t)(r * BLOCK) >= count) continue;
     spot[r] = geo.spot(t[r], 1);
     const uint32_t local = spot[r].bucket - b0;
     const uint32_t j = local * kSlabIndexLen + (spot[r].offset >> geo.sub_shift) / (uint32_t)kSlabIndexStep;
@@ -700,7 +710,7 @@ __global__ __launch_bounds__(kSettleBlock) void k_slab_settle(SlabGeom geo, Slab
   for (int r = 0; r < kSettleRows; ++r) {
     head[r] = kNone;
     cell[r] = 0;
-    if ((uint32_t)(r * kSettleBlock) >= count || !(in & (1u << r))) continue;
+    if ((uint32_t)(r * BLOCK) >= count || !(in & (1u << r))) continue;
     for (uint32_t at = pos[r];;) {
       bool past = false;
 #pragma unroll
@@ -742,7 +752,7 @@ __global__ __launch_bounds__(kSettleBlock) void k_slab_settle(SlabGeom geo, Slab
   // everybody has entered: who holds the slot moves in, and pushes out a level-1 owner that is there
 #pragma unroll
   for (int r = 0; r < kSettleRows; ++r) {
-    if ((uint32_t)(r * kSettleBlock) >= count || !(in & (1u << r)) || (uint32_t)sh.cells[cell[r]] != t[r]) continue;
+    if ((uint32_t)(r * BLOCK) >= count || !(in & (1u << r)) || (uint32_t)sh.cells[cell[r]] != t[r]) continue;
     const uint32_t local = cell[r] >> kSlabPartLog2;
     atomicAdd(&sh.in[local], 1u);
     if (head[r] != kNone) {
@@ -753,7 +763,7 @@ __global__ __launch_bounds__(kSettleBlock) void k_slab_settle(SlabGeom geo, Slab
   }
   __syncthreads();
   u32x4 *out = reinterpret_cast<u32x4 *>(cells + ((size_t)b0 << kSlabPartLog2));
-  for (uint32_t i = threadIdx.x; i < (buckets << kSlabPartLog2) / 2u; i += kSettleBlock) {
+  for (uint32_t i = threadIdx.x; i < (buckets << kSlabPartLog2) / 2u; i += BLOCK) {
     const u32x4 q = clear[i];
     if (q.y | q.w) out[i] = q;  // (the map is zero)
   }
@@ -1159,21 +1169,40 @@ struct SlabPlan {
   size_t bytes;           // of the workspace
 };
 
+// How many of `capacity` entries lose their level-1 slot: a half of capacity^2 / m where slots are drawn evenly, of which the
+// hash makes 0.97 times as many where four does not divide m, 1.3 to 1.45 where it does (1.0 and up at small odd multiples of
+// a large power of two) and 0.50 at powers of two, which count as 0.7: settling pays from fewer there.
+double slab_losers(uint32_t m, int64_t capacity) {
+  const double even = 0.5 * (double)capacity * ((double)capacity / m);
+  return (m & (m - 1u)) == 0 ? 0.7 * even : m & 3u ? even : 1.4 * even;
+}
+
+bool settled_by_few(int partitions) { return (uint32_t)partitions > kGroupsMost; }
+
 // `state` is memory that is zero between calls (see above); everything else comes out of the workspace.
 SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partitions, int dtype, int64_t capacity) {
   SlabPlan p;
   const size_t B = geo.nbuckets;
   const int64_t list_cap = list_capacity(capacity);
-  // The hash loses 1.4 times as many as evenly spread slots would.
-  const double losers = 0.7 * (double)capacity * ((double)capacity / geo.m);
-  p.tb.per_group = std::min(std::max((geo.nbuckets + kGroupsWanted - 1u) / kGroupsWanted, kGroupLeast), kGroupBuckets);
-  p.tb.gpp = (geo.bpp + p.tb.per_group - 1u) / p.tb.per_group;
+  const double losers = slab_losers(geo.m, capacity);
+  const bool settled = losers > std::max(kSettleFrom * geo.nbuckets, kSettleLeast) && geo.span <= kSlabSpan2;
+  const bool few = settled_by_few(partitions);
+  const uint32_t most = few ? kFewGroupsMost : kGroupsMost;
+  uint32_t per = std::min(std::max((geo.nbuckets + kGroupsMost - 1u) / kGroupsMost, kGroupLeast), kGroupBuckets);
+  if (settled) {  // (no more groups than the chip takes at a time, where their sizes allow that)
+    const uint32_t each = std::max(most / (uint32_t)partitions, 1u);
+    per = (geo.bpp + each - 1u) / each;
+    per = few ? std::min(per, kFewBuckets) : std::min(std::max(per, kGroupLeast), kGroupBuckets);
+  }
+  p.tb.per_group = per;
+  p.tb.gpp = (geo.bpp + per - 1u) / per;
   p.tb.group_pad = (p.tb.gpp + 31u) & ~31u;
   const size_t groups = (size_t)p.tb.gpp * partitions;
   p.tb.group_cap = 0;
-  if (losers > kSettleFrom && geo.span <= kSlabSpan2 && p.tb.gpp <= kMostGroups &&
-      (size_t)partitions * p.tb.group_pad <= kMostGroupWords)
-    p.tb.group_cap = std::min((uint32_t)(1.25 * losers / (double)groups) + 512u, kGroupCap);
+  if (settled) {
+    const uint32_t room = (uint32_t)((few ? kFewBlock : kSettleBlock) * kSettleRows);
+    p.tb.group_cap = std::min((uint32_t)(1.25 * losers / (double)groups) + 512u, room);
+  }
   {
     Carver cv(state);
     p.sample_hist[0] = cv.take<uint32_t>(sampled_floor_zero_bytes() / sizeof(uint32_t));
@@ -1245,7 +1274,10 @@ int slab_launch_span(const SlabBalanceArgs &a, const SlabGeom &geo, const SlabPl
     ProfScope prof(kProfSlabChains, s);
     const uint32_t groups = tb.gpp * (uint32_t)tb.partitions;
     if (tb.group_cap) {
-      k_slab_settle<<<dim3(groups), dim3(kSettleBlock), 0, s>>>(geo, tb, a.hash, a.status);
+      if (settled_by_few(tb.partitions))
+        k_slab_settle<kFewBlock, kFewBuckets><<<dim3(groups), dim3(kFewBlock), 0, s>>>(geo, tb, a.hash, a.status);
+      else
+        k_slab_settle<kSettleBlock, kGroupBuckets><<<dim3(groups), dim3(kSettleBlock), 0, s>>>(geo, tb, a.hash, a.status);
       ZEN_LAUNCH_CHECK("k_slab_settle");
     }
     const uint32_t share = std::min(std::max(kChainsResident / groups, 1u), 16u);
@@ -1305,7 +1337,7 @@ bool slab_balance_fits(int64_t n, int64_t m, int partitions, int dtype, int64_t 
   SlabGeom g;
   if (!encode_geometry(m, partitions, capacity, &g)) return false;
   // slab_geometry wants m >= 2^22: a table of 16 MB or more, of which the map takes at most half and the
-  // counters less than 1 MB
+  // counters less than 2 MB
   if (geo) *geo = g;
   return true;
 }
