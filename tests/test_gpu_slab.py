@@ -377,6 +377,33 @@ def test_slab_load_balance_declines_and_general_mode_takes_over(zen, oracle):
     assert np.array_equal(np.concatenate([to_np(v) for v in values]), val_o)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("fast_path", ["wide"], indirect=True)  # (the slabs set nothing aside)
+def test_wide_load_balance_declines_a_bucket_of_shared_slots(zen, oracle, dtype):
+    """6300 records of one bucket share their slot with another: three times what a workgroup has room to set aside."""
+    from zen_repro_amd import _lib
+    from zen_repro_amd.workloads import hash_slot
+
+    n, P, capacity = (1 << 20) + 64, 4, 130000
+    t = torch.arange(1, n)
+    t = t[hash_slot(t, n) < n // P // 32 - 200]
+    slots = hash_slot(t, n)
+    assert 6144 < torch.count_nonzero(torch.bincount(slots)[slots] > 1) < t.numel() < 8192
+    g = np.zeros(n, dtype=np.uint16 if dtype == "bf16" else np.float32)
+    g[t.numpy()] = 0x3F80 if dtype == "bf16" else 1.0
+    idx_o, val_o, splits_o, st_o = oracle.load_balance(g, P, 1, 3)
+    assert st_o == 0 and lb_path(zen, n, P, dtype, capacity) == WIDE
+    tp = zen.TensorPartition(P, 1, 3)
+    d = to_dev(g)
+    for _ in range(2):
+        _, _, _, status = tp.load_balance_flat(d, capacity=capacity, mode=_lib.MODE_FAST)
+        assert status.item() & _lib.STAT_RETRY
+        tp._table(d.device, n).zero_()
+    indices, values, splits = tp.load_balance(d, capacity=capacity)
+    assert np.array_equal(to_np(splits), splits_o)
+    assert np.array_equal(to_np(torch.cat(indices)), idx_o) and np.array_equal(to_np(torch.cat(values)), val_o)
+
+
 def test_slab_load_balance_too_many_candidates_declines(zen, oracle):
     """A capacity far below what is selected: the candidate list overflows, the
     call declines instead of writing out of bounds."""

@@ -274,8 +274,8 @@ __device__ unsigned long long g_wide_dbg[256 * 32];
 // Puts the bucket's records that reach the threshold in order of (level-1 slot, index): indices to sh.idx, values to sh.val
 // (the losers of a slot marked, their places and indices noted in sh.gone and sh.rm), the narrow ranges' first places to
 // memory for the look-ups of other workgroups.  Returns how many there are.  ROUNDS: of kWideBlock records of every part.
-// One round, up to eight records a thread, is written out, its records stay in registers from their load to the end; of
-// three the loops' bodies handle the first kWideLanes registers of a set and then rotate the set, and the records are
+// One round and two, up to sixteen records a thread, are written out, their records stay in registers from their load to the
+// end; of three the loops' bodies handle the first kWideLanes registers of a set and then rotate the set, and the records are
 // loaded again (written out, the code would no longer fit the instruction cache, and every workgroup runs it just once).
 // A chain of LDS and memory trips bounds it, not a rate.  Written out, with the records held and the removed places noted
 // instead of searched for, the launch took 31 us where the loops took 36 (62 M bf16 elements, 0.5 %, 128 workgroups) and
@@ -470,8 +470,12 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
   {
     uint32_t pending = sh.queued;
     if (pending > (uint32_t)kWideQueue) {
+      // more than there is room for: declined, with nothing in the bucket (those without room have no rank of their own, and
+      // what no record is put into must not be taken for an index)
       if (tid == 0) atomicOr(status, ZEN_STAT_RETRY);
-      pending = kWideQueue;
+#pragma unroll
+      for (int i = 0; i < kItems; ++i) rk[i] = kInvalid;
+      pending = n = 0;
     }
     for (uint32_t e = tid; e < pending; e += kWideBlock) {
       const uint32_t my = sh.q_word[e], key = my >> 15;
@@ -504,7 +508,7 @@ __device__ inline uint32_t wide_sort(WideShared<S> &sh, const SlabGeom &geo, con
     for (uint32_t j = tid; j < (uint32_t)kWideIndexLen; j += kWideBlock) {
       const uint32_t s0 = j * kWideIndexStep;
       store_agent(&tb.sub_index[(size_t)b * kWideIndexLen + j],
-                  sh.cnt.start_of(s0) | (sh.cnt.end_of(s0 + kWideIndexStep - 1) << 16));
+                  n ? sh.cnt.start_of(s0) | (sh.cnt.end_of(s0 + kWideIndexStep - 1) << 16) : 0u);
     }
     __syncthreads();
     // room in the partition's log, on its way while the records are put in order
