@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <map>
+#include <optional>
 #include <tuple>
 #include <utility>
 #include <vector>
@@ -210,11 +211,13 @@ py::tuple decode_lists(const py::object &fn, Zeros &zeros, const std::vector<Ten
   return py::make_tuple(rc, dense);
 }
 
+// `told`: a status word that is answered for with this call's own, of work in front of it on the stream.
 py::tuple bitmaps_dense(const py::object &fn, Zeros &zeros, const std::vector<Tensor> &bitmaps,
                         const std::vector<Tensor> &values, int code, const Tensor &dict, int64_t numel, const Tensor &ws,
-                        int64_t stream, int64_t host, int64_t words) {
-  const auto [dense, status] =
-      made([&] { return Two{room(values[0], numel, values[0].scalar_type()), zeros.status(values[0], stream)}; });
+                        int64_t stream, int64_t host, int64_t words, const std::optional<Tensor> &told) {
+  const auto [dense, status] = made([&] {
+    return Two{room(values[0], numel, values[0].scalar_type()), told ? *told : zeros.status(values[0], stream)};
+  });
   const Lists b(bitmaps), v(values);
   const py::object rc = fn(address(dict), numel, bitmaps.size(), b.addresses(), b.counts(), v.addresses(), code, v.counts(),
                            address(dense), address(ws), ws.numel(), address(status), host, words, stream);
@@ -225,10 +228,13 @@ py::tuple bitmap_encode(const py::object &fn, Zeros &zeros, const Tensor &mappin
                         int64_t numel, int64_t count, int64_t stream, int64_t host, int64_t words) {
   const auto [bitmap, status] =
       made([&] { return Two{room(indices, std::max<int64_t>(count, 1) * 4, at::kByte), zeros.status(indices, stream)}; });
-  const py::object rc = fn(address(mapping), mapping.numel(), address(indices), indices.scalar_type() == at::kLong ? 1 : 0,
-                           indices.numel(), py::none(), address(ranks), numel, address(bitmap), address(status), host, words,
-                           stream);
-  return py::make_tuple(rc, bitmap.narrow(0, 0, (mapping.numel() + 7) / 8));
+  const int idx64 = indices.scalar_type() == at::kLong ? 1 : 0;
+  const py::object rc =
+      host ? fn(address(mapping), mapping.numel(), address(indices), idx64, indices.numel(), py::none(), address(ranks), numel,
+                address(bitmap), address(status), host, words, stream)
+           : fn(address(mapping), mapping.numel(), address(indices), idx64, indices.numel(), py::none(), address(ranks), numel,
+                address(bitmap), address(status), stream);
+  return py::make_tuple(rc, bitmap.narrow(0, 0, (mapping.numel() + 7) / 8), status);
 }
 
 py::tuple tables(const py::object &fn, Zeros &zeros, const Tensor &input, int code, int64_t m, int64_t serial_n,
