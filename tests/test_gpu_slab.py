@@ -105,8 +105,8 @@ def slab_buckets(m, P, capacity):
 
 def slab_settles(m, P, capacity):
     """Whether the losers of level 1 are settled group by group (plan_slab)."""
-    losers = 0.5 * capacity ** 2 / m * (0.7 if m & (m - 1) == 0 else 1 if m % 4 else 1.4)
-    return losers > max(135 * slab_buckets(m, P, capacity) * P, 40000)
+    losers = 0.5 * capacity ** 2 / m * (1.4 if m % 4 == 0 and m & (m - 1) else 1)
+    return losers > min(max((150 if P > 256 else 175) * slab_buckets(m, P, capacity) * P, 50000), 450000)
 
 
 @pytest.mark.parametrize("P,log2,density,room,rehash,settled", [
@@ -118,10 +118,13 @@ def slab_settles(m, P, capacity):
     (7, 24, 0.22, 1.05, 3, True),     # the last group of a partition has fewer buckets
     (300, 24, 0.22, 1.05, 3, True),   # more partitions than groups are wanted: groups of three buckets
     (1000, 24, 0.24, 1.02, 2, True),  # ... of one
-    (16, 24, 0.057, 1.0, 3, False),   # fewer than 40 000 losers
-    (16, 24, 0.06, 1.0, 3, True),
-    (257, 24, 0.09, 1.0, 3, False),   # fewer than 135 to a bucket
-    (257, 24, 0.093, 1.0, 3, True),
+    (16, 22, 0.127, 1.0, 3, False),   # fewer than 50 000 losers
+    (16, 22, 0.135, 1.0, 3, True),
+    (16, 24, 0.07, 1.0, 3, False),    # fewer than 175 to a bucket
+    (16, 24, 0.075, 1.0, 3, True),
+    (16, 24, 0.11, 2.0, 3, True),     # a capacity twice what is selected
+    (257, 24, 0.09, 1.0, 3, False),   # fewer than 150 to a bucket
+    (257, 24, 0.1, 1.0, 3, True),
 ])
 @pytest.mark.parametrize("fast_path", ["slabs"], indirect=True)
 def test_slab_load_balance_of_settled_losers(zen, oracle, P, log2, density, room, rehash, settled):
@@ -197,8 +200,8 @@ def test_slab_load_balance_of_losers_in_one_place(zen, oracle, rehash, dtype):
     (3, 0.16, 1.1, 202997, True),
     (16, 0.1, 2.0, 119306, True),
     (16, 0.1, 1.1, 119306, True),
-    (3, 0.078, 1.0, 49630, True),   # just past the line
-    (3, 0.075, 1.0, 45974, False),  # just below it
+    (3, 0.1, 1.0, 80917, True),     # just past the line
+    (3, 0.09, 1.0, 65756, False),   # just below it
 ])
 @pytest.mark.parametrize("fast_path", ["slabs"], indirect=True)
 def test_slab_load_balance_of_many_losers(zen, oracle, P, density, room, losers, settled, dtype):

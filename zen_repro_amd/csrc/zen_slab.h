@@ -79,13 +79,6 @@ struct SlabGeom {
     const uint32_t part = b / bpp, sb = b - part * bpp;
     return part * npp + first_local(sb);
   }
-  __device__ inline uint32_t bucket_and_offset(uint32_t key, uint32_t *offset) const {  // key - first_key(bucket)
-    uint32_t local;
-    const uint32_t part = div_small(key, npp, inv_npp, &local);
-    const uint32_t sb = __umulhi(local, bpp_mult);
-    *offset = local - first_local(sb);
-    return part * bpp + sb;
-  }
   // Where index t looks at rehash level 1 or 2: as probe_slot, with the slot's bucket and its offset there, and without a
   // division (x * npp_mult / 2^32 is the quotient or one less).
   struct Spot {

@@ -81,22 +81,23 @@ __device__ inline uint32_t cell_slot(unsigned long long cell) { return (uint32_t
 // k_slab_settle enters a group's list into its parts of the map in LDS: device-wide atomics are carried out at 25 a
 // nanosecond, and of an entry for each loser in the map and one to count it nine in ten fall away.  Where fewer are
 // expected each goes its way through memory (k_slab_chains), for the other way is a launch more and two barriers in the sort.
-// What settling costs goes with the buckets, what it saves with the losers: it pays from about 135 expected losers to a
-// bucket and 40 000 in all.  Whole calls, bf16, 62 M slots, sixteen partitions, by losers to a bucket, unsettled and settled,
-// us: 120 115.2 and 114.5, 146 122.9 and 122.8, 195 127.0 and 123.4, 208 158.1 and 147.3, 325 202.9 and 180.3, 382 313.8 and
-// 255.5.  250 M: 117 254.6 and 254.2, 144 300.4 and 294.2.  62 M, an odd number: 105 118.4 and 120.9, 174 131.7 and 130.3, 206
-// 203.5 and 188.3.  2^26: 91 122.7 and 123.4, 162 149.0 and 146.5.  2^28: 84 307.1 and 314.6.  Few in all, 4 to 17 M slots:
-// 29 000 55.6 and 54.9, 55.7 and 56.8, 59.9 and 60.6; 39 000 66.6 and 67.4; 44 000 62.8 and 61.3, 61.7 and 60.1; 59 000 69.6
-// and 65.5, 74.7 and 74.5.
-constexpr double kSettleFrom = 135, kSettleLeast = 40000;
+// What settling costs goes with the buckets, what it saves with the losers.  Whole calls, bf16, 62 M slots, sixteen partitions, a
+// capacity 1.05 times what is selected, by expected losers to a bucket, unsettled and settled, us: 120 115.2 and 114.5, 146
+// 122.9 and 122.8, 195 127.0 and 123.4, 208 158.1 and 147.3, 325 202.9 and 180.3, 382 313.8 and 255.5; with a capacity of 1.25
+// times, where fewer come than are expected, 166 402.5 and 403.5 (a pass of the hook).  62 M, an odd number: 105 118.4 and 120.9,
+// 174 131.7 and 130.3, 206 203.5 and 188.3.  2^26: 129 122.7 and 123.4, 232 149.0 and 146.5; 2^28: 120 307.1 and 314.6.  Few in
+// all, 4 to 17 M slots: 29 000 55.6 and 54.9, 55.7 and 56.8, 59.9 and 60.6; 44 000 62.8 and 61.3, 61.7 and 60.1; 59 000 69.6 and
+// 65.5, 74.7 and 74.5.  Many in all, 250 M slots, 3072 and 3584 buckets: 440 000 300.4 and 294.2, 549 000 347.5 and 328.9.
+constexpr double kSettleFrom = 175, kSettleLeast = 50000, kSettleAnyway = 450000;
 constexpr uint32_t kGroupBuckets = 12;         // of a group, at most: their parts of the map and indices fill 121 KB
 constexpr uint32_t kGroupLeast = 4, kGroupsMost = 256;  // (a compute unit to each)
 constexpr uint32_t kMostGroups = kSlabMaxBuckets / kGroupBuckets + 1;  // of a partition
 constexpr int kSettleBlock = 1024;
 constexpr int kSettleRows = 6;                 // losers of a thread, at most
-// More partitions than kGroupsMost: groups of a few buckets, five to a compute unit (and the same line).  62 M slots, 300
-// partitions, by expected losers to a bucket: 99 105.9 and 106.7 us, 166 116.5 and 114.7, 199 157.9 and 147.4, 408 294 and 245; 1024:
-// 87 109.4 and 110.7, 146 126.8 and 123.7, 195 172 and 163; 3000: 99 176 and 179, 166 226 and 213, 326 324 and 271.
+// More partitions than kGroupsMost: groups of a few buckets, five to a compute unit.  62 M slots, by expected losers to a bucket:
+// 300 partitions 99 105.9 and 106.7 us, 159 138.4 and 133.6, 199 157.9 and 147.4, 408 294 and 245; 700: 142 126.7 and 127.8,
+// 171 139.8 and 138.0; 1300: 153 139.0 and 134.2; 3000: 99 176 and 179, 166 226 and 213, 326 324 and 271.
+constexpr double kSettleFewFrom = 150;
 constexpr uint32_t kFewBuckets = 3, kFewGroupsMost = 1280;
 constexpr int kFewBlock = 256;
 constexpr uint32_t kChainsResident = 1024;     // workgroups of k_slab_chains the chip holds at a time
@@ -1170,11 +1171,11 @@ struct SlabPlan {
 };
 
 // How many of `capacity` entries lose their level-1 slot: a half of capacity^2 / m where slots are drawn evenly, of which the
-// hash makes 0.97 times as many where four does not divide m, 1.3 to 1.45 where it does (1.0 and up at small odd multiples of
-// a large power of two) and 0.50 at powers of two, which count as 0.7: settling pays from fewer there.
+// hash makes 1.3 to 1.45 times as many where four divides m (1.0 and up at small odd multiples of a large power of two), 0.97
+// where it does not, and 0.50 at powers of two, which count in full: settling pays from fewer there.
 double slab_losers(uint32_t m, int64_t capacity) {
   const double even = 0.5 * (double)capacity * ((double)capacity / m);
-  return (m & (m - 1u)) == 0 ? 0.7 * even : m & 3u ? even : 1.4 * even;
+  return (m & 3u) == 0 && (m & (m - 1u)) != 0 ? 1.4 * even : even;
 }
 
 bool settled_by_few(int partitions) { return (uint32_t)partitions > kGroupsMost; }
@@ -1185,8 +1186,9 @@ SlabPlan plan_slab(void *workspace, void *state, const SlabGeom &geo, int partit
   const size_t B = geo.nbuckets;
   const int64_t list_cap = list_capacity(capacity);
   const double losers = slab_losers(geo.m, capacity);
-  const bool settled = losers > std::max(kSettleFrom * geo.nbuckets, kSettleLeast) && geo.span <= kSlabSpan2;
   const bool few = settled_by_few(partitions);
+  const double from = std::max((few ? kSettleFewFrom : kSettleFrom) * geo.nbuckets, kSettleLeast);
+  const bool settled = losers > std::min(from, kSettleAnyway) && geo.span <= kSlabSpan2;
   const uint32_t most = few ? kFewGroupsMost : kGroupsMost;
   uint32_t per = std::min(std::max((geo.nbuckets + kGroupsMost - 1u) / kGroupsMost, kGroupLeast), kGroupBuckets);
   if (settled) {  // (no more groups than the chip takes at a time, where their sizes allow that)
