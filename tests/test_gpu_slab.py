@@ -106,7 +106,7 @@ def slab_buckets(m, P, capacity):
 def slab_settles(m, P, capacity):
     """Whether the losers of level 1 are settled group by group (plan_slab)."""
     losers = 0.5 * capacity ** 2 / m * (1.4 if m % 4 == 0 and m & (m - 1) else 1)
-    return losers > min(max((150 if P > 256 else 175) * slab_buckets(m, P, capacity) * P, 50000), 450000)
+    return losers > min(max((190 if P > 256 else 250) * slab_buckets(m, P, capacity) * P, 50000), 400000)
 
 
 @pytest.mark.parametrize("P,log2,density,room,rehash,settled", [
@@ -120,11 +120,11 @@ def slab_settles(m, P, capacity):
     (1000, 24, 0.24, 1.02, 2, True),  # ... of one
     (16, 22, 0.127, 1.0, 3, False),   # fewer than 50 000 losers
     (16, 22, 0.135, 1.0, 3, True),
-    (16, 24, 0.07, 1.0, 3, False),    # fewer than 175 to a bucket
-    (16, 24, 0.075, 1.0, 3, True),
+    (16, 24, 0.1, 1.0, 3, False),     # fewer than 250 to a bucket
+    (16, 24, 0.105, 1.0, 3, True),
     (16, 24, 0.11, 2.0, 3, True),     # a capacity twice what is selected
-    (257, 24, 0.09, 1.0, 3, False),   # fewer than 150 to a bucket
-    (257, 24, 0.1, 1.0, 3, True),
+    (257, 24, 0.13, 1.0, 3, False),   # fewer than 190 to a bucket
+    (257, 24, 0.136, 1.0, 3, True),
 ])
 @pytest.mark.parametrize("fast_path", ["slabs"], indirect=True)
 def test_slab_load_balance_of_settled_losers(zen, oracle, P, log2, density, room, rehash, settled):
@@ -200,8 +200,8 @@ def test_slab_load_balance_of_losers_in_one_place(zen, oracle, rehash, dtype):
     (3, 0.16, 1.1, 202997, True),
     (16, 0.1, 2.0, 119306, True),
     (16, 0.1, 1.1, 119306, True),
-    (3, 0.1, 1.0, 80917, True),     # just past the line
-    (3, 0.09, 1.0, 65756, False),   # just below it
+    (3, 0.125, 1.0, 125090, True),  # just past the line
+    (3, 0.12, 1.0, 115574, False),  # just below it
 ])
 @pytest.mark.parametrize("fast_path", ["slabs"], indirect=True)
 def test_slab_load_balance_of_many_losers(zen, oracle, P, density, room, losers, settled, dtype):

@@ -81,14 +81,15 @@ __device__ inline uint32_t cell_slot(unsigned long long cell) { return (uint32_t
 // k_slab_settle enters a group's list into its parts of the map in LDS: device-wide atomics are carried out at 25 a
 // nanosecond, and of an entry for each loser in the map and one to count it nine in ten fall away.  Where fewer are
 // expected each goes its way through memory (k_slab_chains), for the other way is a launch more and two barriers in the sort.
-// What settling costs goes with the buckets, what it saves with the losers.  Whole calls, bf16, 62 M slots, sixteen partitions, a
-// capacity 1.05 times what is selected, by expected losers to a bucket, unsettled and settled, us: 120 115.2 and 114.5, 146
-// 122.9 and 122.8, 195 127.0 and 123.4, 208 158.1 and 147.3, 325 202.9 and 180.3, 382 313.8 and 255.5; with a capacity of 1.25
-// times, where fewer come than are expected, 166 402.5 and 403.5 (a pass of the hook).  62 M, an odd number: 105 118.4 and 120.9,
-// 174 131.7 and 130.3, 206 203.5 and 188.3.  2^26: 129 122.7 and 123.4, 232 149.0 and 146.5; 2^28: 120 307.1 and 314.6.  Few in
-// all, 4 to 17 M slots: 29 000 55.6 and 54.9, 55.7 and 56.8, 59.9 and 60.6; 44 000 62.8 and 61.3, 61.7 and 60.1; 59 000 69.6 and
-// 65.5, 74.7 and 74.5.  Many in all, 250 M slots, 3072 and 3584 buckets: 440 000 300.4 and 294.2, 549 000 347.5 and 328.9.
-constexpr double kSettleFrom = 175, kSettleLeast = 50000, kSettleAnyway = 450000;
+// What settling costs goes with the buckets, what it saves with the losers.  Whole calls, bf16, 62 M slots, sixteen partitions,
+// by expected losers to a bucket, unsettled and settled, us: with a capacity of 1.05 times what is selected 120 115.2 and 114.5,
+// 146 122.9 and 122.8, 195 127.0 and 123.4, 244 142.2 and 134.7, 325 202.9 and 180.3, 382 313.8 and 255.5; with 1.5 times, of
+// whose losers fewer than a half come, 239 43.5 and 45.3 (sort, settling and chains).  The line lies between the two.  62 M, an odd
+// number: 105 118.4 and 120.9, 174 131.7 and 130.3, 206 203.5 and 188.3.  2^26: 129 122.7 and 123.4, 232 149.0 and 146.5; 2^28:
+// 120 307.1 and 314.6.  Few in all, 4 to 17 M slots: 29 000 55.6 and 54.9, 55.7 and 56.8, 59.9 and 60.6; 44 000 62.8 and 61.3, 61.7
+// and 60.1; 59 000 69.6 and 65.5, 74.7 and 74.5.  Many in all, 250 M slots, 3072 and 3584 buckets: 440 000 300.4 and 294.2,
+// 549 000 347.5 and 328.9.
+constexpr double kSettleFrom = 250, kSettleLeast = 50000, kSettleAnyway = 400000;
 constexpr uint32_t kGroupBuckets = 12;         // of a group, at most: their parts of the map and indices fill 121 KB
 constexpr uint32_t kGroupLeast = 4, kGroupsMost = 256;  // (a compute unit to each)
 constexpr uint32_t kMostGroups = kSlabMaxBuckets / kGroupBuckets + 1;  // of a partition
@@ -96,8 +97,9 @@ constexpr int kSettleBlock = 1024;
 constexpr int kSettleRows = 6;                 // losers of a thread, at most
 // More partitions than kGroupsMost: groups of a few buckets, five to a compute unit.  62 M slots, by expected losers to a bucket:
 // 300 partitions 99 105.9 and 106.7 us, 159 138.4 and 133.6, 199 157.9 and 147.4, 408 294 and 245; 700: 142 126.7 and 127.8,
-// 171 139.8 and 138.0; 1300: 153 139.0 and 134.2; 3000: 99 176 and 179, 166 226 and 213, 326 324 and 271.
-constexpr double kSettleFewFrom = 150;
+// 171 139.8 and 138.0; 1300: 153 139.0 and 134.2; 3000: 99 176 and 179, 166 226 and 213, 326 324 and 271.  (The line leaves room
+// for larger capacities here too.)
+constexpr double kSettleFewFrom = 190;
 constexpr uint32_t kFewBuckets = 3, kFewGroupsMost = 1280;
 constexpr int kFewBlock = 256;
 constexpr uint32_t kChainsResident = 1024;     // workgroups of k_slab_chains the chip holds at a time
@@ -651,7 +653,7 @@ __device__ inline void slab_chain(const SlabGeom &geo, const Probe &g, const Sla
 // owner takes no cell, and the parts hold no more than the chains alone would put there (16.8 M slots, 27.8 % of them taken,
 // 32 partitions: 943 cells in the fullest part; entered first, 1065, more than there are).  Nobody else touches the map while this kernel
 // runs.  Bound by latency (four or five trips to memory, as many phases in LDS) and instructions: a group to a compute
-// unit, its losers to all of the unit's waves.  62 M slots, 436 000 losers in 256 groups 19.5 us, the chains behind it 23
+// unit, its losers to all of the unit's waves.  62 M slots, 436 000 losers in 256 groups 19.4 us, the chains behind it 23.6
 // (without it the chains 50, and 15 to count the entries that moved in).
 template <uint32_t BUCKETS>
 struct SlabSettleLds {
@@ -779,8 +781,8 @@ __global__ __launch_bounds__(BLOCK) void k_slab_settle(SlabGeom geo, SlabTables 
 // workgroups to a group of buckets and as few lanes of a wave as that allows: a wave goes on until the last of them has
 // found its place.  Bound by latency: a probe is three or four dependent trips to memory (the bucket's index, its records,
 // the map), with a wave to its lanes 1.2 us, and by what all wait for in the end, the layout.  62 M slots, 110 000 losers
-// 29.6 -> 25.8 us, 268 M, 18 000 15.8 -> 14.1, 12.9 M, 900 14.9 -> 11.2 (dense waves, a log in one place, divisions, a
-// layout by lines of its own to a lane); 72 000 left of 436 000 settled ones 23.
+// 29.6 -> 26.3 us, 268 M, 18 000 15.8 -> 14.4, 12.9 M, 900 14.9 -> 11.2 (dense waves, a log in one place, divisions, a
+// layout by lines of its own to a lane); 72 000 left of 436 000 settled ones 23.6.
 __global__ __launch_bounds__(kSlabBlock, 8) void k_slab_chains(SlabGeom geo, Probe g, SlabTables tb, unsigned long long *cells,
                                                             uint32_t share, int64_t spp, uint32_t capacity,
                                                             int64_t *__restrict__ splits, HostAnswer answer,
