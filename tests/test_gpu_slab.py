@@ -116,8 +116,10 @@ def slab_settles(m, P, capacity):
     (32, 24, 0.2812, 1.0, 3, True),   # ... 966 and 1091
     (1, 26, 0.08, 1.35, 3, True),     # one partition of all groups
     (7, 24, 0.22, 1.05, 3, True),     # the last group of a partition has fewer buckets
-    (300, 24, 0.22, 1.05, 3, True),   # more partitions than groups are wanted: groups of three buckets
-    (1000, 24, 0.24, 1.02, 2, True),  # ... of one
+    (300, 24, 0.22, 1.05, 3, True),   # more than 256 partitions: groups of one bucket ...
+    (1000, 24, 0.24, 1.02, 2, True),
+    (300, 25, 0.155, 1.05, 3, True),  # ... of two, the last of a partition of one
+    (650, 25, 0.185, 1.0, 3, True),   # ... of three
     (16, 22, 0.127, 1.0, 3, False),   # fewer than 50 000 losers
     (16, 22, 0.135, 1.0, 3, True),
     (16, 24, 0.1, 1.0, 3, False),     # fewer than 250 to a bucket
