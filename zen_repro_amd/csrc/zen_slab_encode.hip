@@ -651,10 +651,10 @@ __device__ inline void slab_chain(const SlabGeom &geo, const Probe &g, const Sla
 // index there, or is pushed out by one, goes on at level 3 too.  A larger level-1 owner is pushed out by the entry that holds
 // its slot in the end, and goes on at level 2.  The owner is asked for first, as a single chain does: a slot with a smaller
 // owner takes no cell, and the parts hold no more than the chains alone would put there (16.8 M slots, 27.8 % of them taken,
-// 32 partitions: 943 cells in the fullest part; entered first, 1065, more than there are).  Nobody else touches the map while this kernel
-// runs.  Bound by latency (four or five trips to memory, as many phases in LDS) and instructions: a group to a compute
-// unit, its losers to all of the unit's waves.  62 M slots, 436 000 losers in 256 groups 19.4 us, the chains behind it 23.6
-// (without it the chains 50, and 15 to count the entries that moved in).
+// 32 partitions: 943 cells in the fullest part; entered first, 1065, more than there are).  Nobody else touches the map
+// while this kernel runs.  Bound by latency (four or five trips to memory, as many phases in LDS) and instructions: a group
+// to a compute unit, its losers to all of the unit's waves.  62 M slots, 436 000 losers in 256 groups 19.4 us, the chains
+// behind it 23.6 (without it the chains 50, and 15 to count the entries that moved in).
 template <uint32_t BUCKETS>
 struct SlabSettleLds {
   unsigned long long cells[BUCKETS << kSlabPartLog2];
